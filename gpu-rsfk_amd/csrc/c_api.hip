@@ -59,13 +59,12 @@ RSFK_API void pymodule_cluster_by_sample_tree(int N, int D, int MIN_TREE_CHILD, 
     std::vector<int> perm, ls, lz;
     int stats[5] = {0, 0, 0, 0, 0};
     {
+        HostStage stage;
         DevMem dp;
         if (N < 1 || D < 1) { set_last_error("N and D must be positive"); die("pymodule_cluster_by_sample_tree"); }
         if (dp.alloc(sizeof(float) * (size_t)N * (size_t)D)) die("pymodule_cluster_by_sample_tree");
-        if (hipMemcpy(dp.p, points, sizeof(float) * (size_t)N * (size_t)D, hipMemcpyHostToDevice) != hipSuccess) {
-            set_last_error("hipMemcpy of the points failed");
-            die("pymodule_cluster_by_sample_tree");
-        }
+        const HostArray in{dp.p, points, sizeof(float) * (size_t)N * (size_t)D};
+        if (stage.to_device(&in, 1, nullptr)) die("pymodule_cluster_by_sample_tree");
         if (build_tree_host(static_cast<const float*>(dp.p), N, D, MIN_TREE_CHILD, MAX_TREE_CHILD, MAX_DEPTH,
                             RANDOM_STATE, perm, ls, lz, stats))
             die("pymodule_cluster_by_sample_tree");
@@ -183,12 +182,11 @@ RSFK_API int rsfk_build_tree_host(const float* points, int N, int D, int MIN_TRE
                                   int leaf_cap, int* stats)
 {
     if (N < 1 || D < 1) { set_last_error("N and D must be positive"); return -2; }
+    HostStage stage;
     DevMem dp;
     if (dp.alloc(sizeof(float) * (size_t)N * (size_t)D)) return -1;
-    if (hipMemcpy(dp.p, points, sizeof(float) * (size_t)N * (size_t)D, hipMemcpyHostToDevice) != hipSuccess) {
-        set_last_error("hipMemcpy of the points failed");
-        return -1;
-    }
+    const HostArray in{dp.p, const_cast<float*>(points), sizeof(float) * (size_t)N * (size_t)D};
+    if (stage.to_device(&in, 1, nullptr)) return -1;
     std::vector<int> pv, ls, lz;
     int st[5];
     if (build_tree_host(static_cast<const float*>(dp.p), N, D, MIN_TREE_CHILD, MAX_TREE_CHILD, MAX_DEPTH,
@@ -281,6 +279,7 @@ RSFK_API int rsfk_last_build_report(char* buf, int capacity) { return build_repo
 RSFK_API void rsfk_release_workspace(void)
 {
     ws_release_all();
+    host_pool_release();
     release_copy_buffers();
 }
 

@@ -860,7 +860,7 @@ int explore_ws_alloc(ExploreWorkspace** out, int N, int K, bool with_bounds)
         dm(&w->bin_start, (size_t)w->n_bins + 1) != hipSuccess ||
         dm(&w->part_off, (size_t)w->n_parts * (size_t)w->n_bins) != hipSuccess || dm(&w->pass, total * w->MW) != hipSuccess || dm(&w->norm_tau, 2 * (size_t)N) != hipSuccess ||
         dm(&w->todo, 2 * ((size_t)N + 1)) != hipSuccess ||
-        hipHostMalloc(reinterpret_cast<void**>(&w->host_count), sizeof(int)) != hipSuccess) {
+        pin_alloc(reinterpret_cast<void**>(&w->host_count), sizeof(int)) != 0) {
         explore_ws_free(w);
         set_last_error("exploration workspace: out of device memory");
         return 1;
@@ -884,7 +884,7 @@ void explore_ws_free(ExploreWorkspace* w)
                     w->bin_eq2, w->fine_size, w->fine_start, w->sub_off};
     for (void* b : bufs)
         ws_free(b);
-    if (w->host_count) (void)hipHostFree(w->host_count);
+    pin_free(w->host_count);
     delete w;
 }
 

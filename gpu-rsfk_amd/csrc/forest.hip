@@ -80,13 +80,13 @@ struct SideStream {
     hipEvent_t big = nullptr;
     int open()
     {
-        RSFK_HIP(hipStreamCreateWithFlags(&side, hipStreamNonBlocking));
+        if (stream_take(&side)) return 1;
         RSFK_HIP(hipEventCreateWithFlags(&big, hipEventDisableTiming));
         return 0;
     }
     ~SideStream()
     {
-        if (side) { (void)hipStreamSynchronize(side); (void)hipStreamDestroy(side); }
+        if (side) { (void)hipStreamSynchronize(side); stream_give(side); }
         if (big) (void)hipEventDestroy(big);
     }
 };
@@ -488,22 +488,20 @@ int knn_ann_forest_host(int n_trees, int K, int N, int NQ, int D, int MIN, int M
 {
     RSFK_CHECK(N >= 1 && D >= 1 && K >= 1 && NQ >= 0, "query-set search: N, D and K must be positive");
     if (NQ == 0) return 0;
+    HostStage stage;
     DevBuf dp, dq, di, dd;
     const size_t nd = (size_t)N * (size_t)D, qd = (size_t)NQ * (size_t)D, nk = (size_t)NQ * (size_t)K;
     if (ws_alloc(&dp.p, nd * sizeof(float)) || ws_alloc(&dq.p, qd * sizeof(float)) || ws_alloc(&di.p, nk * sizeof(int)) ||
         ws_alloc(&dd.p, nk * sizeof(float)))
         return 1;
-    RSFK_HIP(hipMemcpy(dp.p, points, nd * sizeof(float), hipMemcpyHostToDevice));
-    RSFK_HIP(hipMemcpy(dq.p, queries, qd * sizeof(float), hipMemcpyHostToDevice));
-    RSFK_HIP(hipMemcpy(di.p, q_idx, nk * sizeof(int), hipMemcpyHostToDevice));
-    RSFK_HIP(hipMemcpy(dd.p, q_dist, nk * sizeof(float), hipMemcpyHostToDevice));
+    const HostArray in[] = {{dp.p, const_cast<float*>(points), nd * sizeof(float)}, {dq.p, const_cast<float*>(queries), qd * sizeof(float)},
+                            {di.p, q_idx, nk * sizeof(int)}, {dd.p, q_dist, nk * sizeof(float)}};
+    if (stage.to_device(in, 4, nullptr)) return 1;
     const int rc = knn_ann_forest_device(n_trees, K, N, NQ, D, MIN, MAX, MAX_DEPTH, verbose, seed,
                                          static_cast<const float*>(dp.p), static_cast<const float*>(dq.p),
                                          static_cast<int*>(di.p), static_cast<float*>(dd.p), log_forest, nullptr);
     if (rc) return rc;
-    RSFK_HIP(hipMemcpy(q_idx, di.p, nk * sizeof(int), hipMemcpyDeviceToHost));
-    RSFK_HIP(hipMemcpy(q_dist, dd.p, nk * sizeof(float), hipMemcpyDeviceToHost));
-    return 0;
+    return copy_to_host(in + 2, 2, nullptr);
 }
 
 namespace {
@@ -525,28 +523,26 @@ int knn_forest_host(int n_trees, int K, int N, int D, int MIN, int MAX, int MAX_
                     int nnef, const float* points, int* knn_idx, float* knn_dist, float* log_forest, int fresh_rows)
 {
     RSFK_CHECK(N >= 1 && D >= 1 && K >= 1, "forest: N, D and K must be positive");
+    HostStage stage;
     DevBuf dp, di, dd;
     const size_t nd = (size_t)N * (size_t)D, nk = (size_t)N * (size_t)K;
     if (ws_alloc(&dp.p, nd * sizeof(float))) return 1;
     if (ws_alloc(&di.p, nk * sizeof(int))) return 1;
     if (ws_alloc(&dd.p, nk * sizeof(float))) return 1;
-    if (copy_to_device(dp.p, points, nd * sizeof(float))) return 1;
+    const HostArray arrays[] = {{dp.p, const_cast<float*>(points), nd * sizeof(float)}, {di.p, knn_idx, nk * sizeof(int)},
+                                {dd.p, knn_dist, nk * sizeof(float)}};
+    if (stage.to_device(arrays, fresh_rows ? 1 : 3, nullptr)) return 1;
     if (fresh_rows) {
         const unsigned grid = (unsigned)std::min<size_t>((nk + 255) / 256, 65536);
         hipLaunchKernelGGL(k_fresh_rows, dim3(grid), dim3(256), 0, nullptr, static_cast<int*>(di.p), static_cast<float*>(dd.p),
                            nk, K, fresh_rows == 2 ? 1 : 0);
         RSFK_HIP(hipGetLastError());
-    } else {
-        if (copy_to_device(di.p, knn_idx, nk * sizeof(int))) return 1;
-        if (copy_to_device(dd.p, knn_dist, nk * sizeof(float))) return 1;
     }
     const int rc = knn_forest_device(n_trees, K, N, D, MIN, MAX, MAX_DEPTH, verbose, seed, nnef,
                                      static_cast<const float*>(dp.p), static_cast<int*>(di.p),
                                      static_cast<float*>(dd.p), log_forest, nullptr);
     if (rc) return rc;
-    if (copy_to_host(knn_idx, di.p, nk * sizeof(int))) return 1;
-    if (copy_to_host(knn_dist, dd.p, nk * sizeof(float))) return 1;
-    return 0;
+    return copy_to_host(arrays + 1, 2, nullptr);
 }
 
 // One tree; results on the host.  perm: N ints; leaves sorted by start.
@@ -565,15 +561,14 @@ int build_tree_host(const float* d_points, int N, int D, int MIN, int MAX, int M
     const int nl = stats[0], n_big = stats[4], n_small = nl - n_big, cap = tree_ws_leaf_cap(ws.w);
     perm.resize((size_t)N);
     std::vector<int> ls((size_t)nl), lz((size_t)nl);
-    RSFK_HIP(hipMemcpy(perm.data(), tree_ws_perm(ws.w, 0), sizeof(int) * (size_t)N, hipMemcpyDeviceToHost));
-    if (n_small > 0) {
-        RSFK_HIP(hipMemcpy(ls.data(), tree_ws_leaf_start(ws.w, 0), sizeof(int) * (size_t)n_small, hipMemcpyDeviceToHost));
-        RSFK_HIP(hipMemcpy(lz.data(), tree_ws_leaf_size(ws.w, 0), sizeof(int) * (size_t)n_small, hipMemcpyDeviceToHost));
-    }
-    if (n_big > 0) {
-        RSFK_HIP(hipMemcpy(ls.data() + n_small, tree_ws_leaf_start(ws.w, 0) + (cap - n_big), sizeof(int) * (size_t)n_big, hipMemcpyDeviceToHost));
-        RSFK_HIP(hipMemcpy(lz.data() + n_small, tree_ws_leaf_size(ws.w, 0) + (cap - n_big), sizeof(int) * (size_t)n_big, hipMemcpyDeviceToHost));
-    }
+    const int* d_ls = tree_ws_leaf_start(ws.w, 0);
+    const int* d_lz = tree_ws_leaf_size(ws.w, 0);
+    auto part = [](const int* dev, int* host, int n) { return HostArray{const_cast<int*>(dev), host, sizeof(int) * (size_t)n}; };
+    const HostArray out[] = {part(tree_ws_perm(ws.w, 0), perm.data(), N),
+                             part(d_ls, ls.data(), n_small), part(d_lz, lz.data(), n_small),
+                             part(d_ls + (cap - n_big), ls.data() + n_small, n_big),
+                             part(d_lz + (cap - n_big), lz.data() + n_small, n_big)};
+    if (copy_to_host(out, 5, nullptr)) return 1;
     std::vector<int> order((size_t)nl);
     for (int i = 0; i < nl; ++i) order[i] = i;
     std::sort(order.begin(), order.end(), [&](int a, int b) { return ls[a] < ls[b]; });

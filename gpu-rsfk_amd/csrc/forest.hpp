@@ -101,9 +101,28 @@ int launch_bucket_knn_medium(const float* points, int D, int K, const int* ids, 
 int launch_bucket_knn_small(const float* points, int D, int K, const int* ids, const int* starts, const int* sizes,
                             int n_buckets, int stride, bool rows_sorted, int* knn_idx, float* knn_dist, hipStream_t stream);
 
-// host_copy.hip: pageable host memory <-> device memory through pinned buffers, on several threads
-int copy_to_device(void* dev_ptr, const void* host_ptr, size_t bytes);
-int copy_to_host(void* host_ptr, const void* dev_ptr, size_t bytes);
+// host_copy.hip: pageable host memory <-> device memory through pinned buffers, large arrays on several threads
+struct HostArray {
+    void* dev;
+    void* host;
+    size_t bytes;
+};
+// The arrays a call takes to the device.  Small ones are only queued on the stream; the pinned block they pass through
+// is held until the object goes (after the call has waited for the stream).
+class HostStage {
+public:
+    HostStage() = default;
+    HostStage(const HostStage&) = delete;
+    HostStage& operator=(const HostStage&) = delete;
+    ~HostStage();
+    int to_device(const HostArray* a, int n, hipStream_t stream);      // once per object for small arrays
+
+private:
+    void* block_ = nullptr;
+    hipStream_t stream_ = nullptr;
+};
+// Everything queued on the stream first, then the copies; complete on return.
+int copy_to_host(const HostArray* a, int n, hipStream_t stream);
 void release_copy_buffers();
 
 // explore_join.hip

@@ -304,27 +304,23 @@ int symmetrize_host(const int* idx, const float* dist, int N, int K, int drop_se
     RSFK_CHECK(N >= 1 && K >= 1, "graph export: N and K must be positive");
     RSFK_CHECK(idx && indptr && nnz, "graph export: null argument");
     RSFK_CHECK((cols == nullptr) == (vals == nullptr), "graph export: indices and data go together");
+    HostStage stage;
     Buf di, dd, dp, dc, dv;
     const size_t nk = (size_t)N * K;
     if (ws_alloc(&di.p, nk * sizeof(int)) || ws_alloc(&dp.p, ((size_t)N + 1) * sizeof(int))) return 1;
-    RSFK_HIP(hipMemcpy(di.p, idx, nk * sizeof(int), hipMemcpyHostToDevice));
-    if (dist) {
-        if (ws_alloc(&dd.p, nk * sizeof(float))) return 1;
-        RSFK_HIP(hipMemcpy(dd.p, dist, nk * sizeof(float), hipMemcpyHostToDevice));
-    }
+    if (dist && ws_alloc(&dd.p, nk * sizeof(float))) return 1;
     if (cols && cap > 0) {
         if (ws_alloc(&dc.p, (size_t)cap * sizeof(int)) || ws_alloc(&dv.p, (size_t)cap * sizeof(float))) return 1;
     }
+    const HostArray in[] = {{di.p, const_cast<int*>(idx), nk * sizeof(int)}, {dd.p, const_cast<float*>(dist), nk * sizeof(float)}};
+    if (stage.to_device(in, dist ? 2 : 1, nullptr)) return 1;
     const int rc = symmetrize_device(static_cast<const int*>(di.p), static_cast<const float*>(dd.p), N, K, drop_self,
                                      static_cast<int*>(dp.p), static_cast<int*>(dc.p), static_cast<float*>(dv.p), cap, nnz,
                                      nullptr);
     if (rc) return rc;
-    RSFK_HIP(hipMemcpy(indptr, dp.p, ((size_t)N + 1) * sizeof(int), hipMemcpyDeviceToHost));
-    if (dc.p && *nnz > 0) {
-        RSFK_HIP(hipMemcpy(cols, dc.p, (size_t)*nnz * sizeof(int), hipMemcpyDeviceToHost));
-        RSFK_HIP(hipMemcpy(vals, dv.p, (size_t)*nnz * sizeof(float), hipMemcpyDeviceToHost));
-    }
-    return 0;
+    const HostArray out[] = {{dp.p, indptr, ((size_t)N + 1) * sizeof(int)}, {dc.p, cols, (size_t)*nnz * sizeof(int)},
+                             {dv.p, vals, (size_t)*nnz * sizeof(float)}};
+    return copy_to_host(out, dc.p ? 3 : 1, nullptr);
 }
 
 }  // namespace rsfk

@@ -1,11 +1,16 @@
 // Copies between pageable host arrays (what a ctypes caller hands over: numpy buffers) and device memory.
 //
-// hipMemcpy on pageable memory moves the bytes through a bounce buffer on one thread; at N = 1M, D = 100, K = 32 the
-// 656 MB of a call took 38 ms that way, more than half the time of the build itself.  Here a few host threads each
-// take a contiguous slice of the array and move it in pieces through their own pair of pinned buffers
-// (hipHostMalloc; registering the caller's memory is not an option) on their own stream: the memcpy into / out of
-// the pinned buffer of one piece overlaps the DMA of the previous one, and the threads overlap each other.
-// The pinned buffers are kept for the next call; rsfk_release_workspace() frees them.
+// hipMemcpy on pageable memory moves the bytes through a bounce buffer on one thread, and its time has little to do
+// with the size of a small array (320 KB to the device: 133 us, 14 us from pinned memory).  So:
+//   small arrays (all arrays of a call together below 4 MB) go through one pinned block on the calling thread, in
+//     pieces, the memcpy of a piece beside the DMA of the piece before; copies to the device are only queued on the
+//     caller's stream (2.4 MB: 101 us with hipMemcpy, 56 us here).
+//   large ones: host threads take pieces of 2 MB in turn, each through its own pair of pinned buffers (hipHostMalloc;
+//     registering the caller's memory is not an option) on its own stream: the memcpy of one piece overlaps the DMA of
+//     the previous one and the threads overlap each other.  What bounds it is the link (57 GB/s each way); one thread
+//     copies 10 GB/s or so, less where the destination's pages are touched for the first time, hence eight threads
+//     (16 cores on the box).  Four threads with pieces of 8 MB, the form before, had nothing to overlap below 64 MB.
+// The buffers and streams are kept for the next call; rsfk_release_workspace() frees them.
 #include "rsfk_common.hpp"
 #include "forest.hpp"
 #include <algorithm>
@@ -19,9 +24,10 @@ namespace rsfk {
 
 namespace {
 
-constexpr int kCopyThreads = 4;
-constexpr size_t kPiece = (size_t)8 << 20;          // bytes per pinned buffer
-constexpr size_t kSmall = (size_t)4 << 20;          // below this a plain hipMemcpy is used
+constexpr int kCopyThreads = 8;
+constexpr size_t kPiece = (size_t)2 << 20;          // bytes per pinned buffer of a thread
+constexpr size_t kSmall = (size_t)4 << 20;          // up to here on the calling thread
+constexpr size_t kSmallPiece = (size_t)512 << 10;
 
 struct Lane {
     void* pinned[2] = {nullptr, nullptr};
@@ -74,77 +80,124 @@ int make_lanes_locked(Lanes& L, int dev)
     return 0;
 }
 
-// one thread's slice: [begin, end) of the array, to_device or back
-void run_slice(Lane& a, int dev, char* dev_ptr, char* host_ptr, size_t begin, size_t end, bool to_device, std::atomic<int>& err)
+struct Piece {
+    char* dev;
+    char* host;
+    size_t bytes;
+};
+
+// one thread: pieces in turn until none is left
+void run_lane(Lane& a, int dev, const std::vector<Piece>& pieces, std::atomic<size_t>& next, bool to_device, std::atomic<int>& err)
 {
     if (hipSetDevice(dev) != hipSuccess) { err = 1; return; }
-    size_t off[2] = {0, 0}, len[2] = {0, 0};
+    Piece in[2] = {};
     int n = 0;
-    for (size_t at = begin; at < end && !err; at += kPiece, ++n) {
-        const int b = n & 1;
-        const size_t bytes = std::min(kPiece, end - at);
-        if (n >= 2) {
-            // the piece that used this buffer two steps ago
-            if (hipEventSynchronize(a.done[b]) != hipSuccess) { err = 1; return; }
-            if (!to_device) std::memcpy(host_ptr + off[b], a.pinned[b], len[b]);
-        }
-        off[b] = at;
-        len[b] = bytes;
-        if (to_device) {
-            std::memcpy(a.pinned[b], host_ptr + at, bytes);
-            if (hipMemcpyAsync(dev_ptr + at, a.pinned[b], bytes, hipMemcpyHostToDevice, a.stream) != hipSuccess) { err = 1; return; }
-        } else {
-            if (hipMemcpyAsync(a.pinned[b], dev_ptr + at, bytes, hipMemcpyDeviceToHost, a.stream) != hipSuccess) { err = 1; return; }
-        }
-        if (hipEventRecord(a.done[b], a.stream) != hipSuccess) { err = 1; return; }
-    }
-    // drain: the last (up to) two pieces
-    for (int k = std::max(0, n - 2); k < n && !err; ++k) {
-        const int b = k & 1;
+    auto finish = [&](int b) {
         if (hipEventSynchronize(a.done[b]) != hipSuccess) { err = 1; return; }
-        if (!to_device) std::memcpy(host_ptr + off[b], a.pinned[b], len[b]);
+        if (!to_device) std::memcpy(in[b].host, a.pinned[b], in[b].bytes);
+    };
+    for (; !err; ++n) {
+        const size_t i = next.fetch_add(1);
+        if (i >= pieces.size()) break;
+        const int b = n & 1;
+        if (n >= 2) finish(b);                       // the piece that used this buffer two steps ago
+        if (err) break;
+        in[b] = pieces[i];
+        if (to_device) std::memcpy(a.pinned[b], in[b].host, in[b].bytes);
+        const hipError_t e = to_device ? hipMemcpyAsync(in[b].dev, a.pinned[b], in[b].bytes, hipMemcpyHostToDevice, a.stream)
+                                       : hipMemcpyAsync(a.pinned[b], in[b].dev, in[b].bytes, hipMemcpyDeviceToHost, a.stream);
+        if (e != hipSuccess || hipEventRecord(a.done[b], a.stream) != hipSuccess) { err = 1; return; }
     }
+    for (int k = std::max(0, n - 2); k < n && !err; ++k) finish(k & 1);
 }
 
-int staged_copy(void* dev_ptr, void* host_ptr, size_t bytes, bool to_device)
+int large_copy(const std::vector<Piece>& pieces, bool to_device)
 {
-    if (bytes == 0) return 0;
-    if (bytes < kSmall) {
-        if (to_device) RSFK_HIP(hipMemcpy(dev_ptr, host_ptr, bytes, hipMemcpyHostToDevice));
-        else RSFK_HIP(hipMemcpy(host_ptr, dev_ptr, bytes, hipMemcpyDeviceToHost));
-        return 0;
-    }
     int dev = 0;
     RSFK_HIP(hipGetDevice(&dev));
     Lanes& L = lanes();
-    std::lock_guard<std::mutex> lock(L.mu);            // one staged copy at a time
+    std::lock_guard<std::mutex> lock(L.mu);            // one such copy at a time
     if (make_lanes_locked(L, dev)) return 1;
-    // what the device was asked to do before must be done when the copies on the other streams touch the memory
-    RSFK_HIP(hipDeviceSynchronize());
     std::atomic<int> err{0};
-    const size_t per = ((bytes + kCopyThreads - 1) / kCopyThreads + 255) & ~(size_t)255;
+    std::atomic<size_t> next{0};
+    const int n_threads = (int)std::min<size_t>(kCopyThreads, pieces.size());
     std::vector<std::thread> th;
-    for (int t = 0; t < kCopyThreads; ++t) {
-        const size_t b = std::min(bytes, per * t), e = std::min(bytes, per * (t + 1));
-        if (b >= e) break;
-        th.emplace_back(run_slice, std::ref(L.lane[t]), dev, static_cast<char*>(dev_ptr), static_cast<char*>(host_ptr), b, e,
-                        to_device, std::ref(err));
-    }
+    for (int t = 1; t < n_threads; ++t)
+        th.emplace_back(run_lane, std::ref(L.lane[t]), dev, std::cref(pieces), std::ref(next), to_device, std::ref(err));
+    run_lane(L.lane[0], dev, pieces, next, to_device, err);
     for (auto& t : th) t.join();
     RSFK_CHECK(err == 0, "copy between host and device failed");
     return 0;
 }
 
-}  // namespace
-
-int copy_to_device(void* dev_ptr, const void* host_ptr, size_t bytes)
+std::vector<Piece> cut(const HostArray* a, int n, size_t piece)
 {
-    return staged_copy(dev_ptr, const_cast<void*>(host_ptr), bytes, true);
+    std::vector<Piece> out;
+    for (int i = 0; i < n; ++i)
+        for (size_t at = 0; at < a[i].bytes; at += piece)
+            out.push_back({static_cast<char*>(a[i].dev) + at, static_cast<char*>(a[i].host) + at, std::min(piece, a[i].bytes - at)});
+    return out;
 }
 
-int copy_to_host(void* host_ptr, const void* dev_ptr, size_t bytes)
+size_t total_bytes(const HostArray* a, int n)
 {
-    return staged_copy(const_cast<void*>(dev_ptr), host_ptr, bytes, false);
+    size_t t = 0;
+    for (int i = 0; i < n; ++i) t += a[i].bytes;
+    return t;
+}
+
+}  // namespace
+
+HostStage::~HostStage()
+{
+    if (block_) {
+        (void)hipStreamSynchronize(stream_);           // (only on an error path is anything still queued)
+        pin_free(block_);
+    }
+}
+
+int HostStage::to_device(const HostArray* a, int n, hipStream_t stream)
+{
+    const size_t total = total_bytes(a, n);
+    if (total == 0) return 0;
+    if (total > kSmall || block_) return large_copy(cut(a, n, kPiece), true);
+    if (pin_alloc(&block_, total)) return 1;
+    stream_ = stream;
+    char* at = static_cast<char*>(block_);
+    for (const Piece& p : cut(a, n, kSmallPiece)) {
+        std::memcpy(at, p.host, p.bytes);
+        RSFK_HIP(hipMemcpyAsync(p.dev, at, p.bytes, hipMemcpyHostToDevice, stream));
+        at += p.bytes;
+    }
+    return 0;
+}
+
+int copy_to_host(const HostArray* a, int n, hipStream_t stream)
+{
+    const size_t total = total_bytes(a, n);
+    if (total == 0) return 0;
+    if (total > kSmall) {
+        RSFK_HIP(hipStreamSynchronize(stream));        // the copies run on streams of their own
+        return large_copy(cut(a, n, kPiece), false);
+    }
+    struct Guard {
+        void* p = nullptr;
+        ~Guard() { pin_free(p); }
+    } block;
+    if (pin_alloc(&block.p, total)) return 1;
+    const std::vector<Piece> pieces = cut(a, n, 2 * kSmallPiece);
+    char* at = static_cast<char*>(block.p);
+    for (const Piece& p : pieces) {
+        RSFK_HIP(hipMemcpyAsync(at, p.dev, p.bytes, hipMemcpyDeviceToHost, stream));
+        at += p.bytes;
+    }
+    RSFK_HIP(hipStreamSynchronize(stream));
+    at = static_cast<char*>(block.p);
+    for (const Piece& p : pieces) {
+        std::memcpy(p.host, at, p.bytes);
+        at += p.bytes;
+    }
+    return 0;
 }
 
 void release_copy_buffers()

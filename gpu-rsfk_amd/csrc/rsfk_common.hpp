@@ -20,6 +20,12 @@ int ws_alloc(void** out, size_t bytes);
 int ws_try_alloc(void** out, size_t bytes);      // optional block: fails quietly, releases nothing
 void ws_free(void* p);
 void ws_release_all();
+// pinned host memory and non-blocking streams, kept for the next call in the same way
+int pin_alloc(void** out, size_t bytes);
+void pin_free(void* p);
+int stream_take(hipStream_t* out);
+void stream_give(hipStream_t s);
+void host_pool_release();
 
 // Both macros leave the function on failure.  Work that was queued before may still be running and the
 // callers' guards hand their buffers back for reuse on the way out, so the device is drained first.

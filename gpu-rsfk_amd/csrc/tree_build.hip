@@ -1044,9 +1044,9 @@ static void free_ws(TreeBatchWorkspace& w)
                    w.chunk_left, w.leaf_start, w.leaf_size, w.stats, w.ctr, w.recs, w.n_rec, w.planes,
                    w.pm_path, w.pm_side, w.pm_undec, w.pm_map[0], w.pm_map[1], w.pm_sc, w.pm_aq, w.pm_child, w.stat};
     for (void* p : dev) ws_free(p);
-    if (w.h_ctr) (void)hipHostFree(w.h_ctr);
-    if (w.h_stat) (void)hipHostFree(w.h_stat);
-    if (w.h_stats) (void)hipHostFree(w.h_stats);
+    pin_free(w.h_ctr);
+    pin_free(w.h_stat);
+    pin_free(w.h_stats);
     for (hipEvent_t e : w.ev)
         if (e) (void)hipEventDestroy(e);
     w = TreeBatchWorkspace();
@@ -1139,9 +1139,9 @@ int tree_ws_alloc(TreeBatchWorkspace** out, int N, int D, int MIN, int B)
         if (dmalloc(&w->pm_aq, (size_t)B * pm::kMaxGroups * 32 * 32 * w->pm_ks)) return 1;
         if (dmalloc(&w->pm_child, (size_t)w->node_cap)) return 1;
     }
-    RSFK_HIP(hipHostMalloc(reinterpret_cast<void**>(&w->h_ctr), sizeof(LevelCounters)));
-    RSFK_HIP(hipHostMalloc(reinterpret_cast<void**>(&w->h_stats), sizeof(TreeStats) * (size_t)B));
-    RSFK_HIP(hipHostMalloc(reinterpret_cast<void**>(&w->h_stat), sizeof(unsigned long long) * kStatSlots * kStatPitch));
+    if (pin_alloc(reinterpret_cast<void**>(&w->h_ctr), sizeof(LevelCounters))) return 1;
+    if (pin_alloc(reinterpret_cast<void**>(&w->h_stats), sizeof(TreeStats) * (size_t)B)) return 1;
+    if (pin_alloc(reinterpret_cast<void**>(&w->h_stat), sizeof(unsigned long long) * kStatSlots * kStatPitch)) return 1;
     for (hipEvent_t& e : w->ev) RSFK_HIP(hipEventCreate(&e));
     return 0;
 }
