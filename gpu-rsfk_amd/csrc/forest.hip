@@ -154,6 +154,7 @@ int build_report_json(char* buf, int cap)
         {kBucketKernelMedium, "k_bucket_knn_small<72>"}, {kBucketKernelRows, "k_bucket_knn_rows"},
         {kBucketKernelTiled, "k_bucket_knn<per bucket>"}, {kBucketKernelStrip, "k_bucket_knn<per 64 members>"},
         {kBucketKernelGram, "k_bucket_knn_gram"}, {kBucketKernelAuto, "k_bucket_knn_auto"},
+        {kBucketKernelForest, "k_forest_pairs + k_forest_merge"},
         {kBucketKernelPairs, "k_bucket_pairs + k_bucket_merge_pairs"}};
     std::string s = "{";
     auto num = [&](const char* key, double v, bool last = false) {
@@ -244,9 +245,8 @@ int knn_forest_device(int n_trees, int K, int N, int D, int MIN, int MAX, int MA
 
     rep.row_bytes = tree_screen_row_bytes(D, q8_rows != nullptr);
     if (n_trees > 0) {
-        // the bucket kernels read a row's maximum from its last slot: rows the caller passed in unsorted are put
-        // in order once
-        if (launch_sort_rows(d_idx, d_dist, N, K, stream)) return 1;
+        const bool all_at_once = bucket_forest_wanted(n_trees);
+        bool rows_in_order = false;
         const int B = choose_batch(n_trees, N, D, MIN);
         WsGuard ws;
         if (tree_ws_alloc(&ws.w, N, D, MIN, B)) return 1;
@@ -285,6 +285,9 @@ int knn_forest_device(int n_trees, int K, int N, int D, int MIN, int MAX, int MA
             }
             return 0;
         };
+        // ... and of the form that takes the buckets of several trees at once
+        DevBuf forest_dist, forest_info;
+        size_t forest_floats = 0;
         int rc = 0;
         for (int t0 = 0; t0 < n_trees && rc == 0; t0 += B) {
             const int nb = std::min(B, n_trees - t0);
@@ -295,11 +298,46 @@ int knn_forest_device(int n_trees, int K, int N, int D, int MIN, int MAX, int MA
             rep.tree_s += tb;
             rep.tested += tree_ws_counts(ws.w)[0];
             rep.undecided += tree_ws_counts(ws.w)[1];
+            int group = 0;                               // trees whose buckets go together, 0: one tree after the other
+            int max_bucket = 0;
+            if (all_at_once) {
+                for (int j = 0; j < nb; ++j) max_bucket = std::max(max_bucket, stats[5 * j + 2]);
+                group = bucket_forest_group(N, K, max_bucket, nb);
+                const size_t want = group > 0 ? bucket_forest_floats(N, max_bucket, group) : 0;
+                if (want > forest_floats) {
+                    if (forest_dist.p) {
+                        RSFK_HIP(hipStreamSynchronize(stream));
+                        ws_free(forest_dist.p);
+                        forest_dist.p = nullptr;
+                    }
+                    forest_floats = ws_try_alloc(&forest_dist.p, want * sizeof(float)) == 0 ? want : 0;
+                }
+                if (group > 0 && !forest_info.p && ws_try_alloc(&forest_info.p, (size_t)N * (size_t)B * 2 * sizeof(int))) forest_info.p = nullptr;
+                if (want > forest_floats || !forest_info.p) group = 0;
+            }
+            if (group > 0) {
+                (void)hipEventRecord(ev[0].e, stream);
+                for (int j = 0; j < nb && rc == 0; j += group) {
+                    const int T = std::min(group, nb - j);
+                    rc = launch_bucket_knn_forest(d_points, N, D, K, T, tree_ws_perm(ws.w, j), tree_ws_leaf_start(ws.w, j),
+                                                  tree_ws_leaf_size(ws.w, j), tree_ws_leaf_cap(ws.w), tree_ws_stats(ws.w, j),
+                                                  stats.data() + 5 * j, max_bucket, static_cast<float*>(forest_dist.p),
+                                                  static_cast<int*>(forest_info.p), d_idx, d_dist, stream);
+                    for (int u = 0; u < T; ++u) rep.kernels[(size_t)(t0 + j + u)] = kBucketKernelForest;
+                }
+                if (rc) break;
+                rows_in_order = true;
+            } else if (!rows_in_order) {
+                // the bucket kernels read a row's maximum from its last slot: rows the caller passed in unsorted are
+                // put in order once
+                if (launch_sort_rows(d_idx, d_dist, N, K, stream)) return 1;
+                rows_in_order = true;
+            }
             // The larger buckets of a tree (a few per cent of the points at the default sizes: a grid too small to fill
             // the device) run on a second stream beside the small ones: different buckets of one tree touch different
             // rows.  Both parts of tree j wait for both parts of tree j - 1.
             bool big_pending = false;                    // sync.big holds the larger buckets of the previous tree
-            for (int j = 0; j < nb && rc == 0; ++j) {
+            for (int j = 0; j < nb && group == 0 && rc == 0; ++j) {
                 const int n_big = stats[5 * j + 4], n_small = stats[5 * j] - n_big;
                 const bool split = sync.side != nullptr && n_big > 0 && n_small > 0;
                 if (big_pending) (void)hipStreamWaitEvent(stream, sync.big, 0);
@@ -333,7 +371,12 @@ int knn_forest_device(int n_trees, int K, int N, int D, int MIN, int MAX, int MA
             RSFK_HIP(hipStreamSynchronize(stream));
             for (int j = 0; j < nb; ++j) {
                 float ms = 0.0f;
-                (void)hipEventElapsedTime(&ms, ev[j].e, ev[j + 1].e);
+                if (group > 0) {
+                    (void)hipEventElapsedTime(&ms, ev[0].e, ev[nb].e);
+                    ms /= (float)nb;                         // a tree's share
+                } else {
+                    (void)hipEventElapsedTime(&ms, ev[j].e, ev[j + 1].e);
+                }
                 rep.bucket_s += ms * 1e-3;
                 const int t = t0 + j;
                 if (log_forest) {

@@ -18,6 +18,7 @@ int tree_ws_leaf_cap(const TreeBatchWorkspace* w);
 const int* tree_ws_perm(const TreeBatchWorkspace* w, int t);
 const int* tree_ws_leaf_start(const TreeBatchWorkspace* w, int t);
 const int* tree_ws_leaf_size(const TreeBatchWorkspace* w, int t);
+const int* tree_ws_stats(const TreeBatchWorkspace* w, int t);      // five ints: buckets of at most kBucketSplit points, larger ones, ...
 int tree_small_threshold(int D, int N, int B);
 const float* tree_ws_phase_seconds(const TreeBatchWorkspace* w);
 const unsigned long long* tree_ws_counts(const TreeBatchWorkspace* w);
@@ -48,6 +49,7 @@ enum : int {
     kBucketKernelTiled = 16,     // k_bucket_knn<SL, false>: 64 x 64 tiles, a workgroup per bucket
     kBucketKernelStrip = 32,     // k_bucket_knn<SL, true>: 64 x 64 tiles, a workgroup per 64 members of a bucket
     kBucketKernelGram = 64,      // k_bucket_knn_gram: any bucket size, pair matrix bounded on the matrix cores
+    kBucketKernelForest = 512,   // k_forest_pairs + k_forest_merge: the buckets of several trees at once
     kBucketKernelPairs = 256,    // k_bucket_pairs + k_bucket_merge_pairs: 64 x 64 tiles, every pair once, distances through memory
 };
 // Working memory of k_bucket_pairs / k_bucket_merge_pairs: the pair matrices of as many buckets as fit are in it at a
@@ -66,6 +68,14 @@ int launch_bucket_knn_tree(const float* points, const unsigned long long* prev_s
                            int leaf_cap, int n_small, int n_big, int max_bucket, int* knn_idx, float* knn_dist,
                            hipStream_t stream, int part = 0, bool young_rows = true, int* launched = nullptr,
                            const PairScratch* pairs = nullptr);
+
+// bucket_knn_forest.hip: the buckets of several trees at once (small inputs)
+bool bucket_forest_wanted(int n_trees);
+int bucket_forest_group(int N, int K, int max_bucket, int n_trees);
+size_t bucket_forest_floats(int N, int max_bucket, int n_trees);
+int launch_bucket_knn_forest(const float* points, int N, int D, int K, int T, const int* perm, const int* leaf_start, const int* leaf_size,
+                             int leaf_cap, const int* stats, const int* host_stats, int max_bucket, float* pair_dist, int* info,
+                             int* knn_idx, float* knn_dist, hipStream_t stream);
 
 // What the last K-NN-graph build of this process did, as a line of JSON (rsfk_last_build_report): which bucket
 // kernels every tree went to, the counts the algorithmic bytes of the tree build and of the exploration are made of,

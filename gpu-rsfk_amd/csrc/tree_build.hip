@@ -1064,6 +1064,12 @@ const int* tree_ws_perm(const TreeBatchWorkspace* w, int t) { return w->perm[0] 
 const int* tree_ws_leaf_start(const TreeBatchWorkspace* w, int t) { return w->leaf_start + (size_t)t * w->leaf_cap; }
 const int* tree_ws_leaf_size(const TreeBatchWorkspace* w, int t) { return w->leaf_size + (size_t)t * w->leaf_cap; }
 
+const int* tree_ws_stats(const TreeBatchWorkspace* w, int t)
+{
+    static_assert(sizeof(TreeStats) == 5 * sizeof(int), "read as five ints");
+    return reinterpret_cast<const int*>(w->stats + t);
+}
+
 // Nodes of at most this many points are finished by one workgroup (k_tail): 1024, or 2048 for short rows, where a
 // wide level costs more per byte of row it reads (the permutation entries it moves weigh more) -- measured on 10M x 32
 // points 4.46 against 4.81 ms per tree, on 1M x 100 points 0.548 against 0.520 -- and for batches so small (N x B below

@@ -1004,3 +1004,32 @@ def test_rows_of_many_neighbours_on_tied_data(gpu, orc, N, D, K, nnef):
     ip, cc, vv = gpu_rsfk.symmetric_knn_graph(gi, gd, drop_self=True)
     op, oc, ov = orc.symmetrize(gi, gd, drop_self=True)
     assert np.array_equal(ip, op) and np.array_equal(cc, oc) and np.array_equal(vv, ov)
+
+
+# Buckets of several trees at once (k_forest_pairs + k_forest_merge): one, two and four candidates per lane, rows of one
+# and two slots per lane, new rows with and without the point itself, buckets just above a tile, K at the rank limits,
+# duplicated points (equal distances leave the ranking to the insertions), more trees than are in flight.
+@pytest.mark.parametrize("N,D,K,T,mn,mx,nnef,self_in,dup", [
+    (700, 5, 4, 4, 5, 12, 0, True, False),
+    (3001, 33, 31, 11, 32, 66, 1, True, False),
+    (2500, 20, 64, 5, 65, 130, 0, False, False),
+    (4000, 8, 40, 6, 70, 250, 0, True, False),
+    (2000, 12, 100, 7, 101, 256, 0, True, False),
+    (1500, 7, 200, 4, 60, 140, 0, True, False),
+    (2600, 3, 16, 8, 17, 40, 2, True, True),
+    (1800, 4, 20, 5, 80, 200, 0, False, True),
+])
+def test_buckets_of_several_trees_at_once_match_oracle(gpu, orc, rng, monkeypatch, N, D, K, T, mn, mx, nnef, self_in, dup):
+    import gpu_rsfk
+    monkeypatch.setenv("RSFK_FOREST_MERGE", "1")
+    X = rng.standard_normal((N, D)).astype(np.float32)
+    if dup:
+        X[N // 2:] = X[:N - N // 2]
+    _say("several trees at once", N, D, K, T, mn, mx)
+    gi, gd = gpu_rsfk.RSFK(random_state=3).find_nearest_neighbors(
+        X, K, n_trees=T, min_tree_children=mn, max_tree_children=mx, nn_exploring_factor=nnef, point_in_self_neigh=self_in,
+        ensure_valid_indices=False)
+    assert gpu.last_build_report()["bucket_kernels"] == [[0, T - 1, ["k_forest_pairs + k_forest_merge"]]]
+    oi, od = orc.init_lists(N, K, self_in=self_in)
+    orc.forest(X, K, T, mn, mx, 5000, 3, nnef, knn_idx=oi, knn_dist=od)
+    assert_knn_equal(gi, gd, oi, od)
