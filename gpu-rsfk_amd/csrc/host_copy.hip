@@ -25,13 +25,13 @@ namespace rsfk {
 namespace {
 
 constexpr int kCopyThreads = 8;
+constexpr int kCopyStreams = 2;
 constexpr size_t kPiece = (size_t)2 << 20;          // bytes per pinned buffer of a thread
 constexpr size_t kSmall = (size_t)4 << 20;          // up to here on the calling thread
 constexpr size_t kSmallPiece = (size_t)512 << 10;
 
 struct Lane {
     void* pinned[2] = {nullptr, nullptr};
-    hipStream_t stream = nullptr;
     hipEvent_t done[2] = {nullptr, nullptr};
 };
 
@@ -39,6 +39,7 @@ struct Lanes {
     std::mutex mu;
     int device = -1;
     Lane lane[kCopyThreads];
+    hipStream_t stream[kCopyStreams] = {};
     bool ready = false;
 };
 
@@ -57,8 +58,10 @@ void free_lanes_locked(Lanes& L)
             a.pinned[i] = nullptr;
             a.done[i] = nullptr;
         }
-        if (a.stream) (void)hipStreamDestroy(a.stream);
-        a.stream = nullptr;
+    }
+    for (hipStream_t& s : L.stream) {
+        if (s) (void)hipStreamDestroy(s);
+        s = nullptr;
     }
     L.ready = false;
     L.device = -1;
@@ -69,12 +72,12 @@ int make_lanes_locked(Lanes& L, int dev)
     if (L.ready && L.device == dev) return 0;
     free_lanes_locked(L);
     for (Lane& a : L.lane) {
-        RSFK_HIP(hipStreamCreateWithFlags(&a.stream, hipStreamNonBlocking));
         for (int i = 0; i < 2; ++i) {
             RSFK_HIP(hipHostMalloc(&a.pinned[i], kPiece));
             RSFK_HIP(hipEventCreateWithFlags(&a.done[i], hipEventDisableTiming));
         }
     }
+    for (hipStream_t& s : L.stream) RSFK_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
     L.device = dev;
     L.ready = true;
     return 0;
@@ -87,7 +90,7 @@ struct Piece {
 };
 
 // one thread: pieces in turn until none is left
-void run_lane(Lane& a, int dev, const std::vector<Piece>& pieces, std::atomic<size_t>& next, bool to_device, std::atomic<int>& err)
+void run_lane(Lane& a, hipStream_t stream, int dev, const std::vector<Piece>& pieces, std::atomic<size_t>& next, bool to_device, std::atomic<int>& err)
 {
     if (hipSetDevice(dev) != hipSuccess) { err = 1; return; }
     Piece in[2] = {};
@@ -104,9 +107,9 @@ void run_lane(Lane& a, int dev, const std::vector<Piece>& pieces, std::atomic<si
         if (err) break;
         in[b] = pieces[i];
         if (to_device) std::memcpy(a.pinned[b], in[b].host, in[b].bytes);
-        const hipError_t e = to_device ? hipMemcpyAsync(in[b].dev, a.pinned[b], in[b].bytes, hipMemcpyHostToDevice, a.stream)
-                                       : hipMemcpyAsync(a.pinned[b], in[b].dev, in[b].bytes, hipMemcpyDeviceToHost, a.stream);
-        if (e != hipSuccess || hipEventRecord(a.done[b], a.stream) != hipSuccess) { err = 1; return; }
+        const hipError_t e = to_device ? hipMemcpyAsync(in[b].dev, a.pinned[b], in[b].bytes, hipMemcpyHostToDevice, stream)
+                                       : hipMemcpyAsync(a.pinned[b], in[b].dev, in[b].bytes, hipMemcpyDeviceToHost, stream);
+        if (e != hipSuccess || hipEventRecord(a.done[b], stream) != hipSuccess) { err = 1; return; }
     }
     for (int k = std::max(0, n - 2); k < n && !err; ++k) finish(k & 1);
 }
@@ -123,8 +126,8 @@ int large_copy(const std::vector<Piece>& pieces, bool to_device)
     const int n_threads = (int)std::min<size_t>(kCopyThreads, pieces.size());
     std::vector<std::thread> th;
     for (int t = 1; t < n_threads; ++t)
-        th.emplace_back(run_lane, std::ref(L.lane[t]), dev, std::cref(pieces), std::ref(next), to_device, std::ref(err));
-    run_lane(L.lane[0], dev, pieces, next, to_device, err);
+        th.emplace_back(run_lane, std::ref(L.lane[t]), L.stream[t % kCopyStreams], dev, std::cref(pieces), std::ref(next), to_device, std::ref(err));
+    run_lane(L.lane[0], L.stream[0], dev, pieces, next, to_device, err);
     for (auto& t : th) t.join();
     RSFK_CHECK(err == 0, "copy between host and device failed");
     return 0;
