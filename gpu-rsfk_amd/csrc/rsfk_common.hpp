@@ -147,6 +147,8 @@ struct TreeParams {
     int N, D;
     int MIN, MAX, MAX_DEPTH;
     int small;        // nodes with at most this many points are finished by one workgroup
+    int vain;         // a node split in vain this many times in a row ...
+    int chain_max;    // ... and of at most this many points goes to the chain phase (0: never)
     int chunk;        // points per workgroup in the wide (global) passes
     float band;       // half-width of the undecided band of the bfloat16 side screen, relative to sum |n_d||x~_d|
 };

@@ -24,12 +24,16 @@
 //                most `small` points inside LDS (all the re-draw levels that
 //                the min/max rule causes touch only such nodes).
 //
+//   chain phase : nodes the tail kernel has split in vain several times in a row
+//                are finished from the distances of their points (k_chain).
+//
 // Arithmetic follows the reference bit for bit: the hyperplane offset and the
 // side test are sums of 32 lane-strided partials combined by the xor butterfly
 // (create_node.cu:122-135, build_tree_check_points_side.cu:131-149); a half
 // wavefront plays the role of the 32-lane warp.
 #include "rsfk_common.hpp"
 #include "wave64.hpp"
+#include "knn_list.hpp"
 #include "bf16.hpp"
 #include "tree_sweep.hpp"
 #include <vector>
@@ -48,6 +52,7 @@ constexpr int kBlock = 256;
 struct LevelCounters {
     int n_next;        // nodes appended for the next wide level
     int n_tail;        // tail tasks appended so far
+    int n_chain;       // nodes for the chain phase appended so far
     int n_chunks;      // chunks of the current level (written by the scan kernel)
     int overflow;      // set when a queue capacity is exceeded
     // time spent in the three steps of the wide levels (hyperplanes, side tests, scatter), in ticks of the device's
@@ -261,12 +266,12 @@ __device__ __forceinline__ void side_screen8(const float* nvec0, int nstride, co
 // point (local to the caller) | slot of its node << 16.  One half wavefront per point, two points per half
 // wavefront at a time so that their row loads overlap; all threads of the workgroup call.  id_at(pos) gives the
 // point, apply(pos, right) receives the answer in lane 0 of the half wavefront.
+// (h of `halves`: which half wavefront of those that work on the list this is)
 template <typename IdAt, typename Apply>
-__device__ __forceinline__ void resolve_exact(const int* list, int n, const float* nvec0, int nstride, const float* b_of,
+__device__ __forceinline__ void resolve_exact(int halves, int h, const int* list, int n, const float* nvec0, int nstride, const float* b_of,
                                               const float* __restrict__ points, int D, IdAt id_at, Apply apply)
 {
-    const int halves = blockDim.x >> 5;
-    const int h = threadIdx.x >> 5, hl = threadIdx.x & 31;
+    const int hl = threadIdx.x & 31;
     for (int base = 0; base < n; base += 2 * halves) {
         const int ia = base + h, ib = base + halves + h;
         const bool va = ia < n, vb = ib < n;
@@ -303,22 +308,29 @@ __device__ __forceinline__ void resolve_exact(const int* list, int n, const floa
 constexpr int kSideBatch = 4;        // points per group and call of the screen in the wide phase
 constexpr int kTailBatch = 2;        // ... in the tail kernel
 
-// Append a child node either to the next wide level or to the tail queue.  Returns its place in the queue of the next
-// wide level, or -1.
-__device__ __forceinline__ int emit_node(const TreeNode& c, const TreeParams& P, TreeNode* next, int next_cap,
-                                         TreeNode* tail, int tail_cap, LevelCounters* ctr)
+// The queues nodes go to: the next wide level and the tail kernel (one workgroup per node).
+struct NodeQueues {
+    TreeNode* next;
+    int next_cap;
+    TreeNode* tail;
+    int tail_cap;
+    LevelCounters* ctr;
+};
+
+// Append a child node to its queue.  Returns its place in the queue of the next wide level, or -1.
+__device__ __forceinline__ int emit_node(const TreeNode& c, const TreeParams& P, const NodeQueues& Q)
 {
     const bool forced = c.depth >= P.MAX_DEPTH - 1;
     if (!c.leaf && !forced && c.count > P.small) {
-        const int at = atomicAdd(&ctr->n_next, 1);
-        if (at < next_cap) { next[at] = c; return at; }
-        ctr->overflow = 1;
+        const int at = atomicAdd(&Q.ctr->n_next, 1);
+        if (at < Q.next_cap) { Q.next[at] = c; return at; }
+        Q.ctr->overflow = 1;
         return -1;
     }
     TreeNode t = c;
     if (forced) t.leaf = 1;
-    const int at = atomicAdd(&ctr->n_tail, 1);
-    if (at < tail_cap) tail[at] = t; else ctr->overflow = 1;
+    const int at = atomicAdd(&Q.ctr->n_tail, 1);
+    if (at < Q.tail_cap) Q.tail[at] = t; else Q.ctr->overflow = 1;
     return -1;
 }
 
@@ -400,8 +412,7 @@ __global__ void k_init_perm(int* __restrict__ perm, int N, int B)
         perm[i] = (int)(i % (size_t)N);
 }
 
-__global__ void k_init_roots(TreeNode* nodes, TreeNode* tail, LevelCounters* ctr, TreeParams P, int B, int seed0,
-                             int* n_rec, int* pmap)
+__global__ void k_init_roots(NodeQueues Q, TreeParams P, int B, int seed0, int* n_rec, int* pmap)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= B) return;
@@ -411,7 +422,7 @@ __global__ void k_init_roots(TreeNode* nodes, TreeNode* tail, LevelCounters* ctr
     r.rec = 0; r.pad_ = 0;
     r.key = root_key(seed0 + t);
     // the root is never a leaf (src/kernels/build_tree_init.cu:79) unless the depth limit forces it
-    const int at = emit_node(r, P, nodes, B, tail, B, ctr);
+    const int at = emit_node(r, P, Q);
     if (pmap) pmap[t * pm::kPaths] = at;      // path 0 of level 0 = the root, if it is split at all
 }
 
@@ -566,7 +577,7 @@ __global__ __launch_bounds__(kBlock) void k_side(const float* __restrict__ point
         }
     }
     __syncthreads();
-    resolve_exact(deferred, n_def_s, nvec, 0, hp_s, points, P.D,
+    resolve_exact(kBlock >> 5, (int)threadIdx.x >> 5, deferred, n_def_s, nvec, 0, hp_s, points, P.D,
                   [&](int local) { return perm[pos0 + local] & kIdMask; },
                   [&](int local, bool right) {
                       const int id = perm[pos0 + local] & kIdMask;
@@ -586,11 +597,10 @@ __global__ __launch_bounds__(kBlock) void k_side(const float* __restrict__ point
 __global__ __launch_bounds__(kBlock) void k_scatter(TreeParams P, int* __restrict__ perm0, int* __restrict__ perm1,
                                                     const TreeNode* __restrict__ nodes, const int* __restrict__ chunk_base,
                                                     const int* __restrict__ chunk2node, const int* __restrict__ chunk_left,
-                                                    TreeNode* __restrict__ next, int next_cap,
-                                                    TreeNode* __restrict__ tail, int tail_cap, LevelCounters* ctr,
-                                                    TreeRec* __restrict__ recs, int* __restrict__ n_rec, int rec_cap,
-                                                    int2* __restrict__ child)
+                                                    NodeQueues Q, TreeRec* __restrict__ recs, int* __restrict__ n_rec,
+                                                    int rec_cap, int2* __restrict__ child)
 {
+    LevelCounters* ctr = Q.ctr;
     __shared__ int red[2][kBlock / 64];
     const int c = blockIdx.x;
     if (c == 0 && threadIdx.x == 0) phase_tick(ctr, 1);
@@ -674,8 +684,8 @@ __global__ __launch_bounds__(kBlock) void k_scatter(TreeParams P, int* __restric
             index_split(recs + (size_t)nd.tree * rec_cap, n_rec + nd.tree, rec_cap, nd.rec, src[nd.dstart + r1] & kIdMask,
                         src[nd.dstart + r2] & kIdMask, nc, c0.rec, c1.rec, ctr);
         }
-        const int at0 = emit_node(c0, P, next, next_cap, tail, tail_cap, ctr);
-        const int at1 = nc == 2 ? emit_node(c1, P, next, next_cap, tail, tail_cap, ctr) : at0;
+        const int at0 = emit_node(c0, P, Q);
+        const int at1 = nc == 2 ? emit_node(c1, P, Q) : at0;
         // where the members of either side are at the next level (a node with one child keeps them together)
         if (child) child[ni] = make_int2(at0, at1);
     }
@@ -735,7 +745,8 @@ __global__ __launch_bounds__(kBlock) void k_pm_mark(TreeParams P, int* __restric
 struct SmallNode {
     int start, count, dstart, dcount;     // offsets inside the task's segment
     int depth, leaf;
-    int rec, pad_;                        // record of the node in the index of the tree, if one is written
+    int rec;                              // record of the node in the index of the tree, if one is written
+    int vain;                             // splits in a row that left all points together (chain phase)
     uint64_t key;
 };
 
@@ -780,9 +791,10 @@ constexpr int kMaxGroup = 16;        // nodes of one level of a subtree worked o
 // fewer, G) at a time -- their hyperplanes are made together (one wavefront each), all their points are tested in
 // one sweep, and each node is partitioned by one wavefront -- so the number of dependent trips to memory per
 // subtree is a few per level instead of a few per node.
-// TB = threads per workgroup: 256, or 1024 for launches over so few subtrees that workgroups of 256 would leave
-// most of the device idle (the phases of a level then have four times the lanes).
-template <bool Q8, int TB>
+// TB = threads per workgroup: 256, or 512 / 1024 for launches over so few subtrees that workgroups of 256 would leave
+// most of the device idle (the phases of a level then have more lanes).  CHAIN: nodes that are split in vain go to
+// the queue of the chain phase.
+template <bool Q8, int TB, bool CHAIN>
 __global__ __launch_bounds__(TB) void k_tail(const float* __restrict__ points,
                                                  const uint16_t* __restrict__ pb16, const uint8_t* __restrict__ q8, TreeParams P,
                                                  const int* __restrict__ perm0, const int* __restrict__ perm1,
@@ -791,9 +803,10 @@ __global__ __launch_bounds__(TB) void k_tail(const float* __restrict__ points,
                                                  int leaf_cap, int* __restrict__ leaf_start, int* __restrict__ leaf_size,
                                                  TreeStats* stats, LevelCounters* ctr,
                                                  TreeRec* __restrict__ recs_all, int* __restrict__ n_rec_all, int rec_cap,
-                                                 unsigned long long* __restrict__ stat)
+                                                 unsigned long long* __restrict__ stat, TreeNode* __restrict__ chain_all, int chain_cap)
 {
-    // dynamic LDS: seg[small] | tmp[small] | nvec[G][nvec_len(D)] | lrec[node_cap] | level lists 2 x node_cap | fmap[small]
+    // dynamic LDS: seg[small] | tmp[small] | nvec[G][nvec_len(D)] | lrec[node_cap] | level lists 2 x node_cap |
+    // nodes for the chain phase [node_cap] | fmap[small]
     extern __shared__ __align__(16) unsigned char lds_raw[];
     const int Dv = nvec_len(P.D);
     int* seg = reinterpret_cast<int*>(lds_raw);
@@ -804,10 +817,12 @@ __global__ __launch_bounds__(TB) void k_tail(const float* __restrict__ points,
     int2* lrec = reinterpret_cast<int2*>(nvec + (size_t)G * Dv);
     SmallNode* cur = reinterpret_cast<SmallNode*>(lrec + node_cap);
     SmallNode* nxt = cur + node_cap;
-    unsigned char* fmap = reinterpret_cast<unsigned char*>(nxt + node_cap);
+    SmallNode* chain = nxt + node_cap;
+    unsigned char* fmap = reinterpret_cast<unsigned char*>(CHAIN ? chain + node_cap : chain);
     __shared__ float b_s[kMaxGroup], hp_s[kMaxGroup][3];
     __shared__ int left_s[kMaxGroup], pre_s[kMaxGroup + 1], start_s[kMaxGroup], pair_s[kMaxGroup][2];
     __shared__ int n_cur_s, n_nxt_s, nrec_s, kind_s[2], base_s[2], lev_s, mx_s, mn_s, n_def_s;
+    __shared__ int n_chain_s, chain_base_s;
     __shared__ int seen_s, unsure_s;        // points tested over all levels of the subtree, and left to the exact test
 
     const int task = blockIdx.x;
@@ -834,10 +849,10 @@ __global__ __launch_bounds__(TB) void k_tail(const float* __restrict__ points,
     if (tid == 0) {
         SmallNode r;
         r.start = 0; r.count = tk.count; r.dstart = tk.dstart - tk.start; r.dcount = tk.dcount;
-        r.depth = tk.depth; r.leaf = 0; r.key = tk.key; r.rec = tk.rec; r.pad_ = 0;
+        r.depth = tk.depth; r.leaf = 0; r.key = tk.key; r.rec = tk.rec; r.vain = 0;
         cur[0] = r;
         n_cur_s = 1; n_nxt_s = 0; nrec_s = 0; kind_s[0] = 0; kind_s[1] = 0; lev_s = 0; mx_s = 0; mn_s = 0x7fffffff;
-        seen_s = 0; unsure_s = 0;
+        seen_s = 0; unsure_s = 0; n_chain_s = 0;
     }
     __syncthreads();
 
@@ -913,7 +928,7 @@ __global__ __launch_bounds__(TB) void k_tail(const float* __restrict__ points,
             }
             __syncthreads();
             if (tid == 0) { seen_s += total; unsure_s += n_def_s; }
-            resolve_exact(tmp, n_def_s, nvec, Dv, b_s, points, P.D, [&](int pos) { return seg[pos] & kIdMask; },
+            resolve_exact(TB >> 5, tid >> 5, tmp, n_def_s, nvec, Dv, b_s, points, P.D, [&](int pos) { return seg[pos] & kIdMask; },
                           [&](int pos, bool right) { if (right) seg[pos] |= (int)0x80000000; });
             __syncthreads();
             // stable partition, one wavefront per node: seg -> tmp -> seg
@@ -949,12 +964,15 @@ __global__ __launch_bounds__(TB) void k_tail(const float* __restrict__ points,
                     if (c[q].leaf || c[q].depth >= P.MAX_DEPTH - 1) {
                         record_leaf(c[q].start, c[q].count, c[q].depth, c[q].rec);
                     } else {
-                        const int at = atomicAdd(&n_nxt_s, 1);
+                        // a node that keeps all its points again
+                        const int vain = nc == 1 ? nd.vain + 1 : 0;
+                        const bool stuck = CHAIN && vain >= P.vain && c[q].count <= P.chain_max;
+                        const int at = atomicAdd(stuck ? &n_chain_s : &n_nxt_s, 1);
                         if (at < node_cap) {
                             SmallNode sn;
                             sn.start = c[q].start; sn.count = c[q].count; sn.dstart = c[q].dstart; sn.dcount = c[q].dcount;
-                            sn.depth = c[q].depth; sn.leaf = 0; sn.key = c[q].key; sn.rec = c[q].rec; sn.pad_ = 0;
-                            nxt[at] = sn;
+                            sn.depth = c[q].depth; sn.leaf = 0; sn.key = c[q].key; sn.rec = c[q].rec; sn.vain = vain;
+                            (stuck ? chain : nxt)[at] = sn;
                         } else {
                             ctr->overflow = 1;
                         }
@@ -969,6 +987,7 @@ __global__ __launch_bounds__(TB) void k_tail(const float* __restrict__ points,
     }
     for (int i = tid; i < tk.count; i += TB) dst[tk.start + i] = seg[i];
     if (tid == 0) {
+        if (CHAIN) chain_base_s = n_chain_s ? atomicAdd(&ctr->n_chain, n_chain_s) : 0;
         TreeStats* st = stats + tk.tree;
         base_s[0] = kind_s[0] ? atomicAdd(&st->n_leaves, kind_s[0]) : 0;
         base_s[1] = kind_s[1] ? atomicAdd(&st->n_big, kind_s[1]) : 0;
@@ -984,6 +1003,409 @@ __global__ __launch_bounds__(TB) void k_tail(const float* __restrict__ points,
         const int2 r = lrec[i];
         const int count = r.y & 0xffff, rank = r.y >> 16;
         store_leaf(tk.tree, r.x, count, base_s[count > kBucketSplit ? 1 : 0] + rank, leaf_cap, leaf_start, leaf_size, ctr);
+    }
+    for (int i = tid; CHAIN && i < min(n_chain_s, node_cap); i += TB) {
+        const SmallNode sn = chain[i];
+        TreeNode c;
+        c.tree = tk.tree; c.start = tk.start + sn.start; c.count = sn.count; c.dstart = tk.start + sn.dstart; c.dcount = sn.dcount;
+        c.depth = sn.depth; c.buf = 0; c.leaf = 0; c.rec = sn.rec; c.pad_ = 0; c.key = sn.key;
+        const int at = chain_base_s + i;
+        if (at < chain_cap) chain_all[at] = c; else ctr->overflow = 1;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// chain phase: nodes that are split in vain again and again
+// ---------------------------------------------------------------------------
+// A node just above the leaf limit is split again, with a pair of its larger side, until a hyperplane leaves both sides
+// large enough: 200 times in a row for the unluckiest node of 20,000 x 32 points in 50 trees, 430 for 70,000 x 784 with
+// buckets of 91..182.  Each of these levels needs the sides of the one before, so they are a serial chain, and in the tail
+// kernel a link of it costs the whole of a level of a workgroup (17,000 and 51,000 cycles at these two inputs: the trips
+// to memory for the pair's rows, the points' screening rows and the undecided points' rows).  But the points stay the
+// same, and which side of the hyperplane between x1 and x2 a point x is on is whether it is nearer to x1 or to x2.  So a
+// workgroup evaluates the distances of all pairs of the node once (LDS, upper triangle, tiles of 64 x 64), and from then on
+// a link is two reads of LDS per point and a partition in registers.
+//
+// d1, d2: fp32 distances of x to x1, x2, each within 1.01 (D + 3) u of the true one (u = 2^-24).  The exact test compares
+// fl(n.x) with fl(b); the true n.x - b is (d2 - d1) / 2, and the two evaluations are off by at most
+// 1.01 (D/32 + 8) u ||n|| (||x|| + (||x1|| + ||x2||) / 2) together (chains of D/32 terms, five steps of the butterfly,
+// the roundings of n, x1 + x2 and their product; Cauchy-Schwarz), ||n|| = sqrt(d(x1, x2)).  So the sign of d2 - d1 decides
+// when |d2 - d1| > 2.1 (D/32 + 8) u ||n|| (..) + 1.1 (D + 4) u (d1 + d2); otherwise (hardly ever, also for NaN) the point
+// gets the exact test.  ||x|| is bounded by sqrt(D) max |x_d| from the header of the 8-bit row.
+__device__ __forceinline__ int tri_at(int i, int j, int n)
+{
+    const int lo = min(i, j), hi = max(i, j);
+    return lo * n - ((lo * (lo + 1)) >> 1) + hi - lo - 1;
+}
+
+constexpr int kChainPitch = 36;          // floats per staged row of 32 dimensions: odd number of 16-byte units
+
+// The distances of a node of up to kChainSquare points are kept as a square matrix (odd pitch; a point's distances to x1 are
+// a row of it), of a larger one as its upper triangle.
+constexpr int kChainSquare = 120;
+__host__ __device__ inline size_t chain_matrix_floats(int n)
+{
+    return n <= kChainSquare ? (((size_t)n * (size_t)(n | 1)) + 3) / 4 * 4 : ((size_t)n * (n - 1) / 2 + 3) / 4 * 4;
+}
+// bytes of LDS: staged rows (later the normal) | distances | norms, ids, order, second buffer | offset .. | stack | buckets
+__host__ __device__ inline size_t chain_stage_floats(int n, int D)
+{
+    const size_t rows = (size_t)((n + 15) & ~15) * kChainPitch, normal = (size_t)nvec_len(D);
+    return rows > normal ? rows : normal;
+}
+__host__ __device__ inline size_t chain_lds_bytes(int n, int D, int node_cap)
+{
+    return chain_stage_floats(n, D) * 4 + chain_matrix_floats(n) * 4 + (size_t)n * 16 + 16 +
+           (size_t)node_cap * (sizeof(SmallNode) + 8);
+}
+
+// The draws of the next levels of a chain.  The key of a child follows from the key of its parent and the side alone, so
+// the nodes of the next five levels are worked out side by side: lane 2 h + i holds draw i (draw_u32) of the node that
+// is reached from the base by the bits of h below its leading one (h = 1: the base itself).
+struct ChainDraws {
+    uint64_t key;        // of the node of this lane
+    uint32_t draw;
+    int h;               // the present node (uniform)
+
+    __device__ __forceinline__ void start(uint64_t base)
+    {
+        const int lane = lane_id(), node = lane >> 1;
+        key = base;
+        const int depth = node > 0 ? 31 - __clz(node) : 0;
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+            if (s < depth) key = child_key(key, (node >> (depth - 1 - s)) & 1);
+        draw = draw_u32(key, (uint32_t)(lane & 1));
+        h = 1;
+    }
+    __device__ __forceinline__ uint64_t node_key() const
+    {
+        return (uint64_t)(uint32_t)read_lane_i((int)(uint32_t)key, 2 * h) |
+               ((uint64_t)(uint32_t)read_lane_i((int)(uint32_t)(key >> 32), 2 * h) << 32);
+    }
+    // the child on side s is the next node
+    __device__ __forceinline__ void descend(int s)
+    {
+        if (h >= 16) start(child_key(node_key(), s));
+        else h = 2 * h + s;
+    }
+    // pick_pair of the present node
+    __device__ __forceinline__ void pair(int count, int& r1, int& r2) const
+    {
+        const uint32_t r = draw % (uint32_t)count;
+        r1 = read_lane_i((int)r, 2 * h);
+        r2 = read_lane_i((int)r, 2 * h + 1);
+        if (r1 == r2) pick_pair(node_key(), count, r1, r2);
+    }
+};
+
+// NB: blocks of 16 points a node may have (8: distances as a square matrix).
+template <int NB>
+__global__ __launch_bounds__(256) void k_chain(const float* __restrict__ points, const uint8_t* __restrict__ q8, TreeParams P,
+                                               int* __restrict__ perm_out, const TreeNode* __restrict__ tasks, int task_cap,
+                                               int node_cap, int leaf_cap, int* __restrict__ leaf_start,
+                                               int* __restrict__ leaf_size, TreeStats* stats, LevelCounters* ctr,
+                                               TreeRec* __restrict__ recs_all, int* __restrict__ n_rec_all, int rec_cap,
+                                               unsigned long long* __restrict__ stat)
+{
+    extern __shared__ __align__(16) unsigned char chain_lds[];
+    const int nmax = P.chain_max;
+    float* stage = reinterpret_cast<float*>(chain_lds);
+    float* nvec = stage;                                                      // once the distances are there
+    float* tri = stage + chain_stage_floats(nmax, P.D);
+    float* norm = tri + chain_matrix_floats(nmax);
+    int* ids = reinterpret_cast<int*>(norm + nmax);
+    int* ord = ids + nmax;                                                    // position in the node -> place in ids
+    int* tmp = ord + nmax;
+    float* hp = reinterpret_cast<float*>(tmp + nmax);
+    SmallNode* stack = reinterpret_cast<SmallNode*>(hp + 4);
+    int2* lrec = reinterpret_cast<int2*>(stack + node_cap);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int n_tasks = min(ctr->n_chain, task_cap);
+    const bool vec_ok = (P.D & 3) == 0 && ((reinterpret_cast<uintptr_t>(points) & 15) == 0);
+    const float u24 = 1.0f / 16777216.0f;
+    const float tol_n = 2.1f * (float)(P.D / 32 + 8) * u24, tol_d = 1.1f * (float)(P.D + 4) * u24;
+    int seen = 0, unsure = 0;
+
+    for (int task = blockIdx.x; task < n_tasks; task += gridDim.x) {
+        const TreeNode tk = tasks[task];
+        const int n = tk.count;
+        int* seg = perm_out + (size_t)tk.tree * (size_t)P.N + tk.start;
+        __syncthreads();                                                      // the previous task is done with the LDS
+        if (tid < n) {
+            const int id = seg[tid];
+            ids[tid] = id;
+            ord[tid] = tid;
+            if (q8) {
+                const float4 head = *reinterpret_cast<const float4*>(q8 + (size_t)id * (size_t)q8_pitch(P.D));
+                norm[tid] = 1.01f * __builtin_sqrtf((float)P.D) * fmaxf(fabsf(head.y), fabsf(head.y + 255.0f * head.z)) + 0.0f * head.w;
+            }
+        }
+        __syncthreads();
+        if (!q8) {
+            for (int i = wave; i < n; i += 4) {
+                const float* x = points + (size_t)ids[i] * (size_t)P.D;
+                float s = 0.0f;
+                for (int d = lane; d < P.D; d += 64) s = __builtin_fmaf(x[d], x[d], s);
+                s += dpp_f<kDppXor1>(s); s += dpp_f<kDppXor2>(s); s += dpp_f<kDppHalfMirror>(s); s += dpp_f<kDppMirror>(s);
+                s = read_lane_f(s, 0) + read_lane_f(s, 16) + read_lane_f(s, 32) + read_lane_f(s, 48);
+                if (lane == 0) norm[i] = 1.01f * __builtin_sqrtf(s);
+            }
+        }
+        // distances: thread (ty, tx) has the pairs (ty + 16 r, tx + 16 c), c >= r, of all blocks; 32 dimensions of all rows at
+        // a time through LDS, the next 32 under way meanwhile
+        {
+            const int nb = (n + 15) >> 4, ty = tid >> 4, tx = tid & 15;
+            constexpr int kLoads = NB / 2;                                    // 16-byte pieces of a step per thread
+            float acc[NB * (NB + 1) / 2];
+#pragma unroll
+            for (int k = 0; k < NB * (NB + 1) / 2; ++k) acc[k] = 0.0f;
+            float4 pre[kLoads];
+            auto request = [&](int d0) {
+#pragma unroll
+                for (int i = 0; i < kLoads; ++i) {
+                    const int row = (tid >> 3) + 32 * i, d = d0 + 4 * (tid & 7);
+                    pre[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+                    if (row < n && d < P.D) {
+                        const float* src = points + (size_t)ids[row] * (size_t)P.D + d;
+                        if (vec_ok) {
+                            pre[i] = *reinterpret_cast<const float4*>(src);
+                        } else {
+                            pre[i].x = src[0];
+                            if (d + 1 < P.D) pre[i].y = src[1];
+                            if (d + 2 < P.D) pre[i].z = src[2];
+                            if (d + 3 < P.D) pre[i].w = src[3];
+                        }
+                    }
+                }
+            };
+            request(0);
+            for (int d0 = 0; d0 < P.D; d0 += 32) {
+#pragma unroll
+                for (int i = 0; i < kLoads; ++i) {
+                    const int row = (tid >> 3) + 32 * i;
+                    if (row < nb * 16) *reinterpret_cast<float4*>(&stage[row * kChainPitch + 4 * (tid & 7)]) = pre[i];
+                }
+                __syncthreads();
+                if (d0 + 32 < P.D) request(d0 + 32);
+                const int nd = min(32, (P.D - d0 + 3) & ~3);
+                for (int dd = 0; dd < nd; dd += 4) {
+                    float4 av[NB];
+#pragma unroll
+                    for (int r = 0; r < NB; ++r)
+                        if (r < nb) av[r] = *reinterpret_cast<const float4*>(&stage[(ty + 16 * r) * kChainPitch + dd]);
+#pragma unroll
+                    for (int c = 0; c < NB; ++c) {
+                        if (c >= nb) continue;
+                        const float4 bv = *reinterpret_cast<const float4*>(&stage[(tx + 16 * c) * kChainPitch + dd]);
+#pragma unroll
+                        for (int r = 0; r <= c; ++r) {
+                            float& s = acc[c * (c + 1) / 2 + r];
+                            float df;
+                            df = av[r].x - bv.x; s = __builtin_fmaf(df, df, s);
+                            df = av[r].y - bv.y; s = __builtin_fmaf(df, df, s);
+                            df = av[r].z - bv.z; s = __builtin_fmaf(df, df, s);
+                            df = av[r].w - bv.w; s = __builtin_fmaf(df, df, s);
+                        }
+                    }
+                }
+                __syncthreads();
+            }
+#pragma unroll
+            for (int c = 0; c < NB; ++c)
+#pragma unroll
+                for (int r = 0; r <= c; ++r) {
+                    const int i = ty + 16 * r, j = tx + 16 * c;
+                    if (c < nb && i <= j && j < n) {
+                        if constexpr (NB == 8) {
+                            tri[i * (n | 1) + j] = acc[c * (c + 1) / 2 + r];
+                            tri[j * (n | 1) + i] = acc[c * (c + 1) / 2 + r];
+                        } else if (i < j) {
+                            tri[tri_at(i, j, n)] = acc[c * (c + 1) / 2 + r];
+                        }
+                    }
+                }
+        }
+        __syncthreads();
+        if (wave != 0) continue;                                              // the chain is the first wavefront's
+        TreeRec* recs = recs_all ? recs_all + (size_t)tk.tree * rec_cap : nullptr;
+        int* n_rec = recs_all ? n_rec_all + tk.tree : nullptr;
+        int start = 0, count = n, dstart = tk.dstart - tk.start, dcount = tk.dcount, depth = tk.depth, rec = tk.rec;
+        ChainDraws draws;
+        draws.start(tk.key);
+        int sp = 0, nrec = 0, n_kind[2] = {0, 0}, levels = 0, largest = 0, smallest = 0x7fffffff;
+        constexpr int kV = NB / 4;                                            // points per lane
+        auto dist_to = [&](int o, int q) -> float {
+            if constexpr (NB == 8) return tri[o * (n | 1) + q];
+            else return q == o ? 0.0f : tri[tri_at(q, o, n)];
+        };
+        int q[kV];                                                            // places of the node's points, by position
+        auto take_order = [&]() {
+#pragma unroll
+            for (int v = 0; v < kV; ++v) q[v] = ord[min(start + lane + 64 * v, n - 1)];
+        };
+        auto place_at = [&](int pos) {
+            int o = read_lane_i(q[0], pos & 63);
+#pragma unroll
+            for (int v = 1; v < kV; ++v)
+                if ((pos >> 6) == v) o = read_lane_i(q[v], pos & 63);
+            return o;
+        };
+        take_order();
+        while (true) {
+            int r1, r2;
+            draws.pair(dcount, r1, r2);
+            const int o1 = place_at(dstart - start + r1), o2 = place_at(dstart - start + r2);
+            const float nn = tol_n * __builtin_sqrtf(dist_to(o1, o2)), half12 = 0.5f * (norm[o1] + norm[o2]);
+            float d1[kV], d2[kV], nq[kV];
+#pragma unroll
+            for (int v = 0; v < kV; ++v) {
+                d1[v] = dist_to(o1, q[v]);
+                d2[v] = dist_to(o2, q[v]);
+                nq[v] = norm[q[v]];
+            }
+            uint64_t left[kV], again[kV];
+            int a = 0, n_def = 0;
+#pragma unroll
+            for (int v = 0; v < kV; ++v) {
+                const bool valid = lane + 64 * v < count;
+                const float tol = nn * (nq[v] + half12) + tol_d * (d1[v] + d2[v]) + 1e-30f;
+                const bool certain = fabsf(d2[v] - d1[v]) > tol;              // false if anything is NaN
+                left[v] = ballot64(valid && certain && !(d2[v] < d1[v]));
+                again[v] = ballot64(valid && !certain);
+                n_def += __popcll(again[v]);
+            }
+            seen += count;
+            if (n_def > 0) {
+                // the exact test; bit 31 of a point's place in ord carries the answer
+                unsure += n_def;
+                int at = 0;
+#pragma unroll
+                for (int v = 0; v < kV; ++v) {
+                    if ((again[v] >> lane) & 1ull) tmp[at + mask_prefix(again[v])] = lane + 64 * v;
+                    at += __popcll(again[v]);
+                }
+                make_hyperplane_wave(points + (size_t)ids[o1] * P.D, points + (size_t)ids[o2] * P.D, P.D, nvec, hp);
+                wave_lds_sync();
+                resolve_exact(2, lane >> 5, tmp, n_def, nvec, 0, hp, points, P.D, [&](int pos) { return ids[ord[start + pos]]; },
+                              [&](int pos, bool right) { if (right) ord[start + pos] |= (int)0x80000000; });
+                wave_lds_sync();
+#pragma unroll
+                for (int v = 0; v < kV; ++v) {
+                    const bool mine = (again[v] >> lane) & 1ull;
+                    left[v] |= ballot64(mine && ord[start + (mine ? lane + 64 * v : 0)] >= 0);
+                }
+            }
+            // stable partition
+#pragma unroll
+            for (int v = 0; v < kV; ++v) a += __popcll(left[v]);
+            int lbase = 0;
+#pragma unroll
+            for (int v = 0; v < kV; ++v) {
+                const int i = lane + 64 * v;
+                const int lrank = lbase + mask_prefix(left[v]);
+                const bool is_left = lane_bit(left[v]);
+                if (i < count) ord[start + (is_left ? lrank : a + i - lrank)] = q[v];
+                lbase += __popcll(left[v]);
+            }
+            wave_lds_sync();
+            // (split_rules without the nodes around it) one child that stays to be split: the next link
+            const int r = count - a;
+            if (!recs && min(a, r) < P.MIN && count > P.MAX && depth + 1 < P.MAX_DEPTH - 1) {
+                if (a == 0 || r == 0) {
+                    draws.descend(a ? 0 : 1);
+                    dstart = start;
+                    dcount = count;
+                } else {
+                    const bool left_big = a >= r;
+                    draws.descend(left_big ? 0 : 1);
+                    dstart = left_big ? start : start + a;
+                    dcount = left_big ? a : r;
+                }
+                ++depth;
+                take_order();
+                continue;
+            }
+            // children: the first one that is no bucket is next, another waits on the stack
+            TreeNode full, c[2];
+            full.tree = tk.tree; full.start = start; full.count = count; full.dstart = dstart; full.dcount = dcount;
+            full.depth = depth; full.buf = 0; full.leaf = 0; full.rec = rec; full.pad_ = 0; full.key = draws.node_key();
+            const int nc = split_rules(full, a, P.MIN, P.MAX, 0, c[0], c[1]);
+            if (recs) {
+                if (lane == 0) index_split(recs, n_rec, rec_cap, rec, ids[o1], ids[o2], nc, c[0].rec, c[1].rec, ctr);
+                c[0].rec = __builtin_amdgcn_readfirstlane(c[0].rec);
+                c[1].rec = __builtin_amdgcn_readfirstlane(c[1].rec);
+            }
+            bool have = false;
+            for (int k = 0; k < nc; ++k) {
+                if (c[k].leaf || c[k].depth >= P.MAX_DEPTH - 1) {
+                    const int big = c[k].count > kBucketSplit ? 1 : 0;
+                    if (lane == 0) {
+                        if (nrec < node_cap) lrec[nrec] = make_int2(tk.start + c[k].start, c[k].count | (n_kind[big] << 16));
+                        else ctr->overflow = 1;
+                        if (recs) index_bucket(recs, rec_cap, c[k].rec, tk.start + c[k].start, c[k].count, ctr);
+                    }
+                    ++nrec;
+                    ++n_kind[big];
+                    levels = max(levels, c[k].depth + 1);
+                    largest = max(largest, c[k].count);
+                    smallest = min(smallest, c[k].count);
+                } else if (!have) {
+                    have = true;
+                    start = c[k].start; count = c[k].count; dstart = c[k].dstart; dcount = c[k].dcount;
+                    depth = c[k].depth; rec = c[k].rec;
+                    draws.start(c[k].key);
+                } else {
+                    if (lane == 0) {
+                        if (sp < node_cap) {
+                            SmallNode sn;
+                            sn.start = c[k].start; sn.count = c[k].count; sn.dstart = c[k].dstart; sn.dcount = c[k].dcount;
+                            sn.depth = c[k].depth; sn.leaf = 0; sn.key = c[k].key; sn.rec = c[k].rec; sn.vain = 0;
+                            stack[sp] = sn;
+                        } else {
+                            ctr->overflow = 1;
+                        }
+                    }
+                    sp = min(sp + 1, node_cap);
+                }
+            }
+            if (!have) {
+                if (sp == 0) break;
+                --sp;
+                wave_lds_sync();
+                const SmallNode* sn = &stack[sp];
+                start = __builtin_amdgcn_readfirstlane(sn->start);
+                count = __builtin_amdgcn_readfirstlane(sn->count);
+                dstart = __builtin_amdgcn_readfirstlane(sn->dstart);
+                dcount = __builtin_amdgcn_readfirstlane(sn->dcount);
+                depth = __builtin_amdgcn_readfirstlane(sn->depth);
+                rec = __builtin_amdgcn_readfirstlane(sn->rec);
+                draws.start(sn->key);
+            }
+            take_order();
+        }
+        for (int i = lane; i < n; i += 64) seg[i] = ids[ord[i]];
+        int base[2] = {0, 0};
+        if (lane == 0) {
+            TreeStats* st = stats + tk.tree;
+            if (n_kind[0]) base[0] = atomicAdd(&st->n_leaves, n_kind[0]);
+            if (n_kind[1]) base[1] = atomicAdd(&st->n_big, n_kind[1]);
+            // (the extremes settle early: a look before the atomic spares nearly all of them)
+            if (*const_cast<volatile int*>(&st->levels) < levels) atomicMax(&st->levels, levels);
+            if (*const_cast<volatile int*>(&st->max_leaf) < largest) atomicMax(&st->max_leaf, largest);
+            if (*const_cast<volatile int*>(&st->min_leaf) > smallest) atomicMin(&st->min_leaf, smallest);
+        }
+        base[0] = __builtin_amdgcn_readfirstlane(base[0]);
+        base[1] = __builtin_amdgcn_readfirstlane(base[1]);
+        for (int i = lane; i < min(nrec, node_cap); i += 64) {
+            const int2 r = lrec[i];
+            const int m = r.y & 0xffff, rank = r.y >> 16;
+            store_leaf(tk.tree, r.x, m, base[m > kBucketSplit ? 1 : 0] + rank, leaf_cap, leaf_start, leaf_size, ctr);
+        }
+    }
+    if (tid == 0) {
+        stat_add(stat, (int)blockIdx.x, 0, seen);
+        stat_add(stat, (int)blockIdx.x, 1, unsure);
     }
 }
 
@@ -1004,6 +1426,7 @@ struct TreeBatchWorkspace {
     int* perm[2] = {nullptr, nullptr};   // perm[0] is also the output
     TreeNode* nodes[2] = {nullptr, nullptr};
     TreeNode* tail = nullptr;
+    TreeNode* chain = nullptr;           // nodes for the chain phase
     int* chunk_base = nullptr;
     int* chunk2node = nullptr;
     int* chunk_left = nullptr;
@@ -1040,7 +1463,7 @@ struct TreeBatchWorkspace {
 
 static void free_ws(TreeBatchWorkspace& w)
 {
-    void* dev[] = {w.perm[0], w.perm[1], w.nodes[0], w.nodes[1], w.tail, w.chunk_base, w.chunk2node,
+    void* dev[] = {w.perm[0], w.perm[1], w.nodes[0], w.nodes[1], w.tail, w.chain, w.chunk_base, w.chunk2node,
                    w.chunk_left, w.leaf_start, w.leaf_size, w.stats, w.ctr, w.recs, w.n_rec, w.planes,
                    w.pm_path, w.pm_side, w.pm_undec, w.pm_map[0], w.pm_map[1], w.pm_sc, w.pm_aq, w.pm_child, w.stat};
     for (void* p : dev) ws_free(p);
@@ -1082,13 +1505,26 @@ int tree_small_threshold(int D, int N, int B)
     const int v = e && *e ? std::atoi(e) : (D <= 48 || few ? 2048 : 1024);
     return std::min(2048, std::max(64, v));
 }
+// Largest node the chain phase takes (0: none): twice the leaf limit where that fits two workgroups per compute unit
+// (nodes just above the limit are the ones that are split in vain), else what one workgroup can hold.
+int tree_chain_max(int D, int MIN, int MAX)
+{
+    const char* e = std::getenv("RSFK_TREE_CHAIN");
+    if ((e && e[0] == '0') || D > 2048) return 0;            // (the normal takes the place of the staged rows)
+    const int per_min = std::max(MIN, 1);
+    if (MAX + MAX / 8 <= kChainSquare) return std::min(kChainSquare, std::max(64, (2 * MAX + 7) & ~7));
+    int n = 0;
+    for (int m = kChainSquare + 8; m <= 256; m += 8)
+        if (chain_lds_bytes(m, D, m / per_min + 4) <= (size_t)158 * 1024) n = m;
+    return n > MAX ? n : 0;
+}
 constexpr int kWideChunk = 1024;         // points per workgroup in the wide passes (k_side keeps a chunk's undecided points in LDS)
 
 // bytes of device memory a batch of B trees needs
 size_t tree_ws_bytes(int N, int D, int MIN, int B)
 {
     const size_t lc = (size_t)N / (size_t)std::max(MIN, 1) + 2;
-    return bf16_copy_bytes(N, D) + (size_t)B * ((size_t)N * 8 + (size_t)N * 2 + 512 * 1024 + lc * (8 + sizeof(TreeNode)) + ((size_t)N / 1024 + 2) * (2 * sizeof(TreeNode) + 24 + (size_t)(4 + nvec_len(D)) * 4));
+    return bf16_copy_bytes(N, D) + (size_t)B * ((size_t)N * 8 + (size_t)N * 2 + 512 * 1024 + lc * (8 + 2 * sizeof(TreeNode)) + ((size_t)N / 1024 + 2) * (2 * sizeof(TreeNode) + 24 + (size_t)(4 + nvec_len(D)) * 4));
 }
 
 // From now on every build with this workspace also writes the index of each tree (TreeRec records).
@@ -1123,6 +1559,7 @@ int tree_ws_alloc(TreeBatchWorkspace** out, int N, int D, int MIN, int B)
     if (dmalloc(&w->nodes[0], (size_t)w->node_cap)) return 1;
     if (dmalloc(&w->nodes[1], (size_t)w->node_cap)) return 1;
     if (dmalloc(&w->tail, (size_t)w->tail_cap)) return 1;
+    if (dmalloc(&w->chain, (size_t)w->tail_cap)) return 1;
     if (dmalloc(&w->chunk_base, (size_t)w->node_cap + 1)) return 1;
     if (dmalloc(&w->chunk2node, (size_t)w->chunk_cap)) return 1;
     if (dmalloc(&w->chunk_left, (size_t)w->chunk_cap)) return 1;
@@ -1174,6 +1611,8 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
     TreeParams P;
     P.N = N; P.D = D; P.MIN = MIN; P.MAX = MAX; P.MAX_DEPTH = MAX_DEPTH;
     P.small = tree_small_threshold(D, N, w->B);
+    P.chain_max = tree_chain_max(D, MIN, MAX);
+    P.vain = 4;
     P.chunk = kWideChunk;
     // bfloat16 rounding 2^-8 (1 + 2^-7), plus the summation errors of the screen (D/8 terms per lane and a 3-step
     // tree) and of the exact test (D/32 terms per lane and a 5-step tree), 1 % on top
@@ -1198,8 +1637,11 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
         pm_levels = pm::kMaxLevels - 1;
         if (const char* e = std::getenv("RSFK_PM_LEVELS")) pm_levels = std::max(0, std::min(pm::kMaxLevels, std::atoi(e)));
     }
-    hipLaunchKernelGGL(k_init_roots, dim3((nb + 63) / 64), dim3(64), 0, stream, w->nodes[0], w->tail, w->ctr, P, nb, seed0,
-                       w->n_rec, pm_levels > 0 ? w->pm_map[0] : nullptr);
+    NodeQueues Q;
+    Q.next = w->nodes[0]; Q.next_cap = w->node_cap;
+    Q.tail = w->tail; Q.tail_cap = w->tail_cap;
+    Q.ctr = w->ctr;
+    hipLaunchKernelGGL(k_init_roots, dim3((nb + 63) / 64), dim3(64), 0, stream, Q, P, nb, seed0, w->n_rec, pm_levels > 0 ? w->pm_map[0] : nullptr);
     RSFK_HIP(hipGetLastError());
 
     int cur = 0;
@@ -1281,9 +1723,10 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
 #undef RSFK_SIDE_LAUNCH
         }
         const bool map_next = level + 1 < pm_levels;
+        Q.next = w->nodes[cur ^ 1];
         hipLaunchKernelGGL(k_scatter, dim3(n_chunks), dim3(kBlock), 0, stream, P, w->perm[0], w->perm[1], w->nodes[cur],
-                           w->chunk_base, w->chunk2node, w->chunk_left, w->nodes[cur ^ 1], w->node_cap, w->tail, w->tail_cap, w->ctr,
-                           w->recs, w->n_rec, w->rec_cap, map_next ? w->pm_child : nullptr);
+                           w->chunk_base, w->chunk2node, w->chunk_left, Q, w->recs, w->n_rec, w->rec_cap,
+                           map_next ? w->pm_child : nullptr);
         if (map_next) {
             const int n_paths = 1 << level;
             hipLaunchKernelGGL(pm::k_pm_next_map, dim3((unsigned)((nb * n_paths + 255) / 256)), dim3(256), 0, stream,
@@ -1294,7 +1737,16 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
         ++level;
     }
     // tail
+    (void)hipEventRecord(w->ev[0], stream);
     const int n_tail = w->h_ctr->n_tail;
+    // Few subtrees (small inputs, few trees): what counts is how long the longest of them takes.  Workgroups of 1024 threads
+    // while every subtree has a compute unit to itself, of 512 beyond that (so that all of them are resident at once:
+    // 20,000 x 32, 50 trees, 808 subtrees 1.69 -> 1.58 ms for the trees), and nodes that are split in vain leave for the
+    // chain phase.  With more subtrees than that the device is full anyway and the chains run beside the rest: the
+    // chain phase then only adds its matrices (1M x 100, 50 trees: tail 10.7 -> 9.0 ms, chains 6.8 ms).
+    // RSFK_TAIL_BLOCK=256 / 1024 overrides.
+    bool few = n_tail > 0 && n_tail < 8 * 256;
+    if (const char* e = std::getenv("RSFK_TAIL_BLOCK")) few = std::atoi(e) >= 1024;
     RSFK_CHECK(n_tail <= w->tail_cap, "tree batch: tail queue overflow");
     if (n_tail > 0) {
         // (the tail kernel keeps the bfloat16 screen: measured, it is not faster with the 8-bit one)
@@ -1303,30 +1755,44 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
         const int node_cap = P.small / std::max(MIN, 1) + 4;
         const int G = std::max(1, std::min(kMaxGroup, (int)(24 * 1024 / ((size_t)nvec_len(D) * 4))));
         const size_t lds = (size_t)(2 * P.small) * 4 + (size_t)G * nvec_len(D) * 4 + (size_t)node_cap * sizeof(int2) +
-                           2 * (size_t)node_cap * sizeof(SmallNode) + (size_t)P.small;
+                           (few ? 3 : 2) * (size_t)node_cap * sizeof(SmallNode) + (size_t)P.small;
         RSFK_CHECK(lds <= 150 * 1024, "tree batch: D too large for the tail kernel's LDS budget");
         const bool tail_q8 = q8 != nullptr && std::getenv("RSFK_TAIL_BF16") == nullptr;
-        (void)hipEventRecord(w->ev[0], stream);
-        // few subtrees (small inputs, few trees): workgroups of 1024 threads, so that a subtree's levels take less time
-        // (70,000 x 784, 10 trees: 1.24 -> 1.00 ms per tree).  RSFK_TAIL_BLOCK=256 / 1024 overrides.
-        bool wide_wg = n_tail < 8 * 256;
-        if (const char* e = std::getenv("RSFK_TAIL_BLOCK")) wide_wg = std::atoi(e) >= 1024;
-#define RSFK_TAIL_LAUNCH(Q, T)                                                                                             \
+#define RSFK_TAIL_LAUNCH(Q, T, C)                                                                                             \
         do {                                                                                                               \
-            RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_tail<Q, T>),                                      \
+            RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_tail<Q, T, C>),                                      \
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));                          \
-            hipLaunchKernelGGL((k_tail<Q, T>), dim3(n_tail), dim3(T), lds, stream, points, pb16, q8, P, w->perm[0],         \
+            hipLaunchKernelGGL((k_tail<Q, T, C>), dim3(n_tail), dim3(T), lds, stream, points, pb16, q8, P, w->perm[0],         \
                                w->perm[1], w->perm[0], w->tail, n_tail, node_cap, G, w->leaf_cap, w->leaf_start,            \
-                               w->leaf_size, w->stats, w->ctr, w->recs, w->n_rec, w->rec_cap, w->stat);                    \
+                               w->leaf_size, w->stats, w->ctr, w->recs, w->n_rec, w->rec_cap, w->stat, w->chain, w->tail_cap); \
         } while (0)
-        if (tail_q8 && wide_wg) RSFK_TAIL_LAUNCH(true, 1024);
-        else if (tail_q8) RSFK_TAIL_LAUNCH(true, 256);
-        else if (wide_wg) RSFK_TAIL_LAUNCH(false, 1024);
-        else RSFK_TAIL_LAUNCH(false, 256);
+        if (tail_q8 && few && n_tail <= 256) RSFK_TAIL_LAUNCH(true, 1024, true);
+        else if (tail_q8 && few) RSFK_TAIL_LAUNCH(true, 512, true);
+        else if (tail_q8) RSFK_TAIL_LAUNCH(true, 256, false);
+        else if (few) RSFK_TAIL_LAUNCH(false, 512, true);
+        else RSFK_TAIL_LAUNCH(false, 256, false);
 #undef RSFK_TAIL_LAUNCH
-        (void)hipEventRecord(w->ev[1], stream);
         RSFK_HIP(hipGetLastError());
     }
+    if (few && P.chain_max > 0) {
+        const int node_cap = P.chain_max / std::max(MIN, 1) + 4;
+        const size_t lds = chain_lds_bytes(P.chain_max, D, node_cap);
+        const size_t most = (size_t)N * (size_t)nb / (size_t)std::max(MAX - 1, 1) + 1;          // nodes that are no buckets are disjoint
+        const unsigned grid = (unsigned)std::min<size_t>(most, 256 * (size_t)std::max<size_t>(1, (size_t)160 * 1024 / lds));
+#define RSFK_CHAIN_LAUNCH(NBV)                                                                                              \
+        do {                                                                                                               \
+            RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_chain<NBV>),                                      \
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));                          \
+            hipLaunchKernelGGL(k_chain<NBV>, dim3(grid), dim3(256), lds, stream, points, q8, P, w->perm[0], w->chain,       \
+                               w->tail_cap, node_cap, w->leaf_cap, w->leaf_start, w->leaf_size, w->stats, w->ctr, w->recs,  \
+                               w->n_rec, w->rec_cap, w->stat);                                                             \
+        } while (0)
+        if (P.chain_max <= kChainSquare) RSFK_CHAIN_LAUNCH(8);
+        else RSFK_CHAIN_LAUNCH(16);
+#undef RSFK_CHAIN_LAUNCH
+        RSFK_HIP(hipGetLastError());
+    }
+    (void)hipEventRecord(w->ev[1], stream);
     RSFK_HIP(hipMemcpyAsync(w->h_stats, w->stats, sizeof(TreeStats) * (size_t)nb, hipMemcpyDeviceToHost, stream));
     RSFK_HIP(hipMemcpyAsync(w->h_ctr, w->ctr, sizeof(LevelCounters), hipMemcpyDeviceToHost, stream));
     RSFK_HIP(hipMemcpyAsync(w->h_stat, w->stat, sizeof(unsigned long long) * kStatSlots * kStatPitch, hipMemcpyDeviceToHost, stream));
@@ -1336,7 +1802,7 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
         w->counts[0] += w->h_stat[kStatPitch * sl];
         w->counts[1] += w->h_stat[kStatPitch * sl + 1];
     }
-    if (n_tail > 0) {
+    {
         float ms = 0.0f;
         if (hipEventElapsedTime(&ms, w->ev[0], w->ev[1]) == hipSuccess) w->phase_s[3] = ms * 1e-3f;
     }

@@ -58,6 +58,32 @@ def test_tree_partition_is_identical(gpu, orc, rng, monkeypatch, N, D, MIN, MAX,
         assert list(gst) == [len(ls), st[0], st[1], st[2]]
 
 
+# Nodes that are split in vain again and again (MIN at half of MAX), finished from the distances of their points: leaf limits
+# on either side of the square / triangular distance matrix and at the largest node that fits, rows shorter than a
+# staging step, D not a multiple of 4, a common offset and duplicated points (nothing but the exact test decides),
+# a depth limit that falls inside a chain.
+@pytest.mark.parametrize("N,D,MIN,MAX,kind,depth", [
+    (4000, 5, 33, 66, "n", 5000), (3000, 1, 8, 16, "n", 5000), (3000, 37, 53, 106, "n", 5000), (3000, 37, 54, 108, "n", 5000),
+    (5000, 12, 112, 224, "n", 5000), (3000, 100, 33, 66, "offset", 5000), (3000, 6, 20, 40, "dup", 400), (4000, 16, 33, 66, "n", 14),
+    (2500, 260, 60, 120, "n", 5000),
+])
+@pytest.mark.parametrize("screen", ["q8", "bf16"])
+def test_tree_nodes_split_in_vain(gpu, orc, rng, monkeypatch, N, D, MIN, MAX, kind, depth, screen):
+    monkeypatch.setenv("RSFK_TREE_SCREEN", screen)
+    X = rng.standard_normal((N, D)).astype(np.float32)
+    if kind == "offset":
+        X = (X * 1e-3 + 1000.0).astype(np.float32)
+    if kind == "dup":
+        X = X[rng.integers(0, N // 8, N)]
+    for seed in (1, 2):
+        _say("tree split in vain", N, D, MIN, MAX, kind, depth, seed)
+        perm, ls, lz, st = orc.build_tree(X, MIN, MAX, depth, seed)
+        gperm, gls, glz, gst = gpu.build_tree(X, MIN, MAX, depth, seed)
+        assert np.array_equal(gperm, perm)
+        assert np.array_equal(gls, ls) and np.array_equal(glz, lz)
+        assert list(gst) == [len(ls), st[0], st[1], st[2]]
+
+
 def test_tree_edge_cases(gpu, orc, rng):
     # identical points: re-drawn until the depth limit, then one forced bucket
     X = np.ones((3000, 4), np.float32)
