@@ -296,8 +296,7 @@ int q8_copy_fill(const Q8Copy& c, const float* points, int N, int D, hipStream_t
 int q8_copy_mean_rho(const Q8Copy& c, int N, float* mean_rho, hipStream_t stream)
 {
     float sum = 0.0f;
-    RSFK_HIP(hipMemcpyAsync(&sum, c.rho_sum, sizeof(float), hipMemcpyDeviceToHost, stream));
-    RSFK_HIP(hipStreamSynchronize(stream));
+    if (fetch_words(reinterpret_cast<const int*>(c.rho_sum), 1, reinterpret_cast<int*>(&sum), stream)) return 1;
     *mean_rho = N > 0 ? sum / (float)N : 0.0f;
     return 0;
 }

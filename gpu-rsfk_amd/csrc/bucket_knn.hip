@@ -418,10 +418,11 @@ int largest_bucket(const int* sizes, int n, hipStream_t stream, int* out)
     hipError_t e = hipMemcpyAsync(d, &v, sizeof(int), hipMemcpyHostToDevice, stream);
     if (e == hipSuccess) {
         hipLaunchKernelGGL(k_max_size, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, sizes, n, static_cast<int*>(d));
-        e = hipMemcpyAsync(&v, d, sizeof(int), hipMemcpyDeviceToHost, stream);
+        e = hipGetLastError();
     }
-    if (e == hipSuccess) e = hipStreamSynchronize(stream);
+    const int rc = e == hipSuccess ? fetch_words(static_cast<const int*>(d), 1, &v, stream) : 0;
     ws_free(d);
+    if (rc) return 1;
     if (e != hipSuccess) { set_last_error(std::string("largest bucket: ") + hipGetErrorString(e)); return 1; }
     *out = v;
     return 0;

@@ -1124,7 +1124,7 @@ int launch_explore(const float* points, const Bf16Copy* bf, const Bf16Copy* bf_j
         const uint32_t* pass = explore_ws_pass(ws);
         int* listA = explore_ws_todo(ws, 0);
         int* listB = explore_ws_todo(ws, 1);
-        int* host_n = explore_ws_host_count(ws);
+        int n_back = 0;
         // (the bounds of the join, when it kept them and the set with a bound per place still fits)
         const uint16_t* wave_bounds = explore_ws_bounds(ws);
         if (4 * merge_wave_ints(small_table, dpad, K, true) > lds_ints) wave_bounds = nullptr;
@@ -1159,10 +1159,9 @@ int launch_explore(const float* points, const Bf16Copy* bf, const Bf16Copy* bf_j
             if (dispatch_merge(sl, 4, points, N, D, K, old_idx, knn_idx, knn_dist, small_table, dpad, pass, wave_bounds, order,
                                kSample, listA, listA + N, stat, nullptr, stream))
                 return 1;
-            RSFK_HIP(hipMemcpyAsync(host_n, listA + N, sizeof(int), hipMemcpyDeviceToHost, stream));
-            RSFK_HIP(hipStreamSynchronize(stream));
+            if (fetch_words(listA + N, 1, &n_back, stream)) return 1;
             first = kSample;
-            rest_per_wg = *host_n > kSample / 2;
+            rest_per_wg = n_back > kSample / 2;
         }
         if (rest_per_wg) {
             // everything but the sample straight to the workgroup-per-point kernel (its list: the rest of the order)
@@ -1172,9 +1171,8 @@ int launch_explore(const float* points, const Bf16Copy* bf, const Bf16Copy* bf_j
                                   first > 0 ? nullptr : order, stream)) {
             return 1;
         }
-        RSFK_HIP(hipMemcpyAsync(host_n, listA + N, sizeof(int), hipMemcpyDeviceToHost, stream));
-        RSFK_HIP(hipStreamSynchronize(stream));
-        n_todo = *host_n;                                 // what the small set handed back (of the sample, or of all points)
+        if (fetch_words(listA + N, 1, &n_back, stream)) return 1;
+        n_todo = n_back;                                 // what the small set handed back (of the sample, or of all points)
         todo = listA;
         if (n_todo == 0 && !rest_per_wg) return 0;
         if (second) {
@@ -1188,9 +1186,8 @@ int launch_explore(const float* points, const Bf16Copy* bf, const Bf16Copy* bf_j
                 rc = merge_wg(listA, n_todo);
             if (rc)
                 return 1;
-            RSFK_HIP(hipMemcpyAsync(host_n, listB + N, sizeof(int), hipMemcpyDeviceToHost, stream));
-            RSFK_HIP(hipStreamSynchronize(stream));
-            n_todo = *host_n;
+            if (fetch_words(listB + N, 1, &n_back, stream)) return 1;
+            n_todo = n_back;
             if (n_todo == 0) return 0;
             todo = listB;
         }

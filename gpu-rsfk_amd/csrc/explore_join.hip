@@ -62,7 +62,6 @@ struct ExploreWorkspace {
     int* fine_start = nullptr;  // the same + 1
     int* sub_off = nullptr;     // n_sub x fine bins per coarse bin
     int* todo = nullptr;       // two lists of N+1 ints: points left over by a launch; entry N = their number
-    int* host_count = nullptr; // pinned
 };
 namespace {
 
@@ -859,8 +858,7 @@ int explore_ws_alloc(ExploreWorkspace** out, int N, int K, bool with_bounds)
         dm(&w->offs, (size_t)N + 1) != hipSuccess || dm(&w->bin_size, (size_t)w->n_bins) != hipSuccess ||
         dm(&w->bin_start, (size_t)w->n_bins + 1) != hipSuccess ||
         dm(&w->part_off, (size_t)w->n_parts * (size_t)w->n_bins) != hipSuccess || dm(&w->pass, total * w->MW) != hipSuccess || dm(&w->norm_tau, 2 * (size_t)N) != hipSuccess ||
-        dm(&w->todo, 2 * ((size_t)N + 1)) != hipSuccess ||
-        pin_alloc(reinterpret_cast<void**>(&w->host_count), sizeof(int)) != 0) {
+        dm(&w->todo, 2 * ((size_t)N + 1)) != hipSuccess) {
         explore_ws_free(w);
         set_last_error("exploration workspace: out of device memory");
         return 1;
@@ -884,14 +882,12 @@ void explore_ws_free(ExploreWorkspace* w)
                     w->bin_eq2, w->fine_size, w->fine_start, w->sub_off};
     for (void* b : bufs)
         ws_free(b);
-    pin_free(w->host_count);
     delete w;
 }
 
 const uint32_t* explore_ws_pass(const ExploreWorkspace* w) { return w->pass; }
 const uint16_t* explore_ws_bounds(const ExploreWorkspace* w) { return w->bounds; }
 int* explore_ws_todo(ExploreWorkspace* w, int which) { return w->todo + (size_t)which * ((size_t)w->N + 1); }
-int* explore_ws_host_count(ExploreWorkspace* w) { return w->host_count; }
 
 // Fill pass (and bounds) from the snapshot old_idx and the current last slots of knn_dist (rows sorted by distance).
 int launch_explore_join(ExploreWorkspace* w, const Bf16Copy& bf, int N, int D, int K, const int* old_idx,

@@ -145,7 +145,6 @@ void explore_ws_free(ExploreWorkspace* w);
 const uint32_t* explore_ws_pass(const ExploreWorkspace* w);
 const uint16_t* explore_ws_bounds(const ExploreWorkspace* w);
 int* explore_ws_todo(ExploreWorkspace* w, int which);
-int* explore_ws_host_count(ExploreWorkspace* w);
 // order: null, or a permutation of the points that keeps nearby points together (the buckets of a tree): the points
 // are then worked on in that order, a contiguous eighth of it per die (die_local_place)
 int launch_explore_join(ExploreWorkspace* w, const Bf16Copy& bf, int N, int D, int K, const int* old_idx,

@@ -186,8 +186,7 @@ int symmetrize_device(const int* d_idx, const float* d_dist, int N, int K, int d
         RSFK_HIP(rocprim::exclusive_scan(tmp.p, tmp_bytes, static_cast<int*>(len.p), d_indptr, 0, (size_t)N + 1,
                                          rocprim::plus<int>(), stream));
         int total = 0;
-        RSFK_HIP(hipMemcpyAsync(&total, d_indptr + N, sizeof(int), hipMemcpyDeviceToHost, stream));
-        RSFK_HIP(hipStreamSynchronize(stream));
+        if (fetch_words(d_indptr + N, 1, &total, stream)) return 1;
         *nnz = total;
     }
     if (!d_cols || *nnz == 0) return 0;

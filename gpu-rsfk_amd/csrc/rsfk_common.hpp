@@ -26,6 +26,11 @@ void pin_free(void* p);
 int stream_take(hipStream_t* out);
 void stream_give(hipStream_t s);
 void host_pool_release();
+// Waits until a kernel queued on the stream has written `want` to *word (pinned host memory).
+int wait_for_word(const int* word, int want, hipStream_t stream);
+// A few words from the device, after everything queued on the stream.
+constexpr int kFetchMost = 8;
+int fetch_words(const int* dev, int n, int* host, hipStream_t stream);
 
 // Both macros leave the function on failure.  Work that was queued before may still be running and the
 // callers' guards hand their buffers back for reuse on the way out, so the device is drained first.
@@ -114,7 +119,7 @@ struct TreeNode {
     int buf;          // which of the two permutation buffers holds the members
     int leaf;         // 1 = already decided to be a bucket
     int rec;          // where the node is written in the index of the tree (only when an index is recorded)
-    int pad_;
+    int chunk0;       // first of its chunks at a wide level
     uint64_t key;
 };
 

@@ -38,6 +38,7 @@
 #include "tree_sweep.hpp"
 #include <vector>
 #include <algorithm>
+#include <atomic>
 #include <cstdlib>
 #include <cstring>
 #include <chrono>
@@ -49,17 +50,30 @@ namespace {
 constexpr int kBlock = 256;
 
 
+// Counters of a batch.  Those of the queue of level l are in entry l & 3, so that a level can be queued on the stream before
+// the one before it has run.
 struct LevelCounters {
-    int n_next;        // nodes appended for the next wide level
+    struct alignas(8) Queue {
+        int nodes;     // nodes of a wide level
+        int chunks;    // and their chunks
+    } queue[4];
     int n_tail;        // tail tasks appended so far
     int n_chain;       // nodes for the chain phase appended so far
-    int n_chunks;      // chunks of the current level (written by the scan kernel)
     int overflow;      // set when a queue capacity is exceeded
-    // time spent in the three steps of the wide levels (hyperplanes, side tests, scatter), in ticks of the device's
-    // constant-rate clock: the first thread of a kernel that opens a step closes the one before it
+    int pad_;
+    // time spent in the three steps of the wide levels (hyperplanes, side tests, scatter) and in the tail, in ticks of
+    // the device's constant-rate clock: the first thread of a kernel that opens a step closes the one before it
     long long last_tick;
-    long long phase_ticks[3];
+    long long phase_ticks[4];
 };
+
+// What a level tells the host, in pinned memory: its counts, and seq, written last.
+struct LevelNote {
+    int n_nodes, n_chunks, n_tail, overflow;
+    int seq;
+    int pad_[11];
+};
+constexpr int kNotes = 8;               // level l writes note l & 7
 
 // Counts for the report of a build (how many points the side tests of all levels looked at, and how many of them
 // the screen left to the exact test): kStatSlots slots a cache line apart, so that the workgroups' additions do not
@@ -308,30 +322,58 @@ __device__ __forceinline__ void resolve_exact(int halves, int h, const int* list
 constexpr int kSideBatch = 4;        // points per group and call of the screen in the wide phase
 constexpr int kTailBatch = 2;        // ... in the tail kernel
 
-// The queues nodes go to: the next wide level and the tail kernel (one workgroup per node).
+// The queues nodes go to: the next wide level (entry `slot` of the counters) and the tail kernel (one workgroup per node).
 struct NodeQueues {
     TreeNode* next;
-    int next_cap;
+    int next_cap, chunk_cap, slot;
     TreeNode* tail;
     int tail_cap;
     LevelCounters* ctr;
 };
 
-// Append a child node to its queue.  Returns its place in the queue of the next wide level, or -1.
-__device__ __forceinline__ int emit_node(const TreeNode& c, const TreeParams& P, const NodeQueues& Q)
+// Append the nc children of a node to their queues; a node of the next wide level is given its chunks too.  at[i]: place
+// of child i in the queue of the next wide level, or -1.  (All workgroups of a level add to the same few words, one
+// after the other: a queue is one addition for both children, and for its nodes and chunks together.)
+__device__ __forceinline__ void emit_children(const TreeNode (&c)[2], int nc, const TreeParams& P, const NodeQueues& Q, int (&at)[2])
 {
-    const bool forced = c.depth >= P.MAX_DEPTH - 1;
-    if (!c.leaf && !forced && c.count > P.small) {
-        const int at = atomicAdd(&Q.ctr->n_next, 1);
-        if (at < Q.next_cap) { Q.next[at] = c; return at; }
-        Q.ctr->overflow = 1;
-        return -1;
+    bool wide[2], forced[2];
+    int chunks[2], n_wide = 0, n_chunks = 0, n_tail = 0;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        forced[i] = c[i].depth >= P.MAX_DEPTH - 1;
+        wide[i] = i < nc && !c[i].leaf && !forced[i] && c[i].count > P.small;
+        chunks[i] = wide[i] ? (c[i].count + P.chunk - 1) / P.chunk : 0;
+        n_wide += wide[i] ? 1 : 0;
+        n_chunks += chunks[i];
+        n_tail += i < nc && !wide[i] ? 1 : 0;
+        at[i] = -1;
     }
-    TreeNode t = c;
-    if (forced) t.leaf = 1;
-    const int at = atomicAdd(&Q.ctr->n_tail, 1);
-    if (at < Q.tail_cap) Q.tail[at] = t; else Q.ctr->overflow = 1;
-    return -1;
+    int next = 0, chunk = 0, tail = 0;
+    if (n_wide) {
+        const unsigned long long was = atomicAdd(reinterpret_cast<unsigned long long*>(&Q.ctr->queue[Q.slot]),
+                                                 (unsigned long long)(unsigned)n_wide | ((unsigned long long)(unsigned)n_chunks << 32));
+        next = (int)(unsigned)was;
+        chunk = (int)(unsigned)(was >> 32);
+    }
+    if (n_tail) tail = atomicAdd(&Q.ctr->n_tail, n_tail);
+    if ((n_wide && (next + n_wide > Q.next_cap || chunk + n_chunks > Q.chunk_cap)) || (n_tail && tail + n_tail > Q.tail_cap)) {
+        Q.ctr->overflow = 1;
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        if (i >= nc) continue;
+        TreeNode t = c[i];
+        if (wide[i]) {
+            t.chunk0 = chunk;
+            chunk += chunks[i];
+            at[i] = next;
+            Q.next[next++] = t;
+        } else {
+            if (forced[i]) t.leaf = 1;
+            Q.tail[tail++] = t;
+        }
+    }
 }
 
 // The split / min-size-merge / leaf rules for a node whose left side has `a`
@@ -346,7 +388,7 @@ __device__ __forceinline__ int split_rules(const TreeNode& nd, int a, int MIN, i
     c0.depth = c1.depth = nd.depth + 1;
     c0.buf = c1.buf = child_buf;
     c0.rec = c1.rec = 0;
-    c0.pad_ = c1.pad_ = 0;
+    c0.chunk0 = c1.chunk0 = 0;
     if (a == 0 || r == 0) {
         c0.start = nd.start; c0.count = nd.count; c0.dstart = nd.start; c0.dcount = nd.count;
         c0.key = a ? kl : kr; c0.leaf = nd.count <= MAX - 2;
@@ -405,103 +447,74 @@ __device__ __forceinline__ void index_bucket(TreeRec* recs, int rec_cap, int my_
 // wide phase kernels
 // ---------------------------------------------------------------------------
 
-__global__ void k_init_perm(int* __restrict__ perm, int N, int B)
-{
-    const size_t total = (size_t)N * (size_t)B;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (size_t)gridDim.x * blockDim.x)
-        perm[i] = (int)(i % (size_t)N);
-}
+struct TreeStats {          // one per tree of the batch
+    int n_leaves;           // buckets of at most kBucketSplit points, stored from the front of the leaf table
+    int n_big;              // larger buckets, stored from the back of the leaf table
+    int levels;
+    int max_leaf;
+    int min_leaf;
+};
 
-__global__ void k_init_roots(NodeQueues Q, TreeParams P, int B, int seed0, int* n_rec, int* pmap)
+// A batch begins: permutations, counters, and the root of every tree (workgroup 0).
+__global__ __launch_bounds__(256) void k_tree_init(int* __restrict__ perm, NodeQueues Q, TreeParams P, int B, int seed0, int* n_rec, int* pmap,
+                                                   TreeStats* __restrict__ stats, unsigned long long* __restrict__ stat)
 {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    const size_t total = (size_t)P.N * (size_t)B;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (size_t)gridDim.x * blockDim.x)
+        perm[i] = (int)(i % (size_t)P.N);
+    if (blockIdx.x != 0) return;
+    for (int i = threadIdx.x; i < (int)(sizeof(LevelCounters) / sizeof(int)); i += 256) reinterpret_cast<int*>(Q.ctr)[i] = 0;
+    for (int i = threadIdx.x; i < kStatSlots * kStatPitch; i += 256) stat[i] = 0ull;
+    __threadfence();
+    __syncthreads();
+    const int t = threadIdx.x;
     if (t >= B) return;
+    TreeStats s;
+    s.n_leaves = 0; s.n_big = 0; s.levels = 0; s.max_leaf = 0; s.min_leaf = 0x7fffffff;
+    stats[t] = s;
     if (n_rec) n_rec[t] = 1;               // record 0 is the root
     TreeNode r;
     r.tree = t; r.start = 0; r.count = P.N; r.dstart = 0; r.dcount = P.N; r.depth = 0; r.buf = 0; r.leaf = 0;
-    r.rec = 0; r.pad_ = 0;
+    r.rec = 0; r.chunk0 = 0;
     r.key = root_key(seed0 + t);
     // the root is never a leaf (src/kernels/build_tree_init.cu:79) unless the depth limit forces it
-    const int at = emit_node(r, P, Q);
-    if (pmap) pmap[t * pm::kPaths] = at;      // path 0 of level 0 = the root, if it is split at all
+    const TreeNode c[2] = {r, r};
+    int at[2];
+    emit_children(c, 1, P, Q, at);
+    if (pmap) pmap[t * pm::kPaths] = at[0];      // path 0 of level 0 = the root, if it is split at all
 }
 
-// chunk_base[i] = number of chunks of nodes [0,i); one workgroup.
-__global__ __launch_bounds__(1024) void k_scan_chunks(const TreeNode* __restrict__ nodes, int node_cap, int chunk,
-                                                      int* __restrict__ chunk_base, LevelCounters* ctr,
-                                                      unsigned long long* __restrict__ stat)
-{
-    __shared__ int wsum[16];
-    __shared__ int carry_s;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int n_nodes = min(ctr->n_next, node_cap);       // nodes of the level, left by the previous level's scatter
-    if (tid == 0) {
-        carry_s = 0;
-        phase_tick(ctr, 2);
-    }
-    __syncthreads();
-    int members = 0;                                      // points of the nodes this thread looked at
-    for (int base = 0; base < n_nodes; base += 1024) {
-        const int i = base + tid;
-        const int cnt_i = i < n_nodes ? nodes[i].count : 0;
-        members += cnt_i;
-        const int v = (cnt_i + chunk - 1) / chunk;
-        // inclusive scan inside the wavefront
-        int x = v;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int y = __shfl_up(x, o, 64);
-            if (lane >= o) x += y;
-        }
-        if (lane == 63) wsum[wave] = x;
-        __syncthreads();
-        int woff = 0;
-        for (int w = 0; w < wave; ++w) woff += wsum[w];
-        const int carry = carry_s;
-        if (i < n_nodes) chunk_base[i] = carry + woff + x - v;
-        __syncthreads();
-        if (tid == 1023) carry_s = carry + woff + x;
-        __syncthreads();
-    }
-    if (tid == 0) { chunk_base[n_nodes] = carry_s; ctr->n_chunks = carry_s; }
-    members = wave_sum_i(members);
-    if (lane == 0) stat_add(stat, wave, 0, members);
-}
-
-// (also empties the queue of the level being produced, which the scatter kernel of this level fills)
-__global__ void k_fill_chunks(const int* __restrict__ chunk_base, int n_nodes, int n_chunks, int* __restrict__ chunk2node,
-                              LevelCounters* ctr)
-{
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c == 0) {
-        phase_tick(ctr, 0);
-        ctr->n_next = 0;
-    }
-    if (c >= n_chunks) return;
-    int lo = 0, hi = n_nodes - 1;          // last node with chunk_base <= c
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (chunk_base[mid] <= c) lo = mid; else hi = mid - 1;
-    }
-    chunk2node[c] = lo;
-}
-
-// Hyperplanes of the nodes of a wide level, one wavefront per node: record ni of the table is
-// [offset, bound of the 1-norm, sum of the components, 0 | normal, nvec_len(D) floats].  The workgroups of a node
-// (one per chunk, up to a thousand at the first levels) fetch the record instead of each making the hyperplane again.
+// A wide level begins: hyperplanes of its nodes, one wavefront per node -- record ni of the table is
+// [offset, bound of the 1-norm, sum of the components, 0 | normal, nvec_len(D) floats]; the workgroups of a node (one per
+// chunk, up to a thousand at the first levels) fetch the record instead of each making the hyperplane again --, the
+// chunks of the nodes, and the level's counts for the host, which has queued this level from bounds on them.
 __global__ __launch_bounds__(256) void k_level_planes(const float* __restrict__ points, TreeParams P,
                                                       const int* __restrict__ perm0, const int* __restrict__ perm1,
-                                                      const TreeNode* __restrict__ nodes, int n_nodes,
-                                                      float* __restrict__ table, LevelCounters* ctr)
+                                                      const TreeNode* __restrict__ nodes, int level, int node_cap,
+                                                      float* __restrict__ table, int* __restrict__ chunk2node, LevelCounters* ctr,
+                                                      unsigned long long* __restrict__ stat, LevelNote* note, int seq)
 {
     extern __shared__ __align__(16) float lds_p[];          // per wavefront: 4 + nvec_len(D) floats
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    if (blockIdx.x == 0 && threadIdx.x == 0) phase_tick(ctr, -1);
+    const int n_nodes = min(ctr->queue[level & 3].nodes, node_cap);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        phase_tick(ctr, 2);
+        ctr->queue[(level + 1) & 3].nodes = 0;                   // (of the level before the last two: nobody needs it any more)
+        const int n_chunks = ctr->queue[level & 3].chunks;
+        ctr->queue[(level + 1) & 3].chunks = 0;
+        note->n_nodes = n_nodes;
+        note->n_chunks = n_chunks;
+        note->n_tail = ctr->n_tail;
+        note->overflow = ctr->overflow;
+        __hip_atomic_store(&note->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
     const int ni = blockIdx.x * (blockDim.x >> 6) + wave;
     if (ni >= n_nodes) return;
     const int rec = 4 + nvec_len(P.D);
     float* mine = lds_p + (size_t)wave * rec;
     const TreeNode nd = nodes[ni];
+    for (int k = lane; k * P.chunk < nd.count; k += 64) chunk2node[nd.chunk0 + k] = ni;
+    if (lane == 0) stat_add(stat, ni, 0, nd.count);
     const int* perm = (nd.buf ? perm1 : perm0) + (size_t)nd.tree * (size_t)P.N;
     int r1, r2;
     pick_pair(nd.key, nd.dcount, r1, r2);
@@ -521,7 +534,7 @@ __global__ __launch_bounds__(kBlock) void k_side(const float* __restrict__ point
                                                  const uint16_t* __restrict__ pb16, const uint8_t* __restrict__ q8,
                                                  TreeParams P,
                                                  int* __restrict__ perm0, int* __restrict__ perm1,
-                                                 const TreeNode* __restrict__ nodes, const int* __restrict__ chunk_base,
+                                                 const TreeNode* __restrict__ nodes, int slot, LevelCounters* ctr,
                                                  const int* __restrict__ chunk2node, int* __restrict__ chunk_left,
                                                  const float* __restrict__ planes, unsigned long long* __restrict__ stat)
 {
@@ -531,9 +544,11 @@ __global__ __launch_bounds__(kBlock) void k_side(const float* __restrict__ point
     __shared__ int left_s, n_def_s;
     __shared__ int deferred[1024];                          // points of the chunk left to the exact test (chunk <= 1024)
     const int c = blockIdx.x;
+    if (c >= ctr->queue[slot].chunks) return;
+    if (c == 0 && threadIdx.x == 0) phase_tick(ctr, 0);
     const int ni = chunk2node[c];
     const TreeNode nd = nodes[ni];
-    const int k = c - chunk_base[ni];
+    const int k = c - nd.chunk0;
     int* perm = (nd.buf ? perm1 : perm0) + (size_t)nd.tree * (size_t)P.N;
     if (threadIdx.x == 0) { left_s = 0; n_def_s = 0; }
     {
@@ -595,7 +610,7 @@ __global__ __launch_bounds__(kBlock) void k_side(const float* __restrict__ point
 // Stable scatter of one chunk into the other permutation buffer; the workgroup
 // of chunk 0 also applies the split rules and appends the children.
 __global__ __launch_bounds__(kBlock) void k_scatter(TreeParams P, int* __restrict__ perm0, int* __restrict__ perm1,
-                                                    const TreeNode* __restrict__ nodes, const int* __restrict__ chunk_base,
+                                                    const TreeNode* __restrict__ nodes, int slot,
                                                     const int* __restrict__ chunk2node, const int* __restrict__ chunk_left,
                                                     NodeQueues Q, TreeRec* __restrict__ recs, int* __restrict__ n_rec,
                                                     int rec_cap, int2* __restrict__ child)
@@ -603,11 +618,12 @@ __global__ __launch_bounds__(kBlock) void k_scatter(TreeParams P, int* __restric
     LevelCounters* ctr = Q.ctr;
     __shared__ int red[2][kBlock / 64];
     const int c = blockIdx.x;
+    if (c >= ctr->queue[slot].chunks) return;
     if (c == 0 && threadIdx.x == 0) phase_tick(ctr, 1);
     const int ni = chunk2node[c];
     const TreeNode nd = nodes[ni];
-    const int first = chunk_base[ni];
-    const int nch = chunk_base[ni + 1] - first;
+    const int first = nd.chunk0;
+    const int nch = (nd.count + P.chunk - 1) / P.chunk;
     const int k = c - first;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
 
@@ -676,33 +692,34 @@ __global__ __launch_bounds__(kBlock) void k_scatter(TreeParams P, int* __restric
         __syncthreads();
     }
     if (k == 0 && tid == 0) {
-        TreeNode c0, c1;
-        const int nc = split_rules(nd, all, P.MIN, P.MAX, nd.buf ^ 1, c0, c1);
+        TreeNode c[2];
+        const int nc = split_rules(nd, all, P.MIN, P.MAX, nd.buf ^ 1, c[0], c[1]);
         if (recs) {
             int r1, r2;
             pick_pair(nd.key, nd.dcount, r1, r2);
             index_split(recs + (size_t)nd.tree * rec_cap, n_rec + nd.tree, rec_cap, nd.rec, src[nd.dstart + r1] & kIdMask,
-                        src[nd.dstart + r2] & kIdMask, nc, c0.rec, c1.rec, ctr);
+                        src[nd.dstart + r2] & kIdMask, nc, c[0].rec, c[1].rec, ctr);
         }
-        const int at0 = emit_node(c0, P, Q);
-        const int at1 = nc == 2 ? emit_node(c1, P, Q) : at0;
+        int at[2];
+        emit_children(c, nc, P, Q, at);
         // where the members of either side are at the next level (a node with one child keeps them together)
-        if (child) child[ni] = make_int2(at0, at1);
+        if (child) child[ni] = make_int2(at[0], nc == 2 ? at[1] : at[0]);
     }
 }
 
 // What k_side leaves behind, from sides that are already known (one bit per point of the tree, pm::k_pm_sweep and
 // pm::k_pm_resolve): bit 31 of the permutation entries of a chunk and the number of its left members.
 __global__ __launch_bounds__(kBlock) void k_pm_mark(TreeParams P, int* __restrict__ perm0, int* __restrict__ perm1,
-                                                    const TreeNode* __restrict__ nodes, const int* __restrict__ chunk_base,
+                                                    const TreeNode* __restrict__ nodes, const int* __restrict__ n_chunks,
                                                     const int* __restrict__ chunk2node, int* __restrict__ chunk_left,
                                                     const uint32_t* __restrict__ sidebits, int W)
 {
     __shared__ int part[kBlock / 64];
     const int c = blockIdx.x;
+    if (c >= *n_chunks) return;
     const int ni = chunk2node[c];
     const TreeNode nd = nodes[ni];
-    const int k = c - chunk_base[ni];
+    const int k = c - nd.chunk0;
     int* perm = (nd.buf ? perm1 : perm0) + (size_t)nd.tree * (size_t)P.N;
     const uint32_t* bits = sidebits + (size_t)nd.tree * (size_t)W;
     const int pos0 = nd.start + k * P.chunk;
@@ -748,14 +765,6 @@ struct SmallNode {
     int rec;                              // record of the node in the index of the tree, if one is written
     int vain;                             // splits in a row that left all points together (chain phase)
     uint64_t key;
-};
-
-struct TreeStats {          // one per tree of the batch
-    int n_leaves;           // buckets of at most kBucketSplit points, stored from the front of the leaf table
-    int n_big;              // larger buckets, stored from the back of the leaf table
-    int levels;
-    int max_leaf;
-    int min_leaf;
 };
 
 // Entry of the leaf table that the `at`-th bucket of its kind takes: small buckets fill the table of the tree from the
@@ -827,6 +836,7 @@ __global__ __launch_bounds__(TB) void k_tail(const float* __restrict__ points,
 
     const int task = blockIdx.x;
     if (task >= n_tasks) return;
+    if (task == 0 && threadIdx.x == 0) phase_tick(ctr, 2);
     const TreeNode tk = tasks[task];
     const size_t toff = (size_t)tk.tree * (size_t)P.N;
     const int* src = (tk.buf ? perm1 : perm0) + toff;
@@ -1008,7 +1018,7 @@ __global__ __launch_bounds__(TB) void k_tail(const float* __restrict__ points,
         const SmallNode sn = chain[i];
         TreeNode c;
         c.tree = tk.tree; c.start = tk.start + sn.start; c.count = sn.count; c.dstart = tk.start + sn.dstart; c.dcount = sn.dcount;
-        c.depth = sn.depth; c.buf = 0; c.leaf = 0; c.rec = sn.rec; c.pad_ = 0; c.key = sn.key;
+        c.depth = sn.depth; c.buf = 0; c.leaf = 0; c.rec = sn.rec; c.chunk0 = 0; c.key = sn.key;
         const int at = chain_base_s + i;
         if (at < chain_cap) chain_all[at] = c; else ctr->overflow = 1;
     }
@@ -1329,7 +1339,7 @@ __global__ __launch_bounds__(256) void k_chain(const float* __restrict__ points,
             // children: the first one that is no bucket is next, another waits on the stack
             TreeNode full, c[2];
             full.tree = tk.tree; full.start = start; full.count = count; full.dstart = dstart; full.dcount = dcount;
-            full.depth = depth; full.buf = 0; full.leaf = 0; full.rec = rec; full.pad_ = 0; full.key = draws.node_key();
+            full.depth = depth; full.buf = 0; full.leaf = 0; full.rec = rec; full.chunk0 = 0; full.key = draws.node_key();
             const int nc = split_rules(full, a, P.MIN, P.MAX, 0, c[0], c[1]);
             if (recs) {
                 if (lane == 0) index_split(recs, n_rec, rec_cap, rec, ids[o1], ids[o2], nc, c[0].rec, c[1].rec, ctr);
@@ -1409,6 +1419,38 @@ __global__ __launch_bounds__(256) void k_chain(const float* __restrict__ points,
     }
 }
 
+// What a batch tells the host at its end, in pinned memory.
+struct BatchReport {
+    TreeStats stats[64];
+    long long phase_ticks[4];
+    unsigned long long counts[2];
+    int overflow;
+    int seq;
+};
+
+__global__ __launch_bounds__(64) void k_tree_report(const TreeStats* __restrict__ stats, int nb, LevelCounters* ctr,
+                                                    const unsigned long long* __restrict__ stat, BatchReport* out, int seq)
+{
+    const int lane = threadIdx.x;
+    if (lane == 0) phase_tick(ctr, 3);
+    if (lane < nb) out->stats[lane] = stats[lane];
+    static_assert(kStatSlots == 64, "one slot per lane");
+    unsigned long long a = stat[kStatPitch * lane], b = stat[kStatPitch * lane + 1];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        a += __shfl_xor(a, o, 64);
+        b += __shfl_xor(b, o, 64);
+    }
+    if (lane < 4) out->phase_ticks[lane] = ctr->phase_ticks[lane];
+    if (lane == 0) {
+        out->counts[0] = a;
+        out->counts[1] = b;
+        out->overflow = ctr->overflow;
+    }
+    __threadfence_system();
+    if (lane == 0) __hip_atomic_store(&out->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 template <typename T>
 int dmalloc(T** p, size_t n)
 {
@@ -1427,7 +1469,6 @@ struct TreeBatchWorkspace {
     TreeNode* nodes[2] = {nullptr, nullptr};
     TreeNode* tail = nullptr;
     TreeNode* chain = nullptr;           // nodes for the chain phase
-    int* chunk_base = nullptr;
     int* chunk2node = nullptr;
     int* chunk_left = nullptr;
     float* planes = nullptr;             // hyperplanes of the nodes of the current wide level: node_cap x (4 + nvec_len(D))
@@ -1436,17 +1477,14 @@ struct TreeBatchWorkspace {
     TreeStats* stats = nullptr;
     LevelCounters* ctr = nullptr;
     int D = 0;
-    LevelCounters* h_ctr = nullptr;      // pinned
-    TreeStats* h_stats = nullptr;        // pinned
+    LevelNote* notes = nullptr;          // pinned, kNotes
+    BatchReport* h_report = nullptr;     // pinned
     unsigned long long* stat = nullptr;  // kStatSlots x kStatPitch: counts for the report (stat_add)
-    unsigned long long* h_stat = nullptr;        // pinned
     unsigned long long counts[2] = {0, 0};       // of the last batch: points the side tests looked at, undecided ones
     // index of the trees for routing query points (allocated by tree_ws_enable_index)
     TreeRec* recs = nullptr;             // B x rec_cap
     int* n_rec = nullptr;                // B
     int rec_cap = 0;
-    // events around the kernels of a wide level (hyperplanes | side test | scatter) and around the tail kernel
-    hipEvent_t ev[2] = {nullptr, nullptr};          // around the tail kernel
     float phase_s[4] = {0.f, 0.f, 0.f, 0.f};   // of the last batch: side tests, hyperplanes, scatter, tail kernel
     // side tests of the first levels taken point by point (tree_sweep.hpp); allocated when D allows it
     int pm_ks = 0;                       // 32-dimension steps of a row as matrix-core operands (1, 2, 4, 8), 0 = not available
@@ -1463,15 +1501,12 @@ struct TreeBatchWorkspace {
 
 static void free_ws(TreeBatchWorkspace& w)
 {
-    void* dev[] = {w.perm[0], w.perm[1], w.nodes[0], w.nodes[1], w.tail, w.chain, w.chunk_base, w.chunk2node,
+    void* dev[] = {w.perm[0], w.perm[1], w.nodes[0], w.nodes[1], w.tail, w.chain, w.chunk2node,
                    w.chunk_left, w.leaf_start, w.leaf_size, w.stats, w.ctr, w.recs, w.n_rec, w.planes,
                    w.pm_path, w.pm_side, w.pm_undec, w.pm_map[0], w.pm_map[1], w.pm_sc, w.pm_aq, w.pm_child, w.stat};
     for (void* p : dev) ws_free(p);
-    pin_free(w.h_ctr);
-    pin_free(w.h_stat);
-    pin_free(w.h_stats);
-    for (hipEvent_t e : w.ev)
-        if (e) (void)hipEventDestroy(e);
+    pin_free(w.notes);
+    pin_free(w.h_report);
     w = TreeBatchWorkspace();
 }
 
@@ -1560,7 +1595,6 @@ int tree_ws_alloc(TreeBatchWorkspace** out, int N, int D, int MIN, int B)
     if (dmalloc(&w->nodes[1], (size_t)w->node_cap)) return 1;
     if (dmalloc(&w->tail, (size_t)w->tail_cap)) return 1;
     if (dmalloc(&w->chain, (size_t)w->tail_cap)) return 1;
-    if (dmalloc(&w->chunk_base, (size_t)w->node_cap + 1)) return 1;
     if (dmalloc(&w->chunk2node, (size_t)w->chunk_cap)) return 1;
     if (dmalloc(&w->chunk_left, (size_t)w->chunk_cap)) return 1;
     if (dmalloc(&w->planes, (size_t)w->node_cap * (size_t)(4 + nvec_len(D)))) return 1;
@@ -1582,10 +1616,8 @@ int tree_ws_alloc(TreeBatchWorkspace** out, int N, int D, int MIN, int B)
         if (dmalloc(&w->pm_aq, (size_t)B * pm::kMaxGroups * 32 * 32 * w->pm_ks)) return 1;
         if (dmalloc(&w->pm_child, (size_t)w->node_cap)) return 1;
     }
-    if (pin_alloc(reinterpret_cast<void**>(&w->h_ctr), sizeof(LevelCounters))) return 1;
-    if (pin_alloc(reinterpret_cast<void**>(&w->h_stats), sizeof(TreeStats) * (size_t)B)) return 1;
-    if (pin_alloc(reinterpret_cast<void**>(&w->h_stat), sizeof(unsigned long long) * kStatSlots * kStatPitch)) return 1;
-    for (hipEvent_t& e : w->ev) RSFK_HIP(hipEventCreate(&e));
+    if (pin_alloc(reinterpret_cast<void**>(&w->notes), sizeof(LevelNote) * kNotes)) return 1;
+    if (pin_alloc(reinterpret_cast<void**>(&w->h_report), sizeof(BatchReport))) return 1;
     return 0;
 }
 
@@ -1618,31 +1650,29 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
     // tree) and of the exact test (D/32 terms per lane and a 5-step tree), 1 % on top
     P.band = 1.01f * ((1.0f + 1.0f / 128.0f) / 256.0f + (float)(D / 8 + D / 32 + 16) / 16777216.0f);
 
-    {
-        const size_t total = (size_t)N * nb;
-        const int grid = (int)std::min<size_t>((total + 255) / 256, 65536);
-        hipLaunchKernelGGL(k_init_perm, dim3(grid), dim3(256), 0, stream, w->perm[0], N, nb);
-    }
-    std::vector<TreeStats> init((size_t)nb);
-    for (auto& s : init) { s.n_leaves = 0; s.n_big = 0; s.levels = 0; s.max_leaf = 0; s.min_leaf = 0x7fffffff; }
-    std::memcpy(w->h_stats, init.data(), sizeof(TreeStats) * (size_t)nb);
-    RSFK_HIP(hipMemcpyAsync(w->stats, w->h_stats, sizeof(TreeStats) * (size_t)nb, hipMemcpyHostToDevice, stream));
-    RSFK_HIP(hipMemsetAsync(w->ctr, 0, sizeof(LevelCounters), stream));
-    RSFK_HIP(hipMemsetAsync(w->stat, 0, sizeof(unsigned long long) * kStatSlots * kStatPitch, stream));
+    RSFK_CHECK(nb <= 64, "tree batch: at most 64 trees at a time");
     // Levels whose side tests are taken point by point (needs the 8-bit copy).  RSFK_PM_LEVELS overrides (0 = none).
     // The sweep multiplies every tile of points with every block of 16 hyperplanes of a tree, so its cost doubles
-    // per level from the fifth on; measured, the seventh level is the last one it takes faster than k_side.
+    // per level from the fifth on; measured, the seventh level is the last one it takes faster than k_side.  Batches of
+    // less than 2^22 points do not fill the device either way, and k_side is one launch instead of four.
     int pm_levels = 0;
     if (q8 && w->pm_ks) {
-        pm_levels = pm::kMaxLevels - 1;
+        pm_levels = (size_t)N * (size_t)nb >= ((size_t)1 << 22) ? pm::kMaxLevels - 1 : 0;
         if (const char* e = std::getenv("RSFK_PM_LEVELS")) pm_levels = std::max(0, std::min(pm::kMaxLevels, std::atoi(e)));
     }
     NodeQueues Q;
-    Q.next = w->nodes[0]; Q.next_cap = w->node_cap;
+    Q.next = w->nodes[0]; Q.next_cap = w->node_cap; Q.chunk_cap = w->chunk_cap; Q.slot = 0;
     Q.tail = w->tail; Q.tail_cap = w->tail_cap;
     Q.ctr = w->ctr;
-    hipLaunchKernelGGL(k_init_roots, dim3((nb + 63) / 64), dim3(64), 0, stream, Q, P, nb, seed0, w->n_rec, pm_levels > 0 ? w->pm_map[0] : nullptr);
-    RSFK_HIP(hipGetLastError());
+    {
+        const size_t total = (size_t)N * nb;
+        const int grid = (int)std::min<size_t>((total + 255) / 256, 65536);
+        hipLaunchKernelGGL(k_tree_init, dim3(grid), dim3(256), 0, stream, w->perm[0], Q, P, nb, seed0, w->n_rec,
+                           pm_levels > 0 ? w->pm_map[0] : nullptr, w->stats, w->stat);
+        RSFK_HIP(hipGetLastError());
+    }
+    static std::atomic<int> batches{0};
+    const int seq0 = (batches.fetch_add(1) & 0x3ffff) * 8192 + 1;          // notes of an earlier batch never look like this one's
 
     int cur = 0;
     const size_t side_lds = (size_t)(4 + nvec_len(D)) * sizeof(float);
@@ -1661,34 +1691,32 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
         }
     }
     for (float& v : w->phase_s) v = 0.0f;
-    // wide levels
-    int level = 0;
-    while (true) {
-        // one trip to the host per level: the chunk table of the level is made first (from the node count on the
-        // device), then both counts come back together
-        hipLaunchKernelGGL(k_scan_chunks, dim3(1), dim3(1024), 0, stream, w->nodes[cur], w->node_cap, P.chunk, w->chunk_base, w->ctr,
-                           w->stat);
-        RSFK_HIP(hipMemcpyAsync(w->h_ctr, w->ctr, sizeof(LevelCounters), hipMemcpyDeviceToHost, stream));
-        RSFK_HIP(hipStreamSynchronize(stream));
-        RSFK_CHECK(!w->h_ctr->overflow, "tree batch: node queue overflow");
-        const int n_nodes = w->h_ctr->n_next;
-        if (std::getenv("RSFK_TREE_TRACE")) {
-            static double t_prev = 0.0;
-            const double t_now = std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch()).count();
-            std::fprintf(stderr, "level %d: %d nodes, %d chunks, tail %d, previous level %.3f ms\n", level, n_nodes,
-                         w->h_ctr->n_chunks, w->h_ctr->n_tail, level ? (t_now - t_prev) * 1e3 : 0.0);
-            t_prev = t_now;
+    // Wide levels.  A level is three launches over bounds on its counts, which follow from the counts of the level before:
+    // the host reads those from pinned memory while the level before runs, so the stream never waits for the host (a copy
+    // and a synchronisation per level took 14 us, and the table of chunks two launches more).  One level too many is
+    // queued at the end; its workgroups find nothing to do.
+    int n_tail = nb, level = 0;
+    size_t most_nodes = (size_t)nb, most_chunks = (size_t)nb * (((size_t)N + P.chunk - 1) / P.chunk);
+    while (N > P.small) {
+        if (level > 0) {
+            LevelNote* note = w->notes + ((level - 1) & (kNotes - 1));
+            if (wait_for_word(&note->seq, seq0 + ((level - 1) & 8191), stream)) return 1;
+            RSFK_CHECK(!note->overflow && note->n_nodes <= w->node_cap && note->n_chunks <= w->chunk_cap,
+                       "tree batch: node queue overflow");
+            n_tail = note->n_tail;
+            if (std::getenv("RSFK_TREE_TRACE"))
+                std::fprintf(stderr, "level %d: %d nodes, %d chunks, tail %d\n", level - 1, note->n_nodes, note->n_chunks, note->n_tail);
+            if (note->n_nodes == 0) break;
+            // a split makes two nodes of one and adds at most one chunk
+            most_nodes = std::min<size_t>(2 * (size_t)note->n_nodes, (size_t)w->node_cap);
+            most_chunks = std::min<size_t>((size_t)note->n_chunks + (size_t)note->n_nodes, (size_t)w->chunk_cap);
         }
-        if (n_nodes == 0) break;
-        RSFK_CHECK(n_nodes <= w->node_cap, "tree batch: node queue overflow");
-        const int n_chunks = w->h_ctr->n_chunks;
-        RSFK_CHECK(n_chunks <= w->chunk_cap, "tree batch: chunk table overflow");
-        hipLaunchKernelGGL(k_level_planes, dim3((unsigned)((n_nodes + plane_waves - 1) / plane_waves)), dim3(64 * plane_waves),
-                           plane_waves * side_lds, stream, points, P, w->perm[0], w->perm[1], w->nodes[cur], n_nodes, w->planes,
-                           w->ctr);
-        // (also sets n_next := 0 for the level being produced)
-        hipLaunchKernelGGL(k_fill_chunks, dim3((n_chunks + 255) / 256), dim3(256), 0, stream, w->chunk_base, n_nodes, n_chunks,
-                           w->chunk2node, w->ctr);
+        const int slot = level & 3;
+        const int n_chunks = (int)std::min<size_t>(most_chunks, (size_t)w->chunk_cap);
+        int* ctr_chunks = &w->ctr->queue[slot].chunks;
+        hipLaunchKernelGGL(k_level_planes, dim3((unsigned)((most_nodes + plane_waves - 1) / plane_waves)), dim3(64 * plane_waves),
+                           plane_waves * side_lds, stream, points, P, w->perm[0], w->perm[1], w->nodes[cur], level, w->node_cap,
+                           w->planes, w->chunk2node, w->ctr, w->stat, w->notes + (level & (kNotes - 1)), seq0 + (level & 8191));
         const bool swept = level < pm_levels;
         if (swept) {
             // the sides of every point in all trees of the batch, then their marks in the permutations
@@ -1709,13 +1737,13 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
             hipLaunchKernelGGL(pm::k_pm_resolve, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, stream, points, D, W,
                                w->pm_Bs, words, w->pm_path, w->pm_sc, w->planes, rec, w->pm_side, w->pm_undec, w->stat);
             hipLaunchKernelGGL(k_pm_mark, dim3(n_chunks), dim3(kBlock), 0, stream, P, w->perm[0], w->perm[1], w->nodes[cur],
-                               w->chunk_base, w->chunk2node, w->chunk_left, w->pm_side, W);
+                               ctr_chunks, w->chunk2node, w->chunk_left, w->pm_side, W);
         } else {
         // lanes per point in the 8-bit screen: a lane takes 16 coordinates per step
         const int q8_pieces = q8_padded(D) >> 4;
 #define RSFK_SIDE_LAUNCH(Q, L)                                                                                              \
         hipLaunchKernelGGL((k_side<Q, L>), dim3(n_chunks), dim3(kBlock), side_lds, stream, points, pb16, q8, P, w->perm[0],    \
-                           w->perm[1], w->nodes[cur], w->chunk_base, w->chunk2node, w->chunk_left, w->planes, w->stat)
+                           w->perm[1], w->nodes[cur], slot, w->ctr, w->chunk2node, w->chunk_left, w->planes, w->stat)
         if (!q8) RSFK_SIDE_LAUNCH(false, 8);
         else if (q8_pieces <= 2) RSFK_SIDE_LAUNCH(true, 2);
         else if (q8_pieces <= 4) RSFK_SIDE_LAUNCH(true, 4);
@@ -1724,8 +1752,9 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
         }
         const bool map_next = level + 1 < pm_levels;
         Q.next = w->nodes[cur ^ 1];
+        Q.slot = (level + 1) & 3;
         hipLaunchKernelGGL(k_scatter, dim3(n_chunks), dim3(kBlock), 0, stream, P, w->perm[0], w->perm[1], w->nodes[cur],
-                           w->chunk_base, w->chunk2node, w->chunk_left, Q, w->recs, w->n_rec, w->rec_cap,
+                           slot, w->chunk2node, w->chunk_left, Q, w->recs, w->n_rec, w->rec_cap,
                            map_next ? w->pm_child : nullptr);
         if (map_next) {
             const int n_paths = 1 << level;
@@ -1737,8 +1766,6 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
         ++level;
     }
     // tail
-    (void)hipEventRecord(w->ev[0], stream);
-    const int n_tail = w->h_ctr->n_tail;
     // Few subtrees (small inputs, few trees): what counts is how long the longest of them takes.  Workgroups of 1024 threads
     // while every subtree has a compute unit to itself, of 512 beyond that (so that all of them are resident at once:
     // 20,000 x 32, 50 trees, 808 subtrees 1.69 -> 1.58 ms for the trees), and nodes that are split in vain leave for the
@@ -1792,40 +1819,33 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
 #undef RSFK_CHAIN_LAUNCH
         RSFK_HIP(hipGetLastError());
     }
-    (void)hipEventRecord(w->ev[1], stream);
-    RSFK_HIP(hipMemcpyAsync(w->h_stats, w->stats, sizeof(TreeStats) * (size_t)nb, hipMemcpyDeviceToHost, stream));
-    RSFK_HIP(hipMemcpyAsync(w->h_ctr, w->ctr, sizeof(LevelCounters), hipMemcpyDeviceToHost, stream));
-    RSFK_HIP(hipMemcpyAsync(w->h_stat, w->stat, sizeof(unsigned long long) * kStatSlots * kStatPitch, hipMemcpyDeviceToHost, stream));
-    RSFK_HIP(hipStreamSynchronize(stream));
-    w->counts[0] = w->counts[1] = 0;
-    for (int sl = 0; sl < kStatSlots; ++sl) {
-        w->counts[0] += w->h_stat[kStatPitch * sl];
-        w->counts[1] += w->h_stat[kStatPitch * sl + 1];
-    }
+    hipLaunchKernelGGL(k_tree_report, dim3(1), dim3(64), 0, stream, w->stats, nb, w->ctr, w->stat, w->h_report, seq0);
+    RSFK_HIP(hipGetLastError());
+    if (wait_for_word(&w->h_report->seq, seq0, stream)) return 1;
+    const BatchReport& R = *w->h_report;
+    w->counts[0] = R.counts[0];
+    w->counts[1] = R.counts[1];
     {
-        float ms = 0.0f;
-        if (hipEventElapsedTime(&ms, w->ev[0], w->ev[1]) == hipSuccess) w->phase_s[3] = ms * 1e-3f;
-    }
-    {
-        // the steps of the wide levels, from the device's clock (events between the kernels of a level would cost
-        // more than some of the kernels)
+        // the steps, from the device's clock (events between the kernels of a level would cost more than some of the
+        // kernels)
         int dev = 0, khz = 0;
         if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev) == hipSuccess &&
             khz > 0) {
             const float s_per_tick = 1e-3f / (float)khz;
-            w->phase_s[1] = (float)w->h_ctr->phase_ticks[0] * s_per_tick;       // hyperplanes
-            w->phase_s[0] = (float)w->h_ctr->phase_ticks[1] * s_per_tick;       // side tests
-            w->phase_s[2] = (float)w->h_ctr->phase_ticks[2] * s_per_tick;       // scatter
+            w->phase_s[1] = (float)R.phase_ticks[0] * s_per_tick;       // hyperplanes
+            w->phase_s[0] = (float)R.phase_ticks[1] * s_per_tick;       // side tests
+            w->phase_s[2] = (float)R.phase_ticks[2] * s_per_tick;       // scatter
+            w->phase_s[3] = (float)R.phase_ticks[3] * s_per_tick;       // tail
         }
     }
-    RSFK_CHECK(!w->h_ctr->overflow, "tree batch: queue overflow in the tail phase");
+    RSFK_CHECK(!R.overflow, "tree batch: queue overflow in the tail phase");
     for (int t = 0; t < nb; ++t) {
-        const int total = w->h_stats[t].n_leaves + w->h_stats[t].n_big;
+        const int total = R.stats[t].n_leaves + R.stats[t].n_big;
         host_stats[5 * t + 0] = total;
-        host_stats[5 * t + 1] = w->h_stats[t].levels;
-        host_stats[5 * t + 2] = w->h_stats[t].max_leaf;
-        host_stats[5 * t + 3] = total ? w->h_stats[t].min_leaf : 0;
-        host_stats[5 * t + 4] = w->h_stats[t].n_big;
+        host_stats[5 * t + 1] = R.stats[t].levels;
+        host_stats[5 * t + 2] = R.stats[t].max_leaf;
+        host_stats[5 * t + 3] = total ? R.stats[t].min_leaf : 0;
+        host_stats[5 * t + 4] = R.stats[t].n_big;
         RSFK_CHECK(total <= w->leaf_cap, "tree batch: leaf table overflow");
     }
     return 0;
