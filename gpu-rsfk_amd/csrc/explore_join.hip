@@ -799,7 +799,7 @@ size_t explore_ws_bytes(int N, int K)
     return (size_t)N * ((size_t)K * (12 + 4 * mw) + 32) + ((size_t)20 << 20);
 }
 
-int explore_ws_alloc(ExploreWorkspace** out, int N, int K, bool with_bounds)
+int explore_ws_alloc(ExploreWorkspace** out, int N, int K, bool with_bounds, bool graph_only)
 {
     *out = nullptr;
     auto* w = new ExploreWorkspace();
@@ -857,7 +857,7 @@ int explore_ws_alloc(ExploreWorkspace** out, int N, int K, bool with_bounds)
     if (dm(&w->rev, total) != hipSuccess || dm(&w->bin_eq, 2 * total) != hipSuccess ||
         dm(&w->offs, (size_t)N + 1) != hipSuccess || dm(&w->bin_size, (size_t)w->n_bins) != hipSuccess ||
         dm(&w->bin_start, (size_t)w->n_bins + 1) != hipSuccess ||
-        dm(&w->part_off, (size_t)w->n_parts * (size_t)w->n_bins) != hipSuccess || dm(&w->pass, total * w->MW) != hipSuccess || dm(&w->norm_tau, 2 * (size_t)N) != hipSuccess ||
+        dm(&w->part_off, (size_t)w->n_parts * (size_t)w->n_bins) != hipSuccess || (!graph_only && (dm(&w->pass, total * w->MW) != hipSuccess || dm(&w->norm_tau, 2 * (size_t)N) != hipSuccess)) ||
         dm(&w->todo, 2 * ((size_t)N + 1)) != hipSuccess) {
         explore_ws_free(w);
         set_last_error("exploration workspace: out of device memory");
@@ -889,13 +889,18 @@ const uint32_t* explore_ws_pass(const ExploreWorkspace* w) { return w->pass; }
 const uint16_t* explore_ws_bounds(const ExploreWorkspace* w) { return w->bounds; }
 int* explore_ws_todo(ExploreWorkspace* w, int which) { return w->todo + (size_t)which * ((size_t)w->N + 1); }
 
-// Fill pass (and bounds) from the snapshot old_idx and the current last slots of knn_dist (rows sorted by distance).
-int launch_explore_join(ExploreWorkspace* w, const Bf16Copy& bf, int N, int D, int K, const int* old_idx,
-                        const float* knn_dist, hipStream_t stream, const int* order)
+bool explore_ws_takes(int N, int K)
 {
-    RSFK_CHECK(w && w->N == N && w->K == K, "exploration join: workspace does not match");
-    RSFK_CHECK(K >= 1 && K <= 256, "exploration join: K must be in 1..256");
-    RSFK_CHECK((size_t)N * (size_t)K < kMaxEntries, "exploration join: N*K must be below 2^31 - 4096");
+    int shift, n_bins;
+    return (size_t)N * (size_t)K < kMaxEntries && rev_bins(N, &shift, &n_bins);
+}
+const int* explore_ws_offs(const ExploreWorkspace* w) { return w->offs; }
+const int* explore_ws_rev(const ExploreWorkspace* w) { return w->rev; }
+
+// The reversed graph of idx (offs, rev).
+int launch_reversed_graph(ExploreWorkspace* w, const int* old_idx, int N, int K, hipStream_t stream)
+{
+    RSFK_CHECK(w && w->N == N && w->K == K, "reversed graph: workspace does not match");
     const int total = (int)((size_t)N * (size_t)K);
     if (w->staged) {
         const int nc = w->n_coarse, per = 1 << (w->cshift - w->fshift);
@@ -933,6 +938,18 @@ int launch_explore_join(ExploreWorkspace* w, const Bf16Copy& bf, int N, int D, i
     hipLaunchKernelGGL(k_bin_rows, dim3((unsigned)nbins), dim3(kRowsBlock), sizeof(int) << w->shift, stream, w->bin_eq,
                        w->bin_start, w->shift, N, w->offs, w->rev);
     }
+    RSFK_HIP(hipGetLastError());
+    return 0;
+}
+
+// Fill pass (and bounds) from the snapshot old_idx and the current last slots of knn_dist (rows sorted by distance).
+int launch_explore_join(ExploreWorkspace* w, const Bf16Copy& bf, int N, int D, int K, const int* old_idx,
+                        const float* knn_dist, hipStream_t stream, const int* order)
+{
+    RSFK_CHECK(w && w->N == N && w->K == K, "exploration join: workspace does not match");
+    RSFK_CHECK(K >= 1 && K <= 256, "exploration join: K must be in 1..256");
+    RSFK_CHECK((size_t)N * (size_t)K < kMaxEntries, "exploration join: N*K must be below 2^31 - 4096");
+    if (launch_reversed_graph(w, old_idx, N, K, stream)) return 1;
     hipLaunchKernelGGL(k_norm_tau, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, stream, bf.norms, knn_dist, N, K, w->norm_tau);
     RSFK_HIP(hipGetLastError());
 

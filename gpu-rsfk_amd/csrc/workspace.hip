@@ -256,21 +256,23 @@ struct Fetched {
     int word[kFetchMost];
     int seq;
 };
-__global__ void k_fetch(const int* __restrict__ src, int n, Fetched* out)
+__global__ void k_fetch(const int* __restrict__ a, int na, const int* __restrict__ b, int nb, Fetched* out)
 {
-    for (int i = 0; i < n; ++i) out->word[i] = src[i];
+    for (int i = 0; i < na; ++i) out->word[i] = a[i];
+    for (int i = 0; i < nb; ++i) out->word[na + i] = b[i];
     __hip_atomic_store(&out->seq, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 }  // namespace
 
-int fetch_words(const int* dev, int n, int* host, hipStream_t stream)
+int fetch_words(const int* a, int na, const int* b, int nb, int* host, hipStream_t stream)
 {
+    const int n = na + nb;
     RSFK_CHECK(n >= 1 && n <= kFetchMost, "fetch: too many words");
     void* p = nullptr;
     if (pin_alloc(&p, sizeof(Fetched))) return 1;
     Fetched* f = static_cast<Fetched*>(p);
     __atomic_store_n(&f->seq, 0, __ATOMIC_RELEASE);
-    hipLaunchKernelGGL(k_fetch, dim3(1), dim3(1), 0, stream, dev, n, f);
+    hipLaunchKernelGGL(k_fetch, dim3(1), dim3(1), 0, stream, a, na, b, nb, f);
     const hipError_t e = hipGetLastError();
     const int rc = e != hipSuccess ? 1 : wait_for_word(&f->seq, 1, stream);
     if (e != hipSuccess) set_last_error(std::string("fetch: ") + hipGetErrorString(e));

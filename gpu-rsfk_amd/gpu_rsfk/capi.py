@@ -130,15 +130,15 @@ def symmetrize(knn_idx, knn_dist=None, drop_self=False):
         dp = knn_dist.ctypes.data_as(_vp)
     indptr = np.empty(N + 1, np.int32)
     nnz = ctypes.c_longlong(0)
+    # (room for any graph; the rows are cut to what was written, and the rest of the pages is never touched)
+    cols = np.empty(2 * N * K, np.int32)
+    vals = np.empty(2 * N * K, np.float32)
     _check(lib().rsfk_symmetrize_host(knn_idx.ctypes.data_as(_vp), dp, N, K, int(bool(drop_self)),
-                                      indptr.ctypes.data_as(_vp), None, None, 0, ctypes.byref(nnz)))
+                                      indptr.ctypes.data_as(_vp), cols.ctypes.data_as(_vp),
+                                      vals.ctypes.data_as(_vp), 2 * N * K, ctypes.byref(nnz)))
     n = int(nnz.value)
-    cols = np.empty(n, np.int32)
-    vals = np.empty(n, np.float32)
-    if n:
-        _check(lib().rsfk_symmetrize_host(knn_idx.ctypes.data_as(_vp), dp, N, K, int(bool(drop_self)),
-                                          indptr.ctypes.data_as(_vp), cols.ctypes.data_as(_vp),
-                                          vals.ctypes.data_as(_vp), n, ctypes.byref(nnz)))
+    cols.resize(n, refcheck=False)
+    vals.resize(n, refcheck=False)
     return indptr, cols, vals
 
 

@@ -839,6 +839,28 @@ def test_symmetric_graph_matches_oracle(gpu, orc, rng, N, K, drop_self):
     assert np.array_equal(gp2, op) and np.array_equal(gc2, oc) and (gv2 == 0).all()
 
 
+# Rows as unions of the stored neighbours and the reversed entries: rows of one, two and four entries per lane, rows that
+# go to a workgroup (points that very many others store), rows of more candidates than that takes (the other form),
+# empty rows, with and without the point itself.
+@pytest.mark.parametrize("N,K,hubs,drop_self", [(900, 5, 0, True), (3000, 20, 3, False), (5000, 33, 40, True), (6000, 90, 200, True),
+                                                (9000, 12, 1, True), (1500, 300, 5, False), (12000, 3, 2, True)])
+def test_symmetric_graph_with_hubs_matches_oracle(gpu, orc, rng, monkeypatch, N, K, hubs, drop_self):
+    import gpu_rsfk
+    monkeypatch.setenv("RSFK_GRAPH_FLAGS", "0")
+    idx = np.stack([rng.choice(N, K, replace=False) for _ in range(N)]).astype(np.int32)
+    for h in range(hubs):                                       # a point most others store, in slot h (unless they do already)
+        put = (rng.random(N) < 0.3 + 0.7 / (h + 1)) & ~(idx == h).any(1)
+        idx[put, h % K] = h
+    idx[rng.random((N, K)) < 0.05] = -1
+    idx[N // 2:N // 2 + 20] = -1
+    a, b = np.minimum(idx, np.arange(N)[:, None]).astype(np.int64), np.maximum(idx, np.arange(N)[:, None])
+    val = ((a * 7919 + b * 104729) % 10007).astype(np.float32)  # one value per pair
+    _say("symmetrize with hubs", N, K, hubs, drop_self)
+    gp, gc, gv = gpu_rsfk.symmetric_knn_graph(idx, val, drop_self=drop_self)
+    op, oc, ov = orc.symmetrize(idx, val, drop_self=drop_self)
+    assert np.array_equal(gp, op) and np.array_equal(gc, oc) and np.array_equal(gv, ov)
+
+
 def test_symmetric_graph_of_a_built_graph(gpu, capi, orc, rng):
     """On a graph the library built (one distance value per pair) the export equals the oracle's bit for bit; device
     entry point with the two-call protocol (count, then fill)."""
