@@ -16,9 +16,14 @@
 // and a workgroup works on one bucket and up to 16 of its queries: the rows of the bucket pass through LDS once per
 // workgroup instead of once per query, every lane runs the sequential chain of "its" bucket member against four
 // queries whose coordinates are wavefront-uniform, and the candidates are merged into the queries' rows.
+//
+// That is a chain of six launches per tree, which a small set of queries cannot fill; its trees go together instead
+// (launch_ann_forest): the queries are routed through all trees in one launch, and one workgroup per query works on the
+// buckets the query reached in all of them.
 #include "forest.hpp"
 #include "exact_batch.hpp"
 #include <algorithm>
+#include <cstdlib>
 
 namespace rsfk {
 
@@ -42,18 +47,20 @@ __global__ __launch_bounds__(256) void k_zero_ints(int* __restrict__ p, int n)
 // Hyperplane of every two-child node of the index, one wavefront per record: row r of `planes` (pitch floats) is
 // [offset, 0, 0, 0 | normal, zero padded to a multiple of 4].  Normal and offset are the values the builder works with
 // (create_node.cu:122-135: n = x1 - x2, offset = sum n_d (x1_d + x2_d) / 2 as 32 lane-strided partial sums + xor butterfly).
+// blockIdx.y: the tree; the records and the rows of a tree begin rec_cap after those of the tree before it.
 __global__ __launch_bounds__(256) void k_planes(const float* __restrict__ points, int D, const TreeRec* __restrict__ recs,
                                                 const int* __restrict__ n_rec_p, int rec_cap, float* __restrict__ planes,
                                                 int pitch)
 {
     const int lane = threadIdx.x & 63;
-    const int r = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (r >= min(*n_rec_p, rec_cap)) return;
-    const TreeRec rec = recs[r];
+    const int r = blockIdx.x * 4 + (threadIdx.x >> 6), j = blockIdx.y;
+    if (r >= min(n_rec_p[j], rec_cap)) return;
+    const size_t at = (size_t)j * (size_t)rec_cap + (size_t)r;
+    const TreeRec rec = recs[at];
     if (rec.c0 < 0) return;
     const float* x1 = points + (size_t)rec.a * (size_t)D;
     const float* x2 = points + (size_t)rec.b * (size_t)D;
-    float* row = planes + (size_t)r * (size_t)pitch;
+    float* row = planes + at * (size_t)pitch;
     float s = 0.0f;
     if (lane < 32) {
         for (int d = lane; d < D; d += 32) {
@@ -72,13 +79,19 @@ __global__ __launch_bounds__(256) void k_planes(const float* __restrict__ points
 // build_tree_check_points_side.cu:131-149: sum j takes the dimensions j, j+32, ... in turn) and adds them in the order
 // of the xor butterfly; the other three steps of the butterfly run over the eight lanes.  The first 128 dimensions of
 // the query stay in registers.  q_rec[q] = record of the bucket reached, q_rank[q] = arrival number of q among the
-// queries of that bucket (cnt counts them).
+// queries of that bucket (cnt counts them).  FOREST: blockIdx.y is the tree, and reached[q T + tree] = {start, size} of
+// the bucket is all that is kept.
 constexpr int kXR = 4;
-template <bool VEC>
+template <bool VEC, bool FOREST>
 __global__ __launch_bounds__(256) void k_route(const float* __restrict__ planes, int pitch, const float* __restrict__ queries,
                                                int NQ, int D, const TreeRec* __restrict__ recs, int max_steps,
-                                               int* __restrict__ q_rec, int* __restrict__ q_rank, int* __restrict__ cnt)
+                                               int* __restrict__ q_rec, int* __restrict__ q_rank, int* __restrict__ cnt,
+                                               int2* __restrict__ reached)
 {
+    if (FOREST) {
+        recs += (size_t)blockIdx.y * (size_t)max_steps;         // (max_steps: the records a tree has room for)
+        planes += (size_t)blockIdx.y * (size_t)max_steps * (size_t)pitch;
+    }
     const int sub = threadIdx.x & 7;
     const int q = (int)((blockIdx.x * (size_t)blockDim.x + threadIdx.x) >> 3);
     const bool valid = q < NQ;
@@ -124,7 +137,12 @@ __global__ __launch_bounds__(256) void k_route(const float* __restrict__ planes,
         t += dpp_f<kDppHalfMirror>(t);
         if (!done) {
             if (r.c0 < 0) {
-                if (sub == 0) { q_rec[q] = cur; q_rank[q] = atomicAdd(&cnt[cur], 1); }
+                if (FOREST) {
+                    if (sub == 0) reached[(size_t)q * gridDim.y + blockIdx.y] = make_int2(r.a, r.b);
+                } else if (sub == 0) {
+                    q_rec[q] = cur;
+                    q_rank[q] = atomicAdd(&cnt[cur], 1);
+                }
                 done = true;
             } else {
                 cur = t < b ? r.c1 : r.c0;
@@ -356,6 +374,101 @@ __global__ __launch_bounds__(256) void k_ann_leaf(const float* __restrict__ poin
         if (qv[i] && row[i].changed) row[i].store(q_idx + (size_t)qid[i] * K, q_dist + (size_t)qid[i] * K);
 }
 
+// Workgroup q works on query q and the buckets it reached in T trees, wavefront w on those of the trees w, w + 4, ...
+// The members of the buckets are gathered in a list, 64 of them at a time get their exact distance (a lane reads "its"
+// row, the arithmetic of k_ann_leaf) and are merged into the wavefront's copy of the row; at the end the copies are
+// merged.  A row is the K smallest pairs of what it is offered in whatever order, and a pair that a wavefront turns
+// away has K pairs below it in that wavefront's row, all of which the final row is offered.
+// A query meets a near point in many trees: an id that a wavefront has listed goes into a small direct-mapped table the
+// four share, and an id found there is not listed again (whoever put it there evaluates it; an entry that another id has
+// overwritten only costs a repeat, which the row turns away).
+// Bound by the latency of the gathers: 1,000 queries, 50 trees on 20,000 x 64 clustered points take 48 us here, 23 in each of
+// k_planes and k_route (six launches a tree before: 1,780 us).
+constexpr int kAnnSeen = 1024;
+constexpr int kAnnList = 128;         // of a wavefront: fewer than 64 waiting and up to 64 new ones
+template <int SL>
+__global__ __launch_bounds__(256) void k_ann_forest(const float* __restrict__ points, const float* __restrict__ queries, int N, int D,
+                                                    int K, int T, const int* __restrict__ perm, const int2* __restrict__ reached,
+                                                    bool vec_ok, int dpad, int* __restrict__ q_idx, float* __restrict__ q_dist)
+{
+    // dynamic LDS: the query (dpad) | table (kAnnSeen) | lists (4 x kAnnList) | rows of wavefronts 1..3 (ids, distances)
+    extern __shared__ __align__(16) int ann_lds[];
+    float* xrow = reinterpret_cast<float*>(ann_lds);
+    int* seen = ann_lds + dpad;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    int* list = seen + kAnnSeen + wave * kAnnList;
+    int* row_i = seen + kAnnSeen + 4 * kAnnList;
+    float* row_d = reinterpret_cast<float*>(row_i + 3 * 64 * SL);
+    const size_t q = blockIdx.x;
+    // (T is at most 64: lane l holds the bucket of tree wave + 4 l)
+    const int2 mine = lane < 16 && wave + 4 * lane < T ? reached[q * (size_t)T + (size_t)(wave + 4 * lane)] : make_int2(0, 0);
+    for (int d = tid; d < dpad; d += 256) xrow[d] = d < D ? queries[q * (size_t)D + (size_t)d] : 0.0f;
+    for (int e = tid; e < kAnnSeen; e += 256) seen[e] = -1;
+    KnnRow<SL> row;
+    row.load(q_idx + q * (size_t)K, q_dist + q * (size_t)K, K);
+    __syncthreads();
+    ExploreLds L = {};
+    L.xrow = xrow;
+    const int n_mine = (T - wave + 3) >> 2;
+    // the ids of the next tree travel while those of the present one are worked on
+    auto request = [&](int i) {
+        const int start = read_lane_i(mine.x, i & 15), size = i < n_mine ? read_lane_i(mine.y, i & 15) : 0;
+        return lane < size ? perm[(size_t)(wave + 4 * i) * (size_t)N + (size_t)(start + lane)] : -1;
+    };
+    int n = 0;
+    int next = request(0);
+    for (int i = 0; i < n_mine; ++i) {
+        const int start = read_lane_i(mine.x, i), size = read_lane_i(mine.y, i);
+        const int* ids = perm + (size_t)(wave + 4 * i) * (size_t)N + (size_t)start;
+        int id = next;
+        next = request(i + 1);
+        for (int c0 = 0; c0 < size; c0 += 64) {
+            if (c0 > 0) id = c0 + lane < size ? ids[c0 + lane] : -1;
+            int* slot = seen + ((uint32_t)id * 2654435761u >> 22);
+            const bool list_it = id >= 0 && __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != id;
+            const uint64_t m = ballot64(list_it);
+            if (list_it) {
+                __hip_atomic_store(slot, id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                list[n + mask_prefix(m)] = id;
+            }
+            n += __popcll(m);
+            wave_lds_sync();
+            if (n >= 64) {
+                exact_direct<SL>(L, list, 64, points, D, vec_ok, row);
+                n -= 64;
+                const int rest = lane < n ? list[64 + lane] : -1;
+                wave_lds_sync();
+                if (lane < n) list[lane] = rest;
+                wave_lds_sync();
+            }
+        }
+    }
+    if (n > 0) exact_direct<SL>(L, list, n, points, D, vec_ok, row);
+    if (wave > 0) {
+#pragma unroll
+        for (int s = 0; s < SL; ++s) {
+            row_i[(wave - 1) * 64 * SL + 64 * s + lane] = row.changed ? row.idx[s] : -1;
+            row_d[(wave - 1) * 64 * SL + 64 * s + lane] = row.dist[s];
+        }
+    }
+    __syncthreads();
+    if (wave > 0) return;
+#pragma unroll 1
+    for (int w = 0; w < 3; ++w) {
+        bool ok[SL];
+        int c[SL];
+        float d[SL];
+#pragma unroll
+        for (int s = 0; s < SL; ++s) {
+            c[s] = row_i[w * 64 * SL + 64 * s + lane];
+            d[s] = row_d[w * 64 * SL + 64 * s + lane];
+            ok[s] = c[s] >= 0;
+        }
+        row.template merge<SL>(ok, c, d);
+    }
+    if (row.changed) row.store(q_idx + q * (size_t)K, q_dist + q * (size_t)K);
+}
+
 }  // namespace
 
 // floats per row of the table of hyperplanes: offset (4 floats) + normal padded to a multiple of 4
@@ -404,11 +517,11 @@ int launch_ann_tree(const float* points, const float* queries, int NQ, int D, in
     const unsigned g_route = (unsigned)(((size_t)NQ * 8 + 255) / 256);
     const bool vec_q = (D & 3) == 0 && (reinterpret_cast<uintptr_t>(queries) & 15) == 0;
     if (vec_q)
-        hipLaunchKernelGGL(k_route<true>, dim3(g_route), dim3(256), 0, stream, planes, pitch, queries, NQ, D, recs, rec_cap, q_rec,
-                           q_rank, cnt);
+        hipLaunchKernelGGL((k_route<true, false>), dim3(g_route), dim3(256), 0, stream, planes, pitch, queries, NQ, D, recs, rec_cap,
+                           q_rec, q_rank, cnt, nullptr);
     else
-        hipLaunchKernelGGL(k_route<false>, dim3(g_route), dim3(256), 0, stream, planes, pitch, queries, NQ, D, recs, rec_cap, q_rec,
-                           q_rank, cnt);
+        hipLaunchKernelGGL((k_route<false, false>), dim3(g_route), dim3(256), 0, stream, planes, pitch, queries, NQ, D, recs, rec_cap,
+                           q_rec, q_rank, cnt, nullptr);
     const unsigned g_scan = (unsigned)(rec_cap / kScanTile + 1);
     hipLaunchKernelGGL(k_ann_tile_sums, dim3(g_scan), dim3(256), 0, stream, cnt, n_rec_dev, rec_cap, tile_sum);
     hipLaunchKernelGGL(k_ann_scan, dim3(g_scan), dim3(256), 0, stream, cnt, n_rec_dev, rec_cap, tile_sum, qoff, boff, n_blocks);
@@ -432,6 +545,67 @@ int launch_ann_tree(const float* points, const float* queries, int NQ, int D, in
     else if (K <= 256) RSFK_ANN_CASE(4)
     else if (K <= 512) RSFK_ANN_CASE(8)
     else RSFK_ANN_CASE(16)
+#undef RSFK_ANN_CASE
+    RSFK_HIP(hipGetLastError());
+    return 0;
+}
+
+size_t ann_forest_lds(int D, int K) { return sizeof(int) * ((size_t)((D + 31) & ~31) + kAnnSeen + 4 * kAnnList + (size_t)6 * 64 * row_slots(K)); }
+
+// Trees of a batch of nb that are searched together (0: one tree after the other).  Together, a query gathers the rows of its
+// buckets by itself, up to NQ MAX D floats a tree; one after the other, up to 16 queries of a bucket share them, at the price
+// of six launches a tree.  Time of the search, one after the other -> together (uniform points where nothing is said):
+//   20,000 x 64 clustered, buckets of up to 34, 50 trees: 1,000 queries 1.78 -> 0.09 ms, 10,000 1.99 -> 0.44, 40,000 3.59 -> 1.59
+//   1M x 100, up to 66, 50 trees: 2,000 queries (1.3e7 floats) 3.5 -> 1.8 ms, 20,000 (1.3e8) 8.7 -> 9.0, 100,000 16 -> 40
+//   100,000 x 100, up to 66, 50 trees: 10,000 queries (6.6e7) 2.90 -> 2.93 ms, 50,000 5.1 -> 14.2
+//   300,000 x 8, up to 18, 50 trees: 200,000 queries (2.9e7) 10.2 -> 4.7 ms;  5,000 x 129, K = 300, 9 trees: 600 queries (4.7e7)
+//   4.0 -> 1.1;  70,000 x 784, K = 90, 10 trees: 10,000 queries (1.4e9) 2.8 -> 10.1
+int ann_forest_group(int N, int NQ, int D, int K, int MAX, int rec_cap, int nb)
+{
+    const char* e = std::getenv("RSFK_ANN_FOREST");
+    if (e && e[0] == '0') return 0;
+    if (nb < 2 || ann_forest_lds(D, K) > (size_t)64 << 10) return 0;
+    const bool forced = e && e[0] == '1';
+    constexpr double kMostFloats = 5e7;
+    if (!forced && (double)NQ * (double)MAX * (double)D > kMostFloats) return 0;
+    // hyperplanes and buckets reached: 1 GB at most
+    const size_t per_tree = sizeof(float) * (size_t)rec_cap * (size_t)ann_plane_pitch(D) + sizeof(int2) * (size_t)NQ;
+    const int group = (int)std::min<size_t>((size_t)std::min(nb, 64), ((size_t)1 << 30) / per_tree);
+    return group >= 2 ? group : 0;
+}
+
+// The search in T trees at once.  recs, n_rec_dev, perm: those of the first tree, the others follow; planes: T rec_cap rows of
+// ann_plane_pitch(D) floats; reached: 2 NQ T ints.
+int launch_ann_forest(const float* points, const float* queries, int N, int NQ, int D, int K, int T, const int* perm, const TreeRec* recs,
+                      const int* n_rec_dev, int rec_cap, float* planes, int* reached, int* q_idx, float* q_dist, hipStream_t stream)
+{
+    RSFK_CHECK(K >= 1 && K <= kMaxK && T >= 1 && T <= 64, "query-set search: out of range");
+    RSFK_CHECK(recs != nullptr && rec_cap >= 1, "query-set search: the tree has no index");
+    const int pitch = ann_plane_pitch(D);
+    int2* where = reinterpret_cast<int2*>(reached);
+    hipLaunchKernelGGL(k_planes, dim3((unsigned)((rec_cap + 3) / 4), (unsigned)T), dim3(256), 0, stream, points, D, recs, n_rec_dev, rec_cap,
+                       planes, pitch);
+    const dim3 g_route((unsigned)(((size_t)NQ * 8 + 255) / 256), (unsigned)T);
+    const bool vec_q = (D & 3) == 0 && (reinterpret_cast<uintptr_t>(queries) & 15) == 0;
+    if (vec_q)
+        hipLaunchKernelGGL((k_route<true, true>), g_route, dim3(256), 0, stream, planes, pitch, queries, NQ, D, recs, rec_cap, nullptr,
+                           nullptr, nullptr, where);
+    else
+        hipLaunchKernelGGL((k_route<false, true>), g_route, dim3(256), 0, stream, planes, pitch, queries, NQ, D, recs, rec_cap, nullptr,
+                           nullptr, nullptr, where);
+    const bool vec_p = (D & 3) == 0 && (reinterpret_cast<uintptr_t>(points) & 15) == 0;
+    const int dpad = (D + 31) & ~31;
+    const size_t lds = ann_forest_lds(D, K);
+#define RSFK_ANN_CASE(SLV)                                                                                                    \
+    hipLaunchKernelGGL(k_ann_forest<SLV>, dim3((unsigned)NQ), dim3(256), lds, stream, points, queries, N, D, K, T, perm, where,  \
+                       vec_p, dpad, q_idx, q_dist)
+    switch (row_slots(K)) {
+    case 1: RSFK_ANN_CASE(1); break;
+    case 2: RSFK_ANN_CASE(2); break;
+    case 4: RSFK_ANN_CASE(4); break;
+    case 8: RSFK_ANN_CASE(8); break;
+    default: RSFK_ANN_CASE(16); break;
+    }
 #undef RSFK_ANN_CASE
     RSFK_HIP(hipGetLastError());
     return 0;

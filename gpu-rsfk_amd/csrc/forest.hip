@@ -464,22 +464,31 @@ int knn_ann_forest_device(int n_trees, int K, int N, int NQ, int D, int MIN, int
     if (log_forest) std::memset(log_forest, 0, sizeof(float) * ((size_t)16 * n_trees + 2));
     const double t0 = now_s();
     if (n_trees > 0 && NQ > 0) {
-        Bf16Guard bf;
-        if (bf16_copy_alloc(&bf.c, N, D)) return 1;
-        if (bf16_copy_fill(bf.c, d_points, N, D, stream)) return 1;
         Q8Guard q8;
         const uint8_t* q8_rows = nullptr;
         if (make_tree_screen(q8, d_points, N, D, verbose, stream, &q8_rows)) return 1;
+        Bf16Guard bf;                                       // (nobody reads it when the 8-bit copy screens the side tests)
+        if (q8_rows == nullptr && (bf16_copy_alloc(&bf.c, N, D) || bf16_copy_fill(bf.c, d_points, N, D, stream))) return 1;
         const int B = choose_batch(n_trees, N, D, MIN);
         WsGuard ws;
         if (tree_ws_alloc(&ws.w, N, D, MIN, B)) return 1;
         if (tree_ws_enable_index(ws.w, MIN, MAX_DEPTH)) return 1;
         const int rec_cap = tree_ws_rec_cap(ws.w);
-        DevBuf aws;
-        if (ws_alloc(&aws.p, sizeof(int) * ann_ws_ints(NQ, rec_cap))) return 1;
-        if (launch_ann_ws_init(static_cast<int*>(aws.p), NQ, rec_cap, stream)) return 1;
-        DevBuf planes;
-        if (ws_alloc(&planes.p, sizeof(float) * (size_t)rec_cap * (size_t)ann_plane_pitch(D))) return 1;
+        const size_t plane_bytes = sizeof(float) * (size_t)rec_cap * (size_t)ann_plane_pitch(D);
+        DevBuf aws, planes, reached;
+        // trees that are searched together (0, or no memory for it: one tree after the other)
+        int group = ann_forest_group(N, NQ, D, K, MAX, rec_cap, std::min(n_trees, B));
+        if (group > 0 && (ws_try_alloc(&planes.p, plane_bytes * (size_t)group) ||
+                          ws_try_alloc(&reached.p, sizeof(int) * 2 * (size_t)NQ * (size_t)group))) {
+            if (planes.p) ws_free(planes.p);
+            planes.p = nullptr;
+            group = 0;
+        }
+        if (group == 0) {
+            if (ws_alloc(&aws.p, sizeof(int) * ann_ws_ints(NQ, rec_cap))) return 1;
+            if (launch_ann_ws_init(static_cast<int*>(aws.p), NQ, rec_cap, stream)) return 1;
+            if (ws_alloc(&planes.p, plane_bytes)) return 1;
+        }
         std::vector<int> stats((size_t)5 * B);
         std::vector<TimedEvent> ev((size_t)B + 1);          // ev[j]: the search in tree j of a batch begins, ev[nb]: the last ends
         for (auto& e : ev)
@@ -492,7 +501,12 @@ int knn_ann_forest_device(int n_trees, int K, int N, int NQ, int D, int MIN, int
                                   stream);
             if (rc) break;
             const double tt = now_s() - tt0;
-            for (int j = 0; j < nb && rc == 0; ++j) {
+            if (group > 0) (void)hipEventRecord(ev[0].e, stream);
+            for (int j = 0; j < nb && rc == 0 && group > 0; j += group)
+                rc = launch_ann_forest(d_points, d_queries, N, NQ, D, K, std::min(group, nb - j), tree_ws_perm(ws.w, j),
+                                       tree_ws_recs(ws.w, j), tree_ws_n_rec(ws.w, j), rec_cap, static_cast<float*>(planes.p),
+                                       static_cast<int*>(reached.p), d_qidx, d_qdist, stream);
+            for (int j = 0; j < nb && rc == 0 && group == 0; ++j) {
                 (void)hipEventRecord(ev[j].e, stream);
                 rc = launch_ann_tree(d_points, d_queries, NQ, D, K, tree_ws_perm(ws.w, j), tree_ws_recs(ws.w, j),
                                      tree_ws_n_rec(ws.w, j), rec_cap, stats[5 * j + 0], static_cast<int*>(aws.p),
@@ -503,7 +517,12 @@ int knn_ann_forest_device(int n_trees, int K, int N, int NQ, int D, int MIN, int
             RSFK_HIP(hipStreamSynchronize(stream));
             for (int j = 0; j < nb; ++j) {
                 float ms = 0.0f;
-                (void)hipEventElapsedTime(&ms, ev[j].e, ev[j + 1].e);
+                if (group > 0) {
+                    (void)hipEventElapsedTime(&ms, ev[0].e, ev[nb].e);
+                    ms /= (float)nb;                         // a tree's share
+                } else {
+                    (void)hipEventElapsedTime(&ms, ev[j].e, ev[j + 1].e);
+                }
                 const int t = tb0 + j;
                 if (log_forest) {
                     log_forest[(size_t)0 * n_trees + t] = (float)stats[5 * j + 1];   // Tree Depth
@@ -594,12 +613,11 @@ int build_tree_host(const float* d_points, int N, int D, int MIN, int MAX, int M
 {
     WsGuard ws;
     if (tree_ws_alloc(&ws.w, N, D, MIN, 1)) return 1;
-    Bf16Guard bf;
-    if (bf16_copy_alloc(&bf.c, N, D)) return 1;
-    if (bf16_copy_fill(bf.c, d_points, N, D, nullptr)) return 1;
     Q8Guard q8;
     const uint8_t* q8_rows = nullptr;
     if (make_tree_screen(q8, d_points, N, D, 0, nullptr, &q8_rows)) return 1;
+    Bf16Guard bf;                                           // (nobody reads it when the 8-bit copy screens the side tests)
+    if (q8_rows == nullptr && (bf16_copy_alloc(&bf.c, N, D) || bf16_copy_fill(bf.c, d_points, N, D, nullptr))) return 1;
     if (build_tree_batch(ws.w, d_points, bf.c.rows, q8_rows, N, D, MIN, MAX, MAX_DEPTH, seed, 1, stats, nullptr)) return 1;
     const int nl = stats[0], n_big = stats[4], n_small = nl - n_big, cap = tree_ws_leaf_cap(ws.w);
     perm.resize((size_t)N);

@@ -770,6 +770,31 @@ def test_find_nearest_neighbors_ann_matches_oracle(gpu, orc, rng, N, NQ, D, K, T
     assert r._last_search_time > 0
 
 
+# one query; one tree more than the wavefronts take in turn; buckets on both sides of 64 and 128; rows of one, two and
+# more slots per lane; rows that end inside a 16-byte piece; more trees than go together
+@pytest.mark.parametrize("N,NQ,D,K,T,mn,mx", [(300, 1, 1, 1, 2, 3, 6), (2000, 37, 33, 64, 5, 65, 65 * 2), (1500, 300, 64, 65, 9, 66, 128),
+                                              (900, 130, 31, 16, 3, 17, 64), (700, 65, 100, 300, 4, 301, 700), (4000, 90, 7, 5, 70, 6, 12),
+                                              (50, 20, 12, 8, 6, 60, 120), (1200, 33, 260, 20, 8, 21, 65)])
+@pytest.mark.parametrize("data", ["normal", "ties"])
+def test_ann_trees_together_match_oracle(gpu, capi, orc, rng, monkeypatch, N, NQ, D, K, T, mn, mx, data):
+    """All trees of a query in one workgroup == one tree after the other == the oracle, also into rows that hold something."""
+    import torch
+    draw = (lambda n: rng.integers(0, 3, (n, D)).astype(np.float32)) if data == "ties" else (lambda n: rng.standard_normal((n, D)).astype(np.float32))
+    X, Q = draw(N), draw(NQ)
+    dX, dQ = torch.from_numpy(X).cuda(), torch.from_numpy(Q).cuda()
+    oi, od = orc.ann_forest(X, Q, K, T, mn, mx, 5000, 5)
+    orc.ann_forest(X, Q, K, 2, mn, mx, 5000, 77, q_idx=oi, q_dist=od)
+    for form in ("0", "1"):
+        monkeypatch.setenv("RSFK_ANN_FOREST", form)
+        idx = torch.full((NQ, K), -1, dtype=torch.int32, device="cuda")
+        dist = torch.full((NQ, K), float("inf"), dtype=torch.float32, device="cuda")
+        _say("ann together", N, NQ, D, K, T, mn, mx, data, form)
+        for trees, seed in ((T, 5), (2, 77)):
+            capi.knn_ann_device(trees, K, N, NQ, D, mn, mx, 5000, 0, seed, dX.data_ptr(), dQ.data_ptr(), idx.data_ptr(), dist.data_ptr())
+        torch.cuda.synchronize()
+        assert_knn_equal(idx.cpu().numpy(), dist.cpu().numpy(), oi, od)
+
+
 def test_ann_device_entry_point_merges_into_given_rows(gpu, capi, orc, rng):
     """Device-resident call, twice with different seeds on the same rows == the oracle doing the same."""
     import torch
