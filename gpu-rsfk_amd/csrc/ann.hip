@@ -15,12 +15,14 @@
 // The queries are then grouped by the bucket they reached (a count per bucket taken while routing, a scan, a fill)
 // and a workgroup works on one bucket and up to 16 of its queries: the rows of the bucket pass through LDS once per
 // workgroup instead of once per query, every lane runs the sequential chain of "its" bucket member against four
-// queries whose coordinates are wavefront-uniform, and the candidates are merged into the queries' rows.
+// queries whose coordinates are wavefront-uniform, and the candidates are merged into the queries' rows.  Trees after which
+// few pairs still enter a row are searched by the kernel of ann_screen.hip instead, which bounds the pairs first.
 //
 // That is a chain of six launches per tree, which a small set of queries cannot fill; its trees go together instead
 // (launch_ann_forest): the queries are routed through all trees in one launch, and one workgroup per query works on the
 // buckets the query reached in all of them.
 #include "forest.hpp"
+#include "ann.hpp"
 #include "exact_batch.hpp"
 #include <algorithm>
 #include <cstdlib>
@@ -29,7 +31,9 @@ namespace rsfk {
 
 namespace {
 
-constexpr int kQB = 16;               // queries per workgroup
+constexpr int kQB = kAnnDirect;       // queries per workgroup
+constexpr int kLeafGrid = 4096;       // workgroups of k_ann_leaf
+constexpr int kAnnScreenDims = 4096;  // the bounds of the screened form are useless long before
 constexpr int kQW = 4;                // queries a wavefront works on together
 constexpr int kCG = 128;              // bucket members per pass: two per lane
 constexpr int kCH = 32;               // dimensions per staging step
@@ -153,12 +157,17 @@ __global__ __launch_bounds__(256) void k_route(const float* __restrict__ planes,
 }
 
 // Scan over the records of the tree in tiles of 1024 (a workgroup each): qoff = exclusive scan of the query counts,
-// boff = exclusive scan of the numbers of workgroups (16 queries each) the buckets need; both get a closing entry at
+// boff = exclusive scan of the numbers of work items (qb queries each) the buckets need; both get a closing entry at
 // index n_rec.  The two sums travel as the halves of one 64-bit value.
 typedef unsigned long long u64;
 constexpr int kScanTile = 1024;
 
-__device__ __forceinline__ u64 pack_count(int c) { return (u64)(unsigned)c | ((u64)(unsigned)((c + kQB - 1) / kQB) << 32); }
+__device__ __forceinline__ u64 pack_count(int c, int log_qb)
+{
+    return (u64)(unsigned)c | ((u64)(unsigned)((c + (1 << log_qb) - 1) >> log_qb) << 32);
+}
+static_assert(kAnnDirect == 16 && kAnnScreen == 32, "log_queries");
+__device__ __forceinline__ int log_queries(const AnnForm& form) { return form.screened() ? 5 : 4; }
 
 // exclusive scan of 256 values, one per thread; *total = their sum
 __device__ __forceinline__ u64 block_scan_256(u64 v, u64* total, u64* lds4)
@@ -181,14 +190,15 @@ __device__ __forceinline__ u64 block_scan_256(u64 v, u64* total, u64* lds4)
 }
 
 __global__ __launch_bounds__(256) void k_ann_tile_sums(const int* __restrict__ cnt, const int* __restrict__ n_rec_p, int rec_cap,
-                                                       u64* __restrict__ tile_sum)
+                                                       u64* __restrict__ tile_sum, AnnForm form)
 {
     __shared__ u64 lds4[4];
+    const int log_qb = log_queries(form);
     const int n = min(*n_rec_p, rec_cap);
     const int i0 = blockIdx.x * kScanTile + threadIdx.x * 4;
     u64 mine = 0;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) mine += i0 + j < n ? pack_count(cnt[i0 + j]) : 0ull;
+    for (int j = 0; j < 4; ++j) mine += i0 + j < n ? pack_count(cnt[i0 + j], log_qb) : 0ull;
     u64 tot;
     (void)block_scan_256(mine, &tot, lds4);
     if (threadIdx.x == 0) tile_sum[blockIdx.x] = tot;
@@ -197,9 +207,10 @@ __global__ __launch_bounds__(256) void k_ann_tile_sums(const int* __restrict__ c
 // Second step; also sets the counts back to zero for the next tree.
 __global__ __launch_bounds__(256) void k_ann_scan(int* __restrict__ cnt, const int* __restrict__ n_rec_p, int rec_cap,
                                                   const u64* __restrict__ tile_sum, int* __restrict__ qoff,
-                                                  int* __restrict__ boff, int* __restrict__ n_blocks)
+                                                  int* __restrict__ boff, int* __restrict__ n_blocks, AnnForm form)
 {
     __shared__ u64 lds4[4];
+    const int log_qb = log_queries(form);
     const int n = min(*n_rec_p, rec_cap);
     if (blockIdx.x * kScanTile > n) return;                  // index n itself still gets the closing entries
     u64 before = 0;
@@ -209,7 +220,7 @@ __global__ __launch_bounds__(256) void k_ann_scan(int* __restrict__ cnt, const i
     const int i0 = blockIdx.x * kScanTile + threadIdx.x * 4;
     u64 v[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] = i0 + j < n ? pack_count(cnt[i0 + j]) : 0ull;
+    for (int j = 0; j < 4; ++j) v[j] = i0 + j < n ? pack_count(cnt[i0 + j], log_qb) : 0ull;
     u64 tot;
     u64 run = base + block_scan_256(v[0] + v[1] + v[2] + v[3], &tot, lds4);
 #pragma unroll
@@ -225,13 +236,14 @@ __global__ __launch_bounds__(256) void k_ann_scan(int* __restrict__ cnt, const i
     }
 }
 
-// Thread i < NQ puts query i into the list of its bucket; thread i < n_rec writes the descriptors of the workgroups of
+// Thread i < NQ puts query i into the list of its bucket; thread i < n_rec writes the descriptors of the work items of
 // bucket i: {start and size of the bucket in the tree's permutation, first query in qlist, number of queries}.
 __global__ __launch_bounds__(256) void k_ann_fill(int NQ, const int* __restrict__ q_rec, const int* __restrict__ q_rank,
                                                   const int* __restrict__ n_rec_p, int rec_cap, const TreeRec* __restrict__ recs,
                                                   const int* __restrict__ qoff, const int* __restrict__ boff,
-                                                  int* __restrict__ qlist, int4* __restrict__ blk_desc)
+                                                  int* __restrict__ qlist, int4* __restrict__ blk_desc, AnnForm form)
 {
+    const int qb = 1 << log_queries(form);
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i < NQ) qlist[qoff[q_rec[i]] + q_rank[i]] = i;
     if (i < min(*n_rec_p, rec_cap)) {
@@ -240,8 +252,8 @@ __global__ __launch_bounds__(256) void k_ann_fill(int NQ, const int* __restrict_
             const TreeRec rec = recs[i];
             const int q0 = qoff[i], q1 = qoff[i + 1];
             for (int b = b0; b < b1; ++b) {
-                const int first = q0 + (b - b0) * kQB;
-                blk_desc[b] = make_int4(rec.a, rec.b, first, min(kQB, q1 - first));
+                const int first = q0 + (b - b0) * qb;
+                blk_desc[b] = make_int4(rec.a, rec.b, first, min(qb, q1 - first));
             }
         }
     }
@@ -256,7 +268,7 @@ __device__ __forceinline__ void chain4(float& acc, const float4& a, const float4
     df = a.w - x.w; acc = __builtin_fmaf(df, df, acc);
 }
 
-// Workgroup b works on the bucket and the (up to 16) queries of blk_desc[b].  Per staging step 32 dimensions of up to
+// A workgroup takes the work items b = blockIdx.x, + gridDim.x, ...: the bucket and the (up to 16) queries of blk_desc[b].  Per staging step 32 dimensions of up to
 // 128 bucket rows and of the 16 query rows pass through LDS; a lane reads "its" bucket rows (two: lane, lane + 64)
 // with 16-byte reads and the queries' coordinates as broadcasts.  VEC: D is a multiple of 4 and both matrices are
 // 16-byte aligned.
@@ -264,114 +276,121 @@ template <int SL, bool VEC>
 __global__ __launch_bounds__(256) void k_ann_leaf(const float* __restrict__ points, const float* __restrict__ queries, int D,
                                                   int K, const int* __restrict__ perm, const int4* __restrict__ blk_desc,
                                                   const int* __restrict__ n_blocks, const int* __restrict__ qlist,
-                                                  int* __restrict__ q_idx, float* __restrict__ q_dist)
+                                                  int* __restrict__ q_idx, float* __restrict__ q_dist, AnnForm form)
 {
+    if (form.screened()) return;
     __shared__ __align__(16) float tile[kCG * kTP];
     __shared__ __align__(16) float xs[kQB * kCH];
     __shared__ int cand[kCG];
     __shared__ int qid_s[kQB];
-    const int b = blockIdx.x;
-    if (b >= *n_blocks) return;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int4 desc = blk_desc[b];
-    const int start = desc.x, S = desc.y, q0 = desc.z, nq = desc.w;
-    if (tid < kQB) qid_s[tid] = qlist[q0 + (tid < nq ? tid : 0)];      // slots beyond nq repeat the first query (ignored later)
-    __syncthreads();
-
-    int qid[kQW];
-    bool qv[kQW];
-    KnnRow<SL> row[kQW];
-#pragma unroll
-    for (int i = 0; i < kQW; ++i) {
-        const int slot = i * 4 + wave;                        // queries are dealt out to the four wavefronts in turn
-        qv[i] = slot < nq;
-        qid[i] = __builtin_amdgcn_readfirstlane(qid_s[slot]);
-        row[i].load(q_idx + (size_t)qid[i] * K, q_dist + (size_t)qid[i] * K, K);
-    }
-    const int nqw = (nq - wave + 3) >> 2;                     // queries of this wavefront (0..4), the first nqw slots
-
-    const int piece = tid % kPieces, prow = tid / kPieces;    // staging: kPieces lanes per row
-    const bool stage_x = tid < kQB * kPieces;
-    const float* xp = queries + (size_t)qid_s[stage_x ? prow : 0] * (size_t)D;
-    for (int c0 = 0; c0 < S; c0 += kCG) {
-        const int nc = min(kCG, S - c0);
-        __syncthreads();                                      // the previous pass is done with cand
-        if (tid < kCG) cand[tid] = tid < nc ? perm[start + c0 + tid] : -1;
+    const int n_items = *n_blocks;
+    for (int b = blockIdx.x; b < n_items; b += gridDim.x) {
+        const int4 desc = blk_desc[b];
+        const int start = desc.x, S = desc.y, q0 = desc.z, nq = desc.w;
+        if (tid < kQB) qid_s[tid] = qlist[q0 + (tid < nq ? tid : 0)];      // slots beyond nq repeat the first query (ignored later)
         __syncthreads();
-        const float* rp[kLoads];
-        float4 pre[kLoads];
-        float4 prex = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-        for (int i = 0; i < kLoads; ++i) {
-            const int rr = prow + kRowsPer * i;
-            rp[i] = points + (size_t)cand[rr < nc ? rr : 0] * (size_t)D;       // rows beyond nc repeat row 0 (ignored later)
-            pre[i] = load_piece(rp[i], piece * 4, D, VEC);
-        }
-        if (stage_x) prex = load_piece(xp, piece * 4, D, VEC);
-        float acc0[kQW], acc1[kQW];
-#pragma unroll
-        for (int i = 0; i < kQW; ++i) { acc0[i] = 0.0f; acc1[i] = 0.0f; }
-        const bool two = nc > 64;
-        for (int d0 = 0; d0 < D; d0 += kCH) {
-            __syncthreads();                                  // tile reads of the previous step are done
-#pragma unroll
-            for (int i = 0; i < kLoads; ++i)
-                *reinterpret_cast<float4*>(&tile[(prow + kRowsPer * i) * kTP + piece * 4]) = pre[i];
-            if (stage_x) *reinterpret_cast<float4*>(&xs[prow * kCH + piece * 4]) = prex;
-            if (d0 + kCH < D) {
-#pragma unroll
-                for (int i = 0; i < kLoads; ++i) pre[i] = load_piece(rp[i], d0 + kCH + piece * 4, D, VEC);
-                if (stage_x) prex = load_piece(xp, d0 + kCH + piece * 4, D, VEC);
-            }
-            __syncthreads();
-            const int pieces = min(kPieces, (D - d0 + 3) >> 2);
-            const float* m0 = &tile[lane * kTP];
-            const float* m1 = &tile[(lane + 64) * kTP];
-            const float* x0 = &xs[wave * kCH];                // slot i * 4 + wave: stride 4 rows
-            if (nqw > 2) {
-                for (int p = 0; p < pieces; ++p) {
-                    float4 xv[kQW];
-#pragma unroll
-                    for (int i = 0; i < kQW; ++i) xv[i] = *reinterpret_cast<const float4*>(x0 + i * 4 * kCH + 4 * p);
-                    const float4 a0 = *reinterpret_cast<const float4*>(m0 + 4 * p);
-#pragma unroll
-                    for (int i = 0; i < kQW; ++i) chain4(acc0[i], a0, xv[i]);
-                    if (two) {
-                        const float4 a1 = *reinterpret_cast<const float4*>(m1 + 4 * p);
-#pragma unroll
-                        for (int i = 0; i < kQW; ++i) chain4(acc1[i], a1, xv[i]);
-                    }
-                }
-            } else if (nqw > 0) {
-                for (int p = 0; p < pieces; ++p) {
-                    float4 xv[2];
-#pragma unroll
-                    for (int i = 0; i < 2; ++i) xv[i] = *reinterpret_cast<const float4*>(x0 + i * 4 * kCH + 4 * p);
-                    const float4 a0 = *reinterpret_cast<const float4*>(m0 + 4 * p);
-#pragma unroll
-                    for (int i = 0; i < 2; ++i) chain4(acc0[i], a0, xv[i]);
-                    if (two) {
-                        const float4 a1 = *reinterpret_cast<const float4*>(m1 + 4 * p);
-#pragma unroll
-                        for (int i = 0; i < 2; ++i) chain4(acc1[i], a1, xv[i]);
-                    }
-                }
-            }
-        }
-        const int c_lo = cand[lane], c_hi = cand[lane + 64];
+
+        int qid[kQW];
+        bool qv[kQW];
+        KnnRow<SL> row[kQW];
 #pragma unroll
         for (int i = 0; i < kQW; ++i) {
-            if (qv[i]) {
-                const bool okv[2] = {lane < nc, two && lane + 64 < nc};
-                const int cv[2] = {c_lo, c_hi};
-                const float dv[2] = {acc0[i], acc1[i]};
-                row[i].template merge<2>(okv, cv, dv);
+            const int slot = i * 4 + wave;                        // queries are dealt out to the four wavefronts in turn
+            qv[i] = slot < nq;
+            qid[i] = __builtin_amdgcn_readfirstlane(qid_s[slot]);
+            row[i].load(q_idx + (size_t)qid[i] * K, q_dist + (size_t)qid[i] * K, K);
+        }
+        int n_pass = 0;                                           // pairs of this wavefront that are not above a row's last slot
+        const int nqw = (nq - wave + 3) >> 2;                     // queries of this wavefront (0..4), the first nqw slots
+
+        const int piece = tid % kPieces, prow = tid / kPieces;    // staging: kPieces lanes per row
+        const bool stage_x = tid < kQB * kPieces;
+        const float* xp = queries + (size_t)qid_s[stage_x ? prow : 0] * (size_t)D;
+        for (int c0 = 0; c0 < S; c0 += kCG) {
+            const int nc = min(kCG, S - c0);
+            __syncthreads();                                      // the previous pass is done with cand
+            if (tid < kCG) cand[tid] = tid < nc ? perm[start + c0 + tid] : -1;
+            __syncthreads();
+            const float* rp[kLoads];
+            float4 pre[kLoads];
+            float4 prex = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+            for (int i = 0; i < kLoads; ++i) {
+                const int rr = prow + kRowsPer * i;
+                rp[i] = points + (size_t)cand[rr < nc ? rr : 0] * (size_t)D;       // rows beyond nc repeat row 0 (ignored later)
+                pre[i] = load_piece(rp[i], piece * 4, D, VEC);
+            }
+            if (stage_x) prex = load_piece(xp, piece * 4, D, VEC);
+            float acc0[kQW], acc1[kQW];
+#pragma unroll
+            for (int i = 0; i < kQW; ++i) { acc0[i] = 0.0f; acc1[i] = 0.0f; }
+            const bool two = nc > 64;
+            for (int d0 = 0; d0 < D; d0 += kCH) {
+                __syncthreads();                                  // tile reads of the previous step are done
+#pragma unroll
+                for (int i = 0; i < kLoads; ++i)
+                    *reinterpret_cast<float4*>(&tile[(prow + kRowsPer * i) * kTP + piece * 4]) = pre[i];
+                if (stage_x) *reinterpret_cast<float4*>(&xs[prow * kCH + piece * 4]) = prex;
+                if (d0 + kCH < D) {
+#pragma unroll
+                    for (int i = 0; i < kLoads; ++i) pre[i] = load_piece(rp[i], d0 + kCH + piece * 4, D, VEC);
+                    if (stage_x) prex = load_piece(xp, d0 + kCH + piece * 4, D, VEC);
+                }
+                __syncthreads();
+                const int pieces = min(kPieces, (D - d0 + 3) >> 2);
+                const float* m0 = &tile[lane * kTP];
+                const float* m1 = &tile[(lane + 64) * kTP];
+                const float* x0 = &xs[wave * kCH];                // slot i * 4 + wave: stride 4 rows
+                if (nqw > 2) {
+                    for (int p = 0; p < pieces; ++p) {
+                        float4 xv[kQW];
+#pragma unroll
+                        for (int i = 0; i < kQW; ++i) xv[i] = *reinterpret_cast<const float4*>(x0 + i * 4 * kCH + 4 * p);
+                        const float4 a0 = *reinterpret_cast<const float4*>(m0 + 4 * p);
+#pragma unroll
+                        for (int i = 0; i < kQW; ++i) chain4(acc0[i], a0, xv[i]);
+                        if (two) {
+                            const float4 a1 = *reinterpret_cast<const float4*>(m1 + 4 * p);
+#pragma unroll
+                            for (int i = 0; i < kQW; ++i) chain4(acc1[i], a1, xv[i]);
+                        }
+                    }
+                } else if (nqw > 0) {
+                    for (int p = 0; p < pieces; ++p) {
+                        float4 xv[2];
+#pragma unroll
+                        for (int i = 0; i < 2; ++i) xv[i] = *reinterpret_cast<const float4*>(x0 + i * 4 * kCH + 4 * p);
+                        const float4 a0 = *reinterpret_cast<const float4*>(m0 + 4 * p);
+#pragma unroll
+                        for (int i = 0; i < 2; ++i) chain4(acc0[i], a0, xv[i]);
+                        if (two) {
+                            const float4 a1 = *reinterpret_cast<const float4*>(m1 + 4 * p);
+#pragma unroll
+                            for (int i = 0; i < 2; ++i) chain4(acc1[i], a1, xv[i]);
+                        }
+                    }
+                }
+            }
+            const int c_lo = cand[lane], c_hi = cand[lane + 64];
+#pragma unroll
+            for (int i = 0; i < kQW; ++i) {
+                if (qv[i]) {
+                    const bool okv[2] = {lane < nc, two && lane + 64 < nc};
+                    const int cv[2] = {c_lo, c_hi};
+                    const float dv[2] = {acc0[i], acc1[i]};
+                    n_pass += __popcll(ballot64(okv[0] && dv[0] <= row[i].tau)) + __popcll(ballot64(okv[1] && dv[1] <= row[i].tau));
+                    row[i].template merge<2>(okv, cv, dv);
+                }
             }
         }
-    }
 #pragma unroll
-    for (int i = 0; i < kQW; ++i)
-        if (qv[i] && row[i].changed) row[i].store(q_idx + (size_t)qid[i] * K, q_dist + (size_t)qid[i] * K);
+        for (int i = 0; i < kQW; ++i)
+            if (qv[i] && row[i].changed) row[i].store(q_idx + (size_t)qid[i] * K, q_dist + (size_t)qid[i] * K);
+        if (form.counts(b) && lane == 0)
+            atomicAdd(form.word(b), (unsigned long long)(unsigned)n_pass | (wave == 0 ? (unsigned long long)((unsigned)nq * (unsigned)S) << 32 : 0ull));
+        __syncthreads();                                          // done with the ids before the next item's are written
+    }
 }
 
 // Workgroup q works on query q and the buckets it reached in T trees, wavefront w on those of the trees w, w + 4, ...
@@ -482,9 +501,36 @@ size_t ann_ws_ints(int NQ, int rec_cap)
            2 * ((size_t)rec_cap / kScanTile + 2);
 }
 
-// First use of a workspace: the bucket counters start at zero (every tree leaves them so).
-int launch_ann_ws_init(int* ws, int NQ, int rec_cap, hipStream_t stream)
+// The form of a tree's bucket step: the screened one from this share of the pairs downwards, in 1/65536 (kScreenAlways: whatever
+// the share, 0: never).  A wavefront has 32 queries to itself there, so that it takes 250,000 queries to fill the device
+// (30,000 queries / 20,000 x 100, 20 trees 1.7 -> 2.1 ms) and about 32 of them in a bucket (400,000 / 1M x 50: 19 in a
+// bucket of 48, 10 trees 7.2 -> 7.7); in buckets of up to 24 members, where a wavefront of k_ann_leaf has more lanes
+// than members, 12 will do (1M / 1M x 16, 20 trees 18.5 -> 13.9, 300,000 / 300,000 x 200 19.7 -> 16.9).  Longer rows make the
+// gathers of step 3 dearer: 300,000 / 300,000 x 256 in buckets of 33..66 22.0 -> 22.7 ms, 1M / 1M x 100 78.4 -> 69.6, with the
+// line at 20 to 40 % of the pairs alike, 500,000 / 500,000 x 64 13.5 -> 12.1 (20 to 60 % alike), 1M / 60,000 x 8 12.7 -> 9.4
+// at 60 % and 9.9 at 20 %.
+unsigned int ann_screen_share_q16(int N, int NQ, int D, int n_leaves)
 {
+    double pct = D <= 64 ? 60.0 : 30.0;
+    const char* e = std::getenv("RSFK_ANN_SCREEN");             // (read at every call: tests change it)
+    if (e && *e) {
+        if (e[0] == 'a') return kScreenAlways;
+        pct = e[0] >= '0' && e[0] <= '9' ? std::atof(e) : 0.0;
+    } else {
+        const long long leaves = std::max(n_leaves, 1);
+        const bool narrow = (long long)N <= 24 * leaves;
+        if (D > 128 + (narrow ? 72 : 0) || NQ < 250000 || (long long)NQ < leaves * (narrow ? 12 : 32)) return 0;
+    }
+    return (unsigned int)(std::min(100.0, std::max(0.0, pct)) * 65536.0 / 100.0);
+}
+
+size_t ann_stat_words(int n_trees) { return (size_t)kAnnStatWords * (size_t)n_trees; }
+
+// First use of a workspace: the bucket counters start at zero (every tree leaves them so), and so do the numbers of pairs.
+int launch_ann_ws_init(int* ws, int NQ, int rec_cap, unsigned long long* stats, int n_trees, hipStream_t stream)
+{
+    const int n_stat = (int)(2 * ann_stat_words(n_trees));
+    hipLaunchKernelGGL(k_zero_ints, dim3((unsigned)((n_stat + 255) / 256)), dim3(256), 0, stream, reinterpret_cast<int*>(stats), n_stat);
     int* cnt = ws + (size_t)3 * NQ;
     hipLaunchKernelGGL(k_zero_ints, dim3((unsigned)((rec_cap + 255) / 256)), dim3(256), 0, stream, cnt, rec_cap);
     RSFK_HIP(hipGetLastError());
@@ -493,11 +539,12 @@ int launch_ann_ws_init(int* ws, int NQ, int rec_cap, hipStream_t stream)
 
 // One tree of the query-set search: routes the queries through the index recs (*n_rec_dev records, at most rec_cap;
 // the tree has n_leaves buckets), groups them by bucket and offers the base points perm[..] of the bucket a query
-// reached to the query's row.  ws: ann_ws_ints(NQ, rec_cap) ints, prepared by launch_ann_ws_init; planes: rec_cap rows of
+// reached to the query's row.  prev, stats: numbers of pairs of the tree before this one (null: the first) and of this one,
+// kAnnStatWords each.  ws: ann_ws_ints(NQ, rec_cap) ints, prepared by launch_ann_ws_init; planes: rec_cap rows of
 // ann_plane_pitch(D) floats.
-int launch_ann_tree(const float* points, const float* queries, int NQ, int D, int K, const int* perm, const TreeRec* recs,
+int launch_ann_tree(const float* points, const float* queries, int N, int NQ, int D, int K, const int* perm, const TreeRec* recs,
                     const int* n_rec_dev, int rec_cap, int n_leaves, int* ws, float* planes, int* q_idx, float* q_dist,
-                    hipStream_t stream)
+                    const unsigned long long* prev, unsigned long long* stats, hipStream_t stream)
 {
     if (NQ <= 0) return 0;
     RSFK_CHECK(K >= 1 && K <= kMaxK, "query-set search: K must be in 1..1024");
@@ -522,23 +569,29 @@ int launch_ann_tree(const float* points, const float* queries, int NQ, int D, in
     else
         hipLaunchKernelGGL((k_route<false, false>), dim3(g_route), dim3(256), 0, stream, planes, pitch, queries, NQ, D, recs, rec_cap,
                            q_rec, q_rank, cnt, nullptr);
+    // a bucket with c queries takes ceil(c / 16) work items: at most NQ / 16 + (buckets with queries) in all
+    const int most_items = NQ / kQB + std::min(n_leaves, NQ) + 1;
+    const unsigned int share_q16 = ann_screen_share_q16(N, NQ, D, n_leaves);
+    AnnForm form = {K <= 64 && share_q16 != 0 && D <= kAnnScreenDims ? prev : nullptr, stats, share_q16, 0};
+    while ((most_items >> form.shift) > 512) ++form.shift;
     const unsigned g_scan = (unsigned)(rec_cap / kScanTile + 1);
-    hipLaunchKernelGGL(k_ann_tile_sums, dim3(g_scan), dim3(256), 0, stream, cnt, n_rec_dev, rec_cap, tile_sum);
-    hipLaunchKernelGGL(k_ann_scan, dim3(g_scan), dim3(256), 0, stream, cnt, n_rec_dev, rec_cap, tile_sum, qoff, boff, n_blocks);
+    hipLaunchKernelGGL(k_ann_tile_sums, dim3(g_scan), dim3(256), 0, stream, cnt, n_rec_dev, rec_cap, tile_sum, form);
+    hipLaunchKernelGGL(k_ann_scan, dim3(g_scan), dim3(256), 0, stream, cnt, n_rec_dev, rec_cap, tile_sum, qoff, boff, n_blocks, form);
     const unsigned g_fill = (unsigned)((std::max(NQ, rec_cap) + 255) / 256);
     hipLaunchKernelGGL(k_ann_fill, dim3(g_fill), dim3(256), 0, stream, NQ, q_rec, q_rank, n_rec_dev, rec_cap, recs, qoff, boff, qlist,
-                       blk_desc);
-    // a bucket with c queries takes ceil(c / 16) workgroups: at most NQ / 16 + (buckets with queries) in all
-    const unsigned g_leaf = (unsigned)(NQ / kQB + std::min(n_leaves, NQ) + 1);
+                       blk_desc, form);
+    // (the form that is not taken finds out in every workgroup, hence few of them)
+    if (form.prev && launch_ann_screen(points, queries, D, K, perm, blk_desc, n_blocks, most_items, qlist, q_idx, q_dist, form, stream)) return 1;
+    const unsigned g_leaf = (unsigned)std::min(most_items, kLeafGrid);
     const bool vec = (D & 3) == 0 && ((reinterpret_cast<uintptr_t>(points) | reinterpret_cast<uintptr_t>(queries)) & 15) == 0;
 #define RSFK_ANN_CASE(SLV)                                                                                                   \
     {                                                                                                                        \
         if (vec)                                                                                                             \
             hipLaunchKernelGGL((k_ann_leaf<SLV, true>), dim3(g_leaf), dim3(256), 0, stream, points, queries, D, K, perm,       \
-                               blk_desc, n_blocks, qlist, q_idx, q_dist);                                        \
+                               blk_desc, n_blocks, qlist, q_idx, q_dist, form);                                        \
         else                                                                                                                 \
             hipLaunchKernelGGL((k_ann_leaf<SLV, false>), dim3(g_leaf), dim3(256), 0, stream, points, queries, D, K, perm,       \
-                               blk_desc, n_blocks, qlist, q_idx, q_dist);                                        \
+                               blk_desc, n_blocks, qlist, q_idx, q_dist, form);                                        \
     }
     if (K <= 64) RSFK_ANN_CASE(1)
     else if (K <= 128) RSFK_ANN_CASE(2)

@@ -475,7 +475,7 @@ int knn_ann_forest_device(int n_trees, int K, int N, int NQ, int D, int MIN, int
         if (tree_ws_enable_index(ws.w, MIN, MAX_DEPTH)) return 1;
         const int rec_cap = tree_ws_rec_cap(ws.w);
         const size_t plane_bytes = sizeof(float) * (size_t)rec_cap * (size_t)ann_plane_pitch(D);
-        DevBuf aws, planes, reached;
+        DevBuf aws, planes, reached, pair_stats;
         // trees that are searched together (0, or no memory for it: one tree after the other)
         int group = ann_forest_group(N, NQ, D, K, MAX, rec_cap, std::min(n_trees, B));
         if (group > 0 && (ws_try_alloc(&planes.p, plane_bytes * (size_t)group) ||
@@ -486,7 +486,8 @@ int knn_ann_forest_device(int n_trees, int K, int N, int NQ, int D, int MIN, int
         }
         if (group == 0) {
             if (ws_alloc(&aws.p, sizeof(int) * ann_ws_ints(NQ, rec_cap))) return 1;
-            if (launch_ann_ws_init(static_cast<int*>(aws.p), NQ, rec_cap, stream)) return 1;
+            if (ws_alloc(&pair_stats.p, sizeof(unsigned long long) * ann_stat_words(n_trees))) return 1;
+            if (launch_ann_ws_init(static_cast<int*>(aws.p), NQ, rec_cap, static_cast<unsigned long long*>(pair_stats.p), n_trees, stream)) return 1;
             if (ws_alloc(&planes.p, plane_bytes)) return 1;
         }
         std::vector<int> stats((size_t)5 * B);
@@ -508,9 +509,11 @@ int knn_ann_forest_device(int n_trees, int K, int N, int NQ, int D, int MIN, int
                                        static_cast<int*>(reached.p), d_qidx, d_qdist, stream);
             for (int j = 0; j < nb && rc == 0 && group == 0; ++j) {
                 (void)hipEventRecord(ev[j].e, stream);
-                rc = launch_ann_tree(d_points, d_queries, NQ, D, K, tree_ws_perm(ws.w, j), tree_ws_recs(ws.w, j),
+                rc = launch_ann_tree(d_points, d_queries, N, NQ, D, K, tree_ws_perm(ws.w, j), tree_ws_recs(ws.w, j),
                                      tree_ws_n_rec(ws.w, j), rec_cap, stats[5 * j + 0], static_cast<int*>(aws.p),
-                                     static_cast<float*>(planes.p), d_qidx, d_qdist, stream);
+                                     static_cast<float*>(planes.p), d_qidx, d_qdist,
+                                     tb0 + j > 0 ? static_cast<unsigned long long*>(pair_stats.p) + ann_stat_words(tb0 + j - 1) : nullptr,
+                                     static_cast<unsigned long long*>(pair_stats.p) + ann_stat_words(tb0 + j), stream);
             }
             (void)hipEventRecord(ev[nb].e, stream);
             if (rc) break;

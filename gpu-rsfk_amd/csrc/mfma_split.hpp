@@ -21,11 +21,9 @@ __device__ __forceinline__ void split2(float a, float b, uint32_t& hi, uint32_t&
     lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, bf16x2));
 }
 
-// Eight consecutive values of a row in LDS -> matrix-core operands (heads and remainders); adds their squares to nrm.
-__device__ __forceinline__ void load_split(const float* __restrict__ p, bf16x8& hi, bf16x8& lo, float& nrm)
+// Eight consecutive values of a row -> matrix-core operands (heads and remainders); adds their squares to nrm.
+__device__ __forceinline__ void split8(const float4& u, const float4& v, bf16x8& hi, bf16x8& lo, float& nrm)
 {
-    const float4 u = *reinterpret_cast<const float4*>(p);
-    const float4 v = *reinterpret_cast<const float4*>(p + 4);
     uint4 h, l;
     split2(u.x, u.y, h.x, l.x);
     split2(u.z, u.w, h.y, l.y);
@@ -37,6 +35,12 @@ __device__ __forceinline__ void load_split(const float* __restrict__ p, bf16x8& 
     nrm = __builtin_fmaf(u.z, u.z, nrm); nrm = __builtin_fmaf(u.w, u.w, nrm);
     nrm = __builtin_fmaf(v.x, v.x, nrm); nrm = __builtin_fmaf(v.y, v.y, nrm);
     nrm = __builtin_fmaf(v.z, v.z, nrm); nrm = __builtin_fmaf(v.w, v.w, nrm);
+}
+
+// ... of a row in LDS
+__device__ __forceinline__ void load_split(const float* __restrict__ p, bf16x8& hi, bf16x8& lo, float& nrm)
+{
+    split8(*reinterpret_cast<const float4*>(p), *reinterpret_cast<const float4*>(p + 4), hi, lo, nrm);
 }
 
 // Coefficient c of the bound |d~ - d| <= c S, S = |a|^2 + |b|^2, d~ = |a|^2 + |b|^2 - 2 G with G from the three

@@ -795,6 +795,37 @@ def test_ann_trees_together_match_oracle(gpu, capi, orc, rng, monkeypatch, N, NQ
         assert_knn_equal(idx.cpu().numpy(), dist.cpu().numpy(), oi, od)
 
 
+# items of fewer and of more than 32 queries; buckets on both sides of 32 and 64 members; rows that end inside a step and inside
+# a 16-byte piece; distances that overflow, a common offset that leaves the bounds useless, equal distances
+@pytest.mark.parametrize("N,NQ,D,K,T,mn,mx", [(500, 900, 16, 64, 5, 65, 130), (3000, 2500, 100, 32, 6, 33, 66), (700, 333, 31, 5, 9, 6, 12),
+                                              (400, 65, 3, 10, 4, 200, 400), (900, 64, 33, 1, 3, 32, 64), (600, 1000, 130, 20, 4, 21, 33)])
+@pytest.mark.parametrize("data", ["normal", "ties", "offset", "huge"])
+def test_ann_screened_buckets_match_oracle(gpu, capi, orc, rng, monkeypatch, N, NQ, D, K, T, mn, mx, data):
+    """The bucket step that bounds the pairs on the matrix cores first (from the second tree on) == the oracle, also into rows
+    that hold something and are not in order."""
+    import torch
+    draw = {"normal": lambda n: rng.standard_normal((n, D)), "ties": lambda n: rng.integers(0, 3, (n, D)),
+            "offset": lambda n: rng.standard_normal((n, D)) * 1e-2 + 300.0,
+            "huge": lambda n: rng.standard_normal((n, D)) * np.where(rng.random((n, 1)) < 0.1, 3e18, 1.0)}[data]
+    X, Q = draw(N).astype(np.float32), draw(NQ).astype(np.float32)
+    dX, dQ = torch.from_numpy(X).cuda(), torch.from_numpy(Q).cuda()
+    oi, od = orc.ann_forest(X, Q, K, T, mn, mx, 5000, 5)
+    monkeypatch.setenv("RSFK_ANN_FOREST", "0")
+    monkeypatch.setenv("RSFK_ANN_SCREEN", "always")
+    monkeypatch.setenv("RSFK_TREE_SCREEN", "bf16")     # (where sums overflow the 8-bit side tests may part from the oracle's)
+    idx = torch.full((NQ, K), -1, dtype=torch.int32, device="cuda")
+    dist = torch.full((NQ, K), float("inf"), dtype=torch.float32, device="cuda")
+    _say("ann screened", N, NQ, D, K, T, mn, mx, data)
+    capi.knn_ann_device(T, K, N, NQ, D, mn, mx, 5000, 0, 5, dX.data_ptr(), dQ.data_ptr(), idx.data_ptr(), dist.data_ptr())
+    torch.cuda.synchronize()
+    assert_knn_equal(idx.cpu().numpy(), dist.cpu().numpy(), oi, od)
+    idx, dist = idx.flip(1).contiguous(), dist.flip(1).contiguous()
+    orc.ann_forest(X, Q, K, 2, mn, mx, 5000, 77, q_idx=oi, q_dist=od)
+    capi.knn_ann_device(2, K, N, NQ, D, mn, mx, 5000, 0, 77, dX.data_ptr(), dQ.data_ptr(), idx.data_ptr(), dist.data_ptr())
+    torch.cuda.synchronize()
+    assert_knn_equal(idx.cpu().numpy(), dist.cpu().numpy(), oi, od)
+
+
 def test_ann_device_entry_point_merges_into_given_rows(gpu, capi, orc, rng):
     """Device-resident call, twice with different seeds on the same rows == the oracle doing the same."""
     import torch
