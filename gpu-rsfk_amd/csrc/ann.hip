@@ -52,16 +52,23 @@ __global__ __launch_bounds__(256) void k_zero_ints(int* __restrict__ p, int n)
 // [offset, 0, 0, 0 | normal, zero padded to a multiple of 4].  Normal and offset are the values the builder works with
 // (create_node.cu:122-135: n = x1 - x2, offset = sum n_d (x1_d + x2_d) / 2 as 32 lane-strided partial sums + xor butterfly).
 // blockIdx.y: the tree; the records and the rows of a tree begin rec_cap after those of the tree before it.
+// low (null: none): the rows the queries are routed by first, low_pitch floats each: {offset, E, children | normal rounded to
+// bfloat16}, E = (|n - n~| + 2.1 gamma |n|)(1 + 2^-9) with the rounding error as it is and gamma for the fp32 sums of either
+// evaluation: |n.x as the builder sums it - n~.x as k_route sums it| <= E |x|.  A bucket has children -1.
 __global__ __launch_bounds__(256) void k_planes(const float* __restrict__ points, int D, const TreeRec* __restrict__ recs,
                                                 const int* __restrict__ n_rec_p, int rec_cap, float* __restrict__ planes,
-                                                int pitch)
+                                                int pitch, float* __restrict__ low, int low_pitch)
 {
     const int lane = threadIdx.x & 63;
     const int r = blockIdx.x * 4 + (threadIdx.x >> 6), j = blockIdx.y;
     if (r >= min(n_rec_p[j], rec_cap)) return;
     const size_t at = (size_t)j * (size_t)rec_cap + (size_t)r;
     const TreeRec rec = recs[at];
-    if (rec.c0 < 0) return;
+    float* low_row = low ? low + at * (size_t)low_pitch : nullptr;
+    if (rec.c0 < 0) {
+        if (low && lane == 0) *reinterpret_cast<int4*>(low_row) = make_int4(0, 0, -1, -1);
+        return;
+    }
     const float* x1 = points + (size_t)rec.a * (size_t)D;
     const float* x2 = points + (size_t)rec.b * (size_t)D;
     float* row = planes + at * (size_t)pitch;
@@ -76,7 +83,28 @@ __global__ __launch_bounds__(256) void k_planes(const float* __restrict__ points
     }
     s = half_butterfly_sum(s);
     if (lane < 4) row[lane] = lane == 0 ? s : 0.0f;
-    for (int d = lane; d < pitch - 4; d += 64) row[4 + d] = d < D ? x1[d] - x2[d] : 0.0f;
+    float err2 = 0.0f, nrm2 = 0.0f;
+    uint16_t* low_n = low ? reinterpret_cast<uint16_t*>(low_row + 4) : nullptr;
+    for (int d = lane; d < pitch - 4; d += 64) {
+        const float nd = d < D ? x1[d] - x2[d] : 0.0f;
+        row[4 + d] = nd;
+        if (low) {
+            const __bf16 h = (__bf16)nd;
+            const float e = nd - (float)h;
+            err2 = __builtin_fmaf(e, e, err2);
+            nrm2 = __builtin_fmaf(nd, nd, nrm2);
+            low_n[d] = __builtin_bit_cast(uint16_t, h);
+        }
+    }
+    if (!low) return;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        err2 += __shfl_xor(err2, o, 64);
+        nrm2 += __shfl_xor(nrm2, o, 64);
+    }
+    const float gamma = (float)(D + 64) * (1.0f / 8388608.0f);
+    const float E = (sqrtf(err2) + 2.1f * gamma * sqrtf(nrm2)) * (1.0f + 1.0f / 512.0f) + 2e-17f;     // (squares that underflow)
+    if (lane == 0) *reinterpret_cast<int4*>(low_row) = make_int4(__float_as_int(s), __float_as_int(E), rec.c0, rec.c1);
 }
 
 // Eight lanes per query.  A lane owns four of the 32 partial sums of the side test (sums 4s..4s+3 of
@@ -150,6 +178,101 @@ __global__ __launch_bounds__(256) void k_route(const float* __restrict__ planes,
                 done = true;
             } else {
                 cur = t < b ? r.c1 : r.c0;
+            }
+        }
+        if (ballot64(!done) == 0) break;
+    }
+}
+
+// The same for many queries of 65 to 128 dimensions, by the rounded hyperplanes of k_planes: the side is certain when
+// |n~.x - offset| > E |x|, otherwise (1 % of the tests on uniform points) the exact test follows.  Sums of squares that
+// overflow, infinities and NaN leave a test uncertain.
+// k_route is bound by the hyperplanes' bytes from beyond the L2 (16 MB a tree at 1M x 100); these are half as many: 1M queries
+// 0.56 -> 0.49 ms a tree.  Rows of up to 64 dimensions gain nothing (500,000 / 100,000 x 64: search 8.25 -> 8.21 ms) or lose
+// (1M / 1M x 16 14.1 -> 14.6), and so do few queries, for which the second trip counts (20,000 / 1M x 100, 50 trees
+// 8.65 -> 9.01 ms, 100,000, 20 trees 6.91 -> 6.82).
+template <bool VEC>
+__global__ __launch_bounds__(256) void k_route_low(const float* __restrict__ planes, int pitch, const float* __restrict__ low, int low_pitch,
+                                                   const float* __restrict__ queries, int NQ, int D, int rec_cap,
+                                                   int* __restrict__ q_rec, int* __restrict__ q_rank, int* __restrict__ cnt)
+{
+    const int sub = threadIdx.x & 7;
+    const int q = (int)((blockIdx.x * (size_t)blockDim.x + threadIdx.x) >> 3);
+    const bool valid = q < NQ;
+    const float* x = queries + (size_t)(valid ? q : 0) * (size_t)D;
+    const int Dp = pitch - 4;
+    float4 xr[kXR];
+    float norm = 0.0f;
+#pragma unroll
+    for (int k = 0; k < kXR; ++k) {
+        xr[k] = load_piece(x, 32 * k + 4 * sub, D, VEC);
+        norm = __builtin_fmaf(xr[k].x, xr[k].x, norm);
+        norm = __builtin_fmaf(xr[k].y, xr[k].y, norm);
+        norm = __builtin_fmaf(xr[k].z, xr[k].z, norm);
+        norm = __builtin_fmaf(xr[k].w, xr[k].w, norm);
+    }
+    auto group_sum = [](float t) {                       // the last three steps of the butterfly, over the eight lanes
+        t += dpp_f<kDppXor1>(t);
+        t += dpp_f<kDppXor2>(t);
+        t += dpp_f<kDppHalfMirror>(t);
+        return t;
+    };
+    norm = sqrtf(group_sum(norm)) * (1.0f + 1.0f / 512.0f) + 2e-17f;
+    int cur = 0;
+    bool done = !valid;
+    for (int step = 0; step <= rec_cap; ++step) {            // a path is never longer than the number of records
+        const float* lrow = low + (size_t)(done ? 0 : cur) * (size_t)low_pitch;
+        const int4 head = *reinterpret_cast<const int4*>(lrow);
+        uint2 h[kXR];
+#pragma unroll
+        for (int k = 0; k < kXR; ++k) {
+            const int d = 32 * k + 4 * sub;
+            h[k] = d < Dp ? *reinterpret_cast<const uint2*>(lrow + 4 + (d >> 1)) : make_uint2(0u, 0u);
+        }
+        float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
+#pragma unroll
+        for (int k = 0; k < kXR; ++k) {
+            s0 = __builtin_fmaf(__uint_as_float(h[k].x << 16), xr[k].x, s0);
+            s1 = __builtin_fmaf(__uint_as_float(h[k].x & 0xffff0000u), xr[k].y, s1);
+            s2 = __builtin_fmaf(__uint_as_float(h[k].y << 16), xr[k].z, s2);
+            s3 = __builtin_fmaf(__uint_as_float(h[k].y & 0xffff0000u), xr[k].w, s3);
+        }
+        const float t = group_sum((s0 + s1) + (s2 + s3));
+        const float b = __int_as_float(head.x);
+        const bool bucket = head.z < 0;
+        bool below = t < b;
+        // (below 1e33 the bound, at least 2 gamma |n| |x|, leaves no room for a sum that overflows)
+        const float margin = fabsf(t - b), bound = __builtin_fmaf(__int_as_float(head.y), norm, 1e-35f);
+        const bool certain = margin > bound && margin < INFINITY && bound < 1e33f;
+        const bool ask = !done && !bucket && !certain;       // (the eight lanes of a query agree)
+        if (ballot64(ask) != 0) {
+            const float* pl = planes + (size_t)(ask ? cur : 0) * (size_t)pitch + 4;
+            s0 = s1 = s2 = s3 = 0.0f;
+            float4 n4[kXR];
+#pragma unroll
+            for (int k = 0; k < kXR; ++k) {
+                const int d = 32 * k + 4 * sub;
+                n4[k] = ask && d < Dp ? *reinterpret_cast<const float4*>(pl + d) : make_float4(0.f, 0.f, 0.f, 0.f);
+            }
+#pragma unroll
+            for (int k = 0; k < kXR; ++k) {
+                s0 = __builtin_fmaf(n4[k].x, xr[k].x, s0);
+                s1 = __builtin_fmaf(n4[k].y, xr[k].y, s1);
+                s2 = __builtin_fmaf(n4[k].z, xr[k].z, s2);
+                s3 = __builtin_fmaf(n4[k].w, xr[k].w, s3);
+            }
+            const float exact = group_sum((s0 + s1) + (s2 + s3));
+            if (ask) below = exact < b;
+        }
+        if (!done) {
+            if (bucket) {
+                if (sub == 0) {
+                    q_rec[q] = cur;
+                    q_rank[q] = atomicAdd(&cnt[cur], 1);
+                }
+                done = true;
+            } else {
+                cur = below ? head.w : head.z;
             }
         }
         if (ballot64(!done) == 0) break;
@@ -490,8 +613,23 @@ __global__ __launch_bounds__(256) void k_ann_forest(const float* __restrict__ po
 
 }  // namespace
 
+namespace {
+
 // floats per row of the table of hyperplanes: offset (4 floats) + normal padded to a multiple of 4
-int ann_plane_pitch(int D) { return 4 + ((D + 3) & ~3); }
+int plane_pitch(int D) { return 4 + ((D + 3) & ~3); }
+// ... of the rounded ones; 0: not made (see k_route_low).  RSFK_ANN_ROUTE_LOW=1 / 0 says yes or no.
+int low_plane_pitch(int NQ, int D)
+{
+    if (D > 32 * kXR) return 0;
+    const char* e = std::getenv("RSFK_ANN_ROUTE_LOW");
+    const bool wanted = e && *e ? e[0] == '1' : D > 64 && NQ >= 100000;
+    return wanted ? 4 + ((D + 7) & ~7) / 2 : 0;
+}
+
+}  // namespace
+
+// floats of working memory a record of a tree takes (both tables of hyperplanes)
+int ann_plane_pitch(int NQ, int D) { return plane_pitch(D) + low_plane_pitch(NQ, D); }
 
 size_t ann_ws_ints(int NQ, int rec_cap)
 {
@@ -540,8 +678,8 @@ int launch_ann_ws_init(int* ws, int NQ, int rec_cap, unsigned long long* stats, 
 // One tree of the query-set search: routes the queries through the index recs (*n_rec_dev records, at most rec_cap;
 // the tree has n_leaves buckets), groups them by bucket and offers the base points perm[..] of the bucket a query
 // reached to the query's row.  prev, stats: numbers of pairs of the tree before this one (null: the first) and of this one,
-// kAnnStatWords each.  ws: ann_ws_ints(NQ, rec_cap) ints, prepared by launch_ann_ws_init; planes: rec_cap rows of
-// ann_plane_pitch(D) floats.
+// kAnnStatWords each.  ws: ann_ws_ints(NQ, rec_cap) ints, prepared by launch_ann_ws_init; planes: rec_cap
+// ann_plane_pitch(NQ, D) floats.
 int launch_ann_tree(const float* points, const float* queries, int N, int NQ, int D, int K, const int* perm, const TreeRec* recs,
                     const int* n_rec_dev, int rec_cap, int n_leaves, int* ws, float* planes, int* q_idx, float* q_dist,
                     const unsigned long long* prev, unsigned long long* stats, hipStream_t stream)
@@ -558,12 +696,19 @@ int launch_ann_tree(const float* points, const float* queries, int N, int NQ, in
     int4* blk_desc = reinterpret_cast<int4*>(ws + (((boff + rec_cap + 1) - ws + 3) & ~(ptrdiff_t)3));
     int* n_blocks = reinterpret_cast<int*>(blk_desc + ((size_t)NQ / kQB + rec_cap + 1));
     u64* tile_sum = reinterpret_cast<u64*>(ws + ((ann_ws_ints(NQ, rec_cap) - 2 * ((size_t)rec_cap / kScanTile + 2)) & ~(size_t)1));
-    const int pitch = ann_plane_pitch(D);
-    hipLaunchKernelGGL(k_planes, dim3((unsigned)((rec_cap + 3) / 4)), dim3(256), 0, stream, points, D, recs, n_rec_dev, rec_cap,
-                       planes, pitch);
+    const int pitch = plane_pitch(D), low_pitch = low_plane_pitch(NQ, D);
+    float* low = low_pitch ? planes + (size_t)rec_cap * (size_t)pitch : nullptr;
+    hipLaunchKernelGGL(k_planes, dim3((unsigned)((rec_cap + 3) / 4)), dim3(256), 0, stream, points, D, recs, n_rec_dev, rec_cap, planes,
+                       pitch, low, low_pitch);
     const unsigned g_route = (unsigned)(((size_t)NQ * 8 + 255) / 256);
     const bool vec_q = (D & 3) == 0 && (reinterpret_cast<uintptr_t>(queries) & 15) == 0;
-    if (vec_q)
+    if (low && vec_q)
+        hipLaunchKernelGGL(k_route_low<true>, dim3(g_route), dim3(256), 0, stream, planes, pitch, low, low_pitch, queries, NQ, D, rec_cap,
+                           q_rec, q_rank, cnt);
+    else if (low)
+        hipLaunchKernelGGL(k_route_low<false>, dim3(g_route), dim3(256), 0, stream, planes, pitch, low, low_pitch, queries, NQ, D, rec_cap,
+                           q_rec, q_rank, cnt);
+    else if (vec_q)
         hipLaunchKernelGGL((k_route<true, false>), dim3(g_route), dim3(256), 0, stream, planes, pitch, queries, NQ, D, recs, rec_cap,
                            q_rec, q_rank, cnt, nullptr);
     else
@@ -622,22 +767,22 @@ int ann_forest_group(int N, int NQ, int D, int K, int MAX, int rec_cap, int nb)
     constexpr double kMostFloats = 5e7;
     if (!forced && (double)NQ * (double)MAX * (double)D > kMostFloats) return 0;
     // hyperplanes and buckets reached: 1 GB at most
-    const size_t per_tree = sizeof(float) * (size_t)rec_cap * (size_t)ann_plane_pitch(D) + sizeof(int2) * (size_t)NQ;
+    const size_t per_tree = sizeof(float) * (size_t)rec_cap * (size_t)ann_plane_pitch(NQ, D) + sizeof(int2) * (size_t)NQ;
     const int group = (int)std::min<size_t>((size_t)std::min(nb, 64), ((size_t)1 << 30) / per_tree);
     return group >= 2 ? group : 0;
 }
 
-// The search in T trees at once.  recs, n_rec_dev, perm: those of the first tree, the others follow; planes: T rec_cap rows of
-// ann_plane_pitch(D) floats; reached: 2 NQ T ints.
+// The search in T trees at once.  recs, n_rec_dev, perm: those of the first tree, the others follow; planes: T rec_cap
+// ann_plane_pitch(NQ, D) floats; reached: 2 NQ T ints.
 int launch_ann_forest(const float* points, const float* queries, int N, int NQ, int D, int K, int T, const int* perm, const TreeRec* recs,
                       const int* n_rec_dev, int rec_cap, float* planes, int* reached, int* q_idx, float* q_dist, hipStream_t stream)
 {
     RSFK_CHECK(K >= 1 && K <= kMaxK && T >= 1 && T <= 64, "query-set search: out of range");
     RSFK_CHECK(recs != nullptr && rec_cap >= 1, "query-set search: the tree has no index");
-    const int pitch = ann_plane_pitch(D);
     int2* where = reinterpret_cast<int2*>(reached);
+    const int pitch = plane_pitch(D);
     hipLaunchKernelGGL(k_planes, dim3((unsigned)((rec_cap + 3) / 4), (unsigned)T), dim3(256), 0, stream, points, D, recs, n_rec_dev, rec_cap,
-                       planes, pitch);
+                       planes, pitch, nullptr, 0);
     const dim3 g_route((unsigned)(((size_t)NQ * 8 + 255) / 256), (unsigned)T);
     const bool vec_q = (D & 3) == 0 && (reinterpret_cast<uintptr_t>(queries) & 15) == 0;
     if (vec_q)

@@ -474,7 +474,7 @@ int knn_ann_forest_device(int n_trees, int K, int N, int NQ, int D, int MIN, int
         if (tree_ws_alloc(&ws.w, N, D, MIN, B)) return 1;
         if (tree_ws_enable_index(ws.w, MIN, MAX_DEPTH)) return 1;
         const int rec_cap = tree_ws_rec_cap(ws.w);
-        const size_t plane_bytes = sizeof(float) * (size_t)rec_cap * (size_t)ann_plane_pitch(D);
+        const size_t plane_bytes = sizeof(float) * (size_t)rec_cap * (size_t)ann_plane_pitch(NQ, D);
         DevBuf aws, planes, reached, pair_stats;
         // trees that are searched together (0, or no memory for it: one tree after the other)
         int group = ann_forest_group(N, NQ, D, K, MAX, rec_cap, std::min(n_trees, B));

@@ -177,7 +177,7 @@ int symmetrize_host(const int* idx, const float* dist, int N, int K, int drop_se
 
 // ann.hip
 size_t ann_ws_ints(int NQ, int rec_cap);
-int ann_plane_pitch(int D);
+int ann_plane_pitch(int NQ, int D);
 size_t ann_stat_words(int n_trees);
 int launch_ann_ws_init(int* ws, int NQ, int rec_cap, unsigned long long* stats, int n_trees, hipStream_t stream);
 int launch_ann_tree(const float* points, const float* queries, int N, int NQ, int D, int K, const int* perm, const TreeRec* recs,

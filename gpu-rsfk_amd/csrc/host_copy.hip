@@ -6,10 +6,10 @@
 //     pieces, the memcpy of a piece beside the DMA of the piece before; copies to the device are only queued on the
 //     caller's stream (2.4 MB: 101 us with hipMemcpy, 56 us here).
 //   large ones: host threads take pieces of 2 MB in turn, each through its own pair of pinned buffers (hipHostMalloc;
-//     registering the caller's memory is not an option) on its own stream: the memcpy of one piece overlaps the DMA of
+//     registering the caller's memory is not an option) on one of two streams: the memcpy of one piece overlaps the DMA of
 //     the previous one and the threads overlap each other.  What bounds it is the link (57 GB/s each way); one thread
-//     copies 10 GB/s or so, less where the destination's pages are touched for the first time, hence eight threads
-//     (16 cores on the box).  Four threads with pieces of 8 MB, the form before, had nothing to overlap below 64 MB.
+//     copies 10 GB/s or so, less where the destination's pages are touched for the first time, hence eight threads.
+//     Four threads with pieces of 8 MB, the form before, had nothing to overlap below 64 MB.
 // The buffers and streams are kept for the next call; rsfk_release_workspace() frees them.
 #include "rsfk_common.hpp"
 #include "forest.hpp"

@@ -127,7 +127,7 @@ void ws_free(void* p)
 // ---- pinned host memory and side streams --------------------------------------------------------------------------
 //
 // A call needs a few pinned blocks (counters that come back from the device, small arrays on their way) and most calls
-// a second stream.  hipHostMalloc + hipHostFree take 26 us and hipStreamCreate + Destroy 57 us on the box, which
+// a second stream.  hipHostMalloc + hipHostFree take 26 us and hipStreamCreate + Destroy 57 us, which
 // together was a fifth of a small call (10,000 x 32 points, 4 trees: 0.35 of 1.8 ms), so both are kept for the next
 // call: at most 64 MB of idle pinned blocks (rounded up to powers of two) and eight idle streams.
 namespace {

@@ -775,17 +775,21 @@ def test_find_nearest_neighbors_ann_matches_oracle(gpu, orc, rng, N, NQ, D, K, T
 @pytest.mark.parametrize("N,NQ,D,K,T,mn,mx", [(300, 1, 1, 1, 2, 3, 6), (2000, 37, 33, 64, 5, 65, 65 * 2), (1500, 300, 64, 65, 9, 66, 128),
                                               (900, 130, 31, 16, 3, 17, 64), (700, 65, 100, 300, 4, 301, 700), (4000, 90, 7, 5, 70, 6, 12),
                                               (50, 20, 12, 8, 6, 60, 120), (1200, 33, 260, 20, 8, 21, 65)])
-@pytest.mark.parametrize("data", ["normal", "ties"])
+@pytest.mark.parametrize("data", ["normal", "ties", "tiny"])
 def test_ann_trees_together_match_oracle(gpu, capi, orc, rng, monkeypatch, N, NQ, D, K, T, mn, mx, data):
     """All trees of a query in one workgroup == one tree after the other == the oracle, also into rows that hold something."""
     import torch
-    draw = (lambda n: rng.integers(0, 3, (n, D)).astype(np.float32)) if data == "ties" else (lambda n: rng.standard_normal((n, D)).astype(np.float32))
+    if data == "ties":          # points on the hyperplanes: sides that the rounded hyperplanes cannot decide
+        draw = lambda n: rng.integers(0, 3, (n, D)).astype(np.float32)
+    else:                       # "tiny": squares of rounding errors underflow
+        draw = lambda n: (rng.standard_normal((n, D)) * (1e-18 if data == "tiny" else 1.0)).astype(np.float32)
     X, Q = draw(N), draw(NQ)
     dX, dQ = torch.from_numpy(X).cuda(), torch.from_numpy(Q).cuda()
     oi, od = orc.ann_forest(X, Q, K, T, mn, mx, 5000, 5)
     orc.ann_forest(X, Q, K, 2, mn, mx, 5000, 77, q_idx=oi, q_dist=od)
-    for form in ("0", "1"):
-        monkeypatch.setenv("RSFK_ANN_FOREST", form)
+    for form in ("0", "1", "low"):                        # "low": one after the other, routed by the rounded hyperplanes
+        monkeypatch.setenv("RSFK_ANN_FOREST", "1" if form == "1" else "0")
+        monkeypatch.setenv("RSFK_ANN_ROUTE_LOW", "1" if form == "low" else "0")
         idx = torch.full((NQ, K), -1, dtype=torch.int32, device="cuda")
         dist = torch.full((NQ, K), float("inf"), dtype=torch.float32, device="cuda")
         _say("ann together", N, NQ, D, K, T, mn, mx, data, form)
@@ -812,6 +816,7 @@ def test_ann_screened_buckets_match_oracle(gpu, capi, orc, rng, monkeypatch, N, 
     oi, od = orc.ann_forest(X, Q, K, T, mn, mx, 5000, 5)
     monkeypatch.setenv("RSFK_ANN_FOREST", "0")
     monkeypatch.setenv("RSFK_ANN_SCREEN", "always")
+    monkeypatch.setenv("RSFK_ANN_ROUTE_LOW", "1")
     monkeypatch.setenv("RSFK_TREE_SCREEN", "bf16")     # (where sums overflow the 8-bit side tests may part from the oracle's)
     idx = torch.full((NQ, K), -1, dtype=torch.int32, device="cuda")
     dist = torch.full((NQ, K), float("inf"), dtype=torch.float32, device="cuda")
