@@ -420,10 +420,11 @@ int symmetrize_device(const int* d_idx, const float* d_dist, int N, int K, int d
     RSFK_CHECK((long long)N * K < (1ll << 30), "graph export: N * K of 2^30 and more is not supported");
     RSFK_CHECK(d_idx && d_indptr && nnz, "graph export: null argument");
     RSFK_CHECK((d_cols == nullptr) == (d_vals == nullptr), "graph export: indices and data go together");
-    // Graphs of less than 24,576 entries take fewer launches the other way (2,000 x 8: 0.054 against 0.081 ms;
-    // 4,000 x 8: 0.089 against 0.074).  RSFK_GRAPH_FLAGS=1 / 0 says which form (the results are the same).
+    // Up to about 2,800 points the library's sort takes few launches and the other form fewer in all (2,000 x 32: 0.057 against
+    // 0.059 ms, 2,000 x 128: 0.102 against 0.141; 2,500 x 8: 0.049 against 0.048); from there on it takes more (3,000 x 8: 0.076
+    // against 0.050, 3,000 x 90: 0.118 against 0.101).  RSFK_GRAPH_FLAGS=1 / 0 says which form (the results are the same).
     const char* form = std::getenv("RSFK_GRAPH_FLAGS");
-    if (!explore_ws_takes(N, K) || (form && *form ? form[0] == '1' : (size_t)N * (size_t)K < 24576))
+    if (!explore_ws_takes(N, K) || (form && *form ? form[0] == '1' : N < 2800))
         return symmetrize_flags(d_idx, d_dist, N, K, drop_self, d_indptr, d_cols, d_vals, cap, nnz, stream);
     RevGuard rg;
     Buf len, big, ctr;
