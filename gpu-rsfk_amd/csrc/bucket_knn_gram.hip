@@ -82,14 +82,7 @@ struct TileLoads {
             v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
             if (m < rows && piece < np4 && d < D) {
                 const float* src = points + (size_t)ids[m] * (size_t)D + d;
-                if (vec_ok) {
-                    v[i] = *reinterpret_cast<const float4*>(src);
-                } else {
-                    v[i].x = src[0];
-                    if (d + 1 < D) v[i].y = src[1];
-                    if (d + 2 < D) v[i].z = src[2];
-                    if (d + 3 < D) v[i].w = src[3];
-                }
+                v[i] = load_dims(src, D - d, vec_ok);
             }
         }
     }

@@ -71,16 +71,7 @@ __global__ __launch_bounds__(kRowsThreads) void k_bucket_knn_rows(const float* _
     for (int it = tid; it < s * np; it += kRowsThreads) {
         const int m = it / np, pc = it - m * np;
         const float* src = points + (size_t)lids[m] * (size_t)D + 4 * pc;
-        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (vec_ok) {
-            v = *reinterpret_cast<const float4*>(src);
-        } else {
-            const int left = D - 4 * pc;
-            v.x = src[0];
-            if (left > 1) v.y = src[1];
-            if (left > 2) v.z = src[2];
-            if (left > 3) v.w = src[3];
-        }
+        const float4 v = load_dims(src, D - 4 * pc, vec_ok);
         *reinterpret_cast<float4*>(&rows[m * pitch + 4 * pc]) = v;
     }
     __syncthreads();

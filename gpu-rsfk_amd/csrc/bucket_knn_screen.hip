@@ -90,14 +90,7 @@ struct RowLoads {
             v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
             if (m < s && d < D) {
                 const float* src = points + (size_t)lids[m] * (size_t)D + d;
-                if (vec_ok) {
-                    v[i] = *reinterpret_cast<const float4*>(src);
-                } else {
-                    v[i].x = src[0];
-                    if (d + 1 < D) v[i].y = src[1];
-                    if (d + 2 < D) v[i].z = src[2];
-                    if (d + 3 < D) v[i].w = src[3];
-                }
+                v[i] = load_dims(src, D - d, vec_ok);
             }
         }
     }

@@ -27,9 +27,9 @@ struct StagedRows {
         if (r < rows && d0 + seg < D) {
             const float* src = points + (size_t)ids[r] * (size_t)D + d0 + seg;
             const int left = D - d0 - seg;
-            if (vec_ok && left >= 8) {
-                const float4 q0 = *reinterpret_cast<const float4*>(src);
-                const float4 q1 = *reinterpret_cast<const float4*>(src + 4);
+            if (left >= 8) {
+                const float4 q0 = load_dims(src, 4, vec_ok);
+                const float4 q1 = load_dims(src + 4, 4, vec_ok);
                 v[0] = q0.x; v[1] = q0.y; v[2] = q0.z; v[3] = q0.w;
                 v[4] = q1.x; v[5] = q1.y; v[6] = q1.z; v[7] = q1.w;
             } else {

@@ -164,15 +164,7 @@ __device__ __forceinline__ void small_bucket_body(float* __restrict__ lds_f, con
             if (it < items) {
                 const int m = it / np, pc = it - m * np;
                 const float* src = points + (size_t)lids[m] * (size_t)D + d0 + 4 * pc;
-                if (vec_ok) {
-                    pre[i] = *reinterpret_cast<const float4*>(src);
-                } else {
-                    const int left = D - d0 - 4 * pc;
-                    pre[i].x = src[0];
-                    if (left > 1) pre[i].y = src[1];
-                    if (left > 2) pre[i].z = src[2];
-                    if (left > 3) pre[i].w = src[3];
-                }
+                pre[i] = load_dims(src, D - d0 - 4 * pc, vec_ok);
             }
         }
         if (d0 == 0 && tid < kCap) tau[tid] = tau_own;

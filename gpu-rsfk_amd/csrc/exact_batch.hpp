@@ -24,18 +24,7 @@ struct ExploreLds {          // per wavefront; sizes fixed at launch
 // Load one 16-byte piece (4 dimensions) of a candidate row, zero beyond D.
 __device__ __forceinline__ float4 load_piece(const float* __restrict__ row, int d, int D, bool vec_ok)
 {
-    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (d < D) {
-        if (vec_ok) {
-            v = *reinterpret_cast<const float4*>(row + d);
-        } else {
-            v.x = row[d];
-            if (d + 1 < D) v.y = row[d + 1];
-            if (d + 2 < D) v.z = row[d + 2];
-            if (d + 3 < D) v.w = row[d + 3];
-        }
-    }
-    return v;
+    return d < D ? load_dims(row + d, D - d, vec_ok) : make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
 // Exact distances of the first n candidates of `list` to the point, then offer them.  CH = dimensions

@@ -1178,14 +1178,7 @@ __global__ __launch_bounds__(256) void k_chain(const float* __restrict__ points,
                     pre[i] = make_float4(0.f, 0.f, 0.f, 0.f);
                     if (row < n && d < P.D) {
                         const float* src = points + (size_t)ids[row] * (size_t)P.D + d;
-                        if (vec_ok) {
-                            pre[i] = *reinterpret_cast<const float4*>(src);
-                        } else {
-                            pre[i].x = src[0];
-                            if (d + 1 < P.D) pre[i].y = src[1];
-                            if (d + 2 < P.D) pre[i].z = src[2];
-                            if (d + 3 < P.D) pre[i].w = src[3];
-                        }
+                        pre[i] = load_dims(src, P.D - d, vec_ok);
                     }
                 }
             };

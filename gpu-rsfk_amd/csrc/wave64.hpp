@@ -92,6 +92,23 @@ __device__ __forceinline__ float wave_max(float v)
     return fmaxf(fmaxf(r0, r1), fmaxf(r2, r3));
 }
 
+// Four consecutive dimensions of a row, of which `left` are there (at least one), zeros beyond them.  aligned16: the address is a
+// multiple of 16 bytes and all four are there.  Otherwise a row may begin at any multiple of four bytes (rows of 37 dimensions): the vector memory
+// path loads 16 bytes from there too, which the type states.
+typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ float4 load_dims(const float* __restrict__ src, int left, bool aligned16)
+{
+    if (aligned16) return *reinterpret_cast<const float4*>(src);
+    if (left >= 4) {
+        const f32x4_a4 v = *reinterpret_cast<const f32x4_a4*>(src);
+        return make_float4(v.x, v.y, v.z, v.w);
+    }
+    float4 v = make_float4(src[0], 0.f, 0.f, 0.f);
+    if (left > 1) v.y = src[1];
+    if (left > 2) v.z = src[2];
+    return v;
+}
+
 // Orders LDS accesses of one wavefront as seen by its own lanes.  The hardware
 // executes a wavefront's LDS operations in order; this only keeps the compiler
 // from moving LDS accesses across the point.

@@ -831,6 +831,38 @@ def test_ann_screened_buckets_match_oracle(gpu, capi, orc, rng, monkeypatch, N, 
     assert_knn_equal(idx.cpu().numpy(), dist.cpu().numpy(), oi, od)
 
 
+@pytest.mark.parametrize("D", [1, 2, 3, 4, 5, 7, 36, 37, 39, 130])
+@pytest.mark.parametrize("shift", [0, 1, 2, 3])
+def test_rows_that_begin_at_any_float(gpu, capi, orc, rng, monkeypatch, D, shift):
+    """Rows of any length at any multiple of four bytes, the last one at the end of its allocation: forest with exploration (both
+    forms of the bucket step) and query-set search == the oracle."""
+    import torch
+    N, NQ, K, T, mn, mx = 1500, 400, 12, 5, 13, 80
+    X, Q = rng.standard_normal((N, D)).astype(np.float32), rng.standard_normal((NQ, D)).astype(np.float32)
+    oi, od = orc.forest(X, K, T, mn, mx, 5000, 3, 1)
+    ai, ad = orc.ann_forest(X, Q, K, T, mn, mx, 5000, 3)
+    put = lambda A: torch.cat([torch.full((shift,), 1e9), torch.from_numpy(A).flatten()]).cuda()[shift:]
+    dX, dQ = put(X), put(Q)
+    assert dX.data_ptr() % 16 == 4 * shift
+    _say("rows at any float", D, shift)
+    for form in ("0", "1"):
+        monkeypatch.setenv("RSFK_FOREST_MERGE", form)
+        monkeypatch.setenv("RSFK_ANN_FOREST", form)
+        monkeypatch.setenv("RSFK_ANN_SCREEN", "always")
+        idx = torch.full((N, K), -1, dtype=torch.int32, device="cuda")
+        dist = torch.full((N, K), float("inf"), dtype=torch.float32, device="cuda")
+        idx[:, 0] = torch.arange(N, dtype=torch.int32, device="cuda")
+        dist[:, 0] = 0.0
+        torch.cuda.synchronize()
+        capi.knn_forest_device(T, K, N, D, mn, mx, 5000, 0, 3, 1, dX.data_ptr(), idx.data_ptr(), dist.data_ptr())
+        assert_knn_equal(idx.cpu().numpy(), dist.cpu().numpy(), oi, od)
+        idx = torch.full((NQ, K), -1, dtype=torch.int32, device="cuda")
+        dist = torch.full((NQ, K), float("inf"), dtype=torch.float32, device="cuda")
+        torch.cuda.synchronize()
+        capi.knn_ann_device(T, K, N, NQ, D, mn, mx, 5000, 0, 3, dX.data_ptr(), dQ.data_ptr(), idx.data_ptr(), dist.data_ptr())
+        assert_knn_equal(idx.cpu().numpy(), dist.cpu().numpy(), ai, ad)
+
+
 def test_ann_device_entry_point_merges_into_given_rows(gpu, capi, orc, rng):
     """Device-resident call, twice with different seeds on the same rows == the oracle doing the same."""
     import torch
