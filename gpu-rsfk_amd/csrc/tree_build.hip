@@ -36,9 +36,9 @@
 #include "knn_list.hpp"
 #include "bf16.hpp"
 #include "tree_sweep.hpp"
+#include "level_notes.hpp"
 #include <vector>
 #include <algorithm>
-#include <atomic>
 #include <cstdlib>
 #include <cstring>
 #include <chrono>
@@ -66,14 +66,6 @@ struct LevelCounters {
     long long last_tick;
     long long phase_ticks[4];
 };
-
-// What a level tells the host, in pinned memory: its counts, and seq, written last.
-struct LevelNote {
-    int n_nodes, n_chunks, n_tail, overflow;
-    int seq;
-    int pad_[11];
-};
-constexpr int kNotes = 8;               // level l writes note l & 7
 
 // Counts for the report of a build (how many points the side tests of all levels looked at, and how many of them
 // the screen left to the exact test): kStatSlots slots a cache line apart, so that the workgroups' additions do not
@@ -1470,7 +1462,7 @@ struct TreeBatchWorkspace {
     TreeStats* stats = nullptr;
     LevelCounters* ctr = nullptr;
     int D = 0;
-    LevelNote* notes = nullptr;          // pinned, kNotes
+    LevelNotes notes;                    // pinned
     BatchReport* h_report = nullptr;     // pinned
     unsigned long long* stat = nullptr;  // kStatSlots x kStatPitch: counts for the report (stat_add)
     unsigned long long counts[2] = {0, 0};       // of the last batch: points the side tests looked at, undecided ones
@@ -1498,7 +1490,7 @@ static void free_ws(TreeBatchWorkspace& w)
                    w.chunk_left, w.leaf_start, w.leaf_size, w.stats, w.ctr, w.recs, w.n_rec, w.planes,
                    w.pm_path, w.pm_side, w.pm_undec, w.pm_map[0], w.pm_map[1], w.pm_sc, w.pm_aq, w.pm_child, w.stat};
     for (void* p : dev) ws_free(p);
-    pin_free(w.notes);
+    pin_free(w.notes.block());
     pin_free(w.h_report);
     w = TreeBatchWorkspace();
 }
@@ -1609,8 +1601,13 @@ int tree_ws_alloc(TreeBatchWorkspace** out, int N, int D, int MIN, int B)
         if (dmalloc(&w->pm_aq, (size_t)B * pm::kMaxGroups * 32 * 32 * w->pm_ks)) return 1;
         if (dmalloc(&w->pm_child, (size_t)w->node_cap)) return 1;
     }
-    if (pin_alloc(reinterpret_cast<void**>(&w->notes), sizeof(LevelNote) * kNotes)) return 1;
-    if (pin_alloc(reinterpret_cast<void**>(&w->h_report), sizeof(BatchReport))) return 1;
+    void* notes = nullptr;
+    if (pin_alloc(&notes, LevelNotes::kBytes)) return 1;
+    if (pin_alloc(reinterpret_cast<void**>(&w->h_report), sizeof(BatchReport))) {
+        pin_free(notes);
+        return 1;
+    }
+    w->notes.set(notes, &w->h_report->seq);
     return 0;
 }
 
@@ -1657,6 +1654,7 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
     Q.next = w->nodes[0]; Q.next_cap = w->node_cap; Q.chunk_cap = w->chunk_cap; Q.slot = 0;
     Q.tail = w->tail; Q.tail_cap = w->tail_cap;
     Q.ctr = w->ctr;
+    w->notes.begin();
     {
         const size_t total = (size_t)N * nb;
         const int grid = (int)std::min<size_t>((total + 255) / 256, 65536);
@@ -1664,8 +1662,6 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
                            pm_levels > 0 ? w->pm_map[0] : nullptr, w->stats, w->stat);
         RSFK_HIP(hipGetLastError());
     }
-    static std::atomic<int> batches{0};
-    const int seq0 = (batches.fetch_add(1) & 0x3ffff) * 8192 + 1;          // notes of an earlier batch never look like this one's
 
     int cur = 0;
     const size_t side_lds = (size_t)(4 + nvec_len(D)) * sizeof(float);
@@ -1692,8 +1688,8 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
     size_t most_nodes = (size_t)nb, most_chunks = (size_t)nb * (((size_t)N + P.chunk - 1) / P.chunk);
     while (N > P.small) {
         if (level > 0) {
-            LevelNote* note = w->notes + ((level - 1) & (kNotes - 1));
-            if (wait_for_word(&note->seq, seq0 + ((level - 1) & 8191), stream)) return 1;
+            const LevelNote* note = w->notes.of(level - 1);
+            if (wait_for_word(&note->seq, LevelNotes::seq(level - 1), stream)) return 1;
             RSFK_CHECK(!note->overflow && note->n_nodes <= w->node_cap && note->n_chunks <= w->chunk_cap,
                        "tree batch: node queue overflow");
             n_tail = note->n_tail;
@@ -1709,7 +1705,7 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
         int* ctr_chunks = &w->ctr->queue[slot].chunks;
         hipLaunchKernelGGL(k_level_planes, dim3((unsigned)((most_nodes + plane_waves - 1) / plane_waves)), dim3(64 * plane_waves),
                            plane_waves * side_lds, stream, points, P, w->perm[0], w->perm[1], w->nodes[cur], level, w->node_cap,
-                           w->planes, w->chunk2node, w->ctr, w->stat, w->notes + (level & (kNotes - 1)), seq0 + (level & 8191));
+                           w->planes, w->chunk2node, w->ctr, w->stat, w->notes.of(level), LevelNotes::seq(level));
         const bool swept = level < pm_levels;
         if (swept) {
             // the sides of every point in all trees of the batch, then their marks in the permutations
@@ -1812,9 +1808,9 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
 #undef RSFK_CHAIN_LAUNCH
         RSFK_HIP(hipGetLastError());
     }
-    hipLaunchKernelGGL(k_tree_report, dim3(1), dim3(64), 0, stream, w->stats, nb, w->ctr, w->stat, w->h_report, seq0);
+    hipLaunchKernelGGL(k_tree_report, dim3(1), dim3(64), 0, stream, w->stats, nb, w->ctr, w->stat, w->h_report, LevelNotes::kReport);
     RSFK_HIP(hipGetLastError());
-    if (wait_for_word(&w->h_report->seq, seq0, stream)) return 1;
+    if (wait_for_word(&w->h_report->seq, LevelNotes::kReport, stream)) return 1;
     const BatchReport& R = *w->h_report;
     w->counts[0] = R.counts[0];
     w->counts[1] = R.counts[1];

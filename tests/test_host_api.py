@@ -6,6 +6,7 @@ library here."""
 import inspect
 import os
 import re
+import subprocess
 
 import numpy as np
 import pytest
@@ -169,3 +170,49 @@ def test_sizes_the_library_would_refuse_raise_in_python(capi):
         r.find_nearest_neighbors_ann(X, np.zeros((4, 2), np.float32), 4)
     with pytest.raises(ValueError):
         r.cluster_by_sample_tree(np.zeros((0, 3), np.float32))
+
+
+NOTES_PROGRAM = r"""
+#include "level_notes.hpp"
+#include <cstring>
+#include <vector>
+using namespace rsfk;
+int main()
+{
+    struct { int other[31]; int seq; } report;
+    std::vector<unsigned char> block(LevelNotes::kBytes);
+    LevelNotes notes;
+    notes.set(block.data(), &report.seq);
+    // what a finished batch, or anything else that used the blocks, may have left: every level and the report "have arrived"
+    for (int first = 0; first < 8 * LevelNotes::kNotes; first += LevelNotes::kNotes) {
+        for (int l = first; l < first + LevelNotes::kNotes; ++l) {
+            std::memset(notes.of(l), 0x55, sizeof(LevelNote));
+            notes.of(l)->seq = LevelNotes::seq(l);
+        }
+        report.seq = LevelNotes::kReport;
+        if (notes.of(first)->seq != LevelNotes::seq(first)) return 1;            // (the plant is one the host would take)
+        notes.begin();
+        for (int l = 0; l < 8 * LevelNotes::kNotes; ++l)
+            if (notes.of(l)->seq == LevelNotes::seq(l)) return 2;
+        if (report.seq == LevelNotes::kReport) return 3;
+    }
+    // a batch of many levels: a note arrives when its level writes it and not before, whatever the level that had its place
+    notes.begin();
+    for (int l = 0; l < 20000; ++l) {
+        if (notes.of(l)->seq == LevelNotes::seq(l)) return 4;
+        notes.of(l)->seq = LevelNotes::seq(l);
+        if (notes.of(l)->seq != LevelNotes::seq(l) || notes.of(l + 1) == notes.of(l)) return 5;
+    }
+    return 0;
+}
+"""
+
+
+def test_notes_of_a_level_cannot_be_old_memory(tmp_path):
+    """The records a batch of trees answers in come from a pool of pinned blocks that keep their contents: after begin()
+    none of them looks written, whatever the blocks held."""
+    src, exe = tmp_path / "notes.cpp", tmp_path / "notes"
+    src.write_text(NOTES_PROGRAM)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-I", os.path.join(ROOT, "gpu-rsfk_amd", "csrc"), str(src), "-o", str(exe)],
+                   check=True)
+    assert subprocess.run([str(exe)]).returncode == 0
