@@ -49,6 +49,15 @@ struct Q8Copy {
     float* rho_sum = nullptr;     // device scalar: sum over the rows of e1 / (2^-8 mean |x_d|)
 };
 
+// The rule of every screened side test: margin = |approximate n.x - offset|, band = what the approximation and the exact fp32
+// evaluation can differ by when no sum overflows.  Every band has 1e-30 in it, above anything that underflow does to either
+// evaluation, and is at least 16 x 2^-24 of sum |n_d||x_d| (the rounding errors of the sums): below 1e32 no partial sum of
+// the exact evaluation can leave the range of fp32.  Where the approximation or the offset did, the margin is infinite or NaN.
+__device__ __forceinline__ bool side_certain(float margin, float band)
+{
+    return margin > band && band < 1e32f && margin < INFINITY;
+}
+
 int q8_copy_alloc(Q8Copy* c, int N, int D);
 void q8_copy_free(Q8Copy* c);
 int q8_copy_fill(const Q8Copy& c, const float* points, int N, int D, hipStream_t stream);

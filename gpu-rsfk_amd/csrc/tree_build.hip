@@ -210,7 +210,7 @@ __device__ __forceinline__ void side_screen8(const float* nvec0, int nstride, co
             if (LPP >= 8) d += dpp_f<kDppHalfMirror>(d);
             const float lo = __uint_as_float(head[u].y), scale = __uint_as_float(head[u].z), e1 = __uint_as_float(head[u].w);
             const float approx = __builtin_fmaf(scale, d, lo * hp2[u]);
-            const bool certain = fabsf(approx - b[u]) > e1 * hp1[u];       // false if anything is NaN
+            const bool certain = side_certain(fabsf(approx - b[u]), __builtin_fmaf(e1, hp1[u], 1e-30f));
             right[u] = approx < b[u];
             redo[u] = valid[u] && !certain;
         }
@@ -260,7 +260,7 @@ __device__ __forceinline__ void side_screen8(const float* nvec0, int nstride, co
             float d = da[u], a = sa[u];
             d += dpp_f<kDppXor1>(d); d += dpp_f<kDppXor2>(d); d += dpp_f<kDppHalfMirror>(d);
             a += dpp_f<kDppXor1>(a); a += dpp_f<kDppXor2>(a); a += dpp_f<kDppHalfMirror>(a);
-            const bool certain = fabsf(d - b[u]) > a * band + 1e-30f;
+            const bool certain = side_certain(fabsf(d - b[u]), a * band + 1e-30f);
             right[u] = d < b[u];
             redo[u] = valid[u] && !certain;
         }
@@ -1265,7 +1265,7 @@ __global__ __launch_bounds__(256) void k_chain(const float* __restrict__ points,
             for (int v = 0; v < kV; ++v) {
                 const bool valid = lane + 64 * v < count;
                 const float tol = nn * (nq[v] + half12) + tol_d * (d1[v] + d2[v]) + 1e-30f;
-                const bool certain = fabsf(d2[v] - d1[v]) > tol;              // false if anything is NaN
+                const bool certain = side_certain(fabsf(d2[v] - d1[v]), tol);
                 left[v] = ballot64(valid && certain && !(d2[v] < d1[v]));
                 again[v] = ballot64(valid && !certain);
                 n_def += __popcll(again[v]);

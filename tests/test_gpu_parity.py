@@ -84,6 +84,29 @@ def test_tree_nodes_split_in_vain(gpu, orc, rng, monkeypatch, N, D, MIN, MAX, ki
         assert list(gst) == [len(ls), st[0], st[1], st[2]]
 
 
+# Rows whose dot products overflow (all of them near the limit; a tenth of the rows far above the others), overflow in one
+# factor only, or are denormal: every kernel of the side tests (wide levels point by point and node by node, tail, chains).
+@pytest.mark.parametrize("kind", ["near_overflow", "mixed", "spread", "denormal"])
+@pytest.mark.parametrize("env", [dict(SCREEN="q8", PM="7"), dict(SCREEN="q8", PM="0"), dict(SCREEN="q8", PM="0", TAIL="256"), dict(SCREEN="bf16"),
+                                 dict(SCREEN="bf16", TAIL="256")], ids=lambda e: "-".join(e.values()))
+def test_tree_of_rows_whose_sums_leave_fp32(gpu, orc, rng, monkeypatch, kind, env):
+    for name, var in (("SCREEN", "RSFK_TREE_SCREEN"), ("PM", "RSFK_PM_LEVELS"), ("TAIL", "RSFK_TAIL_BLOCK")):
+        if name in env:
+            monkeypatch.setenv(var, env[name])
+    N, D, MIN, MAX, depth = 6000, 48, 17, 34, 60
+    X = rng.standard_normal((N, D))
+    scale = {"near_overflow": 3e18, "denormal": 3e-22, "mixed": np.where(rng.random((N, 1)) < 0.1, 3e18, 1.0),
+             "spread": 10.0 ** rng.uniform(-25, 37, (N, 1))}[kind]
+    X = (X * scale).astype(np.float32)
+    for seed in (1, 2):
+        _say("tree beyond fp32", kind, env, seed)
+        perm, ls, lz, st = orc.build_tree(X, MIN, MAX, depth, seed)
+        gperm, gls, glz, gst = gpu.build_tree(X, MIN, MAX, depth, seed)
+        assert np.array_equal(gperm, perm)
+        assert np.array_equal(gls, ls) and np.array_equal(glz, lz)
+        assert list(gst) == [len(ls), st[0], st[1], st[2]]
+
+
 def test_tree_edge_cases(gpu, orc, rng):
     # identical points: re-drawn until the depth limit, then one forced bucket
     X = np.ones((3000, 4), np.float32)
@@ -817,7 +840,6 @@ def test_ann_screened_buckets_match_oracle(gpu, capi, orc, rng, monkeypatch, N, 
     monkeypatch.setenv("RSFK_ANN_FOREST", "0")
     monkeypatch.setenv("RSFK_ANN_SCREEN", "always")
     monkeypatch.setenv("RSFK_ANN_ROUTE_LOW", "1")
-    monkeypatch.setenv("RSFK_TREE_SCREEN", "bf16")     # (where sums overflow the 8-bit side tests may part from the oracle's)
     idx = torch.full((NQ, K), -1, dtype=torch.int32, device="cuda")
     dist = torch.full((NQ, K), float("inf"), dtype=torch.float32, device="cuda")
     _say("ann screened", N, NQ, D, K, T, mn, mx, data)
