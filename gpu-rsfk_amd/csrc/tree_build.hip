@@ -94,7 +94,10 @@ __host__ __device__ inline int nvec_len(int D) { return (D + 15) & ~15; }
 // Hyperplane of (x1,x2) by one wavefront (all 64 lanes call): normal into LDS nvec[0..nvec_len(D)), and
 // hp[0] = offset (order of create_node.cu:122-135: 32 lane-strided partial sums + xor butterfly),
 // hp[1] = an upper bound of the 1-norm of the normal, hp[2] = the sum of its components (any order: only the
-// 8-bit screen uses them, with a margin).
+// screens use them, with a margin).  A pair with the same coordinates has the normal 0 and every point on its left (0 < 0):
+// its hp[1] is kZeroNormal, which makes the bounds of the screens negative, so that no point is left to the exact test
+// (100,000 x 32, a tenth of the points in groups of 2,000 equal rows, 10 trees: 947 -> 224 ms).
+constexpr float kZeroNormal = -1e30f;
 __device__ __forceinline__ void make_hyperplane_wave(const float* __restrict__ x1, const float* __restrict__ x2,
                                                      int D, float* nvec, float* hp)
 {
@@ -134,7 +137,7 @@ __device__ __forceinline__ void make_hyperplane_wave(const float* __restrict__ x
     s = half_butterfly_sum(s);
     s2 = half_butterfly_sum(s2);
     if (lane == 0) hp[0] = s;
-    if (lane == 32) { hp[1] = s * 1.001f; hp[2] = s2; }
+    if (lane == 32) { hp[1] = s == 0.0f ? kZeroNormal : s * 1.001f; hp[2] = s2; }
 }
 
 // Screen of the side test for eight points per wavefront (right = n.x < b): lanes 8g..8g+7 work on
@@ -221,7 +224,6 @@ __device__ __forceinline__ void side_screen8(const float* nvec0, int nstride, co
     const int sub = lane & 7;
 #pragma unroll
     for (int u = 0; u < NB; ++u) { right[u] = false; redo[u] = valid[u]; }
-    (void)hp1;
     (void)hp2;
     if (pb16 != nullptr) {
         const int Dv = bf16_valid(D);
@@ -260,7 +262,7 @@ __device__ __forceinline__ void side_screen8(const float* nvec0, int nstride, co
             float d = da[u], a = sa[u];
             d += dpp_f<kDppXor1>(d); d += dpp_f<kDppXor2>(d); d += dpp_f<kDppHalfMirror>(d);
             a += dpp_f<kDppXor1>(a); a += dpp_f<kDppXor2>(a); a += dpp_f<kDppHalfMirror>(a);
-            const bool certain = side_certain(fabsf(d - b[u]), a * band + 1e-30f);
+            const bool certain = side_certain(fabsf(d - b[u]), a * band + (1e-30f + fminf(hp1[u], 0.0f)));
             right[u] = d < b[u];
             redo[u] = valid[u] && !certain;
         }
@@ -1034,6 +1036,12 @@ __global__ __launch_bounds__(TB) void k_tail(const float* __restrict__ points,
 // the roundings of n, x1 + x2 and their product; Cauchy-Schwarz), ||n|| = sqrt(d(x1, x2)).  So the sign of d2 - d1 decides
 // when |d2 - d1| > 2.1 (D/32 + 8) u ||n|| (..) + 1.1 (D + 4) u (d1 + d2); otherwise (hardly ever, also for NaN) the point
 // gets the exact test.  ||x|| is bounded by sqrt(D) max |x_d| from the header of the 8-bit row.
+//
+// Where x1 and x2 have the same coordinates the normal is zero and the exact test puts every point on the left (0 < 0, or a
+// comparison with NaN).  Every point is as near to one as to the other, so that d1 and d2 decide nothing, and more than MAX
+// equal rows are split until the depth limit; so such pairs are marked in the matrix, with a distance of -0 (no sum of
+// squares is), and cost a link no test at all.  (20,000 x 32, buckets of 17..34, a tenth of the points in groups of 60
+// equal rows, 10 trees: 137 ms with an exact test of every point, 34 without; the tail kernel, with its own, took 62.)
 __device__ __forceinline__ int tri_at(int i, int j, int n)
 {
     const int lo = min(i, j), hi = max(i, j);
@@ -1123,6 +1131,7 @@ __global__ __launch_bounds__(256) void k_chain(const float* __restrict__ points,
     SmallNode* stack = reinterpret_cast<SmallNode*>(hp + 4);
     int2* lrec = reinterpret_cast<int2*>(stack + node_cap);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    __shared__ int zero_s;                                                    // two points of the node are at distance 0
     const int n_tasks = min(ctr->n_chain, task_cap);
     const bool vec_ok = (P.D & 3) == 0 && ((reinterpret_cast<uintptr_t>(points) & 15) == 0);
     const float u24 = 1.0f / 16777216.0f;
@@ -1134,6 +1143,7 @@ __global__ __launch_bounds__(256) void k_chain(const float* __restrict__ points,
         const int n = tk.count;
         int* seg = perm_out + (size_t)tk.tree * (size_t)P.N + tk.start;
         __syncthreads();                                                      // the previous task is done with the LDS
+        if (tid == 0) zero_s = 0;
         if (tid < n) {
             const int id = seg[tid];
             ids[tid] = id;
@@ -1212,6 +1222,7 @@ __global__ __launch_bounds__(256) void k_chain(const float* __restrict__ points,
                 for (int r = 0; r <= c; ++r) {
                     const int i = ty + 16 * r, j = tx + 16 * c;
                     if (c < nb && i <= j && j < n) {
+                        if (i < j && acc[c * (c + 1) / 2 + r] == 0.0f) zero_s = 1;
                         if constexpr (NB == 8) {
                             tri[i * (n | 1) + j] = acc[c * (c + 1) / 2 + r];
                             tri[j * (n | 1) + i] = acc[c * (c + 1) / 2 + r];
@@ -1222,6 +1233,33 @@ __global__ __launch_bounds__(256) void k_chain(const float* __restrict__ points,
                 }
         }
         __syncthreads();
+        if (zero_s) {
+            // tmp[j]: the first point at distance 0 from j, if it has the coordinates of j (eight lanes compare), else j
+            auto at = [&](int i, int j) { return NB == 8 ? i * (n | 1) + j : tri_at(i, j, n); };
+            for (int j = tid >> 3; j < n; j += 32) {
+                int first = j;
+                for (int i = (tid & 7); i < j && first == j; i += 8)
+                    if (tri[at(i, j)] == 0.0f) first = i;
+#pragma unroll
+                for (int o = 1; o < 8; o <<= 1) first = min(first, __shfl_xor(first, o, 64));
+                const float* xi = points + (size_t)ids[first] * (size_t)P.D;
+                const float* xj = points + (size_t)ids[j] * (size_t)P.D;
+                int differ = 0;
+                for (int d = tid & 7; d < P.D && !differ; d += 8) differ = xi[d] == xj[d] ? 0 : 1;
+#pragma unroll
+                for (int o = 1; o < 8; o <<= 1) differ |= __shfl_xor(differ, o, 64);
+                if ((tid & 7) == 0) tmp[j] = differ ? j : first;
+            }
+            __syncthreads();
+            for (int e = tid; e < n * n; e += 256) {
+                const int i = e / n, j = e - i * n;
+                if (i < j && tmp[i] == tmp[j]) {
+                    tri[at(i, j)] = -0.0f;
+                    if constexpr (NB == 8) tri[at(j, i)] = -0.0f;
+                }
+            }
+            __syncthreads();
+        }
         if (wave != 0) continue;                                              // the chain is the first wavefront's
         TreeRec* recs = recs_all ? recs_all + (size_t)tk.tree * rec_cap : nullptr;
         int* n_rec = recs_all ? n_rec_all + tk.tree : nullptr;
@@ -1251,7 +1289,9 @@ __global__ __launch_bounds__(256) void k_chain(const float* __restrict__ points,
             int r1, r2;
             draws.pair(dcount, r1, r2);
             const int o1 = place_at(dstart - start + r1), o2 = place_at(dstart - start + r2);
-            const float nn = tol_n * __builtin_sqrtf(dist_to(o1, o2)), half12 = 0.5f * (norm[o1] + norm[o2]);
+            const float d12 = dist_to(o1, o2);
+            const bool same = __float_as_int(d12) == (int)0x80000000;         // (x1 and x2 have the same coordinates)
+            const float nn = tol_n * __builtin_sqrtf(d12), half12 = 0.5f * (norm[o1] + norm[o2]);
             float d1[kV], d2[kV], nq[kV];
 #pragma unroll
             for (int v = 0; v < kV; ++v) {
@@ -1265,8 +1305,8 @@ __global__ __launch_bounds__(256) void k_chain(const float* __restrict__ points,
             for (int v = 0; v < kV; ++v) {
                 const bool valid = lane + 64 * v < count;
                 const float tol = nn * (nq[v] + half12) + tol_d * (d1[v] + d2[v]) + 1e-30f;
-                const bool certain = side_certain(fabsf(d2[v] - d1[v]), tol);
-                left[v] = ballot64(valid && certain && !(d2[v] < d1[v]));
+                const bool certain = same || side_certain(fabsf(d2[v] - d1[v]), tol);
+                left[v] = ballot64(valid && certain && (same || !(d2[v] < d1[v])));
                 again[v] = ballot64(valid && !certain);
                 n_def += __popcll(again[v]);
             }

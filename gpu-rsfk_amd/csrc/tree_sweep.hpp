@@ -42,7 +42,7 @@ constexpr int kMaxGroups = kPaths / kSlots;
 
 // One hyperplane as the sweep needs it.
 struct PlaneQ {
-    float b, hp1, hp2, s2;      // offset, bound of ||n||_1, sum of the components, scale of the second 8-bit part
+    float b, hp1, hp2, s2;      // offset, bound of ||n||_1 (or kZeroNormal), sum of the components, scale of the second 8-bit part
     float c0, rres, pad;        // 128 s2 (254 sum m1 + sum m2), bound of sum |r_d| (and of what 254 s2 != s1 does)
     int ni;                     // node of the level's queue, or -1: the points with this path are not split any more
 };

@@ -84,6 +84,36 @@ def test_tree_nodes_split_in_vain(gpu, orc, rng, monkeypatch, N, D, MIN, MAX, ki
         assert list(gst) == [len(ls), st[0], st[1], st[2]]
 
 
+# More equal rows than a bucket holds, in nodes that are split until the depth limit: square and triangular distance matrix, all
+# points in such groups or a few of them, zeros of either sign (equal coordinates of different bits), rows whose distances
+# underflow to zero without being equal, equal rows that hold an infinity.
+@pytest.mark.parametrize("N,D,MIN,MAX,kind", [(3000, 6, 20, 40, "groups"), (4000, 33, 17, 34, "some"), (3000, 12, 54, 108, "groups"),
+                                              (3000, 7, 33, 66, "zeros"), (2500, 5, 20, 40, "underflow"), (2500, 64, 17, 34, "infinite"),
+                                              (2500, 3, 60, 120, "some")])
+@pytest.mark.parametrize("screen", ["q8", "bf16"])
+def test_tree_nodes_of_equal_rows(gpu, orc, rng, monkeypatch, N, D, MIN, MAX, kind, screen):
+    monkeypatch.setenv("RSFK_TREE_SCREEN", screen)
+    g = MAX + MAX // 3
+    X = rng.standard_normal((N, D)).astype(np.float32)
+    m = N if kind == "groups" else N // 4
+    X[:m] = np.repeat(X[:m // g + 1], g, axis=0)[:m]
+    if kind == "zeros":
+        X[:m] = np.where(rng.random((m, D)) < 0.5, np.float32(0.0), np.float32(-0.0))
+    if kind == "underflow":
+        X[:m] += (rng.standard_normal((m, D)) * 1e-25).astype(np.float32)
+        X[: m // 2] = (rng.standard_normal((m // 2, D)) * 1e-25).astype(np.float32)
+    if kind == "infinite":
+        X[:m, 3] = np.inf
+    X = X[rng.permutation(N)]
+    for seed in (1, 2):
+        _say("tree of equal rows", N, D, MIN, MAX, kind, seed)
+        perm, ls, lz, st = orc.build_tree(X, MIN, MAX, 300, seed)
+        gperm, gls, glz, gst = gpu.build_tree(X, MIN, MAX, 300, seed)
+        assert np.array_equal(gperm, perm)
+        assert np.array_equal(gls, ls) and np.array_equal(glz, lz)
+        assert list(gst) == [len(ls), st[0], st[1], st[2]]
+
+
 # Rows whose dot products overflow (all of them near the limit; a tenth of the rows far above the others), overflow in one
 # factor only, or are denormal: every kernel of the side tests (wide levels point by point and node by node, tail, chains).
 @pytest.mark.parametrize("kind", ["near_overflow", "mixed", "spread", "denormal"])
