@@ -818,7 +818,11 @@ int explore_ws_alloc(ExploreWorkspace** out, int N, int K, bool with_bounds, boo
     while ((1 << l) < K) ++l;
     w->div_s = 31 + l;
     w->div_m = (uint32_t)((((uint64_t)1 << w->div_s) + (uint64_t)K - 1) / (uint64_t)K);
-    auto dm = [](void* p, size_t n) { return ws_alloc(reinterpret_cast<void**>(p), std::max<size_t>(n, 1) * sizeof(int)) ? hipErrorOutOfMemory : hipSuccess; };
+    auto dm = [graph_only](void* p, size_t n) {
+        const size_t bytes = std::max<size_t>(n, 1) * sizeof(int);
+        void** out = reinterpret_cast<void**>(p);
+        return (graph_only ? ws_try_alloc(out, bytes) : ws_alloc(out, bytes)) ? hipErrorOutOfMemory : hipSuccess;
+    };
     // Large graphs (2^26 entries and more; RSFK_REV_STAGED=1|0 says otherwise) take the builder that stages its stores
     // in LDS: fine bins whose rows fit into LDS with room to spare, about as many fine bins per coarse bin as there
     // are coarse bins.
@@ -851,7 +855,7 @@ int explore_ws_alloc(ExploreWorkspace** out, int N, int K, bool with_bounds, boo
          dm(&w->fine_start, (size_t)w->n_fine + 1) != hipSuccess ||
          dm(&w->sub_off, (size_t)w->n_sub << (w->cshift - w->fshift)) != hipSuccess)) {
         explore_ws_free(w);
-        set_last_error("exploration workspace: out of device memory");
+        if (!graph_only) set_last_error("exploration workspace: out of device memory");
         return 1;
     }
     if (dm(&w->rev, total) != hipSuccess || dm(&w->bin_eq, 2 * total) != hipSuccess ||
@@ -860,7 +864,7 @@ int explore_ws_alloc(ExploreWorkspace** out, int N, int K, bool with_bounds, boo
         dm(&w->part_off, (size_t)w->n_parts * (size_t)w->n_bins) != hipSuccess || (!graph_only && (dm(&w->pass, total * w->MW) != hipSuccess || dm(&w->norm_tau, 2 * (size_t)N) != hipSuccess)) ||
         dm(&w->todo, 2 * ((size_t)N + 1)) != hipSuccess) {
         explore_ws_free(w);
-        set_last_error("exploration workspace: out of device memory");
+        if (!graph_only) set_last_error("exploration workspace: out of device memory");
         return 1;
     }
     if (with_bounds) {

@@ -12,7 +12,7 @@
 // 3.71 -> 1.70 ms, 100,000 x 100: 1.46 -> 0.63).  Rows of more than 256 entries go to a workgroup each, which sorts them in LDS.
 //
 // The form below (symmetrize_flags) is for callers that cannot allocate, for graphs with a row of more than 4096
-// candidates and for inputs the builder of the reversed graph does not take: (1) a wavefront per point looks its own number up in the rows of its neighbours (coalesced row reads, four
+// candidates, for inputs the builder of the reversed graph does not take and where there is no room for it: (1) a wavefront per point looks its own number up in the rows of its neighbours (coalesced row reads, four
 // neighbours in flight) and counts, per point, the stored neighbours and the missing reverse edges; (2) prefix sum of
 // the row lengths; (3) the edges are written to their rows: the stored ones at compacted positions, the added ones
 // behind them in arrival order; (4) a segmented sort by column (rocPRIM) makes the rows independent of that order.
@@ -405,31 +405,49 @@ struct RevGuard {
     ~RevGuard() { explore_ws_free(w); }
 };
 
-int symmetrize_flags(const int* d_idx, const float* d_dist, int N, int K, int drop_self, int* d_indptr, int* d_cols,
-                     float* d_vals, long long cap, long long* nnz, hipStream_t stream);
+// Where the rows go: arrays of the caller with room for `cap` entries (both null: only the row offsets and the count are wanted),
+// or (make) arrays of the size of the graph, made here once that is known.
+struct GraphOut {
+    int* cols = nullptr;
+    float* vals = nullptr;
+    long long cap = 0;
+    bool make = false;
+    Buf c, v;
+    // nnz is known: 0, or nonzero with the reason when the arrays cannot take it
+    int room(long long nnz)
+    {
+        RSFK_CHECK(nnz <= cap, "graph export: the output arrays are too small for the graph");
+        if (!make) return 0;
+        if (ws_alloc(&c.p, sizeof(int) * (size_t)nnz) || ws_alloc(&v.p, sizeof(float) * (size_t)nnz)) return 1;
+        cols = static_cast<int*>(c.p);
+        vals = static_cast<float*>(v.p);
+        return 0;
+    }
+    bool wanted() const { return make || cols != nullptr; }
+};
 
-}  // namespace
+int symmetrize_flags(const int* d_idx, const float* d_dist, int N, int K, int drop_self, int* d_indptr, GraphOut& out,
+                     long long* nnz, hipStream_t stream);
 
-// d_idx / d_dist: N x K (d_dist may be null: the values are then zero).  d_indptr: N + 1 ints.  d_cols / d_vals: room for
-// `cap` entries, or both null to obtain only d_indptr and *nnz.  Entries that are negative or >= N are no edges;
-// drop_self removes p from its own row.  A row must not hold a point twice.
-int symmetrize_device(const int* d_idx, const float* d_dist, int N, int K, int drop_self, int* d_indptr, int* d_cols,
-                      float* d_vals, long long cap, long long* nnz, hipStream_t stream)
+int symmetrize(const int* d_idx, const float* d_dist, int N, int K, int drop_self, int* d_indptr, GraphOut& out, long long* nnz,
+               hipStream_t stream)
 {
     RSFK_CHECK(N >= 1 && K >= 1 && K <= kMaxK, "graph export: N must be positive and K in 1..1024");
     RSFK_CHECK((long long)N * K < (1ll << 30), "graph export: N * K of 2^30 and more is not supported");
     RSFK_CHECK(d_idx && d_indptr && nnz, "graph export: null argument");
-    RSFK_CHECK((d_cols == nullptr) == (d_vals == nullptr), "graph export: indices and data go together");
     // Up to about 2,800 points the library's sort takes few launches and the other form fewer in all (2,000 x 32: 0.057 against
     // 0.059 ms, 2,000 x 128: 0.102 against 0.141; 2,500 x 8: 0.049 against 0.048); from there on it takes more (3,000 x 8: 0.076
     // against 0.050, 3,000 x 90: 0.118 against 0.101).  RSFK_GRAPH_FLAGS=1 / 0 says which form (the results are the same).
     const char* form = std::getenv("RSFK_GRAPH_FLAGS");
     if (!explore_ws_takes(N, K) || (form && *form ? form[0] == '1' : N < 2800))
-        return symmetrize_flags(d_idx, d_dist, N, K, drop_self, d_indptr, d_cols, d_vals, cap, nnz, stream);
+        return symmetrize_flags(d_idx, d_dist, N, K, drop_self, d_indptr, out, nnz, stream);
     RevGuard rg;
     Buf len, big, ctr;
-    if (explore_ws_alloc(&rg.w, N, K, false, true) || ws_alloc(&len.p, sizeof(int) * ((size_t)N + 1)) ||
-        ws_alloc(&big.p, sizeof(int) * (size_t)N) || ws_alloc(&ctr.p, sizeof(UnionCounters)))
+    // the reversed graph takes 12 bytes per entry (20 from 2^26 entries on), the other form one
+    if (explore_ws_alloc(&rg.w, N, K, false, true))
+        return symmetrize_flags(d_idx, d_dist, N, K, drop_self, d_indptr, out, nnz, stream);
+    if (ws_alloc(&len.p, sizeof(int) * ((size_t)N + 1)) || ws_alloc(&big.p, sizeof(int) * (size_t)N) ||
+        ws_alloc(&ctr.p, sizeof(UnionCounters)))
         return 1;
     UnionCounters* counters = static_cast<UnionCounters*>(ctr.p);
     hipLaunchKernelGGL(k_union_zero, dim3(1), dim3(1), 0, stream, counters);
@@ -452,29 +470,30 @@ int symmetrize_device(const int* d_idx, const float* d_dist, int N, int K, int d
     if (ws_alloc(&tmp.p, tmp_bytes ? tmp_bytes : 256)) return 1;
     RSFK_HIP(rocprim::exclusive_scan(tmp.p, tmp_bytes, static_cast<int*>(len.p), d_indptr, 0, (size_t)N + 1,
                                      rocprim::plus<int>(), stream));
-    if (d_cols) {
+    const auto fill = [&]() -> int {
         const size_t lds = (size_t)4 * (own_ints + 2 * (kUnionWave + 4)) * sizeof(int);
         hipLaunchKernelGGL(k_union_fill, dim3((unsigned)((N + 3) / 4)), dim3(256), lds, stream, d_idx, d_dist, N, K, drop_self, offs, rev,
-                           div_m, div_s, own_ints, d_indptr, counters, cap, d_cols, d_vals);
+                           div_m, div_s, own_ints, d_indptr, counters, out.cap, out.cols, out.vals);
         hipLaunchKernelGGL(k_union_fill_big, dim3(256), dim3(256), 0, stream, d_idx, d_dist, N, K, drop_self, offs, rev, div_m, div_s,
-                           d_indptr, static_cast<int*>(big.p), counters, cap, d_cols, d_vals);
+                           d_indptr, static_cast<int*>(big.p), counters, out.cap, out.cols, out.vals);
         RSFK_HIP(hipGetLastError());
-    }
-    // one trip to the host, after everything has been queued
+        return 0;
+    };
+    // one trip to the host, for arrays of the caller after everything has been queued
+    if (out.cols && fill()) return 1;
     int word[3] = {0, 0, 0};                                     // entries, rows of a workgroup, most candidates of a row
     if (fetch_words(d_indptr + N, 1, reinterpret_cast<const int*>(counters), 2, word, stream)) return 1;
     *nnz = word[0];
-    if (!d_cols || *nnz == 0) return 0;
-    RSFK_CHECK(*nnz <= cap, "graph export: the output arrays are too small for the graph");
-    if (word[2] > kUnionBlock)
-        return symmetrize_flags(d_idx, d_dist, N, K, drop_self, d_indptr, d_cols, d_vals, cap, nnz, stream);
+    if (!out.wanted() || *nnz == 0) return 0;
+    if (word[2] > kUnionBlock) return symmetrize_flags(d_idx, d_dist, N, K, drop_self, d_indptr, out, nnz, stream);
+    if (out.room(*nnz)) return 1;
+    if (out.make && fill()) return 1;
+    if (out.make) RSFK_HIP(hipStreamSynchronize(stream));        // (the working memory goes back to the pool)
     return 0;
 }
 
-namespace {
-
-int symmetrize_flags(const int* d_idx, const float* d_dist, int N, int K, int drop_self, int* d_indptr, int* d_cols,
-                     float* d_vals, long long cap, long long* nnz, hipStream_t stream)
+int symmetrize_flags(const int* d_idx, const float* d_dist, int N, int K, int drop_self, int* d_indptr, GraphOut& out,
+                     long long* nnz, hipStream_t stream)
 {
     Buf flag, own, extra, len;
     if (ws_alloc(&flag.p, (size_t)N * K) || ws_alloc(&own.p, sizeof(int) * (size_t)N) ||
@@ -498,8 +517,10 @@ int symmetrize_flags(const int* d_idx, const float* d_dist, int N, int K, int dr
         if (fetch_words(d_indptr + N, 1, &total, stream)) return 1;
         *nnz = total;
     }
-    if (!d_cols || *nnz == 0) return 0;
-    RSFK_CHECK(*nnz <= cap, "graph export: the output arrays are too small for the graph");
+    if (!out.wanted() || *nnz == 0) return 0;
+    if (out.room(*nnz)) return 1;
+    int* d_cols = out.cols;
+    float* d_vals = out.vals;
     const size_t n = (size_t)*nnz;
     Buf cols, vals;
     if (ws_alloc(&cols.p, sizeof(int) * n) || ws_alloc(&vals.p, sizeof(float) * n)) return 1;
@@ -522,6 +543,20 @@ int symmetrize_flags(const int* d_idx, const float* d_dist, int N, int K, int dr
 }
 
 }  // namespace
+
+// d_idx / d_dist: N x K (d_dist may be null: the values are then zero).  d_indptr: N + 1 ints.  d_cols / d_vals: room for
+// `cap` entries, or both null to obtain only d_indptr and *nnz.  Entries that are negative or >= N are no edges;
+// drop_self removes p from its own row.  A row must not hold a point twice.
+int symmetrize_device(const int* d_idx, const float* d_dist, int N, int K, int drop_self, int* d_indptr, int* d_cols,
+                      float* d_vals, long long cap, long long* nnz, hipStream_t stream)
+{
+    RSFK_CHECK((d_cols == nullptr) == (d_vals == nullptr), "graph export: indices and data go together");
+    GraphOut out;
+    out.cols = d_cols;
+    out.vals = d_vals;
+    out.cap = cap;
+    return symmetrize(d_idx, d_dist, N, K, drop_self, d_indptr, out, nnz, stream);
+}
 
 // ---------------------------------------------------------------------------------------------------------------------
 // The count-only call (row lengths, d_indptr and the number of entries) for callers that cannot allocate device memory:
@@ -615,22 +650,21 @@ int symmetrize_host(const int* idx, const float* dist, int N, int K, int drop_se
     RSFK_CHECK(idx && indptr && nnz, "graph export: null argument");
     RSFK_CHECK((cols == nullptr) == (vals == nullptr), "graph export: indices and data go together");
     HostStage stage;
-    Buf di, dd, dp, dc, dv;
+    Buf di, dd, dp;
     const size_t nk = (size_t)N * K;
     if (ws_alloc(&di.p, nk * sizeof(int)) || ws_alloc(&dp.p, ((size_t)N + 1) * sizeof(int))) return 1;
     if (dist && ws_alloc(&dd.p, nk * sizeof(float))) return 1;
-    if (cols && cap > 0) {
-        if (ws_alloc(&dc.p, (size_t)cap * sizeof(int)) || ws_alloc(&dv.p, (size_t)cap * sizeof(float))) return 1;
-    }
+    GraphOut rows;
+    rows.make = cols != nullptr && cap > 0;
+    rows.cap = cap;
     const HostArray in[] = {{di.p, const_cast<int*>(idx), nk * sizeof(int)}, {dd.p, const_cast<float*>(dist), nk * sizeof(float)}};
     if (stage.to_device(in, dist ? 2 : 1, nullptr)) return 1;
-    const int rc = symmetrize_device(static_cast<const int*>(di.p), static_cast<const float*>(dd.p), N, K, drop_self,
-                                     static_cast<int*>(dp.p), static_cast<int*>(dc.p), static_cast<float*>(dv.p), cap, nnz,
-                                     nullptr);
+    const int rc = symmetrize(static_cast<const int*>(di.p), static_cast<const float*>(dd.p), N, K, drop_self,
+                              static_cast<int*>(dp.p), rows, nnz, nullptr);
     if (rc) return rc;
-    const HostArray out[] = {{dp.p, indptr, ((size_t)N + 1) * sizeof(int)}, {dc.p, cols, (size_t)*nnz * sizeof(int)},
-                             {dv.p, vals, (size_t)*nnz * sizeof(float)}};
-    return copy_to_host(out, dc.p ? 3 : 1, nullptr);
+    const HostArray out[] = {{dp.p, indptr, ((size_t)N + 1) * sizeof(int)}, {rows.cols, cols, (size_t)*nnz * sizeof(int)},
+                             {rows.vals, vals, (size_t)*nnz * sizeof(float)}};
+    return copy_to_host(out, rows.cols ? 3 : 1, nullptr);
 }
 
 }  // namespace rsfk

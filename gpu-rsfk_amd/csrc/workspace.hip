@@ -93,6 +93,7 @@ int ws_alloc_impl(void** out, size_t bytes, bool must)
     if (e != hipSuccess) {
         (void)hipGetLastError();
         set_last_error(std::string("out of device memory (") + std::to_string(bytes) + " bytes): " + hipGetErrorString(e));
+        (void)hipDeviceSynchronize();       // (the caller's guards hand their blocks back on the way out)
         return 1;
     }
     std::lock_guard<std::mutex> lock(P.mu);
@@ -105,8 +106,14 @@ int ws_alloc_impl(void** out, size_t bytes, bool must)
 int ws_alloc(void** out, size_t bytes) { return ws_alloc_impl(out, bytes, true); }
 
 // A block the caller can do without (it only makes something faster): nonzero, with nothing else changed, when the
-// device does not have the room.
-int ws_try_alloc(void** out, size_t bytes) { return ws_alloc_impl(out, bytes, false); }
+// device does not have the room, or when it has RSFK_OPTIONAL_MB megabytes or more (read at every call: tests change it).
+int ws_try_alloc(void** out, size_t bytes)
+{
+    *out = nullptr;
+    const char* most = std::getenv("RSFK_OPTIONAL_MB");
+    if (most && *most && (long long)(bytes >> 20) >= std::atoll(most)) return 1;
+    return ws_alloc_impl(out, bytes, false);
+}
 
 // The caller has made sure that no work that uses the block is still running.
 void ws_free(void* p)

@@ -1006,6 +1006,29 @@ def test_symmetric_graph_with_hubs_matches_oracle(gpu, orc, rng, monkeypatch, N,
     assert np.array_equal(gp, op) and np.array_equal(gc, oc) and np.array_equal(gv, ov)
 
 
+def test_without_the_optional_working_memory(gpu, orc, rng, monkeypatch):
+    """Nothing but speed depends on the blocks a call can do without: with none of them (RSFK_OPTIONAL_MB=0) the export, the
+    build and the query-set search take their other forms and give the same results."""
+    import gpu_rsfk
+    monkeypatch.setenv("RSFK_OPTIONAL_MB", "0")
+    N, D, K, T = 4000, 19, 70, 4
+    X, Q = rng.standard_normal((N, D)).astype(np.float32), rng.standard_normal((50, D)).astype(np.float32)
+    r = gpu_rsfk.RSFK(random_state=3)
+    _say("no optional memory: build")
+    gi, gd = r.find_nearest_neighbors(X, K, n_trees=T, nn_exploring_factor=1)
+    oi, od = orc.forest(X, K, T, K + 1, 2 * (K + 1), 5000, 3, 1)
+    assert_knn_equal(gi, gd, oi, od)
+    assert ["k_forest_pairs + k_forest_merge"] not in [k[2] for k in gpu.last_build_report()["bucket_kernels"]]
+    _say("no optional memory: queries")
+    qi, qd = r.find_nearest_neighbors_ann(X, Q, K, n_trees=T)
+    oi, od = orc.ann_forest(X, Q, K, T, K + 1, 2 * (K + 1), 5000, 3)
+    assert_knn_equal(qi, qd, oi, od)
+    _say("no optional memory: graph")
+    gp, gc, gv = gpu_rsfk.symmetric_knn_graph(gi, gd)
+    op, oc, ov = orc.symmetrize(gi, gd, drop_self=True)
+    assert np.array_equal(gp, op) and np.array_equal(gc, oc) and np.array_equal(gv, ov)
+
+
 def test_symmetric_graph_of_a_built_graph(gpu, capi, orc, rng):
     """On a graph the library built (one distance value per pair) the export equals the oracle's bit for bit; device
     entry point with the two-call protocol (count, then fill)."""
