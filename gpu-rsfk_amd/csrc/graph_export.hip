@@ -9,19 +9,22 @@
 // R(p) = the entries that hold p), (2) a wavefront per point drops from R(p) the points that p stores itself and counts
 // what row p will hold, (3) prefix sum of the row lengths, (4) a wavefront per point gathers the union in LDS, ranks every
 // column by counting the smaller ones and writes it to its place: no atomics on memory, no sort of the result (1M x 32:
-// 3.71 -> 1.70 ms, 100,000 x 100: 1.46 -> 0.63).  Rows of more than 256 entries go to a workgroup each, which sorts them in LDS.
+// 3.71 -> 1.70 ms, 100,000 x 100: 1.46 -> 0.63).  Rows of more than 256 entries go to a workgroup each, which sorts them in LDS;
+// those of points that more than some 4,000 others store (hubs) are gathered together and sorted by (row, column) in memory.
 //
-// The form below (symmetrize_flags) is for callers that cannot allocate, for graphs with a row of more than 4096
-// candidates, for inputs the builder of the reversed graph does not take and where there is no room for it: (1) a wavefront per point looks its own number up in the rows of its neighbours (coalesced row reads, four
+// The form below (symmetrize_flags) is for callers that cannot allocate, for small graphs, for inputs the builder of the
+// reversed graph does not take and where there is no room for it: (1) a wavefront per point looks its own number up in the rows of its neighbours (coalesced row reads, four
 // neighbours in flight) and counts, per point, the stored neighbours and the missing reverse edges; (2) prefix sum of
 // the row lengths; (3) the edges are written to their rows: the stored ones at compacted positions, the added ones
 // behind them in arrival order; (4) a segmented sort by column (rocPRIM) makes the rows independent of that order.
 #include "forest.hpp"
 #include "wave64.hpp"
 #include "knn_list.hpp"
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
+#include <rocprim/device/device_radix_sort.hpp>
 #include <rocprim/device/device_scan.hpp>
 #include <rocprim/device/device_segmented_radix_sort.hpp>
 
@@ -169,10 +172,23 @@ struct Buf {
 constexpr int kUnionWave = 256;            // entries of a row a wavefront ranks (four per lane)
 constexpr int kUnionBlock = 4096;          // candidates of a row a workgroup sorts in LDS
 
+// Rows by the number of their entries and candidates (stored neighbours and reversed entries): a wavefront each up to
+// kUnionWave entries, a workgroup each up to kUnionBlock candidates (`big`), the others (`hubs`) all together.
 struct UnionCounters {
-    int n_big;                             // rows of more than kUnionWave entries
-    int largest;                           // most candidates (stored neighbours and reversed entries) of a row
+    int n_big;
+    int pad;
+    struct alignas(8) Hubs {
+        unsigned entries;                  // of all hubs
+        unsigned n;
+    } hubs;
 };
+struct UnionLists {
+    int* big;                              // points
+    int2* hubs;                            // {point, entries of the hubs before it}
+    UnionCounters* ctr;
+};
+// (a hub has more than kUnionBlock candidates, and all rows together 2 N K)
+size_t most_hubs(size_t entries) { return 2 * entries / (size_t)kUnionBlock + 1; }
 
 // The stored neighbours of p that are edges, in LDS and in order; returns their number.  (own: K ints of the wavefront.)
 __device__ __forceinline__ int own_edges(const int* __restrict__ idx, int N, int K, int p, int drop_self, int* own)
@@ -206,7 +222,7 @@ __device__ __forceinline__ uint64_t in_own(const int* own, int n, int c)
 // len[p] = entries of row p; len[N] = 0.
 __global__ __launch_bounds__(256) void k_union_len(const int* __restrict__ idx, int N, int K, int drop_self, const int* __restrict__ offs,
                                                    const int* __restrict__ rev, uint32_t div_m, int div_s, int own_ints,
-                                                   int* __restrict__ len, int* __restrict__ big, UnionCounters* __restrict__ ctr)
+                                                   int* __restrict__ len, UnionLists L)
 {
     extern __shared__ __align__(16) int union_lds[];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -221,17 +237,29 @@ __global__ __launch_bounds__(256) void k_union_len(const int* __restrict__ idx, 
     const int n = own_edges(idx, N, K, p, drop_self, own);
     wave_lds_sync();
     int total = n;
-    for (int r = r0; r < r1; r += 64) {
-        const int e = r == r0 ? e0 : (r + lane < r1 ? rev[r + lane] : -1);
+    auto count = [&](int e) {
         const int c = (int)(((uint64_t)(uint32_t)e * div_m) >> div_s);
         const bool ok = e >= 0 && !(drop_self && c == p);
         total += __popcll(ballot64(ok) & ~in_own(own, n, c));
+    };
+    if (r0 < r1) count(e0);
+    // (eight loads at a time: R(p) of a hub is long)
+    for (int r = r0 + 64; r < r1; r += 512) {
+        int e[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) e[u] = r + 64 * u + lane < r1 ? rev[r + 64 * u + lane] : -1;
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (r + 64 * u < r1) count(e[u]);
     }
     if (lane == 0) {
         len[p] = total;
-        if (total > kUnionWave) big[atomicAdd(&ctr->n_big, 1)] = p;
-        const int cand = n + r1 - r0;
-        if (cand > 256 && cand > *const_cast<volatile int*>(&ctr->largest)) atomicMax(&ctr->largest, cand);
+        if (n + (r1 - r0) > kUnionBlock) {
+            const unsigned long long was = atomicAdd(reinterpret_cast<unsigned long long*>(&L.ctr->hubs), (unsigned)total | (1ull << 32));
+            L.hubs[was >> 32] = make_int2(p, (int)(unsigned)was);
+        } else if (total > kUnionWave) {
+            L.big[atomicAdd(&L.ctr->n_big, 1)] = p;
+        }
     }
 }
 
@@ -274,11 +302,10 @@ __device__ __forceinline__ void rank_and_store(const int* key, const int* entry,
 __global__ __launch_bounds__(256) void k_union_fill(const int* __restrict__ idx, const float* __restrict__ dist, int N, int K,
                                                     int drop_self, const int* __restrict__ offs, const int* __restrict__ rev,
                                                     uint32_t div_m, int div_s, int own_ints, const int* __restrict__ indptr,
-                                                    const UnionCounters* __restrict__ ctr, long long cap, int* __restrict__ cols,
-                                                    float* __restrict__ vals)
+                                                    long long cap, int* __restrict__ cols, float* __restrict__ vals)
 {
     extern __shared__ __align__(16) int union_lds[];
-    if (ctr->largest > kUnionBlock || indptr[N] > cap) return;          // (the host takes the other form, or reports)
+    if (indptr[N] > cap) return;                                        // (the host reports)
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int p = (int)blockIdx.x * 4 + wave;
     if (p >= N) return;
@@ -330,17 +357,17 @@ __global__ __launch_bounds__(256) void k_union_fill(const int* __restrict__ idx,
 __global__ __launch_bounds__(256) void k_union_fill_big(const int* __restrict__ idx, const float* __restrict__ dist, int N, int K,
                                                         int drop_self, const int* __restrict__ offs, const int* __restrict__ rev,
                                                         uint32_t div_m, int div_s, const int* __restrict__ indptr,
-                                                        const int* __restrict__ big, const UnionCounters* __restrict__ ctr,
-                                                        long long cap, int* __restrict__ cols, float* __restrict__ vals)
+                                                        UnionLists L, long long cap, int* __restrict__ cols,
+                                                        float* __restrict__ vals)
 {
     __shared__ unsigned long long a[kUnionBlock];
     __shared__ int n_s, wave_n[4];
-    if (ctr->largest > kUnionBlock || indptr[N] > cap) return;
+    if (indptr[N] > cap) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int n_big = ctr->n_big;
+    const int n_big = L.ctr->n_big;
     constexpr unsigned long long kNone = ~0ull;
     for (int b = blockIdx.x; b < n_big; b += gridDim.x) {
-        const int p = big[b];
+        const int p = L.big[b];
         __syncthreads();
         if (tid == 0) n_s = 0;
         __syncthreads();
@@ -396,8 +423,70 @@ __global__ __launch_bounds__(256) void k_union_fill_big(const int* __restrict__ 
 
 __global__ void k_union_zero(UnionCounters* ctr)
 {
-    ctr->n_big = 0;
-    ctr->largest = 0;
+    *ctr = UnionCounters();
+}
+
+// Hubs (a row of blockIdx.x each, blockIdx.y: a share of R(p)): the entries of their rows in any order, key = number of the hub
+// << col_bits | column, of equal columns the stored neighbour.  cursor (zero on entry) counts them.  A row of any length is too
+// long for the LDS of one workgroup, but the hubs' rows together are a small part of the graph, so that sorting them costs
+// little beside the rest: 1M x 32 with one hub of 10,000 entries 1.76 ms (3.87 with all rows in the other form), with 20 hubs
+// of 300,000 each 14.5 (72), 100,000 x 16 with one hub of 6,000 0.198 (0.416).
+__global__ __launch_bounds__(256) void k_hub_gather(const int* __restrict__ idx, const float* __restrict__ dist, int N, int K,
+                                                    int drop_self, const int* __restrict__ offs, const int* __restrict__ rev,
+                                                    uint32_t div_m, int div_s, int own_ints, const int2* __restrict__ hubs, int col_bits,
+                                                    int* __restrict__ cursor, unsigned long long* __restrict__ keys,
+                                                    float* __restrict__ vals)
+{
+    extern __shared__ __align__(16) int union_lds[];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int h = blockIdx.x, p = hubs[h].x, first = hubs[h].y;
+    int* own = union_lds + wave * own_ints;
+    const int n = own_edges(idx, N, K, p, drop_self, own);
+    wave_lds_sync();
+    const unsigned long long row = (unsigned long long)(unsigned)h << col_bits;
+    auto put = [&](bool keep, int c, int e) {
+        const uint64_t m = ballot64(keep);
+        if (m == 0) return;
+        int at = lane == 0 ? atomicAdd(&cursor[h], __popcll(m)) : 0;
+        at = first + __builtin_amdgcn_readfirstlane(at) + mask_prefix(m);
+        if (keep) {
+            keys[at] = row | (unsigned)c;
+            vals[at] = dist ? dist[e] : 0.0f;
+        }
+    };
+    if (blockIdx.y == 0 && wave == 0)
+        for (int k0 = 0; k0 < K; k0 += 64) {
+            const int k = k0 + lane, e = p * K + k;
+            const int c = k < K ? idx[e] : -1;
+            put(usable(c, p, N, drop_self), c, e);
+        }
+    const int r1 = offs[p + 1], step = (int)gridDim.y * 256;
+    for (int r = offs[p] + ((int)blockIdx.y * 4 + wave) * 64; r < r1; r += step) {
+        const int e = r + lane < r1 ? rev[r + lane] : -1;
+        const int c = (int)(((uint64_t)(uint32_t)e * div_m) >> div_s);
+        const bool ok = e >= 0 && !(drop_self && c == p);
+        put(lane_bit(ballot64(ok) & ~in_own(own, n, c)), c, e);
+    }
+}
+
+// The sorted entries of the hubs to their rows.
+__global__ __launch_bounds__(256) void k_hub_store(const unsigned long long* __restrict__ keys, const float* __restrict__ sorted, unsigned n,
+                                                   const int2* __restrict__ hubs, int col_bits, const int* __restrict__ indptr,
+                                                   int* __restrict__ cols, float* __restrict__ vals)
+{
+    const unsigned i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= n) return;
+    const unsigned long long key = keys[i];
+    const int2 hub = hubs[key >> col_bits];
+    const int at = indptr[hub.x] + (int)(i - (unsigned)hub.y);
+    cols[at] = (int)(key & ((1ull << col_bits) - 1ull));
+    vals[at] = sorted[i];
+}
+
+__global__ __launch_bounds__(256) void k_zero_counters(int* __restrict__ v, int n)
+{
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) v[i] = 0;
 }
 
 struct RevGuard {
@@ -442,15 +531,15 @@ int symmetrize(const int* d_idx, const float* d_dist, int N, int K, int drop_sel
     if (!explore_ws_takes(N, K) || (form && *form ? form[0] == '1' : N < 2800))
         return symmetrize_flags(d_idx, d_dist, N, K, drop_self, d_indptr, out, nnz, stream);
     RevGuard rg;
-    Buf len, big, ctr;
+    Buf len, big, hubs, ctr;
     // the reversed graph takes 12 bytes per entry (20 from 2^26 entries on), the other form one
     if (explore_ws_alloc(&rg.w, N, K, false, true))
         return symmetrize_flags(d_idx, d_dist, N, K, drop_self, d_indptr, out, nnz, stream);
     if (ws_alloc(&len.p, sizeof(int) * ((size_t)N + 1)) || ws_alloc(&big.p, sizeof(int) * (size_t)N) ||
-        ws_alloc(&ctr.p, sizeof(UnionCounters)))
+        ws_alloc(&hubs.p, sizeof(int2) * most_hubs((size_t)N * (size_t)K)) || ws_alloc(&ctr.p, sizeof(UnionCounters)))
         return 1;
-    UnionCounters* counters = static_cast<UnionCounters*>(ctr.p);
-    hipLaunchKernelGGL(k_union_zero, dim3(1), dim3(1), 0, stream, counters);
+    const UnionLists L = {static_cast<int*>(big.p), static_cast<int2*>(hubs.p), static_cast<UnionCounters*>(ctr.p)};
+    hipLaunchKernelGGL(k_union_zero, dim3(1), dim3(1), 0, stream, L.ctr);
     if (launch_reversed_graph(rg.w, d_idx, N, K, stream)) return 1;
     const int* offs = explore_ws_offs(rg.w);
     const int* rev = explore_ws_rev(rg.w);
@@ -461,7 +550,7 @@ int symmetrize(const int* d_idx, const float* d_dist, int N, int K, int drop_sel
     const uint32_t div_m = (uint32_t)((((uint64_t)1 << div_s) + (uint64_t)K - 1) / (uint64_t)K);
     const int own_ints = (K + 4 + 3) & ~3;
     hipLaunchKernelGGL(k_union_len, dim3((unsigned)(N / 4 + 1)), dim3(256), (size_t)4 * own_ints * sizeof(int), stream, d_idx, N, K,
-                       drop_self, offs, rev, div_m, div_s, own_ints, static_cast<int*>(len.p), static_cast<int*>(big.p), counters);
+                       drop_self, offs, rev, div_m, div_s, own_ints, static_cast<int*>(len.p), L);
     RSFK_HIP(hipGetLastError());
     size_t tmp_bytes = 0;
     RSFK_HIP(rocprim::exclusive_scan(nullptr, tmp_bytes, static_cast<int*>(len.p), d_indptr, 0, (size_t)N + 1,
@@ -473,21 +562,55 @@ int symmetrize(const int* d_idx, const float* d_dist, int N, int K, int drop_sel
     const auto fill = [&]() -> int {
         const size_t lds = (size_t)4 * (own_ints + 2 * (kUnionWave + 4)) * sizeof(int);
         hipLaunchKernelGGL(k_union_fill, dim3((unsigned)((N + 3) / 4)), dim3(256), lds, stream, d_idx, d_dist, N, K, drop_self, offs, rev,
-                           div_m, div_s, own_ints, d_indptr, counters, out.cap, out.cols, out.vals);
+                           div_m, div_s, own_ints, d_indptr, out.cap, out.cols, out.vals);
         hipLaunchKernelGGL(k_union_fill_big, dim3(256), dim3(256), 0, stream, d_idx, d_dist, N, K, drop_self, offs, rev, div_m, div_s,
-                           d_indptr, static_cast<int*>(big.p), counters, out.cap, out.cols, out.vals);
+                           d_indptr, L, out.cap, out.cols, out.vals);
         RSFK_HIP(hipGetLastError());
         return 0;
     };
     // one trip to the host, for arrays of the caller after everything has been queued
     if (out.cols && fill()) return 1;
-    int word[3] = {0, 0, 0};                                     // entries, rows of a workgroup, most candidates of a row
-    if (fetch_words(d_indptr + N, 1, reinterpret_cast<const int*>(counters), 2, word, stream)) return 1;
+    int word[3] = {0, 0, 0};                                     // entries, entries of the hubs, hubs
+    if (fetch_words(d_indptr + N, 1, reinterpret_cast<const int*>(&L.ctr->hubs), 2, word, stream)) return 1;
     *nnz = word[0];
     if (!out.wanted() || *nnz == 0) return 0;
-    if (word[2] > kUnionBlock) return symmetrize_flags(d_idx, d_dist, N, K, drop_self, d_indptr, out, nnz, stream);
+    const int n_hubs = word[2];
+    const size_t n_entries = (size_t)(unsigned)word[1];
+    Buf cursor, keys[2], sorted[2];
+    if (n_hubs > 0) {
+        // 24 bytes per entry of a hub; the other form does without them
+        if (ws_try_alloc(&cursor.p, sizeof(int) * (size_t)n_hubs)) cursor.p = nullptr;
+        bool have = cursor.p != nullptr;
+        for (int i = 0; i < 2 && have; ++i)
+            have = ws_try_alloc(&keys[i].p, sizeof(unsigned long long) * n_entries) == 0 && ws_try_alloc(&sorted[i].p, sizeof(float) * n_entries) == 0;
+        if (!have) return symmetrize_flags(d_idx, d_dist, N, K, drop_self, d_indptr, out, nnz, stream);
+    }
     if (out.room(*nnz)) return 1;
     if (out.make && fill()) return 1;
+    if (n_hubs > 0) {
+        int col_bits = 1, hub_bits = 1;
+        while ((1ll << col_bits) < (long long)N) ++col_bits;
+        while ((1ll << hub_bits) < (long long)n_hubs) ++hub_bits;
+        unsigned long long* key[2] = {static_cast<unsigned long long*>(keys[0].p), static_cast<unsigned long long*>(keys[1].p)};
+        float* val[2] = {static_cast<float*>(sorted[0].p), static_cast<float*>(sorted[1].p)};
+        hipLaunchKernelGGL(k_zero_counters, dim3((unsigned)((n_hubs + 255) / 256)), dim3(256), 0, stream, static_cast<int*>(cursor.p), n_hubs);
+        // about 2,000 workgroups over all hubs, each with 1,024 entries of R(p) or more
+        const size_t mean = n_entries / (size_t)n_hubs;
+        const unsigned shares = (unsigned)std::max<size_t>(1, std::min<size_t>(mean / 1024, (size_t)(2048 / std::min(n_hubs, 2048))));
+        hipLaunchKernelGGL(k_hub_gather, dim3((unsigned)n_hubs, shares), dim3(256), (size_t)4 * own_ints * sizeof(int), stream, d_idx, d_dist,
+                           N, K, drop_self, offs, rev, div_m, div_s, own_ints, L.hubs, col_bits, static_cast<int*>(cursor.p), key[0], val[0]);
+        RSFK_HIP(hipGetLastError());
+        size_t sort_bytes = 0;
+        RSFK_HIP(rocprim::radix_sort_pairs(nullptr, sort_bytes, key[0], key[1], val[0], val[1], n_entries, 0, (unsigned)(col_bits + hub_bits), stream));
+        Buf tmp_sort;
+        if (ws_alloc(&tmp_sort.p, sort_bytes ? sort_bytes : 256)) return 1;
+        RSFK_HIP(rocprim::radix_sort_pairs(tmp_sort.p, sort_bytes, key[0], key[1], val[0], val[1], n_entries, 0, (unsigned)(col_bits + hub_bits), stream));
+        hipLaunchKernelGGL(k_hub_store, dim3((unsigned)((n_entries + 255) / 256)), dim3(256), 0, stream, key[1], val[1], (unsigned)n_entries,
+                           L.hubs, col_bits, d_indptr, out.cols, out.vals);
+        RSFK_HIP(hipGetLastError());
+        RSFK_HIP(hipStreamSynchronize(stream));
+        return 0;
+    }
     if (out.make) RSFK_HIP(hipStreamSynchronize(stream));        // (the working memory goes back to the pool)
     return 0;
 }
@@ -602,12 +725,6 @@ int scratch_on_current_device(unsigned char** out)
     }
     *out = g_scratch_ptr[dev];
     return 0;
-}
-
-__global__ __launch_bounds__(256) void k_zero_counters(int* __restrict__ v, int n)
-{
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < n) v[i] = 0;
 }
 
 }  // namespace

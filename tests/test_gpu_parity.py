@@ -1006,6 +1006,35 @@ def test_symmetric_graph_with_hubs_matches_oracle(gpu, orc, rng, monkeypatch, N,
     assert np.array_equal(gp, op) and np.array_equal(gc, oc) and np.array_equal(gv, ov)
 
 
+@pytest.mark.parametrize("N,K,hubs,optional", [(4100, 2, 1, None), (4200, 1, 1, None), (20000, 9, 60, None), (30000, 4, 3, None), (30000, 4, 3, "0")])
+def test_rows_of_hubs_match_oracle(gpu, capi, orc, rng, monkeypatch, N, K, hubs, optional):
+    """Rows of more candidates than a workgroup sorts (just above 4,096, several hubs, several shares of R(p) per hub), into
+    arrays of the caller, with and without values, and the count alone; without room for the hubs' entries the other form."""
+    import torch
+    if optional is not None:
+        monkeypatch.setenv("RSFK_OPTIONAL_MB", optional)
+    idx = rng.integers(0, N, (N, K)).astype(np.int32)
+    idx[:, 0] = rng.permutation(hubs)[np.minimum(rng.geometric(0.3, N) - 1, hubs - 1)] if hubs > 1 else 0
+    for k in range(1, K):                                       # (a row must not hold a point twice)
+        idx[(idx[:, :k] == idx[:, k:k + 1]).any(1), k] = -1
+    idx[:hubs, 0] = -1
+    a, b = np.minimum(idx, np.arange(N)[:, None]).astype(np.int64), np.maximum(idx, np.arange(N)[:, None])
+    val = ((a * 7919 + b * 104729) % 10007).astype(np.float32)
+    _say("rows of hubs", N, K, hubs, optional)
+    op, oc, ov = orc.symmetrize(idx, val, drop_self=True)
+    assert np.diff(op).max() > 4090
+    di, dd = torch.from_numpy(idx).cuda(), torch.from_numpy(val).cuda()
+    for dist in (dd.data_ptr(), 0):
+        indptr = torch.zeros(N + 1, dtype=torch.int32, device="cuda")
+        assert capi.symmetrize_device(di.data_ptr(), dist, N, K, True, indptr.data_ptr(), 0, 0, 0) == len(oc)
+        cols = torch.full((len(oc),), -1, dtype=torch.int32, device="cuda")
+        vals = torch.full((len(oc),), -1.0, device="cuda")
+        assert capi.symmetrize_device(di.data_ptr(), dist, N, K, True, indptr.data_ptr(), cols.data_ptr(), vals.data_ptr(), len(oc)) == len(oc)
+        torch.cuda.synchronize()
+        assert np.array_equal(indptr.cpu().numpy(), op) and np.array_equal(cols.cpu().numpy(), oc)
+        assert np.array_equal(vals.cpu().numpy(), ov if dist else np.zeros_like(ov))
+
+
 def test_without_the_optional_working_memory(gpu, orc, rng, monkeypatch):
     """Nothing but speed depends on the blocks a call can do without: with none of them (RSFK_OPTIONAL_MB=0) the export, the
     build and the query-set search take their other forms and give the same results."""
