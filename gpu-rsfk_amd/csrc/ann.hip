@@ -758,14 +758,21 @@ size_t ann_forest_lds(int D, int K) { return sizeof(int) * ((size_t)((D + 31) & 
 //   100,000 x 100, up to 66, 50 trees: 10,000 queries (6.6e7) 2.90 -> 2.93 ms, 50,000 5.1 -> 14.2
 //   300,000 x 8, up to 18, 50 trees: 200,000 queries (2.9e7) 10.2 -> 4.7 ms;  5,000 x 129, K = 300, 9 trees: 600 queries (4.7e7)
 //   4.0 -> 1.1;  70,000 x 784, K = 90, 10 trees: 10,000 queries (1.4e9) 2.8 -> 10.1
-int ann_forest_group(int N, int NQ, int D, int K, int MAX, int rec_cap, int nb)
+// Repeated points make buckets far above MAX.  Up to kAnnSeen members the table of the ids a query has met spares it the same
+// rows in every tree (20,000 x 64 in groups of 200 equal rows, 50 trees, 1,000 queries 2.08 -> 0.10 ms).  Beyond that it gathers
+// them T times, and about NQ max_bucket / N queries do so, against one workgroup that takes the whole bucket for 16 of
+// them: 20,000 points, half of them equal, 6 trees, x 16: 8,000 queries 2.3 -> 1.4 ms, 16,000 2.9 -> 2.5;  x 64: 2,000 queries
+// 3.6 -> 2.9, 4,000 3.8 -> 5.9;  x 200: 1,000 queries 9.5 -> 6.3, 2,000 9.0 -> 15.4;  60,000 x 64, a tenth equal: 8,000 queries
+// 2.55 -> 2.56, 16,000 2.5 -> 4.0.  The two are alike at NQ max_bucket / N x D of 0.9e5 to 1.8e5.
+int ann_forest_group(int N, int NQ, int D, int K, int MAX, int max_bucket, int rec_cap, int nb)
 {
     const char* e = std::getenv("RSFK_ANN_FOREST");
     if (e && e[0] == '0') return 0;
     if (nb < 2 || ann_forest_lds(D, K) > (size_t)64 << 10) return 0;
     const bool forced = e && e[0] == '1';
-    constexpr double kMostFloats = 5e7;
+    constexpr double kMostFloats = 5e7, kMostHot = 1.2e5;
     if (!forced && (double)NQ * (double)MAX * (double)D > kMostFloats) return 0;
+    if (!forced && max_bucket > kAnnSeen && (double)NQ * (double)max_bucket * (double)D > kMostHot * (double)N) return 0;
     // hyperplanes and buckets reached: 1 GB at most
     const size_t per_tree = sizeof(float) * (size_t)rec_cap * (size_t)ann_plane_pitch(NQ, D) + sizeof(int2) * (size_t)NQ;
     const int group = (int)std::min<size_t>((size_t)std::min(nb, 64), ((size_t)1 << 30) / per_tree);

@@ -475,21 +475,28 @@ int knn_ann_forest_device(int n_trees, int K, int N, int NQ, int D, int MIN, int
         if (tree_ws_enable_index(ws.w, MIN, MAX_DEPTH)) return 1;
         const int rec_cap = tree_ws_rec_cap(ws.w);
         const size_t plane_bytes = sizeof(float) * (size_t)rec_cap * (size_t)ann_plane_pitch(NQ, D);
-        DevBuf aws, planes, reached, pair_stats;
-        // trees that are searched together (0, or no memory for it: one tree after the other)
-        int group = ann_forest_group(N, NQ, D, K, MAX, rec_cap, std::min(n_trees, B));
-        if (group > 0 && (ws_try_alloc(&planes.p, plane_bytes * (size_t)group) ||
-                          ws_try_alloc(&reached.p, sizeof(int) * 2 * (size_t)NQ * (size_t)group))) {
-            if (planes.p) ws_free(planes.p);
-            planes.p = nullptr;
-            group = 0;
-        }
-        if (group == 0) {
-            if (ws_alloc(&aws.p, sizeof(int) * ann_ws_ints(NQ, rec_cap))) return 1;
+        // working memory of the trees of a batch that are searched together, and of trees that are searched one after the other:
+        // taken when a batch asks for it for the first time (all batches but the last have the same number of trees)
+        DevBuf together_planes, reached, aws, planes, pair_stats;
+        int together = 0;                                   // trees there is room for
+        const auto room_together = [&](int group) -> bool {
+            if (group <= together) return true;
+            if (together > 0) return false;
+            if (ws_try_alloc(&together_planes.p, plane_bytes * (size_t)group)) return false;
+            if (ws_try_alloc(&reached.p, sizeof(int) * 2 * (size_t)NQ * (size_t)group)) {
+                ws_free(together_planes.p);
+                together_planes.p = nullptr;
+                return false;
+            }
+            together = group;
+            return true;
+        };
+        const auto room_alone = [&]() -> int {
+            if (pair_stats.p) return 0;
+            if (ws_alloc(&aws.p, sizeof(int) * ann_ws_ints(NQ, rec_cap)) || ws_alloc(&planes.p, plane_bytes)) return 1;
             if (ws_alloc(&pair_stats.p, sizeof(unsigned long long) * ann_stat_words(n_trees))) return 1;
-            if (launch_ann_ws_init(static_cast<int*>(aws.p), NQ, rec_cap, static_cast<unsigned long long*>(pair_stats.p), n_trees, stream)) return 1;
-            if (ws_alloc(&planes.p, plane_bytes)) return 1;
-        }
+            return launch_ann_ws_init(static_cast<int*>(aws.p), NQ, rec_cap, static_cast<unsigned long long*>(pair_stats.p), n_trees, stream);
+        };
         std::vector<int> stats((size_t)5 * B);
         std::vector<TimedEvent> ev((size_t)B + 1);          // ev[j]: the search in tree j of a batch begins, ev[nb]: the last ends
         for (auto& e : ev)
@@ -502,10 +509,16 @@ int knn_ann_forest_device(int n_trees, int K, int N, int NQ, int D, int MIN, int
                                   stream);
             if (rc) break;
             const double tt = now_s() - tt0;
+            // trees that are searched together (0, or no memory for it: one tree after the other)
+            int max_bucket = 0;
+            for (int j = 0; j < nb; ++j) max_bucket = std::max(max_bucket, stats[5 * j + 2]);
+            int group = ann_forest_group(N, NQ, D, K, MAX, max_bucket, rec_cap, nb);
+            if (group > 0 && !room_together(group)) group = 0;
+            if (group == 0 && room_alone()) return 1;
             if (group > 0) (void)hipEventRecord(ev[0].e, stream);
             for (int j = 0; j < nb && rc == 0 && group > 0; j += group)
                 rc = launch_ann_forest(d_points, d_queries, N, NQ, D, K, std::min(group, nb - j), tree_ws_perm(ws.w, j),
-                                       tree_ws_recs(ws.w, j), tree_ws_n_rec(ws.w, j), rec_cap, static_cast<float*>(planes.p),
+                                       tree_ws_recs(ws.w, j), tree_ws_n_rec(ws.w, j), rec_cap, static_cast<float*>(together_planes.p),
                                        static_cast<int*>(reached.p), d_qidx, d_qdist, stream);
             for (int j = 0; j < nb && rc == 0 && group == 0; ++j) {
                 (void)hipEventRecord(ev[j].e, stream);

@@ -183,7 +183,7 @@ int launch_ann_ws_init(int* ws, int NQ, int rec_cap, unsigned long long* stats, 
 int launch_ann_tree(const float* points, const float* queries, int N, int NQ, int D, int K, const int* perm, const TreeRec* recs,
                     const int* n_rec_dev, int rec_cap, int n_leaves, int* ws, float* planes, int* q_idx, float* q_dist,
                     const unsigned long long* prev, unsigned long long* stats, hipStream_t stream);
-int ann_forest_group(int N, int NQ, int D, int K, int MAX, int rec_cap, int nb);
+int ann_forest_group(int N, int NQ, int D, int K, int MAX, int max_bucket, int rec_cap, int nb);
 int launch_ann_forest(const float* points, const float* queries, int N, int NQ, int D, int K, int T, const int* perm, const TreeRec* recs,
                       const int* n_rec_dev, int rec_cap, float* planes, int* reached, int* q_idx, float* q_dist, hipStream_t stream);
 int knn_ann_forest_device(int n_trees, int K, int N, int NQ, int D, int MIN, int MAX, int MAX_DEPTH, int verbose, int seed,

@@ -852,6 +852,33 @@ def test_ann_trees_together_match_oracle(gpu, capi, orc, rng, monkeypatch, N, NQ
         assert_knn_equal(idx.cpu().numpy(), dist.cpu().numpy(), oi, od)
 
 
+@pytest.mark.parametrize("N,D,K,T", [(3000, 200, 8, 8), (4000, 37, 70, 6)])
+def test_ann_batches_take_the_form_their_buckets_ask_for(gpu, capi, orc, rng, monkeypatch, N, D, K, T):
+    """Half of the points are equal, so that every tree has one bucket far above the leaf limit; the number of queries is such
+    that batches with a larger one are searched tree by tree and the others together, in one call, into rows not in order."""
+    import torch
+    monkeypatch.setenv("RSFK_TREE_BATCH", "2")
+    X = rng.standard_normal((N, D)).astype(np.float32)
+    X[: N // 2] = X[0]
+    X = X[rng.permutation(N)]
+    widest = [orc.build_tree(X, K + 1, 2 * K + 2, 30, 5 + t)[2].max() for t in range(T)]
+    line = np.median([max(widest[t:t + 2]) for t in range(0, T, 2)])
+    NQ = int(1.2e5 * N / (D * line))
+    Q = rng.standard_normal((NQ, D)).astype(np.float32)
+    Q[: NQ // 3] = X[rng.integers(0, N, NQ // 3)]
+    assert min(widest) > 1024 and NQ * (2 * K + 2) * D < 5e7
+    idx = np.full((NQ, K), -1, np.int32)
+    dist = np.full((NQ, K), np.inf, np.float32)
+    orc.ann_forest(X, Q, K, 1, K + 1, 2 * K + 2, 30, 99, q_idx=idx, q_dist=dist)
+    idx, dist = np.ascontiguousarray(idx[:, ::-1]), np.ascontiguousarray(dist[:, ::-1])
+    di, dd, dX, dQ = (torch.from_numpy(a).cuda() for a in (idx, dist, X, Q))
+    orc.ann_forest(X, Q, K, T, K + 1, 2 * K + 2, 30, 5, q_idx=idx, q_dist=dist)
+    _say("ann batches", N, NQ, D, K, T, widest)
+    capi.knn_ann_device(T, K, N, NQ, D, K + 1, 2 * K + 2, 30, 0, 5, dX.data_ptr(), dQ.data_ptr(), di.data_ptr(), dd.data_ptr())
+    torch.cuda.synchronize()
+    assert_knn_equal(di.cpu().numpy(), dd.cpu().numpy(), idx, dist)
+
+
 # items of fewer and of more than 32 queries; buckets on both sides of 32 and 64 members; rows that end inside a step and inside
 # a 16-byte piece; distances that overflow, a common offset that leaves the bounds useless, equal distances
 @pytest.mark.parametrize("N,NQ,D,K,T,mn,mx", [(500, 900, 16, 64, 5, 65, 130), (3000, 2500, 100, 32, 6, 33, 66), (700, 333, 31, 5, 9, 6, 12),
