@@ -17,6 +17,7 @@
 #include <atomic>
 #include <cstring>
 #include <mutex>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -125,8 +126,13 @@ int large_copy(const std::vector<Piece>& pieces, bool to_device)
     std::atomic<size_t> next{0};
     const int n_threads = (int)std::min<size_t>(kCopyThreads, pieces.size());
     std::vector<std::thread> th;
-    for (int t = 1; t < n_threads; ++t)
-        th.emplace_back(run_lane, std::ref(L.lane[t]), L.stream[t % kCopyStreams], dev, std::cref(pieces), std::ref(next), to_device, std::ref(err));
+    th.reserve(kCopyThreads);
+    try {
+        for (int t = 1; t < n_threads; ++t)
+            th.emplace_back(run_lane, std::ref(L.lane[t]), L.stream[t % kCopyStreams], dev, std::cref(pieces), std::ref(next), to_device, std::ref(err));
+    } catch (const std::system_error&) {
+        // (a process at its limit of threads: those that are there take the pieces in turn)
+    }
     run_lane(L.lane[0], L.stream[0], dev, pieces, next, to_device, err);
     for (auto& t : th) t.join();
     RSFK_CHECK(err == 0, "copy between host and device failed");
