@@ -102,7 +102,7 @@ __global__ __launch_bounds__(256) void k_to_q8(const float* __restrict__ points,
         bool bad = false;
         for (int d = lane; d < D; d += 64) {
             const float x = src[d];
-            bad |= !(fabsf(x) <= 3.0e38f);                 // NaN or infinite
+            bad |= !(fabsf(x) <= kQ8Most);
             lo = fminf(lo, x);
             hi = fmaxf(hi, x);
             sabs += fabsf(x);
@@ -140,7 +140,7 @@ __global__ __launch_bounds__(256) void k_to_q8(const float* __restrict__ points,
         // compared with an fp32 evaluation of n.x: all of that stays below c_d (|lo| + 255 scale) per unit of ||n||_1
         const float mag = fabsf(lo) + 255.0f * scale;
         float e1 = 1.01f * err + c_d * mag + 1e-37f;
-        if (bad || !(range <= 3.0e38f)) e1 = __builtin_nanf("");      // the screen never decides for such a row
+        if (bad) e1 = __builtin_nanf("");      // the screen never decides for such a row
         if (lane == 0) {
             float* head = reinterpret_cast<float*>(dst);
             head[0] = 0.0f;
@@ -193,7 +193,7 @@ __global__ __launch_bounds__(256) void k_to_q8_regs(const float* __restrict__ po
                 const float v[4] = {x[k].x, x[k].y, x[k].z, x[k].w};
 #pragma unroll
                 for (int c = 0; c < 4; ++c) {
-                    bad |= !(fabsf(v[c]) <= 3.0e38f);              // NaN or infinite
+                    bad |= !(fabsf(v[c]) <= kQ8Most);
                     lo = fminf(lo, v[c]);
                     hi = fmaxf(hi, v[c]);
                     sabs += fabsf(v[c]);
@@ -235,7 +235,7 @@ __global__ __launch_bounds__(256) void k_to_q8_regs(const float* __restrict__ po
         for (int o = 1; o < LPR; o <<= 1) err = fmaxf(err, __shfl_xor(err, o, 64));
         const float mag = fabsf(lo) + 255.0f * scale;
         float e1 = 1.01f * err + c_d * mag + 1e-37f;
-        if (badi || !(range <= 3.0e38f)) e1 = __builtin_nanf("");      // the screen never decides for such a row
+        if (badi) e1 = __builtin_nanf("");      // the screen never decides for such a row
         if (row_ok && l == 0) {
             *reinterpret_cast<float4*>(dst) = make_float4(0.0f, lo, scale, e1);
             const float bf = sabs / (float)D * (1.0f / 256.0f);

@@ -94,7 +94,7 @@ __host__ __device__ inline int nvec_len(int D) { return (D + 15) & ~15; }
 // Hyperplane of (x1,x2) by one wavefront (all 64 lanes call): normal into LDS nvec[0..nvec_len(D)), and
 // hp[0] = offset (order of create_node.cu:122-135: 32 lane-strided partial sums + xor butterfly),
 // hp[1] = an upper bound of the 1-norm of the normal, hp[2] = the sum of its components (any order: only the
-// screens use them, with a margin).  A pair with the same coordinates has the normal 0 and every point on its left (0 < 0):
+// screens use them, with a margin).  NaN in place of the bound: the screens do not decide (bf16.hpp).  A pair with the same coordinates has the normal 0 and every point on its left (0 < 0):
 // its hp[1] is kZeroNormal, which makes the bounds of the screens negative, so that no point is left to the exact test
 // (100,000 x 32, a tenth of the points in groups of 2,000 equal rows, 10 trees: 947 -> 224 ms).
 constexpr float kZeroNormal = -1e30f;
@@ -137,7 +137,8 @@ __device__ __forceinline__ void make_hyperplane_wave(const float* __restrict__ x
     s = half_butterfly_sum(s);
     s2 = half_butterfly_sum(s2);
     if (lane == 0) hp[0] = s;
-    if (lane == 32) { hp[1] = s == 0.0f ? kZeroNormal : s * 1.001f; hp[2] = s2; }
+    const bool in_range = s <= kNormalMost && fabsf(read_lane_f(s, 0)) < 1e38f;
+    if (lane == 32) { hp[1] = s == 0.0f ? kZeroNormal : in_range ? s * 1.001f : __builtin_nanf(""); hp[2] = s2; }
 }
 
 // Screen of the side test for eight points per wavefront (right = n.x < b): lanes 8g..8g+7 work on
@@ -213,7 +214,7 @@ __device__ __forceinline__ void side_screen8(const float* nvec0, int nstride, co
             if (LPP >= 8) d += dpp_f<kDppHalfMirror>(d);
             const float lo = __uint_as_float(head[u].y), scale = __uint_as_float(head[u].z), e1 = __uint_as_float(head[u].w);
             const float approx = __builtin_fmaf(scale, d, lo * hp2[u]);
-            const bool certain = side_certain(fabsf(approx - b[u]), __builtin_fmaf(e1, hp1[u], 1e-30f));
+            const bool certain = fabsf(approx - b[u]) > __builtin_fmaf(e1, hp1[u], 1e-30f);       // false if anything is NaN
             right[u] = approx < b[u];
             redo[u] = valid[u] && !certain;
         }
@@ -262,7 +263,9 @@ __device__ __forceinline__ void side_screen8(const float* nvec0, int nstride, co
             float d = da[u], a = sa[u];
             d += dpp_f<kDppXor1>(d); d += dpp_f<kDppXor2>(d); d += dpp_f<kDppHalfMirror>(d);
             a += dpp_f<kDppXor1>(a); a += dpp_f<kDppXor2>(a); a += dpp_f<kDppHalfMirror>(a);
-            const bool certain = side_certain(fabsf(d - b[u]), a * band + (1e-30f + fminf(hp1[u], 0.0f)));
+            // (a below 1e37: no partial sum of the exact test overflows; an infinite margin: the offset did)
+            const float margin = fabsf(d - b[u]);
+            const bool certain = margin > a * band + (1e-30f + fminf(hp1[u], 0.0f)) && a < 1e37f && margin < INFINITY;
             right[u] = d < b[u];
             redo[u] = valid[u] && !certain;
         }
@@ -1035,7 +1038,8 @@ __global__ __launch_bounds__(TB) void k_tail(const float* __restrict__ points,
 // 1.01 (D/32 + 8) u ||n|| (||x|| + (||x1|| + ||x2||) / 2) together (chains of D/32 terms, five steps of the butterfly,
 // the roundings of n, x1 + x2 and their product; Cauchy-Schwarz), ||n|| = sqrt(d(x1, x2)).  So the sign of d2 - d1 decides
 // when |d2 - d1| > 2.1 (D/32 + 8) u ||n|| (..) + 1.1 (D + 4) u (d1 + d2); otherwise (hardly ever, also for NaN) the point
-// gets the exact test.  ||x|| is bounded by sqrt(D) max |x_d| from the header of the 8-bit row.
+// gets the exact test.  ||x|| is bounded by sqrt(D) max |x_d| from the header of the 8-bit row.  In a node with a norm of 1e18 or
+// more, or a distance of 1e37 or more, sums of the exact test may overflow, and all points get it.
 //
 // Where x1 and x2 have the same coordinates the normal is zero and the exact test puts every point on the left (0 < 0, or a
 // comparison with NaN).  Every point is as near to one as to the other, so that d1 and d2 decide nothing, and more than MAX
@@ -1131,7 +1135,7 @@ __global__ __launch_bounds__(256) void k_chain(const float* __restrict__ points,
     SmallNode* stack = reinterpret_cast<SmallNode*>(hp + 4);
     int2* lrec = reinterpret_cast<int2*>(stack + node_cap);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    __shared__ int zero_s;                                                    // two points of the node are at distance 0
+    __shared__ int zero_s, huge_s;                                            // two points are at distance 0; a norm or distance is out of range
     const int n_tasks = min(ctr->n_chain, task_cap);
     const bool vec_ok = (P.D & 3) == 0 && ((reinterpret_cast<uintptr_t>(points) & 15) == 0);
     const float u24 = 1.0f / 16777216.0f;
@@ -1143,7 +1147,7 @@ __global__ __launch_bounds__(256) void k_chain(const float* __restrict__ points,
         const int n = tk.count;
         int* seg = perm_out + (size_t)tk.tree * (size_t)P.N + tk.start;
         __syncthreads();                                                      // the previous task is done with the LDS
-        if (tid == 0) zero_s = 0;
+        if (tid == 0) { zero_s = 0; huge_s = 0; }
         if (tid < n) {
             const int id = seg[tid];
             ids[tid] = id;
@@ -1223,6 +1227,7 @@ __global__ __launch_bounds__(256) void k_chain(const float* __restrict__ points,
                     const int i = ty + 16 * r, j = tx + 16 * c;
                     if (c < nb && i <= j && j < n) {
                         if (i < j && acc[c * (c + 1) / 2 + r] == 0.0f) zero_s = 1;
+                        if (!(acc[c * (c + 1) / 2 + r] < 1e37f)) huge_s = 1;
                         if constexpr (NB == 8) {
                             tri[i * (n | 1) + j] = acc[c * (c + 1) / 2 + r];
                             tri[j * (n | 1) + i] = acc[c * (c + 1) / 2 + r];
@@ -1232,6 +1237,7 @@ __global__ __launch_bounds__(256) void k_chain(const float* __restrict__ points,
                     }
                 }
         }
+        if (tid < n && !(norm[tid] < 1e18f)) huge_s = 1;
         __syncthreads();
         if (zero_s) {
             // tmp[j]: the first point at distance 0 from j, if it has the coordinates of j (eight lanes compare), else j
@@ -1272,6 +1278,7 @@ __global__ __launch_bounds__(256) void k_chain(const float* __restrict__ points,
             if constexpr (NB == 8) return tri[o * (n | 1) + q];
             else return q == o ? 0.0f : tri[tri_at(q, o, n)];
         };
+        const float least_tol = huge_s ? INFINITY : 1e-30f;
         int q[kV];                                                            // places of the node's points, by position
         auto take_order = [&]() {
 #pragma unroll
@@ -1290,7 +1297,7 @@ __global__ __launch_bounds__(256) void k_chain(const float* __restrict__ points,
             draws.pair(dcount, r1, r2);
             const int o1 = place_at(dstart - start + r1), o2 = place_at(dstart - start + r2);
             const float d12 = dist_to(o1, o2);
-            const bool same = __float_as_int(d12) == (int)0x80000000;         // (x1 and x2 have the same coordinates)
+            const float least = __float_as_int(d12) == (int)0x80000000 ? -INFINITY : least_tol;      // (the same coordinates)
             const float nn = tol_n * __builtin_sqrtf(d12), half12 = 0.5f * (norm[o1] + norm[o2]);
             float d1[kV], d2[kV], nq[kV];
 #pragma unroll
@@ -1304,9 +1311,9 @@ __global__ __launch_bounds__(256) void k_chain(const float* __restrict__ points,
 #pragma unroll
             for (int v = 0; v < kV; ++v) {
                 const bool valid = lane + 64 * v < count;
-                const float tol = nn * (nq[v] + half12) + tol_d * (d1[v] + d2[v]) + 1e-30f;
-                const bool certain = same || side_certain(fabsf(d2[v] - d1[v]), tol);
-                left[v] = ballot64(valid && certain && (same || !(d2[v] < d1[v])));
+                const float tol = nn * (nq[v] + half12) + tol_d * (d1[v] + d2[v]) + least;
+                const bool certain = fabsf(d2[v] - d1[v]) > tol;              // false if anything is NaN
+                left[v] = ballot64(valid && certain && !(d2[v] < d1[v]));
                 again[v] = ballot64(valid && !certain);
                 n_def += __popcll(again[v]);
             }
