@@ -54,9 +54,10 @@ struct Q8Copy {
 // the exact evaluation could leave the range of fp32 (its comparison then has a side of its own) they must not decide.  With
 // the 8-bit copy that is settled per row and per hyperplane: a row with a coordinate beyond kQ8Most has e1 = NaN, a
 // hyperplane with a 1-norm above kNormalMost, or whose offset is not below 1e38, a bound of the 1-norm that is NaN, and what
-// is left has sums of at most 1e37.  The bfloat16 rows have no header; their sum |n_d||x_d| is tested at every point.  (The
-// test at every point for both: tail kernel and chains of 20,000 x 64, 50 trees 1.02 -> 1.06 ms.)
-constexpr float kQ8Most = 1e17f, kNormalMost = 1e20f;
+// is left has sums of at most 1e38 in the exact evaluation and 3e38 in the approximate one.  The bfloat16 rows have no header;
+// their sum |n_d||x_d| is tested at every point.  (The test at every point for both: tail kernel and chains of 20,000 x 64,
+// 50 trees 1.02 -> 1.06 ms.)
+constexpr float kQ8Most = 1e18f, kNormalMost = 1e20f;
 
 int q8_copy_alloc(Q8Copy* c, int N, int D);
 void q8_copy_free(Q8Copy* c);

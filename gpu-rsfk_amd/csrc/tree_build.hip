@@ -263,9 +263,9 @@ __device__ __forceinline__ void side_screen8(const float* nvec0, int nstride, co
             float d = da[u], a = sa[u];
             d += dpp_f<kDppXor1>(d); d += dpp_f<kDppXor2>(d); d += dpp_f<kDppHalfMirror>(d);
             a += dpp_f<kDppXor1>(a); a += dpp_f<kDppXor2>(a); a += dpp_f<kDppHalfMirror>(a);
-            // (a below 1e37: no partial sum of the exact test overflows; an infinite margin: the offset did)
+            // (a below 1e38: no partial sum of the exact test overflows; an infinite margin: the offset did)
             const float margin = fabsf(d - b[u]);
-            const bool certain = margin > a * band + (1e-30f + fminf(hp1[u], 0.0f)) && a < 1e37f && margin < INFINITY;
+            const bool certain = margin > a * band + (1e-30f + fminf(hp1[u], 0.0f)) && a < 1e38f && margin < INFINITY;
             right[u] = d < b[u];
             redo[u] = valid[u] && !certain;
         }
@@ -1038,8 +1038,9 @@ __global__ __launch_bounds__(TB) void k_tail(const float* __restrict__ points,
 // 1.01 (D/32 + 8) u ||n|| (||x|| + (||x1|| + ||x2||) / 2) together (chains of D/32 terms, five steps of the butterfly,
 // the roundings of n, x1 + x2 and their product; Cauchy-Schwarz), ||n|| = sqrt(d(x1, x2)).  So the sign of d2 - d1 decides
 // when |d2 - d1| > 2.1 (D/32 + 8) u ||n|| (..) + 1.1 (D + 4) u (d1 + d2); otherwise (hardly ever, also for NaN) the point
-// gets the exact test.  ||x|| is bounded by sqrt(D) max |x_d| from the header of the 8-bit row.  In a node with a norm of 1e18 or
-// more, or a distance of 1e37 or more, sums of the exact test may overflow, and all points get it.
+// gets the exact test.  ||x|| is bounded by sqrt(D) max |x_d| from the header of the 8-bit row.  In a node with a norm of 2e19 or
+// more, or a distance of 2e37 or more, sums of the exact test (of up to the norm times the root of the distance) may overflow,
+// and all points get it.
 //
 // Where x1 and x2 have the same coordinates the normal is zero and the exact test puts every point on the left (0 < 0, or a
 // comparison with NaN).  Every point is as near to one as to the other, so that d1 and d2 decide nothing, and more than MAX
@@ -1227,7 +1228,7 @@ __global__ __launch_bounds__(256) void k_chain(const float* __restrict__ points,
                     const int i = ty + 16 * r, j = tx + 16 * c;
                     if (c < nb && i <= j && j < n) {
                         if (i < j && acc[c * (c + 1) / 2 + r] == 0.0f) zero_s = 1;
-                        if (!(acc[c * (c + 1) / 2 + r] < 1e37f)) huge_s = 1;
+                        if (!(acc[c * (c + 1) / 2 + r] < 2e37f)) huge_s = 1;
                         if constexpr (NB == 8) {
                             tri[i * (n | 1) + j] = acc[c * (c + 1) / 2 + r];
                             tri[j * (n | 1) + i] = acc[c * (c + 1) / 2 + r];
@@ -1237,7 +1238,7 @@ __global__ __launch_bounds__(256) void k_chain(const float* __restrict__ points,
                     }
                 }
         }
-        if (tid < n && !(norm[tid] < 1e18f)) huge_s = 1;
+        if (tid < n && !(norm[tid] < 2e19f)) huge_s = 1;
         __syncthreads();
         if (zero_s) {
             // tmp[j]: the first point at distance 0 from j, if it has the coordinates of j (eight lanes compare), else j
