@@ -139,7 +139,7 @@ __global__ __launch_bounds__(256) void k_to_q8(const float* __restrict__ points,
         // err was measured against fl(lo + scale q); the screen evaluates lo sum n + scale sum n q in fp32 and is
         // compared with an fp32 evaluation of n.x: all of that stays below c_d (|lo| + 255 scale) per unit of ||n||_1
         const float mag = fabsf(lo) + 255.0f * scale;
-        float e1 = 1.01f * err + c_d * mag + 1e-37f;
+        float e1 = 1.01f * err + c_d * mag + kQ8Least;
         if (bad) e1 = __builtin_nanf("");      // the screen never decides for such a row
         if (lane == 0) {
             float* head = reinterpret_cast<float*>(dst);
@@ -234,7 +234,7 @@ __global__ __launch_bounds__(256) void k_to_q8_regs(const float* __restrict__ po
 #pragma unroll
         for (int o = 1; o < LPR; o <<= 1) err = fmaxf(err, __shfl_xor(err, o, 64));
         const float mag = fabsf(lo) + 255.0f * scale;
-        float e1 = 1.01f * err + c_d * mag + 1e-37f;
+        float e1 = 1.01f * err + c_d * mag + kQ8Least;
         if (badi) e1 = __builtin_nanf("");      // the screen never decides for such a row
         if (row_ok && l == 0) {
             *reinterpret_cast<float4*>(dst) = make_float4(0.0f, lo, scale, e1);

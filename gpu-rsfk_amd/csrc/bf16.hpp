@@ -50,13 +50,15 @@ struct Q8Copy {
 };
 
 // The screens of the side tests decide where margin > band: margin = |approximate n.x - offset|, band = what the approximation and
-// the exact fp32 evaluation can differ by when no sum overflows, plus 1e-30 for what underflow does to either.  Where a sum of
-// the exact evaluation could leave the range of fp32 (its comparison then has a side of its own) they must not decide.  With
-// the 8-bit copy that is settled per row and per hyperplane: a row with a coordinate beyond kQ8Most has e1 = NaN, a
-// hyperplane with a 1-norm above kNormalMost, or whose offset is not below 1e38, a bound of the 1-norm that is NaN, and what
-// is left has sums of at most 1e38 in the exact evaluation and 3e38 in the approximate one.  The bfloat16 rows have no header;
-// their sum |n_d||x_d| is tested at every point.  (The test at every point for both: tail kernel and chains of 20,000 x 64,
-// 50 trees 1.02 -> 1.06 ms.)
+// the exact fp32 evaluation can differ by.  Where a sum of the exact evaluation could leave the range of fp32 (its comparison
+// then has a side of its own) they must not decide, and what underflow does has to be in the band.  With the 8-bit copy both
+// are settled per row and per hyperplane: a row with a coordinate beyond kQ8Most has e1 = NaN, a hyperplane with a 1-norm
+// above kNormalMost, or whose offset is not below 1e38, a bound of the 1-norm that is NaN, and what is left has sums of at
+// most 1e38 in the exact evaluation and 3e38 in the approximate one; e1 has kQ8Least in it and the bound of the 1-norm
+// kNormalLeast, whose product is above the 2e-45 D that underflow amounts to.  The bfloat16 rows have no header; their sum
+// |n_d||x_d| is tested at every point.  (The test at every point for both: tail kernel and chains of 20,000 x 64, 50 trees
+// 1.02 -> 1.06 ms.)
+constexpr float kQ8Least = 1e-21f, kNormalLeast = 1e-18f;
 constexpr float kQ8Most = 1e18f, kNormalMost = 1e20f;
 
 int q8_copy_alloc(Q8Copy* c, int N, int D);

@@ -137,8 +137,8 @@ __device__ __forceinline__ void make_hyperplane_wave(const float* __restrict__ x
     s = half_butterfly_sum(s);
     s2 = half_butterfly_sum(s2);
     if (lane == 0) hp[0] = s;
-    const bool in_range = s <= kNormalMost && fabsf(read_lane_f(s, 0)) < 1e38f;
-    if (lane == 32) { hp[1] = s == 0.0f ? kZeroNormal : in_range ? s * 1.001f : __builtin_nanf(""); hp[2] = s2; }
+    if (lane == 32) { hp[1] = s == 0.0f ? kZeroNormal : s <= kNormalMost ? s * 1.001f + kNormalLeast : __builtin_nanf(""); hp[2] = s2; }
+    if (lane == 0 && !(fabsf(s) < 1e38f)) hp[1] = __builtin_nanf("");
 }
 
 // Screen of the side test for eight points per wavefront (right = n.x < b): lanes 8g..8g+7 work on
@@ -214,7 +214,7 @@ __device__ __forceinline__ void side_screen8(const float* nvec0, int nstride, co
             if (LPP >= 8) d += dpp_f<kDppHalfMirror>(d);
             const float lo = __uint_as_float(head[u].y), scale = __uint_as_float(head[u].z), e1 = __uint_as_float(head[u].w);
             const float approx = __builtin_fmaf(scale, d, lo * hp2[u]);
-            const bool certain = fabsf(approx - b[u]) > __builtin_fmaf(e1, hp1[u], 1e-30f);       // false if anything is NaN
+            const bool certain = fabsf(approx - b[u]) > e1 * hp1[u];       // false if anything is NaN
             right[u] = approx < b[u];
             redo[u] = valid[u] && !certain;
         }
@@ -799,9 +799,10 @@ constexpr int kMaxGroup = 16;        // nodes of one level of a subtree worked o
 // subtree is a few per level instead of a few per node.
 // TB = threads per workgroup: 256, or 512 / 1024 for launches over so few subtrees that workgroups of 256 would leave
 // most of the device idle (the phases of a level then have more lanes).  CHAIN: nodes that are split in vain go to
-// the queue of the chain phase.
+// the queue of the chain phase.  The form of 256 threads is for many subtrees and lives by six wavefronts per SIMD, for which
+// it has to stay within 80 registers (81 and five wavefronts: 1M x 100, 50 trees 10.8 -> 12.3 ms).
 template <bool Q8, int TB, bool CHAIN>
-__global__ __launch_bounds__(TB) void k_tail(const float* __restrict__ points,
+__global__ __launch_bounds__(TB, TB == 256 ? 6 : 1) void k_tail(const float* __restrict__ points,
                                                  const uint16_t* __restrict__ pb16, const uint8_t* __restrict__ q8, TreeParams P,
                                                  const int* __restrict__ perm0, const int* __restrict__ perm1,
                                                  int* __restrict__ perm_out,

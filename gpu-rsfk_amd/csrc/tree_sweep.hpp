@@ -306,7 +306,7 @@ __global__ __launch_bounds__(256) void k_pm_sweep(const uint8_t* __restrict__ q8
             const float b = qa.x, hp1 = qa.y, hp2 = qa.z, s2 = qa.w, c0 = qb.x, rres = qb.y;
             const float T = __builtin_fmaf(s2, (float)I, c0);
             const float approx = __builtin_fmaf(scale, T, lo * hp2);
-            const float band = __builtin_fmaf(e1, hp1, __builtin_fmaf(mag, rres, 1e-30f));
+            const float band = __builtin_fmaf(e1, hp1, mag * rres);
             const bool certain = fabsf(approx - b) > band;                 // false if anything is NaN
             const uint64_t rm = ballot64(active && certain && approx < b);
             const uint64_t um = ballot64(active && !certain);
