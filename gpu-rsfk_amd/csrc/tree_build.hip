@@ -1809,7 +1809,7 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
     // 20,000 x 32, 50 trees, 808 subtrees 1.69 -> 1.58 ms for the trees), and nodes that are split in vain leave for the
     // chain phase.  With more subtrees than that the device is full anyway and the chains run beside the rest: the
     // chain phase then only adds its matrices (1M x 100, 50 trees: tail 10.7 -> 9.0 ms, chains 6.8 ms).
-    // RSFK_TAIL_BLOCK=256 / 1024 overrides.
+    // RSFK_TAIL_BLOCK=256 / 1024: as with many / as with few subtrees, whatever their number.
     bool few = n_tail > 0 && n_tail < 8 * 256;
     if (const char* e = std::getenv("RSFK_TAIL_BLOCK")) few = std::atoi(e) >= 1024;
     RSFK_CHECK(n_tail <= w->tail_cap, "tree batch: tail queue overflow");
