@@ -89,7 +89,7 @@ __global__ void k_col_mean(float* __restrict__ mu, int D, float inv_n)
 
 // one wavefront per row of the 8-bit copy
 __global__ __launch_bounds__(256) void k_to_q8(const float* __restrict__ points, uint8_t* __restrict__ out,
-                                               float* __restrict__ rho_sum, int N, int D, int pitch, float c_d)
+                                               float* __restrict__ rho_sum, int N, int D, int pitch, float c_d, float most)
 {
     const int lane = threadIdx.x & 63;
     const int wave_global = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
@@ -102,7 +102,7 @@ __global__ __launch_bounds__(256) void k_to_q8(const float* __restrict__ points,
         bool bad = false;
         for (int d = lane; d < D; d += 64) {
             const float x = src[d];
-            bad |= !(fabsf(x) <= kQ8Most);
+            bad |= !(fabsf(x) <= 3.0e38f);                 // NaN or infinite
             lo = fminf(lo, x);
             hi = fmaxf(hi, x);
             sabs += fabsf(x);
@@ -138,9 +138,10 @@ __global__ __launch_bounds__(256) void k_to_q8(const float* __restrict__ points,
         for (int o = 1; o < 64; o <<= 1) err = fmaxf(err, __shfl_xor(err, o, 64));
         // err was measured against fl(lo + scale q); the screen evaluates lo sum n + scale sum n q in fp32 and is
         // compared with an fp32 evaluation of n.x: all of that stays below c_d (|lo| + 255 scale) per unit of ||n||_1
+        // (1.001 for the rounding of ||n||_1 itself)
         const float mag = fabsf(lo) + 255.0f * scale;
-        float e1 = 1.01f * err + c_d * mag + kQ8Least;
-        if (bad) e1 = __builtin_nanf("");      // the screen never decides for such a row
+        float e1 = 1.0111f * err + 1.0011f * (c_d * mag) + kQ8Least;
+        if (bad || !(range <= 3.0e38f)) e1 = __builtin_nanf("");      // the screen never decides for such a row
         if (lane == 0) {
             float* head = reinterpret_cast<float*>(dst);
             head[0] = 0.0f;
@@ -149,6 +150,7 @@ __global__ __launch_bounds__(256) void k_to_q8(const float* __restrict__ points,
             head[3] = e1;
             const float bf = sabs / (float)D * (1.0f / 256.0f);
             rho_acc += (e1 == e1 && bf > 0.0f) ? fminf(e1 / bf, 1000.0f) : 1000.0f;
+            if (!bad && fmaxf(fabsf(lo), fabsf(hi)) > most) rho_acc = INFINITY;
         }
     }
     // one atomic per workgroup (they all hit the same address)
@@ -169,7 +171,7 @@ __global__ __launch_bounds__(256) void k_to_q8(const float* __restrict__ points,
 // Needs D % 4 == 0 and 16-byte aligned points.
 template <int LPR, int PPL>
 __global__ __launch_bounds__(256) void k_to_q8_regs(const float* __restrict__ points, uint8_t* __restrict__ out,
-                                                    float* __restrict__ rho_sum, int N, int D, int pitch, float c_d)
+                                                    float* __restrict__ rho_sum, int N, int D, int pitch, float c_d, float most)
 {
     constexpr int kRowsPerWave = 64 / LPR;
     const int lane = threadIdx.x & 63, sub = lane / LPR, l = lane - sub * LPR;
@@ -193,7 +195,7 @@ __global__ __launch_bounds__(256) void k_to_q8_regs(const float* __restrict__ po
                 const float v[4] = {x[k].x, x[k].y, x[k].z, x[k].w};
 #pragma unroll
                 for (int c = 0; c < 4; ++c) {
-                    bad |= !(fabsf(v[c]) <= kQ8Most);
+                    bad |= !(fabsf(v[c]) <= 3.0e38f);              // NaN or infinite
                     lo = fminf(lo, v[c]);
                     hi = fmaxf(hi, v[c]);
                     sabs += fabsf(v[c]);
@@ -234,12 +236,13 @@ __global__ __launch_bounds__(256) void k_to_q8_regs(const float* __restrict__ po
 #pragma unroll
         for (int o = 1; o < LPR; o <<= 1) err = fmaxf(err, __shfl_xor(err, o, 64));
         const float mag = fabsf(lo) + 255.0f * scale;
-        float e1 = 1.01f * err + c_d * mag + kQ8Least;
-        if (badi) e1 = __builtin_nanf("");      // the screen never decides for such a row
+        float e1 = 1.0111f * err + 1.0011f * (c_d * mag) + kQ8Least;
+        if (badi || !(range <= 3.0e38f)) e1 = __builtin_nanf("");      // the screen never decides for such a row
         if (row_ok && l == 0) {
             *reinterpret_cast<float4*>(dst) = make_float4(0.0f, lo, scale, e1);
             const float bf = sabs / (float)D * (1.0f / 256.0f);
             rho_acc += (e1 == e1 && bf > 0.0f) ? fminf(e1 / bf, 1000.0f) : 1000.0f;
+            if (!badi && fmaxf(fabsf(lo), fabsf(hi)) > most) rho_acc = INFINITY;
         }
     }
     // one atomic per workgroup (they all hit the same address)
@@ -281,13 +284,13 @@ int q8_copy_fill(const Q8Copy& c, const float* points, int N, int D, hipStream_t
     const bool vec_ok = (D & 3) == 0 && (reinterpret_cast<uintptr_t>(points) & 15) == 0;
 #define RSFK_Q8_REGS(L, P)                                                                                                 \
     hipLaunchKernelGGL((k_to_q8_regs<L, P>), dim3(std::min((N + 4 * (64 / L) - 1) / (4 * (64 / L)), 8192)), dim3(256), 0,   \
-                       stream, points, c.rows, c.rho_sum, N, D, pitch, c_d)
+                       stream, points, c.rows, c.rho_sum, N, D, pitch, c_d, q8_most(D))
     if (vec_ok && words <= 16) RSFK_Q8_REGS(16, 1);
     else if (vec_ok && words <= 32) RSFK_Q8_REGS(32, 1);
     else if (vec_ok && words <= 64) RSFK_Q8_REGS(64, 1);
     else if (vec_ok && words <= 128) RSFK_Q8_REGS(64, 2);
     else if (vec_ok && words <= 256) RSFK_Q8_REGS(64, 4);
-    else hipLaunchKernelGGL(k_to_q8, dim3(grid), dim3(256), 0, stream, points, c.rows, c.rho_sum, N, D, pitch, c_d);
+    else hipLaunchKernelGGL(k_to_q8, dim3(grid), dim3(256), 0, stream, points, c.rows, c.rho_sum, N, D, pitch, c_d, q8_most(D));
 #undef RSFK_Q8_REGS
     RSFK_HIP(hipGetLastError());
     return 0;

@@ -38,7 +38,7 @@ struct Bf16Copy {
 // byte per coordinate, q_d = round((x_d - lo) / scale) in 0..255 with lo = min_d x_d and scale = (max_d x_d - lo) / 255,
 // zeros up to the end of the row.  e1 bounds what the quantisation can do to a dot product per unit of the
 // 1-norm of the other vector: for any n, |n.x - (lo sum_d n_d + scale sum_d n_d q_d)| <= e1 ||n||_1, including
-// the fp32 evaluation of either side with at most D/8-term chains (see k_to_q8); NaN where nothing is to be decided.  mean_rho (host, after
+// the fp32 evaluation of either side with at most D/8-term chains (see k_to_q8).  mean_rho (host, after
 // q8_copy_fill has completed) compares e1 with the corresponding quantity of the bfloat16 copy,
 // 2^-8 mean_d |x_d|, averaged over the rows: the 8-bit copy pays off while it is below about 6.
 __host__ __device__ inline int q8_pitch(int D) { return (16 + D + 63) & ~63; }
@@ -51,15 +51,15 @@ struct Q8Copy {
 
 // The screens of the side tests decide where margin > band: margin = |approximate n.x - offset|, band = what the approximation and
 // the exact fp32 evaluation can differ by.  Where a sum of the exact evaluation could leave the range of fp32 (its comparison
-// then has a side of its own) they must not decide, and what underflow does has to be in the band.  With the 8-bit copy both
-// are settled per row and per hyperplane: a row with a coordinate beyond kQ8Most has e1 = NaN, a hyperplane with a 1-norm
-// above kNormalMost, or whose offset is not below 1e38, a bound of the 1-norm that is NaN, and what is left has sums of at
-// most 1e38 in the exact evaluation and 3e38 in the approximate one; e1 has kQ8Least in it and the bound of the 1-norm
-// kNormalLeast, whose product is above the 2e-45 D that underflow amounts to.  The bfloat16 rows have no header; their sum
-// |n_d||x_d| is tested at every point.  (The test at every point for both: tail kernel and chains of 20,000 x 64, 50 trees
-// 1.02 -> 1.06 ms.)
+// then has a side of its own) they must not decide, and what underflow does has to be in the band.
+// 8-bit copy: not used at all when a finite row has a coordinate beyond q8_most(D) (mean_rho is infinite then).  Up to there
+// |n.x| <= 2 D q8_most^2 = 1e38, and neither evaluation nor the offset can overflow; a row or a normal that is not finite has a
+// band that is NaN or infinite.  e1 has kQ8Least in it and the bound of the 1-norm kNormalLeast, whose product is above the
+// 2e-45 D that underflow amounts to.
+// bfloat16 copy: sum |n_d||x_d|, which is part of the band, is compared with 1e38 at every point.  (The same for the 8-bit copy, or
+// limits per row and per hyperplane: tail kernel and chains of 20,000 x 64, 50 trees 1.02 -> 1.06 and 1.04 ms.)
 constexpr float kQ8Least = 1e-21f, kNormalLeast = 1e-18f;
-constexpr float kQ8Most = 1e18f, kNormalMost = 1e20f;
+inline float q8_most(int D) { return 7.07e18f / __builtin_sqrtf((float)D); }
 
 int q8_copy_alloc(Q8Copy* c, int N, int D);
 void q8_copy_free(Q8Copy* c);

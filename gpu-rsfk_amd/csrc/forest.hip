@@ -122,7 +122,7 @@ struct TimedEvent {
 
 // Side tests of the trees are screened on the 8-bit copy when its quantisation error is within a small factor
 // of the bfloat16 rounding error on these points (half the bytes per row), else on the bfloat16 copy.
-// RSFK_TREE_SCREEN=q8 / bf16 forces one of them.  *rows = the 8-bit rows, or null for the bfloat16 screen.
+// RSFK_TREE_SCREEN=q8 / bf16 forces one of them (the first only where its sums cannot overflow: q8_most).  *rows = the 8-bit rows, or null for the bfloat16 screen.
 int make_tree_screen(Q8Guard& q8, const float* d_points, int N, int D, int verbose, hipStream_t stream, const uint8_t** rows)
 {
     *rows = nullptr;
@@ -133,7 +133,7 @@ int make_tree_screen(Q8Guard& q8, const float* d_points, int N, int D, int verbo
     if (q8_copy_alloc(&q8.c, N, D) || q8_copy_fill(q8.c, d_points, N, D, stream)) return 1;
     float rho = 0.0f;
     if (q8_copy_mean_rho(q8.c, N, &rho, stream)) return 1;
-    if (force_q8 || rho <= 6.0f) *rows = q8.c.rows;
+    if (rho <= (force_q8 ? 3.0e38f : 6.0f)) *rows = q8.c.rows;
     if (verbose >= 2)
         std::printf("8-bit copy: quantisation error %.2f x bfloat16 rounding error -> %s screen\n", rho,
                     *rows ? "8-bit" : "bfloat16");

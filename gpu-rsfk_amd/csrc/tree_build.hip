@@ -93,10 +93,10 @@ __host__ __device__ inline int nvec_len(int D) { return (D + 15) & ~15; }
 
 // Hyperplane of (x1,x2) by one wavefront (all 64 lanes call): normal into LDS nvec[0..nvec_len(D)), and
 // hp[0] = offset (order of create_node.cu:122-135: 32 lane-strided partial sums + xor butterfly),
-// hp[1] = an upper bound of the 1-norm of the normal, hp[2] = the sum of its components (any order: only the
-// screens use them, with a margin).  NaN in place of the bound: the screens do not decide (bf16.hpp).  A pair with the same coordinates has the normal 0 and every point on its left (0 < 0):
+// hp[1] = the 1-norm of the normal (kNormalLeast added: bf16.hpp), hp[2] = the sum of its components (any order: only the
+// screens use them, with a margin).  A pair with the same coordinates has the normal 0 and every point on its left (0 < 0):
 // its hp[1] is kZeroNormal, which makes the bounds of the screens negative, so that no point is left to the exact test
-// (100,000 x 32, a tenth of the points in groups of 2,000 equal rows, 10 trees: 947 -> 224 ms).
+// (100,000 x 32, a tenth of the points in groups of 2,000 equal rows, 10 trees: 947 -> 220 ms).
 constexpr float kZeroNormal = -1e30f;
 __device__ __forceinline__ void make_hyperplane_wave(const float* __restrict__ x1, const float* __restrict__ x2,
                                                      int D, float* nvec, float* hp)
@@ -137,8 +137,7 @@ __device__ __forceinline__ void make_hyperplane_wave(const float* __restrict__ x
     s = half_butterfly_sum(s);
     s2 = half_butterfly_sum(s2);
     if (lane == 0) hp[0] = s;
-    if (lane == 32) { hp[1] = s == 0.0f ? kZeroNormal : s <= kNormalMost ? s * 1.001f + kNormalLeast : __builtin_nanf(""); hp[2] = s2; }
-    if (lane == 0 && !(fabsf(s) < 1e38f)) hp[1] = __builtin_nanf("");
+    if (lane == 32) { hp[1] = s == 0.0f ? kZeroNormal : s + kNormalLeast; hp[2] = s2; }
 }
 
 // Screen of the side test for eight points per wavefront (right = n.x < b): lanes 8g..8g+7 work on
@@ -263,9 +262,8 @@ __device__ __forceinline__ void side_screen8(const float* nvec0, int nstride, co
             float d = da[u], a = sa[u];
             d += dpp_f<kDppXor1>(d); d += dpp_f<kDppXor2>(d); d += dpp_f<kDppHalfMirror>(d);
             a += dpp_f<kDppXor1>(a); a += dpp_f<kDppXor2>(a); a += dpp_f<kDppHalfMirror>(a);
-            // (a below 1e38: no partial sum of the exact test overflows; an infinite margin: the offset did)
-            const float margin = fabsf(d - b[u]);
-            const bool certain = margin > a * band + (1e-30f + fminf(hp1[u], 0.0f)) && a < 1e38f && margin < INFINITY;
+            // (a below 1e38: no partial sum of the exact test overflows)
+            const bool certain = fabsf(d - b[u]) > a * band + (1e-30f + fminf(hp1[u], 0.0f)) && a < 1e38f;
             right[u] = d < b[u];
             redo[u] = valid[u] && !certain;
         }
@@ -1222,14 +1220,15 @@ __global__ __launch_bounds__(256) void k_chain(const float* __restrict__ points,
                 }
                 __syncthreads();
             }
+            float least = INFINITY, most = 0.0f;                              // of the distances between two points of the node
 #pragma unroll
             for (int c = 0; c < NB; ++c)
 #pragma unroll
                 for (int r = 0; r <= c; ++r) {
                     const int i = ty + 16 * r, j = tx + 16 * c;
                     if (c < nb && i <= j && j < n) {
-                        if (i < j && acc[c * (c + 1) / 2 + r] == 0.0f) zero_s = 1;
-                        if (!(acc[c * (c + 1) / 2 + r] < 2e37f)) huge_s = 1;
+                        least = fminf(least, i < j ? acc[c * (c + 1) / 2 + r] : INFINITY);
+                        most = fmaxf(most, acc[c * (c + 1) / 2 + r]);
                         if constexpr (NB == 8) {
                             tri[i * (n | 1) + j] = acc[c * (c + 1) / 2 + r];
                             tri[j * (n | 1) + i] = acc[c * (c + 1) / 2 + r];
@@ -1238,6 +1237,8 @@ __global__ __launch_bounds__(256) void k_chain(const float* __restrict__ points,
                         }
                     }
                 }
+            if (least == 0.0f) zero_s = 1;
+            if (!(most < 2e37f)) huge_s = 1;
         }
         if (tid < n && !(norm[tid] < 2e19f)) huge_s = 1;
         __syncthreads();

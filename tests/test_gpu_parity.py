@@ -115,8 +115,8 @@ def test_tree_nodes_of_equal_rows(gpu, orc, rng, monkeypatch, N, D, MIN, MAX, ki
 
 
 # Rows whose dot products overflow (all of them near the limit; a tenth of the rows far above the others), overflow in one
-# factor only, lie about where a screen stops to decide, or are denormal: every kernel of the side tests (wide levels point by point and node by node, tail, chains).
-@pytest.mark.parametrize("kind", ["near_overflow", "mixed", "spread", "limits", "denormal"])
+# factor only, lie just below and above where the 8-bit copy is given up, or are denormal: every kernel of the side tests (wide levels point by point and node by node, tail, chains).
+@pytest.mark.parametrize("kind", ["near_overflow", "mixed", "spread", "below", "above", "denormal"])
 @pytest.mark.parametrize("env", [dict(SCREEN="q8", PM="7"), dict(SCREEN="q8", PM="0"), dict(SCREEN="q8", PM="0", TAIL="256"), dict(SCREEN="bf16"),
                                  dict(SCREEN="bf16", TAIL="256")], ids=lambda e: "-".join(e.values()))
 def test_tree_of_rows_whose_sums_leave_fp32(gpu, orc, rng, monkeypatch, kind, env):
@@ -125,8 +125,9 @@ def test_tree_of_rows_whose_sums_leave_fp32(gpu, orc, rng, monkeypatch, kind, en
             monkeypatch.setenv(var, env[name])
     N, D, MIN, MAX, depth = 6000, 48, 17, 34, 60
     X = rng.standard_normal((N, D))
-    scale = {"near_overflow": 3e18, "denormal": 3e-22, "mixed": np.where(rng.random((N, 1)) < 0.1, 3e18, 1.0),
-             "spread": 10.0 ** rng.uniform(-25, 37, (N, 1)), "limits": 10.0 ** rng.uniform(15, 20, (N, 1))}[kind]
+    most = 7.07e18 / np.sqrt(D) / np.abs(X).max()
+    scale = {"near_overflow": 3e18, "below": 0.999 * most, "above": 1.001 * most, "denormal": 3e-22, "mixed": np.where(rng.random((N, 1)) < 0.1, 3e18, 1.0),
+             "spread": 10.0 ** rng.uniform(-25, 37, (N, 1))}[kind]
     X = (X * scale).astype(np.float32)
     for seed in (1, 2):
         _say("tree beyond fp32", kind, env, seed)
