@@ -61,7 +61,7 @@ __global__ __launch_bounds__(256) void k_planes(const float* __restrict__ points
 {
     const int lane = threadIdx.x & 63;
     const int r = blockIdx.x * 4 + (threadIdx.x >> 6), j = blockIdx.y;
-    if (r >= min(n_rec_p[j], rec_cap)) return;
+    if (r >= min(n_rec_p[kTreeStatPitch * j], rec_cap)) return;
     const size_t at = (size_t)j * (size_t)rec_cap + (size_t)r;
     const TreeRec rec = recs[at];
     float* low_row = low ? low + at * (size_t)low_pitch : nullptr;
@@ -779,7 +779,7 @@ int ann_forest_group(int N, int NQ, int D, int K, int MAX, int max_bucket, int r
     return group >= 2 ? group : 0;
 }
 
-// The search in T trees at once.  recs, n_rec_dev, perm: those of the first tree, the others follow; planes: T rec_cap
+// The search in T trees at once.  recs, n_rec_dev, perm: those of the first tree, the others follow (n_rec_dev: kTreeStatPitch apart); planes: T rec_cap
 // ann_plane_pitch(NQ, D) floats; reached: 2 NQ T ints.
 int launch_ann_forest(const float* points, const float* queries, int N, int NQ, int D, int K, int T, const int* perm, const TreeRec* recs,
                       const int* n_rec_dev, int rec_cap, float* planes, int* reached, int* q_idx, float* q_dist, hipStream_t stream)

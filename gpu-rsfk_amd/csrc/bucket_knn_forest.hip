@@ -38,7 +38,7 @@ struct alignas(16) PairsLds {
     int idb[kTile];
 };
 
-// stats: five ints per tree, {buckets of at most kBucketSplit points, larger ones, ...}: the former fill the front of the
+// stats: kTreeStatPitch ints per tree, {buckets of at most kBucketSplit points, larger ones, ...}: the former fill the front of the
 // tree's leaf table, the latter its back.  tri: tiles on and above the diagonal of the largest bucket (of max_tiles by
 // max_tiles tiles).
 __global__ __launch_bounds__(256) void k_forest_pairs(const float* __restrict__ points, int N, int D, int T, const int* __restrict__ perm,
@@ -48,7 +48,7 @@ __global__ __launch_bounds__(256) void k_forest_pairs(const float* __restrict__ 
 {
     __shared__ PairsLds L;
     const int j = blockIdx.y;
-    const int n_small = stats[5 * j], n_big = stats[5 * j + 1];
+    const int n_small = stats[kTreeStatPitch * j], n_big = stats[kTreeStatPitch * j + 1];
     int slot = blockIdx.x, I = 0, J = 0;
     if (slot >= n_small) {
         const int y = slot - n_small, big = y / tri;

@@ -43,6 +43,17 @@ __device__ __forceinline__ void load_split(const float* __restrict__ p, bf16x8& 
     split8(*reinterpret_cast<const float4*>(p), *reinterpret_cast<const float4*>(p + 4), hi, lo, nrm);
 }
 
+// The same with halves: x = hi + lo + r with |r| <= 2^-20 |x| while |x| is in the range of normal halves (both rounded toward
+// zero); what is below the least of them, 2^-14, may be lost.
+typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
+typedef __attribute__((ext_vector_type(2))) __fp16 half2_rtz;
+__device__ __forceinline__ void split2_half(float a, float b, uint32_t& hi, uint32_t& lo)
+{
+    const half2_rtz h = __builtin_amdgcn_cvt_pkrtz(a, b);
+    hi = __builtin_bit_cast(uint32_t, h);
+    lo = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a - (float)h.x, b - (float)h.y));
+}
+
 // Coefficient c of the bound |d~ - d| <= c S, S = |a|^2 + |b|^2, d~ = |a|^2 + |b|^2 - 2 G with G from the three
 // products above over D16 (= D rounded up to 16) dimensions: dropped products <= 3 * 2^-16 |x||y| <= 1.5 * 2^-16 S;
 // 3 D16 exact products per entry accumulated in fp32, every addition within 2^-23 of the sum of absolute values

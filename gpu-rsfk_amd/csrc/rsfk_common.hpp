@@ -132,6 +132,9 @@ struct TreeRec {
     int a, b, c0, c1;
 };
 
+// Ints from the counts of one tree of a batch to those of the next one (TreeStats, a cache line each).
+constexpr int kTreeStatPitch = 32;
+
 // Buckets of at most this many points are handled by the small-bucket K-NN kernel; the
 // tree builder keeps them apart from the larger ones.
 constexpr int kBucketSplit = 64;
@@ -153,8 +156,7 @@ struct TreeParams {
     int N, D;
     int MIN, MAX, MAX_DEPTH;
     int small;        // nodes with at most this many points are finished by one workgroup
-    int vain;         // a node split in vain this many times in a row ...
-    int chain_max;    // ... and of at most this many points goes to the chain phase (0: never)
+    int chain_max;    // nodes of at most this many points go to the chain phase (0: none)
     int chunk;        // points per workgroup in the wide (global) passes
     float band;       // half-width of the undecided band of the bfloat16 side screen, relative to sum |n_d||x~_d|
 };

@@ -24,8 +24,8 @@
 //                most `small` points inside LDS (all the re-draw levels that
 //                the min/max rule causes touch only such nodes).
 //
-//   chain phase : nodes the tail kernel has split in vain several times in a row
-//                are finished from the distances of their points (k_chain).
+//   chain phase : nodes of some hundred points are finished from the distances of
+//                their points (k_chain).
 //
 // Arithmetic follows the reference bit for bit: the hyperplane offset and the
 // side test are sums of 32 lane-strided partials combined by the xor butterfly
@@ -36,6 +36,7 @@
 #include "knn_list.hpp"
 #include "bf16.hpp"
 #include "tree_sweep.hpp"
+#include "mfma_split.hpp"
 #include "level_notes.hpp"
 #include <vector>
 #include <algorithm>
@@ -58,13 +59,17 @@ struct LevelCounters {
         int chunks;    // and their chunks
     } queue[4];
     int n_tail;        // tail tasks appended so far
-    int n_chain;       // nodes for the chain phase appended so far
+    int n_chain;       // nodes for the chain phase appended so far, at the front of their queue
+    int n_chain_back;  // ... and at its back: those that are hardly split in vain
     int overflow;      // set when a queue capacity is exceeded
-    int pad_;
     // time spent in the three steps of the wide levels (hyperplanes, side tests, scatter) and in the tail, in ticks of
     // the device's constant-rate clock: the first thread of a kernel that opens a step closes the one before it
     long long last_tick;
     long long phase_ticks[4];
+    // nodes of the chain phase taken from the queue, beyond the first one of every workgroup: node i belongs to share i % kShares
+    // (additions to one cache line come one after the other)
+    static constexpr int kShares = 16;
+    struct alignas(128) Share { int taken; } share[kShares];
 };
 
 // Counts for the report of a build (how many points the side tests of all levels looked at, and how many of them
@@ -162,7 +167,8 @@ __device__ __forceinline__ void make_hyperplane_wave(const float* __restrict__ x
 // scale sum_d n_d q_d, undecided band e1 ||n||_1 (hp1 = bound of the 1-norm, hp2 = sum of the components of the
 // normal of the point's node).  Only lane 0 of a group holds the header, so only its right / redo are meaningful
 // (with either copy the callers use lane 0 only).
-template <int NB, bool Q8, int LPP = 8>
+// (KU: pieces of a row a lane has in flight, 8-bit copy)
+template <int NB, bool Q8, int LPP = 8, int KU = 1>
 __device__ __forceinline__ void side_screen8(const float* nvec0, int nstride, const int (&j)[NB], const float (&b)[NB],
                                              const float (&hp1)[NB], const float (&hp2)[NB],
                                              const uint16_t* __restrict__ pb16, const uint8_t* __restrict__ q8,
@@ -184,24 +190,32 @@ __device__ __forceinline__ void side_screen8(const float* nvec0, int nstride, co
             head[u] = make_uint4(0u, 0u, 0u, 0u);
             if (valid[u] && sub == 0) head[u] = *reinterpret_cast<const uint4*>(q8 + (size_t)id[u] * pitch);
         }
-        for (int k = sub; k < pieces; k += LPP) {
-            uint4 w[NB];
+        for (int k0 = sub; k0 < pieces; k0 += KU * LPP) {
+            uint4 w[KU][NB];
 #pragma unroll
-            for (int u = 0; u < NB; ++u) {
-                w[u] = make_uint4(0u, 0u, 0u, 0u);
-                if (valid[u]) w[u] = *reinterpret_cast<const uint4*>(q8 + (size_t)id[u] * pitch + 16 + 16 * k);
-            }
+            for (int y = 0; y < KU; ++y)
 #pragma unroll
-            for (int u = 0; u < NB; ++u) {
-                const float* nvec = nvec0 + (size_t)j[u] * nstride + 16 * k;
-                const uint32_t ww[4] = {w[u].x, w[u].y, w[u].z, w[u].w};
+                for (int u = 0; u < NB; ++u) {
+                    w[y][u] = make_uint4(0u, 0u, 0u, 0u);
+                    if (valid[u] && (KU == 1 || k0 + y * LPP < pieces))
+                        w[y][u] = *reinterpret_cast<const uint4*>(q8 + (size_t)id[u] * pitch + 16 + 16 * (k0 + y * LPP));
+                }
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const float4 nq = *reinterpret_cast<const float4*>(&nvec[4 * q]);
-                    da[u] = __builtin_fmaf(nq.x, (float)((ww[q] >> 0) & 0xffu), da[u]);
-                    da[u] = __builtin_fmaf(nq.y, (float)((ww[q] >> 8) & 0xffu), da[u]);
-                    da[u] = __builtin_fmaf(nq.z, (float)((ww[q] >> 16) & 0xffu), da[u]);
-                    da[u] = __builtin_fmaf(nq.w, (float)((ww[q] >> 24) & 0xffu), da[u]);
+            for (int y = 0; y < KU; ++y) {
+                const int k = k0 + y * LPP;
+                if (KU > 1 && k >= pieces) break;
+#pragma unroll
+                for (int u = 0; u < NB; ++u) {
+                    const float* nvec = nvec0 + (size_t)j[u] * nstride + 16 * k;
+                    const uint32_t ww[4] = {w[y][u].x, w[y][u].y, w[y][u].z, w[y][u].w};
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const float4 nq = *reinterpret_cast<const float4*>(&nvec[4 * q]);
+                        da[u] = __builtin_fmaf(nq.x, (float)((ww[q] >> 0) & 0xffu), da[u]);
+                        da[u] = __builtin_fmaf(nq.y, (float)((ww[q] >> 8) & 0xffu), da[u]);
+                        da[u] = __builtin_fmaf(nq.z, (float)((ww[q] >> 16) & 0xffu), da[u]);
+                        da[u] = __builtin_fmaf(nq.w, (float)((ww[q] >> 24) & 0xffu), da[u]);
+                    }
                 }
             }
         }
@@ -315,7 +329,6 @@ __device__ __forceinline__ void resolve_exact(int halves, int h, const int* list
 }
 
 constexpr int kSideBatch = 4;        // points per group and call of the screen in the wide phase
-constexpr int kTailBatch = 2;        // ... in the tail kernel
 
 // The queues nodes go to: the next wide level (entry `slot` of the counters) and the tail kernel (one workgroup per node).
 struct NodeQueues {
@@ -442,16 +455,20 @@ __device__ __forceinline__ void index_bucket(TreeRec* recs, int rec_cap, int my_
 // wide phase kernels
 // ---------------------------------------------------------------------------
 
-struct TreeStats {          // one per tree of the batch
+// One per tree of the batch, each in a cache line of its own: the workgroups of all trees add to them at the same time, and additions
+// to one line are carried out one after the other (chain phase of 50 trees of 20,000 x 64 points, with an index: 321 us with all trees
+// in a few lines, 207 so).
+struct alignas(4 * kTreeStatPitch) TreeStats {
     int n_leaves;           // buckets of at most kBucketSplit points, stored from the front of the leaf table
     int n_big;              // larger buckets, stored from the back of the leaf table
     int levels;
     int max_leaf;
     int min_leaf;
+    int n_rec;              // records of the index, when one is written
 };
 
 // A batch begins: permutations, counters, and the root of every tree (workgroup 0).
-__global__ __launch_bounds__(256) void k_tree_init(int* __restrict__ perm, NodeQueues Q, TreeParams P, int B, int seed0, int* n_rec, int* pmap,
+__global__ __launch_bounds__(256) void k_tree_init(int* __restrict__ perm, NodeQueues Q, TreeParams P, int B, int seed0, int* pmap,
                                                    TreeStats* __restrict__ stats, unsigned long long* __restrict__ stat)
 {
     const size_t total = (size_t)P.N * (size_t)B;
@@ -466,8 +483,8 @@ __global__ __launch_bounds__(256) void k_tree_init(int* __restrict__ perm, NodeQ
     if (t >= B) return;
     TreeStats s;
     s.n_leaves = 0; s.n_big = 0; s.levels = 0; s.max_leaf = 0; s.min_leaf = 0x7fffffff;
+    s.n_rec = 1;                           // record 0 is the root
     stats[t] = s;
-    if (n_rec) n_rec[t] = 1;               // record 0 is the root
     TreeNode r;
     r.tree = t; r.start = 0; r.count = P.N; r.dstart = 0; r.dcount = P.N; r.depth = 0; r.buf = 0; r.leaf = 0;
     r.rec = 0; r.chunk0 = 0;
@@ -607,7 +624,7 @@ __global__ __launch_bounds__(kBlock) void k_side(const float* __restrict__ point
 __global__ __launch_bounds__(kBlock) void k_scatter(TreeParams P, int* __restrict__ perm0, int* __restrict__ perm1,
                                                     const TreeNode* __restrict__ nodes, int slot,
                                                     const int* __restrict__ chunk2node, const int* __restrict__ chunk_left,
-                                                    NodeQueues Q, TreeRec* __restrict__ recs, int* __restrict__ n_rec,
+                                                    NodeQueues Q, TreeRec* __restrict__ recs, TreeStats* stats,
                                                     int rec_cap, int2* __restrict__ child)
 {
     LevelCounters* ctr = Q.ctr;
@@ -692,7 +709,7 @@ __global__ __launch_bounds__(kBlock) void k_scatter(TreeParams P, int* __restric
         if (recs) {
             int r1, r2;
             pick_pair(nd.key, nd.dcount, r1, r2);
-            index_split(recs + (size_t)nd.tree * rec_cap, n_rec + nd.tree, rec_cap, nd.rec, src[nd.dstart + r1] & kIdMask,
+            index_split(recs + (size_t)nd.tree * rec_cap, &stats[nd.tree].n_rec, rec_cap, nd.rec, src[nd.dstart + r1] & kIdMask,
                         src[nd.dstart + r2] & kIdMask, nc, c[0].rec, c[1].rec, ctr);
         }
         int at[2];
@@ -758,7 +775,6 @@ struct SmallNode {
     int start, count, dstart, dcount;     // offsets inside the task's segment
     int depth, leaf;
     int rec;                              // record of the node in the index of the tree, if one is written
-    int vain;                             // splits in a row that left all points together (chain phase)
     uint64_t key;
 };
 
@@ -789,6 +805,11 @@ __device__ __forceinline__ void emit_leaf(int tree, int gstart, int count, int d
     atomicMin(&st->min_leaf, count);
 }
 
+// Is a node of `count` points likely to be split in vain many times in a row?  A split counts when both sides have at least MIN points,
+// which leaves count - 2 MIN + 1 of the places it may have.
+__device__ __forceinline__ bool often_in_vain(int count, int MIN) { return 8 * (count - 2 * MIN + 1) <= count; }
+
+constexpr int kTailMost = 2048;      // points of the largest node the tail kernel takes
 constexpr int kMaxGroup = 16;        // nodes of one level of a subtree worked on together
 
 // One workgroup finishes the subtree of a task level by level: the nodes of a level are taken kMaxGroup (or
@@ -796,18 +817,20 @@ constexpr int kMaxGroup = 16;        // nodes of one level of a subtree worked o
 // one sweep, and each node is partitioned by one wavefront -- so the number of dependent trips to memory per
 // subtree is a few per level instead of a few per node.
 // TB = threads per workgroup: 256, or 512 / 1024 for launches over so few subtrees that workgroups of 256 would leave
-// most of the device idle (the phases of a level then have more lanes).  CHAIN: nodes that are split in vain go to
-// the queue of the chain phase.  The form of 256 threads is for many subtrees and lives by six wavefronts per SIMD, for which
+// most of the device idle (the phases of a level then have more lanes).  CHAIN: nodes of at most P.chain_max points go
+// to the queue of the chain phase.  The form of 256 threads is for many subtrees and lives by six wavefronts per SIMD, for which
 // it has to stay within 80 registers (81 and five wavefronts: 1M x 100, 50 trees 10.8 -> 12.3 ms).
-template <bool Q8, int TB, bool CHAIN>
-__global__ __launch_bounds__(TB, TB == 256 ? 6 : 1) void k_tail(const float* __restrict__ points,
+// LPP: lanes per point in the screen (k_side), eight with the bfloat16 copy; KU: 16-byte pieces of a point's row each of them has in
+// flight.
+template <bool Q8, int TB, bool CHAIN, int LPP, int KU>
+__global__ __launch_bounds__(TB, CHAIN ? 4 : 6) void k_tail(const float* __restrict__ points,
                                                  const uint16_t* __restrict__ pb16, const uint8_t* __restrict__ q8, TreeParams P,
                                                  const int* __restrict__ perm0, const int* __restrict__ perm1,
                                                  int* __restrict__ perm_out,
                                                  const TreeNode* __restrict__ tasks, int n_tasks, int node_cap, int G,
                                                  int leaf_cap, int* __restrict__ leaf_start, int* __restrict__ leaf_size,
                                                  TreeStats* stats, LevelCounters* ctr,
-                                                 TreeRec* __restrict__ recs_all, int* __restrict__ n_rec_all, int rec_cap,
+                                                 TreeRec* __restrict__ recs_all, int rec_cap,
                                                  unsigned long long* __restrict__ stat, TreeNode* __restrict__ chain_all, int chain_cap)
 {
     // dynamic LDS: seg[small] | tmp[small] | nvec[G][nvec_len(D)] | lrec[node_cap] | level lists 2 x node_cap |
@@ -826,8 +849,9 @@ __global__ __launch_bounds__(TB, TB == 256 ? 6 : 1) void k_tail(const float* __r
     unsigned char* fmap = reinterpret_cast<unsigned char*>(CHAIN ? chain + node_cap : chain);
     __shared__ float b_s[kMaxGroup], hp_s[kMaxGroup][3];
     __shared__ int left_s[kMaxGroup], pre_s[kMaxGroup + 1], start_s[kMaxGroup], pair_s[kMaxGroup][2];
+    __shared__ int piece_s[CHAIN ? kMaxGroup + 1 : 1], lefts_s[CHAIN ? kTailMost / 64 + kMaxGroup : 1];      // pieces of 64 members before a node's, lefts of a piece
     __shared__ int n_cur_s, n_nxt_s, nrec_s, kind_s[2], base_s[2], lev_s, mx_s, mn_s, n_def_s;
-    __shared__ int n_chain_s, chain_base_s;
+    __shared__ int n_chain_s[2], chain_base_s[2], n_chain_all_s;     // (front and back of the queue)
     __shared__ int seen_s, unsure_s;        // points tested over all levels of the subtree, and left to the exact test
 
     const int task = blockIdx.x;
@@ -849,16 +873,26 @@ __global__ __launch_bounds__(TB, TB == 256 ? 6 : 1) void k_tail(const float* __r
         }
         return;
     }
+    if (CHAIN && tk.count <= P.chain_max) {
+        if (src != dst)
+            for (int i = tid; i < tk.count; i += TB) dst[tk.start + i] = src[tk.start + i] & kIdMask;
+        if (tid == 0) {
+            const bool back = !often_in_vain(tk.count, P.MIN);
+            const int at = atomicAdd(back ? &ctr->n_chain_back : &ctr->n_chain, 1);
+            if (at < chain_cap) chain_all[back ? chain_cap - 1 - at : at] = tk; else ctr->overflow = 1;
+        }
+        return;
+    }
     TreeRec* recs = recs_all ? recs_all + (size_t)tk.tree * rec_cap : nullptr;
-    int* n_rec = recs_all ? n_rec_all + tk.tree : nullptr;
+    int* n_rec = &stats[tk.tree].n_rec;
     for (int i = tid; i < tk.count; i += TB) seg[i] = src[tk.start + i] & kIdMask;
     if (tid == 0) {
         SmallNode r;
         r.start = 0; r.count = tk.count; r.dstart = tk.dstart - tk.start; r.dcount = tk.dcount;
-        r.depth = tk.depth; r.leaf = 0; r.key = tk.key; r.rec = tk.rec; r.vain = 0;
+        r.depth = tk.depth; r.leaf = 0; r.key = tk.key; r.rec = tk.rec;
         cur[0] = r;
         n_cur_s = 1; n_nxt_s = 0; nrec_s = 0; kind_s[0] = 0; kind_s[1] = 0; lev_s = 0; mx_s = 0; mn_s = 0x7fffffff;
-        seen_s = 0; unsure_s = 0; n_chain_s = 0;
+        seen_s = 0; unsure_s = 0; n_chain_s[0] = 0; n_chain_s[1] = 0; n_chain_all_s = 0;
     }
     __syncthreads();
 
@@ -872,7 +906,8 @@ __global__ __launch_bounds__(TB, TB == 256 ? 6 : 1) void k_tail(const float* __r
         atomicMin(&mn_s, count);
     };
 
-    const int grp = tid >> 3, sub8 = tid & 7;       // 32 groups of 8 lanes, one point each per iteration
+    const int grp = tid / LPP, sub = tid & (LPP - 1);       // groups of LPP lanes, one point each per iteration
+    constexpr int kTailBatch = CHAIN && Q8 && KU == 1 ? 4 : 2;       // points per group and call of the screen
     while (true) {
         const int n_cur = n_cur_s;
         if (n_cur == 0) break;
@@ -890,8 +925,18 @@ __global__ __launch_bounds__(TB, TB == 256 ? 6 : 1) void k_tail(const float* __r
             if (tid == 0) {
                 n_def_s = 0;
                 int run = 0;
-                for (int j = 0; j < nb; ++j) { pre_s[j] = run; run += cur[b0 + j].count; }
+                int pieces = 0;
+                for (int j = 0; j < nb; ++j) {
+                    const int count = cur[b0 + j].count;
+                    pre_s[j] = run;
+                    run += count;
+                    if (CHAIN) {
+                        piece_s[j] = pieces;
+                        pieces += (count + 63) >> 6;
+                    }
+                }
                 pre_s[nb] = run;
+                if (CHAIN) piece_s[nb] = pieces;
             }
             __syncthreads();
             for (int j = wave; j < nb; j += TB / 64) {
@@ -906,7 +951,7 @@ __global__ __launch_bounds__(TB, TB == 256 ? 6 : 1) void k_tail(const float* __r
             __syncthreads();
             // side of every point of the group's nodes
             const int total = pre_s[nb];
-            constexpr int kTailGroups = TB / 8;
+            constexpr int kTailGroups = TB / LPP;
             const int iters = (total + kTailGroups - 1) / kTailGroups;
             for (int it = 0; it < iters; it += kTailBatch) {
                 int id[kTailBatch], jj[kTailBatch], pos[kTailBatch];
@@ -923,10 +968,10 @@ __global__ __launch_bounds__(TB, TB == 256 ? 6 : 1) void k_tail(const float* __r
                     h1[u] = hp_s[jj[u]][1];
                     h2[u] = hp_s[jj[u]][2];
                 }
-                side_screen8<kTailBatch, Q8>(nvec, Dv, jj, bb, h1, h2, pb16, q8, id, P.D, P.band, valid, right, redo);
+                side_screen8<kTailBatch, Q8, LPP, KU>(nvec, Dv, jj, bb, h1, h2, pb16, q8, id, P.D, P.band, valid, right, redo);
 #pragma unroll
                 for (int u = 0; u < kTailBatch; ++u) {
-                    if (valid[u] && sub8 == 0) {
+                    if (valid[u] && sub == 0) {
                         if (redo[u]) tmp[atomicAdd(&n_def_s, 1)] = pos[u] | (jj[u] << 16);      // tmp is free until the partition
                         else if (right[u]) seg[pos[u]] = id[u] | (int)0x80000000;
                     }
@@ -937,53 +982,108 @@ __global__ __launch_bounds__(TB, TB == 256 ? 6 : 1) void k_tail(const float* __r
             resolve_exact(TB >> 5, tid >> 5, tmp, n_def_s, nvec, Dv, b_s, points, P.D, [&](int pos) { return seg[pos] & kIdMask; },
                           [&](int pos, bool right) { if (right) seg[pos] |= (int)0x80000000; });
             __syncthreads();
-            // stable partition, one wavefront per node: seg -> tmp -> seg
-            for (int j = wave; j < nb; j += TB / 64) {
-                const int st = start_s[j], cnt = pre_s[j + 1] - pre_s[j];
-                int a = 0;
-                for (int r0 = 0; r0 < cnt; r0 += 64) a += __popcll(ballot64(r0 + lane < cnt && seg[st + r0 + lane] >= 0));
-                int lbase = 0;
-                for (int r0 = 0; r0 < cnt; r0 += 64) {
-                    const int i = r0 + lane;
-                    const bool valid = i < cnt;
-                    const int v = valid ? seg[st + i] : 0;
-                    const bool right = v < 0;
-                    const uint64_t m = ballot64(valid && !right);
-                    const int lrank = lbase + mask_prefix(m);
-                    if (valid) tmp[st + (right ? a + i - lrank : lrank)] = v & kIdMask;
-                    lbase += __popcll(m);
+            if constexpr (CHAIN) {
+                // stable partition, 64 members of a node at a time by one wavefront: lefts are counted, then everyone moves
+                // (seg -> tmp -> seg)
+                const int n_pieces = piece_s[nb];
+                auto node_of = [&](int c) { return __popcll(ballot64(lane < nb && piece_s[lane] <= c)) - 1; };
+                for (int c = wave; c < n_pieces; c += TB / 64) {
+                    const int j = node_of(c), i = 64 * (c - piece_s[j]) + lane;
+                    const bool valid = i < pre_s[j + 1] - pre_s[j];
+                    const uint64_t m = ballot64(valid && seg[valid ? start_s[j] + i : 0] >= 0);
+                    if (lane == 0) lefts_s[c] = __popcll(m);
                 }
-                wave_lds_sync();
-                for (int i = lane; i < cnt; i += 64) seg[st + i] = tmp[st + i];
-                if (lane == 0) left_s[j] = a;
+                __syncthreads();
+                for (int c = wave; c < n_pieces; c += TB / 64) {
+                    const int j = node_of(c), first = piece_s[j], st = start_s[j], i = 64 * (c - first) + lane;
+                    const bool valid = i < pre_s[j + 1] - pre_s[j];
+                    const int v = valid ? seg[st + i] : 0;
+                    // (a node has at most 32 pieces)
+                    const int x = lane < piece_s[j + 1] - first ? lefts_s[first + lane] : 0;
+                    const int a = wave_sum_i(x), before = wave_sum_i(lane < c - first ? x : 0);
+                    const bool right = v < 0;
+                    const int lrank = before + mask_prefix(ballot64(valid && !right));
+                    if (valid) tmp[st + (right ? a + i - lrank : lrank)] = v & kIdMask;
+                    if (c == first && lane == 0) left_s[j] = a;
+                }
+                __syncthreads();
+                for (int c = wave; c < n_pieces; c += TB / 64) {
+                    const int j = node_of(c), i = 64 * (c - piece_s[j]) + lane, st = start_s[j];
+                    if (i < pre_s[j + 1] - pre_s[j]) seg[st + i] = tmp[st + i];
+                }
+            } else {
+                // stable partition, one wavefront per node: seg -> tmp -> seg
+                for (int j = wave; j < nb; j += TB / 64) {
+                    const int st = start_s[j], cnt = pre_s[j + 1] - pre_s[j];
+                    int a = 0;
+                    for (int r0 = 0; r0 < cnt; r0 += 64) a += __popcll(ballot64(r0 + lane < cnt && seg[st + r0 + lane] >= 0));
+                    int lbase = 0;
+                    for (int r0 = 0; r0 < cnt; r0 += 64) {
+                        const int i = r0 + lane;
+                        const bool valid = i < cnt;
+                        const int v = valid ? seg[st + i] : 0;
+                        const bool right = v < 0;
+                        const uint64_t m = ballot64(valid && !right);
+                        const int lrank = lbase + mask_prefix(m);
+                        if (valid) tmp[st + (right ? a + i - lrank : lrank)] = v & kIdMask;
+                        lbase += __popcll(m);
+                    }
+                    wave_lds_sync();
+                    for (int i = lane; i < cnt; i += 64) seg[st + i] = tmp[st + i];
+                    if (lane == 0) left_s[j] = a;
+                }
             }
             __syncthreads();
             // children: buckets are recorded, the others wait for the next level
             if (tid < nb) {
                 const SmallNode nd = cur[b0 + tid];
-                TreeNode full, c[2];
+                TreeNode full, c0, c1;
                 full.tree = tk.tree; full.start = nd.start; full.count = nd.count; full.dstart = nd.dstart;
                 full.dcount = nd.dcount; full.depth = nd.depth; full.buf = 0; full.leaf = 0; full.key = nd.key;
-                const int nc = split_rules(full, left_s[tid], P.MIN, P.MAX, 0, c[0], c[1]);
-                if (recs) index_split(recs, n_rec, rec_cap, nd.rec, pair_s[tid][0], pair_s[tid][1], nc, c[0].rec, c[1].rec, ctr);
-                for (int q = 0; q < nc; ++q) {
-                    if (c[q].leaf || c[q].depth >= P.MAX_DEPTH - 1) {
-                        record_leaf(c[q].start, c[q].count, c[q].depth, c[q].rec);
-                    } else {
-                        // a node that keeps all its points again
-                        const int vain = nc == 1 ? nd.vain + 1 : 0;
-                        const bool stuck = CHAIN && vain >= P.vain && c[q].count <= P.chain_max;
-                        const int at = atomicAdd(stuck ? &n_chain_s : &n_nxt_s, 1);
-                        if (at < node_cap) {
-                            SmallNode sn;
-                            sn.start = c[q].start; sn.count = c[q].count; sn.dstart = c[q].dstart; sn.dcount = c[q].dcount;
-                            sn.depth = c[q].depth; sn.leaf = 0; sn.key = c[q].key; sn.rec = c[q].rec; sn.vain = vain;
-                            (stuck ? chain : nxt)[at] = sn;
+                const int nc = split_rules(full, left_s[tid], P.MIN, P.MAX, 0, c0, c1);
+                if (recs) {
+                    // (index_split; one addition for the splits of the group)
+                    const uint64_t both = ballot64(nc == 2);
+                    const int lead = first_lane(both);
+                    int base = 0;
+                    if (lane == lead) base = atomicAdd(n_rec, 2 * (int)__popcll(both));
+                    base = __shfl(base, max(lead, 0), 64) + 2 * mask_prefix(both);
+                    c0.rec = c1.rec = nd.rec;
+                    if (nc == 2) {
+                        c0.rec = base;
+                        c1.rec = base + 1;
+                        if (base + 2 <= rec_cap && nd.rec < rec_cap) {
+                            TreeRec r;
+                            r.a = pair_s[tid][0]; r.b = pair_s[tid][1]; r.c0 = c0.rec; r.c1 = c1.rec;
+                            recs[nd.rec] = r;
                         } else {
                             ctr->overflow = 1;
                         }
                     }
                 }
+                auto child = [&](const TreeNode& c) {
+                    if (c.leaf || c.depth >= P.MAX_DEPTH - 1) {
+                        record_leaf(c.start, c.count, c.depth, c.rec);
+                    } else {
+                        const bool small = CHAIN && c.count <= P.chain_max;
+                        const int at = atomicAdd(small ? &n_chain_all_s : &n_nxt_s, 1);
+                        if (at < node_cap) {
+                            SmallNode sn;
+                            sn.start = c.start; sn.count = c.count; sn.dstart = c.dstart; sn.dcount = c.dcount;
+                            sn.depth = c.depth;
+                            sn.leaf = 0; sn.key = c.key; sn.rec = c.rec;
+                            if (small) {
+                                const int back = often_in_vain(c.count, P.MIN) ? 0 : 1;
+                                sn.leaf = 2 * atomicAdd(&n_chain_s[back], 1) + back;       // (its place in that part of the queue)
+                            }
+                            (small ? chain : nxt)[at] = sn;
+                        } else {
+                            ctr->overflow = 1;
+                        }
+                    }
+                };
+                child(c0);
+                if (nc == 2) child(c1);
             }
             __syncthreads();
         }
@@ -993,7 +1093,10 @@ __global__ __launch_bounds__(TB, TB == 256 ? 6 : 1) void k_tail(const float* __r
     }
     for (int i = tid; i < tk.count; i += TB) dst[tk.start + i] = seg[i];
     if (tid == 0) {
-        if (CHAIN) chain_base_s = n_chain_s ? atomicAdd(&ctr->n_chain, n_chain_s) : 0;
+        if (CHAIN) {
+            chain_base_s[0] = n_chain_s[0] ? atomicAdd(&ctr->n_chain, n_chain_s[0]) : 0;
+            chain_base_s[1] = n_chain_s[1] ? atomicAdd(&ctr->n_chain_back, n_chain_s[1]) : 0;
+        }
         TreeStats* st = stats + tk.tree;
         base_s[0] = kind_s[0] ? atomicAdd(&st->n_leaves, kind_s[0]) : 0;
         base_s[1] = kind_s[1] ? atomicAdd(&st->n_big, kind_s[1]) : 0;
@@ -1010,18 +1113,18 @@ __global__ __launch_bounds__(TB, TB == 256 ? 6 : 1) void k_tail(const float* __r
         const int count = r.y & 0xffff, rank = r.y >> 16;
         store_leaf(tk.tree, r.x, count, base_s[count > kBucketSplit ? 1 : 0] + rank, leaf_cap, leaf_start, leaf_size, ctr);
     }
-    for (int i = tid; CHAIN && i < min(n_chain_s, node_cap); i += TB) {
+    for (int i = tid; CHAIN && i < min(n_chain_all_s, node_cap); i += TB) {
         const SmallNode sn = chain[i];
         TreeNode c;
         c.tree = tk.tree; c.start = tk.start + sn.start; c.count = sn.count; c.dstart = tk.start + sn.dstart; c.dcount = sn.dcount;
         c.depth = sn.depth; c.buf = 0; c.leaf = 0; c.rec = sn.rec; c.chunk0 = 0; c.key = sn.key;
-        const int at = chain_base_s + i;
-        if (at < chain_cap) chain_all[at] = c; else ctr->overflow = 1;
+        const int back = sn.leaf & 1, at = chain_base_s[back] + (sn.leaf >> 1);
+        if (at < chain_cap) chain_all[back ? chain_cap - 1 - at : at] = c; else ctr->overflow = 1;
     }
 }
 
 // ---------------------------------------------------------------------------
-// chain phase: nodes that are split in vain again and again
+// chain phase: small nodes, finished from the distances of their points
 // ---------------------------------------------------------------------------
 // A node just above the leaf limit is split again, with a pair of its larger side, until a hyperplane leaves both sides
 // large enough: 200 times in a row for the unluckiest node of 20,000 x 32 points in 50 trees, 430 for 70,000 x 784 with
@@ -1029,48 +1132,75 @@ __global__ __launch_bounds__(TB, TB == 256 ? 6 : 1) void k_tail(const float* __r
 // kernel a link of it costs the whole of a level of a workgroup (17,000 and 51,000 cycles at these two inputs: the trips
 // to memory for the pair's rows, the points' screening rows and the undecided points' rows).  But the points stay the
 // same, and which side of the hyperplane between x1 and x2 a point x is on is whether it is nearer to x1 or to x2.  So a
-// workgroup evaluates the distances of all pairs of the node once (LDS, upper triangle, tiles of 64 x 64), and from then on
-// a link is two reads of LDS per point and a partition in registers.
+// workgroup bounds the distances of all pairs of the node once, and from then on a link is two reads of LDS per point and a
+// partition in registers.
 //
-// d1, d2: fp32 distances of x to x1, x2, each within 1.01 (D + 3) u of the true one (u = 2^-24).  The exact test compares
-// fl(n.x) with fl(b); the true n.x - b is (d2 - d1) / 2, and the two evaluations are off by at most
-// 1.01 (D/32 + 8) u ||n|| (||x|| + (||x1|| + ||x2||) / 2) together (chains of D/32 terms, five steps of the butterfly,
-// the roundings of n, x1 + x2 and their product; Cauchy-Schwarz), ||n|| = sqrt(d(x1, x2)).  So the sign of d2 - d1 decides
-// when |d2 - d1| > 2.1 (D/32 + 8) u ||n|| (..) + 1.1 (D + 4) u (d1 + d2); otherwise (hardly ever, also for NaN) the point
-// gets the exact test.  ||x|| is bounded by sqrt(D) max |x_d| from the header of the 8-bit row.  In a node with a norm of 2e19 or
-// more, or a distance of 2e37 or more, sums of the exact test (of up to the norm times the root of the distance) may overflow,
-// and all points get it.
+// The distances come from the matrix cores: rows less the row of the node's first point, split into two bfloat16 numbers each
+// (mfma_split.hpp), 32 dimensions at a time; the sums of 32 dimensions are added up outside the matrix cores, so that their error
+// does not grow with the dimension.  They are kept as 16-bit whole numbers of one unit for the node (65534: the largest), which leaves
+// LDS for four nodes of 128 points per compute unit (two as floats).
+//
+// When a link may decide: the exact test compares fl(n.x) with fl(b), the true n.x - b is (d2 - d1) / 2, and the two evaluations
+// are off by at most 1.01 (D/32 + 8) u ||n|| (||x|| + (||x1|| + ||x2||) / 2) together, u = 2^-24 (chains of D/32 terms, five steps
+// of the butterfly, the roundings of n, x1 + x2 and their product; Cauchy-Schwarz), ||n|| = sqrt(d(x1, x2)).  A distance of
+// the matrix is off by at most c S (mfma_split.hpp, S = sum of the squared norms less the first point, plus the rounding of that
+// subtraction) and half a unit.  With the largest norms and the largest distance of the node in the place of those of the three
+// points this is one number for the node: a point's side is certain when |d2 - d1| exceeds it (70,000 x 784: 10 units, 20,000 x 32: 3).
+// The others (a point in some thousands) get the exact test.  Rows that are not finite or far longer than the others (32 times
+// the typical squared norm) have the mark kUnknown in the place of their distances, and get the exact test as well: one
+// such row must not take the resolution from the others.
 //
 // Where x1 and x2 have the same coordinates the normal is zero and the exact test puts every point on the left (0 < 0, or a
 // comparison with NaN).  Every point is as near to one as to the other, so that d1 and d2 decide nothing, and more than MAX
-// equal rows are split until the depth limit; so such pairs are marked in the matrix, with a distance of -0 (no sum of
-// squares is), and cost a link no test at all.  (20,000 x 32, buckets of 17..34, a tenth of the points in groups of 60
-// equal rows, 10 trees: 137 ms with an exact test of every point, 34 without; the tail kernel, with its own, took 62.)
+// equal rows are split until the depth limit; so nodes with a pair that may be equal have their rows compared, and the number of
+// the first equal row is kept for each.  (20,000 x 32, buckets of 17..34, a tenth of the points in groups of 60
+// equal rows, 10 trees: 137 ms with an exact test of every point, 34 without.)
 __device__ __forceinline__ int tri_at(int i, int j, int n)
 {
     const int lo = min(i, j), hi = max(i, j);
     return lo * n - ((lo * (lo + 1)) >> 1) + hi - lo - 1;
 }
 
-constexpr int kChainPitch = 36;          // floats per staged row of 32 dimensions: odd number of 16-byte units
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
-// The distances of a node of up to kChainSquare points are kept as a square matrix (odd pitch; a point's distances to x1 are
-// a row of it), of a larger one as its upper triangle.
-constexpr int kChainSquare = 120;
-__host__ __device__ inline size_t chain_matrix_floats(int n)
+constexpr int kUnknown = 0xffff;         // no distance: the point gets the exact test
+constexpr int kChainStep = 32;           // dimensions staged at a time
+constexpr int kChainPitch = kChainStep + 8;      // 16-bit numbers per staged row: an odd number of 16-byte units
+
+// The distances of a node of up to kChainSquare points are kept as a square matrix (a point's distances to x1 are a row of it; the
+// pitch lets 32 lanes write 8 bytes each down a column without conflicts), of a larger one as its upper triangle.
+constexpr int kChainSquare = 128;
+__host__ __device__ inline size_t chain_matrix_entries(int n)
 {
-    return n <= kChainSquare ? (((size_t)n * (size_t)(n | 1)) + 3) / 4 * 4 : ((size_t)n * (n - 1) / 2 + 3) / 4 * 4;
+    return n <= kChainSquare ? (size_t)((n + 31) & ~31) * (size_t)(((n + 31) & ~31) + 4) : (size_t)n * (n - 1) / 2;
 }
-// bytes of LDS: staged rows (later the normal) | distances | norms, ids, order, second buffer | offset .. | stack | buckets
-__host__ __device__ inline size_t chain_stage_floats(int n, int D)
+__host__ __device__ inline size_t chain_up16(size_t bytes) { return (bytes + 15) & ~(size_t)15; }
+// bytes of LDS: staged rows, later the distances | norms | ids (two nodes) | undecided points | stack | buckets (two nodes) | order,
+// sides, equal rows | records of the index (two nodes)
+__host__ __device__ inline size_t chain_region_bytes(int n)
 {
-    const size_t rows = (size_t)((n + 15) & ~15) * kChainPitch, normal = (size_t)nvec_len(D);
-    return rows > normal ? rows : normal;
+    const size_t rows = (size_t)((n + 31) & ~31) * kChainPitch * 4, matrix = chain_up16(chain_matrix_entries(n) * 2);
+    return rows > matrix ? rows : matrix;
 }
-__host__ __device__ inline size_t chain_lds_bytes(int n, int D, int node_cap)
+// A record of the index of a tree that is written once the places of the node's records are known: of the node itself (at = -1) or the
+// at-th of them; so are the children of a split, c0 and c0 + 1.  A bucket has c0 = -1.
+struct ChainRec {
+    int at, a, b, c0;
+};
+__host__ __device__ inline size_t chain_lds_bytes(int n, int node_cap, bool index)
 {
-    return chain_stage_floats(n, D) * 4 + chain_matrix_floats(n) * 4 + (size_t)n * 16 + 16 +
-           (size_t)node_cap * (sizeof(SmallNode) + 8);
+    return chain_region_bytes(n) + (size_t)((n + 31) & ~31) * 16 + chain_up16((size_t)node_cap * (sizeof(SmallNode) + 16)) +
+           3 * chain_up16((size_t)n) + (index ? (size_t)node_cap * 4 * sizeof(ChainRec) : 0);
+}
+
+// What a distance of the matrix may be off by over S = |a|^2 + |b|^2 (rows less the first one): 3 * 2^-20 S for the products that are
+// dropped and what two halves leave of a number (split2_half); 32 exact products in a row, every addition within 2^-23 of the sum of
+// absolute values whatever the order or rounding mode (the sums of the other products are 2^-9 of those); in units of 2^-24 S the
+// additions of the steps, the squared norms (chains of D/8 terms), four times the rounding of the subtraction of the first row, and
+// the final expression.
+inline float chain_gram_error(int D)
+{
+    return 3.2f / 1048576.0f + (float)(kChainStep + 2) / 8388608.0f + (float)(D / 8 + D / 16 + 24) / 16777216.0f;
 }
 
 // The draws of the next levels of a chain.  The key of a child follows from the key of its parent and the side alone, so
@@ -1103,185 +1233,454 @@ struct ChainDraws {
         if (h >= 16) start(child_key(node_key(), s));
         else h = 2 * h + s;
     }
-    // pick_pair of the present node
-    __device__ __forceinline__ void pair(int count, int& r1, int& r2) const
+    // pick_pair of the present node.  inverse: floor((2^32 - 1) / count); the quotient it gives is at most two too small
+    __device__ __forceinline__ void pair(int count, uint32_t inverse, int& r1, int& r2) const
     {
-        const uint32_t r = draw % (uint32_t)count;
+        uint32_t r = draw - __umulhi(draw, inverse) * (uint32_t)count;
+        r = min(r, r - (uint32_t)count);
+        r = min(r, r - (uint32_t)count);
         r1 = read_lane_i((int)r, 2 * h);
         r2 = read_lane_i((int)r, 2 * h + 1);
         if (r1 == r2) pick_pair(node_key(), count, r1, r2);
     }
 };
 
-// NB: blocks of 16 points a node may have (8: distances as a square matrix).
-template <int NB>
-__global__ __launch_bounds__(256) void k_chain(const float* __restrict__ points, const uint8_t* __restrict__ q8, TreeParams P,
+// The exact test (resolve_exact) of n points of a chain against the hyperplane of the points i1 and i2, by one wavefront: the
+// hyperplane is made again beside the products (make_hyperplane_wave: the same order), so that the rows of the pair and of the points
+// are one trip to memory.
+template <typename IdAt, typename Apply>
+__device__ __forceinline__ void chain_exact(const float* __restrict__ points, int D, int i1, int i2, const int* list, int n, IdAt id_at, Apply apply)
+{
+    const int hl = lane_id() & 31, h = lane_id() >> 5;
+    const float* x1 = points + (size_t)i1 * (size_t)D;
+    const float* x2 = points + (size_t)i2 * (size_t)D;
+    for (int base = 0; base < n; base += 4) {
+        const int ia = base + h, ib = base + 2 + h;
+        const bool va = ia < n, vb = ib < n;
+        const int ea = list[va ? ia : 0], eb = list[vb ? ib : 0];
+        const float* xa = points + (size_t)id_at(ea) * (size_t)D;
+        const float* xb = points + (size_t)id_at(eb) * (size_t)D;
+        float s = 0.0f, sa = 0.0f, sb = 0.0f;
+        for (int d0 = hl; d0 < D; d0 += 256) {
+            float t1[8], t2[8], xv[8], yv[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const int d = d0 + 32 * k;
+                t1[k] = d < D ? x1[d] : 0.0f;
+                t2[k] = d < D ? x2[d] : 0.0f;
+                xv[k] = va && d < D ? xa[d] : 0.0f;
+                yv[k] = vb && d < D ? xb[d] : 0.0f;
+            }
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                if (d0 + 32 * k < D) {
+                    const float nd = t1[k] - t2[k];
+                    const float prod = nd * (t1[k] + t2[k]);
+                    s = s + prod * 0.5f;
+                    sa = __builtin_fmaf(nd, xv[k], sa);
+                    sb = __builtin_fmaf(nd, yv[k], sb);
+                }
+            }
+        }
+        s = half_butterfly_sum(s);
+        sa = half_butterfly_sum(sa);
+        sb = half_butterfly_sum(sb);
+        if (hl == 0) {
+            if (va) apply(ea, sa < s);
+            if (vb) apply(eb, sb < s);
+        }
+    }
+}
+
+// NT: tiles of 32 points a node may have (up to 4: distances as a square matrix).  WAVES: wavefronts that make the matrix; the
+// chain is the first one's, and meanwhile the others fetch the next node's ids.
+template <int NT, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, NT >= 4 ? 2 : 3) void k_chain(const float* __restrict__ points, const uint8_t* __restrict__ q8,
+                                               TreeParams P, float gram_error,
                                                int* __restrict__ perm_out, const TreeNode* __restrict__ tasks, int task_cap,
                                                int node_cap, int leaf_cap, int* __restrict__ leaf_start,
                                                int* __restrict__ leaf_size, TreeStats* stats, LevelCounters* ctr,
-                                               TreeRec* __restrict__ recs_all, int* __restrict__ n_rec_all, int rec_cap,
+                                               TreeRec* __restrict__ recs_all, int rec_cap,
                                                unsigned long long* __restrict__ stat)
 {
     extern __shared__ __align__(16) unsigned char chain_lds[];
-    const int nmax = P.chain_max;
-    float* stage = reinterpret_cast<float*>(chain_lds);
-    float* nvec = stage;                                                      // once the distances are there
-    float* tri = stage + chain_stage_floats(nmax, P.D);
-    float* norm = tri + chain_matrix_floats(nmax);
-    int* ids = reinterpret_cast<int*>(norm + nmax);
-    int* ord = ids + nmax;                                                    // position in the node -> place in ids
-    int* tmp = ord + nmax;
-    float* hp = reinterpret_cast<float*>(tmp + nmax);
-    SmallNode* stack = reinterpret_cast<SmallNode*>(hp + 4);
-    int2* lrec = reinterpret_cast<int2*>(stack + node_cap);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    __shared__ int zero_s, huge_s;                                            // two points are at distance 0; a norm or distance is out of range
-    const int n_tasks = min(ctr->n_chain, task_cap);
+    constexpr bool kSquare = 32 * NT <= kChainSquare;
+    constexpr int kThreads = 64 * WAVES, kPitch = 32 * NT + 4;
+    const int nmax = P.chain_max, npad = (nmax + 31) & ~31;
+    uint16_t* stage_hi = reinterpret_cast<uint16_t*>(chain_lds);
+    uint16_t* stage_lo = stage_hi + npad * kChainPitch;
+    uint16_t* mat = stage_hi;                                                 // once the products are there
+    float* norm = reinterpret_cast<float*>(chain_lds + chain_region_bytes(nmax));
+    int* ids_all = reinterpret_cast<int*>(norm + npad);                       // of this node and of the next one
+    int* tmp = ids_all + 2 * npad;
+    SmallNode* stack = reinterpret_cast<SmallNode*>(tmp + npad);
+    int2* lrec_all = reinterpret_cast<int2*>(stack + node_cap);               // buckets of this node and of the one before
+    unsigned char* ord = reinterpret_cast<unsigned char*>(stack) + chain_up16((size_t)node_cap * (sizeof(SmallNode) + 16));      // position in the node -> place in ids
+    unsigned char* mark = ord + chain_up16((size_t)nmax);                     // by position: the exact test said right
+    unsigned char* same = mark + chain_up16((size_t)nmax);                    // by place: first place with the same coordinates
+    ChainRec* crec_all = reinterpret_cast<ChainRec*>(same + chain_up16((size_t)nmax));
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    __shared__ float most_s[WAVES], least_s[WAVES];
+    __shared__ TreeNode task_s[2];
+    // The queue: first the nodes that may take long (the launch lasts as long as its longest chain), then the others, in kRegions
+    // regions taken in turn, so that the nodes under way belong to different trees and add to different counters.
+    constexpr int kRegions = 64;
+    const int n_front = ctr->n_chain, n_back = ctr->n_chain_back, region = (n_back + kRegions - 1) / kRegions;
+    const int n_tasks = n_front + region * kRegions;
     const bool vec_ok = (P.D & 3) == 0 && ((reinterpret_cast<uintptr_t>(points) & 15) == 0);
     const float u24 = 1.0f / 16777216.0f;
-    const float tol_n = 2.1f * (float)(P.D / 32 + 8) * u24, tol_d = 1.1f * (float)(P.D + 4) * u24;
     int seen = 0, unsure = 0;
-
-    for (int task = blockIdx.x; task < n_tasks; task += gridDim.x) {
-        const TreeNode tk = tasks[task];
-        const int n = tk.count;
-        int* seg = perm_out + (size_t)tk.tree * (size_t)P.N + tk.start;
-        __syncthreads();                                                      // the previous task is done with the LDS
-        if (tid == 0) { zero_s = 0; huge_s = 0; }
-        if (tid < n) {
-            const int id = seg[tid];
-            ids[tid] = id;
-            ord[tid] = tid;
-            if (q8) {
-                const float4 head = *reinterpret_cast<const float4*>(q8 + (size_t)id * (size_t)q8_pitch(P.D));
-                norm[tid] = 1.01f * __builtin_sqrtf((float)P.D) * fmaxf(fabsf(head.y), fabsf(head.y + 255.0f * head.z)) + 0.0f * head.w;
-            }
-        }
-        __syncthreads();
-        if (!q8) {
-            for (int i = wave; i < n; i += 4) {
-                const float* x = points + (size_t)ids[i] * (size_t)P.D;
-                float s = 0.0f;
-                for (int d = lane; d < P.D; d += 64) s = __builtin_fmaf(x[d], x[d], s);
-                s += dpp_f<kDppXor1>(s); s += dpp_f<kDppXor2>(s); s += dpp_f<kDppHalfMirror>(s); s += dpp_f<kDppMirror>(s);
-                s = read_lane_f(s, 0) + read_lane_f(s, 16) + read_lane_f(s, 32) + read_lane_f(s, 48);
-                if (lane == 0) norm[i] = 1.01f * __builtin_sqrtf(s);
-            }
-        }
-        // distances: thread (ty, tx) has the pairs (ty + 16 r, tx + 16 c), c >= r, of all blocks; 32 dimensions of all rows at
-        // a time through LDS, the next 32 under way meanwhile
-        {
-            const int nb = (n + 15) >> 4, ty = tid >> 4, tx = tid & 15;
-            constexpr int kLoads = NB / 2;                                    // 16-byte pieces of a step per thread
-            float acc[NB * (NB + 1) / 2];
+    constexpr int kV = (NT + 1) / 2;                                          // points per lane
+    uint32_t inverse[kV];                                                     // lane l: of l + 1, l + 65, ..
 #pragma unroll
-            for (int k = 0; k < NB * (NB + 1) / 2; ++k) acc[k] = 0.0f;
-            float4 pre[kLoads];
+    for (int v = 0; v < kV; ++v) inverse[v] = 0xffffffffu / (uint32_t)((threadIdx.x & 63) + 1 + 64 * v);
+    // buckets and records of the node before that have not been stored yet: their places are being reserved
+    int pend_n = 0, pend_recs = 0, pend_tree = 0, pend_rec = 0, pend_base[3] = {0, 0, 0};
+    auto store_pending = [&](int which, int lane) {
+        const int2* lrec = lrec_all + which * node_cap;
+        const int b0 = __builtin_amdgcn_readfirstlane(pend_base[0]), b1 = __builtin_amdgcn_readfirstlane(pend_base[1]);
+        for (int i = lane; i < min(pend_n, node_cap); i += 64) {
+            const int2 r = lrec[i];
+            const int m = r.y & 0xffff, rank = r.y >> 16;
+            store_leaf(pend_tree, r.x, m, (m > kBucketSplit ? b1 : b0) + rank, leaf_cap, leaf_start, leaf_size, ctr);
+        }
+        if (recs_all) {
+            const ChainRec* crec = crec_all + which * 2 * node_cap;
+            const int base = __builtin_amdgcn_readfirstlane(pend_base[2]);
+            for (int i = lane; i < min(pend_recs, 2 * node_cap); i += 64) {
+                const ChainRec c = crec[i];
+                const int at = c.at < 0 ? pend_rec : base + c.at;
+                TreeRec r;
+                r.a = c.a; r.b = c.b;
+                r.c0 = c.c0 < 0 ? -1 : base + c.c0;
+                r.c1 = c.c0 < 0 ? -1 : base + c.c0 + 1;
+                if (max(at, r.c1) < rec_cap) recs_all[(size_t)pend_tree * rec_cap + at] = r; else ctr->overflow = 1;
+            }
+        }
+        pend_n = 0;
+    };
+
+    // (the nodes before gridDim.x of a share are the first ones of its workgroups)
+    auto take_next = [&]() {
+        constexpr int S = LevelCounters::kShares;
+        const int mine = (int)blockIdx.x % S;
+        return mine + S * (((int)gridDim.x - mine + S - 1) / S + atomicAdd(&ctr->share[mine].taken, 1));
+    };
+    int turn = 0, next = blockIdx.x;                                          // (next: in the fetching wavefront)
+    constexpr int kFetcher = WAVES > 1 ? 1 : 0;
+    while (true) {
+        // (what follows from the thread's number is worked out for each node: kept across the chain it costs registers)
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));
+        const int lane = tid & 63;
+        int* ids = ids_all + turn * npad;
+        int2* lrec = lrec_all + turn * node_cap;
+        if (wave == kFetcher) {
+            int task = __builtin_amdgcn_readfirstlane(next), place = task;
+            while (task >= n_front && task < n_tasks) {
+                const int i = (task - n_front) % kRegions * region + (task - n_front) / kRegions;
+                place = task_cap - 1 - i;
+                if (i < n_back) break;
+                int again = 0;
+                if (lane == 0) again = take_next();                           // (the last region has no such node)
+                task = place = __builtin_amdgcn_readfirstlane(again);
+            }
+            if (task < n_tasks) {
+                const TreeNode t = tasks[place];
+                const int* from = perm_out + (size_t)t.tree * (size_t)P.N + t.start;
+                for (int i = lane; i < t.count; i += 64) ids[i] = from[i];
+                if (lane == 0) task_s[turn] = t;
+            } else if (lane == 0) {
+                task_s[turn].tree = -1;
+            }
+        }
+        __syncthreads();                                                      // (and the node before is done with the LDS)
+        // (everything about the node in scalar registers: the chain's state is the wavefront's, not its lanes')
+        TreeNode tk = task_s[turn];
+        tk.tree = uniform(tk.tree);
+        if (tk.tree < 0) break;
+        tk.start = uniform(tk.start); tk.dstart = uniform(tk.dstart); tk.dcount = uniform(tk.dcount); tk.depth = uniform(tk.depth);
+        tk.rec = uniform(tk.rec);
+        tk.key = (uint64_t)(uint32_t)uniform((int)(uint32_t)tk.key) | ((uint64_t)(uint32_t)uniform((int)(uint32_t)(tk.key >> 32)) << 32);
+        const int n = uniform(tk.count), nt = (n + 31) >> 5;
+        int* seg = perm_out + (size_t)tk.tree * (size_t)P.N + tk.start;
+        // accumulator e of lane l in tile (ti, tj): pair (32 ti + 8 (e / 4) + e % 4 + 4 (l / 32), 32 tj + l % 32); the tiles of the
+        // upper triangle, column by column, are dealt out to the wavefronts
+        constexpr int kTiles = (NT * (NT + 1) / 2 + WAVES - 1) / WAVES;
+        f32x16 acc[kTiles];
+        int tile_i[kTiles], tile_j[kTiles];
+#pragma unroll
+        for (int t = 0; t < kTiles; ++t) {
+            int k = wave + WAVES * t, tj = 0;
+            while (k > tj) { k -= tj + 1; ++tj; }
+            tile_i[t] = k;
+            tile_j[t] = tj;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[t][e] = 0.0f;
+        }
+        float first_norm = 0.0f;                                              // squared norm of the row that is taken off the others
+        float unit;                                                           // rows are multiplied by this power of two
+        {
+            constexpr int kRows = kThreads / 8, kLoads = 32 * NT / kRows;     // rows per pass; eight threads have 32 dimensions of a row
+            float4 pre[kLoads], base;
+            float nrm[kLoads];
+#pragma unroll
+            for (int i = 0; i < kLoads; ++i) nrm[i] = 0.0f;
             auto request = [&](int d0) {
+                const int d = d0 + 4 * (tid & 7);
+                base = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (d < P.D) base = load_dims(points + (size_t)ids[0] * (size_t)P.D + d, P.D - d, vec_ok);
 #pragma unroll
                 for (int i = 0; i < kLoads; ++i) {
-                    const int row = (tid >> 3) + 32 * i, d = d0 + 4 * (tid & 7);
-                    pre[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-                    if (row < n && d < P.D) {
-                        const float* src = points + (size_t)ids[row] * (size_t)P.D + d;
-                        pre[i] = load_dims(src, P.D - d, vec_ok);
-                    }
+                    const int row = (tid >> 3) + kRows * i;
+                    pre[i] = base;
+                    if (row < n && d < P.D) pre[i] = load_dims(points + (size_t)ids[row] * (size_t)P.D + d, P.D - d, vec_ok);
                 }
             };
             request(0);
-            for (int d0 = 0; d0 < P.D; d0 += 32) {
+            // the largest coordinate of the node's finite rows: from the headers of the 8-bit rows, else from the rows themselves
+            float top = 0.0f;
+            if (q8) {
+                for (int i = tid; i < n; i += kThreads) {
+                    const float4 head = *reinterpret_cast<const float4*>(q8 + (size_t)ids[i] * (size_t)q8_pitch(P.D));
+                    const float m = fmaxf(fabsf(head.y), fabsf(head.y + 255.0f * head.z)) * 1.01f;
+                    if (head.w < INFINITY && m < 1e37f) top = fmaxf(top, m);
+                }
+            } else {
+                for (int i = tid >> 3; i < n; i += kRows) {
+                    const float* x = points + (size_t)ids[i] * (size_t)P.D;
+                    for (int d = tid & 7; d < P.D; d += 8)
+                        if (fabsf(x[d]) < 1e37f) top = fmaxf(top, fabsf(x[d]));
+                }
+            }
+            top = wave_max(top);
+            if (WAVES > 1) {
+                if (lane == 0) most_s[wave] = top;
+                __syncthreads();
+#pragma unroll
+                for (int w = 0; w < WAVES; ++w) top = fmaxf(top, most_s[w]);
+            }
+            // differences stay below 2^15
+            {
+                const int e = (int)(__float_as_uint(top) >> 23);              // top < 2^(e - 126)
+                unit = __uint_as_float((uint32_t)min(max(127 + 14 + 126 - e, 1), 254) << 23);
+                if (!(top > 0.0f)) unit = 1.0f;
+            }
+            for (int d0 = 0; d0 < P.D; d0 += kChainStep) {
+                base.x *= unit; base.y *= unit; base.z *= unit; base.w *= unit;
+                first_norm = __builtin_fmaf(base.x, base.x, first_norm); first_norm = __builtin_fmaf(base.y, base.y, first_norm);
+                first_norm = __builtin_fmaf(base.z, base.z, first_norm); first_norm = __builtin_fmaf(base.w, base.w, first_norm);
 #pragma unroll
                 for (int i = 0; i < kLoads; ++i) {
-                    const int row = (tid >> 3) + 32 * i;
-                    if (row < nb * 16) *reinterpret_cast<float4*>(&stage[row * kChainPitch + 4 * (tid & 7)]) = pre[i];
+                    const int row = (tid >> 3) + kRows * i;
+                    if (row < 32 * nt) {
+                        // (the products with a power of two are exact)
+                        const float x = __builtin_fmaf(pre[i].x, unit, -base.x), y = __builtin_fmaf(pre[i].y, unit, -base.y);
+                        const float z = __builtin_fmaf(pre[i].z, unit, -base.z), w = __builtin_fmaf(pre[i].w, unit, -base.w);
+                        uint2 h, l;
+                        split2_half(x, y, h.x, l.x);
+                        split2_half(z, w, h.y, l.y);
+                        *reinterpret_cast<uint2*>(&stage_hi[row * kChainPitch + 4 * (tid & 7)]) = h;
+                        *reinterpret_cast<uint2*>(&stage_lo[row * kChainPitch + 4 * (tid & 7)]) = l;
+                        nrm[i] = __builtin_fmaf(x, x, nrm[i]); nrm[i] = __builtin_fmaf(y, y, nrm[i]);
+                        nrm[i] = __builtin_fmaf(z, z, nrm[i]); nrm[i] = __builtin_fmaf(w, w, nrm[i]);
+                    }
                 }
                 __syncthreads();
-                if (d0 + 32 < P.D) request(d0 + 32);
-                const int nd = min(32, (P.D - d0 + 3) & ~3);
-                for (int dd = 0; dd < nd; dd += 4) {
-                    float4 av[NB];
+                if (d0 + kChainStep < P.D) request(d0 + kChainStep);
 #pragma unroll
-                    for (int r = 0; r < NB; ++r)
-                        if (r < nb) av[r] = *reinterpret_cast<const float4*>(&stage[(ty + 16 * r) * kChainPitch + dd]);
+                for (int t = 0; t < kTiles; ++t) {
+                    if (tile_j[t] >= nt) continue;
+                    __builtin_amdgcn_sched_barrier(0);
+                    const int ra = (32 * tile_i[t] + (lane & 31)) * kChainPitch + 8 * (lane >> 5);
+                    const int rb = (32 * tile_j[t] + (lane & 31)) * kChainPitch + 8 * (lane >> 5);
+                    f32x16 sum;
 #pragma unroll
-                    for (int c = 0; c < NB; ++c) {
-                        if (c >= nb) continue;
-                        const float4 bv = *reinterpret_cast<const float4*>(&stage[(tx + 16 * c) * kChainPitch + dd]);
+                    for (int e = 0; e < 16; ++e) sum[e] = 0.0f;
 #pragma unroll
-                        for (int r = 0; r <= c; ++r) {
-                            float& s = acc[c * (c + 1) / 2 + r];
-                            float df;
-                            df = av[r].x - bv.x; s = __builtin_fmaf(df, df, s);
-                            df = av[r].y - bv.y; s = __builtin_fmaf(df, df, s);
-                            df = av[r].z - bv.z; s = __builtin_fmaf(df, df, s);
-                            df = av[r].w - bv.w; s = __builtin_fmaf(df, df, s);
-                        }
+                    for (int k = 0; k < kChainStep; k += 16) {
+                        const f16x8 ah = *reinterpret_cast<const f16x8*>(&stage_hi[ra + k]), bl = *reinterpret_cast<const f16x8*>(&stage_lo[rb + k]);
+                        const f16x8 al = *reinterpret_cast<const f16x8*>(&stage_lo[ra + k]), bh = *reinterpret_cast<const f16x8*>(&stage_hi[rb + k]);
+                        sum = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bl, sum, 0, 0, 0);
+                        sum = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, bh, sum, 0, 0, 0);
+                        __builtin_amdgcn_sched_barrier(0);
                     }
+                    acc[t] += sum;
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) sum[e] = 0.0f;
+#pragma unroll
+                    for (int k = 0; k < kChainStep; k += 16) {
+                        const f16x8 ah = *reinterpret_cast<const f16x8*>(&stage_hi[ra + k]), bh = *reinterpret_cast<const f16x8*>(&stage_hi[rb + k]);
+                        sum = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bh, sum, 0, 0, 0);
+                    }
+                    acc[t] += sum;
                 }
                 __syncthreads();
             }
-            float least = INFINITY, most = 0.0f;                              // of the distances between two points of the node
+            // the eight threads of a row add up their squares
 #pragma unroll
-            for (int c = 0; c < NB; ++c)
-#pragma unroll
-                for (int r = 0; r <= c; ++r) {
-                    const int i = ty + 16 * r, j = tx + 16 * c;
-                    if (c < nb && i <= j && j < n) {
-                        least = fminf(least, i < j ? acc[c * (c + 1) / 2 + r] : INFINITY);
-                        most = fmaxf(most, acc[c * (c + 1) / 2 + r]);
-                        if constexpr (NB == 8) {
-                            tri[i * (n | 1) + j] = acc[c * (c + 1) / 2 + r];
-                            tri[j * (n | 1) + i] = acc[c * (c + 1) / 2 + r];
-                        } else if (i < j) {
-                            tri[tri_at(i, j, n)] = acc[c * (c + 1) / 2 + r];
-                        }
-                    }
-                }
-            if (least == 0.0f) zero_s = 1;
-            if (!(most < 2e37f)) huge_s = 1;
+            for (int i = 0; i < kLoads; ++i) {
+                float s = nrm[i];
+                s += dpp_f<kDppXor1>(s); s += dpp_f<kDppXor2>(s); s += dpp_f<kDppHalfMirror>(s);
+                const int row = (tid >> 3) + kRows * i;
+                if ((tid & 7) == 0 && row < 32 * nt) norm[row] = row < n && s < 1e37f ? s : INFINITY;
+            }
+            first_norm += dpp_f<kDppXor1>(first_norm); first_norm += dpp_f<kDppXor2>(first_norm); first_norm += dpp_f<kDppHalfMirror>(first_norm);
         }
-        if (tid < n && !(norm[tid] < 2e19f)) huge_s = 1;
         __syncthreads();
-        if (zero_s) {
-            // tmp[j]: the first point at distance 0 from j, if it has the coordinates of j (eight lanes compare), else j
-            auto at = [&](int i, int j) { return NB == 8 ? i * (n | 1) + j : tri_at(i, j, n); };
-            for (int j = tid >> 3; j < n; j += 32) {
-                int first = j;
-                for (int i = (tid & 7); i < j && first == j; i += 8)
-                    if (tri[at(i, j)] == 0.0f) first = i;
+        // typical squared norm: the mean of the exponents (every wavefront for itself)
+        float norm_most = 0.0f;
+        bool wild;                                                            // there is a row without distances
+        {
+            int ex = 0, some = 0;
+            float s[kV];
 #pragma unroll
-                for (int o = 1; o < 8; o <<= 1) first = min(first, __shfl_xor(first, o, 64));
-                const float* xi = points + (size_t)ids[first] * (size_t)P.D;
-                const float* xj = points + (size_t)ids[j] * (size_t)P.D;
-                int differ = 0;
-                for (int d = tid & 7; d < P.D && !differ; d += 8) differ = xi[d] == xj[d] ? 0 : 1;
-#pragma unroll
-                for (int o = 1; o < 8; o <<= 1) differ |= __shfl_xor(differ, o, 64);
-                if ((tid & 7) == 0) tmp[j] = differ ? j : first;
+            for (int v = 0; v < kV; ++v) {
+                s[v] = lane + 64 * v < n ? norm[lane + 64 * v] : 0.0f;
+                const bool counts = s[v] > 0.0f && s[v] < INFINITY;
+                ex += counts ? (int)(__float_as_uint(s[v]) >> 23) : 0;
+                some += __popcll(ballot64(counts));
             }
+            ex = wave_sum_i(ex);
+            const float norm_limit = fminf(__uint_as_float((uint32_t)min((some ? ex / some : 0) + 6, 250) << 23), 1e37f);
+            bool far = false;
+#pragma unroll
+            for (int v = 0; v < kV; ++v) {
+                if (s[v] <= norm_limit) norm_most = fmaxf(norm_most, s[v]);
+                else far = true;
+            }
+            norm_most = wave_max(norm_most);
+            wild = ballot64(far) != 0;                                        // (all wavefronts have read the same)
+            // rows without distances get an infinite norm, rows beyond the node (zeros) one that makes their distances ordinary ones;
+            // every wavefront writes the same
             __syncthreads();
-            for (int e = tid; e < n * n; e += 256) {
-                const int i = e / n, j = e - i * n;
-                if (i < j && tmp[i] == tmp[j]) {
-                    tri[at(i, j)] = -0.0f;
-                    if constexpr (NB == 8) tri[at(j, i)] = -0.0f;
+#pragma unroll
+            for (int v = 0; v < kV; ++v) {
+                if (s[v] > norm_limit) norm[lane + 64 * v] = INFINITY;
+                if (lane + 64 * v >= n && lane + 64 * v < 32 * nt) norm[lane + 64 * v] = norm_most;
+            }
+            wave_lds_sync();
+        }
+        // the products become distances (infinite, or NaN, where one of the norms is)
+        const float cap = 4.1f * norm_most;                                   // above the distances that are known
+        float most = 0.0f, least = INFINITY;
+#pragma unroll
+        for (int t = 0; t < kTiles; ++t) {
+            if (tile_j[t] >= nt) continue;
+            __builtin_amdgcn_sched_barrier(0);                                // (the norms of one tile at a time: registers)
+            const float nj = norm[32 * tile_j[t] + (lane & 31)];
+            const int own = (lane & 31) - 4 * (lane >> 5);                    // (a row's distance to itself, in a tile on the diagonal)
+            const bool diagonal = tile_i[t] == tile_j[t];
+#pragma unroll
+            for (int e4 = 0; e4 < 4; ++e4) {
+                const float4 n4 = *reinterpret_cast<const float4*>(&norm[32 * tile_i[t] + 8 * e4 + 4 * (lane >> 5)]);
+                const float ni[4] = {n4.x, n4.y, n4.z, n4.w};
+#pragma unroll
+                for (int x = 0; x < 4; ++x) {
+                    const float d = __builtin_fmaf(-2.0f, acc[t][4 * e4 + x], ni[x] + nj);
+                    acc[t][4 * e4 + x] = d;
+                    most = fmaxf(most, fminf(d, cap));
+                    if (!diagonal || own != 8 * e4 + x) least = fminf(least, d);
                 }
+            }
+        }
+        most = wave_max(most);
+        least = -wave_max(-least);
+        if (lane == 0) { most_s[wave] = most; least_s[wave] = least; }
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) { most = fmaxf(most, most_s[w]); least = fminf(least, least_s[w]); }
+        // what a distance may be off by: of all terms, in units of the norms, and what rows lose below the least 16-bit number
+        const float off_d = gram_error * 2.0f * norm_most + 4.5f / 16384.0f * __builtin_sqrtf((float)P.D * norm_most) + (float)P.D * 4e-9f;
+        // (nothing is certain where all distances are tiny, or a sum of the exact test could leave the range of fp32)
+        const float longest = __builtin_sqrtf(norm_most) + __builtin_sqrtf(first_norm), back = 1.0f / unit;
+        const bool usable = most * back * back > 1e-28f && most * back * back < 2e37f && longest * back < 2e19f;
+        const float scale = usable ? 65534.0f / most : 0.0f;
+        const float off = 2.0f * off_d + 4.3f * (float)(P.D / 32 + 8) * u24 * __builtin_sqrtf(most + off_d) * longest + 1e-30f * unit * unit;
+        const float off_units = off * scale + 1.04f;                          // (a distance is rounded to within half a unit)
+        const int limit = uniform(usable && off_units < 60000.0f ? (int)off_units : 1 << 20);
+        auto entry = [&](int i, int j) { return kSquare ? i * kPitch + j : tri_at(i, j, n); };
+#pragma unroll
+        for (int t = 0; t < kTiles; ++t) {
+            if (tile_j[t] >= nt) continue;
+            __builtin_amdgcn_sched_barrier(0);
+            const int j = 32 * tile_j[t] + (lane & 31), i0 = 32 * tile_i[t] + 4 * (lane >> 5);
+#pragma unroll
+            for (int e4 = 0; e4 < 4; ++e4) {
+                uint32_t v[4];
+#pragma unroll
+                for (int x = 0; x < 4; ++x)
+                    v[x] = (uint32_t)__builtin_amdgcn_fmed3f(__builtin_fmaf(acc[t][4 * e4 + x], scale, 0.5f), 0.0f, (float)kUnknown + 0.5f);
+                const int i = i0 + 8 * e4;
+                if constexpr (kSquare) {
+                    // (both triangles of a tile on the diagonal: they differ by less than the error)
+                    *reinterpret_cast<uint2*>(&mat[j * kPitch + i]) = make_uint2(v[0] | (v[1] << 16), v[2] | (v[3] << 16));
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) mat[(i + x) * kPitch + j] = (uint16_t)v[x];
+                } else {
+#pragma unroll
+                    for (int x = 0; x < 4; ++x)
+                        if (i + x < j && j < n) mat[tri_at(i + x, j, n)] = (uint16_t)v[x];
+                }
+            }
+        }
+        if (wild) {
+            __syncthreads();
+            for (int i = 0; i < n; ++i) {
+                if (norm[i] < INFINITY) continue;
+                for (int j = tid; j < n; j += kThreads) {
+                    if constexpr (kSquare) { mat[i * kPitch + j] = kUnknown; mat[j * kPitch + i] = kUnknown; }
+                    else if (i != j) mat[tri_at(i, j, n)] = kUnknown;
+                }
+            }
+        }
+        __syncthreads();
+        const bool equal_rows = uniform(least <= off_d ? 1 : 0) != 0;
+        if (equal_rows) {
+            // same[j]: the first place whose row has the coordinates of row j, of up to four that are near enough (eight lanes compare)
+            const int near = (int)fminf(off_d * scale + 2.0f, 65534.0f);
+            for (int j = tid >> 3; j < n; j += kThreads / 8) {
+                int first = j;
+                for (int from = 0, tries = 0; tries < 4; ++tries) {
+                    int i = j;
+                    for (int c = from + (tid & 7); c < j && i == j; c += 8)
+                        if (mat[entry(c, j)] <= near) i = c;
+#pragma unroll
+                    for (int o = 1; o < 8; o <<= 1) i = min(i, __shfl_xor(i, o, 64));
+                    if (i == j) break;
+                    const float* xi = points + (size_t)ids[i] * (size_t)P.D;
+                    const float* xj = points + (size_t)ids[j] * (size_t)P.D;
+                    int differ = 0;
+                    for (int d = tid & 7; d < P.D && !differ; d += 8) differ = xi[d] == xj[d] ? 0 : 1;
+#pragma unroll
+                    for (int o = 1; o < 8; o <<= 1) differ |= __shfl_xor(differ, o, 64);
+                    if (!differ) { first = i; break; }
+                    from = i + 1;
+                }
+                if ((tid & 7) == 0) same[j] = (unsigned char)first;
             }
             __syncthreads();
         }
-        if (wave != 0) continue;                                              // the chain is the first wavefront's
-        TreeRec* recs = recs_all ? recs_all + (size_t)tk.tree * rec_cap : nullptr;
-        int* n_rec = recs_all ? n_rec_all + tk.tree : nullptr;
-        int start = 0, count = n, dstart = tk.dstart - tk.start, dcount = tk.dcount, depth = tk.depth, rec = tk.rec;
+        if (wave == kFetcher && lane == 0) next = take_next();
+        if (wave != 0) {                                                      // the chain is the first wavefront's
+            turn ^= 1;
+            continue;
+        }
+        if (pend_n) store_pending(turn ^ 1, lane);
+        TreeStats* st = stats + tk.tree;
+        const int levels_seen = *const_cast<volatile int*>(&st->levels), most_seen = *const_cast<volatile int*>(&st->max_leaf),
+                  least_seen = *const_cast<volatile int*>(&st->min_leaf);
+        ChainRec* crec = crec_all + turn * 2 * node_cap;
+        int start = 0, count = n, dstart = tk.dstart - tk.start, dcount = tk.dcount, depth = tk.depth;
+        int rec = -1, n_crec = 0, n_split = 0;                                // (ChainRec)
         ChainDraws draws;
         draws.start(tk.key);
-        int sp = 0, nrec = 0, n_kind[2] = {0, 0}, levels = 0, largest = 0, smallest = 0x7fffffff;
-        constexpr int kV = NB / 4;                                            // points per lane
-        auto dist_to = [&](int o, int q) -> float {
-            if constexpr (NB == 8) return tri[o * (n | 1) + q];
-            else return q == o ? 0.0f : tri[tri_at(q, o, n)];
+        int sp = 0, nrec = 0, n_big = 0, levels = 0, largest = 0, smallest = 0x7fffffff;
+        auto dist_to = [&](int o, int q) -> int {
+            if constexpr (kSquare) return mat[o * kPitch + q];
+            else return q == o ? 0 : mat[tri_at(q, o, n)];
         };
-        const float least_tol = huge_s ? INFINITY : 1e-30f;
         int q[kV];                                                            // places of the node's points, by position
         auto take_order = [&]() {
 #pragma unroll
@@ -1294,118 +1693,151 @@ __global__ __launch_bounds__(256) void k_chain(const float* __restrict__ points,
                 if ((pos >> 6) == v) o = read_lane_i(q[v], pos & 63);
             return o;
         };
-        take_order();
+#pragma unroll
+        for (int v = 0; v < kV; ++v) {
+            q[v] = min(lane + 64 * v, n - 1);
+            if (lane + 64 * v < n) ord[lane + 64 * v] = (unsigned char)(lane + 64 * v);
+        }
+        wave_lds_sync();
         while (true) {
             int r1, r2;
-            draws.pair(dcount, r1, r2);
+            uint32_t inv = (uint32_t)read_lane_i((int)inverse[0], (dcount - 1) & 63);
+#pragma unroll
+            for (int v = 1; v < kV; ++v)
+                if (((dcount - 1) >> 6) == v) inv = (uint32_t)read_lane_i((int)inverse[v], (dcount - 1) & 63);
+            draws.pair(dcount, inv, r1, r2);
             const int o1 = place_at(dstart - start + r1), o2 = place_at(dstart - start + r2);
-            const float d12 = dist_to(o1, o2);
-            const float least = __float_as_int(d12) == (int)0x80000000 ? -INFINITY : least_tol;      // (the same coordinates)
-            const float nn = tol_n * __builtin_sqrtf(d12), half12 = 0.5f * (norm[o1] + norm[o2]);
-            float d1[kV], d2[kV], nq[kV];
+            int d1[kV], d2[kV];
 #pragma unroll
             for (int v = 0; v < kV; ++v) {
                 d1[v] = dist_to(o1, q[v]);
                 d2[v] = dist_to(o2, q[v]);
-                nq[v] = norm[q[v]];
             }
-            uint64_t left[kV], again[kV];
+            uint64_t left[kV], again[kV], all[kV];
             int a = 0, n_def = 0;
 #pragma unroll
             for (int v = 0; v < kV; ++v) {
-                const bool valid = lane + 64 * v < count;
-                const float tol = nn * (nq[v] + half12) + tol_d * (d1[v] + d2[v]) + least;
-                const bool certain = fabsf(d2[v] - d1[v]) > tol;              // false if anything is NaN
-                left[v] = ballot64(valid && certain && !(d2[v] < d1[v]));
-                again[v] = ballot64(valid && !certain);
-                n_def += __popcll(again[v]);
+                const int rest = count - 64 * v;
+                all[v] = rest >= 64 ? ~0ull : (rest > 0 ? (1ull << rest) - 1ull : 0ull);
+                const int diff = d2[v] - d1[v];
+                left[v] = ballot64(diff > limit) & all[v];
+                again[v] = all[v] & ~left[v] & ~ballot64(diff < -limit);
             }
+            if (wild) {
+#pragma unroll
+                for (int v = 0; v < kV; ++v) {
+                    again[v] |= ballot64(max(d1[v], d2[v]) == kUnknown) & all[v];
+                    left[v] &= ~again[v];
+                }
+            }
+            if (equal_rows && uniform(same[o1]) == uniform(same[o2])) {
+#pragma unroll
+                for (int v = 0; v < kV; ++v) {
+                    left[v] = all[v];
+                    again[v] = 0;
+                }
+            }
+#pragma unroll
+            for (int v = 0; v < kV; ++v) n_def += __popcll(again[v]);
             seen += count;
             if (n_def > 0) {
-                // the exact test; bit 31 of a point's place in ord carries the answer
                 unsure += n_def;
                 int at = 0;
 #pragma unroll
                 for (int v = 0; v < kV; ++v) {
-                    if ((again[v] >> lane) & 1ull) tmp[at + mask_prefix(again[v])] = lane + 64 * v;
+                    if (lane_bit(again[v])) tmp[at + mask_prefix(again[v])] = lane + 64 * v;
                     at += __popcll(again[v]);
                 }
-                make_hyperplane_wave(points + (size_t)ids[o1] * P.D, points + (size_t)ids[o2] * P.D, P.D, nvec, hp);
                 wave_lds_sync();
-                resolve_exact(2, lane >> 5, tmp, n_def, nvec, 0, hp, points, P.D, [&](int pos) { return ids[ord[start + pos]]; },
-                              [&](int pos, bool right) { if (right) ord[start + pos] |= (int)0x80000000; });
+                chain_exact(points, P.D, ids[o1], ids[o2], tmp, n_def, [&](int pos) { return ids[ord[start + pos]]; },
+                            [&](int pos, bool right) { mark[pos] = right ? 1 : 0; });
                 wave_lds_sync();
 #pragma unroll
                 for (int v = 0; v < kV; ++v) {
-                    const bool mine = (again[v] >> lane) & 1ull;
-                    left[v] |= ballot64(mine && ord[start + (mine ? lane + 64 * v : 0)] >= 0);
+                    const bool mine = lane_bit(again[v]);
+                    left[v] |= ballot64(mine && mark[mine ? lane + 64 * v : 0] == 0);
                 }
             }
-            // stable partition
 #pragma unroll
             for (int v = 0; v < kV; ++v) a += __popcll(left[v]);
-            int lbase = 0;
-#pragma unroll
-            for (int v = 0; v < kV; ++v) {
-                const int i = lane + 64 * v;
-                const int lrank = lbase + mask_prefix(left[v]);
-                const bool is_left = lane_bit(left[v]);
-                if (i < count) ord[start + (is_left ? lrank : a + i - lrank)] = q[v];
-                lbase += __popcll(left[v]);
-            }
-            wave_lds_sync();
-            // (split_rules without the nodes around it) one child that stays to be split: the next link
             const int r = count - a;
-            if (!recs && min(a, r) < P.MIN && count > P.MAX && depth + 1 < P.MAX_DEPTH - 1) {
+            if (a != 0 && r != 0) {
+                // stable partition
+                int lbase = 0;
+#pragma unroll
+                for (int v = 0; v < kV; ++v) {
+                    const int i = lane + 64 * v;
+                    const int lrank = lbase + mask_prefix(left[v]);
+                    const bool is_left = lane_bit(left[v]);
+                    if (i < count) ord[start + (is_left ? lrank : a + i - lrank)] = (unsigned char)q[v];
+                    lbase += __popcll(left[v]);
+                }
+                wave_lds_sync();
+            }
+            // (split_rules without the nodes around it) one child that stays to be split: the next link.  (It leaves no record in
+            // the index of the tree either, and takes over the one of its parent.)
+            if (min(a, r) < P.MIN && count > P.MAX && depth + 1 < P.MAX_DEPTH - 1) {
+                ++depth;
                 if (a == 0 || r == 0) {
                     draws.descend(a ? 0 : 1);
                     dstart = start;
                     dcount = count;
-                } else {
-                    const bool left_big = a >= r;
-                    draws.descend(left_big ? 0 : 1);
-                    dstart = left_big ? start : start + a;
-                    dcount = left_big ? a : r;
+                    continue;
                 }
-                ++depth;
+                const bool left_big = a >= r;
+                draws.descend(left_big ? 0 : 1);
+                dstart = left_big ? start : start + a;
+                dcount = left_big ? a : r;
                 take_order();
                 continue;
             }
-            // children: the first one that is no bucket is next, another waits on the stack
-            TreeNode full, c[2];
-            full.tree = tk.tree; full.start = start; full.count = count; full.dstart = dstart; full.dcount = dcount;
-            full.depth = depth; full.buf = 0; full.leaf = 0; full.rec = rec; full.chunk0 = 0; full.key = draws.node_key();
-            const int nc = split_rules(full, a, P.MIN, P.MAX, 0, c[0], c[1]);
-            if (recs) {
-                if (lane == 0) index_split(recs, n_rec, rec_cap, rec, ids[o1], ids[o2], nc, c[0].rec, c[1].rec, ctr);
-                c[0].rec = __builtin_amdgcn_readfirstlane(c[0].rec);
-                c[1].rec = __builtin_amdgcn_readfirstlane(c[1].rec);
-            }
-            bool have = false;
-            for (int k = 0; k < nc; ++k) {
-                if (c[k].leaf || c[k].depth >= P.MAX_DEPTH - 1) {
-                    const int big = c[k].count > kBucketSplit ? 1 : 0;
-                    if (lane == 0) {
-                        if (nrec < node_cap) lrec[nrec] = make_int2(tk.start + c[k].start, c[k].count | (n_kind[big] << 16));
-                        else ctr->overflow = 1;
-                        if (recs) index_bucket(recs, rec_cap, c[k].rec, tk.start + c[k].start, c[k].count, ctr);
+            // children (split_rules): the first one that is no bucket is next, another waits on the stack
+            const uint64_t key = draws.node_key();
+            const bool two = min(a, r) >= P.MIN && a != 0 && r != 0;
+            int rec0 = rec;
+            if (two) {
+                // (index_split)
+                if (recs_all) {
+                    if (lane == 0 && n_crec < 2 * node_cap) {
+                        ChainRec x;
+                        x.at = rec; x.a = ids[o1]; x.b = ids[o2]; x.c0 = 2 * n_split;
+                        crec[n_crec] = x;
                     }
+                    ++n_crec;
+                }
+                rec0 = 2 * n_split;
+                ++n_split;
+            }
+            ++depth;
+            bool have = false;
+            auto child = [&](int cstart, int ccount, int cdstart, int cdcount, int side, bool leaf, int crec_at) {
+                if (leaf || depth >= P.MAX_DEPTH - 1) {
+                    const bool big = ccount > kBucketSplit;
+                    if (lane == 0) {
+                        if (nrec < node_cap) lrec[nrec] = make_int2(tk.start + cstart, ccount | ((big ? n_big : nrec - n_big) << 16));
+                        if (recs_all && n_crec < 2 * node_cap) {
+                            ChainRec x;
+                            x.at = crec_at; x.a = tk.start + cstart; x.b = ccount; x.c0 = -1;
+                            crec[n_crec] = x;
+                        }
+                    }
+                    ++n_crec;
                     ++nrec;
-                    ++n_kind[big];
-                    levels = max(levels, c[k].depth + 1);
-                    largest = max(largest, c[k].count);
-                    smallest = min(smallest, c[k].count);
+                    n_big += big ? 1 : 0;
+                    levels = max(levels, depth + 1);
+                    largest = max(largest, ccount);
+                    smallest = min(smallest, ccount);
                 } else if (!have) {
                     have = true;
-                    start = c[k].start; count = c[k].count; dstart = c[k].dstart; dcount = c[k].dcount;
-                    depth = c[k].depth; rec = c[k].rec;
-                    draws.start(c[k].key);
+                    start = cstart; count = ccount; dstart = cdstart; dcount = cdcount;
+                    rec = crec_at;
+                    draws.start(child_key(key, side));
                 } else {
                     if (lane == 0) {
                         if (sp < node_cap) {
                             SmallNode sn;
-                            sn.start = c[k].start; sn.count = c[k].count; sn.dstart = c[k].dstart; sn.dcount = c[k].dcount;
-                            sn.depth = c[k].depth; sn.leaf = 0; sn.key = c[k].key; sn.rec = c[k].rec; sn.vain = 0;
+                            sn.start = cstart; sn.count = ccount; sn.dstart = cdstart; sn.dcount = cdcount;
+                            sn.depth = depth; sn.leaf = 0; sn.key = child_key(key, side); sn.rec = crec_at;
                             stack[sp] = sn;
                         } else {
                             ctr->overflow = 1;
@@ -1413,42 +1845,52 @@ __global__ __launch_bounds__(256) void k_chain(const float* __restrict__ points,
                     }
                     sp = min(sp + 1, node_cap);
                 }
+            };
+            const int start0 = start, count0 = count;
+            if (two) {
+                child(start0, a, start0, a, 0, a <= P.MAX - 2, rec0);
+                child(start0 + a, r, start0 + a, r, 1, r <= P.MAX - 2, rec0 + 1);
+            } else if (a == 0 || r == 0) {
+                child(start0, count0, start0, count0, a ? 0 : 1, count0 <= P.MAX - 2, rec0);
+            } else {
+                const bool left_big = a >= r;
+                child(start0, count0, left_big ? start0 : start0 + a, left_big ? a : r, left_big ? 0 : 1, count0 <= P.MAX, rec0);
             }
             if (!have) {
                 if (sp == 0) break;
                 --sp;
                 wave_lds_sync();
                 const SmallNode* sn = &stack[sp];
-                start = __builtin_amdgcn_readfirstlane(sn->start);
-                count = __builtin_amdgcn_readfirstlane(sn->count);
-                dstart = __builtin_amdgcn_readfirstlane(sn->dstart);
-                dcount = __builtin_amdgcn_readfirstlane(sn->dcount);
-                depth = __builtin_amdgcn_readfirstlane(sn->depth);
-                rec = __builtin_amdgcn_readfirstlane(sn->rec);
-                draws.start(sn->key);
+                start = uniform(sn->start);
+                count = uniform(sn->count);
+                dstart = uniform(sn->dstart);
+                dcount = uniform(sn->dcount);
+                depth = uniform(sn->depth);
+                rec = uniform(sn->rec);
+                draws.start((uint64_t)(uint32_t)uniform((int)(uint32_t)sn->key) | ((uint64_t)(uint32_t)uniform((int)(uint32_t)(sn->key >> 32)) << 32));
             }
             take_order();
         }
         for (int i = lane; i < n; i += 64) seg[i] = ids[ord[i]];
-        int base[2] = {0, 0};
+        // the places of the buckets and records are reserved here and taken after the next node's matrix
+        pend_n = nrec;
+        pend_recs = n_crec;
+        pend_tree = tk.tree;
+        pend_rec = tk.rec;
         if (lane == 0) {
-            TreeStats* st = stats + tk.tree;
-            if (n_kind[0]) base[0] = atomicAdd(&st->n_leaves, n_kind[0]);
-            if (n_kind[1]) base[1] = atomicAdd(&st->n_big, n_kind[1]);
-            // (the extremes settle early: a look before the atomic spares nearly all of them)
-            if (*const_cast<volatile int*>(&st->levels) < levels) atomicMax(&st->levels, levels);
-            if (*const_cast<volatile int*>(&st->max_leaf) < largest) atomicMax(&st->max_leaf, largest);
-            if (*const_cast<volatile int*>(&st->min_leaf) > smallest) atomicMin(&st->min_leaf, smallest);
+            if (nrec > n_big) pend_base[0] = atomicAdd(&st->n_leaves, nrec - n_big);
+            if (n_big) pend_base[1] = atomicAdd(&st->n_big, n_big);
+            if (recs_all && n_split) pend_base[2] = atomicAdd(&st->n_rec, 2 * n_split);
+            if (nrec > node_cap || n_crec > 2 * node_cap) ctr->overflow = 1;
+            // (the extremes settle early: what they were when the chain began spares nearly all of the atomics)
+            if (levels_seen < levels) atomicMax(&st->levels, levels);
+            if (most_seen < largest) atomicMax(&st->max_leaf, largest);
+            if (least_seen > smallest) atomicMin(&st->min_leaf, smallest);
         }
-        base[0] = __builtin_amdgcn_readfirstlane(base[0]);
-        base[1] = __builtin_amdgcn_readfirstlane(base[1]);
-        for (int i = lane; i < min(nrec, node_cap); i += 64) {
-            const int2 r = lrec[i];
-            const int m = r.y & 0xffff, rank = r.y >> 16;
-            store_leaf(tk.tree, r.x, m, base[m > kBucketSplit ? 1 : 0] + rank, leaf_cap, leaf_start, leaf_size, ctr);
-        }
+        turn ^= 1;
     }
-    if (tid == 0) {
+    if (wave == 0 && pend_n) store_pending(turn ^ 1, threadIdx.x);
+    if (threadIdx.x == 0) {
         stat_add(stat, (int)blockIdx.x, 0, seen);
         stat_add(stat, (int)blockIdx.x, 1, unsure);
     }
@@ -1456,7 +1898,7 @@ __global__ __launch_bounds__(256) void k_chain(const float* __restrict__ points,
 
 // What a batch tells the host at its end, in pinned memory.
 struct BatchReport {
-    TreeStats stats[64];
+    int stats[64][5];                    // the first five of TreeStats
     long long phase_ticks[4];
     unsigned long long counts[2];
     int overflow;
@@ -1468,7 +1910,11 @@ __global__ __launch_bounds__(64) void k_tree_report(const TreeStats* __restrict_
 {
     const int lane = threadIdx.x;
     if (lane == 0) phase_tick(ctr, 3);
-    if (lane < nb) out->stats[lane] = stats[lane];
+    if (lane < nb) {
+        const TreeStats s = stats[lane];
+        int* o = out->stats[lane];
+        o[0] = s.n_leaves; o[1] = s.n_big; o[2] = s.levels; o[3] = s.max_leaf; o[4] = s.min_leaf;
+    }
     static_assert(kStatSlots == 64, "one slot per lane");
     unsigned long long a = stat[kStatPitch * lane], b = stat[kStatPitch * lane + 1];
 #pragma unroll
@@ -1518,7 +1964,6 @@ struct TreeBatchWorkspace {
     unsigned long long counts[2] = {0, 0};       // of the last batch: points the side tests looked at, undecided ones
     // index of the trees for routing query points (allocated by tree_ws_enable_index)
     TreeRec* recs = nullptr;             // B x rec_cap
-    int* n_rec = nullptr;                // B
     int rec_cap = 0;
     float phase_s[4] = {0.f, 0.f, 0.f, 0.f};   // of the last batch: side tests, hyperplanes, scatter, tail kernel
     // side tests of the first levels taken point by point (tree_sweep.hpp); allocated when D allows it
@@ -1537,7 +1982,7 @@ struct TreeBatchWorkspace {
 static void free_ws(TreeBatchWorkspace& w)
 {
     void* dev[] = {w.perm[0], w.perm[1], w.nodes[0], w.nodes[1], w.tail, w.chain, w.chunk2node,
-                   w.chunk_left, w.leaf_start, w.leaf_size, w.stats, w.ctr, w.recs, w.n_rec, w.planes,
+                   w.chunk_left, w.leaf_start, w.leaf_size, w.stats, w.ctr, w.recs, w.planes,
                    w.pm_path, w.pm_side, w.pm_undec, w.pm_map[0], w.pm_map[1], w.pm_sc, w.pm_aq, w.pm_child, w.stat};
     for (void* p : dev) ws_free(p);
     pin_free(w.notes.block());
@@ -1559,7 +2004,6 @@ const int* tree_ws_leaf_size(const TreeBatchWorkspace* w, int t) { return w->lea
 
 const int* tree_ws_stats(const TreeBatchWorkspace* w, int t)
 {
-    static_assert(sizeof(TreeStats) == 5 * sizeof(int), "read as five ints");
     return reinterpret_cast<const int*>(w->stats + t);
 }
 
@@ -1573,19 +2017,18 @@ int tree_small_threshold(int D, int N, int B)
     const char* e = std::getenv("RSFK_TREE_SMALL");
     const bool few = (size_t)N * (size_t)std::max(B, 1) < ((size_t)1 << 21);
     const int v = e && *e ? std::atoi(e) : (D <= 48 || few ? 2048 : 1024);
-    return std::min(2048, std::max(64, v));
+    return std::min(kTailMost, std::max(64, v));
 }
-// Largest node the chain phase takes (0: none): twice the leaf limit where that fits two workgroups per compute unit
-// (nodes just above the limit are the ones that are split in vain), else what one workgroup can hold.
+// Largest node the chain phase takes (0: none).  Up to 128 points the matrix costs less than the two or three levels of the tail
+// kernel it stands for.  Larger nodes only where they are likely to be split in vain, which means that less than a quarter of their points is more
+// than the two sides need (3,000 x 200 with buckets of 31..128: one split and a half per node, tail and chains 142 -> 181 us).
 int tree_chain_max(int D, int MIN, int MAX)
 {
     const char* e = std::getenv("RSFK_TREE_CHAIN");
-    if ((e && e[0] == '0') || D > 2048) return 0;            // (the normal takes the place of the staged rows)
-    const int per_min = std::max(MIN, 1);
-    if (MAX + MAX / 8 <= kChainSquare) return std::min(kChainSquare, std::max(64, (2 * MAX + 7) & ~7));
-    int n = 0;
-    for (int m = kChainSquare + 8; m <= 256; m += 8)
-        if (chain_lds_bytes(m, D, m / per_min + 4) <= (size_t)158 * 1024) n = m;
+    if ((e && e[0] == '0') || D > 2048) return 0;
+    if (MAX <= 40) return 64;
+    if (MAX + MAX / 8 <= kChainSquare) return kChainSquare;
+    const int n = std::min(256, 8 * MIN / 3);
     return n > MAX ? n : 0;
 }
 constexpr int kWideChunk = 1024;         // points per workgroup in the wide passes (k_side keeps a chunk's undecided points in LDS)
@@ -1607,12 +2050,11 @@ int tree_ws_enable_index(TreeBatchWorkspace* w, int MIN, int MAX_DEPTH)
     RSFK_CHECK(cap < ((size_t)1 << 30), "tree index: too many nodes");
     w->rec_cap = (int)cap;
     if (dmalloc(&w->recs, (size_t)w->B * cap)) return 1;
-    if (dmalloc(&w->n_rec, (size_t)w->B)) return 1;
     return 0;
 }
 const TreeRec* tree_ws_recs(const TreeBatchWorkspace* w, int t) { return w->recs + (size_t)t * w->rec_cap; }
 int tree_ws_rec_cap(const TreeBatchWorkspace* w) { return w->rec_cap; }
-const int* tree_ws_n_rec(const TreeBatchWorkspace* w, int t) { return w->n_rec + t; }
+const int* tree_ws_n_rec(const TreeBatchWorkspace* w, int t) { return &w->stats[t].n_rec; }
 
 int tree_ws_alloc(TreeBatchWorkspace** out, int N, int D, int MIN, int B)
 {
@@ -1684,7 +2126,6 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
     P.N = N; P.D = D; P.MIN = MIN; P.MAX = MAX; P.MAX_DEPTH = MAX_DEPTH;
     P.small = tree_small_threshold(D, N, w->B);
     P.chain_max = tree_chain_max(D, MIN, MAX);
-    P.vain = 4;
     P.chunk = kWideChunk;
     // bfloat16 rounding 2^-8 (1 + 2^-7), plus the summation errors of the screen (D/8 terms per lane and a 3-step
     // tree) and of the exact test (D/32 terms per lane and a 5-step tree), 1 % on top
@@ -1708,7 +2149,7 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
     {
         const size_t total = (size_t)N * nb;
         const int grid = (int)std::min<size_t>((total + 255) / 256, 65536);
-        hipLaunchKernelGGL(k_tree_init, dim3(grid), dim3(256), 0, stream, w->perm[0], Q, P, nb, seed0, w->n_rec,
+        hipLaunchKernelGGL(k_tree_init, dim3(grid), dim3(256), 0, stream, w->perm[0], Q, P, nb, seed0,
                            pm_levels > 0 ? w->pm_map[0] : nullptr, w->stats, w->stat);
         RSFK_HIP(hipGetLastError());
     }
@@ -1793,7 +2234,7 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
         Q.next = w->nodes[cur ^ 1];
         Q.slot = (level + 1) & 3;
         hipLaunchKernelGGL(k_scatter, dim3(n_chunks), dim3(kBlock), 0, stream, P, w->perm[0], w->perm[1], w->nodes[cur],
-                           slot, w->chunk2node, w->chunk_left, Q, w->recs, w->n_rec, w->rec_cap,
+                           slot, w->chunk2node, w->chunk_left, Q, w->recs, w->stats, w->rec_cap,
                            map_next ? w->pm_child : nullptr);
         if (map_next) {
             const int n_paths = 1 << level;
@@ -1824,37 +2265,55 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
                            (few ? 3 : 2) * (size_t)node_cap * sizeof(SmallNode) + (size_t)P.small;
         RSFK_CHECK(lds <= 150 * 1024, "tree batch: D too large for the tail kernel's LDS budget");
         const bool tail_q8 = q8 != nullptr && std::getenv("RSFK_TAIL_BF16") == nullptr;
-#define RSFK_TAIL_LAUNCH(Q, T, C)                                                                                             \
+#define RSFK_TAIL_LAUNCH(Q, T, C, L, U)                                                                                       \
         do {                                                                                                               \
-            RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_tail<Q, T, C>),                                      \
+            RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_tail<Q, T, C, L, U>),                                \
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));                          \
-            hipLaunchKernelGGL((k_tail<Q, T, C>), dim3(n_tail), dim3(T), lds, stream, points, pb16, q8, P, w->perm[0],         \
+            hipLaunchKernelGGL((k_tail<Q, T, C, L, U>), dim3(n_tail), dim3(T), lds, stream, points, pb16, q8, P, w->perm[0],   \
                                w->perm[1], w->perm[0], w->tail, n_tail, node_cap, G, w->leaf_cap, w->leaf_start,            \
-                               w->leaf_size, w->stats, w->ctr, w->recs, w->n_rec, w->rec_cap, w->stat, w->chain, w->tail_cap); \
+                               w->leaf_size, w->stats, w->ctr, w->recs, w->rec_cap, w->stat, w->chain, w->tail_cap);         \
         } while (0)
-        if (tail_q8 && few && n_tail <= 256) RSFK_TAIL_LAUNCH(true, 1024, true);
-        else if (tail_q8 && few) RSFK_TAIL_LAUNCH(true, 512, true);
-        else if (tail_q8) RSFK_TAIL_LAUNCH(true, 256, false);
-        else if (few) RSFK_TAIL_LAUNCH(false, 512, true);
-        else RSFK_TAIL_LAUNCH(false, 256, false);
+        // Lanes per point: as many as there are pieces of 16 coordinates, up to four; few subtrees wait for the loads of a point, and
+        // four lanes with four pieces in flight each take longer rows (eight beyond 256 dimensions).  With many subtrees eight lanes keep the
+        // kernel in its registers.  (Tail of 10M x 32, 10 trees 9.25 -> 7.29 ms with two lanes instead of eight; 20,000 x 32, 50 trees
+        // 306 -> 211 us, with the partition by pieces.)
+        const int pieces = q8_padded(D) / 16;
+#define RSFK_TAIL_LANES(T)                                                                                                  \
+        do {                                                                                                               \
+            if (pieces <= 2) RSFK_TAIL_LAUNCH(true, T, true, 2, 1);                                                         \
+            else if (pieces <= 4) RSFK_TAIL_LAUNCH(true, T, true, 4, 1);                                                    \
+            else if (pieces <= 16) RSFK_TAIL_LAUNCH(true, T, true, 4, 4);                                                   \
+            else RSFK_TAIL_LAUNCH(true, T, true, 8, 4);                                                                     \
+        } while (0)
+        if (tail_q8 && few && n_tail <= 256) RSFK_TAIL_LANES(1024);
+        else if (tail_q8 && few && (n_tail <= 512 || pieces > 4)) RSFK_TAIL_LANES(512);
+        else if (tail_q8 && few) RSFK_TAIL_LANES(256);
+        else if (tail_q8 && pieces <= 2) RSFK_TAIL_LAUNCH(true, 256, false, 2, 1);
+        else if (tail_q8 && pieces <= 4) RSFK_TAIL_LAUNCH(true, 256, false, 4, 1);
+        else if (tail_q8) RSFK_TAIL_LAUNCH(true, 256, false, 8, 1);
+        else if (few) RSFK_TAIL_LAUNCH(false, 512, true, 8, 1);
+        else RSFK_TAIL_LAUNCH(false, 256, false, 8, 1);
+#undef RSFK_TAIL_LANES
 #undef RSFK_TAIL_LAUNCH
         RSFK_HIP(hipGetLastError());
     }
     if (few && P.chain_max > 0) {
         const int node_cap = P.chain_max / std::max(MIN, 1) + 4;
-        const size_t lds = chain_lds_bytes(P.chain_max, D, node_cap);
-        const size_t most = (size_t)N * (size_t)nb / (size_t)std::max(MAX - 1, 1) + 1;          // nodes that are no buckets are disjoint
+        const size_t lds = chain_lds_bytes(P.chain_max, node_cap, w->recs != nullptr);
+        const size_t most = (size_t)N * (size_t)nb / (size_t)std::max(MAX - 1, 1) + (size_t)nb;      // nodes that are no buckets are disjoint
         const unsigned grid = (unsigned)std::min<size_t>(most, 256 * (size_t)std::max<size_t>(1, (size_t)160 * 1024 / lds));
-#define RSFK_CHAIN_LAUNCH(NBV)                                                                                              \
+        const float gram_error = chain_gram_error(D);
+#define RSFK_CHAIN_LAUNCH(NT, W)                                                                                            \
         do {                                                                                                               \
-            RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_chain<NBV>),                                      \
+            RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_chain<NT, W>),                                    \
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));                          \
-            hipLaunchKernelGGL(k_chain<NBV>, dim3(grid), dim3(256), lds, stream, points, q8, P, w->perm[0], w->chain,       \
-                               w->tail_cap, node_cap, w->leaf_cap, w->leaf_start, w->leaf_size, w->stats, w->ctr, w->recs,  \
-                               w->n_rec, w->rec_cap, w->stat);                                                             \
+            hipLaunchKernelGGL((k_chain<NT, W>), dim3(grid), dim3(64 * W), lds, stream, points, q8, P, gram_error,           \
+                               w->perm[0], w->chain, w->tail_cap, node_cap, w->leaf_cap, w->leaf_start, w->leaf_size, w->stats, w->ctr,  \
+                               w->recs, w->rec_cap, w->stat);                                                               \
         } while (0)
-        if (P.chain_max <= kChainSquare) RSFK_CHAIN_LAUNCH(8);
-        else RSFK_CHAIN_LAUNCH(16);
+        if (P.chain_max <= 64) RSFK_CHAIN_LAUNCH(2, 1);
+        else if (P.chain_max <= kChainSquare) RSFK_CHAIN_LAUNCH(4, 2);
+        else RSFK_CHAIN_LAUNCH(8, 4);
 #undef RSFK_CHAIN_LAUNCH
         RSFK_HIP(hipGetLastError());
     }
@@ -1879,12 +2338,13 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
     }
     RSFK_CHECK(!R.overflow, "tree batch: queue overflow in the tail phase");
     for (int t = 0; t < nb; ++t) {
-        const int total = R.stats[t].n_leaves + R.stats[t].n_big;
+        const int* st = R.stats[t];
+        const int total = st[0] + st[1];
         host_stats[5 * t + 0] = total;
-        host_stats[5 * t + 1] = R.stats[t].levels;
-        host_stats[5 * t + 2] = R.stats[t].max_leaf;
-        host_stats[5 * t + 3] = total ? R.stats[t].min_leaf : 0;
-        host_stats[5 * t + 4] = R.stats[t].n_big;
+        host_stats[5 * t + 1] = st[2];
+        host_stats[5 * t + 2] = st[3];
+        host_stats[5 * t + 3] = total ? st[4] : 0;
+        host_stats[5 * t + 4] = st[1];
         RSFK_CHECK(total <= w->leaf_cap, "tree batch: leaf table overflow");
     }
     return 0;

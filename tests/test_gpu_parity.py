@@ -138,6 +138,37 @@ def test_tree_of_rows_whose_sums_leave_fp32(gpu, orc, rng, monkeypatch, kind, en
         assert list(gst) == [len(ls), st[0], st[1], st[2]]
 
 
+# The forms of the tail and of the chain phase: leaf limits on either side of the sizes of the chain's matrix (nodes of up to 64, 128
+# and 256 points, and none), rows on either side of the lanes that share one, many subtrees (nodes above `small` points are wide) and
+# few; rows without distances (NaN, and a few far longer than the others), clusters within one node, the index that query points
+# are routed by is covered by the tests of the search.
+@pytest.mark.parametrize("N,D,MIN,MAX,small,kind", [
+    (9000, 7, 20, 40, 2048, "n"), (9000, 7, 20, 41, 2048, "n"), (9000, 40, 56, 113, 2048, "n"), (9000, 40, 57, 114, 2048, "n"),
+    (9000, 19, 96, 191, 2048, "n"), (9000, 19, 96, 255, 2048, "n"), (9000, 19, 128, 256, 2048, "n"), (9000, 32, 3, 6, 2048, "n"),
+    (30000, 32, 17, 34, 80, "n"), (30000, 64, 17, 34, 80, "n"), (30000, 65, 17, 34, 80, "n"), (12000, 256, 33, 66, 2048, "n"),
+    (8000, 257, 33, 66, 2048, "n"), (9000, 24, 33, 66, 2048, "nan"), (9000, 24, 33, 66, 2048, "far"), (9000, 24, 96, 192, 2048, "far"),
+    (9000, 36, 33, 66, 2048, "clusters"), (9000, 36, 8, 16, 2048, "clusters"),
+])
+@pytest.mark.parametrize("screen", ["q8", "bf16"])
+def test_tree_forms_of_tail_and_chain(gpu, orc, rng, monkeypatch, N, D, MIN, MAX, small, kind, screen):
+    monkeypatch.setenv("RSFK_TREE_SCREEN", screen)
+    monkeypatch.setenv("RSFK_TREE_SMALL", str(small))
+    X = rng.standard_normal((N, D)).astype(np.float32)
+    if kind == "nan":
+        X[rng.random(N) < 0.01, 1] = np.nan
+    if kind == "far":
+        X[rng.random(N) < 0.02] *= np.float32(1e3)
+    if kind == "clusters":
+        X = (10.0 * rng.standard_normal((40, D))[rng.integers(0, 40, N)] + 1e-3 * X).astype(np.float32)
+    for seed in (1, 2):
+        _say("tree forms", N, D, MIN, MAX, small, kind, screen, seed)
+        perm, ls, lz, st = orc.build_tree(X, MIN, MAX, 300, seed)
+        gperm, gls, glz, gst = gpu.build_tree(X, MIN, MAX, 300, seed)
+        assert np.array_equal(gperm, perm)
+        assert np.array_equal(gls, ls) and np.array_equal(glz, lz)
+        assert list(gst) == [len(ls), st[0], st[1], st[2]]
+
+
 def test_tree_edge_cases(gpu, orc, rng):
     # identical points: re-drawn until the depth limit, then one forced bucket
     X = np.ones((3000, 4), np.float32)
