@@ -156,6 +156,7 @@ struct TreeParams {
     int N, D;
     int MIN, MAX, MAX_DEPTH;
     int small;        // nodes with at most this many points are finished by one workgroup
+    int mid;          // 1: the queue of the wide levels is that of the middle phase
     int chain_max;    // nodes of at most this many points go to the chain phase (0: none)
     int chunk;        // points per workgroup in the wide (global) passes
     float band;       // half-width of the undecided band of the bfloat16 side screen, relative to sum |n_d||x~_d|

@@ -20,6 +20,10 @@
 //                wave64 ballot / mbcnt ranks, child creation by the chunk-0
 //                workgroup of each node, (3) chunk bookkeeping for the next
 //                level.
+//   middle phase: with few points (small inputs, few trees) nodes of up to some
+//                thousand points are split down to `small` by one workgroup
+//                each (k_mid), which replaces most of the wide levels.
+//
 //   tail phase : one workgroup finishes the whole subtree of a node with at
 //                most `small` points inside LDS (all the re-draw levels that
 //                the min/max rule causes touch only such nodes).
@@ -59,6 +63,7 @@ struct LevelCounters {
         int chunks;    // and their chunks
     } queue[4];
     int n_tail;        // tail tasks appended so far
+    int n_mid;         // ... and tasks of the middle phase
     int n_chain;       // nodes for the chain phase appended so far, at the front of their queue
     int n_chain_back;  // ... and at its back: those that are hardly split in vain
     int overflow;      // set when a queue capacity is exceeded
@@ -290,8 +295,8 @@ __device__ __forceinline__ void side_screen8(const float* nvec0, int nstride, co
 // wavefront at a time so that their row loads overlap; all threads of the workgroup call.  id_at(pos) gives the
 // point, apply(pos, right) receives the answer in lane 0 of the half wavefront.
 // (h of `halves`: which half wavefront of those that work on the list this is)
-template <typename IdAt, typename Apply>
-__device__ __forceinline__ void resolve_exact(int halves, int h, const int* list, int n, const float* nvec0, int nstride, const float* b_of,
+template <typename Entry, typename IdAt, typename Apply>
+__device__ __forceinline__ void resolve_exact(int halves, int h, const Entry* list, int n, const float* nvec0, int nstride, const float* b_of,
                                               const float* __restrict__ points, int D, IdAt id_at, Apply apply)
 {
     const int hl = threadIdx.x & 31;
@@ -334,9 +339,10 @@ constexpr int kSideBatch = 4;        // points per group and call of the screen 
 struct NodeQueues {
     TreeNode* next;
     int next_cap, chunk_cap, slot;
-    TreeNode* tail;
+    TreeNode* tail;      // (or the middle phase)
     int tail_cap;
     LevelCounters* ctr;
+    int* n_tail;         // its counter
 };
 
 // Append the nc children of a node to their queues; a node of the next wide level is given its chunks too.  at[i]: place
@@ -363,7 +369,7 @@ __device__ __forceinline__ void emit_children(const TreeNode (&c)[2], int nc, co
         next = (int)(unsigned)was;
         chunk = (int)(unsigned)(was >> 32);
     }
-    if (n_tail) tail = atomicAdd(&Q.ctr->n_tail, n_tail);
+    if (n_tail) tail = atomicAdd(Q.n_tail, n_tail);
     if ((n_wide && (next + n_wide > Q.next_cap || chunk + n_chunks > Q.chunk_cap)) || (n_tail && tail + n_tail > Q.tail_cap)) {
         Q.ctr->overflow = 1;
         return;
@@ -516,7 +522,7 @@ __global__ __launch_bounds__(256) void k_level_planes(const float* __restrict__ 
         ctr->queue[(level + 1) & 3].chunks = 0;
         note->n_nodes = n_nodes;
         note->n_chunks = n_chunks;
-        note->n_tail = ctr->n_tail;
+        note->n_tail = P.mid ? ctr->n_mid : ctr->n_tail;
         note->overflow = ctr->overflow;
         __hip_atomic_store(&note->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
@@ -854,9 +860,8 @@ __global__ __launch_bounds__(TB, CHAIN ? 4 : 6) void k_tail(const float* __restr
     __shared__ int n_chain_s[2], chain_base_s[2], n_chain_all_s;     // (front and back of the queue)
     __shared__ int seen_s, unsure_s;        // points tested over all levels of the subtree, and left to the exact test
 
-    const int task = blockIdx.x;
-    if (task >= n_tasks) return;
-    if (task == 0 && threadIdx.x == 0) phase_tick(ctr, 2);
+    const auto finish = [&](const int task) {
+    if (task == 0 && threadIdx.x == 0) phase_tick(ctr, P.mid ? 3 : 2);
     const TreeNode tk = tasks[task];
     const size_t toff = (size_t)tk.tree * (size_t)P.N;
     const int* src = (tk.buf ? perm1 : perm0) + toff;
@@ -1120,6 +1125,205 @@ __global__ __launch_bounds__(TB, CHAIN ? 4 : 6) void k_tail(const float* __restr
         c.depth = sn.depth; c.buf = 0; c.leaf = 0; c.rec = sn.rec; c.chunk0 = 0; c.key = sn.key;
         const int back = sn.leaf & 1, at = chain_base_s[back] + (sn.leaf >> 1);
         if (at < chain_cap) chain_all[back ? chain_cap - 1 - at : at] = c; else ctr->overflow = 1;
+    }
+    };
+    if constexpr (CHAIN) {
+        // (after the middle phase only the device knows how many there are)
+        const int n = P.mid ? ctr->n_tail : n_tasks;
+        for (int task = blockIdx.x; task < n; task += gridDim.x) {
+            __syncthreads();
+            finish(task);
+        }
+    } else if ((int)blockIdx.x < n_tasks) {
+        finish(blockIdx.x);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// middle phase: one workgroup per node of up to mid_most points
+// ---------------------------------------------------------------------------
+// A wide level of a batch of few points is three launches that leave most of the device idle, about 25 us whatever the level holds,
+// and a tree of 10,000 points has six of them above the nodes the tail kernel takes.  Here one workgroup of 1024 threads keeps the
+// permutation of a node in LDS and splits it, and whatever of its descendants is larger than P.small, one node after the other: no launch
+// and no trip of the permutation to memory in between.  A node costs the trips for the pair's rows, for the screening rows and
+// for the rows of the undecided points and, beyond that, the rate at which one compute unit
+// reads screening rows, which sets the largest node (tree_mid_most).  The others go to the queue of the tail kernel.
+// (K-NN graph of 3,000 x 200, 10 trees 889 -> 831 us, 10,000 x 32, 4 trees 624 -> 590, one tree of 10,000 x 2 235 -> 215; 123,457 x 37, 12 trees
+// and one tree of 592,523 x 20, where the wide levels above remain: the same.)
+constexpr int kMidMost = 12288;          // points (LDS: 4 bytes of permutation and 2 of the list of undecided points each)
+constexpr int kMidThreads = 1024, kMidPer = kMidMost / kMidThreads;
+constexpr int kMidOut = 64;              // nodes for the tail kernel kept before they are given a place in its queue
+
+template <int LPP, int KU>
+__global__ __launch_bounds__(kMidThreads, 4) void k_mid(const float* __restrict__ points, const uint8_t* __restrict__ q8, TreeParams P, int most,
+                                                        const int* __restrict__ perm0, const int* __restrict__ perm1, int* __restrict__ perm_out,
+                                                        const TreeNode* __restrict__ tasks, TreeNode* __restrict__ tail, int tail_cap, int stack_cap,
+                                                        TreeStats* stats, LevelCounters* ctr, TreeRec* __restrict__ recs_all, int rec_cap,
+                                                        unsigned long long* __restrict__ stat)
+{
+    // dynamic LDS: seg[most] | nvec[nvec_len(D)] | nodes to split [stack_cap] | nodes for the tail [kMidOut] | undecided points [most]
+    extern __shared__ __align__(16) unsigned char mid_lds[];
+    int* seg = reinterpret_cast<int*>(mid_lds);
+    float* nvec = reinterpret_cast<float*>(seg + most);
+    SmallNode* stack = reinterpret_cast<SmallNode*>(nvec + nvec_len(P.D));
+    SmallNode* out = stack + stack_cap;
+    uint16_t* list = reinterpret_cast<uint16_t*>(out + kMidOut);
+    constexpr int kWaves = kMidThreads / 64;
+    __shared__ float hp_s[4];
+    __shared__ int count_s[kMidPer * kWaves], all_s, n_def_s, n_stack_s, n_out_s, out_base_s;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (blockIdx.x == 0 && tid == 0) phase_tick(ctr, 2);
+    const TreeNode tk = tasks[blockIdx.x];
+    if (tk.leaf || tk.count <= P.small) {
+        // (nodes beside larger ones that were split at a wide level)
+        if (tid == 0) {
+            const int at = atomicAdd(&ctr->n_tail, 1);
+            if (at < tail_cap) tail[at] = tk; else ctr->overflow = 1;
+        }
+        return;
+    }
+    const int* src = (tk.buf ? perm1 : perm0) + (size_t)tk.tree * (size_t)P.N;
+    int* dst = perm_out + (size_t)tk.tree * (size_t)P.N;
+    for (int i = tid; i < tk.count; i += kMidThreads) seg[i] = src[tk.start + i] & kIdMask;
+    if (tid == 0) {
+        SmallNode r;
+        r.start = 0; r.count = tk.count; r.dstart = tk.dstart - tk.start; r.dcount = tk.dcount;
+        r.depth = tk.depth; r.leaf = 0; r.key = tk.key; r.rec = tk.rec;
+        stack[0] = r;
+        n_stack_s = 1;
+        n_out_s = 0;
+    }
+    __syncthreads();
+    // the nodes that wait for the tail kernel get their places (all threads call)
+    auto give_out = [&]() {
+        const int n = n_out_s;
+        if (tid == 0) out_base_s = n ? atomicAdd(&ctr->n_tail, n) : 0;
+        __syncthreads();
+        for (int i = tid; i < n; i += kMidThreads) {
+            const SmallNode sn = out[i];
+            TreeNode c;
+            c.tree = tk.tree; c.start = tk.start + sn.start; c.count = sn.count; c.dstart = tk.start + sn.dstart; c.dcount = sn.dcount;
+            c.depth = sn.depth; c.buf = 0; c.leaf = sn.leaf; c.rec = sn.rec; c.chunk0 = 0; c.key = sn.key;
+            const int at = out_base_s + i;
+            if (at < tail_cap) tail[at] = c; else ctr->overflow = 1;
+        }
+        if (tid == 0) n_out_s = 0;
+        __syncthreads();
+    };
+    constexpr int kGroups = kMidThreads / LPP, kBatch = KU == 1 ? 4 : 2;
+    const int grp = tid / LPP, sub = tid & (LPP - 1);
+    int seen = 0, unsure = 0;
+    while (true) {
+        const int n_stack = n_stack_s;
+        if (n_stack == 0) break;
+        const SmallNode nd = stack[n_stack - 1];
+        const int st = nd.start, cnt = nd.count;
+        int r1, r2;
+        pick_pair(nd.key, nd.dcount, r1, r2);
+        const int p1 = seg[nd.dstart + r1], p2 = seg[nd.dstart + r2];
+        if (wave == 0) make_hyperplane_wave(points + (size_t)p1 * P.D, points + (size_t)p2 * P.D, P.D, nvec, hp_s);
+        if (tid == 64) n_def_s = 0;
+        __syncthreads();
+        const float b = hp_s[0], n1 = hp_s[1], sn = hp_s[2];
+        for (int it = 0; it * kGroups < cnt; it += kBatch) {
+            int id[kBatch], jz[kBatch], pos[kBatch];
+            float bb[kBatch], h1[kBatch], h2[kBatch];
+            bool valid[kBatch], right[kBatch], redo[kBatch];
+#pragma unroll
+            for (int u = 0; u < kBatch; ++u) {
+                const int i = (it + u) * kGroups + grp;
+                valid[u] = i < cnt;
+                pos[u] = st + min(i, cnt - 1);
+                id[u] = seg[pos[u]] & kIdMask;
+                jz[u] = 0;
+                bb[u] = b;
+                h1[u] = n1;
+                h2[u] = sn;
+            }
+            side_screen8<kBatch, true, LPP, KU>(nvec, 0, jz, bb, h1, h2, nullptr, q8, id, P.D, P.band, valid, right, redo);
+#pragma unroll
+            for (int u = 0; u < kBatch; ++u) {
+                if (valid[u] && sub == 0) {
+                    if (redo[u]) list[atomicAdd(&n_def_s, 1)] = (uint16_t)(pos[u] - st);
+                    else if (right[u]) seg[pos[u]] = id[u] | (int)0x80000000;
+                }
+            }
+        }
+        __syncthreads();
+        const int n_def = n_def_s;
+        seen += cnt;
+        unsure += n_def;
+        resolve_exact(kMidThreads / 32, tid >> 5, list, n_def, nvec, 0, hp_s, points, P.D, [&](int pos) { return seg[st + pos] & kIdMask; },
+                      [&](int pos, bool right) { if (right) seg[st + pos] |= (int)0x80000000; });
+        __syncthreads();
+        // stable partition: a thread's entries are at tid, tid + 1024, ..; they wait in registers while the lefts of every 64 are counted
+        int v[kMidPer];
+#pragma unroll
+        for (int u = 0; u < kMidPer; ++u) {
+            v[u] = -1;
+            if (u * kMidThreads >= cnt) continue;
+            const int i = u * kMidThreads + tid;
+            if (i < cnt) v[u] = seg[st + i];
+            const uint64_t m = ballot64(v[u] >= 0);
+            if (lane == 0) count_s[u * kWaves + wave] = __popcll(m);
+        }
+        __syncthreads();
+        if (wave == 0) {
+            // lefts before each 64, and all of them
+            constexpr int kEach = (kMidPer * kWaves + 63) / 64;
+            const int n = (cnt + kMidThreads - 1) / kMidThreads * kWaves;
+            int x[kEach], run = 0;
+#pragma unroll
+            for (int k = 0; k < kEach; ++k) {
+                x[k] = kEach * lane + k < n ? count_s[kEach * lane + k] : 0;
+                run += x[k];
+            }
+            int before = wave_excl_scan_i(run);
+            if (lane == 63) all_s = before + run;
+#pragma unroll
+            for (int k = 0; k < kEach; ++k) {
+                if (kEach * lane + k < n) count_s[kEach * lane + k] = before;
+                before += x[k];
+            }
+        }
+        __syncthreads();
+        const int a = all_s;
+#pragma unroll
+        for (int u = 0; u < kMidPer; ++u) {
+            if (u * kMidThreads >= cnt) continue;
+            const int i = u * kMidThreads + tid;
+            const int lrank = count_s[u * kWaves + wave] + mask_prefix(ballot64(v[u] >= 0));
+            if (i < cnt) seg[st + (v[u] < 0 ? a + i - lrank : lrank)] = v[u] & kIdMask;
+        }
+        if (tid == 0) {
+            TreeNode full, c0, c1;
+            full.tree = tk.tree; full.start = nd.start; full.count = nd.count; full.dstart = nd.dstart; full.dcount = nd.dcount;
+            full.depth = nd.depth; full.buf = 0; full.leaf = 0; full.rec = nd.rec; full.chunk0 = 0; full.key = nd.key;
+            const int nc = split_rules(full, a, P.MIN, P.MAX, 0, c0, c1);
+            if (recs_all) index_split(recs_all + (size_t)tk.tree * rec_cap, &stats[tk.tree].n_rec, rec_cap, nd.rec, p1, p2, nc, c0.rec, c1.rec, ctr);
+            int n_left = n_stack - 1, n_out = n_out_s;
+            auto child = [&](const TreeNode& c) {
+                const bool forced = c.depth >= P.MAX_DEPTH - 1, split = !c.leaf && !forced && c.count > P.small;
+                SmallNode x;
+                x.start = c.start; x.count = c.count; x.dstart = c.dstart; x.dcount = c.dcount;
+                x.depth = c.depth; x.leaf = c.leaf || forced ? 1 : 0; x.rec = c.rec; x.key = c.key;
+                if (!split) out[n_out++] = x;
+                else if (n_left < stack_cap) stack[n_left++] = x;
+                else ctr->overflow = 1;
+            };
+            child(c0);
+            if (nc == 2) child(c1);
+            n_stack_s = n_left;
+            n_out_s = n_out;
+        }
+        __syncthreads();
+        if (n_out_s > kMidOut - 2) give_out();
+    }
+    for (int i = tid; i < tk.count; i += kMidThreads) dst[tk.start + i] = seg[i];
+    give_out();
+    if (tid == 0) {
+        stat_add(stat, (int)blockIdx.x, 0, seen);
+        stat_add(stat, (int)blockIdx.x, 1, unsure);
     }
 }
 
@@ -1950,6 +2154,8 @@ struct TreeBatchWorkspace {
     TreeNode* nodes[2] = {nullptr, nullptr};
     TreeNode* tail = nullptr;
     TreeNode* chain = nullptr;           // nodes for the chain phase
+    TreeNode* mid = nullptr;             // nodes for the middle phase (when there is one)
+    int mid_most = 0;                    // points of the largest of them
     int* chunk2node = nullptr;
     int* chunk_left = nullptr;
     float* planes = nullptr;             // hyperplanes of the nodes of the current wide level: node_cap x (4 + nvec_len(D))
@@ -1981,7 +2187,7 @@ struct TreeBatchWorkspace {
 
 static void free_ws(TreeBatchWorkspace& w)
 {
-    void* dev[] = {w.perm[0], w.perm[1], w.nodes[0], w.nodes[1], w.tail, w.chain, w.chunk2node,
+    void* dev[] = {w.perm[0], w.perm[1], w.nodes[0], w.nodes[1], w.tail, w.chain, w.mid, w.chunk2node,
                    w.chunk_left, w.leaf_start, w.leaf_size, w.stats, w.ctr, w.recs, w.planes,
                    w.pm_path, w.pm_side, w.pm_undec, w.pm_map[0], w.pm_map[1], w.pm_sc, w.pm_aq, w.pm_child, w.stat};
     for (void* p : dev) ws_free(p);
@@ -2031,13 +2237,27 @@ int tree_chain_max(int D, int MIN, int MAX)
     const int n = std::min(256, 8 * MIN / 3);
     return n > MAX ? n : 0;
 }
+// Largest node the middle phase takes (0: there is none): batches of few points (tree_small_threshold), and nodes whose screening
+// rows one compute unit reads in the time of a wide level, about a megabyte (12,288 points of 32 dimensions, 4,608 of 200).
+// RSFK_TREE_MID=0 switches it off, =n limits the size (tests).
+int tree_mid_most(int D, int N, int B, int small)
+{
+    if ((size_t)N * (size_t)std::max(B, 1) >= ((size_t)1 << 21)) return 0;
+    int n = std::min(kMidMost, (1 << 20) / q8_pitch(D) + 512) & ~63;
+    int least = small + small / 2;
+    if (const char* e = std::getenv("RSFK_TREE_MID")) {
+        n = std::min(n, std::atoi(e) & ~63);
+        least = small + 1;
+    }
+    return n >= least && N > small ? n : 0;
+}
 constexpr int kWideChunk = 1024;         // points per workgroup in the wide passes (k_side keeps a chunk's undecided points in LDS)
 
 // bytes of device memory a batch of B trees needs
 size_t tree_ws_bytes(int N, int D, int MIN, int B)
 {
     const size_t lc = (size_t)N / (size_t)std::max(MIN, 1) + 2;
-    return bf16_copy_bytes(N, D) + (size_t)B * ((size_t)N * 8 + (size_t)N * 2 + 512 * 1024 + lc * (8 + 2 * sizeof(TreeNode)) + ((size_t)N / 1024 + 2) * (2 * sizeof(TreeNode) + 24 + (size_t)(4 + nvec_len(D)) * 4));
+    return bf16_copy_bytes(N, D) + (size_t)B * ((size_t)N * 8 + (size_t)N * 2 + 512 * 1024 + lc * (8 + 3 * sizeof(TreeNode)) + ((size_t)N / 1024 + 2) * (2 * sizeof(TreeNode) + 24 + (size_t)(4 + nvec_len(D)) * 4));
 }
 
 // From now on every build with this workspace also writes the index of each tree (TreeRec records).
@@ -2072,6 +2292,8 @@ int tree_ws_alloc(TreeBatchWorkspace** out, int N, int D, int MIN, int B)
     if (dmalloc(&w->nodes[1], (size_t)w->node_cap)) return 1;
     if (dmalloc(&w->tail, (size_t)w->tail_cap)) return 1;
     if (dmalloc(&w->chain, (size_t)w->tail_cap)) return 1;
+    w->mid_most = tree_mid_most(D, N, B, small);
+    if (w->mid_most && dmalloc(&w->mid, (size_t)w->tail_cap)) return 1;
     if (dmalloc(&w->chunk2node, (size_t)w->chunk_cap)) return 1;
     if (dmalloc(&w->chunk_left, (size_t)w->chunk_cap)) return 1;
     if (dmalloc(&w->planes, (size_t)w->node_cap * (size_t)(4 + nvec_len(D)))) return 1;
@@ -2143,13 +2365,21 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
     }
     NodeQueues Q;
     Q.next = w->nodes[0]; Q.next_cap = w->node_cap; Q.chunk_cap = w->chunk_cap; Q.slot = 0;
-    Q.tail = w->tail; Q.tail_cap = w->tail_cap;
+    // The middle phase needs the 8-bit copy, and is for launches over few subtrees (below; RSFK_TAIL_BLOCK=256: as with many).
+    const char* tail_block = std::getenv("RSFK_TAIL_BLOCK");
+    const bool tail_q8 = q8 != nullptr && std::getenv("RSFK_TAIL_BF16") == nullptr;
+    const bool mid = w->mid_most > 0 && tail_q8 && pm_levels == 0 && !(tail_block && std::atoi(tail_block) < 1024);
+    P.mid = mid ? 1 : 0;
+    TreeParams PW = P;                                                        // of the wide levels
+    if (mid) PW.small = w->mid_most;
+    Q.tail = mid ? w->mid : w->tail; Q.tail_cap = w->tail_cap;
     Q.ctr = w->ctr;
+    Q.n_tail = mid ? &w->ctr->n_mid : &w->ctr->n_tail;
     w->notes.begin();
     {
         const size_t total = (size_t)N * nb;
         const int grid = (int)std::min<size_t>((total + 255) / 256, 65536);
-        hipLaunchKernelGGL(k_tree_init, dim3(grid), dim3(256), 0, stream, w->perm[0], Q, P, nb, seed0,
+        hipLaunchKernelGGL(k_tree_init, dim3(grid), dim3(256), 0, stream, w->perm[0], Q, PW, nb, seed0,
                            pm_levels > 0 ? w->pm_map[0] : nullptr, w->stats, w->stat);
         RSFK_HIP(hipGetLastError());
     }
@@ -2177,7 +2407,7 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
     // queued at the end; its workgroups find nothing to do.
     int n_tail = nb, level = 0;
     size_t most_nodes = (size_t)nb, most_chunks = (size_t)nb * (((size_t)N + P.chunk - 1) / P.chunk);
-    while (N > P.small) {
+    while (N > PW.small) {
         if (level > 0) {
             const LevelNote* note = w->notes.of(level - 1);
             if (wait_for_word(&note->seq, LevelNotes::seq(level - 1), stream)) return 1;
@@ -2195,7 +2425,7 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
         const int n_chunks = (int)std::min<size_t>(most_chunks, (size_t)w->chunk_cap);
         int* ctr_chunks = &w->ctr->queue[slot].chunks;
         hipLaunchKernelGGL(k_level_planes, dim3((unsigned)((most_nodes + plane_waves - 1) / plane_waves)), dim3(64 * plane_waves),
-                           plane_waves * side_lds, stream, points, P, w->perm[0], w->perm[1], w->nodes[cur], level, w->node_cap,
+                           plane_waves * side_lds, stream, points, PW, w->perm[0], w->perm[1], w->nodes[cur], level, w->node_cap,
                            w->planes, w->chunk2node, w->ctr, w->stat, w->notes.of(level), LevelNotes::seq(level));
         const bool swept = level < pm_levels;
         if (swept) {
@@ -2233,7 +2463,7 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
         const bool map_next = level + 1 < pm_levels;
         Q.next = w->nodes[cur ^ 1];
         Q.slot = (level + 1) & 3;
-        hipLaunchKernelGGL(k_scatter, dim3(n_chunks), dim3(kBlock), 0, stream, P, w->perm[0], w->perm[1], w->nodes[cur],
+        hipLaunchKernelGGL(k_scatter, dim3(n_chunks), dim3(kBlock), 0, stream, PW, w->perm[0], w->perm[1], w->nodes[cur],
                            slot, w->chunk2node, w->chunk_left, Q, w->recs, w->stats, w->rec_cap,
                            map_next ? w->pm_child : nullptr);
         if (map_next) {
@@ -2252,9 +2482,31 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
     // chain phase.  With more subtrees than that the device is full anyway and the chains run beside the rest: the
     // chain phase then only adds its matrices (1M x 100, 50 trees: tail 10.7 -> 9.0 ms, chains 6.8 ms).
     // RSFK_TAIL_BLOCK=256 / 1024: as with many / as with few subtrees, whatever their number.
-    bool few = n_tail > 0 && n_tail < 8 * 256;
-    if (const char* e = std::getenv("RSFK_TAIL_BLOCK")) few = std::atoi(e) >= 1024;
     RSFK_CHECK(n_tail <= w->tail_cap, "tree batch: tail queue overflow");
+    if (mid && n_tail > 0) {
+        const int stack_cap = w->mid_most / std::max(P.small, 1) + 4;
+        const size_t lds = (size_t)w->mid_most * 6 + (size_t)nvec_len(D) * 4 + (size_t)(stack_cap + kMidOut) * sizeof(SmallNode);
+        const int pieces = q8_padded(D) / 16;
+#define RSFK_MID_LAUNCH(L, U)                                                                                               \
+        do {                                                                                                               \
+            RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_mid<L, U>),                                       \
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));                          \
+            hipLaunchKernelGGL((k_mid<L, U>), dim3(n_tail), dim3(kMidThreads), lds, stream, points, q8, P, w->mid_most,     \
+                               w->perm[0], w->perm[1], w->perm[0], w->mid, w->tail, w->tail_cap, stack_cap, w->stats, w->ctr,  \
+                               w->recs, w->rec_cap, w->stat);                                                               \
+        } while (0)
+        if (pieces <= 2) RSFK_MID_LAUNCH(2, 1);
+        else if (pieces <= 4) RSFK_MID_LAUNCH(4, 1);
+        else if (pieces <= 16) RSFK_MID_LAUNCH(4, 4);
+        else RSFK_MID_LAUNCH(8, 4);
+#undef RSFK_MID_LAUNCH
+        RSFK_HIP(hipGetLastError());
+        // (how many nodes it leaves to the tail only the device knows; that many are usual, and the tail kernel takes any number)
+        n_tail = (int)std::min<size_t>((size_t)N * (size_t)nb * 5 / (size_t)(3 * P.small) + (size_t)nb, (size_t)w->tail_cap);
+    }
+    bool few = n_tail > 0 && n_tail < 8 * 256;
+    if (tail_block) few = std::atoi(tail_block) >= 1024;
+    if (mid) few = true;
     if (n_tail > 0) {
         // (the tail kernel keeps the bfloat16 screen: measured, it is not faster with the 8-bit one)
         // nodes of a level of a subtree (and its buckets): at most small / MIN + 1; hyperplanes kept together:
@@ -2264,7 +2516,6 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
         const size_t lds = (size_t)(2 * P.small) * 4 + (size_t)G * nvec_len(D) * 4 + (size_t)node_cap * sizeof(int2) +
                            (few ? 3 : 2) * (size_t)node_cap * sizeof(SmallNode) + (size_t)P.small;
         RSFK_CHECK(lds <= 150 * 1024, "tree batch: D too large for the tail kernel's LDS budget");
-        const bool tail_q8 = q8 != nullptr && std::getenv("RSFK_TAIL_BF16") == nullptr;
 #define RSFK_TAIL_LAUNCH(Q, T, C, L, U)                                                                                       \
         do {                                                                                                               \
             RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_tail<Q, T, C, L, U>),                                \

@@ -169,6 +169,29 @@ def test_tree_forms_of_tail_and_chain(gpu, orc, rng, monkeypatch, N, D, MIN, MAX
         assert list(gst) == [len(ls), st[0], st[1], st[2]]
 
 
+# The middle phase: nodes it takes whole (N at most its largest), from the wide levels, of sizes around a thread's last entry, one that
+# is barely larger than what the tail takes; equal rows (splits in vain up to the depth limit); leaf limits above the tail's nodes.
+@pytest.mark.parametrize("N,D,MIN,MAX,small,mid,kind", [
+    (1025, 5, 17, 34, 64, 12288, "n"), (12288, 3, 64, 256, 2048, 12288, "n"), (12289, 3, 64, 256, 2048, 12288, "n"), (30000, 32, 17, 34, 96, 1024, "n"),
+    (30000, 64, 33, 66, 128, 4096, "n"), (12000, 65, 33, 66, 128, 1088, "n"), (9000, 257, 17, 34, 64, 2048, "n"), (15000, 16, 400, 1000, 200, 12288, "n"),
+    (6000, 9, 5, 10, 64, 12288, "dup"), (5000, 4, 1, 3, 64, 12288, "n"),
+])
+def test_tree_middle_phase(gpu, orc, rng, monkeypatch, N, D, MIN, MAX, small, mid, kind):
+    monkeypatch.setenv("RSFK_TREE_SCREEN", "q8")
+    monkeypatch.setenv("RSFK_TREE_SMALL", str(small))
+    monkeypatch.setenv("RSFK_TREE_MID", str(mid))
+    X = rng.standard_normal((N, D)).astype(np.float32)
+    if kind == "dup":
+        X[: N // 3] = X[0]
+    for depth in (200, 6):
+        _say("tree middle phase", N, D, MIN, MAX, small, mid, kind, depth)
+        perm, ls, lz, st = orc.build_tree(X, MIN, MAX, depth, 3)
+        gperm, gls, glz, gst = gpu.build_tree(X, MIN, MAX, depth, 3)
+        assert np.array_equal(gperm, perm)
+        assert np.array_equal(gls, ls) and np.array_equal(glz, lz)
+        assert list(gst) == [len(ls), st[0], st[1], st[2]]
+
+
 def test_tree_edge_cases(gpu, orc, rng):
     # identical points: re-drawn until the depth limit, then one forced bucket
     X = np.ones((3000, 4), np.float32)
