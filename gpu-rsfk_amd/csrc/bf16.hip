@@ -89,7 +89,7 @@ __global__ void k_col_mean(float* __restrict__ mu, int D, float inv_n)
 
 // one wavefront per row of the 8-bit copy
 __global__ __launch_bounds__(256) void k_to_q8(const float* __restrict__ points, uint8_t* __restrict__ out,
-                                               float* __restrict__ rho_sum, int N, int D, int pitch, float c_d, float most)
+                                               float* __restrict__ rho_parts, int N, int D, int pitch, float c_d, float most)
 {
     const int lane = threadIdx.x & 63;
     const int wave_global = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
@@ -153,13 +153,14 @@ __global__ __launch_bounds__(256) void k_to_q8(const float* __restrict__ points,
             if (!bad && fmaxf(fabsf(lo), fabsf(hi)) > most) rho_acc = INFINITY;
         }
     }
-    // one atomic per workgroup (they all hit the same address)
+    // one part per workgroup, added up by fetch_sum (atomics on one address come one after the other: 14 ns each, 36 of 46 us of
+    // the copy of 20,000 x 64)
     __shared__ float part[4];
     if (lane == 0) part[threadIdx.x >> 6] = rho_acc;
     __syncthreads();
     if (threadIdx.x == 0) {
         const float t = part[0] + part[1] + part[2] + part[3];
-        if (t != 0.0f) atomicAdd(rho_sum, t);
+        rho_parts[blockIdx.x] = t;
     }
 }
 
@@ -168,16 +169,16 @@ __global__ __launch_bounds__(256) void k_to_q8(const float* __restrict__ points,
 // 16-byte pieces, and stay in registers between the pass that finds the range and the pass that rounds.  Produces the
 // bytes and headers of k_to_q8 (minimum, maximum and rounding do not depend on the order; the sum of the absolute
 // values, which only feeds the average that chooses between the screens, is added up in another order).
-// Needs D % 4 == 0 and 16-byte aligned points.
-template <int LPR, int PPL>
+// WHOLE: D % 4 == 0 and 16-byte aligned points.
+template <int LPR, int PPL, bool WHOLE>
 __global__ __launch_bounds__(256) void k_to_q8_regs(const float* __restrict__ points, uint8_t* __restrict__ out,
-                                                    float* __restrict__ rho_sum, int N, int D, int pitch, float c_d, float most)
+                                                    float* __restrict__ rho_parts, int N, int D, int pitch, float c_d, float most)
 {
     constexpr int kRowsPerWave = 64 / LPR;
     const int lane = threadIdx.x & 63, sub = lane / LPR, l = lane - sub * LPR;
     const int wave_global = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const int n_waves = (gridDim.x * blockDim.x) >> 6;
-    const int words = (pitch - 16) >> 2, pieces = D >> 2;
+    const int words = (pitch - 16) >> 2, pieces = (D + 3) >> 2;
     float rho_acc = 0.0f;
     for (int rb = wave_global * kRowsPerWave; rb < N; rb += n_waves * kRowsPerWave) {
         const int r = rb + sub;
@@ -191,10 +192,11 @@ __global__ __launch_bounds__(256) void k_to_q8_regs(const float* __restrict__ po
             const int pc = l + k * LPR;
             x[k] = make_float4(0.f, 0.f, 0.f, 0.f);
             if (row_ok && pc < pieces) {
-                x[k] = *reinterpret_cast<const float4*>(src + 4 * pc);
+                x[k] = load_dims(src + 4 * pc, D - 4 * pc, WHOLE);
                 const float v[4] = {x[k].x, x[k].y, x[k].z, x[k].w};
 #pragma unroll
                 for (int c = 0; c < 4; ++c) {
+                    if (!WHOLE && 4 * pc + c >= D) continue;
                     bad |= !(fabsf(v[c]) <= 3.0e38f);              // NaN or infinite
                     lo = fminf(lo, v[c]);
                     hi = fmaxf(hi, v[c]);
@@ -224,6 +226,7 @@ __global__ __launch_bounds__(256) void k_to_q8_regs(const float* __restrict__ po
                     const float v[4] = {x[k].x, x[k].y, x[k].z, x[k].w};
 #pragma unroll
                     for (int c = 0; c < 4; ++c) {
+                        if (!WHOLE && 4 * pc + c >= D) continue;
                         float t = __builtin_rintf((v[c] - lo) * inv);
                         t = fminf(fmaxf(t, 0.0f), 255.0f);
                         packed |= (uint32_t)t << (8 * c);
@@ -245,7 +248,6 @@ __global__ __launch_bounds__(256) void k_to_q8_regs(const float* __restrict__ po
             if (!badi && fmaxf(fabsf(lo), fabsf(hi)) > most) rho_acc = INFINITY;
         }
     }
-    // one atomic per workgroup (they all hit the same address)
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) rho_acc += __shfl_xor(rho_acc, o, 64);
     __shared__ float part[4];
@@ -253,7 +255,7 @@ __global__ __launch_bounds__(256) void k_to_q8_regs(const float* __restrict__ po
     __syncthreads();
     if (threadIdx.x == 0) {
         const float t = part[0] + part[1] + part[2] + part[3];
-        if (t != 0.0f) atomicAdd(rho_sum, t);
+        rho_parts[blockIdx.x] = t;
     }
 }
 
@@ -262,35 +264,40 @@ __global__ __launch_bounds__(256) void k_to_q8_regs(const float* __restrict__ po
 int q8_copy_alloc(Q8Copy* c, int N, int D)
 {
     if (ws_alloc(reinterpret_cast<void**>(&c->rows), std::max<size_t>((size_t)N * q8_pitch(D), 64))) return 1;
-    if (ws_alloc(reinterpret_cast<void**>(&c->rho_sum), 16)) return 1;
+    if (ws_alloc(reinterpret_cast<void**>(&c->rho_parts), kQ8MostGrid * sizeof(float))) return 1;
     return 0;
 }
 
 void q8_copy_free(Q8Copy* c)
 {
     ws_free(c->rows);
-    ws_free(c->rho_sum);
+    ws_free(c->rho_parts);
     c->rows = nullptr;
-    c->rho_sum = nullptr;
+    c->rho_parts = nullptr;
 }
 
-int q8_copy_fill(const Q8Copy& c, const float* points, int N, int D, hipStream_t stream)
+int q8_copy_fill(Q8Copy& c, const float* points, int N, int D, hipStream_t stream)
 {
-    RSFK_HIP(hipMemsetAsync(c.rho_sum, 0, sizeof(float), stream));
-    const int grid = std::min((N + 3) / 4, 4096);
     // (D/8 + D/32 + D + 32) 2^-24: chains of the screen and of the exact test, sum of the normal, rounding of lo + scale q
     const float c_d = (float)(D / 8 + D / 32 + D + 32) / 16777216.0f;
     const int pitch = q8_pitch(D), words = (pitch - 16) >> 2;
-    const bool vec_ok = (D & 3) == 0 && (reinterpret_cast<uintptr_t>(points) & 15) == 0;
+    const bool whole = (D & 3) == 0 && (reinterpret_cast<uintptr_t>(points) & 15) == 0;
+    const auto grid = [&](int rows_per_group, int most) {
+        c.n_parts = std::min((N + rows_per_group - 1) / rows_per_group, most);
+        return dim3((unsigned)c.n_parts);
+    };
 #define RSFK_Q8_REGS(L, P)                                                                                                 \
-    hipLaunchKernelGGL((k_to_q8_regs<L, P>), dim3(std::min((N + 4 * (64 / L) - 1) / (4 * (64 / L)), 8192)), dim3(256), 0,   \
-                       stream, points, c.rows, c.rho_sum, N, D, pitch, c_d, q8_most(D))
-    if (vec_ok && words <= 16) RSFK_Q8_REGS(16, 1);
-    else if (vec_ok && words <= 32) RSFK_Q8_REGS(32, 1);
-    else if (vec_ok && words <= 64) RSFK_Q8_REGS(64, 1);
-    else if (vec_ok && words <= 128) RSFK_Q8_REGS(64, 2);
-    else if (vec_ok && words <= 256) RSFK_Q8_REGS(64, 4);
-    else hipLaunchKernelGGL(k_to_q8, dim3(grid), dim3(256), 0, stream, points, c.rows, c.rho_sum, N, D, pitch, c_d, q8_most(D));
+    do {                                                                                                                   \
+        const dim3 g = grid(4 * (64 / L), kQ8MostGrid);                                                                     \
+        if (whole) hipLaunchKernelGGL((k_to_q8_regs<L, P, true>), g, dim3(256), 0, stream, points, c.rows, c.rho_parts, N, D, pitch, c_d, q8_most(D)); \
+        else hipLaunchKernelGGL((k_to_q8_regs<L, P, false>), g, dim3(256), 0, stream, points, c.rows, c.rho_parts, N, D, pitch, c_d, q8_most(D)); \
+    } while (0)
+    if (words <= 16) RSFK_Q8_REGS(16, 1);
+    else if (words <= 32) RSFK_Q8_REGS(32, 1);
+    else if (words <= 64) RSFK_Q8_REGS(64, 1);
+    else if (words <= 128) RSFK_Q8_REGS(64, 2);
+    else if (words <= 256) RSFK_Q8_REGS(64, 4);
+    else hipLaunchKernelGGL(k_to_q8, grid(4, 4096), dim3(256), 0, stream, points, c.rows, c.rho_parts, N, D, pitch, c_d, q8_most(D));
 #undef RSFK_Q8_REGS
     RSFK_HIP(hipGetLastError());
     return 0;
@@ -299,7 +306,7 @@ int q8_copy_fill(const Q8Copy& c, const float* points, int N, int D, hipStream_t
 int q8_copy_mean_rho(const Q8Copy& c, int N, float* mean_rho, hipStream_t stream)
 {
     float sum = 0.0f;
-    if (fetch_words(reinterpret_cast<const int*>(c.rho_sum), 1, reinterpret_cast<int*>(&sum), stream)) return 1;
+    if (fetch_sum(c.rho_parts, c.n_parts, &sum, stream)) return 1;
     *mean_rho = N > 0 ? sum / (float)N : 0.0f;
     return 0;
 }

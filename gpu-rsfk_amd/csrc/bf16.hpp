@@ -44,9 +44,11 @@ struct Bf16Copy {
 __host__ __device__ inline int q8_pitch(int D) { return (16 + D + 63) & ~63; }
 __host__ __device__ inline int q8_padded(int D) { return (D + 15) & ~15; }      // coordinates in whole 16-byte pieces
 
+constexpr int kQ8MostGrid = 8192;       // workgroups (and parts of the statistic) of the kernel that makes the copy
 struct Q8Copy {
     uint8_t* rows = nullptr;      // N x q8_pitch(D)
-    float* rho_sum = nullptr;     // device scalar: sum over the rows of e1 / (2^-8 mean |x_d|)
+    float* rho_parts = nullptr;   // device, n_parts of them: sums over rows of e1 / (2^-8 mean |x_d|)
+    int n_parts = 0;
 };
 
 // The screens of the side tests decide where margin > band: margin = |approximate n.x - offset|, band = what the approximation and
@@ -63,7 +65,7 @@ inline float q8_most(int D) { return 7.07e18f / __builtin_sqrtf((float)D); }
 
 int q8_copy_alloc(Q8Copy* c, int N, int D);
 void q8_copy_free(Q8Copy* c);
-int q8_copy_fill(const Q8Copy& c, const float* points, int N, int D, hipStream_t stream);
+int q8_copy_fill(Q8Copy& c, const float* points, int N, int D, hipStream_t stream);
 int q8_copy_mean_rho(const Q8Copy& c, int N, float* mean_rho, hipStream_t stream);     // synchronises the stream
 
 size_t bf16_copy_bytes(int N, int D);

@@ -32,6 +32,8 @@ int wait_for_word(const int* word, int want, hipStream_t stream);
 constexpr int kFetchMost = 8;
 int fetch_words(const int* a, int na, const int* b, int nb, int* host, hipStream_t stream);
 inline int fetch_words(const int* dev, int n, int* host, hipStream_t stream) { return fetch_words(dev, n, nullptr, 0, host, stream); }
+// ... the sum of n numbers there.
+int fetch_sum(const float* a, int n, float* host, hipStream_t stream);
 
 // Both macros leave the function on failure.  Work that was queued before may still be running and the
 // callers' guards hand their buffers back for reuse on the way out, so the device is drained first.

@@ -13,6 +13,7 @@
 #include <algorithm>
 #include <cstdlib>
 #include <map>
+#include <cstring>
 #include <mutex>
 #include <vector>
 
@@ -287,6 +288,22 @@ __global__ void k_fetch(const int* __restrict__ a, int na, const int* __restrict
     for (int i = 0; i < nb; ++i) out->word[na + i] = b[i];
     __hip_atomic_store(&out->seq, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
+// One workgroup of 256 threads.
+__global__ void k_fetch_sum(const float* __restrict__ a, int n, Fetched* out)
+{
+    __shared__ float part[256];
+    float t = 0.0f;
+    for (int i = threadIdx.x; i < n; i += 256) t += a[i];
+    part[threadIdx.x] = t;
+    __syncthreads();
+    for (int o = 128; o > 0; o >>= 1) {
+        if ((int)threadIdx.x < o) part[threadIdx.x] += part[threadIdx.x + o];
+        __syncthreads();
+    }
+    if (threadIdx.x != 0) return;
+    out->word[0] = __float_as_int(part[0]);
+    __hip_atomic_store(&out->seq, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 }  // namespace
 
 int fetch_words(const int* a, int na, const int* b, int nb, int* host, hipStream_t stream)
@@ -302,6 +319,21 @@ int fetch_words(const int* a, int na, const int* b, int nb, int* host, hipStream
     const int rc = e != hipSuccess ? 1 : wait_for_word(&f->seq, 1, stream);
     if (e != hipSuccess) set_last_error(std::string("fetch: ") + hipGetErrorString(e));
     for (int i = 0; i < n && !rc; ++i) host[i] = f->word[i];
+    pin_free(p);
+    return rc;
+}
+
+int fetch_sum(const float* a, int n, float* host, hipStream_t stream)
+{
+    void* p = nullptr;
+    if (pin_alloc(&p, sizeof(Fetched))) return 1;
+    Fetched* f = static_cast<Fetched*>(p);
+    __atomic_store_n(&f->seq, 0, __ATOMIC_RELEASE);
+    hipLaunchKernelGGL(k_fetch_sum, dim3(1), dim3(256), 0, stream, a, n, f);
+    const hipError_t e = hipGetLastError();
+    const int rc = e != hipSuccess ? 1 : wait_for_word(&f->seq, 1, stream);
+    if (e != hipSuccess) set_last_error(std::string("fetch: ") + hipGetErrorString(e));
+    if (!rc) std::memcpy(host, &f->word[0], sizeof(float));
     pin_free(p);
     return rc;
 }
