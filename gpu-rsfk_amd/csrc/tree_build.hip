@@ -1213,6 +1213,15 @@ __global__ __launch_bounds__(kMidThreads, 4) void k_mid(const float* __restrict_
     constexpr int kGroups = kMidThreads / LPP, kBatch = KU == 1 ? 4 : 2;
     const int grp = tid / LPP, sub = tid & (LPP - 1);
     int seen = 0, unsure = 0;
+    // the steps of the first workgroup stand for those of all (phase_tick)
+    const bool timed = blockIdx.x == 0 && tid == 0;
+    long long since = timed ? (long long)wall_clock64() : 0, ticks[3] = {0, 0, 0};
+    auto step = [&](int which) {
+        if (!timed) return;
+        const long long now = (long long)wall_clock64();
+        ticks[which] += now - since;
+        since = now;
+    };
     while (true) {
         const int n_stack = n_stack_s;
         if (n_stack == 0) break;
@@ -1224,6 +1233,7 @@ __global__ __launch_bounds__(kMidThreads, 4) void k_mid(const float* __restrict_
         if (wave == 0) make_hyperplane_wave(points + (size_t)p1 * P.D, points + (size_t)p2 * P.D, P.D, nvec, hp_s);
         if (tid == 64) n_def_s = 0;
         __syncthreads();
+        step(0);
         const float b = hp_s[0], n1 = hp_s[1], sn = hp_s[2];
         for (int it = 0; it * kGroups < cnt; it += kBatch) {
             int id[kBatch], jz[kBatch], pos[kBatch];
@@ -1256,6 +1266,7 @@ __global__ __launch_bounds__(kMidThreads, 4) void k_mid(const float* __restrict_
         resolve_exact(kMidThreads / 32, tid >> 5, list, n_def, nvec, 0, hp_s, points, P.D, [&](int pos) { return seg[st + pos] & kIdMask; },
                       [&](int pos, bool right) { if (right) seg[st + pos] |= (int)0x80000000; });
         __syncthreads();
+        step(1);
         // stable partition: a thread's entries are at tid, tid + 1024, ..; they wait in registers while the lefts of every 64 are counted
         int v[kMidPer];
 #pragma unroll
@@ -1318,9 +1329,14 @@ __global__ __launch_bounds__(kMidThreads, 4) void k_mid(const float* __restrict_
         }
         __syncthreads();
         if (n_out_s > kMidOut - 2) give_out();
+        step(2);
     }
     for (int i = tid; i < tk.count; i += kMidThreads) dst[tk.start + i] = seg[i];
     give_out();
+    if (timed) {
+        for (int k = 0; k < 3; ++k) ctr->phase_ticks[k] += ticks[k];
+        ctr->last_tick = (long long)wall_clock64();
+    }
     if (tid == 0) {
         stat_add(stat, (int)blockIdx.x, 0, seen);
         stat_add(stat, (int)blockIdx.x, 1, unsure);
