@@ -145,7 +145,7 @@ int explore_ws_alloc(ExploreWorkspace** out, int N, int K, bool with_bounds = fa
 bool explore_ws_takes(int N, int K);
 int launch_reversed_graph(ExploreWorkspace* w, const int* idx, int N, int K, hipStream_t stream);
 const int* explore_ws_offs(const ExploreWorkspace* w);       // N + 1
-const int* explore_ws_rev(const ExploreWorkspace* w);        // entry numbers p K + k, in compressed rows by the neighbour
+int* explore_ws_rev(const ExploreWorkspace* w);        // entry numbers p K + k, in compressed rows by the neighbour
 void explore_ws_free(ExploreWorkspace* w);
 const uint32_t* explore_ws_pass(const ExploreWorkspace* w);
 const uint16_t* explore_ws_bounds(const ExploreWorkspace* w);
