@@ -219,47 +219,138 @@ __device__ __forceinline__ uint64_t in_own(const int* own, int n, int c)
     return m;
 }
 
-// len[p] = entries of row p; len[N] = 0.
+// A wavefront takes PTS consecutive points, whose stored neighbours and reversed entries follow each other in memory: what such a
+// wavefront waits for is its trips (offsets, then rows and reversed entries, then distances), not bytes or instructions (1M x 32, one
+// point per wavefront: lengths 0.30 ms, rows 0.53; four: 0.18 and 0.32.  With 4 or 16 slots per neighbour the lengths take 0.23 and 0.26).
+inline int union_points(int K) { return K <= 32 ? 4 : (K <= 64 ? 2 : 1); }
+
+// The stored neighbours of a point as a table in LDS of 2^bits slots, 8 per neighbour: of those that fall on the same slot the last one
+// written is there, the others (two per row of 32) are listed.  Whether a column is among them is one read, where comparing it
+// with all of them takes 104 instructions at K = 32.
+constexpr int kTableMostK = 128;
+inline int table_bits(int K)
+{
+    int bits = 4;
+    while ((1 << bits) < 8 * K) ++bits;
+    return bits;
+}
+__device__ __forceinline__ int table_slot(int c, int bits) { return (int)(((uint32_t)c * 2654435761u) >> (32 - bits)); }
+
+// len[p] = entries of row p; len[N] = 0.  Entries of the reversed graph that add nothing to row p get bit 31 in rev.
+// TABLE: PTS K at most kTableMostK; LDS of a wavefront: PTS tables, listed neighbours and the points they belong to [2 PTS K].
+// Otherwise PTS = 1, and the stored neighbours are in LDS as they are.
+template <int PTS, bool TABLE>
 __global__ __launch_bounds__(256) void k_union_len(const int* __restrict__ idx, int N, int K, int drop_self, const int* __restrict__ offs,
-                                                   const int* __restrict__ rev, uint32_t div_m, int div_s, int own_ints,
+                                                   int* __restrict__ rev, uint32_t div_m, int div_s, int lds_ints, int bits,
                                                    int* __restrict__ len, UnionLists L)
 {
     extern __shared__ __align__(16) int union_lds[];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int p = (int)blockIdx.x * 4 + wave;
-    if (p >= N) {
-        if (p == N && lane == 0) len[N] = 0;
-        return;
-    }
-    int* own = union_lds + wave * own_ints;
-    const int r0 = offs[p], r1 = offs[p + 1];
-    const int e0 = r0 + lane < r1 ? rev[r0 + lane] : -1;
-    const int n = own_edges(idx, N, K, p, drop_self, own);
-    wave_lds_sync();
-    int total = n;
-    auto count = [&](int e) {
-        const int c = (int)(((uint64_t)(uint32_t)e * div_m) >> div_s);
-        const bool ok = e >= 0 && !(drop_self && c == p);
-        total += __popcll(ballot64(ok) & ~in_own(own, n, c));
+    const int p0 = ((int)blockIdx.x * 4 + wave) * PTS;
+    if (p0 == 0 && lane == 0) len[N] = 0;
+    if (p0 >= N) return;
+    int* own = union_lds + wave * lds_ints;
+    int* listed = own + (PTS << bits);
+    const int off = offs[min(p0 + min(lane, PTS), N)];
+    int at[PTS + 1];
+#pragma unroll
+    for (int j = 0; j <= PTS; ++j) at[j] = read_lane_i(off, j);
+    const int r0 = at[0], r1 = at[PTS];
+    constexpr int kAhead = 4;
+    int e[kAhead];
+    auto request = [&](int r) {
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) e[u] = r + 64 * u + lane < r1 ? rev[r + 64 * u + lane] : -1;
     };
-    if (r0 < r1) count(e0);
-    // (eight loads at a time: R(p) of a hub is long)
-    for (int r = r0 + 64; r < r1; r += 512) {
-        int e[8];
+    request(r0);
+    int n[PTS], n_listed = 0;
 #pragma unroll
-        for (int u = 0; u < 8; ++u) e[u] = r + 64 * u + lane < r1 ? rev[r + 64 * u + lane] : -1;
+    for (int j = 0; j < PTS; ++j) n[j] = 0;
+    if constexpr (TABLE) {
+        constexpr int kOwn = kTableMostK / 64;
+        int c[kOwn], mine[kOwn];
+        bool ok[kOwn];
 #pragma unroll
-        for (int u = 0; u < 8; ++u)
-            if (r + 64 * u < r1) count(e[u]);
-    }
-    if (lane == 0) {
-        len[p] = total;
-        if (n + (r1 - r0) > kUnionBlock) {
-            const unsigned long long was = atomicAdd(reinterpret_cast<unsigned long long*>(&L.ctr->hubs), (unsigned)total | (1ull << 32));
-            L.hubs[was >> 32] = make_int2(p, (int)(unsigned)was);
-        } else if (total > kUnionWave) {
-            L.big[atomicAdd(&L.ctr->n_big, 1)] = p;
+        for (int v = 0; v < kOwn; ++v) {
+            const int i = lane + 64 * v;
+            mine[v] = PTS == 1 ? 0 : (int)(((uint64_t)(uint32_t)i * div_m) >> div_s);       // i / K
+            const bool in = i < PTS * K && p0 + mine[v] < N;
+            c[v] = in ? idx[(size_t)p0 * K + i] : -1;
         }
+        for (int i = 4 * lane; i < (PTS << bits); i += 256) *reinterpret_cast<int4*>(own + i) = make_int4(-1, -1, -1, -1);
+#pragma unroll
+        for (int v = 0; v < kOwn; ++v) {
+            ok[v] = usable(c[v], p0 + mine[v], N, drop_self);
+#pragma unroll
+            for (int j = 0; j < PTS; ++j) n[j] += __popcll(ballot64(ok[v] && (PTS == 1 || mine[v] == j)));
+        }
+        wave_lds_sync();
+#pragma unroll
+        for (int v = 0; v < kOwn; ++v)
+            if (ok[v]) own[(mine[v] << bits) + table_slot(c[v], bits)] = c[v];
+        wave_lds_sync();
+#pragma unroll
+        for (int v = 0; v < kOwn; ++v) {
+            const uint64_t lost = ballot64(ok[v] && own[((ok[v] ? mine[v] : 0) << bits) + table_slot(c[v], bits)] != c[v]);
+            if (lost == 0) continue;
+            if (lane_bit(lost)) {
+                const int slot = n_listed + mask_prefix(lost);
+                listed[2 * slot] = c[v];
+                listed[2 * slot + 1] = mine[v];
+            }
+            n_listed += __popcll(lost);
+        }
+    } else {
+        n[0] = own_edges(idx, N, K, p0, drop_self, own);
+    }
+    wave_lds_sync();
+    int total[PTS];
+#pragma unroll
+    for (int j = 0; j < PTS; ++j) total[j] = n[j];
+    for (int r = r0; r < r1; r += 64 * kAhead) {
+        int now[kAhead];
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) now[u] = e[u];
+        if (r + 64 * kAhead < r1) request(r + 64 * kAhead);
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            if (r + 64 * u >= r1) continue;
+            const int place = r + 64 * u + lane;
+            int j = 0;
+#pragma unroll
+            for (int x = 1; x < PTS; ++x) j += place >= at[x] ? 1 : 0;
+            const int c = (int)(((uint64_t)(uint32_t)now[u] * div_m) >> div_s);
+            const uint64_t here = ballot64(now[u] >= 0);
+            uint64_t not_new;
+            if constexpr (TABLE) {
+                not_new = ballot64(own[(j << bits) + table_slot(c, bits)] == c);
+                for (int l = 0; l < n_listed; ++l) not_new |= ballot64(listed[2 * l] == c && (PTS == 1 || listed[2 * l + 1] == j));
+            } else {
+                not_new = in_own(own, n[0], c);
+            }
+            if (drop_self) not_new |= ballot64(c == p0 + j);
+            not_new &= here;
+            if (lane_bit(not_new)) rev[place] = now[u] | (int)0x80000000;
+#pragma unroll
+            for (int x = 0; x < PTS; ++x) total[x] += __popcll(here & ~not_new & (PTS == 1 ? ~0ull : ballot64(j == x)));
+        }
+    }
+    // lane j: the result of point p0 + j
+    int mine = total[0], seen = n[0] + at[1] - at[0];
+#pragma unroll
+    for (int j = 1; j < PTS; ++j)
+        if (lane == j) {
+            mine = total[j];
+            seen = n[j] + at[j + 1] - at[j];
+        }
+    const int p = p0 + lane;
+    if (lane >= PTS || p >= N) return;
+    len[p] = mine;
+    if (seen > kUnionBlock) {
+        const unsigned long long was = atomicAdd(reinterpret_cast<unsigned long long*>(&L.ctr->hubs), (unsigned)mine | (1ull << 32));
+        L.hubs[was >> 32] = make_int2(p, (int)(unsigned)was);
+    } else if (mine > kUnionWave) {
+        L.big[atomicAdd(&L.ctr->n_big, 1)] = p;
     }
 }
 
@@ -299,22 +390,13 @@ __device__ __forceinline__ void rank_and_store(const int* key, const int* entry,
 // Row p from the stored neighbours and the reversed entries that are not among them (a wavefront each).  What bounds it: the
 // gather of the reversed entries' distances (one 4-byte word per added edge) and the comparisons (two instructions per
 // column and lane).
-__global__ __launch_bounds__(256) void k_union_fill(const int* __restrict__ idx, const float* __restrict__ dist, int N, int K,
-                                                    int drop_self, const int* __restrict__ offs, const int* __restrict__ rev,
-                                                    uint32_t div_m, int div_s, int own_ints, const int* __restrict__ indptr,
-                                                    long long cap, int* __restrict__ cols, float* __restrict__ vals)
+// (r0, r1: its reversed entries; row0, n_row: its place in the result; key, entry: kUnionWave + 4 each)
+__device__ __forceinline__ void union_row(const int* __restrict__ idx, const float* __restrict__ dist, int N, int K, int drop_self, int p,
+                                          int r0, int r1, const int* __restrict__ rev, uint32_t div_m, int div_s, int row0, int n_row, int* key,
+                                          int* entry, int* __restrict__ cols, float* __restrict__ vals)
 {
-    extern __shared__ __align__(16) int union_lds[];
-    if (indptr[N] > cap) return;                                        // (the host reports)
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int p = (int)blockIdx.x * 4 + wave;
-    if (p >= N) return;
-    const int row0 = indptr[p], n_row = indptr[p + 1] - row0;
     if (n_row == 0 || n_row > kUnionWave) return;
-    int* own = union_lds + wave * (own_ints + 2 * (kUnionWave + 4));
-    int* key = own + own_ints;
-    int* entry = key + kUnionWave + 4;
-    const int r0 = offs[p], r1 = offs[p + 1];
+    const int lane = threadIdx.x & 63;
     const int e0 = r0 + lane < r1 ? rev[r0 + lane] : -1;
     int n = 0;
     for (int k0 = 0; k0 < K; k0 += 64) {
@@ -324,20 +406,16 @@ __global__ __launch_bounds__(256) void k_union_fill(const int* __restrict__ idx,
         const uint64_t m = ballot64(ok);
         if (ok) {
             const int at = n + mask_prefix(m);
-            own[at] = c;
             key[at] = c;
             entry[at] = p * K + k;
         }
         n += __popcll(m);
     }
-    if (lane < 4) own[n + lane] = -1;
-    wave_lds_sync();
     int total = n;
     for (int r = r0; r < r1; r += 64) {
         const int e = r == r0 ? e0 : (r + lane < r1 ? rev[r + lane] : -1);
         const int c = (int)(((uint64_t)(uint32_t)e * div_m) >> div_s);
-        const bool ok = e >= 0 && !(drop_self && c == p);
-        const uint64_t m = ballot64(ok) & ~in_own(own, n, c);
+        const uint64_t m = ballot64(e >= 0);                             // (k_union_len has marked those that add nothing)
         if (lane_bit(m)) {
             const int at = total + mask_prefix(m);
             key[at] = c;
@@ -350,6 +428,149 @@ __global__ __launch_bounds__(256) void k_union_fill(const int* __restrict__ idx,
     if (n_row <= 64) rank_and_store<1>(key, entry, n_row, dist, cols + row0, vals + row0);
     else if (n_row <= 128) rank_and_store<2>(key, entry, n_row, dist, cols + row0, vals + row0);
     else rank_and_store<4>(key, entry, n_row, dist, cols + row0, vals + row0);
+}
+
+__global__ __launch_bounds__(256) void k_union_fill(const int* __restrict__ idx, const float* __restrict__ dist, int N, int K,
+                                                    int drop_self, const int* __restrict__ offs, const int* __restrict__ rev,
+                                                    uint32_t div_m, int div_s, const int* __restrict__ indptr,
+                                                    long long cap, int* __restrict__ cols, float* __restrict__ vals)
+{
+    __shared__ __align__(16) int lds[4][2 * (kUnionWave + 4)];
+    if (indptr[N] > cap) return;                                        // (the host reports)
+    const int wave = threadIdx.x >> 6, p = (int)blockIdx.x * 4 + wave;
+    if (p >= N) return;
+    const int row0 = indptr[p];
+    union_row(idx, dist, N, K, drop_self, p, offs[p], offs[p + 1], rev, div_m, div_s, row0, indptr[p + 1] - row0, lds[wave],
+              lds[wave] + kUnionWave + 4, cols, vals);
+}
+
+// The same for PTS points per wavefront, PTS K <= 128, whose rows have at most kUnionWave entries and kUnionFew together (others go one by
+// one, as above).  LDS of a wavefront: keys and entries, each row from a multiple of four on.
+constexpr int kUnionFew = 448;
+template <int PTS>
+__global__ __launch_bounds__(256) void k_union_fill_few(const int* __restrict__ idx, const float* __restrict__ dist, int N, int K,
+                                                        int drop_self, const int* __restrict__ offs, const int* __restrict__ rev,
+                                                        uint32_t div_m, int div_s, const int* __restrict__ indptr,
+                                                        long long cap, int* __restrict__ cols, float* __restrict__ vals)
+{
+    constexpr int kRoom = kUnionFew + 4 * PTS;
+    __shared__ __align__(16) int lds[4][2 * kRoom];
+    if (indptr[N] > cap) return;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int p0 = ((int)blockIdx.x * 4 + wave) * PTS;
+    if (p0 >= N) return;
+    int* key = lds[wave];
+    int* entry = key + kRoom;
+    const int off = offs[min(p0 + min(lane, PTS), N)], ind = indptr[min(p0 + min(lane, PTS), N)];
+    int at[PTS + 1], row[PTS + 1], first[PTS + 1];                       // reversed entries, rows in the result, rows in LDS
+    bool few = true;
+    first[0] = 0;
+#pragma unroll
+    for (int j = 0; j <= PTS; ++j) {
+        at[j] = read_lane_i(off, j);
+        row[j] = read_lane_i(ind, j);
+        if (j > 0) {
+            first[j] = first[j - 1] + ((row[j] - row[j - 1] + 3) & ~3);
+            few = few && row[j] - row[j - 1] <= kUnionWave;
+        }
+    }
+    if (!few || row[PTS] - row[0] > kUnionFew) {
+        for (int j = 0; j < PTS; ++j) {
+            wave_lds_sync();
+            if (p0 + j < N) union_row(idx, dist, N, K, drop_self, p0 + j, at[j], at[j + 1], rev, div_m, div_s, row[j], row[j + 1] - row[j], key, entry, cols, vals);
+        }
+        return;
+    }
+    const int r1 = at[PTS];
+    constexpr int kOwn = 2, kAhead = 4;
+    int c[kOwn], mine[kOwn], e[kAhead];
+#pragma unroll
+    for (int v = 0; v < kOwn; ++v) {
+        const int i = lane + 64 * v;
+        mine[v] = (int)(((uint64_t)(uint32_t)i * div_m) >> div_s);
+        c[v] = i < PTS * K && p0 + mine[v] < N ? idx[(size_t)p0 * K + i] : -1;
+    }
+    auto request = [&](int r) {
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) e[u] = r + 64 * u + lane < r1 ? rev[r + 64 * u + lane] : -1;
+    };
+    request(at[0]);
+    int next[PTS];                                                       // where the next entry of a row goes
+#pragma unroll
+    for (int j = 0; j < PTS; ++j) next[j] = first[j];
+    auto put = [&](bool ok, int j, int col, int ent) {
+        int to = 0;
+#pragma unroll
+        for (int x = 0; x < PTS; ++x) {
+            const uint64_t m = ballot64(ok && j == x);
+            to = j == x ? next[x] + mask_prefix(m) : to;
+            next[x] += __popcll(m);
+        }
+        if (ok) {
+            key[to] = col;
+            entry[to] = ent;
+        }
+    };
+#pragma unroll
+    for (int v = 0; v < kOwn; ++v) put(usable(c[v], p0 + mine[v], N, drop_self), mine[v], c[v], p0 * K + lane + 64 * v);
+    for (int r = at[0]; r < r1; r += 64 * kAhead) {
+        int now[kAhead];
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) now[u] = e[u];
+        if (r + 64 * kAhead < r1) request(r + 64 * kAhead);
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            if (r + 64 * u >= r1) continue;
+            const int place = r + 64 * u + lane;
+            int j = 0;
+#pragma unroll
+            for (int x = 1; x < PTS; ++x) j += place >= at[x] ? 1 : 0;
+            put(now[u] >= 0, j, (int)(((uint64_t)(uint32_t)now[u] * div_m) >> div_s), now[u]);
+        }
+    }
+    // (what fills a row up to a multiple of four counts for nobody)
+#pragma unroll
+    for (int j = 0; j < PTS; ++j)
+        if (lane < first[j + 1] - next[j]) key[next[j] + lane] = 0x7fffffff;
+    wave_lds_sync();
+    const int n = first[PTS];
+    for (int i0 = 0; i0 < n; i0 += 128) {
+        int k[2], rank[2], to[2], s0[2], s1[2];
+        float v[2];
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+            const int i = i0 + 64 * x + lane;
+            k[x] = i < n ? key[i] : 0x7fffffff;
+            v[x] = k[x] != 0x7fffffff && dist ? dist[entry[i]] : 0.0f;
+            rank[x] = 0;
+            to[x] = row[0];
+            s0[x] = 0;
+            s1[x] = first[1];
+#pragma unroll
+            for (int y = 1; y < PTS; ++y)
+                if (i >= first[y]) {
+                    to[x] = row[y];
+                    s0[x] = first[y];
+                    s1[x] = first[y + 1];
+                }
+            if (k[x] == 0x7fffffff) s1[x] = s0[x];
+        }
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+            for (int j = s0[x]; j < s1[x]; j += 4) {
+                const int4 o = *reinterpret_cast<const int4*>(key + j);
+                rank[x] += o.x < k[x] ? 1 : 0;
+                rank[x] += o.y < k[x] ? 1 : 0;
+                rank[x] += o.z < k[x] ? 1 : 0;
+                rank[x] += o.w < k[x] ? 1 : 0;
+            }
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+            if (k[x] != 0x7fffffff) {
+                cols[to[x] + rank[x]] = k[x];
+                vals[to[x] + rank[x]] = v[x];
+            }
+    }
 }
 
 // Rows of more than kUnionWave entries: all candidates (column << 32 | entry number, stored neighbours before reversed entries
@@ -379,7 +600,7 @@ __global__ __launch_bounds__(256) void k_union_fill_big(const int* __restrict__ 
         for (int r = r0 + tid; r < r1; r += 256) {
             const int e = rev[r];
             const int c = (int)(((uint64_t)(uint32_t)e * div_m) >> div_s);
-            if (!(drop_self && c == p)) a[atomicAdd(&n_s, 1)] = ((unsigned long long)(unsigned)c << 32) | 0x80000000ull | (unsigned)e;
+            if (e >= 0) a[atomicAdd(&n_s, 1)] = ((unsigned long long)(unsigned)c << 32) | 0x80000000ull | (unsigned)e;
         }
         __syncthreads();
         const int n = n_s;
@@ -433,16 +654,12 @@ __global__ void k_union_zero(UnionCounters* ctr)
 // of 300,000 each 14.5 (72), 100,000 x 16 with one hub of 6,000 0.198 (0.416).
 __global__ __launch_bounds__(256) void k_hub_gather(const int* __restrict__ idx, const float* __restrict__ dist, int N, int K,
                                                     int drop_self, const int* __restrict__ offs, const int* __restrict__ rev,
-                                                    uint32_t div_m, int div_s, int own_ints, const int2* __restrict__ hubs, int col_bits,
+                                                    uint32_t div_m, int div_s, const int2* __restrict__ hubs, int col_bits,
                                                     int* __restrict__ cursor, unsigned long long* __restrict__ keys,
                                                     float* __restrict__ vals)
 {
-    extern __shared__ __align__(16) int union_lds[];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int h = blockIdx.x, p = hubs[h].x, first = hubs[h].y;
-    int* own = union_lds + wave * own_ints;
-    const int n = own_edges(idx, N, K, p, drop_self, own);
-    wave_lds_sync();
     const unsigned long long row = (unsigned long long)(unsigned)h << col_bits;
     auto put = [&](bool keep, int c, int e) {
         const uint64_t m = ballot64(keep);
@@ -464,8 +681,7 @@ __global__ __launch_bounds__(256) void k_hub_gather(const int* __restrict__ idx,
     for (int r = offs[p] + ((int)blockIdx.y * 4 + wave) * 64; r < r1; r += step) {
         const int e = r + lane < r1 ? rev[r + lane] : -1;
         const int c = (int)(((uint64_t)(uint32_t)e * div_m) >> div_s);
-        const bool ok = e >= 0 && !(drop_self && c == p);
-        put(lane_bit(ballot64(ok) & ~in_own(own, n, c)), c, e);
+        put(e >= 0, c, e);
     }
 }
 
@@ -542,15 +758,23 @@ int symmetrize(const int* d_idx, const float* d_dist, int N, int K, int drop_sel
     hipLaunchKernelGGL(k_union_zero, dim3(1), dim3(1), 0, stream, L.ctr);
     if (launch_reversed_graph(rg.w, d_idx, N, K, stream)) return 1;
     const int* offs = explore_ws_offs(rg.w);
-    const int* rev = explore_ws_rev(rg.w);
+    int* rev = explore_ws_rev(rg.w);
     // e / K for 0 <= e < 2^30
     int l = 0;
     while ((1 << l) < K) ++l;
     const int div_s = 31 + l;
     const uint32_t div_m = (uint32_t)((((uint64_t)1 << div_s) + (uint64_t)K - 1) / (uint64_t)K);
-    const int own_ints = (K + 4 + 3) & ~3;
-    hipLaunchKernelGGL(k_union_len, dim3((unsigned)(N / 4 + 1)), dim3(256), (size_t)4 * own_ints * sizeof(int), stream, d_idx, N, K,
-                       drop_self, offs, rev, div_m, div_s, own_ints, static_cast<int*>(len.p), L);
+    const int pts = union_points(K), bits = table_bits(K);
+    const unsigned grid = (unsigned)((N + 4 * pts - 1) / (4 * pts));
+    const int len_ints = K <= kTableMostK ? (pts << bits) + ((2 * pts * K + 3) & ~3) : (K + 4 + 3) & ~3;
+#define RSFK_UNION_LEN(PTS, TABLE)                                                                                          \
+    hipLaunchKernelGGL((k_union_len<PTS, TABLE>), dim3(grid), dim3(256), (size_t)4 * len_ints * sizeof(int), stream, d_idx, N, K,  \
+                       drop_self, offs, rev, div_m, div_s, len_ints, TABLE ? bits : 0, static_cast<int*>(len.p), L)
+    if (pts == 4) RSFK_UNION_LEN(4, true);
+    else if (pts == 2) RSFK_UNION_LEN(2, true);
+    else if (K <= kTableMostK) RSFK_UNION_LEN(1, true);
+    else RSFK_UNION_LEN(1, false);
+#undef RSFK_UNION_LEN
     RSFK_HIP(hipGetLastError());
     size_t tmp_bytes = 0;
     RSFK_HIP(rocprim::exclusive_scan(nullptr, tmp_bytes, static_cast<int*>(len.p), d_indptr, 0, (size_t)N + 1,
@@ -560,9 +784,15 @@ int symmetrize(const int* d_idx, const float* d_dist, int N, int K, int drop_sel
     RSFK_HIP(rocprim::exclusive_scan(tmp.p, tmp_bytes, static_cast<int*>(len.p), d_indptr, 0, (size_t)N + 1,
                                      rocprim::plus<int>(), stream));
     const auto fill = [&]() -> int {
-        const size_t lds = (size_t)4 * (own_ints + 2 * (kUnionWave + 4)) * sizeof(int);
-        hipLaunchKernelGGL(k_union_fill, dim3((unsigned)((N + 3) / 4)), dim3(256), lds, stream, d_idx, d_dist, N, K, drop_self, offs, rev,
-                           div_m, div_s, own_ints, d_indptr, out.cap, out.cols, out.vals);
+        if (pts == 4)
+            hipLaunchKernelGGL(k_union_fill_few<4>, dim3(grid), dim3(256), 0, stream, d_idx, d_dist, N, K, drop_self, offs, rev, div_m, div_s,
+                               d_indptr, out.cap, out.cols, out.vals);
+        else if (pts == 2)
+            hipLaunchKernelGGL(k_union_fill_few<2>, dim3(grid), dim3(256), 0, stream, d_idx, d_dist, N, K, drop_self, offs, rev, div_m, div_s,
+                               d_indptr, out.cap, out.cols, out.vals);
+        else
+            hipLaunchKernelGGL(k_union_fill, dim3(grid), dim3(256), 0, stream, d_idx, d_dist, N, K, drop_self, offs, rev, div_m, div_s,
+                               d_indptr, out.cap, out.cols, out.vals);
         hipLaunchKernelGGL(k_union_fill_big, dim3(256), dim3(256), 0, stream, d_idx, d_dist, N, K, drop_self, offs, rev, div_m, div_s,
                            d_indptr, L, out.cap, out.cols, out.vals);
         RSFK_HIP(hipGetLastError());
@@ -597,8 +827,8 @@ int symmetrize(const int* d_idx, const float* d_dist, int N, int K, int drop_sel
         // about 2,000 workgroups over all hubs, each with 1,024 entries of R(p) or more
         const size_t mean = n_entries / (size_t)n_hubs;
         const unsigned shares = (unsigned)std::max<size_t>(1, std::min<size_t>(mean / 1024, (size_t)(2048 / std::min(n_hubs, 2048))));
-        hipLaunchKernelGGL(k_hub_gather, dim3((unsigned)n_hubs, shares), dim3(256), (size_t)4 * own_ints * sizeof(int), stream, d_idx, d_dist,
-                           N, K, drop_self, offs, rev, div_m, div_s, own_ints, L.hubs, col_bits, static_cast<int*>(cursor.p), key[0], val[0]);
+        hipLaunchKernelGGL(k_hub_gather, dim3((unsigned)n_hubs, shares), dim3(256), 0, stream, d_idx, d_dist,
+                           N, K, drop_self, offs, rev, div_m, div_s, L.hubs, col_bits, static_cast<int*>(cursor.p), key[0], val[0]);
         RSFK_HIP(hipGetLastError());
         size_t sort_bytes = 0;
         RSFK_HIP(rocprim::radix_sort_pairs(nullptr, sort_bytes, key[0], key[1], val[0], val[1], n_entries, 0, (unsigned)(col_bits + hub_bits), stream));

@@ -442,6 +442,21 @@ def test_explore_matches_oracle(gpu, orc, rng, monkeypatch, N, D, K, self_in, jo
         assert not (gi == np.arange(N)[:, None]).any()
 
 
+@pytest.mark.parametrize("N,D,K", [(6000, 20, 16), (3000, 48, 90), (20001, 6, 5)])
+def test_explore_with_the_reversed_graph_by_tiles(gpu, orc, rng, monkeypatch, N, D, K):
+    """RSFK_REV_STAGED=2: the builder of medium graphs, bins of one point to 32, more than a tile of entries per part."""
+    monkeypatch.setenv("RSFK_REV_STAGED", "2")
+    X = rng.random((N, D), dtype=np.float32)
+    oi, od = orc.init_lists(N, K, self_in=True)
+    perm, ls, lz, _ = orc.build_tree(X, K + 1, 2 * K + 2, 5000, 0)
+    orc.bucket_knn(X, K, perm, lz, oi, od, starts=ls)
+    gi, gd = oi.copy(), od.copy()
+    _say("explore tiles", N, D, K)
+    orc.explore(X, K, oi, od)
+    gpu.explore(X, K, gi, gd, 1)
+    assert_knn_equal(gi, gd, oi, od)
+
+
 # ---------------------------------------------------------------------------
 # the whole call, through the entry points the Python package binds
 # ---------------------------------------------------------------------------
@@ -1085,6 +1100,34 @@ def test_symmetric_graph_with_hubs_matches_oracle(gpu, orc, rng, monkeypatch, N,
     _say("symmetrize with hubs", N, K, hubs, drop_self)
     gp, gc, gv = gpu_rsfk.symmetric_knn_graph(idx, val, drop_self=drop_self)
     op, oc, ov = orc.symmetrize(idx, val, drop_self=drop_self)
+    assert np.array_equal(gp, op) and np.array_equal(gc, oc) and np.array_equal(gv, ov)
+
+
+# The forms of the row lengths and rows: four, two and one point per wavefront (K up to 32, 64 and beyond), stored neighbours as a table
+# or as they are (K above 128), a last wavefront with points beyond N, rows on either side of what a wavefront takes together, hubs; the
+# reversed graph by tiles (RSFK_REV_STAGED=2) and entry by entry.
+@pytest.mark.parametrize("N,K,hubs", [(4001, 1, 0), (4003, 31, 2), (4001, 32, 0), (3001, 33, 2), (3001, 64, 0), (2999, 65, 3), (3001, 128, 0), (2801, 129, 2),
+                                      (40000, 8, 5)])
+@pytest.mark.parametrize("staged", ["0", "2"])
+def test_symmetric_graph_forms(gpu, orc, rng, monkeypatch, N, K, hubs, staged):
+    import gpu_rsfk
+    monkeypatch.setenv("RSFK_GRAPH_FLAGS", "0")
+    monkeypatch.setenv("RSFK_REV_STAGED", staged)
+    idx = ((np.arange(N)[:, None] + np.cumsum(rng.integers(1, 4, (N, K)), axis=1)) % N).astype(np.int32)
+    back = rng.random((N, K)) < 0.5                             # (half of the neighbours on the other side: mutual edges)
+    idx = np.where(back, (2 * np.arange(N)[:, None] - idx) % N, idx).astype(np.int32)
+    for p in range(N):
+        if len(np.unique(idx[p])) < K:
+            idx[p] = (p + 1 + np.arange(K)) % N
+    for h in range(hubs):
+        put = (rng.random(N) < (0.02, 0.2, 0.7)[h % 3]) & ~(idx == h).any(1)
+        idx[put, h % K] = h
+    idx[rng.random((N, K)) < 0.02] = -1
+    a, b = np.minimum(idx, np.arange(N)[:, None]).astype(np.int64), np.maximum(idx, np.arange(N)[:, None])
+    val = ((a * 7919 + b * 104729) % 10007).astype(np.float32)  # one value per pair
+    _say("symmetrize forms", N, K, hubs, staged)
+    gp, gc, gv = gpu_rsfk.symmetric_knn_graph(idx, val, drop_self=True)
+    op, oc, ov = orc.symmetrize(idx, val, drop_self=True)
     assert np.array_equal(gp, op) and np.array_equal(gc, oc) and np.array_equal(gv, ov)
 
 
