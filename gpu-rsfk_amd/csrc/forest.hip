@@ -609,18 +609,20 @@ int knn_forest_host(int n_trees, int K, int N, int D, int MIN, int MAX, int MAX_
     if (ws_alloc(&dd.p, nk * sizeof(float))) return 1;
     const HostArray arrays[] = {{dp.p, const_cast<float*>(points), nd * sizeof(float)}, {di.p, knn_idx, nk * sizeof(int)},
                                 {dd.p, knn_dist, nk * sizeof(float)}};
+    HostResult result;
     if (stage.to_device(arrays, fresh_rows ? 1 : 3, nullptr)) return 1;
     if (fresh_rows) {
         const unsigned grid = (unsigned)std::min<size_t>((nk + 255) / 256, 65536);
         hipLaunchKernelGGL(k_fresh_rows, dim3(grid), dim3(256), 0, nullptr, static_cast<int*>(di.p), static_cast<float*>(dd.p),
                            nk, K, fresh_rows == 2 ? 1 : 0);
         RSFK_HIP(hipGetLastError());
+        result.begin(arrays + 1, 2);
     }
     const int rc = knn_forest_device(n_trees, K, N, D, MIN, MAX, MAX_DEPTH, verbose, seed, nnef,
                                      static_cast<const float*>(dp.p), static_cast<int*>(di.p),
                                      static_cast<float*>(dd.p), log_forest, nullptr);
     if (rc) return rc;
-    return copy_to_host(arrays + 1, 2, nullptr);
+    return result.finish(arrays + 1, 2, nullptr);
 }
 
 // One tree; results on the host.  perm: N ints; leaves sorted by start.

@@ -1,6 +1,8 @@
 // Internal interfaces between the translation units of the library.
 #pragma once
 #include "rsfk_common.hpp"
+#include <atomic>
+#include <thread>
 #include "bf16.hpp"
 #include <vector>
 
@@ -133,6 +135,21 @@ private:
 };
 // Everything queued on the stream first, then the copies; complete on return.
 int copy_to_host(const HostArray* a, int n, hipStream_t stream);
+// The same for results into arrays that may be fresh: begin() once the call's work has started (addresses and sizes on the host count),
+// so that a thread makes the arrays' pages while the device works; it ends with finish() or the object.
+class HostResult {
+public:
+    HostResult() = default;
+    HostResult(const HostResult&) = delete;
+    HostResult& operator=(const HostResult&) = delete;
+    ~HostResult();
+    void begin(const HostArray* a, int n);
+    int finish(const HostArray* a, int n, hipStream_t stream);         // complete on return
+
+private:
+    std::thread pages_;
+    std::atomic<bool> stop_{false};
+};
 void release_copy_buffers();
 
 // explore_join.hip

@@ -1131,6 +1131,27 @@ def test_symmetric_graph_forms(gpu, orc, rng, monkeypatch, N, K, hubs, staged):
     assert np.array_equal(gp, op) and np.array_equal(gc, oc) and np.array_equal(gv, ov)
 
 
+@pytest.mark.parametrize("N,lead", [(16384, 0), (16385, 0), (16385, 4), (140000, 1020), (140001, 4092)])
+def test_results_into_fresh_pages(gpu, capi, rng, N, lead):
+    """Result arrays of up to 4 MiB and of more, anywhere on pages that do not exist yet: the results, and nothing beside them."""
+    import mmap
+    K, D = 32, 4
+    X = rng.standard_normal((N, D)).astype(np.float32)
+    nk = N * K
+    want_idx, want_dist = np.zeros((N, K), np.int32), np.zeros((N, K), np.float32)
+    want_dist += 1.0                                            # (present pages)
+    log = np.zeros(64, np.float32)
+    _say("results into fresh pages", N, lead)
+    call = capi.lib().rsfk_knn_forest_fresh_host
+    args = (1, K, N, D, K + 1, 3 * K, 5000, 0, 5, 0, 1)
+    assert call(*args, X.ctypes.data, want_idx.ctypes.data, want_dist.ctypes.data, log.ctypes.data) == 0
+    maps = [np.frombuffer(mmap.mmap(-1, lead + 4 * nk + 8192), np.uint8) for _ in range(2)]
+    assert call(*args, X.ctypes.data, maps[0].ctypes.data + lead, maps[1].ctypes.data + lead, log.ctypes.data) == 0
+    for m, want in zip(maps, (want_idx, want_dist)):
+        assert np.array_equal(m[lead:lead + 4 * nk].view(want.dtype), want.ravel())
+        assert not m[:lead].any() and not m[lead + 4 * nk:].any()
+
+
 @pytest.mark.parametrize("N,K,hubs,optional", [(4100, 2, 1, None), (4200, 1, 1, None), (20000, 9, 60, None), (30000, 4, 3, None), (30000, 4, 3, "0")])
 def test_rows_of_hubs_match_oracle(gpu, capi, orc, rng, monkeypatch, N, K, hubs, optional):
     """Rows of more candidates than a workgroup sorts (just above 4,096, several hubs, several shares of R(p) per hub), into
