@@ -439,6 +439,23 @@ static int resident_rows_cap(int D, int K)
     return bucket_rows_cap(D, K);
 }
 
+// Trees of a build whose bucket step still finds rows that are far from done.
+constexpr int kYoungTrees = 2;
+
+// Buckets whose points fit into LDS whole: are the pairs bounded on the matrix cores first?  From the third tree on, when few
+// enough pass: about K / (trees before * points of a bucket) of the candidates can still enter a row, and the screened form, whose
+// cost is that of its candidates, is ahead up to a tenth (largest bucket for the points).  Per tree, direct -> screened, 1M points:
+// K = 64, D = 36, buckets of 65..256: third tree 1.81 -> 2.14 ms, fourth 1.52 -> 1.40, eighth 1.06 -> 0.71; K = 64, D = 20, buckets of
+// 65..130: fourth 0.92 -> 1.07, fifth 0.78 -> 0.82, sixth 0.73 -> 0.68; K = 40, D = 32, buckets of 41..82: third 0.27 -> 0.31, fourth
+// 0.21 -> 0.19; 10M, K = 32, D = 32, buckets of 64..256: second 13.8 -> 17.2, third 10.0 -> 7.8, tenth 6.4 -> 2.8.
+// RSFK_BUCKET_SCREEN=never / always says so for every tree.
+static bool resident_rows_screened(int K, int max_bucket, int trees_before)
+{
+    const unsigned int share = bucket_screen_share_q16();
+    if (share == 0 || share == kScreenAlways) return share != 0;
+    return trees_before >= kYoungTrees && 10ll * K <= (long long)trees_before * max_bucket;
+}
+
 int bucket_gram_from()
 {
     // Off unless asked for: on the shapes measured so far (bucket sizes 33..256, D 32..784, K 32 and 90) the direct
@@ -533,13 +550,13 @@ int launch_bucket_knn(const float* points, int N, int D, int K, const int* ids, 
 // known to be sorted by distance.  stats (8 zeroed words; with K <= 64 and sorted rows): the small buckets go to the
 // kernel that chooses between the direct and the screened form from the pairs of the tree before (prev_stats, null for
 // the first tree) and leaves its own numbers in stats.  part: 0 = all buckets, 1 = only the small ones, 2 = only the larger ones (the two
-// kinds touch different rows, so the two parts of one tree may run side by side).  young_rows: the rows may be new or
-// far from done (first trees of a build).  pairs: working memory for the buckets that reach the general kernel (null:
+// kinds touch different rows, so the two parts of one tree may run side by side).  trees_before: trees of the build
+// whose buckets have been through.  pairs: working memory for the buckets that reach the general kernel (null:
 // its forms that need none); launches that may run side by side need one each.
 int launch_bucket_knn_tree(const float* points, const unsigned long long* prev_stats, unsigned long long* stats,
                            bool rows_sorted, bool gram, int D, int K, const int* ids, const int* starts, const int* sizes,
                            int leaf_cap, int n_small, int n_big, int max_bucket, int* knn_idx, float* knn_dist,
-                           hipStream_t stream, int part, bool young_rows, int* launched, const PairScratch* pairs)
+                           hipStream_t stream, int part, int trees_before, int* launched, const PairScratch* pairs)
 {
     RSFK_CHECK(K >= 1 && K <= kMaxK, "bucket K-NN: K must be in 1..1024");
     RSFK_CHECK(D >= 1, "bucket K-NN: D must be positive");
@@ -591,10 +608,15 @@ int launch_bucket_knn_tree(const float* points, const unsigned long long* prev_s
         const int rows_cap = resident_rows_cap(D, K);
         if (rows_cap > skip_upto) {
             used |= kBucketKernelRows;
-            if (launch_bucket_knn_rows(points, D, K, ids, starts + off, sizes + off, n_big, 0, skip_upto + 1,
-                                       max_bucket >= 0 ? std::min(max_bucket, rows_cap) : rows_cap, rows_sorted, young_rows, knn_idx,
-                                       knn_dist, stream))
+            const int upto = max_bucket >= 0 ? std::min(max_bucket, rows_cap) : rows_cap;
+            if (rows_sorted && resident_rows_screened(K, upto, trees_before)) {
+                if (launch_bucket_knn_rows_screen(points, D, K, ids, starts + off, sizes + off, n_big, skip_upto + 1, upto, knn_idx,
+                                                  knn_dist, stream))
+                    return 1;
+            } else if (launch_bucket_knn_rows(points, D, K, ids, starts + off, sizes + off, n_big, 0, skip_upto + 1, upto,
+                                              rows_sorted, trees_before < kYoungTrees, knn_idx, knn_dist, stream)) {
                 return 1;
+            }
             if (max_bucket >= 0 && max_bucket <= rows_cap) return 0;
             skip_upto = rows_cap;
         }

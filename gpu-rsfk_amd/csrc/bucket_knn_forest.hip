@@ -310,9 +310,14 @@ bool bucket_forest_wanted(int n_trees)
 // have kernels of their own that skip most of a late tree's pairs; their chain of launches is the slower one up to about
 // 200,000 points (time of the bucket step, one tree after the other -> together: 20,000 x 32, 50 trees 3.03 -> 0.31 ms,
 // 150,000 x 100, 10 trees 1.61 -> 0.94, 250,000 x 20, K = 10, 40 trees 3.11 -> 3.28, 400,000 x 100, 50 trees
-// 9.1 -> 9.8).  Larger buckets and longer rows gain at every size that fits (200,000 x 32, buckets of 64..256, 10 trees
-// 3.84 -> 1.81 ms, 1M 10.9 -> 9.1; 70,000 x 784, K = 90, 10 trees 5.0 -> 3.7).
-int bucket_forest_group(int N, int K, int max_bucket, int n_trees)
+// 9.1 -> 9.8).  Larger buckets and longer rows gain at every size that fits (70,000 x 784, K = 90, 10 trees 5.0 -> 3.7), but for
+// many trees over many points whose buckets fit into LDS whole and have far more points than a row has slots: there the later
+// trees skip most pairs as well.  The line is at N * (trees of the build) * largest bucket / K = 80 million (whole build, one tree after
+// the other / together; normal points): 1M x 32, K = 32, buckets of 64..256: 4 trees (32M) 7.1 / 6.5 ms, 10 trees (80M) 10.9 / 12.5, 30
+// trees 22.4 / 31.4; 1M x 20, K = 8, buckets of 64..256: 4 trees (128M) 4.7 / 5.3, 10 trees 7.3 / 10.6; 1M x 36, K = 64, buckets of
+// 65..256: 10 trees (40M) 18.7 / 15.7, 30 trees (120M) 36.4 / 36.9; 300,000 x 32, K = 32, buckets of 64..256: 10 trees (24M) 4.7 / 4.0, 30
+// trees (72M) 8.9 / 8.9; 300,000 x 20, K = 8, buckets of 64..128: 30 trees (144M) 7.7 / 8.0.
+int bucket_forest_group(int N, int D, int K, int max_bucket, int n_trees, int all_trees)
 {
     constexpr size_t kFloats = (size_t)1 << 29;
     constexpr int kMostPoints = 200000;
@@ -320,6 +325,9 @@ int bucket_forest_group(int N, int K, int max_bucket, int n_trees)
     const char* e = std::getenv("RSFK_FOREST_MERGE");
     const bool forced = e && e[0] == '1';
     if (!forced && N > kMostPoints && K <= 64 && max_bucket <= medium_bucket_cap()) return 0;
+    if (!forced && N > kMostPoints && K <= 64 && max_bucket <= bucket_rows_cap(D, K) &&
+        (long long)N * all_trees * max_bucket >= 80000000ll * K)
+        return 0;
     const int group = (int)std::min<size_t>((size_t)std::min(n_trees, 64), kFloats / ((size_t)N * (size_t)forest_pitch(max_bucket)));
     return group >= std::min(2, n_trees) ? group : 0;
 }

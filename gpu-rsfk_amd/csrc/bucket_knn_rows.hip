@@ -31,6 +31,7 @@
 #include "knn_list.hpp"
 #include "forest.hpp"
 #include "bucket_small_body.hpp"
+#include "bucket_rows_stage.hpp"
 #include <algorithm>
 
 namespace rsfk {
@@ -50,7 +51,7 @@ __global__ __launch_bounds__(kRowsThreads) void k_bucket_knn_rows(const float* _
                                                                    const int* __restrict__ ids, const int* __restrict__ starts,
                                                                    const int* __restrict__ sizes, int stride, int min_size,
                                                                    int max_size, int* __restrict__ knn_idx,
-                                                                   float* __restrict__ knn_dist, int pitch, int rows_sorted)
+                                                                   float* __restrict__ knn_dist, int pitch, uint32_t per_np, int rows_sorted)
 {
     extern __shared__ __align__(16) float lds_r[];
     float* rows = lds_r;                                          // 64 NT rows of `pitch` floats
@@ -68,12 +69,7 @@ __global__ __launch_bounds__(kRowsThreads) void k_bucket_knn_rows(const float* _
     for (int i = tid; i < 64 * NT; i += kRowsThreads) lids[i] = i < s ? bid[i] : -1;
     __syncthreads();
     // rows beyond s stay as they are: their distances are never offered
-    for (int it = tid; it < s * np; it += kRowsThreads) {
-        const int m = it / np, pc = it - m * np;
-        const float* src = points + (size_t)lids[m] * (size_t)D + 4 * pc;
-        const float4 v = load_dims(src, D - 4 * pc, vec_ok);
-        *reinterpret_cast<float4*>(&rows[m * pitch + 4 * pc]) = v;
-    }
+    stage_rows<kRowsThreads>(rows, pitch, lids, s, points, D, per_np, vec_ok);
     __syncthreads();
 
     const int nt = (s + 63) >> 6;
@@ -260,25 +256,26 @@ int launch_rows_cfg(const float* points, int D, int K, const int* ids, const int
     auto kern = k_bucket_knn_rows<NT, DENSE>;
     RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     hipLaunchKernelGGL(kern, dim3((unsigned)n_buckets), dim3(kRowsThreads), lds, stream, points, D, K, ids, starts, sizes, stride,
-                       min_size, max_size, knn_idx, knn_dist, pitch, rows_sorted ? 1 : 0);
+                       min_size, max_size, knn_idx, knn_dist, pitch, rows_per_piece(D), rows_sorted ? 1 : 0);
     RSFK_HIP(hipGetLastError());
     return 0;
 }
 
-int rows_pitch(int D)
+}  // namespace
+
+// Floats from one staged row to the next.
+int bucket_rows_pitch(int D)
 {
     int pitch = (D + 3) & ~3;
     if (((pitch >> 2) & 1) == 0) pitch += 4;              // odd number of 16-byte units: rows start in different banks
     return pitch;
 }
 
-}  // namespace
-
 // Largest bucket the kernel takes for points of D dimensions and rows of K neighbours (0: none).
 int bucket_rows_cap(int D, int K)
 {
     if (K > 64) return 0;
-    const int per_point = rows_pitch(D) * (int)sizeof(float) + (int)sizeof(int);
+    const int per_point = bucket_rows_pitch(D) * (int)sizeof(float) + (int)sizeof(int);
     const int tiles = std::min(4, (kRowsLdsBytes - 3 * 64 * kRowsWaves * (int)sizeof(int)) / (64 * per_point));
     return 64 * tiles;
 }
@@ -292,7 +289,7 @@ int launch_bucket_knn_rows(const float* points, int D, int K, const int* ids, co
     if (n_buckets <= 0 || max_size < 2) return 0;
     RSFK_CHECK(K >= 1 && K <= 64 && D >= 1, "bucket kernel with resident rows: K must be in 1..64 and D positive");
     RSFK_CHECK(max_size <= bucket_rows_cap(D, K), "bucket kernel with resident rows: buckets too large for the LDS");
-    const int pitch = rows_pitch(D);
+    const int pitch = bucket_rows_pitch(D);
     const int tiles = (max_size + 63) / 64;
 #define RSFK_ROWS_CASE(NTV, DV)                                                                                             \
     return launch_rows_cfg<NTV, DV>(points, D, K, ids, starts, sizes, n_buckets, stride, min_size, max_size, knn_idx, knn_dist, \

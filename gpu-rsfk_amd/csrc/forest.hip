@@ -265,7 +265,6 @@ int knn_forest_device(int n_trees, int K, int N, int D, int MIN, int MAX, int MA
         unsigned long long* d_pairs = static_cast<unsigned long long*>(pair_stats.p);
         rep.screen_share_q16 = bucket_screen_share_q16();
         const int gram_from = bucket_gram_from();
-        constexpr int kYoungTrees = 2;          // trees of a build whose bucket step still finds rows that are far from done
         SideStream sync;
         if (std::getenv("RSFK_KNN_ONE_STREAM") == nullptr && sync.open()) return 1;
         // working memory of the bucket kernels that pass the distances of a bucket's pairs through memory (only
@@ -302,7 +301,7 @@ int knn_forest_device(int n_trees, int K, int N, int D, int MIN, int MAX, int MA
             int max_bucket = 0;
             if (all_at_once) {
                 for (int j = 0; j < nb; ++j) max_bucket = std::max(max_bucket, stats[5 * j + 2]);
-                group = bucket_forest_group(N, K, max_bucket, nb);
+                group = bucket_forest_group(N, D, K, max_bucket, nb, n_trees);
                 const size_t want = group > 0 ? bucket_forest_floats(N, max_bucket, group) : 0;
                 if (want > forest_floats) {
                     if (forest_dist.p) {
@@ -354,12 +353,12 @@ int knn_forest_device(int n_trees, int K, int N, int D, int MIN, int MAX, int MA
                 rc = launch_bucket_knn_tree(d_points, t > 0 ? d_pairs + (size_t)8 * (t - 1) : nullptr, d_pairs + (size_t)8 * t, true,
                                             gram, D, K, tree_ws_perm(ws.w, j), tree_ws_leaf_start(ws.w, j),
                                             tree_ws_leaf_size(ws.w, j), tree_ws_leaf_cap(ws.w), n_small, n_big, stats[5 * j + 2],
-                                            d_idx, d_dist, stream, split ? 1 : 0, t0 + j < kYoungTrees, &rep.kernels[(size_t)(t0 + j)],
+                                            d_idx, d_dist, stream, split ? 1 : 0, t0 + j, &rep.kernels[(size_t)(t0 + j)],
                                             &pair_mem[0]);
                 if (!rc && split) {
                     rc = launch_bucket_knn_tree(d_points, nullptr, nullptr, true, gram, D, K, tree_ws_perm(ws.w, j), tree_ws_leaf_start(ws.w, j),
                                                 tree_ws_leaf_size(ws.w, j), tree_ws_leaf_cap(ws.w), n_small, n_big,
-                                                stats[5 * j + 2], d_idx, d_dist, sync.side, 2, t0 + j < kYoungTrees,
+                                                stats[5 * j + 2], d_idx, d_dist, sync.side, 2, t0 + j,
                                                 &rep.kernels[(size_t)(t0 + j)], &pair_mem[1]);
                     (void)hipEventRecord(sync.big, sync.side);
                 }

@@ -68,12 +68,12 @@ size_t bucket_pairs_scratch_floats(int D, int K, int n_buckets, int max_bucket);
 int launch_bucket_knn_tree(const float* points, const unsigned long long* prev_stats, unsigned long long* stats,
                            bool rows_sorted, bool gram, int D, int K, const int* ids, const int* starts, const int* sizes,
                            int leaf_cap, int n_small, int n_big, int max_bucket, int* knn_idx, float* knn_dist,
-                           hipStream_t stream, int part = 0, bool young_rows = true, int* launched = nullptr,
+                           hipStream_t stream, int part = 0, int trees_before = 0, int* launched = nullptr,
                            const PairScratch* pairs = nullptr);
 
 // bucket_knn_forest.hip: the buckets of several trees at once (small inputs)
 bool bucket_forest_wanted(int n_trees);
-int bucket_forest_group(int N, int K, int max_bucket, int n_trees);
+int bucket_forest_group(int N, int D, int K, int max_bucket, int n_trees, int all_trees);
 size_t bucket_forest_floats(int N, int max_bucket, int n_trees);
 int launch_bucket_knn_forest(const float* points, int N, int D, int K, int T, const int* perm, const int* leaf_start, const int* leaf_size,
                              int leaf_cap, const int* stats, const int* host_stats, int max_bucket, float* pair_dist, int* info,
@@ -101,9 +101,14 @@ unsigned int bucket_screen_share_q16();
 
 // bucket_knn_rows.hip
 int bucket_rows_cap(int D, int K);
+int bucket_rows_pitch(int D);
 int launch_bucket_knn_rows(const float* points, int D, int K, const int* ids, const int* starts, const int* sizes, int n_buckets,
                            int stride, int min_size, int max_size, bool rows_sorted, bool young_rows, int* knn_idx,
                            float* knn_dist, hipStream_t stream);
+
+// bucket_knn_rows_screen.hip
+int launch_bucket_knn_rows_screen(const float* points, int D, int K, const int* ids, const int* starts, const int* sizes,
+                                  int n_buckets, int min_size, int max_size, int* knn_idx, float* knn_dist, hipStream_t stream);
 
 // bucket_knn_small.hip
 int small_bucket_cap();

@@ -513,6 +513,45 @@ def test_find_nearest_neighbors_matches_oracle(gpu, orc, rng, monkeypatch, N, D,
     assert_knn_equal(gi, gd, oi, od)
 
 
+@pytest.mark.parametrize("data", ["normal", "clusters", "offset", "equal", "huge", "tiny", "rows"])
+@pytest.mark.parametrize("N,D,K,mn,mx", [(3000, 2, 5, 60, 128), (3100, 16, 64, 65, 192), (2900, 17, 32, 64, 256), (3000, 32, 32, 64, 256),
+                                         (4000, 33, 1, 64, 160), (3000, 36, 64, 65, 256), (2500, 44, 40, 60, 192),
+                                         (2600, 49, 33, 60, 128), (2400, 64, 63, 64, 128), (2300, 68, 20, 60, 128)])
+@pytest.mark.parametrize("screen", ["rule", "always"])
+def test_later_trees_of_resident_buckets(gpu, capi, orc, rng, monkeypatch, N, D, K, mn, mx, data, screen):
+    """Buckets that fit into LDS whole, pairs bounded on the matrix cores (any remainder of dimensions, tiles and rows; bounds that
+    drop nothing, rows that differ by less than the bound, equal rows), slots found by counting: from the tree the rule says, and from
+    the first one on (more candidates of a member than lanes).  "rows": the caller's rows hold neighbours already, in any order."""
+    monkeypatch.setenv("RSFK_FOREST_MERGE", "0")
+    if screen == "always":
+        monkeypatch.setenv("RSFK_BUCKET_SCREEN", "always")
+    X = rng.standard_normal((N, D)).astype(np.float32)
+    if data == "clusters":
+        X = (0.01 * X + 30 * rng.standard_normal((40, D)).astype(np.float32)[rng.integers(0, 40, N)]).astype(np.float32)
+    elif data == "offset":
+        X += np.float32(2000)
+    elif data == "equal":
+        X = np.round(X[rng.integers(0, N, N)] * np.float32(1.5)).astype(np.float32)
+    elif data == "huge":
+        X *= np.float32(2e18)
+        X[:: 97] *= np.float32(1e-19)
+    elif data == "tiny":
+        X *= np.float32(1e-19)
+        X[:: 97] *= np.float32(1e-19)
+    T = 7
+    _say("later trees, resident buckets", N, D, K, mn, mx, data, screen)
+    gi, gd = orc.init_lists(N, K, self_in=True)
+    if data == "rows":
+        orc.forest(X, K, 1, mn, mx, 5000, 90, 0, knn_idx=gi, knn_dist=gd)
+        order = np.argsort(rng.random((N, K)), axis=1)
+        gi, gd = (np.ascontiguousarray(np.take_along_axis(v, order, axis=1)) for v in (gi, gd))
+    oi, od = gi.copy(), gd.copy()
+    log = np.zeros(16 * T + 2, np.float32)
+    capi.lib().pymodule_rsfk_knn(T, K, N, D, mn, mx, 5000, 0, 3, 0, X.ctypes.data, gi.ctypes.data, gd.ctypes.data, log.ctypes.data)
+    orc.forest(X, K, T, mn, mx, 5000, 3, 0, knn_idx=oi, knn_dist=od)
+    assert_knn_equal(gi, gd, oi, od)
+
+
 # The workloads of the benchmark configurations 3, 4 and 5 (clustered D=256; sparse D=784 with K=90 and one
 # exploration pass, the only shape that runs the general bucket kernel with two slots per lane together with the
 # workgroup-per-point exploration merge; standard normal D=32 with buckets of 64..256 points), as forest +
