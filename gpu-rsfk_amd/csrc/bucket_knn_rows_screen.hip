@@ -61,14 +61,6 @@ struct WaveLds {
     float mean[16 * KS];                      // the common point
 };
 
-// A (distance, index) pair as a double whose order is that of the pairs (distances >= 0, indices >= 0; an empty slot (+inf, -1) is above
-// every pair): the exponent is moved away from the denormals.
-__device__ __forceinline__ double pair_key(float d, int c)
-{
-    return __hiloint2double((int)(__float_as_uint(d + 0.0f) + 0x00100000u), c);
-}
-__device__ __forceinline__ float pair_dist(double key) { return __uint_as_float((uint32_t)__double2hiint(key) - 0x00100000u); }
-
 // NT: buckets of up to 64 NT points; KS: steps of 16 dimensions.
 template <int NT, int KS>
 __global__ __launch_bounds__(kRowsThreads, 3) void k_bucket_knn_rows_screen(const float* __restrict__ points, int D, int K,

@@ -19,6 +19,7 @@ struct ExploreLds {          // per wavefront; sizes fixed at launch
     int* queue2;             // candidates that passed the screen, waiting for the exact distance
     float* xrow;             // the point's coordinates, zero padded to bf16_valid(D)
     float* tile;             // 64 x (chunk + 4) words
+    double* rank;            // rank_words(SL) words for merge_ranked (exact_direct; exact_batch has them in its tile)
 };
 
 // Load one 16-byte piece (4 dimensions) of a candidate row, zero beyond D.
@@ -33,8 +34,9 @@ __device__ __forceinline__ float4 load_piece(const float* __restrict__ row, int 
 // two steps are in flight while a third is being used (two register buffers that take turns, so that waiting for
 // one does not wait for the other): for kernels with few wavefronts per SIMD, whose gathers would otherwise wait
 // for each other.  GROUP: 16-byte pieces of a row whose reads from the tile are requested together (0: one at a time, the
-// form that needs the fewest registers).
-template <int SL, int CH = kChunk, bool DEEP = false, int GROUP = 0>
+// form that needs the fewest registers).  RANK: no point of the list is in the row or on the list twice, but at this very distance: the batch is
+// merged by merge_ranked.
+template <int SL, int CH = kChunk, bool DEEP = false, int GROUP = 0, bool RANK = false>
 __device__ __forceinline__ void exact_batch(const ExploreLds& L, const int* list, int n,
                                             const float* __restrict__ points, int D, bool vec_ok, KnnRow<SL>& row,
                                             float tau_cap = INFINITY)
@@ -118,13 +120,19 @@ __device__ __forceinline__ void exact_batch(const ExploreLds& L, const int* list
             if (!step(pre[0], d0, CH)) { finished = false; break; }
     }
     wave_lds_sync();
-    row.merge(lane < n && finished, my_c, acc);          // unfinished sums are all above the last slot
+    // (unfinished sums are all above the last slot)
+    if (RANK) {
+        static_assert(!RANK || rank_words(SL) <= 64 * kP, "the ranks' working memory takes the place of the tile");
+        row.merge_ranked(lane < n && finished, my_c, acc, reinterpret_cast<double*>(L.tile));
+    } else {
+        row.merge(lane < n && finished, my_c, acc);
+    }
 }
 
 // The same without the tile: lane l reads the row of candidate l itself, 32 dimensions (eight 16-byte pieces) per
 // step, and runs its chain from registers; the point's coordinates come from L.xrow (every lane reads the same
 // word).  For short rows: no LDS besides xrow, no synchronisation inside the batch.
-template <int SL>
+template <int SL, bool RANK = false>
 __device__ __forceinline__ void exact_direct(const ExploreLds& L, const int* list, int n, const float* __restrict__ points,
                                              int D, bool vec_ok, KnnRow<SL>& row, float tau_cap = INFINITY)
 {
@@ -153,7 +161,9 @@ __device__ __forceinline__ void exact_direct(const ExploreLds& L, const int* lis
         // partial sums only grow: once all of them are above the row maximum nothing can enter
         if (ballot64(lane < n && acc <= tau0) == 0) { finished = false; break; }
     }
-    row.merge(lane < n && finished, my_c, acc);          // unfinished sums are all above the last slot
+    // (unfinished sums are all above the last slot)
+    if (RANK) row.merge_ranked(lane < n && finished, my_c, acc, L.rank);
+    else row.merge(lane < n && finished, my_c, acc);
 }
 
 }  // namespace rsfk

@@ -351,6 +351,10 @@ constexpr int kMergeTile = 64 * (kMergeChunk + 4);
 // Rows of at most this many (padded) dimensions are read by the lane that runs their chain, 32 dimensions at a time,
 // without the transposing tile in LDS (exact_direct): the LDS of a wavefront shrinks by the tile.
 __host__ __device__ inline int merge_tile_ints(int dpad, int direct_max) { return dpad <= direct_max ? 0 : kMergeTile; }
+__host__ __device__ inline int merge_rank_at(int table, int K, bool with_bounds)
+{
+    return table + ((K + 3) & ~3) + (with_bounds ? table / 4 * 7 : 0);
+}
 int merge_direct_max()
 {
     static const int v = [] {
@@ -429,6 +433,8 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_merge(const float* __res
     // with bounds: the smallest lower bound seen for the id in the same place of the set (bfloat16 bits), behind the
     // list of marks
     int* tbound = bounds ? L.srow + K + table_size / 4 * 3 : nullptr;
+    // without the tile: the ranks' working memory, in place of the list of marks or behind the bounds
+    if (!TILE) L.rank = reinterpret_cast<double*>(base + dpad + merge_rank_at(table_size, K, bounds != nullptr));
     const int KP = (K + 31) & ~31;
     const bool vec_ok = (D & 3) == 0 && ((reinterpret_cast<uintptr_t>(points) & 15) == 0);
 
@@ -526,8 +532,8 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_merge(const float* __res
     int n_exact = 0;                                      // exact distances of this point (wave-uniform)
     auto batch = [&](const int* list, int n) {
         n_exact += n;
-        if (!TILE) exact_direct<SL>(L, list, n, points, D, vec_ok, row);
-        else exact_batch<SL, kMergeChunk, true, kChainGroup>(L, list, n, points, D, vec_ok, row);    // two steps of gathers in flight
+        if (!TILE) exact_direct<SL, true>(L, list, n, points, D, vec_ok, row);
+        else exact_batch<SL, kMergeChunk, true, kChainGroup, true>(L, list, n, points, D, vec_ok, row);    // two steps of gathers in flight
     };
     if (tbound == nullptr || U <= 64) {
         for (int off = 0; off < U; off += 64) {
@@ -760,7 +766,7 @@ __global__ __launch_bounds__(256) void k_explore_merge_wg(const float* __restric
         const int n_now = min(64, have);
         n_exact += n_now;
         const float cap_now = __uint_as_float(*reinterpret_cast<volatile uint32_t*>(&tau_s));
-        exact_batch<SL, kWgChunk, true, kChainGroup>(L, ids, n_now, points, D, vec_ok, row, cap_now);
+        exact_batch<SL, kWgChunk, true, kChainGroup, true>(L, ids, n_now, points, D, vec_ok, row, cap_now);
         if (lane == 0) atomicMin(&tau_s, __float_as_uint(row.tau));   // non-negative floats order like their bits
         have -= n_now;
         const int left = lane < have ? ids[64 + lane] : 0;        // the candidates beyond the batch move to the front
@@ -1001,7 +1007,10 @@ int launch_merge(const float* points, int N, int D, int K, const int* old_idx, i
 // marks | with_bounds: a bound per place of the set
 int merge_wave_ints(int table, int dpad, int K, bool with_bounds = false)
 {
-    return (merge_tile_ints(dpad, merge_direct_max()) + dpad + table + K + table / 4 * 3 + (with_bounds ? table : 0) + 3) / 4 * 4;
+    const int tile = merge_tile_ints(dpad, merge_direct_max());
+    const int lists = table + K + table / 4 * 3 + (with_bounds ? table : 0);
+    const int ranks = tile > 0 ? 0 : merge_rank_at(table, K, with_bounds) + rank_words(row_slots(K));
+    return (tile + dpad + std::max(lists, ranks) + 3) / 4 * 4;
 }
 
 int dispatch_merge(int sl, int waves, const float* points, int N, int D, int K, const int* old_idx, int* knn_idx,

@@ -21,9 +21,7 @@
 // comparison per slot gives the mask of the lanes that change, and that mask
 // shifted by one gives the lanes that take the value of the slot below: no
 // reduction and no re-reading of the maximum between the candidates of a batch.
-// (Merging a batch by ranking -- a count per candidate and per slot, then one
-// scatter -- was measured slower: about as many vector instructions per accepted
-// candidate and three times the scalar ones.)
+// Large batches of new points go by merge_ranked instead, which inserts nothing.
 // Rows that arrive unsorted (anything the caller passes in) are detected on load
 // and rebuilt; rows are always written back sorted.  Slot positions are not part
 // of the interface.
@@ -48,6 +46,20 @@ __device__ __forceinline__ uint64_t mask_pair_above(float d1, int c1, float d2, 
 }
 // this lane's bit of a mask
 __device__ __forceinline__ bool lane_bit(uint64_t mask) { return __builtin_amdgcn_inverse_ballot_w64(mask); }
+
+// A (distance, index) pair as a double whose order is that of the pairs (distances >= 0, indices >= 0; an empty slot (+inf, -1) is above
+// every pair): the exponent is moved away from the denormals.
+__device__ __forceinline__ double pair_key(float d, int c)
+{
+    return __hiloint2double((int)(__float_as_uint(d + 0.0f) + 0x00100000u), c);
+}
+__device__ __forceinline__ float pair_dist(double key) { return __uint_as_float((uint32_t)__double2hiint(key) - 0x00100000u); }
+
+// Batches with no more entering candidates than this are inserted.
+constexpr int kFewEnter = 4;
+
+// Working memory of merge_ranked, in words of four bytes: the row as keys, the distances of a batch, the slots it takes.
+__host__ __device__ constexpr int rank_words(int sl) { return 2 * 64 * sl + 64 + 4 + 2 * sl; }
 
 template <int SL>
 struct KnnRow {
@@ -214,6 +226,82 @@ struct KnnRow {
             refresh_tau();
             changed = true;
         }
+    }
+
+    // The same for a batch of one candidate per lane whose points are not in the row (a set has seen to that, or they are in it at this
+    // very distance).  A batch of which many enter is not inserted one by one (14 vector and 16 scalar instructions each, and
+    // most of what enters first is pushed out again): every candidate finds its slot by itself -- the entries of the row below it
+    // by binary search, the entering candidates below it by counting distances --, and an entry of the row moves up by the candidates
+    // that end below it: 60 instructions and two per candidate.  (Exploration merge of 123,457 x 37, K = 45: 1.04 -> 0.95 ms, 1M x
+    // 256, K = 32: 14.8 -> 13.8, 70,000 x 784, K = 90: 16.5 -> 16.0; 10M x 32, K = 32: a quarter fewer instructions at the same 23.9 ms, the rate of
+    // its gathers.  Where the line for the insertions lies, 2, 4 or 10 entering candidates, makes no difference.)  Where two distances are equal the insertions decide.
+    // buf: rank_words(SL) words of LDS, 16-byte aligned.
+    __device__ __forceinline__ void merge_ranked(bool ok, int c, float d, double* buf)
+    {
+        const bool in = ok && enters(c, d);
+        const uint64_t m = ballot64(in);
+        const int n = __popcll(m);
+        if (n <= kFewEnter) {
+            if (n != 0) merge(ok, c, d);
+            return;
+        }
+        const int lane = lane_id();
+        float* cand = reinterpret_cast<float*>(buf + 64 * SL);
+        uint32_t* places = reinterpret_cast<uint32_t*>(cand + 68);
+        const double key = pair_key(d, c);
+        wave_lds_sync();
+#pragma unroll
+        for (int s = 0; s < SL; ++s) buf[lane + 64 * s] = pair_key(dist[s], idx[s]);       // (slots beyond the row: above every candidate)
+        if (in) cand[mask_prefix(m)] = d;
+        if (lane < 4) cand[n + lane] = INFINITY;
+        if (lane < 2 * SL) places[lane] = 0;
+        wave_lds_sync();
+        int pos = 0;                                         // (a candidate that enters is below the last slot)
+#pragma unroll
+        for (int step = 32 * SL; step > 0; step >>= 1)
+            if (step < kk && buf[pos + step - 1] < key) pos += step;
+        const int hi = __double2hiint(key);
+        bool level = __double2hiint(buf[pos]) == hi || (pos > 0 && __double2hiint(buf[pos - 1]) == hi);
+        int rank = pos;
+        for (int k = 0; k < n; k += 4) {
+            const float4 v = *reinterpret_cast<const float4*>(cand + k);
+            rank += v.x < d ? 1 : 0;
+            rank += v.y < d ? 1 : 0;
+            rank += v.z < d ? 1 : 0;
+            rank += v.w < d ? 1 : 0;
+        }
+        const bool stays = in && rank < kk;
+        const uint32_t bit = 1u << (rank & 31);
+        if (stays) level |= (atomicOr(&places[rank >> 5], bit) & bit) != 0;
+        if (ballot64(in && level) != 0) {
+            merge(ok, c, d);
+            return;
+        }
+        wave_lds_sync();
+        double v[SL];
+        bool is_new[SL];
+        int before = 0;
+#pragma unroll
+        for (int s = 0; s < SL; ++s) {
+            const uint64_t taken = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)places[2 * s]) |
+                                   (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)places[2 * s + 1]) << 32;
+            is_new[s] = lane_bit(taken);
+            v[s] = buf[lane + 64 * s - before - mask_prefix(taken)];
+            before += __popcll(taken);
+        }
+        wave_lds_sync();
+        if (stays) buf[rank] = key;
+        wave_lds_sync();
+#pragma unroll
+        for (int s = 0; s < SL; ++s) {
+            if (is_new[s]) v[s] = buf[lane + 64 * s];
+            if (lane + 64 * s < kk) {
+                idx[s] = __double2loint(v[s]);
+                dist[s] = pair_dist(v[s]);
+            }
+        }
+        changed = true;
+        refresh_tau();
     }
 
     __device__ __forceinline__ void merge(bool ok, int c, float d)

@@ -457,6 +457,28 @@ def test_explore_with_the_reversed_graph_by_tiles(gpu, orc, rng, monkeypatch, N,
     assert_knn_equal(gi, gd, oi, od)
 
 
+@pytest.mark.parametrize("values", ["any", "whole", "near"])
+@pytest.mark.parametrize("N,D,K", [(1500, 6, 1), (3000, 3, 32), (3000, 33, 33), (2500, 130, 31), (2000, 8, 64), (1500, 200, 64), (1800, 20, 65),
+                                   (1500, 12, 128), (1500, 140, 90), (1600, 10, 200)])
+def test_explore_batches_merged_by_rank(gpu, orc, rng, N, D, K, values):
+    """Rows of one, two and four slots per lane, with and without the tile, a wavefront and a workgroup per point; few and many entering
+    candidates; distances that are equal (whole numbers) or differ in the last bits."""
+    X = rng.standard_normal((N, D)).astype(np.float32)
+    if values == "whole":
+        X = np.round(X * np.float32(1.2)).astype(np.float32)
+    elif values == "near":
+        X = (np.float32(1) + np.float32(2.0 ** -20) * np.round(X * 8)).astype(np.float32)
+    oi, od = orc.init_lists(N, K, self_in=True)
+    perm, ls, lz, _ = orc.build_tree(X, K + 1, 2 * K + 2, 5000, 0)
+    orc.bucket_knn(X, K, perm, lz, oi, od, starts=ls)
+    gi, gd = oi.copy(), od.copy()
+    _say("explore by rank", N, D, K, values)
+    for _ in range(2):                                          # (the second pass: few enter)
+        orc.explore(X, K, oi, od)
+        gpu.explore(X, K, gi, gd, 1)
+        assert_knn_equal(gi, gd, oi, od)
+
+
 # ---------------------------------------------------------------------------
 # the whole call, through the entry points the Python package binds
 # ---------------------------------------------------------------------------
