@@ -36,6 +36,7 @@
 #include "mfma_split.hpp"
 #include "forest.hpp"
 #include "bucket_rows_stage.hpp"
+#include "row_turn.hpp"
 #include <algorithm>
 
 namespace rsfk {
@@ -45,18 +46,10 @@ namespace {
 constexpr int kRowsThreads = 256;
 constexpr int kRowsWaves = kRowsThreads / 64;
 constexpr int kListCap = 256;                 // pairs on a wavefront's list: at least the candidates of one member
-constexpr int kFlight = 4;                    // K-NN rows of kFlight * 64 slots together are merged into at a time
-constexpr int kRowRoom = 272;                 // ... and their room in LDS, in slots
-constexpr int kMostRows = 16;
-constexpr int kGap = 3;
-static_assert(64 + kGap * kMostRows <= 128, "the places of a turn's candidates");
 
 // Per wavefront.
 template <int KS>
-struct WaveLds {
-    double row[kRowRoom];                     // K-NN rows, as keys
-    float cand[128];                          // the distances of a turn's new candidates, kGap free places (+inf) after every member's
-    int4 slot[kMostRows];                     // per row: its point, -, the final places of new candidates (two words)
+struct WaveLds : TurnLds {
     uint16_t list[kListCap];                  // pairs: member << 8 | candidate
     float mean[16 * KS];                      // the common point
 };
@@ -150,14 +143,7 @@ __global__ __launch_bounds__(kRowsThreads, 3) void k_bucket_knn_rows_screen(cons
     }
     __syncthreads();
 
-    const int row_pitch = (K + 3) & ~1;                           // (16 bytes from row to row on top: they start in different banks)
-    const int n_room = min(kMostRows, min(64 * kFlight / K, kRowRoom / row_pitch));
-    int rk[kFlight];                                              // row << 8 | entry of this lane's slots of the buffer
-#pragma unroll
-    for (int x = 0; x < kFlight; ++x) {
-        const int q = lane + 64 * x, r = (q * per_k) >> 16;       // (q / K: q < 256, per_k = 65536 / K rounded up)
-        rk[x] = r << 8 | (q - r * K);
-    }
+    RowTurn turn(K, per_k);
     const int nj = (s + 31) >> 5;
     for (int T = wave; T < nj; T += kRowsWaves) {
         const int i = 32 * T + col;
@@ -234,7 +220,7 @@ __global__ __launch_bounds__(kRowsThreads, 3) void k_bucket_knn_rows_screen(cons
             for (int i0 = g0; i0 < g1;) {
                 // members i0 .. i1 - 1: a lane per pair and room for the rows; or one member whose pairs take several turns
                 const int first = read_lane_i(from, i0), seq0 = read_lane_i(seq, i0);
-                const bool fits = upto - first <= 64 && seq + (both > 0 ? 1 : 0) - seq0 <= n_room;
+                const bool fits = upto - first <= 64 && seq + (both > 0 ? 1 : 0) - seq0 <= turn.n_room;
                 const int i1 = i0 + max(1, __popc((uint32_t)ballot64(fits && col >= i0 && col < g1)));
                 const int total = read_lane_i(upto, i1 - 1) - first;
                 const bool act_here = both > 0 && col >= i0 && col < i1;
@@ -245,18 +231,7 @@ __global__ __launch_bounds__(kRowsThreads, 3) void k_bucket_knn_rows_screen(cons
                     wave_lds_sync();
                     if (act_here && half == 0) L.slot[seq - seq0] = make_int4(gid, 0, 0, 0);
                     wave_lds_sync();
-                    // the rows: slot q of the buffer is entry q % K of row q / K
-                    int xi[kFlight], xd[kFlight];
-#pragma unroll
-                    for (int x = 0; x < kFlight; ++x) {
-                        xi[x] = -1;
-                        xd[x] = 0;
-                        if ((rk[x] >> 8) < n_rows) {
-                            const size_t at = (size_t)L.slot[rk[x] >> 8].x * (size_t)K + (rk[x] & 255);
-                            xi[x] = knn_idx[at];
-                            xd[x] = __float_as_int(knn_dist[at]);
-                        }
-                    }
+                    turn.request(L, n_rows, knn_idx, knn_dist);
                     // the exact distances
                     const int entry = lane < n ? L.list[first - base + e0 + lane] : 0;
                     const int pcol = entry >> 8, j = entry & 255;
@@ -281,89 +256,7 @@ __global__ __launch_bounds__(kRowsThreads, 3) void k_bucket_knn_rows_screen(cons
                     const int prow = __shfl(seq, pcol, 64) - seq0;
                     // (at the distance of the last slot the index decides: by the rank)
                     const bool enter = lane < n && d < INFINITY && d <= last;
-                    const double key = pair_key(d, cid);
-#pragma unroll
-                    for (int x = 0; x < kFlight; ++x)
-                        if ((rk[x] >> 8) < n_rows) L.row[(rk[x] >> 8) * row_pitch + (rk[x] & 255)] = pair_key(__int_as_float(xd[x]), xi[x]);
-                    wave_lds_sync();
-                    // against the row: is the candidate there already, how many entries are below it
-                    int below = 0;
-                    bool there = false, level;
-                    {
-                        const double* r = L.row + (enter ? prow * row_pitch : 0);
-#pragma unroll 4
-                        for (int k = 0; k < K / 2; ++k) {
-                            const double2 v = *reinterpret_cast<const double2*>(r + 2 * k);
-                            there |= __double2loint(v.x) == cid || __double2loint(v.y) == cid;
-                            below += v.x < key ? 1 : 0;
-                            below += v.y < key ? 1 : 0;
-                        }
-                        if (K & 1) {
-                            const double v = r[K - 1];
-                            there |= __double2loint(v) == cid;
-                            below += v < key ? 1 : 0;
-                        }
-                        level = __double2hiint(r[max(below - 1, 0)]) == __double2hiint(key) ||
-                                __double2hiint(r[min(below, K - 1)]) == __double2hiint(key);
-                    }
-                    // against the member's other new candidates: by distance alone, where that decides
-                    const bool fresh = enter && !there;
-                    const int end = fresh ? min(count, n - lo) : 0;
-                    const int mine_at = kGap * prow + lo;
-                    *reinterpret_cast<float2*>(&L.cand[2 * lane]) = make_float2(INFINITY, INFINITY);
-                    wave_lds_sync();
-                    if (fresh) L.cand[kGap * prow + lane] = d;
-                    wave_lds_sync();
-                    const int below_row = below;
-                    for (int k = 0; ballot64(k < end) != 0; k += 4) {
-                        const float* c = L.cand + (k < end ? mine_at + k : 124);
-#pragma unroll
-                        for (int u = 0; u < 4; ++u) below += c[u] < d ? 1 : 0;
-                    }
-                    bool in = fresh && below < K;
-                    uint32_t* places = reinterpret_cast<uint32_t*>(&L.slot[prow]) + 2;
-                    const uint32_t bit = 1u << (below & 31);
-                    const bool taken = in && (atomicOr(places + (below >> 5), bit) & bit) != 0;
-                    if (ballot64(taken || (fresh && level)) != 0) {
-                        // (two candidates at one distance, with or without an entry of the row between them: the indices decide)
-                        if (in) atomicAnd(places + (below >> 5), ~bit);
-                        below = below_row;
-                        for (int k = 0; k < n; ++k) {
-                            const bool other = read_lane_i(fresh ? prow : -1, k) == prow;
-                            below += other && pair_above(d, cid, read_lane_f(d, k), read_lane_i(cid, k)) ? 1 : 0;
-                        }
-                        in = fresh && below < K;
-                        if (in) atomicOr(places + (below >> 5), 1u << (below & 31));
-                    }
-                    if (ballot64(in) == 0) continue;
-                    wave_lds_sync();
-                    // the new rows: an entry moves up by the candidates that end below it
-                    double xv[kFlight];
-                    uint32_t is_new = 0, changed = 0;
-#pragma unroll
-                    for (int x = 0; x < kFlight; ++x) {
-                        xv[x] = 0.0;
-                        if ((rk[x] >> 8) < n_rows) {
-                            const int k = rk[x] & 255;
-                            const int2 m2 = *(reinterpret_cast<const int2*>(&L.slot[rk[x] >> 8]) + 1);
-                            const uint64_t m = ((uint64_t)(uint32_t)m2.y << 32) | (uint32_t)m2.x;
-                            if (m != 0) changed |= 1u << x;
-                            if ((m >> k) & 1) is_new |= 1u << x;
-                            xv[x] = L.row[(rk[x] >> 8) * row_pitch + k - __popcll(m & ((1ull << k) - 1))];
-                        }
-                    }
-                    wave_lds_sync();
-                    if (in) L.row[prow * row_pitch + below] = key;
-                    wave_lds_sync();
-#pragma unroll
-                    for (int x = 0; x < kFlight; ++x) {
-                        if ((is_new >> x) & 1) xv[x] = L.row[(rk[x] >> 8) * row_pitch + (rk[x] & 255)];
-                        if ((changed >> x) & 1) {
-                            const size_t at = (size_t)L.slot[rk[x] >> 8].x * (size_t)K + (rk[x] & 255);
-                            knn_idx[at] = __double2loint(xv[x]);
-                            knn_dist[at] = pair_dist(xv[x]);
-                        }
-                    }
+                    turn.merge(L, n_rows, n, enter, prow, lo, count, cid, d, knn_idx, knn_dist);
                 }
             }
             g0 = g1;
@@ -383,7 +276,7 @@ int launch_cfg(const float* points, int D, int K, const int* ids, const int* sta
     auto kern = k_bucket_knn_rows_screen<NT, KS>;
     RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     hipLaunchKernelGGL(kern, dim3((unsigned)n_buckets), dim3(kRowsThreads), lds, stream, points, D, K, ids, starts, sizes, min_size,
-                       max_size, knn_idx, knn_dist, pitch, (65536 + K - 1) / K, rows_per_piece(D), c_err, over);
+                       max_size, knn_idx, knn_dist, pitch, turn_per_k(K), rows_per_piece(D), c_err, over);
     RSFK_HIP(hipGetLastError());
     return 0;
 }

@@ -28,10 +28,11 @@
 //      chains of its pairs of the list (arithmetic of euclidean_distance_sqr,
 //      compute_knn_from_buckets.cu:40-54: a pair has the same distance value as in
 //      every other kernel);
-//   4. an exact distance that is not above the last slot of a row goes into the
-//      bucket's distance matrix in LDS and sets the member's bit in that row's
-//      candidate set (nothing else of the matrix is written or read); the rows
-//      with a candidate are merged as in the other kernel.
+//   4. an exact distance that is not above the last slot of a row is an offer to it.  The offers are put in the order of the
+//      rows, in LDS, and go into them by turns of up to 64 offers and 256 slots (row_turn.hpp), half of the offers per wavefront.
+//      Rows merged one after the other took 46 % of the kernel's time in a late tree and more before: 1M x 100, K = 32, fourth tree
+//      0.70 -> 0.47 ms, tenth 0.41 -> 0.35, 50th 0.25 -> 0.25 (0.9 GB moved: 3.7 TB/s); 1M x 256 fourth 0.92 -> 0.75, tenth 0.56 -> 0.54.
+//      A bucket with more pairs than the list holds keeps a distance matrix in LDS, and its rows are merged as in the other kernel.
 //
 // Requires every K-NN row to be sorted on entry (the last slot is its maximum);
 // launch_sort_rows establishes that once per build.
@@ -39,6 +40,7 @@
 #include "knn_list.hpp"
 #include "forest.hpp"
 #include "mfma_split.hpp"
+#include "row_turn.hpp"
 #include "bucket_small_body.hpp"
 #include <algorithm>
 #include <cstdlib>
@@ -68,6 +70,15 @@ struct alignas(16) ScreenMeta {
     float nrm[2][kCap];
     int n_pairs[4];
     uint16_t list[kListCap];
+};
+
+// In the place of the staged rows, once the exact distances are known: the offers (a pair is offered to one or both of its rows) in
+// the order of the rows, and what the turns need.
+struct alignas(16) ScreenTurns {
+    TurnLds turn[2];
+    float dist[2 * kListCap];
+    uint16_t pair[2 * kListCap];            // row << 6 | candidate
+    uint16_t off[kCap];                     // first offer of a row
 };
 
 // The rows of the bucket on their way from HBM to LDS: 16 lanes (a quarter wavefront) per row, a lane moves 16 bytes
@@ -115,6 +126,7 @@ struct RowLoads {
 constexpr int kPitch = kChunk + 4;                        // an odd number of 16-byte units: rows start in different banks
 constexpr int kRegion = kCap * kPitch > kCap * kDistPitch ? kCap * kPitch : kCap * kDistPitch;
 constexpr size_t kScreenLdsBytes = sizeof(float) * kRegion + sizeof(ScreenMeta);
+static_assert(sizeof(ScreenTurns) <= sizeof(float) * kRegion, "the turns take the place of the rows");
 static_assert(kScreenLdsBytes <= 160 * 1024 / 8, "eight workgroups per compute unit");
 
 template <bool SINGLE>
@@ -122,7 +134,7 @@ __device__ __forceinline__ void screen_bucket_body(float* __restrict__ lds, cons
                                                    const int* __restrict__ ids, const int* __restrict__ starts,
                                                    const int* __restrict__ sizes, int stride, int* __restrict__ knn_idx,
                                                    float* __restrict__ knn_dist, float c_err, float one_minus_gamma,
-                                                   unsigned long long* __restrict__ stats, int stat_shift)
+                                                   unsigned long long* __restrict__ stats, int stat_shift, int per_k)
 {
     float* rows = lds;                                    // kRegion floats: the rows, later the distance matrix
     float* dist = lds;
@@ -302,7 +314,70 @@ __device__ __forceinline__ void screen_bucket_body(float* __restrict__ lds, cons
             chains(min(kChunk, (D - c * kChunk + 3) & ~3) >> 2);
         }
     }
-    __syncthreads();                                  // rows no longer needed: the region becomes the distance matrix
+    __syncthreads();                                  // rows no longer needed: their place is used for what follows
+    if (!all_pairs) {
+        // ---- 4. few offers: they are put in the order of the rows (LDS: offers, then working memory of the turns) and merged by turns
+        auto offer = [&](auto&& to) {
+#pragma unroll
+            for (int r = 0; r < kMaxRounds; ++r) {
+                if (tid + r * kThreads < n_list) {
+                    const uint32_t e = entry(r);
+                    const int i = (int)(e & 63u), j = (int)(e >> 6);
+                    if (acc[r] <= M.tau[i]) to(i, j, acc[r]);
+                    if (acc[r] <= M.tau[j]) to(j, i, acc[r]);
+                }
+            }
+        };
+        offer([&](int i, int j, float) { atomicOr(&M.cand[i], 1ull << j); });
+        __syncthreads();
+        ScreenTurns& W = *reinterpret_cast<ScreenTurns*>(lds);
+        TurnLds& L = W.turn[wave];
+        const int cnt = __popcll(M.cand[lane]);
+        const int upto = wave_excl_scan_i(cnt) + cnt, off = upto - cnt;
+        const int all = read_lane_i(upto, 63);
+        if (all == 0) return;
+        if (wave == 0) W.off[lane] = (uint16_t)off;
+        const int half_way = __popcll(ballot64(2 * off < all));   // rows of the first wavefront: half of the offers
+        const int r0 = wave == 0 ? 0 : half_way, r1 = wave == 0 ? half_way : kCap;
+        const int seq = mask_prefix(ballot64(cnt > 0));
+        const int gid = lids[lane];
+        RowTurn turn(K, per_k);
+        int first = 0, seq0 = 0, next = r0, n = 0, n_rows = 0;
+        auto pick = [&]() {
+            // rows next .. i1 - 1: a lane per offer and room for the rows
+            const int i0 = next;
+            first = read_lane_i(off, i0);
+            seq0 = read_lane_i(seq, i0);
+            const bool fits = upto - first <= 64 && seq + (cnt > 0 ? 1 : 0) - seq0 <= turn.n_room;
+            next = i0 + max(1, __popcll(ballot64(fits && lane >= i0 && lane < r1)));
+            n = read_lane_i(upto, next - 1) - first;
+            const bool here = cnt > 0 && lane >= i0 && lane < next;
+            n_rows = __popcll(ballot64(here));
+            wave_lds_sync();
+            if (here) L.slot[seq - seq0] = make_int4(gid, 0, 0, 0);
+            wave_lds_sync();
+            turn.request(L, n_rows, knn_idx, knn_dist);
+        };
+        if (next < r1) pick();
+        __syncthreads();
+        offer([&](int i, int j, float d) {
+            const int at = W.off[i] + __popcll(M.cand[i] & ((1ull << j) - 1));
+            W.dist[at] = d;
+            W.pair[at] = (uint16_t)(i << 6 | j);
+        });
+        __syncthreads();
+        while (n_rows > 0 || next < r1) {
+            const int e = lane < n ? W.pair[first + lane] : 0;
+            const float d = lane < n ? W.dist[first + lane] : INFINITY;
+            const int i = e >> 6;
+            const int prow = __shfl(seq, i, 64) - seq0, lo = __shfl(off, i, 64) - first, count = __shfl(cnt, i, 64);
+            turn.merge(L, n_rows, n, lane < n && d < INFINITY, prow, lo, count, lids[e & 63], d, knn_idx, knn_dist);
+            n_rows = 0;
+            if (next < r1) pick();
+        }
+        return;
+    }
+    // the distance matrix
     // (only the entries a row may take are written, and cand says which they are: nothing else of the matrix is read)
 #pragma unroll
     for (int r = 0; r < kMaxRounds; ++r) {
@@ -322,7 +397,7 @@ __device__ __forceinline__ void screen_bucket_body(float* __restrict__ lds, cons
     }
     __syncthreads();
 
-    // ---- 4. top-K update: a wavefront walks its members that have a candidate, eight at a time, with the rows of the
+    // ---- 4. rows of the matrix: a wavefront walks its members that have a candidate, eight at a time, with the rows of the
     //         next eight in flight
     const int my_id = lids[lane];
     uint32_t active = (uint32_t)ballot64(lane < 32 && M.cand[fm < kCap ? fm : 0] != 0ull);
@@ -381,11 +456,11 @@ __global__ __launch_bounds__(kThreads, 4) void k_bucket_knn_screen(const float* 
                                                                    const int* __restrict__ starts,
                                                                    const int* __restrict__ sizes, int stride,
                                                                    int* __restrict__ knn_idx, float* __restrict__ knn_dist,
-                                                                   float c_err, float one_minus_gamma)
+                                                                   float c_err, float one_minus_gamma, int per_k)
 {
     extern __shared__ __align__(16) float lds_s[];
     screen_bucket_body<SINGLE>(lds_s, points, D, K, ids, starts, sizes, stride, knn_idx, knn_dist, c_err, one_minus_gamma,
-                               nullptr, 0);
+                               nullptr, 0, per_k);
 }
 
 // The kernel of a forest's trees: every workgroup looks at the numbers of pairs the tree before this one left behind
@@ -403,7 +478,7 @@ __global__ __launch_bounds__(kThreads, 4) void k_bucket_knn_auto(const float* __
                                                                  int region_floats,
                                                                  const unsigned long long* __restrict__ prev,
                                                                  unsigned int share_q16,
-                                                                 unsigned long long* __restrict__ stats, int stat_shift)
+                                                                 unsigned long long* __restrict__ stats, int stat_shift, int per_k)
 {
     extern __shared__ __align__(16) float lds_a[];
     bool screened = share_q16 == kScreenAlways;
@@ -416,7 +491,7 @@ __global__ __launch_bounds__(kThreads, 4) void k_bucket_knn_auto(const float* __
     }
     if (screened)
         screen_bucket_body<SINGLE>(lds_a, points, D, K, ids, starts, sizes, 0, knn_idx, knn_dist, c_err, one_minus_gamma, stats,
-                                   stat_shift);
+                                   stat_shift, per_k);
     else
         small_bucket::small_bucket_body<kCap, kThreads, 33>(lds_a, points, D, K, ids, starts, sizes, 0, 2, knn_idx, knn_dist,
                                                             chunk, pitch, region_floats, 1, stats, stat_shift);
@@ -461,10 +536,10 @@ int launch_bucket_knn_screen(const float* points, int D, int K, const int* ids, 
     const dim3 grid((unsigned)n_buckets), block(kThreads);
     if (D <= kChunk)
         hipLaunchKernelGGL(k_bucket_knn_screen<true>, grid, block, kScreenLdsBytes, stream, points, D, K, ids, starts, sizes,
-                           stride, knn_idx, knn_dist, c_err, one_minus_gamma);
+                           stride, knn_idx, knn_dist, c_err, one_minus_gamma, turn_per_k(K));
     else
         hipLaunchKernelGGL(k_bucket_knn_screen<false>, grid, block, kScreenLdsBytes, stream, points, D, K, ids, starts, sizes,
-                           stride, knn_idx, knn_dist, c_err, one_minus_gamma);
+                           stride, knn_idx, knn_dist, c_err, one_minus_gamma, turn_per_k(K));
     RSFK_HIP(hipGetLastError());
     return 0;
 }
@@ -492,24 +567,22 @@ int launch_bucket_knn_auto(const float* points, int D, int K, const int* ids, co
     const dim3 grid((unsigned)n_buckets), block(kThreads);
     if (D <= kChunk)
         hipLaunchKernelGGL(k_bucket_knn_auto<true>, grid, block, lds, stream, points, D, K, ids, starts, sizes, knn_idx, knn_dist,
-                           c_err, one_minus_gamma, chunk, pitch, region_floats, prev, share_q16, stats, stat_shift);
+                           c_err, one_minus_gamma, chunk, pitch, region_floats, prev, share_q16, stats, stat_shift, turn_per_k(K));
     else
         hipLaunchKernelGGL(k_bucket_knn_auto<false>, grid, block, lds, stream, points, D, K, ids, starts, sizes, knn_idx, knn_dist,
-                           c_err, one_minus_gamma, chunk, pitch, region_floats, prev, share_q16, stats, stat_shift);
+                           c_err, one_minus_gamma, chunk, pitch, region_floats, prev, share_q16, stats, stat_shift, turn_per_k(K));
     RSFK_HIP(hipGetLastError());
     return 0;
 }
 
-// The small buckets of a tree take the screened form of the kernel when, in the tree before, less than this share
-// (in 1 / 65536) of the pairs had to be evaluated exactly.  Every pair that passes the bound costs more in the
-// screened form (its chain reads two rows from LDS on its own, where the direct form shares them among the four pairs
-// of a block, and the rows pass through LDS twice), every pair that does not costs less: measured on uniform 100-
-// dimensional and clustered 256-dimensional points the two forms take the same time when about four fifths of the
-// pairs pass (the second tree of a build), and the screened form is ahead from the third tree on (43 to 48 %).  RSFK_BUCKET_SCREEN=<percent> overrides; "never" = 0; "always" = the screened form for every tree and for the
+// Share of the pairs of the tree before that had to be evaluated exactly, below which a tree takes the screened form.  The tree
+// before says more than this one will: 1M x 100 and 1M x 256, the third tree sees about four fifths from the second and has
+// less than half itself, and takes 0.69 and 1.02 ms screened, 0.88 and 1.12 direct; the second tree sees all pairs of the first, whose rows
+// are new, and stays direct.  RSFK_BUCKET_SCREEN=<percent> overrides; "never" = 0; "always" = the screened form for every tree and for the
 // stage-level call as well (kScreenAlways).
 unsigned int bucket_screen_share_q16()
 {
-    double pct = 60.0;
+    double pct = 90.0;
     const char* e = std::getenv("RSFK_BUCKET_SCREEN");          // (read at every call: tests change it)
     if (e && *e) {
         if (e[0] == 'a') return kScreenAlways;

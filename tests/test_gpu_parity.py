@@ -538,10 +538,11 @@ def test_find_nearest_neighbors_matches_oracle(gpu, orc, rng, monkeypatch, N, D,
 @pytest.mark.parametrize("data", ["normal", "clusters", "offset", "equal", "huge", "tiny", "rows"])
 @pytest.mark.parametrize("N,D,K,mn,mx", [(3000, 2, 5, 60, 128), (3100, 16, 64, 65, 192), (2900, 17, 32, 64, 256), (3000, 32, 32, 64, 256),
                                          (4000, 33, 1, 64, 160), (3000, 36, 64, 65, 256), (2500, 44, 40, 60, 192),
-                                         (2600, 49, 33, 60, 128), (2400, 64, 63, 64, 128), (2300, 68, 20, 60, 128)])
+                                         (2600, 49, 33, 60, 128), (2400, 64, 63, 64, 128), (2300, 68, 20, 60, 128),
+                                         (3000, 20, 16, 17, 40), (3000, 100, 32, 32, 64), (2500, 64, 1, 4, 10), (2500, 130, 31, 32, 64)])
 @pytest.mark.parametrize("screen", ["rule", "always"])
-def test_later_trees_of_resident_buckets(gpu, capi, orc, rng, monkeypatch, N, D, K, mn, mx, data, screen):
-    """Buckets that fit into LDS whole, pairs bounded on the matrix cores (any remainder of dimensions, tiles and rows; bounds that
+def test_later_trees_bound_pairs_and_merge_by_turns(gpu, capi, orc, rng, monkeypatch, N, D, K, mn, mx, data, screen):
+    """Buckets that fit into LDS whole, and of at most 64 points, pairs bounded on the matrix cores (any remainder of dimensions, tiles and rows; bounds that
     drop nothing, rows that differ by less than the bound, equal rows), slots found by counting: from the tree the rule says, and from
     the first one on (more candidates of a member than lanes).  "rows": the caller's rows hold neighbours already, in any order."""
     monkeypatch.setenv("RSFK_FOREST_MERGE", "0")
