@@ -816,6 +816,7 @@ __device__ __forceinline__ void emit_leaf(int tree, int gstart, int count, int d
 __device__ __forceinline__ bool often_in_vain(int count, int MIN) { return 8 * (count - 2 * MIN + 1) <= count; }
 
 constexpr int kTailMost = 2048;      // points of the largest node the tail kernel takes
+constexpr int kVainMost = 4;         // splits in vain in a row after which a node leaves for the chain phase
 constexpr int kMaxGroup = 16;        // nodes of one level of a subtree worked on together
 
 // One workgroup finishes the subtree of a task level by level: the nodes of a level are taken kMaxGroup (or
@@ -824,7 +825,7 @@ constexpr int kMaxGroup = 16;        // nodes of one level of a subtree worked o
 // subtree is a few per level instead of a few per node.
 // TB = threads per workgroup: 256, or 512 / 1024 for launches over so few subtrees that workgroups of 256 would leave
 // most of the device idle (the phases of a level then have more lanes).  CHAIN: nodes of at most P.chain_max points go
-// to the queue of the chain phase.  The form of 256 threads is for many subtrees and lives by six wavefronts per SIMD, for which
+// to the queue of the chain phase; otherwise those of them that have been split in vain kVainMost times in a row.  The form of 256 threads is for many subtrees and lives by six wavefronts per SIMD, for which
 // it has to stay within 80 registers (81 and five wavefronts: 1M x 100, 50 trees 10.8 -> 12.3 ms).
 // LPP: lanes per point in the screen (k_side), eight with the bfloat16 copy; KU: 16-byte pieces of a point's row each of them has in
 // flight.
@@ -1066,6 +1067,33 @@ __global__ __launch_bounds__(TB, CHAIN ? 4 : 6) void k_tail(const float* __restr
                         }
                     }
                 }
+                // (many subtrees: a node leaves for the chain phase when it has been split in vain kVainMost times in a row)
+                bool leaves = false;
+                if constexpr (!CHAIN) {
+                    const bool vain = nc == 1 && !c0.leaf && c0.depth < P.MAX_DEPTH - 1;
+                    leaves = vain && nd.leaf >= kVainMost - 1 && c0.count <= P.chain_max;
+                    const bool front = often_in_vain(c0.count, P.MIN);
+                    const uint64_t m = ballot64(leaves), mf = ballot64(leaves && front), mb = m & ~mf;
+                    if (m != 0) {
+                        const int lead = first_lane(m);
+                        int at_f = 0, at_b = 0;
+                        if (lane == lead) {
+                            if (mf != 0) at_f = atomicAdd(&ctr->n_chain, (int)__popcll(mf));
+                            if (mb != 0) at_b = atomicAdd(&ctr->n_chain_back, (int)__popcll(mb));
+                        }
+                        at_f = __shfl(at_f, lead, 64) + mask_prefix(mf);
+                        at_b = __shfl(at_b, lead, 64) + mask_prefix(mb);
+                        if (leaves) {
+                            TreeNode c = c0;
+                            c.start += tk.start;
+                            c.dstart += tk.start;
+                            c.buf = 0;
+                            c.chunk0 = 0;
+                            const int at = front ? at_f : at_b;
+                            if (at < chain_cap) chain_all[front ? at : chain_cap - 1 - at] = c; else ctr->overflow = 1;
+                        }
+                    }
+                }
                 auto child = [&](const TreeNode& c) {
                     if (c.leaf || c.depth >= P.MAX_DEPTH - 1) {
                         record_leaf(c.start, c.count, c.depth, c.rec);
@@ -1076,7 +1104,8 @@ __global__ __launch_bounds__(TB, CHAIN ? 4 : 6) void k_tail(const float* __restr
                             SmallNode sn;
                             sn.start = c.start; sn.count = c.count; sn.dstart = c.dstart; sn.dcount = c.dcount;
                             sn.depth = c.depth;
-                            sn.leaf = 0; sn.key = c.key; sn.rec = c.rec;
+                            sn.leaf = !CHAIN && nc == 1 ? nd.leaf + 1 : 0;             // (splits in vain before this one)
+                            sn.key = c.key; sn.rec = c.rec;
                             if (small) {
                                 const int back = often_in_vain(c.count, P.MIN) ? 0 : 1;
                                 sn.leaf = 2 * atomicAdd(&n_chain_s[back], 1) + back;       // (its place in that part of the queue)
@@ -1087,7 +1116,7 @@ __global__ __launch_bounds__(TB, CHAIN ? 4 : 6) void k_tail(const float* __restr
                         }
                     }
                 };
-                child(c0);
+                if (!leaves) child(c0);
                 if (nc == 2) child(c1);
             }
             __syncthreads();
@@ -2494,9 +2523,13 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
     // tail
     // Few subtrees (small inputs, few trees): what counts is how long the longest of them takes.  Workgroups of 1024 threads
     // while every subtree has a compute unit to itself, of 512 beyond that (so that all of them are resident at once:
-    // 20,000 x 32, 50 trees, 808 subtrees 1.69 -> 1.58 ms for the trees), and nodes that are split in vain leave for the
-    // chain phase.  With more subtrees than that the device is full anyway and the chains run beside the rest: the
-    // chain phase then only adds its matrices (1M x 100, 50 trees: tail 10.7 -> 9.0 ms, chains 6.8 ms).
+    // 20,000 x 32, 50 trees, 808 subtrees 1.69 -> 1.58 ms for the trees), and every node the chain phase takes leaves for it.
+    // With more subtrees than that the device is full anyway and that would only add the matrices (1M x 100, 50 trees: tail 10.9 ->
+    // 9.5 ms, chains 9.9 ms), so a node stays until it has been split in vain kVainMost times in a row: those that
+    // never come to an end keep a workgroup waiting for one node, a level per split.  Whole build without / with, kVainMost = 4:
+    // clustered points 82,121 x 244, K = 5, 50 trees 32.3 -> 15.0 ms; 200,000 x 100, K = 8, 40 trees 29.6 -> 13.2; 1M x 16, K = 4, 20 trees
+    // 48.0 -> 32.1; 1M x 256, K = 32, 20 trees 93.5 -> 91.5; uniform points 1M x 100, K = 32, 50 trees 51.7 -> 50.3; 1M x 32, K = 5, 10 trees
+    // 11.37 -> 11.46.  After 1, 2 or 3 splits in vain the last three take 94.6 / 93.6 / 93.4, 52.0 / 50.7 / 50.3, 12.9 / 12.2 / 11.9 ms.
     // RSFK_TAIL_BLOCK=256 / 1024: as with many / as with few subtrees, whatever their number.
     RSFK_CHECK(n_tail <= w->tail_cap, "tree batch: tail queue overflow");
     if (mid && n_tail > 0) {
@@ -2564,7 +2597,7 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
 #undef RSFK_TAIL_LAUNCH
         RSFK_HIP(hipGetLastError());
     }
-    if (few && P.chain_max > 0) {
+    if (P.chain_max > 0) {
         const int node_cap = P.chain_max / std::max(MIN, 1) + 4;
         const size_t lds = chain_lds_bytes(P.chain_max, node_cap, w->recs != nullptr);
         const size_t most = (size_t)N * (size_t)nb / (size_t)std::max(MAX - 1, 1) + (size_t)nb;      // nodes that are no buckets are disjoint

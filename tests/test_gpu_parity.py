@@ -147,10 +147,13 @@ def test_tree_of_rows_whose_sums_leave_fp32(gpu, orc, rng, monkeypatch, kind, en
     (9000, 19, 96, 191, 2048, "n"), (9000, 19, 96, 255, 2048, "n"), (9000, 19, 128, 256, 2048, "n"), (9000, 32, 3, 6, 2048, "n"),
     (30000, 32, 17, 34, 80, "n"), (30000, 64, 17, 34, 80, "n"), (30000, 65, 17, 34, 80, "n"), (12000, 256, 33, 66, 2048, "n"),
     (8000, 257, 33, 66, 2048, "n"), (9000, 24, 33, 66, 2048, "nan"), (9000, 24, 33, 66, 2048, "far"), (9000, 24, 96, 192, 2048, "far"),
-    (9000, 36, 33, 66, 2048, "clusters"), (9000, 36, 8, 16, 2048, "clusters"),
+    (9000, 36, 33, 66, 2048, "clusters"), (9000, 36, 8, 16, 2048, "clusters"), (6000, 9, 5, 10, 2048, "dup"), (20000, 50, 4, 8, 500, "clusters"),
 ])
 @pytest.mark.parametrize("screen", ["q8", "bf16"])
-def test_tree_forms_of_tail_and_chain(gpu, orc, rng, monkeypatch, N, D, MIN, MAX, small, kind, screen):
+@pytest.mark.parametrize("subtrees", ["few", "many"])
+def test_tree_forms_of_tail_and_chain(gpu, orc, rng, monkeypatch, N, D, MIN, MAX, small, kind, screen, subtrees):
+    if subtrees == "many":                                      # nodes leave for the chain phase after splits in vain
+        monkeypatch.setenv("RSFK_TAIL_BLOCK", "256")
     monkeypatch.setenv("RSFK_TREE_SCREEN", screen)
     monkeypatch.setenv("RSFK_TREE_SMALL", str(small))
     X = rng.standard_normal((N, D)).astype(np.float32)
@@ -158,6 +161,8 @@ def test_tree_forms_of_tail_and_chain(gpu, orc, rng, monkeypatch, N, D, MIN, MAX
         X[rng.random(N) < 0.01, 1] = np.nan
     if kind == "far":
         X[rng.random(N) < 0.02] *= np.float32(1e3)
+    if kind == "dup":
+        X[: N // 3] = X[0]
     if kind == "clusters":
         X = (10.0 * rng.standard_normal((40, D))[rng.integers(0, 40, N)] + 1e-3 * X).astype(np.float32)
     for seed in (1, 2):
@@ -167,6 +172,20 @@ def test_tree_forms_of_tail_and_chain(gpu, orc, rng, monkeypatch, N, D, MIN, MAX
         assert np.array_equal(gperm, perm)
         assert np.array_equal(gls, ls) and np.array_equal(glz, lz)
         assert list(gst) == [len(ls), st[0], st[1], st[2]]
+
+
+@pytest.mark.parametrize("K", [3, 12])
+def test_index_of_nodes_that_leave_the_tail(gpu, orc, rng, monkeypatch, K):
+    """Many subtrees: the index that query points are routed by, where nodes leave for the chain phase after splits in vain."""
+    import gpu_rsfk
+    monkeypatch.setenv("RSFK_TAIL_BLOCK", "256")
+    N, NQ, D = 20000, 1500, 30
+    X = (10.0 * rng.standard_normal((50, D))[rng.integers(0, 50, N + NQ)] + 0.3 * rng.standard_normal((N + NQ, D))).astype(np.float32)
+    X, Q = np.ascontiguousarray(X[:N]), np.ascontiguousarray(X[N:])
+    _say("index, splits in vain", K)
+    gi, gd = gpu_rsfk.RSFK(random_state=5).find_nearest_neighbors_ann(X, Q, K, n_trees=3)
+    oi, od = orc.ann_forest(X, Q, K, 3, K + 1, 2 * (K + 1), 5000, 5)
+    assert_knn_equal(gi, gd, oi, od)
 
 
 # The middle phase: nodes it takes whole (N at most its largest), from the wide levels, of sizes around a thread's last entry, one that
