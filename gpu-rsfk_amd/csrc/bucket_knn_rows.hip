@@ -31,7 +31,7 @@
 #include "knn_list.hpp"
 #include "forest.hpp"
 #include "bucket_small_body.hpp"
-#include "bucket_rows_stage.hpp"
+#include "bucket_knn_stage.hpp"
 #include <algorithm>
 
 namespace rsfk {

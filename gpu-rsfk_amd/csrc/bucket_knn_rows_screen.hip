@@ -35,8 +35,8 @@
 #include "knn_list.hpp"
 #include "mfma_split.hpp"
 #include "forest.hpp"
-#include "bucket_rows_stage.hpp"
-#include "row_turn.hpp"
+#include "bucket_knn_stage.hpp"
+#include "bucket_knn_turn.hpp"
 #include <algorithm>
 
 namespace rsfk {

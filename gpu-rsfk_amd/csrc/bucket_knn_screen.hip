@@ -29,7 +29,7 @@
 //      compute_knn_from_buckets.cu:40-54: a pair has the same distance value as in
 //      every other kernel);
 //   4. an exact distance that is not above the last slot of a row is an offer to it.  The offers are put in the order of the
-//      rows, in LDS, and go into them by turns of up to 64 offers and 256 slots (row_turn.hpp), half of the offers per wavefront.
+//      rows, in LDS, and go into them by turns of up to 64 offers and 256 slots (bucket_knn_turn.hpp), half of the offers per wavefront.
 //      Rows merged one after the other took 46 % of the kernel's time in a late tree and more before: 1M x 100, K = 32, fourth tree
 //      0.70 -> 0.47 ms, tenth 0.41 -> 0.35, 50th 0.25 -> 0.25 (0.9 GB moved: 3.7 TB/s); 1M x 256 fourth 0.92 -> 0.75, tenth 0.56 -> 0.54.
 //      A bucket with more pairs than the list holds keeps a distance matrix in LDS, and its rows are merged as in the other kernel.
@@ -40,7 +40,7 @@
 #include "knn_list.hpp"
 #include "forest.hpp"
 #include "mfma_split.hpp"
-#include "row_turn.hpp"
+#include "bucket_knn_turn.hpp"
 #include "bucket_small_body.hpp"
 #include <algorithm>
 #include <cstdlib>
