@@ -547,13 +547,12 @@ int launch_bucket_knn(const float* points, int N, int D, int K, const int* ids, 
 
 // Host launcher for the leaf table of one tree: n_small buckets of at most kBucketSplit points at the front of
 // (starts, sizes), n_big larger ones at the back of the table of leaf_cap entries.  rows_sorted: every K-NN row is
-// known to be sorted by distance.  stats (8 zeroed words; with K <= 64 and sorted rows): the small buckets go to the
-// kernel that chooses between the direct and the screened form from the pairs of the tree before (prev_stats, null for
-// the first tree) and leaves its own numbers in stats.  part: 0 = all buckets, 1 = only the small ones, 2 = only the larger ones (the two
+// known to be sorted by distance.  form (may be null; with K <= 64 and sorted rows): the small buckets go to the kernel that
+// chooses between the direct and the screened form.  part: 0 = all buckets, 1 = only the small ones, 2 = only the larger ones (the two
 // kinds touch different rows, so the two parts of one tree may run side by side).  trees_before: trees of the build
 // whose buckets have been through.  pairs: working memory for the buckets that reach the general kernel (null:
 // its forms that need none); launches that may run side by side need one each.
-int launch_bucket_knn_tree(const float* points, const unsigned long long* prev_stats, unsigned long long* stats,
+int launch_bucket_knn_tree(const float* points, const SmallBucketForm* form,
                            bool rows_sorted, bool gram, int D, int K, const int* ids, const int* starts, const int* sizes,
                            int leaf_cap, int n_small, int n_big, int max_bucket, int* knn_idx, float* knn_dist,
                            hipStream_t stream, int part, int trees_before, int* launched, const PairScratch* pairs)
@@ -583,9 +582,9 @@ int launch_bucket_knn_tree(const float* points, const unsigned long long* prev_s
                                       stream);
     }
     if (n_small > 0 && part != 2) {
-        if (K <= 64 && stats && rows_sorted) {
+        if (K <= 64 && form && rows_sorted) {
             used |= kBucketKernelAuto;
-            if (launch_bucket_knn_auto(points, D, K, ids, starts, sizes, n_small, knn_idx, knn_dist, prev_stats, stats, stream))
+            if (launch_bucket_knn_auto(points, D, K, ids, starts, sizes, n_small, knn_idx, knn_dist, *form, stream))
                 return 1;
         } else if (K <= 64) {
             used |= kBucketKernelSmall;

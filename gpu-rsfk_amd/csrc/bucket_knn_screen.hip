@@ -120,15 +120,8 @@ struct RowLoads {
 // pass takes the chunks from the last to the first, so that the first one is still in LDS when the exact chains --
 // which must run from dimension 0 upwards -- begin; only the chunks after it pass through LDS a second time, and the
 // first of those is requested before the bounds are evaluated.
-// stats (may be null): the workgroups whose number is a multiple of 2^stat_shift add pairs of the bucket << 32 | pairs
-// that got an exact distance to one of its 8 words (a sample of the buckets, see small_bucket_body).
-// The work of one workgroup on bucket blockIdx.x; lds: kScreenLdsBytes bytes of LDS.
-constexpr int kPitch = kChunk + 4;                        // an odd number of 16-byte units: rows start in different banks
-constexpr int kRegion = kCap * kPitch > kCap * kDistPitch ? kCap * kPitch : kCap * kDistPitch;
-constexpr size_t kScreenLdsBytes = sizeof(float) * kRegion + sizeof(ScreenMeta);
-static_assert(sizeof(ScreenTurns) <= sizeof(float) * kRegion, "the turns take the place of the rows");
-static_assert(kScreenLdsBytes <= 160 * 1024 / 8, "eight workgroups per compute unit");
-
+// stats (may be null): the workgroups whose number is a multiple of 2^stat_shift add the numbers of pairs of their bucket to
+// two of its words, for bucket_form (a sample of the buckets, see small_bucket_body).
 template <bool SINGLE>
 __device__ __forceinline__ void screen_bucket_body(float* __restrict__ lds, const float* __restrict__ points, int D, int K,
                                                    const int* __restrict__ ids, const int* __restrict__ starts,
@@ -254,8 +247,13 @@ __device__ __forceinline__ void screen_bucket_body(float* __restrict__ lds, cons
     }
     __syncthreads();
     const int n_passed = M.n_pairs[0];
-    if (stats && tid == 0 && (bkt & ((1 << stat_shift) - 1)) == 0)
-        atomicAdd(&stats[(bkt >> stat_shift) & 7], ((unsigned long long)(s * (s - 1) / 2) << 32) | (unsigned long long)n_passed);
+    const bool sampled = stats && (bkt & ((1 << stat_shift) - 1)) == 0;
+    unsigned long long* const words = stats + ((bkt >> stat_shift) & 3);
+    const unsigned long long pairs = (unsigned long long)(s * (s - 1) / 2) << 32;
+    if (sampled && tid == 0) {
+        atomicAdd(words + 4, pairs | (unsigned long long)n_passed);
+        if (n_passed == 0) atomicAdd(words, pairs);
+    }
     if (n_passed == 0) return;                        // no pair of this bucket can change a row
 
     // ---- 3. exact distances of the listed pairs: thread t takes entries t, t + 128, ...
@@ -313,6 +311,16 @@ __device__ __forceinline__ void screen_bucket_body(float* __restrict__ lds, cons
             if (c + 1 < n_chunks) ld.request(lids, s, points, D, (c + 1) * kChunk, vec_ok);
             chains(min(kChunk, (D - c * kChunk + 3) & ~3) >> 2);
         }
+    }
+    if (sampled) {
+        int offered = 0;
+#pragma unroll
+        for (int r = 0; r < kMaxRounds; ++r) {
+            const uint32_t e = entry(r);
+            if (tid + r * kThreads < n_list && acc[r] <= fmaxf(M.tau[e & 63u], M.tau[e >> 6])) ++offered;
+        }
+        offered = wave_sum_i(offered);
+        if (lane == 0 && (wave == 0 || offered > 0)) atomicAdd(words, (unsigned long long)offered | (wave == 0 ? pairs : 0ull));
     }
     __syncthreads();                                  // rows no longer needed: their place is used for what follows
     if (!all_pairs) {
@@ -463,12 +471,9 @@ __global__ __launch_bounds__(kThreads, 4) void k_bucket_knn_screen(const float* 
                                nullptr, 0, per_k);
 }
 
-// The kernel of a forest's trees: every workgroup looks at the numbers of pairs the tree before this one left behind
-// (prev: 8 words, pairs << 32 | pairs that had to be evaluated exactly, as both forms of the kernel count them in a
-// sample of the buckets) and
-// takes the screened form when fewer than share_q16 / 65536 of the pairs had to be, the direct form otherwise (and
-// for the first tree, prev == null).  One scalar load and a few scalar instructions per workgroup; both forms leave
-// their own numbers in stats for the next tree.  All K-NN rows sorted on entry.
+// The kernel of a forest's trees: every workgroup looks at the numbers of pairs the tree before this one left behind (prev; null:
+// the first tree, direct) and takes the form that bucket_form says.  One scalar load and a few scalar instructions per workgroup;
+// both forms leave their own numbers in stats for the next tree.  All K-NN rows sorted on entry.
 template <bool SINGLE>
 __global__ __launch_bounds__(kThreads, 4) void k_bucket_knn_auto(const float* __restrict__ points, int D, int K,
                                                                  const int* __restrict__ ids, const int* __restrict__ starts,
@@ -477,24 +482,18 @@ __global__ __launch_bounds__(kThreads, 4) void k_bucket_knn_auto(const float* __
                                                                  float one_minus_gamma, int chunk, int pitch,
                                                                  int region_floats,
                                                                  const unsigned long long* __restrict__ prev,
-                                                                 unsigned int share_q16,
+                                                                 BucketFormRule rule,
                                                                  unsigned long long* __restrict__ stats, int stat_shift, int per_k)
 {
     extern __shared__ __align__(16) float lds_a[];
-    bool screened = share_q16 == kScreenAlways;
-    if (prev && !screened) {
-        unsigned long long sum = 0;                      // (the halves cannot carry into each other: a tree has < 2^32 pairs)
-#pragma unroll
-        for (int i = 0; i < 8; ++i) sum += prev[i];
-        const unsigned long long listed = sum & 0xffffffffull, total = sum >> 32;
-        screened = total > 0 && (listed << 16) < total * share_q16;
-    }
-    if (screened)
+    BucketForm form = {rule.share_q16 == kScreenAlways, false};
+    if (prev) form = bucket_form(prev, rule);
+    if (form.screened)
         screen_bucket_body<SINGLE>(lds_a, points, D, K, ids, starts, sizes, 0, knn_idx, knn_dist, c_err, one_minus_gamma, stats,
                                    stat_shift, per_k);
     else
         small_bucket::small_bucket_body<kCap, kThreads, 33>(lds_a, points, D, K, ids, starts, sizes, 0, 2, knn_idx, knn_dist,
-                                                            chunk, pitch, region_floats, 1, stats, stat_shift);
+                                                            chunk, pitch, region_floats, 1, stats, stat_shift, form.vain);
 }
 
 // one wavefront per row: rows that are not sorted by distance are rebuilt by insertion
@@ -545,11 +544,8 @@ int launch_bucket_knn_screen(const float* points, int D, int K, const int* ids, 
 }
 
 // The small buckets (2..64 points, starts / sizes form) of one tree of a forest; every K-NN row sorted on entry.
-// prev: the 8 words a launch of this kind (or of either form) left for the tree before, or null for the first tree;
-// stats: 8 zeroed words for this tree.  The form of the kernel is chosen on the device from prev (k_bucket_knn_auto).
 int launch_bucket_knn_auto(const float* points, int D, int K, const int* ids, const int* starts, const int* sizes,
-                           int n_buckets, int* knn_idx, float* knn_dist, const unsigned long long* prev,
-                           unsigned long long* stats, hipStream_t stream)
+                           int n_buckets, int* knn_idx, float* knn_dist, const SmallBucketForm& form, hipStream_t stream)
 {
     if (n_buckets <= 0) return 0;
     RSFK_CHECK(K >= 1 && K <= 64 && D >= 1, "small-bucket kernel: K must be in 1..64 and D positive");
@@ -560,24 +556,23 @@ int launch_bucket_knn_auto(const float* points, int D, int K, const int* ids, co
     small_bucket::small_bucket_shape(D, &chunk, &pitch);
     const int region_floats = small_bucket::small_bucket_region_floats<kCap, kThreads, 33>(pitch);
     const size_t lds = std::max(kScreenLdsBytes, small_bucket::small_bucket_lds_bytes<kCap, kThreads, 33>(pitch));
-    const unsigned int share_q16 = bucket_screen_share_q16();
-    // about 256 to 512 of the buckets are counted
+    // about 128 to 256 of the buckets are counted, with three additions to one cache line each
     int stat_shift = 0;
-    while ((n_buckets >> (stat_shift + 1)) >= 256) ++stat_shift;
+    while ((n_buckets >> (stat_shift + 1)) >= 128) ++stat_shift;
     const dim3 grid((unsigned)n_buckets), block(kThreads);
     if (D <= kChunk)
         hipLaunchKernelGGL(k_bucket_knn_auto<true>, grid, block, lds, stream, points, D, K, ids, starts, sizes, knn_idx, knn_dist,
-                           c_err, one_minus_gamma, chunk, pitch, region_floats, prev, share_q16, stats, stat_shift, turn_per_k(K));
+                           c_err, one_minus_gamma, chunk, pitch, region_floats, form.prev, form.rule, form.words, stat_shift, turn_per_k(K));
     else
         hipLaunchKernelGGL(k_bucket_knn_auto<false>, grid, block, lds, stream, points, D, K, ids, starts, sizes, knn_idx, knn_dist,
-                           c_err, one_minus_gamma, chunk, pitch, region_floats, prev, share_q16, stats, stat_shift, turn_per_k(K));
+                           c_err, one_minus_gamma, chunk, pitch, region_floats, form.prev, form.rule, form.words, stat_shift, turn_per_k(K));
     RSFK_HIP(hipGetLastError());
     return 0;
 }
 
-// Share of the pairs of the tree before that had to be evaluated exactly, below which a tree takes the screened form.  The tree
-// before says more than this one will: 1M x 100 and 1M x 256, the third tree sees about four fifths from the second and has
-// less than half itself, and takes 0.69 and 1.02 ms screened, 0.88 and 1.12 direct; the second tree sees all pairs of the first, whose rows
+// Share of the pairs of the tree before that were offered to a row, below which a tree takes the screened form.  The tree before
+// says more than this one will: 1M x 100 and 1M x 256, K = 32, the third tree sees about four fifths from the second and has less than
+// half itself, and takes 0.69 and 1.02 ms screened, 0.88 and 1.12 direct; the second tree sees all pairs of the first, whose rows
 // are new, and stays direct.  RSFK_BUCKET_SCREEN=<percent> overrides; "never" = 0; "always" = the screened form for every tree and for the
 // stage-level call as well (kScreenAlways).
 unsigned int bucket_screen_share_q16()
@@ -590,6 +585,38 @@ unsigned int bucket_screen_share_q16()
     }
     pct = std::min(100.0, std::max(0.0, pct));
     return (unsigned int)(pct * 65536.0 / 100.0 + (pct >= 100.0 ? 1.0 : 0.0));
+}
+
+// The screened form against the direct one, 1M points (time of a tree, screened / direct, third ... tenth tree):
+//   points of a bucket   D = 4         32            64            100           256 (400,000)
+//    6.8                 1.29 .. 1.37  1.21 .. 1.27  1.17 .. 1.19  1.34 .. 1.32  1.27 .. 1.20
+//    9.5                 1.07 .. 1.23  1.00 .. 1.26  0.98 .. 1.17  1.15 .. 1.32  1.13 .. 1.23
+//   12.2                 0.89 .. 1.09  0.85 .. 1.13  0.83 .. 1.06  0.98 .. 1.20  1.02 .. 1.16
+//   14.9                 0.81 .. 1.00  0.76 .. 1.03  0.75 .. 0.97  0.87 .. 1.09  0.92 .. 1.07
+//   17.6                 0.75 .. 0.93  0.70 .. 0.94  0.70 .. 0.89  0.81 .. 0.99  0.86 .. 1.01
+//   23                   0.71 .. 0.85  0.63 .. 0.79  0.64 .. 0.77  0.71 .. 0.84  0.78 .. 0.84
+// Few points leave few chains to save; what the screened form gains there it gains at merging the offers, as long as about three per
+// row are left.  So: from 16 points on; from 12 (14 with more than one chunk of dimensions) while a row gets three offers.
+// The bound is a share of the norms: points far from the origin, or of two dimensions, it does not tell apart.  Buckets of about 40
+// points (always screened / direct, 50 trees; share of the pairs that is listed for nothing, from the third tree on):
+//   D = 8, uniform + 10   K = 4: 1.28 (0.37 .. 0.36)   8: 1.16 (0.39 .. 0.36)   31: 1.16 (0.31 .. 0.40)
+//   D = 16, uniform + 12  K = 4: 1.13 (0.18 .. 0.11)   8: 1.01 (0.21 .. 0.13)   31: 1.03 (0.21 .. 0.20)
+//   D = 32, uniform + 16  K = 4: 1.18 (0.34 .. 0.21)   8: 1.10 (0.43 .. 0.28)   31: 1.10 (0.41 .. 0.43)
+//   D = 64, uniform + 12  K = 4: 0.95 (0.28 .. 0.15)   8: 0.92 (0.38 .. 0.21)   31: 1.01 (0.39 .. 0.37); + 16: 1.2 (0.6 .. 0.4)
+//   D = 100, uniform + 10 K = 4: 0.97 (0.32 .. 0.16)   8: 0.96 (0.42 .. 0.24)   31: 1.04 (0.41 .. 0.40); + 14: 1.3 (0.7 .. 0.6)
+// So: no longer once 1/3 + D/384 of the pairs, at most half of them, were listed for nothing.  Buckets of at most 42 points keep all their
+// pairs in the list and are merged by turns whatever the bound leaves (23 points, every pair listed: 0.7 .. 0.9 while an eighth
+// of the pairs is offered): with fewer than 28 points on average, 7/8.
+BucketFormRule bucket_form_rule(double mean, int D)
+{
+    constexpr unsigned int kNever = 0xffffffffu;
+    BucketFormRule rule = {bucket_screen_share_q16(), 0u, kNever};
+    const char* e = std::getenv("RSFK_BUCKET_SCREEN");
+    if (e && *e) return rule;                                    // (a share, always or never: nothing else is asked)
+    if (mean < (D <= kChunk ? 12.0 : 14.0)) rule.share_q16 = 0;
+    else if (mean < 16.0) rule.least_q16 = (unsigned int)(3.0 * 65536.0 / mean);
+    rule.vain_q16 = (unsigned int)(65536.0 * (mean < 28.0 ? 0.875 : std::min(0.5, 1.0 / 3.0 + D / 384.0)));
+    return rule;
 }
 
 }  // namespace rsfk

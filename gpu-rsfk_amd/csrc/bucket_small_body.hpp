@@ -84,16 +84,16 @@ struct SmallCfg {
 // The work of one workgroup (THREADS threads) on bucket blockIdx.x.  lds_f: the workgroup's LDS,
 // small_bucket_lds_bytes<...>(pitch) bytes.  min_size: smaller buckets are left to another launch.
 // stats (may be null): the workgroups whose number is a multiple of 2^stat_shift add pairs of the bucket << 32 | pairs
-// whose distance is not above the last slot of one of the two rows (what the screened kernel would have to evaluate
-// exactly) to one of its 8 words -- a sample of the buckets: one addition per workgroup to so few words would take
-// longer than the kernel.
+// whose distance is not above the last slot of one of the two rows to one of its first four words (bucket_form) -- a sample
+// of the buckets: one addition per workgroup to so few words would take longer than the kernel.  vain: the bound of the screened
+// form does not decide enough, and this is passed on to the trees after this one (the bound stays as it is and the last slots fall).
 template <int CAP, int THREADS, int SPACING>
 __device__ __forceinline__ void small_bucket_body(float* __restrict__ lds_f, const float* __restrict__ points, int D, int K,
                                                   const int* __restrict__ ids, const int* __restrict__ starts,
                                                   const int* __restrict__ sizes, int stride, int min_size,
                                                   int* __restrict__ knn_idx, float* __restrict__ knn_dist, int chunk,
                                                   int pitch, int region_floats, int rows_sorted,
-                                                  unsigned long long* __restrict__ stats, int stat_shift)
+                                                  unsigned long long* __restrict__ stats, int stat_shift, bool vain = false)
 {
     using Cfg = SmallCfg<CAP, THREADS, SPACING>;
     constexpr int kCap = CAP, kThreads = THREADS, kWaves = Cfg::kWaves, kSpacing = SPACING;
@@ -229,9 +229,9 @@ __device__ __forceinline__ void small_bucket_body(float* __restrict__ lds_f, con
 
     if (stats && (blockIdx.x & ((1u << stat_shift) - 1u)) == 0) {
         n_pass = wave_sum_i(n_pass);
-        if (lane == 0)
-            atomicAdd(&stats[(blockIdx.x >> stat_shift) & 7],
-                      (unsigned long long)n_pass | (wave == 0 ? (unsigned long long)(s * (s - 1) / 2) << 32 : 0ull));
+        const unsigned long long pairs = (unsigned long long)(s * (s - 1) / 2);
+        if (lane == 0) atomicAdd(&stats[(blockIdx.x >> stat_shift) & 3], (unsigned long long)n_pass | (wave == 0 ? pairs << 32 : 0ull));
+        if (vain && threadIdx.x == 0) atomicAdd(&stats[4 + ((blockIdx.x >> stat_shift) & 3)], pairs << 32 | pairs);
     }
     __syncthreads();                           // distance matrix complete
 

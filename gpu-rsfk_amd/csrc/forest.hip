@@ -40,7 +40,8 @@ namespace {
 struct BuildReport {
     int N = 0, D = 0, K = 0, n_trees = 0, passes = 0, row_bytes = 0;
     std::vector<int> kernels;                          // per tree: kBucketKernel... bits
-    std::vector<unsigned long long> pairs;             // per tree: pairs of its small buckets << 32 | those evaluated exactly
+    std::vector<unsigned long long> form_words;        // per tree: numbers of pairs of its small buckets (bucket_form)
+    std::vector<BucketFormRule> rules;                 // per tree: what its form was chosen by
     unsigned int screen_share_q16 = 0;
     unsigned long long tested = 0, undecided = 0;      // tree build: point-levels, and those left to the exact test
     unsigned long long exact = 0;                      // exploration: exact distances over all passes
@@ -177,25 +178,23 @@ int build_report_json(char* buf, int cap)
         a = b + 1;
     }
     s += "], ";
-    // k_bucket_knn_auto: share of the pairs of a tree's small buckets that had to be evaluated exactly, and the form of
-    // the kernel that share selected for the next tree (the first tree takes the direct form)
+    // k_bucket_knn_auto: share of the pairs of a tree's small buckets that the bound left to the exact test (screened form) or that
+    // were not above the last slot of one of their rows (direct form), and which of the two the tree before selected
+    std::string forms;
     s += "\"bucket_pair_share\": [";
-    for (size_t t = 0; t < r.pairs.size(); ++t) {
-        const double total = (double)(r.pairs[t] >> 32), listed = (double)(r.pairs[t] & 0xffffffffull);
+    for (size_t t = 0; t < r.rules.size(); ++t) {
+        const unsigned long long* w = r.form_words.data() + kFormWords * t;
+        const bool first = t == 0 && r.rules[t].share_q16 != kScreenAlways;
+        const bool scr = !first && (r.kernels[t] & kBucketKernelAuto) && bucket_form(t > 0 ? w - kFormWords : w, r.rules[t]).screened;
+        unsigned long long sum = 0;
+        for (int i = 0; i < kFormWords / 2; ++i) sum += w[scr ? kFormWords / 2 + i : i];
+        const double total = (double)(sum >> 32), exact = (double)(sum & 0xffffffffull);
         char tmp[32];
-        std::snprintf(tmp, sizeof tmp, "%s%.4f", t ? ", " : "", total > 0 ? listed / total : 0.0);
+        std::snprintf(tmp, sizeof tmp, "%s%.4f", t ? ", " : "", total > 0 ? exact / total : 0.0);
         s += tmp;
+        forms += std::string(t ? ", " : "") + (scr ? "1" : "0");
     }
-    s += "], \"bucket_screened\": [";
-    for (size_t t = 0; t < r.pairs.size(); ++t) {
-        bool scr = r.screen_share_q16 == kScreenAlways;
-        if (t > 0 && !scr) {
-            const unsigned long long total = r.pairs[t - 1] >> 32, listed = r.pairs[t - 1] & 0xffffffffull;
-            scr = total > 0 && (listed << 16) < total * r.screen_share_q16;
-        }
-        s += std::string(t ? ", " : "") + ((r.kernels[t] & kBucketKernelAuto) && scr ? "1" : "0");
-    }
-    s += "], ";
+    s += "], \"bucket_screened\": [" + forms + "], ";
     num("bucket_screen_share", r.screen_share_q16 == kScreenAlways ? 2.0 : r.screen_share_q16 / 65536.0);
     num("tree_points_tested", (double)r.tested); num("tree_points_undecided", (double)r.undecided);
     num("tree_screen_row_bytes", r.row_bytes); num("tree_seconds", r.tree_s); num("bucket_seconds", r.bucket_s);
@@ -256,14 +255,15 @@ int knn_forest_device(int n_trees, int K, int N, int D, int MIN, int MAX, int MA
         std::vector<TimedEvent> ev((size_t)B + 1);
         for (auto& e : ev)
             if (e.create()) return 1;
-        // numbers of pairs of every tree's small buckets (8 words per tree, added up on the host for the report): the
-        // kernel of tree t reads those of tree t - 1 to choose its form
+        // numbers of pairs of every tree's small buckets (bucket_form; also for the report): the kernel of tree t reads those of
+        // tree t - 1 to choose its form
         DevBuf pair_stats;
-        const size_t stat_words = (size_t)8 * (size_t)n_trees;
+        const size_t stat_words = (size_t)kFormWords * (size_t)n_trees;
         if (ws_alloc(&pair_stats.p, sizeof(unsigned long long) * stat_words)) return 1;
         RSFK_HIP(hipMemsetAsync(pair_stats.p, 0, sizeof(unsigned long long) * stat_words, stream));
         unsigned long long* d_pairs = static_cast<unsigned long long*>(pair_stats.p);
         rep.screen_share_q16 = bucket_screen_share_q16();
+        rep.rules.assign((size_t)n_trees, BucketFormRule{rep.screen_share_q16, 0, 0});
         const int gram_from = bucket_gram_from();
         SideStream sync;
         if (std::getenv("RSFK_KNN_ONE_STREAM") == nullptr && sync.open()) return 1;
@@ -350,13 +350,17 @@ int knn_forest_device(int n_trees, int K, int N, int D, int MIN, int MAX, int MA
                     if (pair_room(0, split ? want_small : std::max(want_small, want_big))) return 1;
                     if (split && pair_room(1, want_big)) return 1;
                 }
-                rc = launch_bucket_knn_tree(d_points, t > 0 ? d_pairs + (size_t)8 * (t - 1) : nullptr, d_pairs + (size_t)8 * t, true,
-                                            gram, D, K, tree_ws_perm(ws.w, j), tree_ws_leaf_start(ws.w, j),
+                // (points of a small bucket: exact where all are small, else with the larger ones halfway between their limits)
+                const double in_big = 0.5 * n_big * (kBucketSplit + 1 + stats[5 * j + 2]);
+                rep.rules[(size_t)t] = bucket_form_rule(std::max(0.0, (double)N - in_big) / std::max(1, n_small), D);
+                const SmallBucketForm form = {t > 0 ? d_pairs + (size_t)kFormWords * (t - 1) : nullptr, d_pairs + (size_t)kFormWords * t,
+                                              rep.rules[(size_t)t]};
+                rc = launch_bucket_knn_tree(d_points, &form, true, gram, D, K, tree_ws_perm(ws.w, j), tree_ws_leaf_start(ws.w, j),
                                             tree_ws_leaf_size(ws.w, j), tree_ws_leaf_cap(ws.w), n_small, n_big, stats[5 * j + 2],
                                             d_idx, d_dist, stream, split ? 1 : 0, t0 + j, &rep.kernels[(size_t)(t0 + j)],
                                             &pair_mem[0]);
                 if (!rc && split) {
-                    rc = launch_bucket_knn_tree(d_points, nullptr, nullptr, true, gram, D, K, tree_ws_perm(ws.w, j), tree_ws_leaf_start(ws.w, j),
+                    rc = launch_bucket_knn_tree(d_points, nullptr, true, gram, D, K, tree_ws_perm(ws.w, j), tree_ws_leaf_start(ws.w, j),
                                                 tree_ws_leaf_size(ws.w, j), tree_ws_leaf_cap(ws.w), n_small, n_big,
                                                 stats[5 * j + 2], d_idx, d_dist, sync.side, 2, t0 + j,
                                                 &rep.kernels[(size_t)(t0 + j)], &pair_mem[1]);
@@ -403,10 +407,8 @@ int knn_forest_device(int n_trees, int K, int N, int D, int MIN, int MAX, int MA
             RSFK_HIP(hipMemcpyAsync(order.p, tree_ws_perm(ws.w, (n_trees - 1) % B), sizeof(int) * (size_t)N, hipMemcpyDeviceToDevice, stream));
             RSFK_HIP(hipStreamSynchronize(stream));
         }
-        std::vector<unsigned long long> h_pairs(stat_words);
-        RSFK_HIP(hipMemcpy(h_pairs.data(), d_pairs, sizeof(unsigned long long) * stat_words, hipMemcpyDeviceToHost));
-        rep.pairs.assign((size_t)n_trees, 0);
-        for (size_t i = 0; i < stat_words; ++i) rep.pairs[i / 8] += h_pairs[i];
+        rep.form_words.resize(stat_words);
+        RSFK_HIP(hipMemcpy(rep.form_words.data(), d_pairs, sizeof(unsigned long long) * stat_words, hipMemcpyDeviceToHost));
     }
     const double t_forest = now_s() - t_forest0;
     if (verbose >= 1) std::printf("Creating RSFK forest takes %lf seconds\n", t_forest);

@@ -65,7 +65,41 @@ struct PairScratch {
 // several parts.
 size_t pair_scratch_max();
 size_t bucket_pairs_scratch_floats(int D, int K, int n_buckets, int max_bucket);
-int launch_bucket_knn_tree(const float* points, const unsigned long long* prev_stats, unsigned long long* stats,
+// Form of k_bucket_knn_auto (every pair exact, or bounded on the matrix cores first), from what the tree before left in kFormWords
+// words, in a sample of its buckets: words 0..3, pairs << 32 | offered, the pairs that are not above the last slot of one of their rows;
+// words 4..7, pairs << 32 | listed, the pairs that the bound of the screened form left to the exact test, if that form ran.
+constexpr int kFormWords = 8;
+constexpr unsigned int kScreenAlways = 0xffffffffu;
+struct BucketFormRule {
+    unsigned int share_q16;      // screened below this share of offered pairs (in 1 / 65536); kScreenAlways: always
+    unsigned int least_q16;      // ... and not below this one
+    unsigned int vain_q16;       // ... and not once listed less offered pairs were at least this share
+};
+struct BucketForm {
+    bool screened, vain;
+};
+__host__ __device__ __forceinline__ BucketForm bucket_form(const unsigned long long* __restrict__ words, BucketFormRule rule)
+{
+    if (rule.share_q16 == kScreenAlways) return {true, false};
+    unsigned long long a = 0, b = 0;                     // (the halves cannot carry into each other: a tree has < 2^32 pairs)
+#pragma unroll
+    for (int i = 0; i < kFormWords / 2; ++i) {
+        a += words[i];
+        b += words[kFormWords / 2 + i];
+    }
+    const unsigned long long offered = a & 0xffffffffull, pairs = a >> 32, listed = b & 0xffffffffull, bounded = b >> 32;
+    const bool vain = bounded > 0 && ((listed - offered) << 16) >= bounded * rule.vain_q16;
+    return {!vain && pairs > 0 && (offered << 16) < pairs * rule.share_q16 && (offered << 16) >= pairs * rule.least_q16, vain};
+}
+// mean: points of a small bucket of the tree
+BucketFormRule bucket_form_rule(double mean, int D);
+// The small buckets of a tree with sorted rows: words of the tree before (null: first tree) and, zeroed, of this one
+struct SmallBucketForm {
+    const unsigned long long* prev;
+    unsigned long long* words;
+    BucketFormRule rule;
+};
+int launch_bucket_knn_tree(const float* points, const SmallBucketForm* form,
                            bool rows_sorted, bool gram, int D, int K, const int* ids, const int* starts, const int* sizes,
                            int leaf_cap, int n_small, int n_big, int max_bucket, int* knn_idx, float* knn_dist,
                            hipStream_t stream, int part = 0, int trees_before = 0, int* launched = nullptr,
@@ -90,13 +124,10 @@ int launch_sort_rows(int* knn_idx, float* knn_dist, int N, int K, hipStream_t st
 int launch_bucket_knn_screen(const float* points, int D, int K, const int* ids, const int* starts, const int* sizes,
                              int n_buckets, int stride, int* knn_idx, float* knn_dist, hipStream_t stream);
 // Buckets of up to 64 points of one tree of a forest, the form of the kernel (every pair exact, or bounded on the matrix
-// cores first) chosen on the device from the numbers of pairs the tree before left in prev (8 words; null: first tree);
-// stats: 8 zeroed words for this tree's numbers.
+// cores first) chosen on the device (bucket_form).
 int launch_bucket_knn_auto(const float* points, int D, int K, const int* ids, const int* starts, const int* sizes,
-                           int n_buckets, int* knn_idx, float* knn_dist, const unsigned long long* prev,
-                           unsigned long long* stats, hipStream_t stream);
+                           int n_buckets, int* knn_idx, float* knn_dist, const SmallBucketForm& form, hipStream_t stream);
 // share of the pairs (in 1 / 65536) below which the screened form is taken (RSFK_BUCKET_SCREEN); kScreenAlways: always
-constexpr unsigned int kScreenAlways = 0xffffffffu;
 unsigned int bucket_screen_share_q16();
 
 // bucket_knn_rows.hip

@@ -594,6 +594,33 @@ def test_later_trees_bound_pairs_and_merge_by_turns(gpu, capi, orc, rng, monkeyp
     assert_knn_equal(gi, gd, oi, od)
 
 
+# (forms: the trees whose pairs the rule bounds first; "+" = as the tree before)
+@pytest.mark.parametrize("N,D,K,mn,mx,offset,forms", [
+    (6000, 8, 4, 5, 10, 0, "00+"),            # few points in a bucket: never
+    (6000, 70, 5, 9, 18, 0, "00+"),           # ... more of them, but two chunks of dimensions
+    (6000, 16, 8, 10, 20, 0, "001"),          # while a row still gets three offers
+    (6000, 16, 16, 17, 34, 0, "001+"),
+    (6000, 8, 16, 20, 60, 300, "0010+"),      # a bound that does not tell the points apart: once
+    (6000, 70, 16, 20, 60, 300, "0010+"),
+    (6000, 16, 16, 17, 34, 300, "0011"),      # ... in buckets whose pairs all fit into the list
+    (6000, 16, 16, 20, 60, 0, "001+"),
+])
+def test_form_of_the_small_buckets_follows_its_rule(gpu, capi, orc, rng, monkeypatch, N, D, K, mn, mx, offset, forms):
+    monkeypatch.setenv("RSFK_FOREST_MERGE", "0")
+    X = (rng.random((N, D)) + offset).astype(np.float32)
+    T = 8
+    _say("form of the small buckets", N, D, K, mn, mx, offset)
+    gi, gd = orc.init_lists(N, K, self_in=True)
+    oi, od = gi.copy(), gd.copy()
+    log = np.zeros(16 * T + 2, np.float32)
+    capi.lib().pymodule_rsfk_knn(T, K, N, D, mn, mx, 5000, 0, 5, 0, X.ctypes.data, gi.ctypes.data, gd.ctypes.data, log.ctypes.data)
+    orc.forest(X, K, T, mn, mx, 5000, 5, 0, knn_idx=oi, knn_dist=od)
+    assert_knn_equal(gi, gd, oi, od)
+    took = "".join(str(v) for v in gpu.last_build_report()["bucket_screened"])
+    want = forms[:-1] + forms[-2] * (T + 1 - len(forms)) if forms.endswith("+") else forms
+    assert took.startswith(want), took
+
+
 # The workloads of the benchmark configurations 3, 4 and 5 (clustered D=256; sparse D=784 with K=90 and one
 # exploration pass, the only shape that runs the general bucket kernel with two slots per lane together with the
 # workgroup-per-point exploration merge; standard normal D=32 with buckets of 64..256 points), as forest +
