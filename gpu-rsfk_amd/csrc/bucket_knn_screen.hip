@@ -122,6 +122,13 @@ struct RowLoads {
 // first of those is requested before the bounds are evaluated.
 // stats (may be null): the workgroups whose number is a multiple of 2^stat_shift add the numbers of pairs of their bucket to
 // two of its words, for bucket_form (a sample of the buckets, see small_bucket_body).
+// The work of one workgroup on bucket blockIdx.x; lds: kScreenLdsBytes bytes of LDS.
+constexpr int kPitch = kChunk + 4;                        // an odd number of 16-byte units: rows start in different banks
+constexpr int kRegion = kCap * kPitch > kCap * kDistPitch ? kCap * kPitch : kCap * kDistPitch;
+constexpr size_t kScreenLdsBytes = sizeof(float) * kRegion + sizeof(ScreenMeta);
+static_assert(sizeof(ScreenTurns) <= sizeof(float) * kRegion, "the turns take the place of the rows");
+static_assert(kScreenLdsBytes <= 160 * 1024 / 8, "eight workgroups per compute unit");
+
 template <bool SINGLE>
 __device__ __forceinline__ void screen_bucket_body(float* __restrict__ lds, const float* __restrict__ points, int D, int K,
                                                    const int* __restrict__ ids, const int* __restrict__ starts,
