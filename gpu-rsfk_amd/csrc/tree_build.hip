@@ -779,8 +779,10 @@ __global__ __launch_bounds__(kBlock) void k_pm_mark(TreeParams P, int* __restric
 // ---------------------------------------------------------------------------
 struct SmallNode {
     int start, count, dstart, dcount;     // offsets inside the task's segment
-    int depth, leaf;
+    int depth;
     int rec;                              // record of the node in the index of the tree, if one is written
+    int vain;                             // tail phase: splits in vain just before this node
+    int place;                            // tail phase, nodes for the chain phase: place among those of its end of the queue
     uint64_t key;
 };
 
@@ -895,7 +897,7 @@ __global__ __launch_bounds__(TB, CHAIN ? 4 : 6) void k_tail(const float* __restr
     if (tid == 0) {
         SmallNode r;
         r.start = 0; r.count = tk.count; r.dstart = tk.dstart - tk.start; r.dcount = tk.dcount;
-        r.depth = tk.depth; r.leaf = 0; r.key = tk.key; r.rec = tk.rec;
+        r.depth = tk.depth; r.vain = 0; r.key = tk.key; r.rec = tk.rec;
         cur[0] = r;
         n_cur_s = 1; n_nxt_s = 0; nrec_s = 0; kind_s[0] = 0; kind_s[1] = 0; lev_s = 0; mx_s = 0; mn_s = 0x7fffffff;
         seen_s = 0; unsure_s = 0; n_chain_s[0] = 0; n_chain_s[1] = 0; n_chain_all_s = 0;
@@ -1071,7 +1073,7 @@ __global__ __launch_bounds__(TB, CHAIN ? 4 : 6) void k_tail(const float* __restr
                 bool leaves = false;
                 if constexpr (!CHAIN) {
                     const bool vain = nc == 1 && !c0.leaf && c0.depth < P.MAX_DEPTH - 1;
-                    leaves = vain && nd.leaf >= kVainMost - 1 && c0.count <= P.chain_max;
+                    leaves = vain && nd.vain >= kVainMost - 1 && c0.count <= P.chain_max;
                     const bool front = often_in_vain(c0.count, P.MIN);
                     const uint64_t m = ballot64(leaves), mf = ballot64(leaves && front), mb = m & ~mf;
                     if (m != 0) {
@@ -1104,12 +1106,9 @@ __global__ __launch_bounds__(TB, CHAIN ? 4 : 6) void k_tail(const float* __restr
                             SmallNode sn;
                             sn.start = c.start; sn.count = c.count; sn.dstart = c.dstart; sn.dcount = c.dcount;
                             sn.depth = c.depth;
-                            sn.leaf = !CHAIN && nc == 1 ? nd.leaf + 1 : 0;             // (splits in vain before this one)
+                            sn.vain = !CHAIN && nc == 1 ? nd.vain + 1 : 0;
                             sn.key = c.key; sn.rec = c.rec;
-                            if (small) {
-                                const int back = often_in_vain(c.count, P.MIN) ? 0 : 1;
-                                sn.leaf = 2 * atomicAdd(&n_chain_s[back], 1) + back;       // (its place in that part of the queue)
-                            }
+                            if (small) sn.place = atomicAdd(&n_chain_s[often_in_vain(c.count, P.MIN) ? 0 : 1], 1);
                             (small ? chain : nxt)[at] = sn;
                         } else {
                             ctr->overflow = 1;
@@ -1152,7 +1151,7 @@ __global__ __launch_bounds__(TB, CHAIN ? 4 : 6) void k_tail(const float* __restr
         TreeNode c;
         c.tree = tk.tree; c.start = tk.start + sn.start; c.count = sn.count; c.dstart = tk.start + sn.dstart; c.dcount = sn.dcount;
         c.depth = sn.depth; c.buf = 0; c.leaf = 0; c.rec = sn.rec; c.chunk0 = 0; c.key = sn.key;
-        const int back = sn.leaf & 1, at = chain_base_s[back] + (sn.leaf >> 1);
+        const int back = often_in_vain(sn.count, P.MIN) ? 0 : 1, at = chain_base_s[back] + sn.place;
         if (at < chain_cap) chain_all[back ? chain_cap - 1 - at : at] = c; else ctr->overflow = 1;
     }
     };
@@ -1183,6 +1182,10 @@ constexpr int kMidMost = 12288;          // points (LDS: 4 bytes of permutation 
 constexpr int kMidThreads = 1024, kMidPer = kMidMost / kMidThreads;
 constexpr int kMidOut = 64;              // nodes for the tail kernel kept before they are given a place in its queue
 
+struct MidNode : SmallNode {
+    int leaf;                             // a bucket, or to be one at the depth limit
+};
+
 template <int LPP, int KU>
 __global__ __launch_bounds__(kMidThreads, 4) void k_mid(const float* __restrict__ points, const uint8_t* __restrict__ q8, TreeParams P, int most,
                                                         const int* __restrict__ perm0, const int* __restrict__ perm1, int* __restrict__ perm_out,
@@ -1194,8 +1197,8 @@ __global__ __launch_bounds__(kMidThreads, 4) void k_mid(const float* __restrict_
     extern __shared__ __align__(16) unsigned char mid_lds[];
     int* seg = reinterpret_cast<int*>(mid_lds);
     float* nvec = reinterpret_cast<float*>(seg + most);
-    SmallNode* stack = reinterpret_cast<SmallNode*>(nvec + nvec_len(P.D));
-    SmallNode* out = stack + stack_cap;
+    MidNode* stack = reinterpret_cast<MidNode*>(nvec + nvec_len(P.D));
+    MidNode* out = stack + stack_cap;
     uint16_t* list = reinterpret_cast<uint16_t*>(out + kMidOut);
     constexpr int kWaves = kMidThreads / 64;
     __shared__ float hp_s[4];
@@ -1215,7 +1218,7 @@ __global__ __launch_bounds__(kMidThreads, 4) void k_mid(const float* __restrict_
     int* dst = perm_out + (size_t)tk.tree * (size_t)P.N;
     for (int i = tid; i < tk.count; i += kMidThreads) seg[i] = src[tk.start + i] & kIdMask;
     if (tid == 0) {
-        SmallNode r;
+        MidNode r;
         r.start = 0; r.count = tk.count; r.dstart = tk.dstart - tk.start; r.dcount = tk.dcount;
         r.depth = tk.depth; r.leaf = 0; r.key = tk.key; r.rec = tk.rec;
         stack[0] = r;
@@ -1229,7 +1232,7 @@ __global__ __launch_bounds__(kMidThreads, 4) void k_mid(const float* __restrict_
         if (tid == 0) out_base_s = n ? atomicAdd(&ctr->n_tail, n) : 0;
         __syncthreads();
         for (int i = tid; i < n; i += kMidThreads) {
-            const SmallNode sn = out[i];
+            const MidNode sn = out[i];
             TreeNode c;
             c.tree = tk.tree; c.start = tk.start + sn.start; c.count = sn.count; c.dstart = tk.start + sn.dstart; c.dcount = sn.dcount;
             c.depth = sn.depth; c.buf = 0; c.leaf = sn.leaf; c.rec = sn.rec; c.chunk0 = 0; c.key = sn.key;
@@ -1254,7 +1257,7 @@ __global__ __launch_bounds__(kMidThreads, 4) void k_mid(const float* __restrict_
     while (true) {
         const int n_stack = n_stack_s;
         if (n_stack == 0) break;
-        const SmallNode nd = stack[n_stack - 1];
+        const MidNode nd = stack[n_stack - 1];
         const int st = nd.start, cnt = nd.count;
         int r1, r2;
         pick_pair(nd.key, nd.dcount, r1, r2);
@@ -1344,7 +1347,7 @@ __global__ __launch_bounds__(kMidThreads, 4) void k_mid(const float* __restrict_
             int n_left = n_stack - 1, n_out = n_out_s;
             auto child = [&](const TreeNode& c) {
                 const bool forced = c.depth >= P.MAX_DEPTH - 1, split = !c.leaf && !forced && c.count > P.small;
-                SmallNode x;
+                MidNode x;
                 x.start = c.start; x.count = c.count; x.dstart = c.dstart; x.dcount = c.dcount;
                 x.depth = c.depth; x.leaf = c.leaf || forced ? 1 : 0; x.rec = c.rec; x.key = c.key;
                 if (!split) out[n_out++] = x;
@@ -2086,7 +2089,7 @@ __global__ __launch_bounds__(64 * WAVES, NT >= 4 ? 2 : 3) void k_chain(const flo
                         if (sp < node_cap) {
                             SmallNode sn;
                             sn.start = cstart; sn.count = ccount; sn.dstart = cdstart; sn.dcount = cdcount;
-                            sn.depth = depth; sn.leaf = 0; sn.key = child_key(key, side); sn.rec = crec_at;
+                            sn.depth = depth; sn.key = child_key(key, side); sn.rec = crec_at;
                             stack[sp] = sn;
                         } else {
                             ctr->overflow = 1;
@@ -2534,7 +2537,7 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
     RSFK_CHECK(n_tail <= w->tail_cap, "tree batch: tail queue overflow");
     if (mid && n_tail > 0) {
         const int stack_cap = w->mid_most / std::max(P.small, 1) + 4;
-        const size_t lds = (size_t)w->mid_most * 6 + (size_t)nvec_len(D) * 4 + (size_t)(stack_cap + kMidOut) * sizeof(SmallNode);
+        const size_t lds = (size_t)w->mid_most * 6 + (size_t)nvec_len(D) * 4 + (size_t)(stack_cap + kMidOut) * sizeof(MidNode);
         const int pieces = q8_padded(D) / 16;
 #define RSFK_MID_LAUNCH(L, U)                                                                                               \
         do {                                                                                                               \
