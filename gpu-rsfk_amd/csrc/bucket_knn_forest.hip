@@ -20,6 +20,7 @@
 #include "bucket_knn_tile.hpp"
 #include "bucket_small_body.hpp"
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 
 namespace rsfk {
@@ -312,11 +313,13 @@ bool bucket_forest_wanted(int n_trees)
 // 150,000 x 100, 10 trees 1.61 -> 0.94, 250,000 x 20, K = 10, 40 trees 3.11 -> 3.28, 400,000 x 100, 50 trees
 // 9.1 -> 9.8).  Larger buckets and longer rows gain at every size that fits (70,000 x 784, K = 90, 10 trees 5.0 -> 3.7), but for
 // many trees over many points whose buckets fit into LDS whole and have far more points than a row has slots: there the later
-// trees skip most pairs as well.  The line is at N * (trees of the build) * largest bucket / K = 80 million (whole build, one tree after
-// the other / together; normal points): 1M x 32, K = 32, buckets of 64..256: 4 trees (32M) 7.1 / 6.5 ms, 10 trees (80M) 10.9 / 12.5, 30
-// trees 22.4 / 31.4; 1M x 20, K = 8, buckets of 64..256: 4 trees (128M) 4.7 / 5.3, 10 trees 7.3 / 10.6; 1M x 36, K = 64, buckets of
-// 65..256: 10 trees (40M) 18.7 / 15.7, 30 trees (120M) 36.4 / 36.9; 300,000 x 32, K = 32, buckets of 64..256: 10 trees (24M) 4.7 / 4.0, 30
-// trees (72M) 8.9 / 8.9; 300,000 x 20, K = 8, buckets of 64..128: 30 trees (144M) 7.7 / 8.0.
+// trees skip most pairs as well, and what the trees together move leaves the caches.  The line is at N sqrt(trees of the build) (largest bucket)
+// / K^(3/4) = 31 million (1 + 1/D)^2, in the middle of what 664 builds of 2 to 64 dimensions, 6 to 60 trees, 200,000 to 2.5M points and buckets
+// up to 73 .. 256 say (bucket step, one tree after the other / together): 210,000 x 4, K = 25, buckets of 50..200, 50 trees (27M) 8.2 / 5.3 ms;
+// 210,000 x 2, K = 32, 64..256, 50 trees (28M) 12.8 / 6.2; 400,000 x 32, K = 32, 64..256, 12 trees (26M) 1.14 times, 50 trees (54M) 0.82;
+// 400,000 x 2, K = 32, 64..256, 50 trees (54M; the line is at 70M) 18.0 / 12.0; 1M x 16, K = 16, 40..160, 6 trees (49M) 0.81, 50,
+// K = 50, 64..256, 12 trees (47M) 1.07; 1.5M x 5, K = 7, 35..140, 26 trees (253M) 8.5 / 18.9.  With this line a step takes 0.6 % longer than the
+// better form on (geometric) average, at worst 1.3 times; a line on N trees bucket / K took 3.7 %, at worst 2.4 times.
 int bucket_forest_group(int N, int D, int K, int max_bucket, int n_trees, int all_trees)
 {
     constexpr size_t kFloats = (size_t)1 << 29;
@@ -326,7 +329,7 @@ int bucket_forest_group(int N, int D, int K, int max_bucket, int n_trees, int al
     const bool forced = e && e[0] == '1';
     if (!forced && N > kMostPoints && K <= 64 && max_bucket <= medium_bucket_cap()) return 0;
     if (!forced && N > kMostPoints && K <= 64 && max_bucket <= bucket_rows_cap(D, K) &&
-        (long long)N * all_trees * max_bucket >= 80000000ll * K)
+        N * std::sqrt((double)all_trees) * max_bucket >= 3.1e7 * (1.0 + 1.0 / D) * (1.0 + 1.0 / D) * std::pow((double)K, 0.75))
         return 0;
     const int group = (int)std::min<size_t>((size_t)std::min(n_trees, 64), kFloats / ((size_t)N * (size_t)forest_pitch(max_bucket)));
     return group >= std::min(2, n_trees) ? group : 0;
