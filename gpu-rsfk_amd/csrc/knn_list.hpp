@@ -241,10 +241,15 @@ struct KnnRow {
         const bool in = ok && enters(c, d);
         const uint64_t m = ballot64(in);
         const int n = __popcll(m);
-        if (n <= kFewEnter) {
-            if (n != 0) merge(ok, c, d);
-            return;
-        }
+        if (n == 0) return;
+        // (One copy of the insertions in the code: with three of them the exploration of 98,603 x 5, K = 82 took 42.6 ms, with one 42.2, by insertions
+        // alone 41.9; 500,000 x 4, K = 16 1.36, 1.34, 1.39; 40,000 x 64, K = 100 7.78, 7.64, 8.04.)
+        if (n <= kFewEnter || !place_ranked(in, m, n, c, d, buf)) merge(ok, c, d);
+    }
+
+    // false: two distances are equal, and nothing has been changed
+    __device__ __forceinline__ bool place_ranked(bool in, uint64_t m, int n, int c, float d, double* buf)
+    {
         const int lane = lane_id();
         float* cand = reinterpret_cast<float*>(buf + 64 * SL);
         uint32_t* places = reinterpret_cast<uint32_t*>(cand + 68);
@@ -273,10 +278,7 @@ struct KnnRow {
         const bool stays = in && rank < kk;
         const uint32_t bit = 1u << (rank & 31);
         if (stays) level |= (atomicOr(&places[rank >> 5], bit) & bit) != 0;
-        if (ballot64(in && level) != 0) {
-            merge(ok, c, d);
-            return;
-        }
+        if (ballot64(in && level) != 0) return false;
         wave_lds_sync();
         double v[SL];
         bool is_new[SL];
@@ -302,6 +304,7 @@ struct KnnRow {
         }
         changed = true;
         refresh_tau();
+        return true;
     }
 
     __device__ __forceinline__ void merge(bool ok, int c, float d)
