@@ -594,6 +594,19 @@ def test_later_trees_bound_pairs_and_merge_by_turns(gpu, capi, orc, rng, monkeyp
     assert_knn_equal(gi, gd, oi, od)
 
 
+@pytest.mark.parametrize("N,D,K,mn,mx,T,together", [(204551, 4, 25, 50, 200, 50, True), (400000, 2, 32, 64, 256, 50, True),
+                                                    (400000, 32, 32, 64, 256, 50, False), (400000, 32, 32, 64, 256, 6, True)])
+def test_many_points_take_the_trees_together_by_rule(gpu, rng, N, D, K, mn, mx, T, together):
+    import gpu_rsfk
+    X = rng.random((N, D), dtype=np.float32)
+    _say("trees together or not", N, D, K, mn, mx, T)
+    gi, gd = gpu_rsfk.RSFK(random_state=1).find_nearest_neighbors(X, K, n_trees=T, min_tree_children=mn, max_tree_children=mx, nn_exploring_factor=0)
+    named = set(name for _, _, names in gpu.last_build_report()["bucket_kernels"] for name in names)
+    assert (named == {"k_forest_pairs + k_forest_merge"}) == together, named
+    some = rng.integers(0, N, 200)
+    assert np.allclose(gd[some], ((X[some][:, None] - X[gi[some]]) ** 2).sum(2), rtol=1e-5) and rows_have_no_duplicates(gi[some])
+
+
 # (forms: the trees whose pairs the rule bounds first; "+" = as the tree before)
 @pytest.mark.parametrize("N,D,K,mn,mx,offset,forms", [
     (6000, 8, 4, 5, 10, 0, "00+"),            # few points in a bucket: never
