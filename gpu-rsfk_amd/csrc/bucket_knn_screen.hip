@@ -594,16 +594,20 @@ unsigned int bucket_screen_share_q16()
     return (unsigned int)(pct * 65536.0 / 100.0 + (pct >= 100.0 ? 1.0 : 0.0));
 }
 
-// The screened form against the direct one, 1M points (time of a tree, screened / direct, third ... tenth tree):
-//   points of a bucket   D = 4         32            64            100           256 (400,000)
-//    6.8                 1.29 .. 1.37  1.21 .. 1.27  1.17 .. 1.19  1.34 .. 1.32  1.27 .. 1.20
-//    9.5                 1.07 .. 1.23  1.00 .. 1.26  0.98 .. 1.17  1.15 .. 1.32  1.13 .. 1.23
-//   12.2                 0.89 .. 1.09  0.85 .. 1.13  0.83 .. 1.06  0.98 .. 1.20  1.02 .. 1.16
-//   14.9                 0.81 .. 1.00  0.76 .. 1.03  0.75 .. 0.97  0.87 .. 1.09  0.92 .. 1.07
-//   17.6                 0.75 .. 0.93  0.70 .. 0.94  0.70 .. 0.89  0.81 .. 0.99  0.86 .. 1.01
-//   23                   0.71 .. 0.85  0.63 .. 0.79  0.64 .. 0.77  0.71 .. 0.84  0.78 .. 0.84
-// Few points leave few chains to save; what the screened form gains there it gains at merging the offers, as long as about three per
-// row are left.  So: from 16 points on; from 12 (14 with more than one chunk of dimensions) while a row gets three offers.
+// The screened form against the direct one (time of a tree, screened / direct; share of the pairs that the direct form was offered):
+//   points of a     D = 4                   16                      64                      126                     300
+//   bucket, tree    3      10    100        3      10    100        3      10    100        3      10    100        3      10    100
+//    6.8            1.29   1.29  1.26       1.25   1.23  1.04       1.16   1.11  0.82       1.31   1.20  0.85       1.30   1.16  0.80
+//    9.5            1.13   1.16  1.13       1.09   1.25  1.20       1.03   1.15  0.93       1.17   1.24  0.96       1.21   1.23  0.90
+//   12.2            0.98   1.04  1.01       0.92   1.15  1.26       0.89   1.06  1.00       1.02   1.16  1.05       1.11   1.19  0.99
+//   14.9            0.89   0.96  0.91       0.82   1.06  1.27       0.80   0.98  1.07       0.92   1.07  1.10       1.01   1.11  1.04
+//   17.6            0.83   0.88  0.85       0.76   0.95  1.24       0.73   0.89  1.09       0.83   0.98  1.12       0.91   1.01  1.05
+//   23              0.76   0.82  0.77       0.65   0.82  1.12       0.65   0.76  1.04       0.73   0.81  1.04       0.79   0.84  0.95
+//   offered         0.7    0.22  0.22       0.7    0.11  0.03       0.7    0.11  0.01       0.7    0.11  0.01       0.7    0.10  0.01
+// Few points leave few chains to save; what the screened form gains there it gains at merging the offers, while there are enough of
+// them (three per row with 12 points, 1.8 with 17.6, 0.6 with 23), and where most buckets get no offer and end with the list. So:
+// from 26 points on; from 12 (14 with more than one chunk of dimensions) while a row gets 3 (26 - points) / 14 offers; and whenever less
+// than one bucket in two gets an offer.
 // The bound is a share of the norms: points far from the origin, or of two dimensions, it does not tell apart.  Buckets of about 40
 // points (always screened / direct, 50 trees; share of the pairs that is listed for nothing, from the third tree on):
 //   D = 8, uniform + 10   K = 4: 1.28 (0.37 .. 0.36)   8: 1.16 (0.39 .. 0.36)   31: 1.16 (0.31 .. 0.40)
@@ -613,16 +617,21 @@ unsigned int bucket_screen_share_q16()
 //   D = 100, uniform + 10 K = 4: 0.97 (0.32 .. 0.16)   8: 0.96 (0.42 .. 0.24)   31: 1.04 (0.41 .. 0.40); + 14: 1.3 (0.7 .. 0.6)
 // So: no longer once 1/3 + D/384 of the pairs, at most half of them, were listed for nothing.  Buckets of at most 42 points keep all their
 // pairs in the list and are merged by turns whatever the bound leaves (23 points, every pair listed: 0.7 .. 0.9 while an eighth
-// of the pairs is offered): with fewer than 28 points on average, 7/8.
+// of the pairs is offered): with fewer than 28 points on average, 7/8; but twice the line of the few offers, where it is those that count.
+// (400 trees of 5 to 10 points, 20 dimensions, uniform + 20: 1.29 times the direct form without that.)
 BucketFormRule bucket_form_rule(double mean, int D)
 {
     constexpr unsigned int kNever = 0xffffffffu;
-    BucketFormRule rule = {bucket_screen_share_q16(), 0u, kNever};
+    BucketFormRule rule = {bucket_screen_share_q16(), 0u, 0u, kNever};
     const char* e = std::getenv("RSFK_BUCKET_SCREEN");
     if (e && *e) return rule;                                    // (a share, always or never: nothing else is asked)
-    if (mean < (D <= kChunk ? 12.0 : 14.0)) rule.share_q16 = 0;
-    else if (mean < 16.0) rule.least_q16 = (unsigned int)(3.0 * 65536.0 / mean);
-    rule.vain_q16 = (unsigned int)(65536.0 * (mean < 28.0 ? 0.875 : std::min(0.5, 1.0 / 3.0 + D / 384.0)));
+    mean = std::max(mean, 2.0);
+    const auto q16 = [](double share) { return (unsigned int)(65536.0 * std::min(share, 1.0)); };
+    if (mean < 26.0) {
+        rule.least_q16 = mean < (D <= kChunk ? 12.0 : 14.0) ? kNever : q16(3.0 * (26.0 - mean) / (14.0 * mean));
+        rule.few_q16 = q16(1.0 / (mean * mean));
+    }
+    rule.vain_q16 = q16(mean < 28.0 ? 0.875 : std::min(0.5, 1.0 / 3.0 + D / 384.0));
     return rule;
 }
 

@@ -263,7 +263,7 @@ int knn_forest_device(int n_trees, int K, int N, int D, int MIN, int MAX, int MA
         RSFK_HIP(hipMemsetAsync(pair_stats.p, 0, sizeof(unsigned long long) * stat_words, stream));
         unsigned long long* d_pairs = static_cast<unsigned long long*>(pair_stats.p);
         rep.screen_share_q16 = bucket_screen_share_q16();
-        rep.rules.assign((size_t)n_trees, BucketFormRule{rep.screen_share_q16, 0, 0});
+        rep.rules.assign((size_t)n_trees, BucketFormRule{rep.screen_share_q16, 0, 0, 0});
         const int gram_from = bucket_gram_from();
         SideStream sync;
         if (std::getenv("RSFK_KNN_ONE_STREAM") == nullptr && sync.open()) return 1;

@@ -72,8 +72,9 @@ constexpr int kFormWords = 8;
 constexpr unsigned int kScreenAlways = 0xffffffffu;
 struct BucketFormRule {
     unsigned int share_q16;      // screened below this share of offered pairs (in 1 / 65536); kScreenAlways: always
-    unsigned int least_q16;      // ... and not below this one
-    unsigned int vain_q16;       // ... and not once listed less offered pairs were at least this share
+    unsigned int least_q16;      // ... and not below this one, unless
+    unsigned int few_q16;        // ... it is below this one,
+    unsigned int vain_q16;       // ... and not once listed less offered pairs were at least this share (twice few_q16 where few are offered)
 };
 struct BucketForm {
     bool screened, vain;
@@ -88,8 +89,10 @@ __host__ __device__ __forceinline__ BucketForm bucket_form(const unsigned long l
         b += words[kFormWords / 2 + i];
     }
     const unsigned long long offered = a & 0xffffffffull, pairs = a >> 32, listed = b & 0xffffffffull, bounded = b >> 32;
-    const bool vain = bounded > 0 && ((listed - offered) << 16) >= bounded * rule.vain_q16;
-    return {!vain && pairs > 0 && (offered << 16) < pairs * rule.share_q16 && (offered << 16) >= pairs * rule.least_q16, vain};
+    const unsigned long long o = offered << 16, nothing = (listed - offered) << 16;      // (listed pairs that no row can take)
+    const bool few = o < pairs * rule.few_q16;
+    const bool vain = bounded > 0 && nothing >= bounded * (few ? 2 * rule.few_q16 : rule.vain_q16);
+    return {!vain && (few || (o < pairs * rule.share_q16 && o >= pairs * rule.least_q16)), vain};
 }
 // mean: points of a small bucket of the tree
 BucketFormRule bucket_form_rule(double mean, int D);
