@@ -222,7 +222,14 @@ __device__ __forceinline__ uint64_t in_own(const int* own, int n, int c)
 // A wavefront takes PTS consecutive points, whose stored neighbours and reversed entries follow each other in memory: what such a
 // wavefront waits for is its trips (offsets, then rows and reversed entries, then distances), not bytes or instructions (1M x 32, one
 // point per wavefront: lengths 0.30 ms, rows 0.53; four: 0.18 and 0.32.  With 4 or 16 slots per neighbour the lengths take 0.23 and 0.26).
-inline int union_points(int K) { return K <= 32 ? 4 : (K <= 64 ? 2 : 1); }
+// Few points do not fill the device, and a wavefront's work counts (lengths and rows in us with one, two and four points: 3,001 x 32 9.2,
+// 13.8, 17.5; 14,009 x 32 16.6, 16.8, 21.0; 60,013 x 32 46.9, 40.6, 41.3; 6,007 x 16 8.2, 8.4, 10.7; 20,011 x 16 17.1, 14.5, 13.8; 14,009 x 5
+// 12.3, 9.8, 9.6; 30,011 x 48 32.6, 34.6).
+inline int union_points(int N, int K)
+{
+    if (K <= 32 && N / 1000 >= K) return 4;
+    return K <= 64 && N / 500 >= K ? 2 : 1;
+}
 
 // The stored neighbours of a point as a table in LDS of 2^bits slots, 8 per neighbour: of those that fall on the same slot the last one
 // written is there, the others (two per row of 32) are listed.  Whether a column is among them is one read, where comparing it
@@ -764,7 +771,7 @@ int symmetrize(const int* d_idx, const float* d_dist, int N, int K, int drop_sel
     while ((1 << l) < K) ++l;
     const int div_s = 31 + l;
     const uint32_t div_m = (uint32_t)((((uint64_t)1 << div_s) + (uint64_t)K - 1) / (uint64_t)K);
-    const int pts = union_points(K), bits = table_bits(K);
+    const int pts = union_points(N, K), bits = table_bits(K);
     const unsigned grid = (unsigned)((N + 4 * pts - 1) / (4 * pts));
     const int len_ints = K <= kTableMostK ? (pts << bits) + ((2 * pts * K + 3) & ~3) : (K + 4 + 3) & ~3;
 #define RSFK_UNION_LEN(PTS, TABLE)                                                                                          \

@@ -1255,6 +1255,28 @@ def test_symmetric_graph_forms(gpu, orc, rng, monkeypatch, N, K, hubs, staged):
     assert np.array_equal(gp, op) and np.array_equal(gc, oc) and np.array_equal(gv, ov)
 
 
+# Points per wavefront by the points and the neighbours: two and four with rows of many neighbours, on either side of the lines.
+@pytest.mark.parametrize("N,K,hubs", [(31999, 32, 0), (32003, 32, 2), (31003, 31, 0), (15999, 32, 0), (16001, 32, 2), (16497, 33, 0), (16503, 33, 3), (32003, 64, 2)])
+def test_symmetric_graph_points_per_wavefront(gpu, orc, rng, monkeypatch, N, K, hubs):
+    import gpu_rsfk
+    monkeypatch.setenv("RSFK_GRAPH_FLAGS", "0")
+    idx = ((np.arange(N)[:, None] + np.cumsum(rng.integers(1, 4, (N, K)), axis=1)) % N).astype(np.int32)
+    back = rng.random((N, K)) < 0.5
+    idx = np.where(back, (2 * np.arange(N)[:, None] - idx) % N, idx).astype(np.int32)
+    same = (np.diff(np.sort(idx, axis=1), axis=1) == 0).any(1)
+    idx[same] = (np.flatnonzero(same)[:, None] + 1 + np.arange(K)) % N
+    for h in range(hubs):
+        put = (rng.random(N) < (0.005, 0.02, 0.3)[h % 3]) & ~(idx == h).any(1)
+        idx[put, h % K] = h
+    idx[rng.random((N, K)) < 0.02] = -1
+    a, b = np.minimum(idx, np.arange(N)[:, None]).astype(np.int64), np.maximum(idx, np.arange(N)[:, None])
+    val = ((a * 7919 + b * 104729) % 10007).astype(np.float32)  # one value per pair
+    _say("symmetrize, points per wavefront", N, K, hubs)
+    gp, gc, gv = gpu_rsfk.symmetric_knn_graph(idx, val, drop_self=True)
+    op, oc, ov = orc.symmetrize(idx, val, drop_self=True)
+    assert np.array_equal(gp, op) and np.array_equal(gc, oc) and np.array_equal(gv, ov)
+
+
 @pytest.mark.parametrize("N,lead", [(16384, 0), (16385, 0), (16385, 4), (140000, 1020), (140001, 4092)])
 def test_results_into_fresh_pages(gpu, capi, rng, N, lead):
     """Result arrays of up to 4 MiB and of more, anywhere on pages that do not exist yet: the results, and nothing beside them."""
