@@ -1181,6 +1181,21 @@ def test_ann_recall_rises_with_the_number_of_trees(gpu, rng):
     assert rec[0] < rec[1] < rec[2] and rec[2] > 0.5
 
 
+@pytest.mark.parametrize("N,mn,mx", [(40, 3, 6), (3000, 3, 6), (4000, 4, 9), (9000, 3, 7), (21000, 2, 5), (70000, 2, 4)])
+def test_queries_are_counted_whatever_the_records(gpu, capi, orc, rng, monkeypatch, N, mn, mx):
+    """Counters of the buckets a line apart, closer, and side by side (from few to many records of a tree), one tree after the other."""
+    monkeypatch.setenv("RSFK_ANN_FOREST", "0")
+    D, K, T, NQ = 3, 4, 3, 2500
+    X, Q = rng.random((N, D), dtype=np.float32), rng.random((NQ, D), dtype=np.float32)
+    Q[:1500] = Q[0]                                             # (most of them reach one bucket)
+    qi, qd = np.full((NQ, K), -1, np.int32), np.full((NQ, K), np.inf, np.float32)
+    _say("queries by records", N, mn, mx)
+    log = np.zeros(16 * T + 2, np.float32)
+    capi.lib().pymodule_rsfk_knn_ann(T, K, N, NQ, D, mn, mx, 5000, 0, 11, 0, X.ctypes.data, Q.ctypes.data, qi.ctypes.data, qd.ctypes.data, log.ctypes.data)
+    oi, od = orc.ann_forest(X, Q, K, T, mn, mx, 5000, 11)
+    assert_knn_equal(qi, qd, oi, od)
+
+
 # ---------------------------------------------------------------------------
 # symmetrised graph export
 # ---------------------------------------------------------------------------
