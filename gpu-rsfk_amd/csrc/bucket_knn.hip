@@ -448,12 +448,15 @@ constexpr int kYoungTrees = 2;
 // K = 64, D = 36, buckets of 65..256: third tree 1.81 -> 2.14 ms, fourth 1.52 -> 1.40, eighth 1.06 -> 0.71; K = 64, D = 20, buckets of
 // 65..130: fourth 0.92 -> 1.07, fifth 0.78 -> 0.82, sixth 0.73 -> 0.68; K = 40, D = 32, buckets of 41..82: third 0.27 -> 0.31, fourth
 // 0.21 -> 0.19; 10M, K = 32, D = 32, buckets of 64..256: second 13.8 -> 17.2, third 10.0 -> 7.8, tenth 6.4 -> 2.8.
+// With few dimensions the trees find the same neighbours again and again, which are offered every time, and the chains are short: long rows
+// stay with the direct form (24 trees of 400,000 points, screened by the line above / direct: D = 2, buckets of 64..256, K = 32 0.91, 36 1.02,
+// 45 1.17, 64 1.34; D = 4, K = 40 0.96, 45 1.03, 64 1.23; D = 6, K = 50 0.98, 64 1.10; D = 8, K = 64 1.00; buckets of up to 2K 1.0 to 1.1 times these).
 // RSFK_BUCKET_SCREEN=never / always says so for every tree.
-static bool resident_rows_screened(int K, int max_bucket, int trees_before)
+static bool resident_rows_screened(int D, int K, int max_bucket, int trees_before)
 {
     const unsigned int share = bucket_screen_share_q16();
     if (share == 0 || share == kScreenAlways) return share != 0;
-    return trees_before >= kYoungTrees && 10ll * K <= (long long)trees_before * max_bucket;
+    return trees_before >= kYoungTrees && 10ll * K <= (long long)trees_before * max_bucket && K <= 28ll + 4ll * D;
 }
 
 int bucket_gram_from()
@@ -608,7 +611,7 @@ int launch_bucket_knn_tree(const float* points, const SmallBucketForm* form,
         if (rows_cap > skip_upto) {
             used |= kBucketKernelRows;
             const int upto = max_bucket >= 0 ? std::min(max_bucket, rows_cap) : rows_cap;
-            if (rows_sorted && resident_rows_screened(K, upto, trees_before)) {
+            if (rows_sorted && resident_rows_screened(D, K, upto, trees_before)) {
                 if (launch_bucket_knn_rows_screen(points, D, K, ids, starts + off, sizes + off, n_big, skip_upto + 1, upto, knn_idx,
                                                   knn_dist, stream))
                     return 1;
