@@ -187,8 +187,8 @@ __global__ __launch_bounds__(256) void k_route(const float* __restrict__ planes,
 // The same for many queries of 65 to 128 dimensions, by the rounded hyperplanes of k_planes: the side is certain when
 // |n~.x - offset| > E |x|, otherwise (1 % of the tests on uniform points) the exact test follows.  Sums of squares that
 // overflow, infinities and NaN leave a test uncertain.
-// k_route is bound by the hyperplanes' bytes from beyond the L2 (16 MB a tree at 1M x 100); these are half as many: 1M queries
-// 0.56 -> 0.49 ms a tree.  Rows of up to 64 dimensions gain nothing (500,000 / 100,000 x 64: search 8.25 -> 8.21 ms) or lose
+// k_route is bound by the hyperplanes' bytes from beyond the L2 (16 MB a tree at 1M x 100; 2.4 GB fetched at 4.3 TB/s); these are half as
+// many: 1M queries 0.56 -> 0.49 ms a tree, 1.3 GB at 2.6 TB/s and bound by instruction issue (vector ALUs 71 % busy).  Rows of up to 64 dimensions gain nothing (500,000 / 100,000 x 64: search 8.25 -> 8.21 ms) or lose
 // (1M / 1M x 16 14.1 -> 14.6), and so do few queries, for which the second trip counts (20,000 / 1M x 100, 50 trees
 // 8.65 -> 9.01 ms, 100,000, 20 trees 6.91 -> 6.82).
 template <bool VEC>

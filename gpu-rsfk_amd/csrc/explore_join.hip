@@ -443,8 +443,8 @@ __global__ __launch_bounds__(kRowsBlock) void k_staged_rows(const int2* __restri
 // some thousand bins, and the lines of those stores leave the L2 before their neighbours arrive (1M x 32: 0.8 GB written
 // for 0.26 GB of payload).  Here the records of a tile of 16,384 entries are sorted by bin in LDS first (their neighbours and 16-bit
 // places in the tile, six bytes each), at most 1024 bins, so that a bin gets a run of 16 records (a cache line) per tile.  The rows of a bin
-// are then assembled in LDS, a quarter, a half or all of its points at a time (the workgroups of a bin read its records from the L2),
-// and written whole.  1M x 32: scatter 0.49 -> 0.11 ms, rows 0.26 -> 0.18; export of the graph of 100,000 x 32 182 -> 170 us, 30,000 x 100
+// are then assembled in LDS, a quarter, a half or all of its points at a time, and written whole.  (The workgroups of a bin are on different
+// dies, and each reads all its records twice, from beyond the L2: 1M x 32, two of them, 0.97 GB for 0.26 GB of records at 6 TB/s.)  1M x 32: scatter 0.49 -> 0.11 ms, rows 0.26 -> 0.18; export of the graph of 100,000 x 32 182 -> 170 us, 30,000 x 100
 // 241 -> 208, 50,000 x 32 the same.
 constexpr int kTileThreads = 1024, kTilePer = 16, kTile = kTileThreads * kTilePer;
 constexpr int kTileMaxBins = 1024;
