@@ -134,8 +134,8 @@ struct TreeRec {
     int a, b, c0, c1;
 };
 
-// Ints from the counts of one tree of a batch to those of the next one (TreeStats, a cache line each).
-constexpr int kTreeStatPitch = 32;
+// Ints from the counts of one tree of a batch to those of the next one (TreeStats, two cache lines each).
+constexpr int kTreeStatPitch = 64;
 
 // Buckets of at most this many points are handled by the small-bucket K-NN kernel; the
 // tree builder keeps them apart from the larger ones.
