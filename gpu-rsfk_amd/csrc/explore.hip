@@ -1079,27 +1079,26 @@ bool explore_merge_uses_bounds(int D, int K)
 // One exploration pass.  old_idx is scratch of N*K ints (receives the snapshot).
 // bf may be null (or hold null rows): every candidate then gets the exact distance.
 // Rows short enough for the LDS of the merge kernels: the exploration then takes its candidates from the join, and
-// the general kernel (the only user of the uncentred copy) only sees what the merge kernels hand back.
+// the general kernel (the only user of the bfloat16 copy) only sees what the merge kernels hand back.
 bool explore_merge_fits(int D, int K)
 {
     const int small_table = std::min(4096, std::max(256, next_pow2(16 * K)));
     return K <= kMaxKJoin && 4 * merge_wave_ints(small_table, bf16_valid(D), K) <= 150 * 1024 / 4;
 }
 
-// ws may be null; with a workspace and a bfloat16 copy for the join (bf_join, may be centred; bf must not be)
+// ws may be null; with a workspace and the copy for the join (jc)
 // the candidates come from the join over the reversed graph (explore_join.hip), which needs rows sorted by
 // distance.
-int launch_explore(const float* points, const Bf16Copy* bf, const Bf16Copy* bf_join, int N, int D, int K, int* knn_idx,
+int launch_explore(const float* points, const Bf16Copy* bf, const JoinCopy* jc, int N, int D, int K, int* knn_idx,
                    float* knn_dist, int* old_idx, ExploreWorkspace* ws, hipStream_t stream, bool rows_sorted,
                    unsigned long long* stat, const int* order)
 {
     if (N <= 0) return 0;
     RSFK_CHECK(K >= 1 && K <= kMaxK, "exploration: K must be in 1..1024");
-    RSFK_CHECK(bf == nullptr || bf->mu == nullptr, "exploration: the general kernel needs an uncentred copy");
     const int dpad = bf16_valid(D);
     const int small_table = std::min(4096, std::max(256, next_pow2(16 * K)));
     // (rows too long for the LDS of the merge kernel: every point enumerates its own candidates)
-    const bool join = ws != nullptr && bf_join != nullptr && bf_join->rows != nullptr && explore_merge_fits(D, K);
+    const bool join = ws != nullptr && jc != nullptr && jc->rows != nullptr && explore_merge_fits(D, K);
     // (rows_sorted: the caller knows that every row is in order, e.g. after the bucket step of a forest)
     if (join && !rows_sorted && launch_sort_rows(knn_idx, knn_dist, N, K, stream)) return 1;
     RSFK_HIP(hipMemcpyAsync(old_idx, knn_idx, sizeof(int) * (size_t)N * (size_t)K, hipMemcpyDeviceToDevice, stream));
@@ -1129,7 +1128,7 @@ int launch_explore(const float* points, const Bf16Copy* bf, const Bf16Copy* bf_j
         // Marks from the join, then the merge kernel with a small set (little LDS, many wavefronts per CU).
         // The points it cannot take come back in a list and get a second launch with the largest set that
         // fits; what is left after that goes to the general kernel below.
-        if (launch_explore_join(ws, *bf_join, N, D, K, old_idx, knn_dist, stream, order)) return 1;
+        if (launch_explore_join(ws, *jc, N, D, K, old_idx, knn_dist, stream, order)) return 1;
         const uint32_t* pass = explore_ws_pass(ws);
         int* listA = explore_ws_todo(ws, 0);
         int* listB = explore_ws_todo(ws, 1);

@@ -4,15 +4,20 @@
 // neighbours c of its neighbours q -- but enumerated from the middle: for every q, all
 // pairs (p, c) with p in R(q) = {points that list q} and c in N(q).  The rows of N(q)
 // and R(q) are then loaded once per q instead of once per pair, and the pair distances
-// of a 32 x 32 tile come from one chain of matrix-core instructions on the bfloat16
-// copy of the points (v_mfma_f32_32x32x16_bf16: Gram matrix G, d~ = n_p + n_c - 2 G).
+// of a 32 x 32 tile come from one chain of matrix-core instructions on the float16
+// copy of the points (v_mfma_f32_32x32x16_f16: Gram matrix G, d~ = n_p + n_c - 2 G).
 //
-// d~ is only used to discard.  With S = n_p + n_c (norms of the bfloat16 rows), u = 2^-8:
-//   rounding to bfloat16:   |d(real) - d~(real)| <= 2u sqrt(d~ Q) + u^2 Q,  Q = 2 S  (Cauchy-Schwarz)
+// d~ is only used to discard.  All in the units of the copy (join_copy.hpp: distances times s^2), with S = n_p + n_c (norms of its
+// rows) and e_p, e_c what rounding took from the two rows:
+//   rounding to float16:    sqrt(d(real)) >= sqrt(d~(real)) - e_p - e_c  (triangle inequality)
 //   Gram matrix and norms:  |d~(computed) - d~(real)| <= E1 = (D' + 16) 2^-21 S
 //   fp32 chain:             result >= d(real) (1 - gamma),  gamma = (D + 8) 2^-22
-// so L = (d~ - E1 - 1.01 (2u sqrt((d~ + E1) Q) + u^2 Q)) (1 - gamma) is a lower bound of the exact fp32
-// distance, and a pair is dropped when L is above the last slot of row p.
+// so a pair is dropped when d~ - E1 is above (bar_p + e_c)^2, bar_p = s sqrt(last slot of row p / (1 - gamma)) + e_p: its exact
+// distance is then above the last slot.  e_p is the length measured when the copy was made; for e_c the kernel of short rows, which
+// has 8 bytes per point for all of this, takes what holds for any row, 2^-11 |row| + 2^-14 sqrt(D).
+// (Measured against rows in bfloat16 with 2^-8 |row| for e: exact distances per point 1M x 100 28 -> 22, 1M x 256 in 64 clusters
+// 74 -> 39, sparse 70,000 x 784 with K = 90 185 -> 140, 10M x 32 49 -> 42; merge 3.54 -> 2.77, 13.9 -> 8.25, 15.9 -> 12.6 and 23.6 ->
+// 20.1 ms.  bfloat16 with the measured e: 24, 41, 147 and 45.)
 // The outcome is one bit per (entry of the graph, neighbour slot): pass[p K + k] for the
 // entry (p, k) = q has bit n set iff neighbour n of q may enter row p (an element of R(q)
 // is the number p K + k of the entry, so the join knows where to write and the merge
@@ -30,6 +35,7 @@
 #include "wave64.hpp"
 #include "forest.hpp"
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 
 namespace rsfk {
@@ -50,7 +56,7 @@ struct ExploreWorkspace {
     int* bin_start = nullptr;  // n_bins + 1
     int* part_off = nullptr;   // n_parts x n_bins: where the entries of a part start inside a bin
     uint32_t* pass = nullptr;  // N*K*MW, indexed by entry number
-    float2* norm_tau = nullptr; // N: norm of the bfloat16 row and last slot of the K-NN row of a point, side by side
+    float2* recs = nullptr;    // N: norm of a point's row in the copy, and the bar its candidates have to pass (k_join_records)
     uint16_t* bounds = nullptr; // N*K*32*MW lower bounds of the marked pairs (bfloat16, rounded down), or null
     bool tiled = false;         // the builder of medium graphs: bins of 2^cshift points, rows of 2^fshift of them at a time
     // the builder for large graphs (staged_rev_*): two scatters through LDS instead of one straight to memory
@@ -66,10 +72,9 @@ struct ExploreWorkspace {
 };
 namespace {
 
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 
-constexpr float kU = 1.0f / 256.0f;         // unit roundoff of bfloat16
 constexpr int kMaxBins = 6144;
 constexpr int kMaxShift = 13;
 // entry numbers are ints, and the passes over the graph look 768 entries ahead of the one they test
@@ -575,18 +580,48 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_rows(const int2* __restri
     }
 }
 
-// What the join needs of a point besides its row, in one 8-byte record (one gather instead of two).
-__global__ void k_norm_tau(const float* __restrict__ norms, const float* __restrict__ knn_dist, int N, int K,
-                           float2* __restrict__ out)
+// What the join needs of a point besides its row, in one 8-byte record (one gather instead of two): (norm, bar).
+// A sum bar + e_c is at least 1 + 2^-21 times the sum of the values it stands for, which covers the roundings of the sum, its square
+// and the comparison.  1e-30 under the root covers what underflow takes from the chain.  An infinite or NaN last slot makes bar
+// infinite or NaN, a row that is not finite makes d~ - E1 NaN, and a comparison with that drops nothing.
+constexpr float kJoinUp = 1.0f + 1.0f / 1048576.0f;
+__global__ void k_join_records(const float* __restrict__ norms, const float* __restrict__ errs, const float* __restrict__ scale,
+                               const float* __restrict__ knn_dist, int N, int K, float one_minus_gamma, float2* __restrict__ out)
 {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p < N) out[p] = make_float2(norms[p], knn_dist[(size_t)p * K + (K - 1)]);
+    if (p >= N) return;
+    const float tau = knn_dist[(size_t)p * K + (K - 1)];
+    out[p] = make_float2(norms[p], (*scale * sqrtf(tau / one_minus_gamma + 1e-30f) + errs[p]) * kJoinUp);
 }
 
-// One wavefront per q.  Per-wavefront LDS (ints): cq[KP] | pid[32] | pn[32] | ptau[32] | pe[32], KP = K rounded up to 32.
+// d~ - E1 of a pair, from S = n_p + n_c and the product g of the rows
+__device__ __forceinline__ float join_least(float S, float g, float kappa)
+{
+    return __builtin_fmaf(-kappa, S, __builtin_fmaf(-2.0f, g, S));
+}
+
+// May the pair enter row p?  (true when anything is NaN; a tie at the last slot may still enter: smaller index)
+__device__ __forceinline__ bool join_may(float least, float bar, float e_c)
+{
+    const float w = bar + e_c;
+    return !(least > w * w);
+}
+
+// The lower bound of the exact distance of a marked pair, as kept for the merge: upper 16 bits, which rounds down.  2^-20 for the
+// square root (one unit) and the roundings here.  A bound below zero (or NaN) says nothing: 0.
+__device__ __forceinline__ uint32_t join_bound16(float least, float e_p, float e_c, float inv_scale, float one_minus_gamma)
+{
+    constexpr float kDown = 1.0f - 1.0f / 1048576.0f;
+    const float t = __builtin_fmaf(__builtin_amdgcn_sqrtf(fmaxf(least, 0.0f)), kDown, -(e_p + e_c) * kJoinUp) * inv_scale;
+    const float lower = __builtin_fmaf(t * t, one_minus_gamma * kDown, -1e-30f);
+    return t > 0.0f && lower > 0.0f ? __float_as_uint(lower) >> 16 : 0u;
+}
+
+// One wavefront per q.  Per-wavefront LDS (ints): cq[KP] | pid[32] | pn[32] | pbar[32] | perr[32] | pe[32], KP = K rounded up to 32.
+// (five wavefronts per SIMD: 1M x 256 8.7 -> 8.2 ms against four, for three spilled registers)
 template <int WAVES, bool BOUNDS>
-__global__ __launch_bounds__(64 * WAVES) void k_explore_join(Bf16Copy bf, int N, int K, const int* __restrict__ old_idx,
-                                                              const float2* __restrict__ norm_tau,
+__global__ __launch_bounds__(64 * WAVES, 5) void k_explore_join(JoinCopy jc, int N, int D, int K, const int* __restrict__ old_idx,
+                                                              const float2* __restrict__ recs,
                                                               const int* __restrict__ offs, const int* __restrict__ rev,
                                                               uint32_t* __restrict__ pass, uint16_t* __restrict__ bounds, int KP, int bpitch, int ksteps,
                                                               float kappa, float one_minus_gamma, int wave_lds_ints,
@@ -602,9 +637,11 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_join(Bf16Copy bf, int N,
     int* cq = lds_join + (size_t)wave * (size_t)wave_lds_ints;
     int* pid = cq + KP;
     float* pn = reinterpret_cast<float*>(pid + 32);
-    float* ptau = pn + 32;
-    int* pe = reinterpret_cast<int*>(ptau + 32);
+    float* pbar = pn + 32;
+    float* perr = pbar + 32;
+    int* pe = reinterpret_cast<int*>(perr + 32);
     const int MW = KP >> 5;
+    const float inv_scale = 1.0f / *jc.scale(D);
 
     for (int k = lane; k < KP; k += 64) {
         int c = k < K ? old_idx[(size_t)q * K + k] : -1;
@@ -621,34 +658,35 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_join(Bf16Copy bf, int N,
             const int p = my_e >= 0 ? (int)(((uint64_t)div_m * (uint64_t)(uint32_t)my_e) >> div_s) : -1;
             pid[lane] = p;
             pe[lane] = my_e;
-            const float2 nt = p >= 0 ? norm_tau[p] : make_float2(0.0f, 0.0f);
-            pn[lane] = nt.x;
-            ptau[lane] = nt.y;
+            const float2 rec = p >= 0 ? recs[p] : make_float2(0.0f, 0.0f);
+            pn[lane] = rec.x;
+            pbar[lane] = rec.y;
+            if (BOUNDS) perr[lane] = p >= 0 ? jc.errs[p] : 0.0f;
         }
         wave_lds_sync();
 
         const int pm = pid[lane & 31];
-        const uint16_t* ra = bf.rows + (size_t)(pm >= 0 ? pm : q) * (size_t)bpitch + 8 * (lane >> 5);
+        const uint16_t* ra = jc.rows + (size_t)(pm >= 0 ? pm : q) * (size_t)bpitch + 8 * (lane >> 5);
         const int mbase = 4 * (lane >> 5);
         for (int ct = 0; ct < MW; ++ct) {
             const int cid = cq[ct * 32 + (lane & 31)];
-            const uint16_t* rb = bf.rows + (size_t)(cid >= 0 ? cid : q) * (size_t)bpitch + 8 * (lane >> 5);
-            const float cn = cid >= 0 ? norm_tau[cid].x : 0.0f;
+            const uint16_t* rb = jc.rows + (size_t)(cid >= 0 ? cid : q) * (size_t)bpitch + 8 * (lane >> 5);
+            const float cn = recs[cid >= 0 ? cid : q].x, ce = jc.errs[cid >= 0 ? cid : q] * kJoinUp;
             f32x16 g;
 #pragma unroll
             for (int i = 0; i < 16; ++i) g[i] = 0.0f;
             for (int k0 = 0; k0 < ksteps; k0 += 4) {
-                bf16x8 a[4], b[4];
+                f16x8 a[4], b[4];
 #pragma unroll
                 for (int u = 0; u < 4; ++u) {
                     if (k0 + u < ksteps) {
-                        a[u] = *reinterpret_cast<const bf16x8*>(ra + 16 * (k0 + u));
-                        b[u] = *reinterpret_cast<const bf16x8*>(rb + 16 * (k0 + u));
+                        a[u] = *reinterpret_cast<const f16x8*>(ra + 16 * (k0 + u));
+                        b[u] = *reinterpret_cast<const f16x8*>(rb + 16 * (k0 + u));
                     }
                 }
 #pragma unroll
                 for (int u = 0; u < 4; ++u)
-                    if (k0 + u < ksteps) g = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[u], b[u], g, 0, 0, 0);
+                    if (k0 + u < ksteps) g = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[u], b[u], g, 0, 0, 0);
             }
             // Accumulator i of lane l: point m = 4 (l / 32) + 8 (i / 4) + i % 4 of the tile, column = neighbour l % 32
             // of this group of 32.  The ballot over the wavefront therefore holds the 32-bit masks of two points:
@@ -657,21 +695,12 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_join(Bf16Copy bf, int N,
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
                 const int m = mbase + 8 * (i >> 2) + (i & 3);
-                const float S = pn[m] + cn;
-                const float dt = __builtin_fmaf(-2.0f, g[i], S);
-                const float e1 = kappa * S;
-                const float dhi = fmaxf(dt + e1, 0.0f);
-                const float Q = 2.0001f * S;
-                const float ebf = 1.01f * (2.0f * kU * __builtin_sqrtf(dhi * Q) + kU * kU * Q);
-                const float lower = (dt - e1 - ebf) * one_minus_gamma - 1e-30f;
-                const bool skip = lower > ptau[m];        // false if anything is NaN; a tie at the last slot may still enter (smaller index)
-                const bool marked = cid >= 0 && !skip;
+                const float least = join_least(pn[m] + cn, g[i], kappa);
+                const bool marked = cid >= 0 && join_may(least, pbar[m], ce);
                 const uint64_t bm = ballot64(marked);
-                if (BOUNDS && marked && m < np) {
-                    // a bound below zero (or NaN) says nothing: 0.  Dropping the low half of a positive float rounds down.
-                    const uint32_t lb = lower > 0.0f ? __float_as_uint(lower) >> 16 : 0u;
-                    bounds[(size_t)pe[m] * (size_t)KP + ct * 32 + (lane & 31)] = (uint16_t)lb;
-                }
+                if (BOUNDS && marked && m < np)
+                    bounds[(size_t)pe[m] * (size_t)KP + ct * 32 + (lane & 31)] =
+                        (uint16_t)join_bound16(least, perr[m], ce, inv_scale, one_minus_gamma);
                 const int m_lo = 8 * (i >> 2) + (i & 3);
                 if (lane == m_lo) mine = (uint32_t)bm;
                 if (lane == m_lo + 4) mine = (uint32_t)(bm >> 32);
@@ -686,17 +715,17 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_join(Bf16Copy bf, int N,
 // and stay in registers for all tiles of R(q); the norm and last slot of the points of a tile travel while their rows
 // are fetched.  A wavefront then has three dependent trips to memory per q (row offsets and neighbours | their rows
 // and the elements of R(q) | the rows of those points) instead of five, and short rows leave room for twice the
-// wavefronts per SIMD.  The bound is that of k_explore_join, term by term.
+// wavefronts per SIMD.  The bound is that of k_explore_join.
 template <int WAVES, int KS>
-__global__ __launch_bounds__(64 * WAVES) void k_explore_join_short(Bf16Copy bf, int N, int K, const int* __restrict__ old_idx,
-                                                                    const float2* __restrict__ norm_tau,
+__global__ __launch_bounds__(64 * WAVES) void k_explore_join_short(JoinCopy jc, int N, int K, const int* __restrict__ old_idx,
+                                                                    const float2* __restrict__ recs,
                                                                     const int* __restrict__ offs, const int* __restrict__ rev,
                                                                     uint32_t* __restrict__ pass, int bpitch, int ksteps,
-                                                                    float kappa, float one_minus_gamma, uint32_t div_m, int div_s,
+                                                                    float kappa, float any_rel, float any_abs, uint32_t div_m, int div_s,
                                                                     const int* __restrict__ order)
 {
     __shared__ int pid_s[WAVES][32];
-    __shared__ float pn_s[WAVES][32], ptau_s[WAVES][32];
+    __shared__ float pn_s[WAVES][32], pbar_s[WAVES][32];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int item = die_local_place(blockIdx.x, gridDim.x) * WAVES + wave;
     if (item >= N) return;                                // whole wavefront leaves together
@@ -706,48 +735,49 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_join_short(Bf16Copy bf, 
     int cid = col < K ? old_idx[(size_t)q * K + col] : -1;
     if (R <= 0) return;
     if (cid < 0 || cid >= N) cid = -1;
-    const uint16_t* rb = bf.rows + (size_t)(cid >= 0 ? cid : q) * (size_t)bpitch + 8 * hi;
-    bf16x8 b[KS];
+    const uint16_t* rb = jc.rows + (size_t)(cid >= 0 ? cid : q) * (size_t)bpitch + 8 * hi;
+    f16x8 b[KS];
 #pragma unroll
     for (int u = 0; u < KS; ++u) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) b[u][i] = (__bf16)0.0f;
-        if (u < ksteps) b[u] = *reinterpret_cast<const bf16x8*>(rb + 16 * u);
+        for (int i = 0; i < 8; ++i) b[u][i] = (_Float16)0.0f;
+        if (u < ksteps) b[u] = *reinterpret_cast<const f16x8*>(rb + 16 * u);
     }
-    const float cn = cid >= 0 ? norm_tau[cid].x : 0.0f;
+    const float cn = recs[cid >= 0 ? cid : q].x;
+    const float ce = __builtin_fmaf(any_rel, __builtin_amdgcn_sqrtf(cn), any_abs);
     const int mbase = 4 * hi;
     int* pid = pid_s[wave];
     float* pn = pn_s[wave];
-    float* ptau = ptau_s[wave];
+    float* pbar = pbar_s[wave];
 
     for (int pt0 = 0; pt0 < R; pt0 += 32) {
         const int np = min(32, R - pt0);
         int my_e = -1;                                    // lanes 0..31: the graph entry (p, k) with q = neighbour k of p
-        float2 nt = make_float2(0.0f, 0.0f);
+        float2 rec = make_float2(0.0f, 0.0f);
         if (lane < 32) {
             my_e = lane < np ? rev[(size_t)r0 + pt0 + lane] : -1;
             const int p = my_e >= 0 ? (int)(((uint64_t)div_m * (uint64_t)(uint32_t)my_e) >> div_s) : -1;
             pid[lane] = p;
-            if (p >= 0) nt = norm_tau[p];
+            if (p >= 0) rec = recs[p];
         }
         wave_lds_sync();
         const int pm = pid[col];
-        const uint16_t* ra = bf.rows + (size_t)(pm >= 0 ? pm : q) * (size_t)bpitch + 8 * hi;
-        bf16x8 a[KS];
+        const uint16_t* ra = jc.rows + (size_t)(pm >= 0 ? pm : q) * (size_t)bpitch + 8 * hi;
+        f16x8 a[KS];
 #pragma unroll
         for (int u = 0; u < KS; ++u) {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) a[u][i] = (__bf16)0.0f;
-            if (u < ksteps) a[u] = *reinterpret_cast<const bf16x8*>(ra + 16 * u);
+            for (int i = 0; i < 8; ++i) a[u][i] = (_Float16)0.0f;
+            if (u < ksteps) a[u] = *reinterpret_cast<const f16x8*>(ra + 16 * u);
         }
         f32x16 g;
 #pragma unroll
         for (int i = 0; i < 16; ++i) g[i] = 0.0f;
 #pragma unroll
-        for (int u = 0; u < KS; ++u) g = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[u], b[u], g, 0, 0, 0);
+        for (int u = 0; u < KS; ++u) g = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[u], b[u], g, 0, 0, 0);
         if (lane < 32) {
-            pn[lane] = nt.x;
-            ptau[lane] = nt.y;
+            pn[lane] = rec.x;
+            pbar[lane] = rec.y;
         }
         wave_lds_sync();
         // Accumulator i of lane l: point m = 4 (l / 32) + 8 (i / 4) + i % 4 of the tile, column = neighbour l % 32.
@@ -755,15 +785,8 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_join_short(Bf16Copy bf, 
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
             const int m = mbase + 8 * (i >> 2) + (i & 3);
-            const float S = pn[m] + cn;
-            const float dt = __builtin_fmaf(-2.0f, g[i], S);
-            const float e1 = kappa * S;
-            const float dhi = fmaxf(dt + e1, 0.0f);
-            const float Q = 2.0001f * S;
-            const float ebf = 1.01f * (2.0f * kU * __builtin_sqrtf(dhi * Q) + kU * kU * Q);
-            const float lower = (dt - e1 - ebf) * one_minus_gamma - 1e-30f;
-            const bool skip = lower > ptau[m];            // false if anything is NaN; a tie at the last slot may still enter
-            const uint64_t bm = ballot64(cid >= 0 && !skip);
+            const float least = join_least(pn[m] + cn, g[i], kappa);
+            const uint64_t bm = ballot64(cid >= 0 && join_may(least, pbar[m], ce));
             const int m_lo = 8 * (i >> 2) + (i & 3);
             if (lane == m_lo) mine = (uint32_t)bm;
             if (lane == m_lo + 4) mine = (uint32_t)(bm >> 32);
@@ -779,13 +802,14 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_join_short(Bf16Copy bf, 
 // points of R(q) and all neighbours of q pass through LDS together, 64 dimensions at a time (the next 64 are requested
 // while these are used), and the wavefronts share the pairs (tile of R(q), group of neighbours) among them, each
 // keeping the accumulators of its pairs: every row is read once per 96 points of R(q).  Bound and outputs are those
-// of k_explore_join.  NPW = pairs per wavefront (3: K <= 128, 6: K <= 256).
+// of k_explore_join.  NPW = pairs per wavefront (3: K <= 128, 6: K <= 256); the
+// first at three wavefronts per SIMD: 70,000 x 784, K = 90 6.9 -> 5.1 ms against two.
 constexpr int kJwP = 96;                    // points of R(q) worked on together (three tiles)
-constexpr int kJwRowBytes = 144;            // 64 bfloat16 values + 16 bytes: rows start in different banks
+constexpr int kJwRowBytes = 144;            // 64 float16 values + 16 bytes: rows start in different banks
 
 template <bool BOUNDS, int NPW>
-__global__ __launch_bounds__(256) void k_explore_join_wg(Bf16Copy bf, int N, int K, const int* __restrict__ old_idx,
-                                                         const float2* __restrict__ norm_tau, const int* __restrict__ offs,
+__global__ __launch_bounds__(256, NPW == 3 ? 3 : 1) void k_explore_join_wg(JoinCopy jc, int N, int D, int K, const int* __restrict__ old_idx,
+                                                         const float2* __restrict__ recs, const int* __restrict__ offs,
                                                          const int* __restrict__ rev, uint32_t* __restrict__ pass,
                                                          uint16_t* __restrict__ bounds, int KP, int bpitch, int ksteps,
                                                          float kappa, float one_minus_gamma, uint32_t div_m, int div_s,
@@ -796,10 +820,12 @@ __global__ __launch_bounds__(256) void k_explore_join_wg(Bf16Copy bf, int N, int
     unsigned char* rowsb = lds_jw;                                         // kJwP + KP rows of 144 bytes
     int* cq = reinterpret_cast<int*>(rowsb + (size_t)(kJwP + KP) * kJwRowBytes);
     float* cn = reinterpret_cast<float*>(cq + KP);
-    int* pid = reinterpret_cast<int*>(cn + KP);
+    float* cerr = cn + KP;
+    int* pid = reinterpret_cast<int*>(cerr + KP);
     int* pe = pid + kJwP;
     float* pn = reinterpret_cast<float*>(pe + kJwP);
-    float* ptau = pn + kJwP;
+    float* pbar = pn + kJwP;
+    float* perr = pbar + kJwP;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int n = lane & 31, h = lane >> 5;
     const int item = die_local_place(blockIdx.x, gridDim.x);
@@ -809,11 +835,13 @@ __global__ __launch_bounds__(256) void k_explore_join_wg(Bf16Copy bf, int N, int
     if (R <= 0) return;
     const int MW = KP >> 5;
     const int nrows = kJwP + KP;
+    const float inv_scale = 1.0f / *jc.scale(D);
     for (int k = tid; k < KP; k += 256) {
         int c = k < K ? old_idx[(size_t)q * K + k] : -1;
         if (c < 0 || c >= N) c = -1;
         cq[k] = c;
-        cn[k] = c >= 0 ? norm_tau[c].x : 0.0f;
+        cn[k] = c >= 0 ? recs[c].x : 0.0f;
+        cerr[k] = c >= 0 ? jc.errs[c] * kJoinUp : 0.0f;
     }
     for (int pg = 0; pg < R; pg += kJwP) {
         const int npg = min(kJwP, R - pg);
@@ -822,11 +850,12 @@ __global__ __launch_bounds__(256) void k_explore_join_wg(Bf16Copy bf, int N, int
         if (tid < kJwP) {
             const int e = tid < npg ? rev[(size_t)r0 + pg + tid] : -1;
             const int p = e >= 0 ? (int)(((uint64_t)div_m * (uint64_t)(uint32_t)e) >> div_s) : -1;
-            const float2 nt = p >= 0 ? norm_tau[p] : make_float2(0.0f, 0.0f);
+            const float2 rec = p >= 0 ? recs[p] : make_float2(0.0f, 0.0f);
             pid[tid] = p;
             pe[tid] = e;
-            pn[tid] = nt.x;
-            ptau[tid] = nt.y;
+            pn[tid] = rec.x;
+            pbar[tid] = rec.y;
+            if (BOUNDS) perr[tid] = p >= 0 ? jc.errs[p] : 0.0f;
         }
         __syncthreads();
         f32x16 acc[NPW];
@@ -846,7 +875,7 @@ __global__ __launch_bounds__(256) void k_explore_join_wg(Bf16Copy bf, int N, int
                     const int id = r < kJwP ? pid[r] : cq[r - kJwP];
                     const int el = c0 * 16 + pc * 8;
                     if (id >= 0 && el < ksteps * 16)
-                        pre[j] = *reinterpret_cast<const uint4*>(bf.rows + (size_t)id * (size_t)bpitch + el);
+                        pre[j] = *reinterpret_cast<const uint4*>(jc.rows + (size_t)id * (size_t)bpitch + el);
                 }
             }
         };
@@ -870,9 +899,9 @@ __global__ __launch_bounds__(256) void k_explore_join_wg(Bf16Copy bf, int N, int
 #pragma unroll
                     for (int u = 0; u < 4; ++u) {
                         if (c0 + u < ksteps) {
-                            const bf16x8 a = *reinterpret_cast<const bf16x8*>(ra + 32 * u);
-                            const bf16x8 b = *reinterpret_cast<const bf16x8*>(rb + 32 * u);
-                            acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc[i], 0, 0, 0);
+                            const f16x8 a = *reinterpret_cast<const f16x8*>(ra + 32 * u);
+                            const f16x8 b = *reinterpret_cast<const f16x8*>(rb + 32 * u);
+                            acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, acc[i], 0, 0, 0);
                         }
                     }
                 }
@@ -887,26 +916,16 @@ __global__ __launch_bounds__(256) void k_explore_join_wg(Bf16Copy bf, int N, int
                 const int pt = pair / MW, ct = pair - pt * MW;
                 const int col = ct * 32 + n;
                 const int cid = cq[col];
-                const float cnv = cn[col];
+                const float cnv = cn[col], ce = cerr[col];
                 uint32_t mine = 0;
 #pragma unroll
                 for (int j = 0; j < 16; ++j) {
                     const int m = pt * 32 + 4 * h + 8 * (j >> 2) + (j & 3);
-                    const float S = pn[m] + cnv;
-                    const float dt = __builtin_fmaf(-2.0f, acc[i][j], S);
-                    const float e1 = kappa * S;
-                    const float dhi = fmaxf(dt + e1, 0.0f);
-                    const float Q = 2.0001f * S;
-                    const float ebf = 1.01f * (2.0f * kU * __builtin_sqrtf(dhi * Q) + kU * kU * Q);
-                    const float lower = (dt - e1 - ebf) * one_minus_gamma - 1e-30f;
-                    const bool skip = lower > ptau[m];            // false if anything is NaN; a tie at the last slot may still enter
-                    const bool marked = cid >= 0 && !skip;
+                    const float least = join_least(pn[m] + cnv, acc[i][j], kappa);
+                    const bool marked = cid >= 0 && join_may(least, pbar[m], ce);
                     const uint64_t bm = ballot64(marked);
-                    if (BOUNDS && marked && m < npg) {
-                        // a bound below zero (or NaN) says nothing: 0.  Dropping the low half of a positive float rounds down.
-                        const uint32_t lb = lower > 0.0f ? __float_as_uint(lower) >> 16 : 0u;
-                        bounds[(size_t)pe[m] * (size_t)KP + col] = (uint16_t)lb;
-                    }
+                    if (BOUNDS && marked && m < npg)
+                        bounds[(size_t)pe[m] * (size_t)KP + col] = (uint16_t)join_bound16(least, perr[m], ce, inv_scale, one_minus_gamma);
                     const int m_lo = 8 * (j >> 2) + (j & 3);
                     if (lane == m_lo) mine = (uint32_t)bm;
                     if (lane == m_lo + 4) mine = (uint32_t)(bm >> 32);
@@ -1016,7 +1035,7 @@ int explore_ws_alloc(ExploreWorkspace** out, int N, int K, bool with_bounds, boo
     if (dm(&w->rev, total) != hipSuccess || dm(&w->bin_eq, 2 * total) != hipSuccess ||
         dm(&w->offs, (size_t)N + 1) != hipSuccess || dm(&w->bin_size, (size_t)w->n_bins) != hipSuccess ||
         dm(&w->bin_start, (size_t)w->n_bins + 1) != hipSuccess ||
-        dm(&w->part_off, (size_t)w->n_parts * (size_t)w->n_bins) != hipSuccess || (!graph_only && (dm(&w->pass, total * w->MW) != hipSuccess || dm(&w->norm_tau, 2 * (size_t)N) != hipSuccess)) ||
+        dm(&w->part_off, (size_t)w->n_parts * (size_t)w->n_bins) != hipSuccess || (!graph_only && (dm(&w->pass, total * w->MW) != hipSuccess || dm(&w->recs, 2 * (size_t)N) != hipSuccess)) ||
         dm(&w->todo, 2 * ((size_t)N + 1)) != hipSuccess) {
         explore_ws_free(w);
         if (!graph_only) set_last_error("exploration workspace: out of device memory");
@@ -1037,7 +1056,7 @@ int explore_ws_alloc(ExploreWorkspace** out, int N, int K, bool with_bounds, boo
 void explore_ws_free(ExploreWorkspace* w)
 {
     if (!w) return;
-    void* bufs[] = {w->rev, w->bin_eq, w->offs, w->bin_size, w->bin_start, w->part_off, w->pass, w->norm_tau, w->todo, w->bounds,
+    void* bufs[] = {w->rev, w->bin_eq, w->offs, w->bin_size, w->bin_start, w->part_off, w->pass, w->recs, w->todo, w->bounds,
                     w->bin_eq2, w->fine_size, w->fine_start, w->sub_off};
     for (void* b : bufs)
         ws_free(b);
@@ -1117,30 +1136,33 @@ int launch_reversed_graph(ExploreWorkspace* w, const int* old_idx, int N, int K,
 }
 
 // Fill pass (and bounds) from the snapshot old_idx and the current last slots of knn_dist (rows sorted by distance).
-int launch_explore_join(ExploreWorkspace* w, const Bf16Copy& bf, int N, int D, int K, const int* old_idx,
+int launch_explore_join(ExploreWorkspace* w, const JoinCopy& jc, int N, int D, int K, const int* old_idx,
                         const float* knn_dist, hipStream_t stream, const int* order)
 {
     RSFK_CHECK(w && w->N == N && w->K == K, "exploration join: workspace does not match");
     RSFK_CHECK(K >= 1 && K <= 256, "exploration join: K must be in 1..256");
     RSFK_CHECK((size_t)N * (size_t)K < kMaxEntries, "exploration join: N*K must be below 2^31 - 4096");
     if (launch_reversed_graph(w, old_idx, N, K, stream)) return 1;
-    hipLaunchKernelGGL(k_norm_tau, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, stream, bf.norms, knn_dist, N, K, w->norm_tau);
-    RSFK_HIP(hipGetLastError());
 
     constexpr int kWaves = 4;
     const int KP = (K + 31) & ~31;
-    const int wave_ints = (KP + 128 + 3) & ~3;
+    const int wave_ints = (KP + 160 + 3) & ~3;
     const size_t lds = (size_t)kWaves * (size_t)wave_ints * sizeof(int);
-    const int ksteps = (bf16_valid(D) + 15) / 16;
-    RSFK_CHECK(ksteps * 16 <= bf16_pitch(D), "exploration join: bfloat16 rows too short");
+    const int ksteps = (D + 15) / 16;
+    RSFK_CHECK(ksteps * 16 <= join_pitch(D), "exploration join: rows of the copy too short");
     const float kappa = (float)(ksteps * 16 + 16) * (1.0f / 2097152.0f);            // (Dp + 16) 2^-21
     const float one_minus_gamma = 1.0f - (float)(D + 8) * (1.0f / 4194304.0f);      // 1 - (D + 8) 2^-22
     RSFK_CHECK(one_minus_gamma > 0.5f, "exploration join: D too large");
+    hipLaunchKernelGGL(k_join_records, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, stream, jc.norms, jc.errs, jc.scale(D),
+                       knn_dist, N, K, one_minus_gamma, w->recs);
+    RSFK_HIP(hipGetLastError());
     if (!w->bounds && KP == 32 && ksteps <= 8) {
         const dim3 grid(grid_for_dies(((size_t)N + kWaves - 1) / kWaves)), block(64 * kWaves);
+        // rounding of any row: 2^-11 of a value, 2^-14 of one set to zero, and errs' own terms (3e-3 covers these and the root)
+        const float any_rel = 1.003f / 2048.0f, any_abs = 1.001f * std::sqrt((float)D) / 16384.0f + 1e-6f;
 #define RSFK_JOIN_SHORT(KSV)                                                                                                \
-        hipLaunchKernelGGL((k_explore_join_short<kWaves, KSV>), grid, block, 0, stream, bf, N, K, old_idx, w->norm_tau, w->offs, \
-                           w->rev, w->pass, bf16_pitch(D), ksteps, kappa, one_minus_gamma, w->div_m, w->div_s, order)
+        hipLaunchKernelGGL((k_explore_join_short<kWaves, KSV>), grid, block, 0, stream, jc, N, K, old_idx, w->recs, w->offs, \
+                           w->rev, w->pass, join_pitch(D), ksteps, kappa, any_rel, any_abs, w->div_m, w->div_s, order)
         if (ksteps <= 2) RSFK_JOIN_SHORT(2);
         else if (ksteps <= 4) RSFK_JOIN_SHORT(4);
         else RSFK_JOIN_SHORT(8);
@@ -1148,13 +1170,13 @@ int launch_explore_join(ExploreWorkspace* w, const Bf16Copy& bf, int N, int D, i
     } else if (KP > 32 && join_wg_on()) {
         // one workgroup per q: every row once per 96 points of R(q).  (Rows of at most 32 neighbours have one pair per
         // tile of R(q): too little for four wavefronts; 1M x 256, K = 32: 8.1 ms against 12.6.)
-        const size_t lds_wg = (size_t)(kJwP + KP) * kJwRowBytes + (size_t)KP * 8 + (size_t)kJwP * 16;
+        const size_t lds_wg = (size_t)(kJwP + KP) * kJwRowBytes + (size_t)KP * 12 + (size_t)kJwP * 20;
 #define RSFK_JOIN_WG(BV, NV)                                                                                                \
         do {                                                                                                               \
             RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_explore_join_wg<BV, NV>),                         \
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_wg));                       \
-            hipLaunchKernelGGL((k_explore_join_wg<BV, NV>), dim3(grid_for_dies((size_t)N)), dim3(256), lds_wg, stream, bf, N, K,  \
-                               old_idx, w->norm_tau, w->offs, w->rev, w->pass, w->bounds, KP, bf16_pitch(D), ksteps, kappa,  \
+            hipLaunchKernelGGL((k_explore_join_wg<BV, NV>), dim3(grid_for_dies((size_t)N)), dim3(256), lds_wg, stream, jc, N, D, K,  \
+                               old_idx, w->recs, w->offs, w->rev, w->pass, w->bounds, KP, join_pitch(D), ksteps, kappa,  \
                                one_minus_gamma, w->div_m, w->div_s, order);                                                \
         } while (0)
         if (w->bounds && KP <= 128) RSFK_JOIN_WG(true, 3);
@@ -1164,11 +1186,11 @@ int launch_explore_join(ExploreWorkspace* w, const Bf16Copy& bf, int N, int D, i
 #undef RSFK_JOIN_WG
     } else if (w->bounds)
         hipLaunchKernelGGL((k_explore_join<kWaves, true>), dim3(grid_for_dies(((size_t)N + kWaves - 1) / kWaves)), dim3(64 * kWaves), lds,
-                           stream, bf, N, K, old_idx, w->norm_tau, w->offs, w->rev, w->pass, w->bounds, KP, bf16_pitch(D), ksteps,
+                           stream, jc, N, D, K, old_idx, w->recs, w->offs, w->rev, w->pass, w->bounds, KP, join_pitch(D), ksteps,
                            kappa, one_minus_gamma, wave_ints, w->div_m, w->div_s, order);
     else
         hipLaunchKernelGGL((k_explore_join<kWaves, false>), dim3(grid_for_dies(((size_t)N + kWaves - 1) / kWaves)), dim3(64 * kWaves), lds,
-                           stream, bf, N, K, old_idx, w->norm_tau, w->offs, w->rev, w->pass, w->bounds, KP, bf16_pitch(D), ksteps,
+                           stream, jc, N, D, K, old_idx, w->recs, w->offs, w->rev, w->pass, w->bounds, KP, join_pitch(D), ksteps,
                            kappa, one_minus_gamma, wave_ints, w->div_m, w->div_s, order);
     RSFK_HIP(hipGetLastError());
     return 0;

@@ -95,6 +95,10 @@ struct Bf16Guard {
     Bf16Copy c;
     ~Bf16Guard() { bf16_copy_free(&c); }
 };
+struct JoinCopyGuard {
+    JoinCopy c;
+    ~JoinCopyGuard() { join_copy_free(&c); }
+};
 struct ExploreWsGuard {
     ExploreWorkspace* w = nullptr;
     ~ExploreWsGuard() { explore_ws_free(w); }
@@ -418,17 +422,17 @@ int knn_forest_device(int n_trees, int K, int N, int D, int MIN, int MAX, int MA
         DevBuf old;
         if (ws_alloc(&old.p, sizeof(int) * (size_t)N * (size_t)K)) return 1;
         ExploreWsGuard ews;      // without a workspace every point enumerates its own candidates
-        Bf16Guard bfc;           // centred copy for the join
+        JoinCopyGuard jc;
         DevBuf stat;             // count of the exact distances (for the report)
         if (ws_alloc(&stat.p, sizeof(unsigned long long) * kExploreStatWords)) return 1;
         RSFK_HIP(hipMemsetAsync(stat.p, 0, sizeof(unsigned long long) * kExploreStatWords, stream));
         if (explore_join_enabled(N, K)) {
             if (explore_ws_alloc(&ews.w, N, K, explore_join_keeps_bounds(N, D, K))) return 1;
-            if (bf16_copy_alloc(&bfc.c, N, D, true) || bf16_copy_fill(bfc.c, d_points, N, D, stream)) return 1;
+            if (join_copy_alloc(&jc.c, N, D) || join_copy_fill(jc.c, d_points, N, D, stream)) return 1;
         }
         for (int it = 0; it < nnef; ++it) {
             // (the bucket step of the forest, and every exploration pass, leave all rows in order)
-            if (launch_explore(d_points, plain_copy ? &bf.c : nullptr, &bfc.c, N, D, K, d_idx, d_dist, static_cast<int*>(old.p), ews.w, stream,
+            if (launch_explore(d_points, plain_copy ? &bf.c : nullptr, &jc.c, N, D, K, d_idx, d_dist, static_cast<int*>(old.p), ews.w, stream,
                                n_trees > 0 || it > 0, static_cast<unsigned long long*>(stat.p), static_cast<const int*>(order.p)))
                 return 1;
         }

@@ -4,6 +4,7 @@
 #include <atomic>
 #include <thread>
 #include "bf16.hpp"
+#include "join_copy.hpp"
 #include <vector>
 
 namespace rsfk {
@@ -208,7 +209,7 @@ const uint16_t* explore_ws_bounds(const ExploreWorkspace* w);
 int* explore_ws_todo(ExploreWorkspace* w, int which);
 // order: null, or a permutation of the points that keeps nearby points together (the buckets of a tree): the points
 // are then worked on in that order, a contiguous eighth of it per die (die_local_place)
-int launch_explore_join(ExploreWorkspace* w, const Bf16Copy& bf, int N, int D, int K, const int* old_idx,
+int launch_explore_join(ExploreWorkspace* w, const JoinCopy& jc, int N, int D, int K, const int* old_idx,
                         const float* knn_dist, hipStream_t stream, const int* order = nullptr);
 
 // explore.hip
@@ -216,7 +217,7 @@ int launch_explore_join(ExploreWorkspace* w, const Bf16Copy& bf, int N, int D, i
 // order of their lower bounds (the workspace should then be allocated with room for the bounds)
 bool explore_merge_uses_bounds(int D, int K);
 bool explore_join_keeps_bounds(int N, int D, int K);
-int launch_explore(const float* points, const Bf16Copy* bf, const Bf16Copy* bf_join, int N, int D, int K, int* knn_idx,
+int launch_explore(const float* points, const Bf16Copy* bf, const JoinCopy* jc, int N, int D, int K, int* knn_idx,
                    float* knn_dist, int* old_idx, ExploreWorkspace* ws, hipStream_t stream, bool rows_sorted = false,
                    unsigned long long* stat = nullptr,       // stat: kExploreStatWords words, or null (count_exact)
                    const int* order = nullptr);              // order: see launch_explore_join

@@ -1,0 +1,29 @@
+// 16-bit copy of the points for the join of the exploration (explore_join.hip).
+//
+// Row p holds s (x - mu) in float16 (round to nearest; below 2^-14, the least normal number, zero), mu the column means and s a
+// power of two, padded with zeros to join_pitch(D) values; norms[p] = sum of the squares of the values as rounded, errs[p] >=
+// |s (x_p - mu) - row p| as vectors, measured when the row is made.  Distances do not change under a common shift, and what rounding
+// takes shrinks with the norms.  s is such that the largest value lies between 2^12 and 2^15: nothing overflows, and values down to
+// 2^-26 of the largest keep their 11 bits.  (bfloat16 needs no s, but keeps 8 bits: at the same bytes its rounding is eight times as
+// large.)  A row that is not finite has a norm that is not finite.
+#pragma once
+#include "rsfk_common.hpp"
+
+namespace rsfk {
+
+// rows start on 64-byte boundaries; the kernels take 16 dimensions per step
+__host__ __device__ inline int join_pitch(int D) { return (D + 31) & ~31; }
+
+struct JoinCopy {
+    uint16_t* rows = nullptr;     // N x join_pitch(D)
+    float* norms = nullptr;       // N, in units of s^2
+    float* errs = nullptr;        // N, in units of s
+    float* mu = nullptr;          // column means, then s, then D words of working memory
+    __host__ __device__ const float* scale(int D) const { return mu + D; }
+};
+
+int join_copy_alloc(JoinCopy* c, int N, int D);
+void join_copy_free(JoinCopy* c);
+int join_copy_fill(const JoinCopy& c, const float* points, int N, int D, hipStream_t stream);
+
+}  // namespace rsfk

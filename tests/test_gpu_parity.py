@@ -498,6 +498,39 @@ def test_explore_batches_merged_by_rank(gpu, orc, rng, N, D, K, values):
         assert_knn_equal(gi, gd, oi, od)
 
 
+@pytest.mark.parametrize("values", ["far", "tiny", "huge", "outlier", "spread", "notfinite"])
+@pytest.mark.parametrize("N,D,K", [(2500, 16, 8), (2500, 33, 32), (1500, 129, 20), (1500, 40, 70)])
+def test_explore_screens_rows_of_any_magnitude(gpu, orc, rng, N, D, K, values):
+    """The float16 copy of the join has one scale for all rows: points far from the origin, at the ends of the range of fp32 (squares
+    that vanish or overflow), one row that sets the scale for all others, columns of very different size, rows that are not finite.
+    The three kernels of the join (short rows, long rows, a workgroup per point)."""
+    X = rng.standard_normal((N, D)).astype(np.float32)
+    perm, ls, lz, _ = orc.build_tree(X, K + 1, 2 * K + 2, 5000, 0)
+    if values == "far":
+        X = (X + np.float32(3.0e4)).astype(np.float32)
+    elif values == "tiny":
+        X = (X * np.float32(1e-21)).astype(np.float32)
+    elif values == "huge":
+        X = (X * np.float32(2e18)).astype(np.float32)
+    elif values == "outlier":
+        X[7] = np.float32(1e12)
+    elif values == "spread":
+        X = (X * np.logspace(-9, 9, D)[None, :]).astype(np.float32)
+    else:
+        X[3, D // 2] = np.nan
+        X[11, 0] = np.inf
+        X[N - 1, D - 1] = -np.inf
+        X[0, 1] = np.nan
+    oi, od = orc.init_lists(N, K, self_in=True)
+    orc.bucket_knn(X, K, perm, lz, oi, od, starts=ls)
+    gi, gd = oi.copy(), od.copy()
+    _say("explore magnitudes", N, D, K, values)
+    for _ in range(2):
+        orc.explore(X, K, oi, od)
+        gpu.explore(X, K, gi, gd, 1)
+        assert_knn_equal(gi, gd, oi, od)
+
+
 # ---------------------------------------------------------------------------
 # the whole call, through the entry points the Python package binds
 # ---------------------------------------------------------------------------
