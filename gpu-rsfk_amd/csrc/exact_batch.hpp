@@ -28,27 +28,24 @@ __device__ __forceinline__ float4 load_piece(const float* __restrict__ row, int 
     return d < D ? load_dims(row + d, D - d, vec_ok) : make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
-// Exact distances of the first n candidates of `list` to the point, then offer them.  CH = dimensions
-// staged per step (32 or 16): a step moves 64 rows x CH floats through the tile.  tau_cap: a bound the caller
-// knows for the row's final last slot (candidates above it need not be finished), else +inf.  DEEP: the loads of
+// Exact distances of the first n candidates of `list` to the point, by one wavefront: lane l < ROWS has that of candidate l.  False: the
+// sums were left where all of them were above limit.  CH = dimensions staged per step: a step moves ROWS rows x CH floats through the
+// tile (ROWS (CH + 4) words).  DEEP: the loads of
 // two steps are in flight while a third is being used (two register buffers that take turns, so that waiting for
 // one does not wait for the other): for kernels with few wavefronts per SIMD, whose gathers would otherwise wait
 // for each other.  GROUP: 16-byte pieces of a row whose reads from the tile are requested together (0: one at a time, the
-// form that needs the fewest registers).  RANK: no point of the list is in the row or on the list twice, but at this very distance: the batch is
-// merged by merge_ranked.
-template <int SL, int CH = kChunk, bool DEEP = false, int GROUP = 0, bool RANK = false>
-__device__ __forceinline__ void exact_batch(const ExploreLds& L, const int* list, int n,
-                                            const float* __restrict__ points, int D, bool vec_ok, KnnRow<SL>& row,
-                                            float tau_cap = INFINITY)
+// form that needs the fewest registers).
+template <int CH, int ROWS, bool DEEP, int GROUP>
+__device__ __forceinline__ bool exact_distances(float* tile, const float* xrow, const int* list, int n, const float* __restrict__ points,
+                                                int D, bool vec_ok, float limit, float& acc)
 {
     constexpr int kPieces = CH / 4;         // 16-byte pieces of a row per step = lanes per row
     constexpr int kRows = 64 / kPieces;     // rows per load instruction
-    constexpr int kLoads = 64 / kRows;      // load instructions per step
+    constexpr int kLoads = ROWS / kRows;    // load instructions per step
     constexpr int kP = CH + 4;              // tile pitch: odd number of 16-byte units
     const int lane = lane_id();
     const int sub = lane / kPieces;         // which of the rows of a load instruction
     const int piece = lane % kPieces;       // which 16-byte piece of the segment
-    const int my_c = lane < n ? list[lane] : -1;
     const float* rp[kLoads];
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) {
@@ -63,20 +60,19 @@ __device__ __forceinline__ void exact_batch(const ExploreLds& L, const int* list
                 buf[i] = rp[i] ? load_piece(rp[i], d0 + piece * 4, D, vec_ok) : make_float4(0.f, 0.f, 0.f, 0.f);
         }
     };
-    float acc = 0.0f;
-    const float tau0 = fminf(row.tau, tau_cap);
+    acc = 0.0f;
     // one step: the buffer's values (dimensions d0 ..) go through the tile, the buffer is refilled with the step
     // `ahead` dimensions later, the chains advance.  Returns false when no candidate can enter any more.
     auto step = [&](float4 (&buf)[kLoads], int d0, int ahead) {
         wave_lds_sync();                 // previous step's tile reads are done
 #pragma unroll
         for (int i = 0; i < kLoads; ++i)
-            *reinterpret_cast<float4*>(&L.tile[(i * kRows + sub) * kP + piece * 4]) = buf[i];
+            *reinterpret_cast<float4*>(&tile[(i * kRows + sub) * kP + piece * 4]) = buf[i];
         request(buf, d0 + ahead);
         wave_lds_sync();
         const int pieces = min(kPieces, (D - d0 + 3) >> 2);
-        const float* mine = &L.tile[lane * kP];
-        const float* xs = &L.xrow[d0];
+        const float* mine = &tile[(ROWS < 64 ? lane & (ROWS - 1) : lane) * kP];
+        const float* xs = &xrow[d0];
         auto chain4 = [&](const float4& a, const float4& x) {
             float df;
             df = a.x - x.x; acc = __builtin_fmaf(df, df, acc);
@@ -104,8 +100,8 @@ __device__ __forceinline__ void exact_batch(const ExploreLds& L, const int* list
             for (int q = 0; q < pieces; ++q)
                 chain4(*reinterpret_cast<const float4*>(mine + 4 * q), *reinterpret_cast<const float4*>(xs + 4 * q));
         }
-        // partial sums only grow: once all of them are above the row maximum nothing can enter
-        return ballot64(lane < n && acc <= tau0) != 0;
+        // partial sums only grow: once all of them are above the limit nothing can enter
+        return ballot64(lane < n && acc <= limit) != 0;
     };
     bool finished = true;
     request(pre[0], 0);
@@ -120,9 +116,24 @@ __device__ __forceinline__ void exact_batch(const ExploreLds& L, const int* list
             if (!step(pre[0], d0, CH)) { finished = false; break; }
     }
     wave_lds_sync();
+    return finished;
+}
+
+// The same for up to 64 candidates, which are then offered to the row.  tau_cap: a bound the caller
+// knows for the row's final last slot (candidates above it need not be finished), else +inf.  RANK: no point of the list is in the row
+// or on the list twice, but at this very distance: the batch is merged by merge_ranked.
+template <int SL, int CH = kChunk, bool DEEP = false, int GROUP = 0, bool RANK = false>
+__device__ __forceinline__ void exact_batch(const ExploreLds& L, const int* list, int n,
+                                            const float* __restrict__ points, int D, bool vec_ok, KnnRow<SL>& row,
+                                            float tau_cap = INFINITY)
+{
+    const int lane = lane_id();
+    const int my_c = lane < n ? list[lane] : -1;
+    float acc;
     // (unfinished sums are all above the last slot)
+    const bool finished = exact_distances<CH, 64, DEEP, GROUP>(L.tile, L.xrow, list, n, points, D, vec_ok, fminf(row.tau, tau_cap), acc);
     if (RANK) {
-        static_assert(!RANK || rank_words(SL) <= 64 * kP, "the ranks' working memory takes the place of the tile");
+        static_assert(!RANK || rank_words(SL) <= 64 * (CH + 4), "the ranks' working memory takes the place of the tile");
         row.merge_ranked(lane < n && finished, my_c, acc, reinterpret_cast<double*>(L.tile));
     } else {
         row.merge(lane < n && finished, my_c, acc);

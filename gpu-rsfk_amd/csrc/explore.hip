@@ -42,6 +42,7 @@
 #include "knn_list.hpp"
 #include "forest.hpp"
 #include "exact_batch.hpp"
+#include "join_bounds.hpp"
 #include <algorithm>
 
 namespace rsfk {
@@ -343,6 +344,8 @@ __device__ __forceinline__ int graph_entry(const int* __restrict__ old_idx, int 
 }
 
 constexpr int kMergeChunk = 16;
+// up to this many candidates of a point are evaluated without a look at their codes
+constexpr int kFewCandidates = 32;
 // 16-byte pieces of a candidate's row a lane requests from the tile together (exact_batch): 16 dimensions per wait for
 // LDS.  (Measured: 1M x 256 pass 26.2 -> 24.8 ms, 70k x 784 pass 26.2 -> 25.0 ms; eight pieces cost the workgroup
 // kernel its second wavefront per SIMD: 39 ms.)
@@ -373,8 +376,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_merge(const float* __res
                                                                const int* __restrict__ old_idx, int* __restrict__ knn_idx,
                                                                float* __restrict__ knn_dist, int table_size,
                                                                int wave_lds_ints, int dpad, int direct_max,
-                                                               const uint32_t* __restrict__ pass,
-                                                               const uint16_t* __restrict__ bounds,
+                                                               const uint32_t* __restrict__ pass, JoinBounds jb,
                                                                const int* __restrict__ todo_in, int n_in,
                                                                int* __restrict__ todo_out, int* __restrict__ n_out,
                                                                unsigned long long* __restrict__ stat,
@@ -430,8 +432,8 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_merge(const float* __res
     L.queue2 = nullptr;
     L.table = base + tile_ints + dpad;
     L.srow = L.table + table_size;
-    // with bounds: the smallest lower bound seen for the id in the same place of the set (bfloat16 bits), behind the
-    // list of marks
+    const uint16_t* __restrict__ bounds = jb.codes;
+    // with bounds: the code of the id in the same place of the set, behind the list of marks
     int* tbound = bounds ? L.srow + K + table_size / 4 * 3 : nullptr;
     // without the tile: the ranks' working memory, in place of the list of marks or behind the bounds
     if (!TILE) L.rank = reinterpret_cast<double*>(base + dpad + merge_rank_at(table_size, K, bounds != nullptr));
@@ -497,7 +499,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_merge(const float* __res
             if (i < n_marked) {
                 const int e = marked[i];
                 c[u] = old_idx[(size_t)L.srow[e & 255] * K + (e >> 8)];
-                // the join's lower bound of the pair: entry p K + k of the graph, column = slot in the neighbour's row
+                // the join's code of the pair: entry p K + k of the graph, column = slot in the neighbour's row
                 if (bounds) lb[u] = bounds[((size_t)p * K + (e & 255)) * (size_t)KP + (e >> 8)];
             }
         }
@@ -530,41 +532,69 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_merge(const float* __res
     }
     wave_lds_sync();
     int n_exact = 0;                                      // exact distances of this point (wave-uniform)
+    float reach = INFINITY;                               // what the row's last slot will be at most
     auto batch = [&](const int* list, int n) {
         n_exact += n;
-        if (!TILE) exact_direct<SL, true>(L, list, n, points, D, vec_ok, row);
-        else exact_batch<SL, kMergeChunk, true, kChainGroup, true>(L, list, n, points, D, vec_ok, row);    // two steps of gathers in flight
+        if (!TILE) exact_direct<SL, true>(L, list, n, points, D, vec_ok, row, reach);
+        else exact_batch<SL, kMergeChunk, true, kChainGroup, true>(L, list, n, points, D, vec_ok, row, reach);    // two steps of gathers in flight
     };
-    if (tbound == nullptr || U <= 64) {
+    if (tbound == nullptr || U <= kFewCandidates) {
         for (int off = 0; off < U; off += 64) {
             wave_lds_sync();
             batch(L.table + off, min(64, U - off));
         }
     } else {
-        // Nearer bounds first: a round takes the candidates that are left, whose bound is not above the row's last
-        // slot (it shrinks from round to round) and -- while more than a batch of them is left -- not above the
-        // mean of these bounds.  A candidate whose bound is above the last slot cannot enter the row and is never
-        // read.  The ids of a round are gathered in the list of marks, which is no longer needed.  (Taking exactly
-        // the 64 nearest bounds of every round, found by bisection, was measured slower: the bounds of a point take
-        // few distinct values at 16 bits, and the search costs more than the order gains.)
+        // The reach of the row: the smallest upper end of a code at or below which the row and its candidates have K entries.
+        // (The candidates are distinct and not in the row.  Codes of 0 have no upper end.)
+        const CodeReader codes(jb, p);
+        {
+            constexpr int kIn = 4;                        // steps of 64 candidates whose codes stay in registers
+            int cc[kIn], rc[SL];
+#pragma unroll
+            for (int u = 0; u < kIn; ++u) {
+                const int b = 64 * u + lane < U ? tbound[64 * u + lane] : 0;
+                cc[u] = b > 0 ? b : kCodeTop;
+            }
+#pragma unroll
+            for (int s = 0; s < SL; ++s) rc[s] = codes.code_of(row.dist[s]);
+            int lo = 1, hi = kCodeTop;
+            while (lo < hi) {
+                const int mid = (lo + hi) >> 1;
+                int n = 0;
+#pragma unroll
+                for (int u = 0; u < kIn; ++u) n += __popcll(ballot64(cc[u] <= mid));
+                for (int t0 = 64 * kIn; t0 < U; t0 += 64) {
+                    const int b = t0 + lane < U ? tbound[t0 + lane] : 0;
+                    n += __popcll(ballot64(b > 0 && b <= mid));
+                }
+#pragma unroll
+                for (int s = 0; s < SL; ++s) n += __popcll(ballot64(rc[s] <= mid));
+                if (n >= K) hi = mid;
+                else lo = mid + 1;
+            }
+            if (lo < kCodeTop) reach = codes.reach(lo);
+        }
+        // What is beyond it is never read.  What is left goes in rounds, nearer bounds first: a round takes the candidates whose bound
+        // is not above the row's last slot (it shrinks from round to round) and -- while more than a batch of them is left -- not above
+        // the mean of these bounds.  The ids of a round are gathered in the list of marks, which is no longer needed.
         constexpr int kDone = 0x7fffffff;
         int* round_ids = marked;
         while (true) {
-            const float tau_now = row.tau;
+            const int last = codes.last_code(fminf(row.tau, reach));
             int n_el = 0, sum = 0;
             for (int t0 = 0; t0 < U; t0 += 64) {
                 const int b = t0 + lane < U ? tbound[t0 + lane] : kDone;
-                const bool el = b != kDone && !(__uint_as_float((uint32_t)b << 16) > tau_now);
+                const bool el = b <= last;
                 n_el += __popcll(ballot64(el));
                 sum += el ? b : 0;
             }
             if (n_el == 0) break;
             sum = wave_sum_i(sum);
-            const int cut = n_el <= 64 ? 0xffff : sum / n_el;           // (the smallest bound is never above the mean)
+            const int cut = n_el <= 64 ? last : min(last, sum / n_el);  // (the smallest bound is never above the mean)
             int n_round = 0;
             for (int t0 = 0; t0 < U; t0 += 64) {
                 const int b = t0 + lane < U ? tbound[t0 + lane] : kDone;
-                const bool take = b != kDone && !(__uint_as_float((uint32_t)b << 16) > tau_now) && b <= cut;
+                const bool take = b <= cut;
                 const uint64_t m = ballot64(take);
                 if (take) {
                     round_ids[n_round + mask_prefix(m)] = L.table[t0 + lane];
@@ -584,122 +614,125 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_merge(const float* __res
 }
 
 // The same for rows so long that the set of one point takes most of the LDS a wavefront could get (K above about 45:
-// a point has up to K^2 marks): one workgroup of four wavefronts per point, and the candidates are taken in the
-// order of their lower bounds.
+// a point has up to K^2 marks): one workgroup of four wavefronts per point.
 //
-// A candidate can only end up in the row if its exact distance is at most the row's last slot at the end, and that
-// slot falls fast once the nearest candidates are in.  In the order of the marks most candidates enter at some
-// moment and are pushed out again later (three quarters of them on 70,000 x 784 rows with K = 90), each at the price
-// of gathering a whole fp32 row.  Here:
-//   1. all threads list the marked (neighbour, slot) pairs of the point together with the lower bound L the join
-//      kept for each (explore_join.hip; 0 when it kept none), one 32-bit word per pair;
-//   2. every wavefront walks its quarter of the list in rounds with a rising limit: the smallest limit that takes 64
-//      marks it has not taken yet (found by bisection on the 16 bits of the bounds), never above the shared last
-//      slot -- near candidates first, without sorting anything.  A pair whose bound is above the shared last slot at
-//      its turn is never looked at.  The others have their id read, pass through a hash set (seeded with the row;
-//      drops repeats -- only a saving: a repeated candidate would be rejected by the row), get the exact distance,
-//      64 at a time and what is left at the end of the round, and are merged into the wavefront's copy of the row.
-//      Between the rounds the wavefronts work out what the last slot of their four rows taken together would be
-//      (shared_last_slot below, no merge needed), which is the limit nobody goes beyond: measured on 70,000 x 784 rows
-//      with K = 90, 184 exact distances per point instead of 544 with a limit from each wavefront's own row, for the
-//      85 entries of a row that change;
-//   3. the four rows become one in two steps (2 -> 0 and 3 -> 1, then 1 -> 0), entries above that limit left out,
-//      and the first wavefront stores the result.
-// A bound is below the exact distance of its pair, the shared last slot is never below the final one: a dropped
+// A candidate can only end up in the row if its exact distance is at most the row's last slot at the end, and every exact distance is
+// a whole fp32 row gathered.  Here:
+//   1. all threads list the marked (neighbour, slot) pairs of the point with the codes the join kept for them (join_bounds.hpp);
+//   2. the ids of the few hundred with the least codes are gathered and pass a hash set (seeded with the row; drops repeats): what is
+//      new goes to the list of candidates;
+//   3. the codes say how far the row will reach at most: K of its entries and candidates lie below (join_bounds.hpp).  Where that is
+//      beyond the codes taken so far, more of them go through 2 (this is rare);
+//   4. the candidates whose bound is not above the reach get the exact distance, the four wavefronts sharing them, at most 256 at a
+//      time and nearer bounds first (mostly that is all of them), and
+//   5. the row and the new distances, as (distance, index) keys in LDS, are merged by counting: a new key's slot is the number of
+//      keys of the row below it (binary search) and of new ones (all of them compared), an old key moves up by the new ones
+//      below it.
+// A bound is below the exact distance of its pair, the reach is never below the row's final last slot: a dropped
 // candidate could not have been in the final row, so the result is the one of any other order.
-// (Sorting the list by the bounds first, a bitonic network over up to 4096 words in LDS, cost more than it saved.)
-// LDS (ints): table[kWgTable] | srow[K] | jrow[K] | xrow[dpad] | marked[cap] | 4 tiles | 3 rows for the exchange | 4 x 128 ids
-// | distances of the row as loaded [K] | distances of the four rows as last shown [4][K].
+// (Measured at 70,000 x 784, K = 90: 2,725 marks of 1,466 distinct points, 97 exact distances per point against 140 by rounds without the
+// reach and 85 entries that change; 12.6 -> 4.8 ms = 4.6 TB/s of rows.  Of the first form's 188 k cycles per point 50 k were the exact
+// distances, 48 k the merge of four rows by insertions, 29 k the set of all marks.  Where marks are many and points few (122,376
+// x 4 in 64 clusters, K = 84) the exploration takes a seventh.)
+// LDS (ints): set[set_size] | marked[cap], later 4 tiles | ids of the candidates [most] | their codes [most / 2] | srow[K] |
+// xrow[dpad] | keys: row [K], merged row [K], new [256] | ids of the new ones [256].
 constexpr int kWgChunk = 32;
 constexpr int kWgTile = 64 * (kWgChunk + 4);
-constexpr int kWgTable = 2048;              // hash set; when three quarters are taken, new ids are no longer recorded
 constexpr int kWgMinCap = 1024;             // the kernel is not used when fewer marks than this would fit
+constexpr int kWgMaxCap = 6656;             // marks per point
+constexpr int kWgMost = 1536;               // candidates per point
+constexpr int kWgMaxSteps = kWgMost / 256;  // of them per thread
+constexpr int kWgLeast = 512;               // the kernel is not used when the set has room for fewer
+constexpr int kWgGather = 12;               // marks of a thread whose ids are requested together
+constexpr int kWgNew = 256;                 // exact distances of a round
+static_assert(32 * (2 * kWgChunk + 4) <= kWgTile, "32 rows of twice the dimensions fit the tile");
+struct WgSizes { int cap, most, set_size; };
 
-constexpr int kWgMaxRounds = 12;            // the last one takes everything that is left below the last slot
-constexpr int kWgMaxCap = 6656;             // marks per point: 26 steps of the walk of a wavefront
-constexpr int kWgMaxSteps = kWgMaxCap / 256;
-
-// distance in slot k of a row (k is the same in all lanes)
-template <int SL>
-__device__ __forceinline__ float row_slot_dist(const KnnRow<SL>& row, int k)
+// Candidates c[] (none where negative) into the set, four probes in flight: which of them are new.
+__device__ __forceinline__ void set_insert4(int* table, int mask, const int (&c)[4], bool (&fresh)[4])
 {
-    float v = INFINITY;
+    uint32_t h[4];
+    int old[4];
 #pragma unroll
-    for (int s = 0; s < SL; ++s)
-        if ((k >> 6) == s) v = read_lane_f(row.dist[s], k & 63);
-    return v;
+    for (int u = 0; u < 4; ++u) {
+        h[u] = hash_id(c[u]) & (uint32_t)mask;
+        old[u] = c[u] >= 0 ? atomicCAS(&table[h[u]], kEmpty, c[u]) : 0;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        fresh[u] = false;
+        if (c[u] < 0) continue;
+        for (int i = 0; i <= mask; ++i) {
+            if (old[u] == kEmpty) { fresh[u] = true; break; }
+            if (old[u] == c[u] || old[u] == -c[u] - 1) break;
+            h[u] = (h[u] + 1) & (uint32_t)mask;
+            old[u] = atomicCAS(&table[h[u]], kEmpty, c[u]);
+        }
+    }
 }
 
 template <int SL>
-__global__ __launch_bounds__(256) void k_explore_merge_wg(const float* __restrict__ points, int N, int D, int K,
+__global__ __launch_bounds__(256, 3) void k_explore_merge_wg(const float* __restrict__ points, int N, int D, int K,
                                                           const int* __restrict__ old_idx, int* __restrict__ knn_idx,
-                                                          float* __restrict__ knn_dist, int cap, int dpad,
-                                                          const uint32_t* __restrict__ pass,
-                                                          const uint16_t* __restrict__ bounds,
+                                                          float* __restrict__ knn_dist, WgSizes sz, int dpad,
+                                                          const uint32_t* __restrict__ pass, JoinBounds jb,
                                                           const int* __restrict__ todo_in, int n_in,
                                                           int* __restrict__ todo_out, int* __restrict__ n_out,
                                                           unsigned long long* __restrict__ stat)
 {
     extern __shared__ __align__(16) int lds_w[];
-    __shared__ int wave_tot[4];
-    __shared__ int n_set_s;
-    __shared__ uint32_t tau_s;                                    // bits of the smallest last slot reached so far
+    __shared__ int wave_tot[4], count_s[2][4];
+    __shared__ int n_cand_s, n_new_s;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     // (the list of points a launch before this one left over is in the order in which that launch came to them)
     const int slot = die_local_place(blockIdx.x, gridDim.x);
     if (slot >= (todo_in ? n_in : N)) return;
     const int p = todo_in ? todo_in[slot] : slot;
-    const int MW = (K + 31) >> 5, KP = MW * 32;
+    const int MW = (K + 31) >> 5, KP = MW * 32, kq = (K + 3) & ~3;
     int* table = lds_w;
-    int* srow = table + kWgTable;
-    int* jrow = srow + ((K + 3) & ~3);                            // number of graph entry (p, k), -1 without a valid neighbour
-    float* xrow = reinterpret_cast<float*>(jrow + ((K + 3) & ~3));
-    uint32_t* marked = reinterpret_cast<uint32_t*>(xrow + dpad);
-    int* tiles = reinterpret_cast<int*>(marked + cap);
-    int* xch = tiles + 4 * kWgTile;                               // rows on their way to another wavefront: [3][idx | dist][64 SL]
-    int* ids = xch + 6 * 64 * SL + 128 * wave;                    // this wavefront's candidates: a batch and what is left over
-    const int kq = (K + 3) & ~3;
-    float* old_d = reinterpret_cast<float*>(xch + 6 * 64 * SL + 4 * 128);  // distances of the row as it was loaded
-    float* seen_d = old_d + kq;                                   // [4][kq]: the rows of the wavefronts as they last showed them
+    uint32_t* marked = reinterpret_cast<uint32_t*>(table + sz.set_size);
+    int* tiles = lds_w;                                           // (in the place of the set and the marks)
+    int* cand = lds_w + max(sz.set_size + sz.cap, 4 * kWgTile);
+    uint16_t* cand_code = reinterpret_cast<uint16_t*>(cand + sz.most);
+    int* srow = cand + sz.most + sz.most / 2;
+    float* xrow = reinterpret_cast<float*>(srow + kq);
+    double* row_key = reinterpret_cast<double*>(xrow + dpad);     // the row, sorted
+    double* out_key = row_key + kq;
+    double* new_key = out_key + kq;
+    int* new_id = reinterpret_cast<int*>(new_key + kWgNew);
     const bool vec_ok = (D & 3) == 0 && ((reinterpret_cast<uintptr_t>(points) & 15) == 0);
 
-    // thread k takes neighbour k (K <= 256): its entry of the snapshot and its mark words are requested together with
-    // the point's row and coordinates (none of these addresses depends on another's data)
-    const int k = threadIdx.x;
-    const size_t entry = (size_t)p * K + (k < K ? k : 0);
-    const int q_own = old_idx[entry];
-    uint32_t pw[8];                                               // MW <= 8
+    // The mark words of the point (K MW of them in one piece) are dealt out to the threads; they are requested together with the
+    // entries of the snapshot they belong to and with the point's row and coordinates (none of these addresses depends on another's data).
+    const int words = K * MW, per_mw = 65536 / MW + 1;            // (word / MW, exact below 2048)
+    uint32_t pw[8];                                               // K MW <= 2048
+    int pq[8];
 #pragma unroll
-    for (int w = 0; w < 8; ++w) pw[w] = w < MW ? pass[entry * MW + w] : 0u;
+    for (int j = 0; j < 8; ++j) {
+        const int t = (int)threadIdx.x + 256 * j;
+        pw[j] = t < words ? pass[(size_t)p * words + t] : 0u;
+        pq[j] = t < words ? old_idx[(size_t)p * K + ((t * per_mw) >> 16)] : -1;
+    }
     KnnRow<SL> row;
     row.load(knn_idx + (size_t)p * K, knn_dist + (size_t)p * K, K);
     const float* xp = points + (size_t)p * D;
     for (int d = threadIdx.x; d < dpad; d += 256) xrow[d] = d < D ? xp[d] : 0.0f;
-    for (int i = threadIdx.x; i < kWgTable; i += 256) table[i] = kEmpty;
+    for (int i = threadIdx.x; i < sz.set_size; i += 256) table[i] = kEmpty;
+    int* hist = new_id;                                           // marks by the upper 8 bits of their codes
+    hist[threadIdx.x] = 0;
 
     // ---- 1. the marked pairs of the point
-    const int j = k < K && q_own >= 0 && q_own < N ? (int)entry : -1;     // (the join writes nothing for other entries)
-    if (k < K) {
-        srow[k] = q_own;
-        jrow[k] = j;
-    }
-#pragma unroll
-    for (int s = 0; s < SL; ++s) {
-        if (lane + 64 * s < K) {
-            seen_d[wave * kq + lane + 64 * s] = row.dist[s];      // every wavefront starts from the same sorted row
-            if (wave == 0) old_d[lane + 64 * s] = row.dist[s];
-        }
-    }
     int mine = 0;
-    if (j >= 0) {
 #pragma unroll
-        for (int w = 0; w < 8; ++w) mine += __popc(pw[w]);
+    for (int j = 0; j < 8; ++j) {
+        if (!(pq[j] >= 0 && pq[j] < N)) pw[j] = 0u;               // (the join writes nothing for such entries)
+        mine += __popc(pw[j]);
     }
     const int in_wave = wave_excl_scan_i(mine);
     if (lane == 63) wave_tot[wave] = in_wave + mine;
     if (threadIdx.x == 0) {
-        n_set_s = 0;
-        tau_s = __float_as_uint(row.tau);
+        n_cand_s = 0;
+        n_new_s = 0;
     }
     __syncthreads();
     int at = in_wave, n_marked = 0;
@@ -709,264 +742,304 @@ __global__ __launch_bounds__(256) void k_explore_merge_wg(const float* __restric
         n_marked += wave_tot[w];
     }
     if (n_marked == 0) return;
-    if (n_marked > cap) {
+    if (n_marked > sz.cap) {
         if (threadIdx.x == 0) todo_out[atomicAdd(n_out, 1)] = p;
         return;
     }
-    if (j >= 0) {
 #pragma unroll
-        for (int w = 0; w < 8; ++w) {
-            uint32_t m = pw[w];
-            while (m) {
-                const int b = __ffs(m) - 1;
-                m &= m - 1;
-                marked[at++] = (uint32_t)((32 * w + b) << 8) | (uint32_t)k;
-            }
+    for (int j = 0; j < 8; ++j) {
+        const int t = (int)threadIdx.x + 256 * j;
+        if (256 * j >= words) break;
+        const int k = (t * per_mw) >> 16, w = t - k * MW;
+        if (pw[j]) srow[k] = pq[j];                               // (the same value for every word of the entry)
+        uint32_t m = pw[j];
+        while (m) {
+            const int b = __ffs(m) - 1;
+            m &= m - 1;
+            marked[at++] = (uint32_t)((32 * w + b) << 8) | (uint32_t)k;
         }
     }
-    if (wave == 0) {                                              // seeds: ids that are in the row already
-        const int mask = kWgTable - 1;
-        int seeded = 0;
+    const int mask = sz.set_size - 1;
+    if (wave == 3) {                                              // seeds: the point, and ids that are in the row already
+        if (lane == 0) set_insert(table, mask, p, true);
 #pragma unroll
-        for (int s = 0; s < SL; ++s)
-            if (row.idx[s] >= 0) { set_insert(table, mask, row.idx[s], true); ++seeded; }
-        seeded = wave_sum_i(seeded);
-        if (lane == 0) atomicAdd(&n_set_s, seeded);
+        for (int s = 0; s < SL; ++s) {
+            if (row.idx[s] >= 0) set_insert(table, mask, row.idx[s], true);
+            if (lane + 64 * s < K) row_key[lane + 64 * s] = pair_key(row.dist[s], row.idx[s]);
+        }
     }
     __syncthreads();
-    if (bounds) {
-        // the bounds of the listed pairs, by all threads (a thread's own marks one after the other would wait for
-        // one 2-byte read at a time)
-        for (int i0 = threadIdx.x; i0 < n_marked; i0 += 4 * 256) {
-            uint32_t e[4], lb[4];
+    const uint16_t* __restrict__ codes_p = jb.codes ? jb.codes + (size_t)p * K * KP : nullptr;
+    if (codes_p) {
+        for (int i0 = threadIdx.x; i0 < n_marked; i0 += kWgGather * 256) {
+            uint32_t e[kWgGather], code[kWgGather];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int i = i0 + 256 * u;
-                e[u] = i < n_marked ? marked[i] : 0u;
-                lb[u] = i < n_marked ? (uint32_t)bounds[(size_t)jrow[e[u] & 255u] * KP + ((e[u] >> 8) & 255u)] : 0u;
+            for (int u = 0; u < kWgGather; ++u) {
+                e[u] = i0 + 256 * u < n_marked ? marked[i0 + 256 * u] : 0u;
+                code[u] = i0 + 256 * u < n_marked ? codes_p[(e[u] & 255u) * KP + (e[u] >> 8)] : 0u;
             }
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
-                if (i0 + 256 * u < n_marked) marked[i0 + 256 * u] = e[u] | (lb[u] << 16);
+            for (int u = 0; u < kWgGather; ++u) {
+                if (i0 + 256 * u < n_marked) {
+                    marked[i0 + 256 * u] = e[u] | code[u] << 16;
+                    atomicAdd(&hist[code[u] >> 8], 1);
+                }
+            }
         }
         __syncthreads();
     }
 
-    // ---- 2. my quarter of the list, nearer bounds first
-    ExploreLds L;
-    L.tile = reinterpret_cast<float*>(tiles + wave * kWgTile);
-    L.xrow = xrow;
-    L.queue2 = nullptr;
-    L.table = nullptr;
-    L.srow = nullptr;
-    int have = 0;                                                 // candidates waiting in ids (wave-uniform)
-    int n_exact = 0;                                              // exact distances this wavefront asked for
-    auto run_batch = [&]() {
-        wave_lds_sync();
-        const int n_now = min(64, have);
-        n_exact += n_now;
-        const float cap_now = __uint_as_float(*reinterpret_cast<volatile uint32_t*>(&tau_s));
-        exact_batch<SL, kWgChunk, true, kChainGroup, true>(L, ids, n_now, points, D, vec_ok, row, cap_now);
-        if (lane == 0) atomicMin(&tau_s, __float_as_uint(row.tau));   // non-negative floats order like their bits
-        have -= n_now;
-        const int left = lane < have ? ids[64 + lane] : 0;        // the candidates beyond the batch move to the front
-        wave_lds_sync();
-        if (lane < have) ids[lane] = left;
-    };
-    // The last slot of the four rows taken together, without merging them.  The wavefronts evaluate disjoint sets of
-    // new candidates (the hash set, as long as it records), none of them in the row as loaded, so for any t the
-    // candidates and old entries at a distance <= t number at least sum_w c_w(t) - 3 o(t), with c_w(t) the entries
-    // <= t of the row of wavefront w and o(t) those of the row as loaded (a row holds every old entry below its own
-    // last slot, and what it dropped is above it).  The smallest t among this wavefront's own entries for which
-    // that number reaches K is at least the last slot of the final row.  Rows of the other wavefronts are read as
-    // they were last shown, possibly half-way through being shown again: entries only fall, the search only moves
-    // past an entry it has seen to be <= t, so a stale or mixed row gives a smaller count and a larger t.
-    auto shared_last_slot = [&]() {
+    const CodeReader codes(jb, p);
+    float tau = row.tau;                                          // the last slot, as far as it is known
+    int rc[SL];
 #pragma unroll
-        for (int s = 0; s < SL; ++s)
-            if (lane + 64 * s < K) seen_d[wave * kq + lane + 64 * s] = row.dist[s];
-        wave_lds_sync();
-        int top = 1;
-        while (2 * top <= K) top *= 2;
-        // the searches of a lane (its SL entries in the three other rows and in the row as loaded) advance together:
-        // their reads do not wait for each other
-        int pos[SL][4];
-#pragma unroll
-        for (int s = 0; s < SL; ++s)
-#pragma unroll
-            for (int w = 0; w < 4; ++w) pos[s][w] = 0;
-        const volatile float* arr[4];
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            const int other = w + (w >= wave ? 1 : 0);            // 0..3 without this wavefront, then 4 = the row as loaded
-            arr[w] = other < 4 ? seen_d + other * kq : old_d;
-        }
-        for (int b = top; b > 0; b >>= 1) {
-#pragma unroll
-            for (int s = 0; s < SL; ++s) {
-                const float t = row.dist[s];
-#pragma unroll
-                for (int w = 0; w < 4; ++w) {
-                    const int np = pos[s][w] + b;
-                    if (np <= K && arr[w][np - 1] <= t) pos[s][w] = np;
-                }
-            }
-        }
-        float best = INFINITY;
-#pragma unroll
-        for (int s = 0; s < SL; ++s) {
-            const int slot = lane + 64 * s;
-            const float t = row.dist[s];
-            // (arr[0..2]: the other wavefronts, arr[3]: the row as loaded)
-            const int total = slot + 1 + pos[s][0] + pos[s][1] + pos[s][2] - 3 * pos[s][3];
-            const uint64_t okm = ballot64(slot < K && t < INFINITY && total >= K);
-            if (okm != 0 && best == INFINITY) best = read_lane_f(t, first_lane(okm));   // rows are sorted: the first is the smallest
-        }
-        // (read after the rows: once the set no longer records, two wavefronts may hold the same candidate)
-        const bool recording = *reinterpret_cast<volatile int*>(&n_set_s) < kWgTable / 4 * 3;
-        if (recording && lane == 0 && best < INFINITY) atomicMin(&tau_s, __float_as_uint(best));
-    };
-    // the bounds of this wavefront's marks (upper 16 bits of the fp32 number; non-negative floats order like their bits)
-    int lb16[kWgMaxSteps];
-#pragma unroll
-    for (int u = 0; u < kWgMaxSteps; ++u) {
-        const int at = 64 * wave + 256 * u + lane;
-        lb16[u] = at < n_marked ? (int)(marked[at] >> 16) : 0x7fffffff;
-    }
-    auto marks_upto = [&](int from, int upto) {                   // marks with from < bound <= upto
+    for (int s = 0; s < SL; ++s) rc[s] = codes.code_of(row.dist[s]);
+    int lb16[kWgMaxSteps];                                        // the codes of this thread's candidates: threadIdx.x + 256 u
+    int it = 0, n_cand = 0;
+    auto count_upto = [&](int from, int upto) {                   // candidates of the workgroup with from < code <= upto
         int n = 0;
 #pragma unroll
         for (int u = 0; u < kWgMaxSteps; ++u) {
-            if (64 * wave + 256 * u >= n_marked) break;
+            if (256 * u >= n_cand) break;
             n += __popcll(ballot64(lb16[u] > from && lb16[u] <= upto));
         }
-        return n;
+        ++it;
+        if (lane == 0) count_s[it & 1][wave] = n;
+        __syncthreads();
+        return count_s[it & 1][0] + count_s[it & 1][1] + count_s[it & 1][2] + count_s[it & 1][3];
     };
-    int least = 0x7fffffff;                                       // the smallest bound of this wavefront's marks
-#pragma unroll
-    for (int u = 0; u < kWgMaxSteps; ++u) least = min(least, lb16[u]);
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) least = min(least, __shfl_xor(least, o, 64));
-    int prev = -1;                                                // bounds up to here have been taken
-    bool rows_moved = false;                                      // a batch has run since the last slots were compared
-    for (int r = 0; r < kWgMaxRounds; ++r) {
-        if (rows_moved) {
-            shared_last_slot();
-            rows_moved = false;
+    int cut = -1;                                                 // marks with codes up to here have become candidates
+    for (int want = 6 * K;; want *= 2) {
+        // the codes that take at least `want` marks, in steps of 256
+        const int from = cut;
+        cut = kCodeTop;
+        if (codes_p && n_marked > want) {
+            int run = 0, bins = 0;
+            for (int b0 = 0; b0 < 256; b0 += 64) {
+                const int h = hist[b0 + lane];
+                const uint64_t below = ballot64(run + wave_excl_scan_i(h) + h < want);     // (a prefix of the bins)
+                bins += __popcll(below);
+                if (below != ~0ull) break;
+                run += wave_sum_i(h);
+            }
+            cut = max(from, 256 * bins + 255);
         }
-        const int lim = (int)(*reinterpret_cast<volatile uint32_t*>(&tau_s) >> 16);   // bound <= last slot iff its 16 bits <= lim
-        if (lim <= prev) break;
-        // the smallest limit that takes a batch; everything up to the last slot when that is less (or in the last round)
-        int lo = max(prev + 1, min(least, lim)), hi = lim;
-        if (r + 1 < kWgMaxRounds) {
-            while (lo < hi) {
-                const int mid = (lo + hi) >> 1;
-                if (marks_upto(prev, mid) >= 64 - have) hi = mid;
+
+        // ---- 2. the distinct ones
+        for (int i0 = threadIdx.x; i0 < n_marked; i0 += kWgGather * 256) {
+            int c[kWgGather], code[kWgGather];
+#pragma unroll
+            for (int u = 0; u < kWgGather; ++u) {
+                c[u] = -1;
+                code[u] = 0;
+                if (i0 + 256 * u < n_marked) {
+                    const uint32_t e = marked[i0 + 256 * u];
+                    code[u] = (int)(e >> 16);
+                    if (code[u] > from && code[u] <= cut) c[u] = old_idx[(size_t)srow[e & 255u] * K + ((e >> 8) & 255u)];
+                }
+                if (c[u] >= N) c[u] = -1;
+            }
+            for (int g = 0; g < kWgGather; g += 4) {
+                if (i0 - (int)threadIdx.x + 256 * g >= n_marked) break;
+                if (*reinterpret_cast<volatile int*>(&n_cand_s) > sz.most) break;
+                int c4[4], code4[4];
+                bool fresh[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    c4[u] = g == 0 ? c[u] : (g == 4 ? c[u + 4] : c[u + 8]);
+                    code4[u] = g == 0 ? code[u] : (g == 4 ? code[u + 4] : code[u + 8]);
+                }
+                set_insert4(table, mask, c4, fresh);
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const uint64_t fm = ballot64(fresh[u]);
+                    if (fm == 0) continue;
+                    int first = 0;
+                    if (lane == 0) first = atomicAdd(&n_cand_s, __popcll(fm));
+                    first = __builtin_amdgcn_readfirstlane(first) + mask_prefix(fm);
+                    if (fresh[u] && first < sz.most) {
+                        cand[first] = c4[u];
+                        cand_code[first] = (uint16_t)code4[u];
+                    }
+                }
+            }
+        }
+        __syncthreads();
+        n_cand = n_cand_s;
+        if (n_cand > sz.most) {                                   // too many that may matter
+            if (threadIdx.x == 0) todo_out[atomicAdd(n_out, 1)] = p;
+            return;
+        }
+
+        // ---- 3. how far the row reaches (every wavefront for itself: no barriers)
+        if (codes_p) {
+            constexpr int kIn = kWgMost / 64;
+            int lo = 1, hi = kCodeTop;
+            if (n_cand <= 64 * (kIn / 2)) {
+                int cc[kIn / 2];
+#pragma unroll
+                for (int u = 0; u < kIn / 2; ++u) {
+                    const int b = 64 * u + lane < n_cand ? (int)cand_code[64 * u + lane] : 0;
+                    cc[u] = b > 0 ? b : kCodeTop;
+                }
+                while (lo < hi) {
+                    const int mid = (lo + hi) >> 1;
+                    int n = 0;
+#pragma unroll
+                    for (int u = 0; u < kIn / 2; ++u) {
+                        if (64 * u >= n_cand) break;
+                        n += __popcll(ballot64(cc[u] <= mid));
+                    }
+#pragma unroll
+                    for (int s = 0; s < SL; ++s) n += __popcll(ballot64(rc[s] <= mid));
+                    if (n >= K) hi = mid;
+                    else lo = mid + 1;
+                }
+            } else {
+                while (lo < hi) {
+                    const int mid = (lo + hi) >> 1;
+                    int n = 0;
+                    for (int t0 = 0; t0 < n_cand; t0 += 64) {
+                        const int b = t0 + lane < n_cand ? (int)cand_code[t0 + lane] : 0;
+                        n += __popcll(ballot64(b > 0 && b <= mid));
+                    }
+#pragma unroll
+                    for (int s = 0; s < SL; ++s) n += __popcll(ballot64(rc[s] <= mid));
+                    if (n >= K) hi = mid;
+                    else lo = mid + 1;
+                }
+            }
+            if (lo < kCodeTop) tau = fminf(tau, codes.reach(lo));
+        }
+        if (cut >= kCodeTop || codes.last_code(tau) <= cut) break;
+        __syncthreads();                                          // (n_cand_s has been read)
+    }
+    if (n_cand == 0) return;
+#pragma unroll
+    for (int u = 0; u < kWgMaxSteps; ++u) {
+        const int i = threadIdx.x + 256 * u;
+        lb16[u] = i < n_cand ? (int)cand_code[i] : 0x7fffffff;
+    }
+
+    // ---- 4. the exact distances of a round
+    float* tile = reinterpret_cast<float*>(tiles + wave * kWgTile);
+    const int k = threadIdx.x;                                    // (the slot of the row and the new key this thread places)
+    bool changed = false;
+    int n_exact = 0;
+    while (true) {
+        const int last = codes_p ? codes.last_code(tau) : kCodeTop;
+        const int n_left = count_upto(-1, last);                  // (a barrier: the set, and the keys of the round before, have been read)
+        if (n_left == 0) break;
+        int upto = last;
+        if (n_left > kWgNew) {
+            // the least codes of them (equal codes: any of them)
+            int lo = 0;
+            while (lo < upto) {
+                const int mid = (lo + upto) >> 1;
+                if (count_upto(-1, mid) >= kWgNew / 4 * 3) upto = mid;
                 else lo = mid + 1;
             }
-        } else {
-            lo = lim;
-        }
-        const int upto = lo;
-        // first the ids of everything this round takes (all reads travel together), then the candidates one step
-        // of the walk after the other
-        int c[kWgMaxSteps];
-#pragma unroll
-        for (int u = 0; u < kWgMaxSteps; ++u) {
-            const int at = 64 * wave + 256 * u + lane;
-            c[u] = -1;
-            if (lb16[u] > prev && lb16[u] <= upto) {              // (false beyond the list)
-                const uint32_t e = marked[at];
-                c[u] = old_idx[(size_t)srow[e & 255u] * K + ((e >> 8) & 255u)];
-            }
         }
 #pragma unroll
         for (int u = 0; u < kWgMaxSteps; ++u) {
-            if (64 * wave + 256 * u >= n_marked) break;
-            bool fresh = c[u] >= 0 && c[u] < N && c[u] != p;
-            if (ballot64(fresh) == 0) continue;
-            // the shared last slot may have fallen since the ids were requested
-            const float tau_now = __uint_as_float(*reinterpret_cast<volatile uint32_t*>(&tau_s));
-            if (fresh && __uint_as_float((uint32_t)lb16[u] << 16) > tau_now) fresh = false;
-            if (fresh && *reinterpret_cast<volatile int*>(&n_set_s) < kWgTable / 4 * 3) {
-                fresh = set_insert(table, kWgTable - 1, c[u], false);
-                if (fresh) atomicAdd(&n_set_s, 1);
-            }
-            const uint64_t fm = ballot64(fresh);
-            if (fresh) ids[have + mask_prefix(fm)] = c[u];        // have < 64 here: at most 127 entries
-            have += __popcll(fm);
-            if (have >= 64) {
-                run_batch();
-                rows_moved = true;
+            if (256 * u >= n_cand) break;
+            const bool take = lb16[u] <= upto;
+            const uint64_t m = ballot64(take);
+            if (m == 0) continue;
+            int first = 0;
+            if (lane == 0) first = atomicAdd(&n_new_s, __popcll(m));
+            first = __builtin_amdgcn_readfirstlane(first) + mask_prefix(m);
+            if (take && first < kWgNew) {
+                new_id[first] = cand[threadIdx.x + 256 * u];
+                lb16[u] = 0x7fffffff;
             }
         }
-        prev = upto;
-        if (have > 0) {                                           // the next round's limit comes from the rows
-            run_batch();
-            rows_moved = true;
+        __syncthreads();
+        const int n = min(kWgNew, n_new_s);
+        const int share = (n + 3) >> 2, own = min(wave * share, n), n_own = min(share, n - own);      // at most 64
+        if (n_own > 0) {
+            float d;
+            bool finished;
+            if (share <= 32) finished = exact_distances<2 * kWgChunk, 32, true, kChainGroup>(tile, xrow, new_id + own, n_own, points, D, vec_ok, tau, d);
+            else finished = exact_distances<kWgChunk, 64, true, kChainGroup>(tile, xrow, new_id + own, n_own, points, D, vec_ok, tau, d);
+            // (what cannot enter: a key above all others)
+            if (lane < n_own) new_key[own + lane] = finished && d < INFINITY ? pair_key(d, new_id[own + lane]) : INFINITY;
+            n_exact += n_own;
+        }
+        if (threadIdx.x == 0 && (n & 1)) new_key[n] = INFINITY;   // (read in twos)
+        __syncthreads();
+        if (threadIdx.x == 0) n_new_s = 0;
+        // ---- 5. the row and the new keys (pairs are distinct, but for empty slots of the row)
+        const double mine_old = k < K ? row_key[k] : INFINITY, mine_new = k < n ? new_key[k] : INFINITY;
+        int rank_old = k, rank_new = 0;
+        for (int step = 256; step > 0; step >>= 1)
+            if (rank_new + step <= K && row_key[rank_new + step - 1] < mine_new) rank_new += step;
+        for (int i = 0; i < n; i += 2) {
+            const double2 v = *reinterpret_cast<const double2*>(new_key + i);
+            rank_old += v.x < mine_old ? 1 : 0;
+            rank_old += v.y < mine_old ? 1 : 0;
+            rank_new += v.x < mine_new ? 1 : 0;
+            rank_new += v.y < mine_new ? 1 : 0;
+        }
+        const bool enters = k < n && mine_new < INFINITY && rank_new < K;
+        if (k < K && rank_old < K) out_key[rank_old] = mine_old;
+        if (enters) out_key[rank_new] = mine_new;
+        const uint64_t em = ballot64(enters);
+        ++it;
+        if (lane == 0) count_s[it & 1][wave] = em != 0;
+        __syncthreads();
+        if (count_s[it & 1][0] | count_s[it & 1][1] | count_s[it & 1][2] | count_s[it & 1][3]) {
+            changed = true;
+            double* t = row_key;
+            row_key = out_key;
+            out_key = t;
+            tau = fminf(tau, pair_dist(row_key[K - 1]));
         }
     }
-    if (have > 0) run_batch();
     count_exact(stat, n_exact);
-
-    // ---- 3. one row out of four: wavefronts 0 and 1 take the rows of 2 and 3, then 0 takes the row of 1
-    float tau_all = INFINITY;
-    auto put_row = [&](int at) {
-#pragma unroll
-        for (int s = 0; s < SL; ++s) {
-            xch[(at * 2 + 0) * (64 * SL) + lane + 64 * s] = row.idx[s];
-            xch[(at * 2 + 1) * (64 * SL) + lane + 64 * s] = __float_as_int(row.dist[s]);
-        }
-    };
-    auto take_row = [&](int at) {
-#pragma unroll
-        for (int s = 0; s < SL; ++s) {
-            const int c = xch[(at * 2 + 0) * (64 * SL) + lane + 64 * s];
-            const float d = __int_as_float(xch[(at * 2 + 1) * (64 * SL) + lane + 64 * s]);
-            row.merge(lane + 64 * s < K && c >= 0 && d <= tau_all, c, d);
-        }
-    };
-    // The last slot of the four rows together, once more with all batches done: entries above it (most of what the
-    // rows still share with the row as loaded) need not be offered to the row that takes them.
-    __syncthreads();
-    shared_last_slot();
-    __syncthreads();
-    tau_all = __uint_as_float(tau_s);
-    if (wave >= 2) put_row(wave - 2);
-    __syncthreads();
-    if (wave < 2) take_row(wave);
-    if (wave == 1) put_row(2);
-    __syncthreads();
-    if (wave == 0) {
-        take_row(2);
-        if (row.changed) row.store(knn_idx + (size_t)p * K, knn_dist + (size_t)p * K);
+    if (changed && k < K) {
+        const double v = row_key[k];
+        knn_idx[(size_t)p * K + k] = __double2loint(v);
+        knn_dist[(size_t)p * K + k] = pair_dist(v);
     }
 }
 
-// marks per point the workgroup-per-point merge can take with the LDS of a compute unit shared by two workgroups
-int merge_wg_cap(int dpad, int K, int sl)
+// Sizes of the workgroup-per-point merge with the LDS of a compute unit shared by two workgroups; no marks (cap) at all where it does
+// not fit.
+int merge_wg_ints(const WgSizes& sz, int dpad, int K, int sl)
 {
-    const int budget = 78 * 1024 / 4;
-    const int fixed = kWgTable + 2 * ((K + 3) & ~3) + dpad + 4 * kWgTile + 6 * 64 * sl + 4 * 128 + 5 * ((K + 3) & ~3);
-    return std::min(std::min(budget - fixed, K * K), kWgMaxCap);
+    return (std::max(sz.set_size + sz.cap, 4 * kWgTile) + sz.most + sz.most / 2 + dpad + 5 * ((K + 3) & ~3) + 3 * kWgNew + 3) / 4 * 4;
 }
 
-int merge_wg_ints(int cap, int dpad, int K, int sl)
+WgSizes merge_wg_sizes(int dpad, int K, int sl)
 {
-    return (kWgTable + 2 * ((K + 3) & ~3) + dpad + cap + 4 * kWgTile + 6 * 64 * sl + 4 * 128 + 5 * ((K + 3) & ~3) + 3) / 4 * 4;
+    // three workgroups per compute unit where that leaves room for kWgMaxCap marks, else two
+    for (int share = 3; share >= 2; --share) {
+        const int budget = (160 * 1024 / share - 1024) / 4;
+        for (int set = 2048; set >= 1024; set >>= 1) {
+            WgSizes sz;
+            sz.set_size = set;
+            sz.most = std::min(kWgMost, (set / 8 * 7 - K - 1) & ~7);
+            if (sz.most < kWgLeast) continue;
+            sz.cap = std::min({budget - merge_wg_ints({0, sz.most, set}, dpad, K, sl) + std::max(0, 4 * kWgTile - set), K * K + 3, kWgMaxCap}) & ~3;
+            const int enough = share == 3 ? std::min((K * K + 3) & ~3, kWgMaxCap) : kWgMinCap;
+            if (sz.cap >= enough && sz.cap >= kWgMinCap && merge_wg_ints(sz, dpad, K, sl) <= budget) return sz;
+        }
+    }
+    return {0, 0, 0};
 }
 
 template <int SL>
-int launch_merge_wg(const float* points, int N, int D, int K, const int* old_idx, int* knn_idx, float* knn_dist, int cap,
-                    int dpad, const uint32_t* pass, const uint16_t* bounds, const int* todo_in, int n_in,
+int launch_merge_wg(const float* points, int N, int D, int K, const int* old_idx, int* knn_idx, float* knn_dist,
+                    const WgSizes& sz, int dpad, const uint32_t* pass, const JoinBounds& bounds, const int* todo_in, int n_in,
                     int* todo_out, int* n_out, unsigned long long* stat, hipStream_t stream)
 {
-    const size_t lds = (size_t)merge_wg_ints(cap, dpad, K, SL) * sizeof(int);
+    const size_t lds = (size_t)merge_wg_ints(sz, dpad, K, SL) * sizeof(int);
     RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_explore_merge_wg<SL>),
                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     const int n_work = todo_in ? n_in : N;
     hipLaunchKernelGGL((k_explore_merge_wg<SL>), dim3(grid_for_dies((size_t)n_work)), dim3(256), lds, stream, points, N, D, K, old_idx,
-                       knn_idx, knn_dist, cap, dpad, pass, bounds, todo_in, n_in, todo_out, n_out, stat);
+                       knn_idx, knn_dist, sz, dpad, pass, bounds, todo_in, n_in, todo_out, n_out, stat);
     RSFK_HIP(hipGetLastError());
     return 0;
 }
@@ -980,7 +1053,7 @@ int next_pow2(int v)
 
 template <int SL, int WAVES>
 int launch_merge(const float* points, int N, int D, int K, const int* old_idx, int* knn_idx, float* knn_dist, int table,
-                 int wave_ints, int dpad, const uint32_t* pass, const uint16_t* bounds, const int* todo_in, int n_in,
+                 int wave_ints, int dpad, const uint32_t* pass, const JoinBounds& bounds, const int* todo_in, int n_in,
                  int* todo_out, int* n_out, unsigned long long* stat, const int* order, hipStream_t stream)
 {
     const size_t lds = (size_t)WAVES * (size_t)wave_ints * sizeof(int);
@@ -1014,10 +1087,10 @@ int merge_wave_ints(int table, int dpad, int K, bool with_bounds = false)
 }
 
 int dispatch_merge(int sl, int waves, const float* points, int N, int D, int K, const int* old_idx, int* knn_idx,
-                   float* knn_dist, int table, int dpad, const uint32_t* pass, const uint16_t* bounds, const int* todo_in,
+                   float* knn_dist, int table, int dpad, const uint32_t* pass, const JoinBounds& bounds, const int* todo_in,
                    int n_in, int* todo_out, int* n_out, unsigned long long* stat, const int* order, hipStream_t stream)
 {
-    const int wi = merge_wave_ints(table, dpad, K, bounds != nullptr);
+    const int wi = merge_wave_ints(table, dpad, K, bounds.codes != nullptr);
 #define RSFK_MERGE_CASE(SLV, WV)                                                                                        \
     if (sl == SLV && waves == WV)                                                                                       \
         return launch_merge<SLV, WV>(points, N, D, K, old_idx, knn_idx, knn_dist, table, wi, dpad, pass, bounds, \
@@ -1072,7 +1145,7 @@ bool explore_merge_uses_bounds(int D, int K)
     const int want = std::max(next_pow2(K * K + K + 2), next_pow2(4 * K + 66));
     int big_waves = 4;
     while (big_waves > 1 && merge_wave_ints(want, dpad, K) > lds_ints / big_waves) big_waves >>= 1;
-    return big_waves < 4 && merge_wg_cap(dpad, K, sl) >= kWgMinCap;
+    return big_waves < 4 && merge_wg_sizes(dpad, K, sl).cap > 0;
 }
 
 
@@ -1134,26 +1207,27 @@ int launch_explore(const float* points, const Bf16Copy* bf, const JoinCopy* jc, 
         int* listB = explore_ws_todo(ws, 1);
         int n_back = 0;
         // (the bounds of the join, when it kept them and the set with a bound per place still fits)
-        const uint16_t* wave_bounds = explore_ws_bounds(ws);
-        if (4 * merge_wave_ints(small_table, dpad, K, true) > lds_ints) wave_bounds = nullptr;
+        JoinBounds wave_bounds = explore_ws_bounds(ws), no_bounds = wave_bounds;
+        no_bounds.codes = nullptr;
+        if (4 * merge_wave_ints(small_table, dpad, K, true) > lds_ints) wave_bounds = no_bounds;
         int big_table = want, big_waves = 4;
         while (big_waves > 1 && merge_wave_ints(big_table, dpad, K) > lds_ints / big_waves) big_waves >>= 1;
         // fewer than four wavefronts per workgroup would leave the compute units nearly empty: such sets get one
         // workgroup per point instead
         const bool per_wg = big_waves < 4;
-        const int wg_cap = merge_wg_cap(dpad, K, sl);
+        const WgSizes wg = merge_wg_sizes(dpad, K, sl);
         if (!per_wg)
             while (big_table > small_table && merge_wave_ints(big_table, dpad, K) > lds_ints / big_waves) big_table >>= 1;
-        const bool second = per_wg ? wg_cap >= kWgMinCap : big_table > small_table;
+        const bool second = per_wg ? wg.cap > 0 : big_table > small_table;
         auto merge_wg = [&](const int* list, int n) {
-            const uint16_t* bounds = explore_ws_bounds(ws);
+            const JoinBounds& bounds = explore_ws_bounds(ws);
             if (sl == 1)
-                return launch_merge_wg<1>(points, N, D, K, old_idx, knn_idx, knn_dist, wg_cap, dpad, pass, bounds, list, n, listB,
+                return launch_merge_wg<1>(points, N, D, K, old_idx, knn_idx, knn_dist, wg, dpad, pass, bounds, list, n, listB,
                                           listB + N, stat, stream);
             if (sl == 2)
-                return launch_merge_wg<2>(points, N, D, K, old_idx, knn_idx, knn_dist, wg_cap, dpad, pass, bounds, list, n, listB,
+                return launch_merge_wg<2>(points, N, D, K, old_idx, knn_idx, knn_dist, wg, dpad, pass, bounds, list, n, listB,
                                           listB + N, stat, stream);
-            return launch_merge_wg<4>(points, N, D, K, old_idx, knn_idx, knn_dist, wg_cap, dpad, pass, bounds, list, n, listB,
+            return launch_merge_wg<4>(points, N, D, K, old_idx, knn_idx, knn_dist, wg, dpad, pass, bounds, list, n, listB,
                                       listB + N, stat, stream);
         };
         // Where the workgroup-per-point kernel may follow, the small set is first tried on a sample (the first points of
@@ -1189,7 +1263,7 @@ int launch_explore(const float* points, const Bf16Copy* bf, const JoinCopy* jc, 
                 rc = 0;
             else if (!per_wg)
                 rc = dispatch_merge(sl, big_waves, points, N, D, K, old_idx, knn_idx, knn_dist, big_table, dpad, pass,
-                                    nullptr, listA, n_todo, listB, listB + N, stat, nullptr, stream);
+                                    no_bounds, listA, n_todo, listB, listB + N, stat, nullptr, stream);
             else
                 rc = merge_wg(listA, n_todo);
             if (rc)

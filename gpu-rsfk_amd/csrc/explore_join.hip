@@ -27,13 +27,14 @@
 // otherwise; no atomics on shared counters, no buffer that can overflow.
 //
 // For the merge kernel that works through a point's candidates in the order of their
-// bounds (explore.hip: rows with many candidates), L itself is kept for every marked
-// pair, rounded down to a bfloat16 number (16 bits per pair of the join).
+// bounds (explore.hip: rows with many candidates), the bound is kept for every marked
+// pair as a 16-bit code (join_bounds.hpp).
 //
 // Steps: R in compressed rows (counting sort of the graph entries by neighbour, see k_bin_count) -> join.
 #include "rsfk_common.hpp"
 #include "wave64.hpp"
 #include "forest.hpp"
+#include "join_bounds.hpp"
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
@@ -57,7 +58,8 @@ struct ExploreWorkspace {
     int* part_off = nullptr;   // n_parts x n_bins: where the entries of a part start inside a bin
     uint32_t* pass = nullptr;  // N*K*MW, indexed by entry number
     float2* recs = nullptr;    // N: norm of a point's row in the copy, and the bar its candidates have to pass (k_join_records)
-    uint16_t* bounds = nullptr; // N*K*32*MW lower bounds of the marked pairs (bfloat16, rounded down), or null
+    JoinBounds view;           // what the merge kernels read (set by launch_explore_join)
+    uint16_t* bounds = nullptr; // N*K*32*MW codes of the marked pairs (join_bounds.hpp), or null
     bool tiled = false;         // the builder of medium graphs: bins of 2^cshift points, rows of 2^fshift of them at a time
     // the builder for large graphs (staged_rev_*): two scatters through LDS instead of one straight to memory
     bool staged = false;
@@ -584,14 +586,38 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_rows(const int2* __restri
 // A sum bar + e_c is at least 1 + 2^-21 times the sum of the values it stands for, which covers the roundings of the sum, its square
 // and the comparison.  1e-30 under the root covers what underflow takes from the chain.  An infinite or NaN last slot makes bar
 // infinite or NaN, a row that is not finite makes d~ - E1 NaN, and a comparison with that drops nothing.
-constexpr float kJoinUp = 1.0f + 1.0f / 1048576.0f;
-__global__ void k_join_records(const float* __restrict__ norms, const float* __restrict__ errs, const float* __restrict__ scale,
-                               const float* __restrict__ knn_dist, int N, int K, float one_minus_gamma, float2* __restrict__ out)
+// The last workgroup has no points: it takes the largest norm and error of any finite row from the parts of them (join_copy.hip).
+__global__ __launch_bounds__(256) void k_join_records(JoinCopy jc, float* __restrict__ scale, const float* __restrict__ knn_dist, int N, int K,
+                                                      float one_minus_gamma, float2* __restrict__ out)
 {
+    if (blockIdx.x + 1 == gridDim.x) {
+        __shared__ float2 part[256];
+        float2 most = make_float2(0.0f, 0.0f);
+#pragma unroll 8
+        for (int i = threadIdx.x; i < jc.n_parts; i += 256) {
+            const float2 v = jc.parts[i];
+            most = make_float2(fmaxf(most.x, v.x), fmaxf(most.y, v.y));
+        }
+        part[threadIdx.x] = most;
+        __syncthreads();
+        for (int o = 128; o > 0; o >>= 1) {
+            if ((int)threadIdx.x < o) {
+                const float2 v = part[threadIdx.x + o];
+                most = make_float2(fmaxf(most.x, v.x), fmaxf(most.y, v.y));
+                part[threadIdx.x] = most;
+            }
+            __syncthreads();
+        }
+        if (threadIdx.x == 0) {
+            scale[1] = most.x;
+            scale[2] = most.y;
+        }
+        return;
+    }
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= N) return;
     const float tau = knn_dist[(size_t)p * K + (K - 1)];
-    out[p] = make_float2(norms[p], (*scale * sqrtf(tau / one_minus_gamma + 1e-30f) + errs[p]) * kJoinUp);
+    out[p] = make_float2(jc.norms[p], (scale[0] * sqrtf(tau / one_minus_gamma + 1e-30f) + jc.errs[p]) * kJoinUp);
 }
 
 // d~ - E1 of a pair, from S = n_p + n_c and the product g of the rows
@@ -607,24 +633,14 @@ __device__ __forceinline__ bool join_may(float least, float bar, float e_c)
     return !(least > w * w);
 }
 
-// The lower bound of the exact distance of a marked pair, as kept for the merge: upper 16 bits, which rounds down.  2^-20 for the
-// square root (one unit) and the roundings here.  A bound below zero (or NaN) says nothing: 0.
-__device__ __forceinline__ uint32_t join_bound16(float least, float e_p, float e_c, float inv_scale, float one_minus_gamma)
-{
-    constexpr float kDown = 1.0f - 1.0f / 1048576.0f;
-    const float t = __builtin_fmaf(__builtin_amdgcn_sqrtf(fmaxf(least, 0.0f)), kDown, -(e_p + e_c) * kJoinUp) * inv_scale;
-    const float lower = __builtin_fmaf(t * t, one_minus_gamma * kDown, -1e-30f);
-    return t > 0.0f && lower > 0.0f ? __float_as_uint(lower) >> 16 : 0u;
-}
-
-// One wavefront per q.  Per-wavefront LDS (ints): cq[KP] | pid[32] | pn[32] | pbar[32] | perr[32] | pe[32], KP = K rounded up to 32.
+// One wavefront per q.  Per-wavefront LDS (ints): cq[KP] | pid[32] | pn[32] | pbar[32] | perr[32] | pper[32] | pe[32], KP = K rounded up to 32.
 // (five wavefronts per SIMD: 1M x 256 8.7 -> 8.2 ms against four, for three spilled registers)
 template <int WAVES, bool BOUNDS>
-__global__ __launch_bounds__(64 * WAVES, 5) void k_explore_join(JoinCopy jc, int N, int D, int K, const int* __restrict__ old_idx,
+__global__ __launch_bounds__(64 * WAVES, 5) void k_explore_join(JoinCopy jc, int N, int K, const int* __restrict__ old_idx,
                                                               const float2* __restrict__ recs,
                                                               const int* __restrict__ offs, const int* __restrict__ rev,
                                                               uint32_t* __restrict__ pass, uint16_t* __restrict__ bounds, int KP, int bpitch, int ksteps,
-                                                              float kappa, float one_minus_gamma, int wave_lds_ints,
+                                                              float kappa, int wave_lds_ints,
                                                               uint32_t div_m, int div_s, const int* __restrict__ order)
 {
     extern __shared__ __align__(16) int lds_join[];
@@ -639,9 +655,9 @@ __global__ __launch_bounds__(64 * WAVES, 5) void k_explore_join(JoinCopy jc, int
     float* pn = reinterpret_cast<float*>(pid + 32);
     float* pbar = pn + 32;
     float* perr = pbar + 32;
-    int* pe = reinterpret_cast<int*>(perr + 32);
+    float* pper = perr + 32;
+    int* pe = reinterpret_cast<int*>(pper + 32);
     const int MW = KP >> 5;
-    const float inv_scale = 1.0f / *jc.scale(D);
 
     for (int k = lane; k < KP; k += 64) {
         int c = k < K ? old_idx[(size_t)q * K + k] : -1;
@@ -661,7 +677,10 @@ __global__ __launch_bounds__(64 * WAVES, 5) void k_explore_join(JoinCopy jc, int
             const float2 rec = p >= 0 ? recs[p] : make_float2(0.0f, 0.0f);
             pn[lane] = rec.x;
             pbar[lane] = rec.y;
-            if (BOUNDS) perr[lane] = p >= 0 ? jc.errs[p] : 0.0f;
+            if (BOUNDS) {
+                perr[lane] = p >= 0 ? jc.errs[p] : 0.0f;
+                pper[lane] = 65534.0f / join_span(rec);
+            }
         }
         wave_lds_sync();
 
@@ -700,7 +719,7 @@ __global__ __launch_bounds__(64 * WAVES, 5) void k_explore_join(JoinCopy jc, int
                 const uint64_t bm = ballot64(marked);
                 if (BOUNDS && marked && m < np)
                     bounds[(size_t)pe[m] * (size_t)KP + ct * 32 + (lane & 31)] =
-                        (uint16_t)join_bound16(least, perr[m], ce, inv_scale, one_minus_gamma);
+                        (uint16_t)join_code(least, perr[m], ce, pper[m]);
                 const int m_lo = 8 * (i >> 2) + (i & 3);
                 if (lane == m_lo) mine = (uint32_t)bm;
                 if (lane == m_lo + 4) mine = (uint32_t)(bm >> 32);
@@ -808,11 +827,11 @@ constexpr int kJwP = 96;                    // points of R(q) worked on together
 constexpr int kJwRowBytes = 144;            // 64 float16 values + 16 bytes: rows start in different banks
 
 template <bool BOUNDS, int NPW>
-__global__ __launch_bounds__(256, NPW == 3 ? 3 : 1) void k_explore_join_wg(JoinCopy jc, int N, int D, int K, const int* __restrict__ old_idx,
+__global__ __launch_bounds__(256, NPW == 3 ? 3 : 1) void k_explore_join_wg(JoinCopy jc, int N, int K, const int* __restrict__ old_idx,
                                                          const float2* __restrict__ recs, const int* __restrict__ offs,
                                                          const int* __restrict__ rev, uint32_t* __restrict__ pass,
                                                          uint16_t* __restrict__ bounds, int KP, int bpitch, int ksteps,
-                                                         float kappa, float one_minus_gamma, uint32_t div_m, int div_s,
+                                                         float kappa, uint32_t div_m, int div_s,
                                                          const int* __restrict__ order)
 {
     constexpr int kPieces = (kJwP + (NPW == 3 ? 128 : 256)) * 8 / 256;      // 16-byte pieces a thread stages per step
@@ -826,6 +845,7 @@ __global__ __launch_bounds__(256, NPW == 3 ? 3 : 1) void k_explore_join_wg(JoinC
     float* pn = reinterpret_cast<float*>(pe + kJwP);
     float* pbar = pn + kJwP;
     float* perr = pbar + kJwP;
+    float* pper = perr + kJwP;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int n = lane & 31, h = lane >> 5;
     const int item = die_local_place(blockIdx.x, gridDim.x);
@@ -835,7 +855,6 @@ __global__ __launch_bounds__(256, NPW == 3 ? 3 : 1) void k_explore_join_wg(JoinC
     if (R <= 0) return;
     const int MW = KP >> 5;
     const int nrows = kJwP + KP;
-    const float inv_scale = 1.0f / *jc.scale(D);
     for (int k = tid; k < KP; k += 256) {
         int c = k < K ? old_idx[(size_t)q * K + k] : -1;
         if (c < 0 || c >= N) c = -1;
@@ -855,7 +874,10 @@ __global__ __launch_bounds__(256, NPW == 3 ? 3 : 1) void k_explore_join_wg(JoinC
             pe[tid] = e;
             pn[tid] = rec.x;
             pbar[tid] = rec.y;
-            if (BOUNDS) perr[tid] = p >= 0 ? jc.errs[p] : 0.0f;
+            if (BOUNDS) {
+                perr[tid] = p >= 0 ? jc.errs[p] : 0.0f;
+                pper[tid] = 65534.0f / join_span(rec);
+            }
         }
         __syncthreads();
         f32x16 acc[NPW];
@@ -925,7 +947,7 @@ __global__ __launch_bounds__(256, NPW == 3 ? 3 : 1) void k_explore_join_wg(JoinC
                     const bool marked = cid >= 0 && join_may(least, pbar[m], ce);
                     const uint64_t bm = ballot64(marked);
                     if (BOUNDS && marked && m < npg)
-                        bounds[(size_t)pe[m] * (size_t)KP + col] = (uint16_t)join_bound16(least, perr[m], ce, inv_scale, one_minus_gamma);
+                        bounds[(size_t)pe[m] * (size_t)KP + col] = (uint16_t)join_code(least, perr[m], ce, pper[m]);
                     const int m_lo = 8 * (j >> 2) + (j & 3);
                     if (lane == m_lo) mine = (uint32_t)bm;
                     if (lane == m_lo + 4) mine = (uint32_t)(bm >> 32);
@@ -1064,7 +1086,7 @@ void explore_ws_free(ExploreWorkspace* w)
 }
 
 const uint32_t* explore_ws_pass(const ExploreWorkspace* w) { return w->pass; }
-const uint16_t* explore_ws_bounds(const ExploreWorkspace* w) { return w->bounds; }
+const JoinBounds& explore_ws_bounds(const ExploreWorkspace* w) { return w->view; }
 int* explore_ws_todo(ExploreWorkspace* w, int which) { return w->todo + (size_t)which * ((size_t)w->N + 1); }
 
 bool explore_ws_takes(int N, int K)
@@ -1146,20 +1168,28 @@ int launch_explore_join(ExploreWorkspace* w, const JoinCopy& jc, int N, int D, i
 
     constexpr int kWaves = 4;
     const int KP = (K + 31) & ~31;
-    const int wave_ints = (KP + 160 + 3) & ~3;
+    const int wave_ints = (KP + 192 + 3) & ~3;
     const size_t lds = (size_t)kWaves * (size_t)wave_ints * sizeof(int);
     const int ksteps = (D + 15) / 16;
     RSFK_CHECK(ksteps * 16 <= join_pitch(D), "exploration join: rows of the copy too short");
     const float kappa = (float)(ksteps * 16 + 16) * (1.0f / 2097152.0f);            // (Dp + 16) 2^-21
     const float one_minus_gamma = 1.0f - (float)(D + 8) * (1.0f / 4194304.0f);      // 1 - (D + 8) 2^-22
     RSFK_CHECK(one_minus_gamma > 0.5f, "exploration join: D too large");
-    hipLaunchKernelGGL(k_join_records, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, stream, jc.norms, jc.errs, jc.scale(D),
-                       knn_dist, N, K, one_minus_gamma, w->recs);
+    // rounding of any row: 2^-11 of a value, 2^-14 of one set to zero, and errs' own terms (3e-3 covers these and the root)
+    const float any_rel = 1.003f / 2048.0f, any_abs = 1.001f * std::sqrt((float)D) / 16384.0f + 1e-6f;
+    w->view.codes = w->bounds;
+    w->view.recs = w->recs;
+    w->view.errs = jc.errs;
+    w->view.scale = jc.scale(D);
+    w->view.kappa = kappa;
+    w->view.one_minus_gamma = one_minus_gamma;
+    w->view.any_rel = any_rel;
+    w->view.any_abs = any_abs;
+    hipLaunchKernelGGL(k_join_records, dim3((unsigned)((N + 255) / 256) + 1), dim3(256), 0, stream, jc, jc.scale(D), knn_dist, N, K,
+                       one_minus_gamma, w->recs);
     RSFK_HIP(hipGetLastError());
     if (!w->bounds && KP == 32 && ksteps <= 8) {
         const dim3 grid(grid_for_dies(((size_t)N + kWaves - 1) / kWaves)), block(64 * kWaves);
-        // rounding of any row: 2^-11 of a value, 2^-14 of one set to zero, and errs' own terms (3e-3 covers these and the root)
-        const float any_rel = 1.003f / 2048.0f, any_abs = 1.001f * std::sqrt((float)D) / 16384.0f + 1e-6f;
 #define RSFK_JOIN_SHORT(KSV)                                                                                                \
         hipLaunchKernelGGL((k_explore_join_short<kWaves, KSV>), grid, block, 0, stream, jc, N, K, old_idx, w->recs, w->offs, \
                            w->rev, w->pass, join_pitch(D), ksteps, kappa, any_rel, any_abs, w->div_m, w->div_s, order)
@@ -1170,14 +1200,14 @@ int launch_explore_join(ExploreWorkspace* w, const JoinCopy& jc, int N, int D, i
     } else if (KP > 32 && join_wg_on()) {
         // one workgroup per q: every row once per 96 points of R(q).  (Rows of at most 32 neighbours have one pair per
         // tile of R(q): too little for four wavefronts; 1M x 256, K = 32: 8.1 ms against 12.6.)
-        const size_t lds_wg = (size_t)(kJwP + KP) * kJwRowBytes + (size_t)KP * 12 + (size_t)kJwP * 20;
+        const size_t lds_wg = (size_t)(kJwP + KP) * kJwRowBytes + (size_t)KP * 12 + (size_t)kJwP * 24;
 #define RSFK_JOIN_WG(BV, NV)                                                                                                \
         do {                                                                                                               \
             RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_explore_join_wg<BV, NV>),                         \
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_wg));                       \
-            hipLaunchKernelGGL((k_explore_join_wg<BV, NV>), dim3(grid_for_dies((size_t)N)), dim3(256), lds_wg, stream, jc, N, D, K,  \
+            hipLaunchKernelGGL((k_explore_join_wg<BV, NV>), dim3(grid_for_dies((size_t)N)), dim3(256), lds_wg, stream, jc, N, K,  \
                                old_idx, w->recs, w->offs, w->rev, w->pass, w->bounds, KP, join_pitch(D), ksteps, kappa,  \
-                               one_minus_gamma, w->div_m, w->div_s, order);                                                \
+                               w->div_m, w->div_s, order);                                                \
         } while (0)
         if (w->bounds && KP <= 128) RSFK_JOIN_WG(true, 3);
         else if (w->bounds) RSFK_JOIN_WG(true, 6);
@@ -1186,12 +1216,12 @@ int launch_explore_join(ExploreWorkspace* w, const JoinCopy& jc, int N, int D, i
 #undef RSFK_JOIN_WG
     } else if (w->bounds)
         hipLaunchKernelGGL((k_explore_join<kWaves, true>), dim3(grid_for_dies(((size_t)N + kWaves - 1) / kWaves)), dim3(64 * kWaves), lds,
-                           stream, jc, N, D, K, old_idx, w->recs, w->offs, w->rev, w->pass, w->bounds, KP, join_pitch(D), ksteps,
-                           kappa, one_minus_gamma, wave_ints, w->div_m, w->div_s, order);
+                           stream, jc, N, K, old_idx, w->recs, w->offs, w->rev, w->pass, w->bounds, KP, join_pitch(D), ksteps,
+                           kappa, wave_ints, w->div_m, w->div_s, order);
     else
         hipLaunchKernelGGL((k_explore_join<kWaves, false>), dim3(grid_for_dies(((size_t)N + kWaves - 1) / kWaves)), dim3(64 * kWaves), lds,
-                           stream, jc, N, D, K, old_idx, w->recs, w->offs, w->rev, w->pass, w->bounds, KP, join_pitch(D), ksteps,
-                           kappa, one_minus_gamma, wave_ints, w->div_m, w->div_s, order);
+                           stream, jc, N, K, old_idx, w->recs, w->offs, w->rev, w->pass, w->bounds, KP, join_pitch(D), ksteps,
+                           kappa, wave_ints, w->div_m, w->div_s, order);
     RSFK_HIP(hipGetLastError());
     return 0;
 }

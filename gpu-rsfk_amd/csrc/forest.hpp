@@ -205,7 +205,8 @@ const int* explore_ws_offs(const ExploreWorkspace* w);       // N + 1
 int* explore_ws_rev(const ExploreWorkspace* w);        // entry numbers p K + k, in compressed rows by the neighbour
 void explore_ws_free(ExploreWorkspace* w);
 const uint32_t* explore_ws_pass(const ExploreWorkspace* w);
-const uint16_t* explore_ws_bounds(const ExploreWorkspace* w);
+struct JoinBounds;
+const JoinBounds& explore_ws_bounds(const ExploreWorkspace* w);
 int* explore_ws_todo(ExploreWorkspace* w, int which);
 // order: null, or a permutation of the points that keeps nearby points together (the buckets of a tree): the points
 // are then worked on in that order, a contiguous eighth of it per die (die_local_place)

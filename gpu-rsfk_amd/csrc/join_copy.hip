@@ -131,8 +131,8 @@ __global__ __launch_bounds__(256) void k_col_mean(const float* __restrict__ poin
 // 0.35 ms, 5.7 TB/s (a wavefront per row, a value per lane: 1.13); 1M x 256 0.26 (0.42), 1M x 100 0.12 (0.22).
 template <int LPR, bool WHOLE>
 __global__ __launch_bounds__(256) void k_to_join(const float* __restrict__ points, uint16_t* __restrict__ out, float* __restrict__ norms,
-                                                 float* __restrict__ errs, const float* __restrict__ mu, const float* __restrict__ scale,
-                                                 int N, int D, int pitch)
+                                                 float* __restrict__ errs, float2* __restrict__ parts, const float* __restrict__ mu,
+                                                 const float* __restrict__ scale, int N, int D, int pitch)
 {
     constexpr int kRowsPerWave = 64 / LPR;
     const int lane = threadIdx.x & 63, sub = lane / LPR, l = lane - sub * LPR;
@@ -140,6 +140,7 @@ __global__ __launch_bounds__(256) void k_to_join(const float* __restrict__ point
     const int n_waves = (gridDim.x * blockDim.x) >> 6;
     const float s = *scale;
     const float sums = 1.0f + (float)(D + 16) * (1.0f / 16777216.0f);      // sums of D squares, in any order
+    float most_q = 0.0f, most_e = 0.0f;
     for (int rb = wave_global * kRowsPerWave; rb < N; rb += n_waves * kRowsPerWave) {
         const int r = rb + sub;
         const bool row_ok = r < N;
@@ -172,18 +173,35 @@ __global__ __launch_bounds__(256) void k_to_join(const float* __restrict__ point
             e += __shfl_xor(e, o, 64);
         }
         // fl(x - mu) is within 2^-24 |fl(x - mu)| of x - mu, which is at most 1.1 |row| and what was set to zero (1e-8 stands for it)
+        e = sums * (sqrtf(e) + (1.2f / 16777216.0f) * sqrtf(q)) + 1e-8f;
         if (row_ok && l == 0) {
             norms[r] = q;
-            errs[r] = sums * (sqrtf(e) + (1.2f / 16777216.0f) * sqrtf(q)) + 1e-8f;
+            errs[r] = e;
+        }
+        if (row_ok && q <= 3.0e38f) {
+            most_q = fmaxf(most_q, q);
+            most_e = fmaxf(most_e, e);
         }
     }
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        most_q = fmaxf(most_q, __shfl_xor(most_q, o, 64));
+        most_e = fmaxf(most_e, __shfl_xor(most_e, o, 64));
+    }
+    __shared__ float2 part[4];
+    if (lane == 0) part[threadIdx.x >> 6] = make_float2(most_q, most_e);
+    __syncthreads();
+    if (threadIdx.x == 0)
+        parts[blockIdx.x] = make_float2(fmaxf(fmaxf(part[0].x, part[1].x), fmaxf(part[2].x, part[3].x)),
+                                        fmaxf(fmaxf(part[0].y, part[1].y), fmaxf(part[2].y, part[3].y)));
 }
 
 }  // namespace
 
 int join_copy_alloc(JoinCopy* c, int N, int D)
 {
-    if (ws_alloc(reinterpret_cast<void**>(&c->mu), ((size_t)2 * D + 1) * sizeof(float))) return 1;
+    if (ws_alloc(reinterpret_cast<void**>(&c->mu), ((size_t)2 * D + 3) * sizeof(float))) return 1;
+    if (ws_alloc(reinterpret_cast<void**>(&c->parts), kJoinMostGrid * sizeof(float2))) return 1;
     if (ws_alloc(reinterpret_cast<void**>(&c->rows), std::max<size_t>((size_t)N * join_pitch(D) * 2, 16))) return 1;
     if (ws_alloc(reinterpret_cast<void**>(&c->norms), std::max<size_t>((size_t)N * 4, 16))) return 1;
     if (ws_alloc(reinterpret_cast<void**>(&c->errs), std::max<size_t>((size_t)N * 4, 16))) return 1;
@@ -196,14 +214,15 @@ void join_copy_free(JoinCopy* c)
     ws_free(c->norms);
     ws_free(c->errs);
     ws_free(c->mu);
+    ws_free(c->parts);
     *c = JoinCopy();
 }
 
-int join_copy_fill(const JoinCopy& c, const float* points, int N, int D, hipStream_t stream)
+int join_copy_fill(JoinCopy& c, const float* points, int N, int D, hipStream_t stream)
 {
     float* scale = c.mu + D;
-    uint32_t* spread = reinterpret_cast<uint32_t*>(scale + 1);
-    hipLaunchKernelGGL(k_col_clear, dim3((2 * D + 1 + 255) / 256), dim3(256), 0, stream, reinterpret_cast<uint32_t*>(c.mu), 2 * D + 1);
+    uint32_t* spread = reinterpret_cast<uint32_t*>(scale + 3);
+    hipLaunchKernelGGL(k_col_clear, dim3((2 * D + 3 + 255) / 256), dim3(256), 0, stream, reinterpret_cast<uint32_t*>(c.mu), 2 * D + 3);
     // (a workgroup ends with two atomics per column, carried out one after the other: 123,457 x 37 with 64 rows each 0.062 ms, with 256
     // 0.022)
     const int g = std::max(1, std::min(N / (D <= 128 ? 256 : 64), 2048));
@@ -214,9 +233,10 @@ int join_copy_fill(const JoinCopy& c, const float* points, int N, int D, hipStre
     const int pitch = join_pitch(D);
 #define RSFK_TO_JOIN(L)                                                                                                            \
     do {                                                                                                                           \
-        const dim3 grid((unsigned)std::min<size_t>(((size_t)N + 4 * (64 / L) - 1) / (4 * (64 / L)), 65536));                         \
-        if (whole) hipLaunchKernelGGL((k_to_join<L, true>), grid, dim3(256), 0, stream, points, c.rows, c.norms, c.errs, c.mu, scale, N, D, pitch); \
-        else hipLaunchKernelGGL((k_to_join<L, false>), grid, dim3(256), 0, stream, points, c.rows, c.norms, c.errs, c.mu, scale, N, D, pitch); \
+        c.n_parts = (int)std::min<size_t>(((size_t)N + 4 * (64 / L) - 1) / (4 * (64 / L)), kJoinMostGrid);                           \
+        const dim3 grid((unsigned)c.n_parts);                                                                                      \
+        if (whole) hipLaunchKernelGGL((k_to_join<L, true>), grid, dim3(256), 0, stream, points, c.rows, c.norms, c.errs, c.parts, c.mu, scale, N, D, pitch); \
+        else hipLaunchKernelGGL((k_to_join<L, false>), grid, dim3(256), 0, stream, points, c.rows, c.norms, c.errs, c.parts, c.mu, scale, N, D, pitch); \
     } while (0)
     if (pitch <= 32) RSFK_TO_JOIN(8);
     else if (pitch <= 64) RSFK_TO_JOIN(16);

@@ -14,16 +14,20 @@ namespace rsfk {
 // rows start on 64-byte boundaries; the kernels take 16 dimensions per step
 __host__ __device__ inline int join_pitch(int D) { return (D + 31) & ~31; }
 
+constexpr int kJoinMostGrid = 8192;     // workgroups (and parts) of the kernel that makes the copy
+
 struct JoinCopy {
     uint16_t* rows = nullptr;     // N x join_pitch(D)
     float* norms = nullptr;       // N, in units of s^2
     float* errs = nullptr;        // N, in units of s
-    float* mu = nullptr;          // column means, then s, then D words of working memory
-    __host__ __device__ const float* scale(int D) const { return mu + D; }
+    float* mu = nullptr;          // column means, then (s, largest norm, largest error of the finite rows), then D words of working memory
+    float2* parts = nullptr;      // n_parts: largest norm and error of the finite rows a workgroup made (join_records completes them)
+    int n_parts = 0;
+    float* scale(int D) const { return mu + D; }
 };
 
 int join_copy_alloc(JoinCopy* c, int N, int D);
 void join_copy_free(JoinCopy* c);
-int join_copy_fill(const JoinCopy& c, const float* points, int N, int D, hipStream_t stream);
+int join_copy_fill(JoinCopy& c, const float* points, int N, int D, hipStream_t stream);
 
 }  // namespace rsfk

@@ -531,6 +531,30 @@ def test_explore_screens_rows_of_any_magnitude(gpu, orc, rng, N, D, K, values):
         assert_knn_equal(gi, gd, oi, od)
 
 
+@pytest.mark.parametrize("codes", [True, False])
+@pytest.mark.parametrize("N,D,K,leaf,spread", [(1500, 10, 46, 47, 1.0), (2500, 70, 64, 20, 1.0), (4000, 33, 65, 66, 1.0), (1200, 6, 128, 129, 0.02),
+                                               (5000, 12, 100, 60, 1.0), (3000, 20, 256, 257, 1.0), (2000, 5, 200, 70, 0.05), (9000, 64, 90, 91, 1.0)])
+def test_explore_with_a_workgroup_per_point(gpu, orc, rng, monkeypatch, N, D, K, leaf, spread, codes):
+    """Long rows: one and several slots per lane; rows that are full and rows that are not (small leaves: hundreds of candidates enter,
+    several rounds, more candidates than the list takes); few distinct candidates among thousands of marks (small spread: 40 clusters);
+    without the codes of the join (RSFK_OPTIONAL_MB=0: no memory for them)."""
+    if not codes:
+        monkeypatch.setenv("RSFK_OPTIONAL_MB", "0")
+    X = rng.standard_normal((N, D)).astype(np.float32)
+    if spread < 1.0:
+        X = (X[rng.integers(0, 40, N)] + np.float32(spread) * X).astype(np.float32)
+    oi, od = orc.init_lists(N, K, self_in=True)
+    for seed in range(2):
+        perm, ls, lz, _ = orc.build_tree(X, leaf, 2 * leaf, 5000, seed)
+        orc.bucket_knn(X, K, perm, lz, oi, od, starts=ls)
+    gi, gd = oi.copy(), od.copy()
+    _say("explore workgroup", N, D, K, leaf, spread, codes)
+    for _ in range(2):
+        orc.explore(X, K, oi, od)
+        gpu.explore(X, K, gi, gd, 1)
+        assert_knn_equal(gi, gd, oi, od)
+
+
 # ---------------------------------------------------------------------------
 # the whole call, through the entry points the Python package binds
 # ---------------------------------------------------------------------------
