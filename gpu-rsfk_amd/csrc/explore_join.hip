@@ -13,8 +13,10 @@
 //   Gram matrix and norms:  |d~(computed) - d~(real)| <= E1 = (D' + 16) 2^-21 S
 //   fp32 chain:             result >= d(real) (1 - gamma),  gamma = (D + 8) 2^-22
 // so a pair is dropped when d~ - E1 is above (bar_p + e_c)^2, bar_p = s sqrt(last slot of row p / (1 - gamma)) + e_p: its exact
-// distance is then above the last slot.  e_p is the length measured when the copy was made; for e_c the kernel of short rows, which
-// has 8 bytes per point for all of this, takes what holds for any row, 2^-11 |row| + 2^-14 sqrt(D).
+// distance is then above the last slot.  For e the smaller is taken of what holds for any row of that norm, 2^-11 |row| + 2^-14 sqrt(D),
+// and of the largest length measured when the copy was made; norms come from the rows themselves, which the kernels have in registers.
+// So the bar, four bytes, is all that is gathered besides the rows.  (Records of norm and bar for both sides: 1M x 256
+// 8.0 -> 7.0 ms, 10M x 32 27.2 -> 24.6, 1M x 100 3.66 -> 3.45.)
 // (Measured against rows in bfloat16 with 2^-8 |row| for e: exact distances per point 1M x 100 28 -> 22, 1M x 256 in 64 clusters
 // 74 -> 39, sparse 70,000 x 784 with K = 90 185 -> 140, 10M x 32 49 -> 42; merge 3.54 -> 2.77, 13.9 -> 8.25, 15.9 -> 12.6 and 23.6 ->
 // 20.1 ms.  bfloat16 with the measured e: 24, 41, 147 and 45.)
@@ -57,7 +59,7 @@ struct ExploreWorkspace {
     int* bin_start = nullptr;  // n_bins + 1
     int* part_off = nullptr;   // n_parts x n_bins: where the entries of a part start inside a bin
     uint32_t* pass = nullptr;  // N*K*MW, indexed by entry number
-    float2* recs = nullptr;    // N: norm of a point's row in the copy, and the bar its candidates have to pass (k_join_records)
+    float* bars = nullptr;     // N: the bar the candidates of a point have to pass (k_join_bars)
     JoinBounds view;           // what the merge kernels read (set by launch_explore_join)
     uint16_t* bounds = nullptr; // N*K*32*MW codes of the marked pairs (join_bounds.hpp), or null
     bool tiled = false;         // the builder of medium graphs: bins of 2^cshift points, rows of 2^fshift of them at a time
@@ -582,13 +584,13 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_rows(const int2* __restri
     }
 }
 
-// What the join needs of a point besides its row, in one 8-byte record (one gather instead of two): (norm, bar).
+// The bar of a point: s sqrt(last slot of its row / (1 - gamma)) + e_p.
 // A sum bar + e_c is at least 1 + 2^-21 times the sum of the values it stands for, which covers the roundings of the sum, its square
-// and the comparison.  1e-30 under the root covers what underflow takes from the chain.  An infinite or NaN last slot makes bar
+// and the comparison.  1e-30 under the root covers what underflow takes from the chain.  An infinite or NaN last slot makes the bar
 // infinite or NaN, a row that is not finite makes d~ - E1 NaN, and a comparison with that drops nothing.
 // The last workgroup has no points: it takes the largest norm and error of any finite row from the parts of them (join_copy.hip).
-__global__ __launch_bounds__(256) void k_join_records(JoinCopy jc, float* __restrict__ scale, const float* __restrict__ knn_dist, int N, int K,
-                                                      float one_minus_gamma, float2* __restrict__ out)
+__global__ __launch_bounds__(256) void k_join_bars(JoinCopy jc, float* __restrict__ scale, const float* __restrict__ knn_dist, int N, int K,
+                                                   float one_minus_gamma, float* __restrict__ out)
 {
     if (blockIdx.x + 1 == gridDim.x) {
         __shared__ float2 part[256];
@@ -610,14 +612,14 @@ __global__ __launch_bounds__(256) void k_join_records(JoinCopy jc, float* __rest
         }
         if (threadIdx.x == 0) {
             scale[1] = most.x;
-            scale[2] = most.y;
+            scale[2] = most.y * kJoinUp;
         }
         return;
     }
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= N) return;
     const float tau = knn_dist[(size_t)p * K + (K - 1)];
-    out[p] = make_float2(jc.norms[p], (scale[0] * sqrtf(tau / one_minus_gamma + 1e-30f) + jc.errs[p]) * kJoinUp);
+    out[p] = (scale[0] * sqrtf(tau / one_minus_gamma + 1e-30f) + jc.errs[p]) * kJoinUp;
 }
 
 // d~ - E1 of a pair, from S = n_p + n_c and the product g of the rows
@@ -633,14 +635,27 @@ __device__ __forceinline__ bool join_may(float least, float bar, float e_c)
     return !(least > w * w);
 }
 
+// squares of eight values of a row added up (lanes l and l + 32 have the values of a row in turns of eight)
+__device__ __forceinline__ float half_norm(f16x8 v, float acc)
+{
+    typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
+#pragma unroll
+    for (int i = 0; i < 8; i += 2) {
+        const f16x2 h = {v[i], v[i + 1]};
+        acc = __builtin_amdgcn_fdot2(h, h, acc, false);
+    }
+    return acc;
+}
+
 // One wavefront per q.  Per-wavefront LDS (ints): cq[KP] | pid[32] | pn[32] | pbar[32] | perr[32] | pper[32] | pe[32], KP = K rounded up to 32.
-// (five wavefronts per SIMD: 1M x 256 8.7 -> 8.2 ms against four, for three spilled registers)
+// Workgroups (x, y): every gridDim.y-th tile of R(q), the y-th first.  (Five wavefronts per SIMD: 1M x 256 7.6 -> 7.0 ms against four
+// with the next 64 dimensions in flight.)
 template <int WAVES, bool BOUNDS>
 __global__ __launch_bounds__(64 * WAVES, 5) void k_explore_join(JoinCopy jc, int N, int K, const int* __restrict__ old_idx,
-                                                              const float2* __restrict__ recs,
+                                                              const float* __restrict__ bars,
                                                               const int* __restrict__ offs, const int* __restrict__ rev,
                                                               uint32_t* __restrict__ pass, uint16_t* __restrict__ bounds, int KP, int bpitch, int ksteps,
-                                                              float kappa, int wave_lds_ints,
+                                                              float kappa, float any_rel, float any_abs, int wave_lds_ints,
                                                               uint32_t div_m, int div_s, const int* __restrict__ order)
 {
     extern __shared__ __align__(16) int lds_join[];
@@ -649,7 +664,7 @@ __global__ __launch_bounds__(64 * WAVES, 5) void k_explore_join(JoinCopy jc, int
     if (item >= N) return;                                // whole wavefront leaves together
     const int q = order ? order[item] : item;
     const int r0 = offs[q], R = offs[q + 1] - r0;
-    if (R <= 0) return;
+    if (R <= 32 * (int)blockIdx.y) return;
     int* cq = lds_join + (size_t)wave * (size_t)wave_lds_ints;
     int* pid = cq + KP;
     float* pn = reinterpret_cast<float*>(pid + 32);
@@ -658,6 +673,7 @@ __global__ __launch_bounds__(64 * WAVES, 5) void k_explore_join(JoinCopy jc, int
     float* pper = perr + 32;
     int* pe = reinterpret_cast<int*>(pper + 32);
     const int MW = KP >> 5;
+    const float most_norm = jc.mu[jc.D + 1], most_err = jc.mu[jc.D + 2];
 
     for (int k = lane; k < KP; k += 64) {
         int c = k < K ? old_idx[(size_t)q * K + k] : -1;
@@ -665,7 +681,7 @@ __global__ __launch_bounds__(64 * WAVES, 5) void k_explore_join(JoinCopy jc, int
         cq[k] = c;
     }
 
-    for (int pt0 = 0; pt0 < R; pt0 += 32) {
+    for (int pt0 = 32 * (int)blockIdx.y; pt0 < R; pt0 += 32 * (int)gridDim.y) {
         const int np = min(32, R - pt0);
         wave_lds_sync();                                  // reads of the previous tile are done (and cq is written)
         int my_e = -1;                                    // lanes 0..31: the graph entry (p, k) with q = neighbour k of p
@@ -674,13 +690,9 @@ __global__ __launch_bounds__(64 * WAVES, 5) void k_explore_join(JoinCopy jc, int
             const int p = my_e >= 0 ? (int)(((uint64_t)div_m * (uint64_t)(uint32_t)my_e) >> div_s) : -1;
             pid[lane] = p;
             pe[lane] = my_e;
-            const float2 rec = p >= 0 ? recs[p] : make_float2(0.0f, 0.0f);
-            pn[lane] = rec.x;
-            pbar[lane] = rec.y;
-            if (BOUNDS) {
-                perr[lane] = p >= 0 ? jc.errs[p] : 0.0f;
-                pper[lane] = 65534.0f / join_span(rec);
-            }
+            const float bar = p >= 0 ? bars[p] : 0.0f;
+            pbar[lane] = bar;
+            if (BOUNDS) pper[lane] = 65534.0f / join_span(bar, most_norm);
         }
         wave_lds_sync();
 
@@ -690,7 +702,7 @@ __global__ __launch_bounds__(64 * WAVES, 5) void k_explore_join(JoinCopy jc, int
         for (int ct = 0; ct < MW; ++ct) {
             const int cid = cq[ct * 32 + (lane & 31)];
             const uint16_t* rb = jc.rows + (size_t)(cid >= 0 ? cid : q) * (size_t)bpitch + 8 * (lane >> 5);
-            const float cn = recs[cid >= 0 ? cid : q].x, ce = jc.errs[cid >= 0 ? cid : q] * kJoinUp;
+            float an = 0.0f, cn = 0.0f;                   // norms of the row of point l % 32 of the tile and of neighbour l % 32
             f32x16 g;
 #pragma unroll
             for (int i = 0; i < 16; ++i) g[i] = 0.0f;
@@ -704,9 +716,23 @@ __global__ __launch_bounds__(64 * WAVES, 5) void k_explore_join(JoinCopy jc, int
                     }
                 }
 #pragma unroll
-                for (int u = 0; u < 4; ++u)
-                    if (k0 + u < ksteps) g = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[u], b[u], g, 0, 0, 0);
+                for (int u = 0; u < 4; ++u) {
+                    if (k0 + u < ksteps) {
+                        g = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[u], b[u], g, 0, 0, 0);
+                        an = half_norm(a[u], an);
+                        cn = half_norm(b[u], cn);
+                    }
+                }
             }
+            an += __shfl_xor(an, 32, 64);
+            cn += __shfl_xor(cn, 32, 64);
+            const float ce = join_err(cn, any_rel, any_abs, most_err);
+            wave_lds_sync();
+            if (lane < 32) {
+                pn[lane] = an;
+                if (BOUNDS) perr[lane] = join_err(an, any_rel, any_abs, most_err);
+            }
+            wave_lds_sync();
             // Accumulator i of lane l: point m = 4 (l / 32) + 8 (i / 4) + i % 4 of the tile, column = neighbour l % 32
             // of this group of 32.  The ballot over the wavefront therefore holds the 32-bit masks of two points:
             // low half for m = 8 (i / 4) + i % 4, high half for m + 4.
@@ -737,7 +763,7 @@ __global__ __launch_bounds__(64 * WAVES, 5) void k_explore_join(JoinCopy jc, int
 // wavefronts per SIMD.  The bound is that of k_explore_join.
 template <int WAVES, int KS>
 __global__ __launch_bounds__(64 * WAVES) void k_explore_join_short(JoinCopy jc, int N, int K, const int* __restrict__ old_idx,
-                                                                    const float2* __restrict__ recs,
+                                                                    const float* __restrict__ bars,
                                                                     const int* __restrict__ offs, const int* __restrict__ rev,
                                                                     uint32_t* __restrict__ pass, int bpitch, int ksteps,
                                                                     float kappa, float any_rel, float any_abs, uint32_t div_m, int div_s,
@@ -752,7 +778,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_join_short(JoinCopy jc, 
     const int r0 = offs[q], R = offs[q + 1] - r0;
     const int col = lane & 31, hi = lane >> 5;
     int cid = col < K ? old_idx[(size_t)q * K + col] : -1;
-    if (R <= 0) return;
+    if (R <= 32 * (int)blockIdx.y) return;
     if (cid < 0 || cid >= N) cid = -1;
     const uint16_t* rb = jc.rows + (size_t)(cid >= 0 ? cid : q) * (size_t)bpitch + 8 * hi;
     f16x8 b[KS];
@@ -762,22 +788,25 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_join_short(JoinCopy jc, 
         for (int i = 0; i < 8; ++i) b[u][i] = (_Float16)0.0f;
         if (u < ksteps) b[u] = *reinterpret_cast<const f16x8*>(rb + 16 * u);
     }
-    const float cn = recs[cid >= 0 ? cid : q].x;
-    const float ce = __builtin_fmaf(any_rel, __builtin_amdgcn_sqrtf(cn), any_abs);
+    float cn = 0.0f;
+#pragma unroll
+    for (int u = 0; u < KS; ++u) cn = half_norm(b[u], cn);
+    cn += __shfl_xor(cn, 32, 64);
+    const float ce = join_err(cn, any_rel, any_abs, jc.mu[jc.D + 2]);
     const int mbase = 4 * hi;
     int* pid = pid_s[wave];
     float* pn = pn_s[wave];
     float* pbar = pbar_s[wave];
 
-    for (int pt0 = 0; pt0 < R; pt0 += 32) {
+    for (int pt0 = 32 * (int)blockIdx.y; pt0 < R; pt0 += 32 * (int)gridDim.y) {
         const int np = min(32, R - pt0);
         int my_e = -1;                                    // lanes 0..31: the graph entry (p, k) with q = neighbour k of p
-        float2 rec = make_float2(0.0f, 0.0f);
+        float bar = 0.0f;
         if (lane < 32) {
             my_e = lane < np ? rev[(size_t)r0 + pt0 + lane] : -1;
             const int p = my_e >= 0 ? (int)(((uint64_t)div_m * (uint64_t)(uint32_t)my_e) >> div_s) : -1;
             pid[lane] = p;
-            if (p >= 0) rec = recs[p];
+            if (p >= 0) bar = bars[p];
         }
         wave_lds_sync();
         const int pm = pid[col];
@@ -794,9 +823,13 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_join_short(JoinCopy jc, 
         for (int i = 0; i < 16; ++i) g[i] = 0.0f;
 #pragma unroll
         for (int u = 0; u < KS; ++u) g = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[u], b[u], g, 0, 0, 0);
+        float an = 0.0f;
+#pragma unroll
+        for (int u = 0; u < KS; ++u) an = half_norm(a[u], an);
+        an += __shfl_xor(an, 32, 64);
         if (lane < 32) {
-            pn[lane] = rec.x;
-            pbar[lane] = rec.y;
+            pn[lane] = an;
+            pbar[lane] = bar;
         }
         wave_lds_sync();
         // Accumulator i of lane l: point m = 4 (l / 32) + 8 (i / 4) + i % 4 of the tile, column = neighbour l % 32.
@@ -828,10 +861,10 @@ constexpr int kJwRowBytes = 144;            // 64 float16 values + 16 bytes: row
 
 template <bool BOUNDS, int NPW>
 __global__ __launch_bounds__(256, NPW == 3 ? 3 : 1) void k_explore_join_wg(JoinCopy jc, int N, int K, const int* __restrict__ old_idx,
-                                                         const float2* __restrict__ recs, const int* __restrict__ offs,
+                                                         const float* __restrict__ bars, const int* __restrict__ offs,
                                                          const int* __restrict__ rev, uint32_t* __restrict__ pass,
                                                          uint16_t* __restrict__ bounds, int KP, int bpitch, int ksteps,
-                                                         float kappa, uint32_t div_m, int div_s,
+                                                         float kappa, float any_rel, float any_abs, uint32_t div_m, int div_s,
                                                          const int* __restrict__ order)
 {
     constexpr int kPieces = (kJwP + (NPW == 3 ? 128 : 256)) * 8 / 256;      // 16-byte pieces a thread stages per step
@@ -852,31 +885,33 @@ __global__ __launch_bounds__(256, NPW == 3 ? 3 : 1) void k_explore_join_wg(JoinC
     if (item >= N) return;                                                 // the whole workgroup leaves together
     const int q = order ? order[item] : item;
     const int r0 = offs[q], R = offs[q + 1] - r0;
-    if (R <= 0) return;
+    if (R <= kJwP * (int)blockIdx.y) return;
     const int MW = KP >> 5;
     const int nrows = kJwP + KP;
+    const float most_norm = jc.mu[jc.D + 1], most_err = jc.mu[jc.D + 2];
     for (int k = tid; k < KP; k += 256) {
         int c = k < K ? old_idx[(size_t)q * K + k] : -1;
         if (c < 0 || c >= N) c = -1;
         cq[k] = c;
-        cn[k] = c >= 0 ? recs[c].x : 0.0f;
-        cerr[k] = c >= 0 ? jc.errs[c] * kJoinUp : 0.0f;
+        const float n_c = c >= 0 ? jc.norms[c] : 0.0f;
+        cn[k] = n_c;
+        cerr[k] = join_err(n_c, any_rel, any_abs, most_err);
     }
-    for (int pg = 0; pg < R; pg += kJwP) {
+    for (int pg = kJwP * (int)blockIdx.y; pg < R; pg += kJwP * (int)gridDim.y) {
         const int npg = min(kJwP, R - pg);
         const int npairs = ((npg + 31) >> 5) * MW;
         __syncthreads();                                                   // the previous group is done with the LDS
         if (tid < kJwP) {
             const int e = tid < npg ? rev[(size_t)r0 + pg + tid] : -1;
             const int p = e >= 0 ? (int)(((uint64_t)div_m * (uint64_t)(uint32_t)e) >> div_s) : -1;
-            const float2 rec = p >= 0 ? recs[p] : make_float2(0.0f, 0.0f);
+            const float n_p = p >= 0 ? jc.norms[p] : 0.0f, bar = p >= 0 ? bars[p] : 0.0f;
             pid[tid] = p;
             pe[tid] = e;
-            pn[tid] = rec.x;
-            pbar[tid] = rec.y;
+            pn[tid] = n_p;
+            pbar[tid] = bar;
             if (BOUNDS) {
-                perr[tid] = p >= 0 ? jc.errs[p] : 0.0f;
-                pper[tid] = 65534.0f / join_span(rec);
+                perr[tid] = join_err(n_p, any_rel, any_abs, most_err);
+                pper[tid] = 65534.0f / join_span(bar, most_norm);
             }
         }
         __syncthreads();
@@ -1057,7 +1092,7 @@ int explore_ws_alloc(ExploreWorkspace** out, int N, int K, bool with_bounds, boo
     if (dm(&w->rev, total) != hipSuccess || dm(&w->bin_eq, 2 * total) != hipSuccess ||
         dm(&w->offs, (size_t)N + 1) != hipSuccess || dm(&w->bin_size, (size_t)w->n_bins) != hipSuccess ||
         dm(&w->bin_start, (size_t)w->n_bins + 1) != hipSuccess ||
-        dm(&w->part_off, (size_t)w->n_parts * (size_t)w->n_bins) != hipSuccess || (!graph_only && (dm(&w->pass, total * w->MW) != hipSuccess || dm(&w->recs, 2 * (size_t)N) != hipSuccess)) ||
+        dm(&w->part_off, (size_t)w->n_parts * (size_t)w->n_bins) != hipSuccess || (!graph_only && (dm(&w->pass, total * w->MW) != hipSuccess || dm(&w->bars, (size_t)N) != hipSuccess)) ||
         dm(&w->todo, 2 * ((size_t)N + 1)) != hipSuccess) {
         explore_ws_free(w);
         if (!graph_only) set_last_error("exploration workspace: out of device memory");
@@ -1078,7 +1113,7 @@ int explore_ws_alloc(ExploreWorkspace** out, int N, int K, bool with_bounds, boo
 void explore_ws_free(ExploreWorkspace* w)
 {
     if (!w) return;
-    void* bufs[] = {w->rev, w->bin_eq, w->offs, w->bin_size, w->bin_start, w->part_off, w->pass, w->recs, w->todo, w->bounds,
+    void* bufs[] = {w->rev, w->bin_eq, w->offs, w->bin_size, w->bin_start, w->part_off, w->pass, w->bars, w->todo, w->bounds,
                     w->bin_eq2, w->fine_size, w->fine_start, w->sub_off};
     for (void* b : bufs)
         ws_free(b);
@@ -1168,6 +1203,10 @@ int launch_explore_join(ExploreWorkspace* w, const JoinCopy& jc, int N, int D, i
 
     constexpr int kWaves = 4;
     const int KP = (K + 31) & ~31;
+    // A few points are in hundreds of rows, and a launch over few points ends with the tiles of these, one after the other: they are
+    // dealt out to several wavefronts (3,000 x 200, K = 30: 0.102 ms per pass with one, 0.029 with 16; 20,000 x 32 0.037, 0.038 with 3,
+    // 0.056 with 16; 1M x 256 7.0, 7.2 with 2).
+    const unsigned parts = (unsigned)std::max(1, std::min(16, 65536 / N));
     const int wave_ints = (KP + 192 + 3) & ~3;
     const size_t lds = (size_t)kWaves * (size_t)wave_ints * sizeof(int);
     const int ksteps = (D + 15) / 16;
@@ -1178,20 +1217,20 @@ int launch_explore_join(ExploreWorkspace* w, const JoinCopy& jc, int N, int D, i
     // rounding of any row: 2^-11 of a value, 2^-14 of one set to zero, and errs' own terms (3e-3 covers these and the root)
     const float any_rel = 1.003f / 2048.0f, any_abs = 1.001f * std::sqrt((float)D) / 16384.0f + 1e-6f;
     w->view.codes = w->bounds;
-    w->view.recs = w->recs;
-    w->view.errs = jc.errs;
-    w->view.scale = jc.scale(D);
+    w->view.bars = w->bars;
+    w->view.norms = jc.norms;
+    w->view.scale = jc.scale();
     w->view.kappa = kappa;
     w->view.one_minus_gamma = one_minus_gamma;
     w->view.any_rel = any_rel;
     w->view.any_abs = any_abs;
-    hipLaunchKernelGGL(k_join_records, dim3((unsigned)((N + 255) / 256) + 1), dim3(256), 0, stream, jc, jc.scale(D), knn_dist, N, K,
-                       one_minus_gamma, w->recs);
+    hipLaunchKernelGGL(k_join_bars, dim3((unsigned)((N + 255) / 256) + 1), dim3(256), 0, stream, jc, jc.scale(), knn_dist, N, K,
+                       one_minus_gamma, w->bars);
     RSFK_HIP(hipGetLastError());
     if (!w->bounds && KP == 32 && ksteps <= 8) {
-        const dim3 grid(grid_for_dies(((size_t)N + kWaves - 1) / kWaves)), block(64 * kWaves);
+        const dim3 grid(grid_for_dies(((size_t)N + kWaves - 1) / kWaves), parts), block(64 * kWaves);
 #define RSFK_JOIN_SHORT(KSV)                                                                                                \
-        hipLaunchKernelGGL((k_explore_join_short<kWaves, KSV>), grid, block, 0, stream, jc, N, K, old_idx, w->recs, w->offs, \
+        hipLaunchKernelGGL((k_explore_join_short<kWaves, KSV>), grid, block, 0, stream, jc, N, K, old_idx, w->bars, w->offs, \
                            w->rev, w->pass, join_pitch(D), ksteps, kappa, any_rel, any_abs, w->div_m, w->div_s, order)
         if (ksteps <= 2) RSFK_JOIN_SHORT(2);
         else if (ksteps <= 4) RSFK_JOIN_SHORT(4);
@@ -1205,9 +1244,9 @@ int launch_explore_join(ExploreWorkspace* w, const JoinCopy& jc, int N, int D, i
         do {                                                                                                               \
             RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_explore_join_wg<BV, NV>),                         \
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_wg));                       \
-            hipLaunchKernelGGL((k_explore_join_wg<BV, NV>), dim3(grid_for_dies((size_t)N)), dim3(256), lds_wg, stream, jc, N, K,  \
-                               old_idx, w->recs, w->offs, w->rev, w->pass, w->bounds, KP, join_pitch(D), ksteps, kappa,  \
-                               w->div_m, w->div_s, order);                                                \
+            hipLaunchKernelGGL((k_explore_join_wg<BV, NV>), dim3(grid_for_dies((size_t)N), parts), dim3(256), lds_wg, stream, jc, N, K,  \
+                               old_idx, w->bars, w->offs, w->rev, w->pass, w->bounds, KP, join_pitch(D), ksteps, kappa,  \
+                               any_rel, any_abs, w->div_m, w->div_s, order);                                                \
         } while (0)
         if (w->bounds && KP <= 128) RSFK_JOIN_WG(true, 3);
         else if (w->bounds) RSFK_JOIN_WG(true, 6);
@@ -1215,13 +1254,13 @@ int launch_explore_join(ExploreWorkspace* w, const JoinCopy& jc, int N, int D, i
         else RSFK_JOIN_WG(false, 6);
 #undef RSFK_JOIN_WG
     } else if (w->bounds)
-        hipLaunchKernelGGL((k_explore_join<kWaves, true>), dim3(grid_for_dies(((size_t)N + kWaves - 1) / kWaves)), dim3(64 * kWaves), lds,
-                           stream, jc, N, K, old_idx, w->recs, w->offs, w->rev, w->pass, w->bounds, KP, join_pitch(D), ksteps,
-                           kappa, wave_ints, w->div_m, w->div_s, order);
+        hipLaunchKernelGGL((k_explore_join<kWaves, true>), dim3(grid_for_dies(((size_t)N + kWaves - 1) / kWaves), parts), dim3(64 * kWaves), lds,
+                           stream, jc, N, K, old_idx, w->bars, w->offs, w->rev, w->pass, w->bounds, KP, join_pitch(D), ksteps,
+                           kappa, any_rel, any_abs, wave_ints, w->div_m, w->div_s, order);
     else
-        hipLaunchKernelGGL((k_explore_join<kWaves, false>), dim3(grid_for_dies(((size_t)N + kWaves - 1) / kWaves)), dim3(64 * kWaves), lds,
-                           stream, jc, N, K, old_idx, w->recs, w->offs, w->rev, w->pass, w->bounds, KP, join_pitch(D), ksteps,
-                           kappa, wave_ints, w->div_m, w->div_s, order);
+        hipLaunchKernelGGL((k_explore_join<kWaves, false>), dim3(grid_for_dies(((size_t)N + kWaves - 1) / kWaves), parts), dim3(64 * kWaves), lds,
+                           stream, jc, N, K, old_idx, w->bars, w->offs, w->rev, w->pass, w->bounds, KP, join_pitch(D), ksteps,
+                           kappa, any_rel, any_abs, wave_ints, w->div_m, w->div_s, order);
     RSFK_HIP(hipGetLastError());
     return 0;
 }

@@ -3,7 +3,7 @@
 // All lengths are in the units of the float16 copy (join_copy.hpp: s times those of the points).  For a pair (p, c) the join has
 // least = d~ - E1 <= d~(real) and t = max(0, sqrt(least) - e_p - e_c), a lower bound of the distance of the points.  Kept is
 //   code = 1 + min(65534, floor(65534 t / span_p)),   0: nothing is known (a row that is not finite),
-// span_p = the bar of point p (k_join_records), or four times its distance from the centre where its row is not full.  A code stands
+// span_p = the bar of point p (k_join_bars), or four times the largest distance from the centre where its row is not full.  A code stands
 // for an interval: the pair's exact distance (the fp32 chain) is at least what its lower end gives, and at most what its upper end
 // gives with the errors put on instead of taken off:
 //   sqrt(d~(real)) <= sqrt((t + e_p + e_c)^2 + 2 E1),   sqrt(d) <= that + e_p + e_c,   chain <= d (1 + gamma),
@@ -20,17 +20,23 @@ constexpr int kCodeTop = 65535;
 
 struct JoinBounds {
     const uint16_t* codes = nullptr;   // N*K*KP words by graph entry and neighbour slot, or null
-    const float2* recs = nullptr;      // norm and bar of a point (k_join_records)
-    const float* errs = nullptr;       // JoinCopy::errs
+    const float* bars = nullptr;       // bar of a point (k_join_bars)
+    const float* norms = nullptr;      // JoinCopy::norms
     const float* scale = nullptr;      // JoinCopy::scale: s, largest norm, largest error
     float kappa = 0.0f;                // E1 = kappa S
     float one_minus_gamma = 1.0f;
     float any_rel = 0.0f, any_abs = 0.0f;   // e <= any_rel |row| + any_abs of any row
 };
 
-__device__ __forceinline__ float join_span(float2 rec)
+__device__ __forceinline__ float join_span(float bar, float most_norm)
 {
-    return rec.y <= 3.0e38f ? rec.y : 4.0f * sqrtf(rec.x);
+    return bar <= 3.0e38f ? bar : 4.0f * sqrtf(most_norm);
+}
+
+// What the rounding of any row took at most, from the norm of the row and from the largest that was measured (most_err).
+__device__ __forceinline__ float join_err(float norm, float any_rel, float any_abs, float most_err)
+{
+    return fminf(__builtin_fmaf(any_rel, __builtin_amdgcn_sqrtf(norm), any_abs), most_err);
 }
 
 // per = 65534 / span
@@ -48,16 +54,15 @@ struct CodeReader {
 
     __device__ __forceinline__ CodeReader(const JoinBounds& b, int p)
     {
-        const float2 rec = b.recs[p];
-        const float span = join_span(rec), root = sqrtf(rec.x);
+        const float norm = b.norms[p], span = join_span(b.bars[p], b.scale[1]), root = sqrtf(norm);
         s = *b.scale;
         inv_s = 1.0f / s;
         omg = b.one_minus_gamma;
         per = 65534.0f / span;
         len = span / 65534.0f;
         const float far = fminf(root + 2.0f * span, sqrtf(b.scale[1]) * kJoinUp);        // lengths of other points
-        E = (b.errs[p] + fminf(b.any_rel * far + b.any_abs, b.scale[2])) * (1.0f + 1.0f / 131072.0f);
-        E1 = 2.0f * kJoinUp * b.kappa * (rec.x + far * far);
+        E = (join_err(norm, b.any_rel, b.any_abs, b.scale[2]) + fminf(b.any_rel * far + b.any_abs, b.scale[2])) * (1.0f + 1.0f / 131072.0f);
+        E1 = 2.0f * kJoinUp * b.kappa * (norm + far * far);
         if (!((span + E) * (span + E) + E1 < 3.9f * span * span)) E = INFINITY;       // (what it leads to does not stay within 2 span)
     }
     // a pair with a code above this has an exact distance above tau

@@ -200,6 +200,7 @@ __global__ __launch_bounds__(256) void k_to_join(const float* __restrict__ point
 
 int join_copy_alloc(JoinCopy* c, int N, int D)
 {
+    c->D = D;
     if (ws_alloc(reinterpret_cast<void**>(&c->mu), ((size_t)2 * D + 3) * sizeof(float))) return 1;
     if (ws_alloc(reinterpret_cast<void**>(&c->parts), kJoinMostGrid * sizeof(float2))) return 1;
     if (ws_alloc(reinterpret_cast<void**>(&c->rows), std::max<size_t>((size_t)N * join_pitch(D) * 2, 16))) return 1;

@@ -21,9 +21,10 @@ struct JoinCopy {
     float* norms = nullptr;       // N, in units of s^2
     float* errs = nullptr;        // N, in units of s
     float* mu = nullptr;          // column means, then (s, largest norm, largest error of the finite rows), then D words of working memory
-    float2* parts = nullptr;      // n_parts: largest norm and error of the finite rows a workgroup made (join_records completes them)
+    float2* parts = nullptr;      // n_parts: largest norm and error of the finite rows a workgroup made (k_join_bars completes them)
     int n_parts = 0;
-    float* scale(int D) const { return mu + D; }
+    int D = 0;
+    float* scale() const { return mu + D; }
 };
 
 int join_copy_alloc(JoinCopy* c, int N, int D);
