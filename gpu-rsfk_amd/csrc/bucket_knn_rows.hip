@@ -19,11 +19,9 @@
 //      ends, which at these dimensions costs less than carrying a distance matrix
 //      through LDS and a second visit of the rows;
 //   3. all candidates of a member are then offered to its row (knn_list.hpp), held
-//      in registers, and the row is stored if it changed.  When far more candidates
-//      are below the row's last slot than the row has slots, a histogram of their
-//      distances first removes those that cannot stay, and into a row that is new
-//      the rest is written by rank (counted, not inserted).  The K-NN rows of the
-//      next two members are requested before the chains of these two start.
+//      in registers, and the row is stored if it changed.  Where more than a few candidates are below
+//      the row's last slot (the first trees of a build) the two are merged by counting (place_young).
+//      The K-NN rows of the next two members are requested before the chains of these two start.
 //
 // No distance matrix, no flags, no barrier after the staging; a row is owned by
 // one wavefront (no locks).
@@ -43,11 +41,17 @@ constexpr int kRowsWaves = kRowsThreads / 64;
 constexpr int kRowsStep = 32;                 // dimensions of the two members held in registers at a time
 constexpr int kRowsLdsBytes = 40 * 1024;      // four workgroups per compute unit
 
+constexpr int kYoungLeast = 12;               // candidates below the last slot from which a row is merged by counting
+// Rows that are not new: in few dimensions most points of the second tree's bucket that are near enough are in the row already, and the
+// insertions drop those at little cost.  Calls of two trees of 1M points, buckets of 64..256, K = 32, before and with this: D = 2 3.82 and 3.65
+// ms (4.9 by counting alone), 4 4.17 and 3.87, 6 4.36 and 4.02, 8 4.47 and 3.81, 32 4.86 and 4.08.
+constexpr int kYoungDims = 6;
+
 // NT = tiles of 64 candidates: buckets of up to 64 NT points.  Buckets outside min_size..max_size are left alone.
-// DENSE: with the histogram step for members most of whose candidates are below the last slot (the first trees of a
-// build; the code costs the later ones a few per cent when it is merely present).
+// DENSE: with the merge by counting (the first trees of a build; the code costs the later ones a few per cent when it is merely
+// present).  Four wavefronts per SIMD: at three (130 registers) the first tree takes 11.7 ms, the second 13.0.
 template <int NT, bool DENSE>
-__global__ __launch_bounds__(kRowsThreads) void k_bucket_knn_rows(const float* __restrict__ points, int D, int K,
+__global__ __launch_bounds__(kRowsThreads, 4) void k_bucket_knn_rows(const float* __restrict__ points, int D, int K,
                                                                    const int* __restrict__ ids, const int* __restrict__ starts,
                                                                    const int* __restrict__ sizes, int stride, int min_size,
                                                                    int max_size, int* __restrict__ knn_idx,
@@ -86,6 +90,134 @@ __global__ __launch_bounds__(kRowsThreads) void k_bucket_knn_rows(const float* _
             rd = knn_dist[at];
         }
     };
+    // The row and its candidates by counting: false, with nothing done, where that does not pay or where more than 64 of them are
+    // left.  A histogram over 64 equal intervals of the distances of the candidates below the last slot and of the row's entries
+    // tells in which interval the K-th smallest lies; what is in later intervals has K others below it and cannot stay.  What is left
+    // is put in the order of the intervals (a counting sort in LDS), and its place inside its interval found by looking at the
+    // few others there.  Candidates that are points of the row already are found by a filter of 2,048 bits over the row's ids.
+    // (10M x 32, buckets of 64..256: first tree 12.2 -> 10.6 ms, second, whose rows
+    // used to take insertions, 14.1 -> 9.2; 530 and 470 vector instructions per point, 190 of them the chains.)
+    auto place_young = [&](int m, int ri, float rd, const KnnRow<1>& row, bool (&ok)[NT], const float (&acc)[NT]) -> bool {
+        bool in[NT];
+        int n_in = 0;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            // (no NaN and no infinite distance; one at the last slot may have the smaller index)
+            in[t] = ok[t] && acc[t] <= row.tau && acc[t] < INFINITY;
+            n_in += __popcll(ballot64(in[t]));
+        }
+        if (n_in < kYoungLeast || row.changed) return false;          // (a row that had to be put in order is stored whole)
+        const bool mine = lane < K && row.idx[0] >= 0 && row.dist[0] < INFINITY;
+        const int n_row = __popcll(ballot64(mine));
+        const bool insert = n_row > 1 && D < kYoungDims;             // the histogram of the candidates alone, then insertions
+        if (insert && n_in <= K + 16) return false;
+        if (ballot64(lane < K && row.idx[0] >= 0 && !mine) != 0) return false;
+        // the intervals: from the least of them to the last slot of a full row, or to the mean of the candidates (to the largest, where
+        // fewer than K are below the mean); what is beyond is in the last one
+        float lo = n_row > 1 && lane > 0 && mine ? row.dist[0] : INFINITY, sum = 0.0f;      // (not the point itself, which is at 0)
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+            if (in[t]) { lo = fminf(lo, acc[t]); sum += acc[t]; }
+        lo = -wave_max(-lo);
+        float hi = row.tau;
+        if (!(hi < INFINITY)) {
+            hi = wave_total_f(sum) * __builtin_amdgcn_rcpf((float)n_in);
+            int n_below = n_row;
+#pragma unroll
+            for (int t = 0; t < NT; ++t) n_below += __popcll(ballot64(in[t] && acc[t] < hi));
+            if (n_below < K + 8) {
+                hi = mine ? row.dist[0] : 0.0f;
+#pragma unroll
+                for (int t = 0; t < NT; ++t)
+                    if (in[t]) hi = fmaxf(hi, acc[t]);
+                hi = wave_max(hi);
+            }
+        }
+        if (!(hi > lo)) return false;
+        const float scale = 63.5f / (hi - lo);
+        auto bin_of = [&](float d) { return min(63, (int)(fmaxf(d - lo, 0.0f) * scale)); };   // does not decrease when the distance grows
+        wave_lds_sync();
+        hist[lane] = 0;
+        wave_lds_sync();
+        int bin[NT];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            bin[t] = bin_of(acc[t]);
+            if (in[t]) atomicAdd(&hist[bin[t]], 1);
+        }
+        const int bin_row = bin_of(row.dist[0]);
+        if (mine && !insert) atomicAdd(&hist[bin_row], 1);
+        wave_lds_sync();
+        const int h = hist[lane];
+        const int before = wave_excl_scan_i(h);
+        const int all = n_in + n_row;
+        const int need = insert ? K : min(all, K + (n_row > 1 ? 4 : 0));      // (some may be there twice)
+        const int cross = first_lane(ballot64(before + h >= need));
+        const int n_left = read_lane_i(before + h, cross);
+        if (insert || n_left > 64) {
+            // (insertions, of those that can stay)
+            if (insert || n_row <= 1)
+#pragma unroll
+                for (int t = 0; t < NT; ++t) ok[t] = in[t] && bin[t] <= cross;
+            return false;
+        }
+        wave_lds_sync();
+        hist[lane] = before;
+        wave_lds_sync();
+        constexpr int kOfRow = (int)0x80000000;
+        int2* left = reinterpret_cast<int2*>(hist + 64);              // (distance, id, with kOfRow for the row's own)
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+            if (in[t] && bin[t] <= cross) left[atomicAdd(&hist[bin[t]], 1)] = make_int2(__float_as_int(acc[t]), cid[t]);
+        if (mine && bin_row <= cross) left[atomicAdd(&hist[bin_row], 1)] = make_int2(__float_as_int(row.dist[0]), row.idx[0] | kOfRow);
+        wave_lds_sync();
+        const bool here = lane < n_left;
+        const int2 v = here ? left[lane] : make_int2(0x7f800000, kOfRow);
+        const float d = __int_as_float(v.x);
+        const int c = v.y & ~kOfRow;
+        const int b = here ? bin_of(d) : 0;
+        int i = here && b > 0 ? hist[b - 1] : 0;                      // (hist: where the intervals end)
+        const int end = here ? hist[b] : 0;
+        int rank = i;
+        while (ballot64(i < end) != 0) {
+            if (i < end) {
+                const int2 o = left[i];
+                rank += pair_above(d, c, __int_as_float(o.x), o.y & ~kOfRow) ? 1 : 0;
+                ++i;
+            }
+        }
+        // candidates that are in the row: the filter first, then the row's ids
+        bool twice = false;
+        if (n_row > 1) {
+            auto bit_of = [](int id) { return (id ^ (id >> 11)) & 2047; };
+            wave_lds_sync();
+            hist[lane] = 0;
+            wave_lds_sync();
+            if (mine) atomicOr(&hist[bit_of(row.idx[0]) >> 5], 1 << (bit_of(row.idx[0]) & 31));
+            wave_lds_sync();
+            uint64_t maybe = ballot64(v.y >= 0 && ((hist[bit_of(c) >> 5] >> (bit_of(c) & 31)) & 1));
+            while (maybe) {
+                const int j = first_lane(maybe);
+                maybe &= maybe - 1;
+                const int cj = read_lane_i(c, j);
+                const bool held = ballot64(mine && row.idx[0] == cj) != 0;
+                twice |= held && lane == j;
+            }
+        }
+        uint64_t again = ballot64(twice);
+        if (n_left < all && n_left - __popcll(again) < K) return false;       // (so many twice that the interval was too early)
+        while (again) {
+            const int j = first_lane(again);
+            again &= again - 1;
+            rank -= pair_above(d, c, read_lane_f(d, j), read_lane_i(c, j)) ? 1 : 0;
+        }
+        if (here && !twice && rank < K) {
+            const size_t to = (size_t)lids[m] * (size_t)K + rank;
+            knn_idx[to] = c;
+            knn_dist[to] = d;
+        }
+        return true;
+    };
     auto finish = [&](int m, int ri, float rd, const float (&acc)[NT]) {
         KnnRow<1> row;
         row.idx[0] = ri;
@@ -95,91 +227,7 @@ __global__ __launch_bounds__(kRowsThreads) void k_bucket_knn_rows(const float* _
         bool ok[NT];
 #pragma unroll
         for (int t = 0; t < NT; ++t) ok[t] = t < nt && cid[t] >= 0 && 64 * t + lane != m;
-        // the first 64 candidates tell whether most candidates are below the row's last slot
-        // (the histogram below only ever sees candidates that passed enters(): a NaN distance would otherwise land in
-        // its first interval and push finite candidates out)
-        int n_ok = DENSE ? __popcll(ballot64(ok[0] && row.enters(cid[0], acc[0]))) : 0;
-        if (DENSE && n_ok > min(40, K + 16)) {
-            n_ok = 0;
-#pragma unroll
-            for (int t = 0; t < NT; ++t) {
-                ok[t] = ok[t] && row.enters(cid[t], acc[t]);
-                n_ok += __popcll(ballot64(ok[t]));
-            }
-        }
-        if (DENSE && n_ok > K + 16) {
-            // Many more candidates below the last slot than the row has slots (rows that are new or far from done):
-            // inserting them one after the other would push most of them out again.  A histogram of their distances
-            // over 64 equal intervals tells in which interval the K-th smallest lies; a candidate in a later interval
-            // has K candidates below it and cannot stay in the row, so it is not inserted at all.
-            float lo = INFINITY, hi = 0.0f;
-#pragma unroll
-            for (int t = 0; t < NT; ++t)
-                if (ok[t]) { lo = fminf(lo, acc[t]); hi = fmaxf(hi, acc[t]); }
-            lo = -wave_max(-lo);
-            hi = wave_max(hi);
-            if (hi > lo) {
-                const float scale = 63.5f / (hi - lo);
-                wave_lds_sync();
-                hist[lane] = 0;
-                wave_lds_sync();
-                int bin[NT];
-#pragma unroll
-                for (int t = 0; t < NT; ++t) {
-                    bin[t] = min(63, max(0, (int)((acc[t] - lo) * scale)));       // does not decrease when the distance grows
-                    if (ok[t]) atomicAdd(&hist[bin[t]], 1);
-                }
-                wave_lds_sync();
-                const int h = hist[lane];
-                const int upto = wave_excl_scan_i(h) + h;
-                const int cross = first_lane(ballot64(upto >= K));
-#pragma unroll
-                for (int t = 0; t < NT; ++t) ok[t] = ok[t] && bin[t] <= cross;
-            }
-        }
-        if (DENSE && n_ok > 0 && small_bucket::fresh_row(ri, rd, lids[m], K)) {
-            // A new row (nothing in it but, possibly, the point itself): the candidates that are left are not inserted
-            // one after the other -- their places in the row are their ranks among themselves.  They are gathered in
-            // lanes 0.. (through LDS), ranked by counting, and stored where they belong.
-            const bool has_self = read_lane_i(ri, 0) >= 0;
-            int n_left = has_self ? 1 : 0;
-#pragma unroll
-            for (int t = 0; t < NT; ++t) n_left += __popcll(ballot64(ok[t] && row.enters(cid[t], acc[t])));
-            if (n_left <= 64) {
-                float* cd = reinterpret_cast<float*>(hist + 64);
-                int* ci = hist + 128;
-                wave_lds_sync();
-                int at = 0;
-                if (has_self) {
-                    if (lane == 0) { cd[0] = rd; ci[0] = ri; }
-                    at = 1;
-                }
-#pragma unroll
-                for (int t = 0; t < NT; ++t) {
-                    const bool in = ok[t] && row.enters(cid[t], acc[t]);
-                    const uint64_t mk = ballot64(in);
-                    if (in) {
-                        const int p = at + mask_prefix(mk);
-                        cd[p] = acc[t];
-                        ci[p] = cid[t];
-                    }
-                    at += __popcll(mk);
-                }
-                wave_lds_sync();
-                const float d = lane < n_left ? cd[lane] : INFINITY;
-                const int c = lane < n_left ? ci[lane] : -1;
-                float place[1] = {d};
-                if (small_bucket::place_by_rank<1>(place, n_left)) {          // (not with equal distances: those take the usual way)
-                    const int slot = __float_as_int(place[0]);
-                    if (slot >= 0 && slot < K) {
-                        const size_t to = (size_t)lids[m] * (size_t)K + slot;
-                        knn_idx[to] = c;
-                        knn_dist[to] = d;
-                    }
-                    return;
-                }
-            }
-        }
+        if (DENSE && place_young(m, ri, rd, row, ok, acc)) return;
         // tile after tile: the last slot a tile leaves behind already turns away candidates of the next
 #pragma unroll
         for (int t = 0; t < NT; ++t)

@@ -81,6 +81,15 @@ __device__ __forceinline__ float half_butterfly_sum(float v)
 }
 
 // maximum over all 64 lanes, returned in every lane (wave-uniform value)
+__device__ __forceinline__ float wave_total_f(float v)
+{
+    v += dpp_f<kDppXor1>(v);
+    v += dpp_f<kDppXor2>(v);
+    v += dpp_f<kDppHalfMirror>(v);
+    v += dpp_f<kDppMirror>(v);
+    return (read_lane_f(v, 0) + read_lane_f(v, 16)) + (read_lane_f(v, 32) + read_lane_f(v, 48));
+}
+
 __device__ __forceinline__ float wave_max(float v)
 {
     v = fmaxf(v, dpp_f<kDppXor1>(v));
@@ -142,13 +151,14 @@ __device__ __forceinline__ uint32_t wave_or_u32(uint32_t x)
 // exclusive prefix sum over the lanes of the wavefront
 __device__ __forceinline__ int wave_excl_scan_i(int v)
 {
-    const int lane = lane_id();
+    // inside the rows of 16 lanes, then lane 15 of a row into the next, then lane 31 into the upper half (DPP; lanes out of reach add 0)
     int incl = v;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const int t = __shfl_up(incl, o, 64);
-        if (lane >= o) incl += t;
-    }
+    incl += __builtin_amdgcn_update_dpp(0, incl, 0x111, 0xf, 0xf, false);        // row_shr:1, 2, 4, 8
+    incl += __builtin_amdgcn_update_dpp(0, incl, 0x112, 0xf, 0xf, false);
+    incl += __builtin_amdgcn_update_dpp(0, incl, 0x114, 0xf, 0xf, false);
+    incl += __builtin_amdgcn_update_dpp(0, incl, 0x118, 0xf, 0xf, false);
+    incl += __builtin_amdgcn_update_dpp(0, incl, 0x142, 0xa, 0xf, false);        // row_bcast:15 into rows 1 and 3
+    incl += __builtin_amdgcn_update_dpp(0, incl, 0x143, 0xc, 0xf, false);        // row_bcast:31 into rows 2 and 3
     return incl - v;
 }
 

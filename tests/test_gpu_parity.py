@@ -344,6 +344,39 @@ def test_bucket_knn_rows_that_start_new(gpu, orc, rng, start, data, K):
         assert rows_have_no_duplicates(gi)
 
 
+@pytest.mark.parametrize("data", ["continuous", "grid", "mixed", "notfinite"])
+@pytest.mark.parametrize("start", ["self", "empty", "self_far"])
+@pytest.mark.parametrize("K,MIN,MAX", [(8, 40, 120), (32, 64, 256), (60, 61, 200), (64, 33, 190)])
+def test_bucket_knn_resident_rows_merged_by_counting(gpu, orc, rng, K, MIN, MAX, start, data):
+    """Buckets of 73..256 points whose rows are merged by counting: rows that are new, rows of which most points are in the bucket
+    again (the same partition twice), rows that are neither new nor full, equal distances, duplicated points, points that are not
+    finite, and rows too long for one wavefront to count."""
+    N, D = 4000, 5
+    X = rng.standard_normal((N, D)).astype(np.float32)
+    perm, ls, lz, _ = orc.build_tree(X, MIN, MAX, 5000, 3)
+    parts = [(perm, ls, lz), (perm, ls, lz), orc.build_tree(X, MIN, MAX, 5000, 4)[:3]]
+    if data == "grid":
+        X = rng.integers(0, 3, (N, D)).astype(np.float32)
+    elif data == "mixed":
+        some = rng.random(N) < 0.1
+        X[some] = rng.integers(0, 2, (int(some.sum()), D)).astype(np.float32)
+    elif data == "notfinite":
+        X[rng.integers(0, N, 30), rng.integers(0, D, 30)] = np.nan
+        X[rng.integers(0, N, 30), 0] = np.inf
+    oi = np.full((N, K), -1, np.int32)
+    od = np.full((N, K), np.inf, np.float32)
+    if start != "empty":
+        oi[:, 0] = np.arange(N)
+        od[:, 0] = 0.0 if start == "self" else 0.3
+    gi, gd = oi.copy(), od.copy()
+    for perm, ls, lz in parts:
+        _say("bucket_knn by counting", K, MIN, MAX, start, data)
+        orc.bucket_knn(X, K, perm, lz, oi, od, starts=ls)
+        gpu.bucket_knn(X, K, perm, lz, gi, gd, starts=ls)
+        assert_knn_equal(gi, gd, oi, od)
+        assert rows_have_no_duplicates(gi)
+
+
 def test_bucket_knn_single_bucket_is_exact_knn(gpu, rng):
     """One bucket holding every point: the kernel must return exact K-NN."""
     for N, D, K in [(300, 8, 16), (700, 20, 32)]:
