@@ -52,12 +52,11 @@ __global__ __launch_bounds__(256) void k_zero_ints(int* __restrict__ p, int n)
 // [offset, 0, 0, 0 | normal, zero padded to a multiple of 4].  Normal and offset are the values the builder works with
 // (create_node.cu:122-135: n = x1 - x2, offset = sum n_d (x1_d + x2_d) / 2 as 32 lane-strided partial sums + xor butterfly).
 // blockIdx.y: the tree; the records and the rows of a tree begin rec_cap after those of the tree before it.
-// low (null: none): the rows the queries are routed by first, low_pitch floats each: {offset, E, children | normal rounded to
-// bfloat16}, E = (|n - n~| + 2.1 gamma |n|)(1 + 2^-9) with the rounding error as it is and gamma for the fp32 sums of either
-// evaluation: |n.x as the builder sums it - n~.x as k_route sums it| <= E |x|.  A bucket has children -1.
+// low (null: none): the rows the queries are routed by first, low_pitch floats each: {-b~ (NaN: never certain), 0, children | n~}
+// (SideBound, ann.hpp; mu, scale: of the copy of the queries).  A bucket has children -1.
 __global__ __launch_bounds__(256) void k_planes(const float* __restrict__ points, int D, const TreeRec* __restrict__ recs,
                                                 const int* __restrict__ n_rec_p, int rec_cap, float* __restrict__ planes,
-                                                int pitch, float* __restrict__ low, int low_pitch)
+                                                int pitch, float* __restrict__ low, int low_pitch, const float* __restrict__ mu, const float* __restrict__ scale)
 {
     const int lane = threadIdx.x & 63;
     const int r = blockIdx.x * 4 + (threadIdx.x >> 6), j = blockIdx.y;
@@ -83,28 +82,13 @@ __global__ __launch_bounds__(256) void k_planes(const float* __restrict__ points
     }
     s = half_butterfly_sum(s);
     if (lane < 4) row[lane] = lane == 0 ? s : 0.0f;
-    float err2 = 0.0f, nrm2 = 0.0f;
-    uint16_t* low_n = low ? reinterpret_cast<uint16_t*>(low_row + 4) : nullptr;
-    for (int d = lane; d < pitch - 4; d += 64) {
-        const float nd = d < D ? x1[d] - x2[d] : 0.0f;
-        row[4 + d] = nd;
-        if (low) {
-            const __bf16 h = (__bf16)nd;
-            const float e = nd - (float)h;
-            err2 = __builtin_fmaf(e, e, err2);
-            nrm2 = __builtin_fmaf(nd, nd, nrm2);
-            low_n[d] = __builtin_bit_cast(uint16_t, h);
-        }
-    }
+    for (int d = lane; d < pitch - 4; d += 64) row[4 + d] = d < D ? x1[d] - x2[d] : 0.0f;
     if (!low) return;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        err2 += __shfl_xor(err2, o, 64);
-        nrm2 += __shfl_xor(nrm2, o, 64);
-    }
-    const float gamma = (float)(D + 64) * (1.0f / 8388608.0f);
-    const float E = (sqrtf(err2) + 2.1f * gamma * sqrtf(nrm2)) * (1.0f + 1.0f / 512.0f) + 2e-17f;     // (squares that underflow)
-    if (lane == 0) *reinterpret_cast<int4*>(low_row) = make_int4(__float_as_int(s), __float_as_int(E), rec.c0, rec.c1);
+    const RoundedPlane pl = rounded_plane(x1, x2, D, __shfl(s, 0, 64), mu, *scale);
+    uint16_t* low_n = reinterpret_cast<uint16_t*>(low_row + 4);
+    for (int d = lane; d < ((D + 7) & ~7); d += 64) low_n[d] = rounded_value(d < D ? x1[d] - x2[d] : 0.0f, pl);
+    if (lane == 0)
+        *reinterpret_cast<int4*>(low_row) = make_int4(__float_as_int(pl.sound ? -pl.b : __builtin_nanf("")), 0, rec.c0, rec.c1);
 }
 
 // Eight lanes per query.  A lane owns four of the 32 partial sums of the side test (sums 4s..4s+3 of
@@ -117,8 +101,8 @@ constexpr int kXR = 4;
 template <bool VEC, bool FOREST>
 __global__ __launch_bounds__(256) void k_route(const float* __restrict__ planes, int pitch, const float* __restrict__ queries,
                                                int NQ, int D, const TreeRec* __restrict__ recs, int max_steps,
-                                               int* __restrict__ q_rec, int* __restrict__ q_rank, int* __restrict__ cnt, int cnt_shift,
-                                               int2* __restrict__ reached)
+                                               const int* __restrict__ start, int* __restrict__ q_rec, int* __restrict__ q_rank, int* __restrict__ cnt,
+                                               int cnt_shift, int2* __restrict__ reached)
 {
     if (FOREST) {
         recs += (size_t)blockIdx.y * (size_t)max_steps;         // (max_steps: the records a tree has room for)
@@ -132,7 +116,7 @@ __global__ __launch_bounds__(256) void k_route(const float* __restrict__ planes,
     float4 xr[kXR];
 #pragma unroll
     for (int k = 0; k < kXR; ++k) xr[k] = load_piece(x, 32 * k + 4 * sub, D, VEC);
-    int cur = 0;
+    int cur = start && valid ? start[q] : 0;             // (where the first levels have been taken already: ann_top.hip)
     bool done = !valid;
     for (int step = 0; step <= max_steps; ++step) {          // a path is never longer than the number of records
         const int at = done ? 0 : cur;
@@ -184,85 +168,75 @@ __global__ __launch_bounds__(256) void k_route(const float* __restrict__ planes,
     }
 }
 
-// The same for many queries of 65 to 128 dimensions, by the rounded hyperplanes of k_planes: the side is certain when
-// |n~.x - offset| > E |x|, otherwise (1 % of the tests on uniform points) the exact test follows.  Sums of squares that
-// overflow, infinities and NaN leave a test uncertain.
-// k_route is bound by the hyperplanes' bytes from beyond the L2 (16 MB a tree at 1M x 100; 2.4 GB fetched at 4.3 TB/s); these are half as
-// many: 1M queries 0.56 -> 0.49 ms a tree, 1.3 GB at 2.6 TB/s and bound by instruction issue (vector ALUs 71 % busy).  Rows of up to 64 dimensions gain nothing (500,000 / 100,000 x 64: search 8.25 -> 8.21 ms) or lose
-// (1M / 1M x 16 14.1 -> 14.6), and so do few queries, for which the second trip counts (20,000 / 1M x 100, 50 trees
-// 8.65 -> 9.01 ms, 100,000, 20 trees 6.91 -> 6.82).
-template <bool VEC>
+// The same for many queries of up to 128 dimensions, by the rounded hyperplanes of k_planes and the rounded queries of jc, 8 NH dimensions per
+// lane and two per instruction (v_dot2_f32_f16); a test that is not certain is taken exactly.
+// Bound by the hyperplanes that miss the L2 (4.3 TB/s of them, vector ALUs half busy), hence their two cache lines.  1M queries, a tree
+// of 1M x 100: 0.48 ms with bfloat16 hyperplanes, fp32 queries and all levels, 0.27 where ann_top.hip has taken the first seven.  Tried:
+// the queries of a subtree on one die (misses 9.4 -> 5.4 million lines, but the queries come in no order then: 0.44).
+template <int NH>
 __global__ __launch_bounds__(256) void k_route_low(const float* __restrict__ planes, int pitch, const float* __restrict__ low, int low_pitch,
-                                                   const float* __restrict__ queries, int NQ, int D, int rec_cap,
+                                                   const float* __restrict__ queries, JoinCopy jc, const float* __restrict__ scale,
+                                                   const float* __restrict__ mu_len, SideBound sb, int NQ, int D, bool vec, int rec_cap, const int* __restrict__ start,
                                                    int* __restrict__ q_rec, int* __restrict__ q_rank, int* __restrict__ cnt, int cnt_shift)
 {
+    typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
     const int sub = threadIdx.x & 7;
     const int q = (int)((blockIdx.x * (size_t)blockDim.x + threadIdx.x) >> 3);
     const bool valid = q < NQ;
-    const float* x = queries + (size_t)(valid ? q : 0) * (size_t)D;
-    const int Dp = pitch - 4;
-    float4 xr[kXR];
-    float norm = 0.0f;
+    const size_t at_q = (size_t)(valid ? q : 0);
+    const int pieces = (D + 7) >> 3, Dp = pitch - 4;
+    uint4 x[NH];
 #pragma unroll
-    for (int k = 0; k < kXR; ++k) {
-        xr[k] = load_piece(x, 32 * k + 4 * sub, D, VEC);
-        norm = __builtin_fmaf(xr[k].x, xr[k].x, norm);
-        norm = __builtin_fmaf(xr[k].y, xr[k].y, norm);
-        norm = __builtin_fmaf(xr[k].z, xr[k].z, norm);
-        norm = __builtin_fmaf(xr[k].w, xr[k].w, norm);
-    }
+    for (int k = 0; k < NH; ++k)
+        x[k] = NH * sub + k < pieces ? *reinterpret_cast<const uint4*>(jc.rows + at_q * (size_t)join_pitch(D) + 8 * (NH * sub + k)) : make_uint4(0, 0, 0, 0);
+    const float Z = sb.query(jc.norms[at_q], jc.errs[at_q], *scale, *mu_len);
     auto group_sum = [](float t) {                       // the last three steps of the butterfly, over the eight lanes
         t += dpp_f<kDppXor1>(t);
         t += dpp_f<kDppXor2>(t);
         t += dpp_f<kDppHalfMirror>(t);
         return t;
     };
-    norm = sqrtf(group_sum(norm)) * (1.0f + 1.0f / 512.0f) + 2e-17f;
-    int cur = 0;
+    int cur = start && valid ? start[q] : 0;             // (where the first levels have been taken already: ann_top.hip)
     bool done = !valid;
     for (int step = 0; step <= rec_cap; ++step) {            // a path is never longer than the number of records
         const float* lrow = low + (size_t)(done ? 0 : cur) * (size_t)low_pitch;
         const int4 head = *reinterpret_cast<const int4*>(lrow);
-        uint2 h[kXR];
+        uint4 n[NH];
 #pragma unroll
-        for (int k = 0; k < kXR; ++k) {
-            const int d = 32 * k + 4 * sub;
-            h[k] = d < Dp ? *reinterpret_cast<const uint2*>(lrow + 4 + (d >> 1)) : make_uint2(0u, 0u);
-        }
-        float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
+        for (int k = 0; k < NH; ++k)
+            n[k] = NH * sub + k < pieces ? *reinterpret_cast<const uint4*>(lrow + 4 + 4 * (NH * sub + k)) : make_uint4(0, 0, 0, 0);
+        float t0 = 0.0f, t1 = 0.0f;
+        auto dot = [](uint32_t a, uint32_t b, float c) {
+            return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, a), __builtin_bit_cast(f16x2, b), c, false);
+        };
 #pragma unroll
-        for (int k = 0; k < kXR; ++k) {
-            s0 = __builtin_fmaf(__uint_as_float(h[k].x << 16), xr[k].x, s0);
-            s1 = __builtin_fmaf(__uint_as_float(h[k].x & 0xffff0000u), xr[k].y, s1);
-            s2 = __builtin_fmaf(__uint_as_float(h[k].y << 16), xr[k].z, s2);
-            s3 = __builtin_fmaf(__uint_as_float(h[k].y & 0xffff0000u), xr[k].w, s3);
+        for (int k = 0; k < NH; ++k) {
+            t0 = dot(n[k].x, x[k].x, t0);
+            t1 = dot(n[k].y, x[k].y, t1);
+            t0 = dot(n[k].z, x[k].z, t0);
+            t1 = dot(n[k].w, x[k].w, t1);
         }
-        const float t = group_sum((s0 + s1) + (s2 + s3));
-        const float b = __int_as_float(head.x);
+        const float mb = __int_as_float(head.x), t = group_sum(t0 + t1) + mb;
         const bool bucket = head.z < 0;
-        bool below = t < b;
-        // (below 1e33 the bound, at least 2 gamma |n| |x|, leaves no room for a sum that overflows)
-        const float margin = fabsf(t - b), bound = __builtin_fmaf(__int_as_float(head.y), norm, 1e-35f);
-        const bool certain = margin > bound && margin < INFINITY && bound < 1e33f;
+        bool below = t < 0.0f;
+        const bool certain = fabsf(t) > __builtin_fmaf(fabsf(mb), sb.of_offset(), Z);        // (not with a NaN)
         const bool ask = !done && !bucket && !certain;       // (the eight lanes of a query agree)
         if (ballot64(ask) != 0) {
-            const float* pl = planes + (size_t)(ask ? cur : 0) * (size_t)pitch + 4;
-            s0 = s1 = s2 = s3 = 0.0f;
-            float4 n4[kXR];
+            const float* pl = planes + (size_t)(ask ? cur : 0) * (size_t)pitch;
+            const float* xq = queries + at_q * (size_t)D;
+            float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
 #pragma unroll
             for (int k = 0; k < kXR; ++k) {
                 const int d = 32 * k + 4 * sub;
-                n4[k] = ask && d < Dp ? *reinterpret_cast<const float4*>(pl + d) : make_float4(0.f, 0.f, 0.f, 0.f);
-            }
-#pragma unroll
-            for (int k = 0; k < kXR; ++k) {
-                s0 = __builtin_fmaf(n4[k].x, xr[k].x, s0);
-                s1 = __builtin_fmaf(n4[k].y, xr[k].y, s1);
-                s2 = __builtin_fmaf(n4[k].z, xr[k].z, s2);
-                s3 = __builtin_fmaf(n4[k].w, xr[k].w, s3);
+                const float4 n4 = ask && d < Dp ? *reinterpret_cast<const float4*>(pl + 4 + d) : make_float4(0.f, 0.f, 0.f, 0.f);
+                const float4 x4 = ask ? load_piece(xq, d, D, vec) : make_float4(0.f, 0.f, 0.f, 0.f);
+                s0 = __builtin_fmaf(n4.x, x4.x, s0);
+                s1 = __builtin_fmaf(n4.y, x4.y, s1);
+                s2 = __builtin_fmaf(n4.z, x4.z, s2);
+                s3 = __builtin_fmaf(n4.w, x4.w, s3);
             }
             const float exact = group_sum((s0 + s1) + (s2 + s3));
-            if (ask) below = exact < b;
+            if (ask) below = exact < pl[0];
         }
         if (!done) {
             if (bucket) {
@@ -617,13 +591,16 @@ namespace {
 
 // floats per row of the table of hyperplanes: offset (4 floats) + normal padded to a multiple of 4
 int plane_pitch(int D) { return 4 + ((D + 3) & ~3); }
-// ... of the rounded ones; 0: not made (see k_route_low).  RSFK_ANN_ROUTE_LOW=1 / 0 says yes or no.
-int low_plane_pitch(int NQ, int D)
+// ... of the rounded ones; 0: not made (see k_route_low).  RSFK_ANN_ROUTE_LOW=1 / 0 says yes or no.  Making them costs with the points,
+// what they give comes with the queries and the dimensions (20 trees, without -> with): 300,000 / 300,000 x 128 13.9 -> 13.3 ms, x 50 9.41 -> 9.27,
+// x 20 7.66 -> 7.65, x 8 7.67 -> 7.61; 60,000 points, 1M queries x 50 19.1 -> 18.8, x 20 14.8 -> 14.9; 1M points, 100,000 queries x 128
+// 20.3 -> 20.0, x 50 13.5 -> 13.6; 50,000 queries and fewer the same.
+int low_plane_pitch(int N, int NQ, int D)
 {
     if (D > 32 * kXR) return 0;
     const char* e = std::getenv("RSFK_ANN_ROUTE_LOW");
-    const bool wanted = e && *e ? e[0] == '1' : D > 64 && NQ >= 100000;
-    return wanted ? 4 + ((D + 7) & ~7) / 2 : 0;
+    const bool wanted = e && *e ? e[0] == '1' : NQ >= 100000 && (D > 64 || (D > 32 && (long long)NQ * 4 >= N));
+    return wanted ? (16 + 2 * ((D + 7) & ~7) + 63) / 64 * 16 : 0;         // (whole pieces of 64 bytes)
 }
 
 // Atomics on one cache line are carried out one after the other, about 14 ns each, and every query is counted by one: with few
@@ -640,7 +617,8 @@ int count_shift(int rec_cap)
 }  // namespace
 
 // floats of working memory a record of a tree takes (both tables of hyperplanes)
-int ann_plane_pitch(int NQ, int D) { return plane_pitch(D) + low_plane_pitch(NQ, D); }
+int ann_plane_pitch(int N, int NQ, int D) { return plane_pitch(D) + low_plane_pitch(N, NQ, D); }
+bool ann_low_wanted(int N, int NQ, int D) { return low_plane_pitch(N, NQ, D) > 0; }
 
 size_t ann_ws_ints(int NQ, int rec_cap)
 {
@@ -690,10 +668,11 @@ int launch_ann_ws_init(int* ws, int NQ, int rec_cap, unsigned long long* stats, 
 // One tree of the query-set search: routes the queries through the index recs (*n_rec_dev records, at most rec_cap;
 // the tree has n_leaves buckets), groups them by bucket and offers the base points perm[..] of the bucket a query
 // reached to the query's row.  prev, stats: numbers of pairs of the tree before this one (null: the first) and of this one,
-// kAnnStatWords each.  ws: ann_ws_ints(NQ, rec_cap) ints, prepared by launch_ann_ws_init; planes: rec_cap
-// ann_plane_pitch(NQ, D) floats.
+// kAnnStatWords each.  q_copy: null, or the copy of the queries.  start: the records from which the queries go on (null: the root).  ws: ann_ws_ints(NQ, rec_cap) ints, prepared by launch_ann_ws_init; planes: rec_cap
+// ann_plane_pitch(N, NQ, D) floats and 256 bytes.
 int launch_ann_tree(const float* points, const float* queries, int N, int NQ, int D, int K, const int* perm, const TreeRec* recs,
-                    const int* n_rec_dev, int rec_cap, int n_leaves, int* ws, float* planes, int* q_idx, float* q_dist,
+                    const int* n_rec_dev, int rec_cap, int n_leaves, const JoinCopy* q_copy, const int* start,
+                    int* ws, float* planes, int* q_idx, float* q_dist,
                     const unsigned long long* prev, unsigned long long* stats, hipStream_t stream)
 {
     if (NQ <= 0) return 0;
@@ -709,24 +688,24 @@ int launch_ann_tree(const float* points, const float* queries, int N, int NQ, in
     int4* blk_desc = reinterpret_cast<int4*>(ws + (((boff + rec_cap + 1) - ws + 3) & ~(ptrdiff_t)3));
     int* n_blocks = reinterpret_cast<int*>(blk_desc + ((size_t)NQ / kQB + rec_cap + 1));
     u64* tile_sum = reinterpret_cast<u64*>(ws + ((ann_ws_ints(NQ, rec_cap) - 2 * ((size_t)rec_cap / kScanTile + 2)) & ~(size_t)1));
-    const int pitch = plane_pitch(D), low_pitch = low_plane_pitch(NQ, D);
-    float* low = low_pitch ? planes + (size_t)rec_cap * (size_t)pitch : nullptr;
+    const int pitch = plane_pitch(D), low_pitch = q_copy ? low_plane_pitch(N, NQ, D) : 0;
+    float* low = low_pitch ? reinterpret_cast<float*>((reinterpret_cast<uintptr_t>(planes + (size_t)rec_cap * (size_t)pitch) + 255) & ~(uintptr_t)255) : nullptr;
     hipLaunchKernelGGL(k_planes, dim3((unsigned)((rec_cap + 3) / 4)), dim3(256), 0, stream, points, D, recs, n_rec_dev, rec_cap, planes,
-                       pitch, low, low_pitch);
+                       pitch, low, low_pitch, low ? q_copy->mu : nullptr, low ? q_copy->scale() : nullptr);
     const unsigned g_route = (unsigned)(((size_t)NQ * 8 + 255) / 256);
     const bool vec_q = (D & 3) == 0 && (reinterpret_cast<uintptr_t>(queries) & 15) == 0;
-    if (low && vec_q)
-        hipLaunchKernelGGL(k_route_low<true>, dim3(g_route), dim3(256), 0, stream, planes, pitch, low, low_pitch, queries, NQ, D, rec_cap,
-                           q_rec, q_rank, cnt, cnt_shift);
+    if (low && D <= 64)
+        hipLaunchKernelGGL(k_route_low<1>, dim3(g_route), dim3(256), 0, stream, planes, pitch, low, low_pitch, queries, *q_copy, q_copy->scale(),
+                           q_copy->mu_len(), SideBound(D), NQ, D, vec_q, rec_cap, start, q_rec, q_rank, cnt, cnt_shift);
     else if (low)
-        hipLaunchKernelGGL(k_route_low<false>, dim3(g_route), dim3(256), 0, stream, planes, pitch, low, low_pitch, queries, NQ, D, rec_cap,
-                           q_rec, q_rank, cnt, cnt_shift);
+        hipLaunchKernelGGL(k_route_low<2>, dim3(g_route), dim3(256), 0, stream, planes, pitch, low, low_pitch, queries, *q_copy, q_copy->scale(),
+                           q_copy->mu_len(), SideBound(D), NQ, D, vec_q, rec_cap, start, q_rec, q_rank, cnt, cnt_shift);
     else if (vec_q)
         hipLaunchKernelGGL((k_route<true, false>), dim3(g_route), dim3(256), 0, stream, planes, pitch, queries, NQ, D, recs, rec_cap,
-                           q_rec, q_rank, cnt, cnt_shift, nullptr);
+                           start, q_rec, q_rank, cnt, cnt_shift, nullptr);
     else
         hipLaunchKernelGGL((k_route<false, false>), dim3(g_route), dim3(256), 0, stream, planes, pitch, queries, NQ, D, recs, rec_cap,
-                           q_rec, q_rank, cnt, cnt_shift, nullptr);
+                           start, q_rec, q_rank, cnt, cnt_shift, nullptr);
     // a bucket with c queries takes ceil(c / 16) work items: at most NQ / 16 + (buckets with queries) in all
     const int most_items = NQ / kQB + std::min(n_leaves, NQ) + 1;
     const unsigned int share_q16 = ann_screen_share_q16(N, NQ, D, n_leaves);
@@ -787,13 +766,13 @@ int ann_forest_group(int N, int NQ, int D, int K, int MAX, int max_bucket, int r
     if (!forced && (double)NQ * (double)MAX * (double)D > kMostFloats) return 0;
     if (!forced && max_bucket > kAnnSeen && (double)NQ * (double)max_bucket * (double)D > kMostHot * (double)N) return 0;
     // hyperplanes and buckets reached: 1 GB at most
-    const size_t per_tree = sizeof(float) * (size_t)rec_cap * (size_t)ann_plane_pitch(NQ, D) + sizeof(int2) * (size_t)NQ;
+    const size_t per_tree = sizeof(float) * (size_t)rec_cap * (size_t)ann_plane_pitch(N, NQ, D) + sizeof(int2) * (size_t)NQ;
     const int group = (int)std::min<size_t>((size_t)std::min(nb, 64), ((size_t)1 << 30) / per_tree);
     return group >= 2 ? group : 0;
 }
 
 // The search in T trees at once.  recs, n_rec_dev, perm: those of the first tree, the others follow (n_rec_dev: kTreeStatPitch apart); planes: T rec_cap
-// ann_plane_pitch(NQ, D) floats; reached: 2 NQ T ints.
+// ann_plane_pitch(N, NQ, D) floats; reached: 2 NQ T ints.
 int launch_ann_forest(const float* points, const float* queries, int N, int NQ, int D, int K, int T, const int* perm, const TreeRec* recs,
                       const int* n_rec_dev, int rec_cap, float* planes, int* reached, int* q_idx, float* q_dist, hipStream_t stream)
 {
@@ -802,15 +781,15 @@ int launch_ann_forest(const float* points, const float* queries, int N, int NQ, 
     int2* where = reinterpret_cast<int2*>(reached);
     const int pitch = plane_pitch(D);
     hipLaunchKernelGGL(k_planes, dim3((unsigned)((rec_cap + 3) / 4), (unsigned)T), dim3(256), 0, stream, points, D, recs, n_rec_dev, rec_cap,
-                       planes, pitch, nullptr, 0);
+                       planes, pitch, nullptr, 0, nullptr, nullptr);
     const dim3 g_route((unsigned)(((size_t)NQ * 8 + 255) / 256), (unsigned)T);
     const bool vec_q = (D & 3) == 0 && (reinterpret_cast<uintptr_t>(queries) & 15) == 0;
     if (vec_q)
         hipLaunchKernelGGL((k_route<true, true>), g_route, dim3(256), 0, stream, planes, pitch, queries, NQ, D, recs, rec_cap, nullptr,
-                           nullptr, nullptr, 0, where);
+                           nullptr, nullptr, nullptr, 0, where);
     else
         hipLaunchKernelGGL((k_route<false, true>), g_route, dim3(256), 0, stream, planes, pitch, queries, NQ, D, recs, rec_cap, nullptr,
-                           nullptr, nullptr, 0, where);
+                           nullptr, nullptr, nullptr, 0, where);
     const bool vec_p = (D & 3) == 0 && (reinterpret_cast<uintptr_t>(points) & 15) == 0;
     const int dpad = (D + 31) & ~31;
     const size_t lds = ann_forest_lds(D, K);

@@ -479,7 +479,7 @@ int knn_ann_forest_device(int n_trees, int K, int N, int NQ, int D, int MIN, int
         if (tree_ws_alloc(&ws.w, N, D, MIN, B)) return 1;
         if (tree_ws_enable_index(ws.w, MIN, MAX_DEPTH)) return 1;
         const int rec_cap = tree_ws_rec_cap(ws.w);
-        const size_t plane_bytes = sizeof(float) * (size_t)rec_cap * (size_t)ann_plane_pitch(NQ, D);
+        const size_t plane_bytes = sizeof(float) * (size_t)rec_cap * (size_t)ann_plane_pitch(N, NQ, D);
         // working memory of the trees of a batch that are searched together, and of trees that are searched one after the other:
         // taken when a batch asks for it for the first time (all batches but the last have the same number of trees)
         DevBuf together_planes, reached, aws, planes, pair_stats;
@@ -498,9 +498,28 @@ int knn_ann_forest_device(int n_trees, int K, int N, int NQ, int D, int MIN, int
         };
         const auto room_alone = [&]() -> int {
             if (pair_stats.p) return 0;
-            if (ws_alloc(&aws.p, sizeof(int) * ann_ws_ints(NQ, rec_cap)) || ws_alloc(&planes.p, plane_bytes)) return 1;
+            if (ws_alloc(&aws.p, sizeof(int) * ann_ws_ints(NQ, rec_cap)) || ws_alloc(&planes.p, plane_bytes + 256)) return 1;
             if (ws_alloc(&pair_stats.p, sizeof(unsigned long long) * ann_stat_words(n_trees))) return 1;
             return launch_ann_ws_init(static_cast<int*>(aws.p), NQ, rec_cap, static_cast<unsigned long long*>(pair_stats.p), n_trees, stream);
+        };
+        // trees that are searched one after the other: the copy of the queries, and for as many trees together as there is room for
+        // (512 MB at most) where every query goes on after the first levels; without these the queries are routed exactly
+        JoinCopyGuard q_copy;
+        DevBuf top_ws, top_start;
+        bool copied = false;
+        int top_trees = ann_top_wanted(NQ, D) ? (int)std::min<size_t>((size_t)B, ((size_t)512 << 20) / (sizeof(int) * (size_t)NQ)) : 0;
+        const auto room_routing = [&]() -> int {
+            if (copied || (top_trees <= 0 && !ann_low_wanted(N, NQ, D))) return 0;
+            if (join_copy_alloc(&q_copy.c, NQ, D, true)) {
+                join_copy_free(&q_copy.c);
+                top_trees = 0;
+                return 0;
+            }
+            copied = true;
+            if (top_trees > 0 && (ws_try_alloc(&top_start.p, sizeof(int) * (size_t)NQ * (size_t)top_trees) ||
+                                  ws_try_alloc(&top_ws.p, ann_top_bytes(top_trees, D))))
+                top_trees = 0;
+            return join_copy_fill(q_copy.c, d_queries, NQ, D, stream);
         };
         std::vector<int> stats((size_t)5 * B);
         std::vector<TimedEvent> ev((size_t)B + 1);          // ev[j]: the search in tree j of a batch begins, ev[nb]: the last ends
@@ -519,7 +538,7 @@ int knn_ann_forest_device(int n_trees, int K, int N, int NQ, int D, int MIN, int
             for (int j = 0; j < nb; ++j) max_bucket = std::max(max_bucket, stats[5 * j + 2]);
             int group = ann_forest_group(N, NQ, D, K, MAX, max_bucket, rec_cap, nb);
             if (group > 0 && !room_together(group)) group = 0;
-            if (group == 0 && room_alone()) return 1;
+            if (group == 0 && (room_alone() || room_routing())) return 1;
             if (group > 0) (void)hipEventRecord(ev[0].e, stream);
             for (int j = 0; j < nb && rc == 0 && group > 0; j += group)
                 rc = launch_ann_forest(d_points, d_queries, N, NQ, D, K, std::min(group, nb - j), tree_ws_perm(ws.w, j),
@@ -527,8 +546,13 @@ int knn_ann_forest_device(int n_trees, int K, int N, int NQ, int D, int MIN, int
                                        static_cast<int*>(reached.p), d_qidx, d_qdist, stream);
             for (int j = 0; j < nb && rc == 0 && group == 0; ++j) {
                 (void)hipEventRecord(ev[j].e, stream);
+                if (top_trees > 0 && j % top_trees == 0 &&
+                    launch_ann_top(d_points, q_copy.c, NQ, D, std::min(top_trees, nb - j), tree_ws_recs(ws.w, j), tree_ws_n_rec(ws.w, j), rec_cap,
+                                   top_ws.p, static_cast<int*>(top_start.p), stream))
+                    return 1;
+                const int* start = top_trees > 0 ? static_cast<const int*>(top_start.p) + (size_t)(j % top_trees) * (size_t)NQ : nullptr;
                 rc = launch_ann_tree(d_points, d_queries, N, NQ, D, K, tree_ws_perm(ws.w, j), tree_ws_recs(ws.w, j),
-                                     tree_ws_n_rec(ws.w, j), rec_cap, stats[5 * j + 0], static_cast<int*>(aws.p),
+                                     tree_ws_n_rec(ws.w, j), rec_cap, stats[5 * j + 0], copied ? &q_copy.c : nullptr, start, static_cast<int*>(aws.p),
                                      static_cast<float*>(planes.p), d_qidx, d_qdist,
                                      tb0 + j > 0 ? static_cast<unsigned long long*>(pair_stats.p) + ann_stat_words(tb0 + j - 1) : nullptr,
                                      static_cast<unsigned long long*>(pair_stats.p) + ann_stat_words(tb0 + j), stream);

@@ -110,18 +110,27 @@ __global__ __launch_bounds__(256) void k_col_mean(const float* __restrict__ poin
                                                   const uint32_t* __restrict__ spread, float* __restrict__ scale, int D, float inv_n)
 {
     __shared__ uint32_t part[256];
+    __shared__ float part_q[256];
     uint32_t far = 0u;
+    float q = 0.0f;
     for (int d = threadIdx.x; d < D; d += 256) {
-        mu[d] = finite_or_zero(points[d]) + finite_or_zero(mu[d] * inv_n);
+        const float m = finite_or_zero(points[d]) + finite_or_zero(mu[d] * inv_n);
+        mu[d] = m;
+        q = __builtin_fmaf(m, m, q);
         far = max(far, spread[d]);
     }
     part[threadIdx.x] = far;
+    part_q[threadIdx.x] = q;
     __syncthreads();
     for (int o = 128; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o) part[threadIdx.x] = max(part[threadIdx.x], part[threadIdx.x + o]);
+        if ((int)threadIdx.x < o) {
+            part[threadIdx.x] = max(part[threadIdx.x], part[threadIdx.x + o]);
+            part_q[threadIdx.x] += part_q[threadIdx.x + o];
+        }
         __syncthreads();
     }
     if (threadIdx.x == 0) {
+        scale[3] = sqrtf(part_q[0]) * (1.0f + 1.0f / 1024.0f) + 1e-18f;
         const int e = (int)(part[0] >> 23) - 126;                          // f < 2^e
         *scale = __uint_as_float((uint32_t)(127 + max(-100, min(100, 14 - e))) << 23);
     }
@@ -198,14 +207,18 @@ __global__ __launch_bounds__(256) void k_to_join(const float* __restrict__ point
 
 }  // namespace
 
-int join_copy_alloc(JoinCopy* c, int N, int D)
+int join_copy_alloc(JoinCopy* c, int N, int D, bool optional)
 {
     c->D = D;
-    if (ws_alloc(reinterpret_cast<void**>(&c->mu), ((size_t)2 * D + 3) * sizeof(float))) return 1;
-    if (ws_alloc(reinterpret_cast<void**>(&c->parts), kJoinMostGrid * sizeof(float2))) return 1;
-    if (ws_alloc(reinterpret_cast<void**>(&c->rows), std::max<size_t>((size_t)N * join_pitch(D) * 2, 16))) return 1;
-    if (ws_alloc(reinterpret_cast<void**>(&c->norms), std::max<size_t>((size_t)N * 4, 16))) return 1;
-    if (ws_alloc(reinterpret_cast<void**>(&c->errs), std::max<size_t>((size_t)N * 4, 16))) return 1;
+    const auto get = [optional](void* p, size_t bytes) {
+        void** out = reinterpret_cast<void**>(p);
+        return optional ? ws_try_alloc(out, bytes) : ws_alloc(out, bytes);
+    };
+    if (get(&c->mu, ((size_t)2 * D + 4) * sizeof(float))) return 1;
+    if (get(&c->parts, kJoinMostGrid * sizeof(float2))) return 1;
+    if (get(&c->rows, std::max<size_t>((size_t)N * join_pitch(D) * 2, 16))) return 1;
+    if (get(&c->norms, std::max<size_t>((size_t)N * 4, 16))) return 1;
+    if (get(&c->errs, std::max<size_t>((size_t)N * 4, 16))) return 1;
     return 0;
 }
 
@@ -222,8 +235,8 @@ void join_copy_free(JoinCopy* c)
 int join_copy_fill(JoinCopy& c, const float* points, int N, int D, hipStream_t stream)
 {
     float* scale = c.mu + D;
-    uint32_t* spread = reinterpret_cast<uint32_t*>(scale + 3);
-    hipLaunchKernelGGL(k_col_clear, dim3((2 * D + 3 + 255) / 256), dim3(256), 0, stream, reinterpret_cast<uint32_t*>(c.mu), 2 * D + 3);
+    uint32_t* spread = reinterpret_cast<uint32_t*>(scale + 4);
+    hipLaunchKernelGGL(k_col_clear, dim3((2 * D + 4 + 255) / 256), dim3(256), 0, stream, reinterpret_cast<uint32_t*>(c.mu), 2 * D + 4);
     // (a workgroup ends with two atomics per column, carried out one after the other: 123,457 x 37 with 64 rows each 0.062 ms, with 256
     // 0.022)
     const int g = std::max(1, std::min(N / (D <= 128 ? 256 : 64), 2048));

@@ -1,4 +1,5 @@
-// 16-bit copy of the points for the join of the exploration (explore_join.hip).
+// 16-bit copy of the points for the join of the exploration (explore_join.hip), and of the queries for the first levels of their
+// way through the trees (ann_top.hip).
 //
 // Row p holds s (x - mu) in float16 (round to nearest; below 2^-14, the least normal number, zero), mu the column means and s a
 // power of two, padded with zeros to join_pitch(D) values; norms[p] = sum of the squares of the values as rounded, errs[p] >=
@@ -20,14 +21,16 @@ struct JoinCopy {
     uint16_t* rows = nullptr;     // N x join_pitch(D)
     float* norms = nullptr;       // N, in units of s^2
     float* errs = nullptr;        // N, in units of s
-    float* mu = nullptr;          // column means, then (s, largest norm, largest error of the finite rows), then D words of working memory
+    float* mu = nullptr;          // column means, then (s, largest norm, largest error of the finite rows, a bound of |mu|), then D words of working memory
     float2* parts = nullptr;      // n_parts: largest norm and error of the finite rows a workgroup made (k_join_bars completes them)
     int n_parts = 0;
     int D = 0;
     float* scale() const { return mu + D; }
+    float* mu_len() const { return mu + D + 3; }
 };
 
-int join_copy_alloc(JoinCopy* c, int N, int D);
+// optional: as blocks the caller can do without (ws_try_alloc)
+int join_copy_alloc(JoinCopy* c, int N, int D, bool optional = false);
 void join_copy_free(JoinCopy* c);
 int join_copy_fill(JoinCopy& c, const float* points, int N, int D, hipStream_t stream);
 

@@ -1163,6 +1163,37 @@ def test_ann_batches_take_the_form_their_buckets_ask_for(gpu, capi, orc, rng, mo
     assert_knn_equal(di.cpu().numpy(), dd.cpu().numpy(), idx, dist)
 
 
+# one query, and the sizes around a wavefront's 64; every number of 16-dimension steps, rows that end inside one; trees that end within
+# the first seven levels (the first one at its root) and go on below; queries in no tree's cloud
+@pytest.mark.parametrize("N,NQ,D,K,T,mn,mx", [(40, 1, 3, 5, 3, 50, 100), (300, 63, 1, 4, 5, 5, 11), (2500, 64, 16, 3, 6, 4, 9), (5000, 65, 17, 2, 9, 3, 6),
+                                              (1500, 500, 37, 8, 4, 9, 18), (2000, 257, 64, 16, 3, 17, 64), (6000, 129, 65, 5, 4, 6, 12), (900, 300, 81, 6, 3, 7, 14),
+                                              (3000, 1000, 100, 4, 5, 5, 10), (1200, 100, 112, 4, 4, 5, 10), (4000, 200, 128, 10, 3, 11, 22)])
+@pytest.mark.parametrize("data", ["normal", "ties", "tiny", "offset", "huge", "apart"])
+def test_ann_first_levels_of_all_trees_match_oracle(gpu, capi, orc, rng, monkeypatch, N, NQ, D, K, T, mn, mx, data):
+    """Queries that take the first seven levels by rounded hyperplanes on the matrix cores, then the others exactly, by rounded ones, and
+    without the memory for either == the oracle."""
+    import torch
+    draw = {"normal": lambda n: rng.standard_normal((n, D)), "ties": lambda n: rng.integers(0, 3, (n, D)),
+            "tiny": lambda n: rng.standard_normal((n, D)) * 1e-18, "offset": lambda n: rng.standard_normal((n, D)) * 1e-2 + 300.0,
+            "huge": lambda n: rng.standard_normal((n, D)) * np.where(rng.random((n, 1)) < 0.1, 3e18, 1.0),
+            "apart": lambda n: rng.standard_normal((n, D)) * (1.0 if n == N else 1e6) + (0.0 if n == N else -70.0)}[data]
+    X, Q = draw(N).astype(np.float32), draw(NQ).astype(np.float32)
+    dX, dQ = torch.from_numpy(X).cuda(), torch.from_numpy(Q).cuda()
+    oi, od = orc.ann_forest(X, Q, K, T, mn, mx, 5000, 5)
+    monkeypatch.setenv("RSFK_ANN_FOREST", "0")
+    monkeypatch.setenv("RSFK_ANN_TOP", "1")
+    for low, optional in (("0", None), ("1", None), ("1", "0")):
+        monkeypatch.setenv("RSFK_ANN_ROUTE_LOW", low)
+        if optional is not None:
+            monkeypatch.setenv("RSFK_OPTIONAL_MB", optional)
+        idx = torch.full((NQ, K), -1, dtype=torch.int32, device="cuda")
+        dist = torch.full((NQ, K), float("inf"), dtype=torch.float32, device="cuda")
+        _say("ann first levels", N, NQ, D, K, T, mn, mx, data, low, optional)
+        capi.knn_ann_device(T, K, N, NQ, D, mn, mx, 5000, 0, 5, dX.data_ptr(), dQ.data_ptr(), idx.data_ptr(), dist.data_ptr())
+        torch.cuda.synchronize()
+        assert_knn_equal(idx.cpu().numpy(), dist.cpu().numpy(), oi, od)
+
+
 # items of fewer and of more than 32 queries; buckets on both sides of 32 and 64 members; rows that end inside a step and inside
 # a 16-byte piece; distances that overflow, a common offset that leaves the bounds useless, equal distances
 @pytest.mark.parametrize("N,NQ,D,K,T,mn,mx", [(500, 900, 16, 64, 5, 65, 130), (3000, 2500, 100, 32, 6, 33, 66), (700, 333, 31, 5, 9, 6, 12),
