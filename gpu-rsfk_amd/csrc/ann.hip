@@ -636,8 +636,9 @@ size_t ann_ws_ints(int NQ, int rec_cap)
 // gathers of step 3 dearer: 300,000 / 300,000 x 256 in buckets of 33..66 22.0 -> 22.7 ms, 1M / 1M x 100 78.4 -> 69.6, with the
 // line at 20 to 40 % of the pairs alike, 500,000 / 500,000 x 64 13.5 -> 12.1 (20 to 60 % alike), 1M / 60,000 x 8 12.7 -> 9.4
 // at 60 % and 9.9 at 20 %.
-unsigned int ann_screen_share_q16(int N, int NQ, int D, int n_leaves)
+unsigned int ann_screen_share_q16(int N, int NQ, int D, int K, int n_leaves)
 {
+    if (K > 64 || D > kAnnScreenDims) return 0;
     double pct = D <= 64 ? 60.0 : 30.0;
     const char* e = std::getenv("RSFK_ANN_SCREEN");             // (read at every call: tests change it)
     if (e && *e) {
@@ -668,11 +669,12 @@ int launch_ann_ws_init(int* ws, int NQ, int rec_cap, unsigned long long* stats, 
 // One tree of the query-set search: routes the queries through the index recs (*n_rec_dev records, at most rec_cap;
 // the tree has n_leaves buckets), groups them by bucket and offers the base points perm[..] of the bucket a query
 // reached to the query's row.  prev, stats: numbers of pairs of the tree before this one (null: the first) and of this one,
-// kAnnStatWords each.  q_copy: null, or the copy of the queries.  start: the records from which the queries go on (null: the root).  ws: ann_ws_ints(NQ, rec_cap) ints, prepared by launch_ann_ws_init; planes: rec_cap
+// kAnnStatWords each.  q_copy, p_copy: null, or the copy of the queries, of the points
+// (with q_copy only: the screened bucket step reads them).  start: the records from which the queries go on (null: the root).  ws: ann_ws_ints(NQ, rec_cap) ints, prepared by launch_ann_ws_init; planes: rec_cap
 // ann_plane_pitch(N, NQ, D) floats and 256 bytes.
 int launch_ann_tree(const float* points, const float* queries, int N, int NQ, int D, int K, const int* perm, const TreeRec* recs,
-                    const int* n_rec_dev, int rec_cap, int n_leaves, const JoinCopy* q_copy, const int* start,
-                    int* ws, float* planes, int* q_idx, float* q_dist,
+                    const int* n_rec_dev, int rec_cap, int n_leaves, const JoinCopy* q_copy, const JoinCopy* p_copy,
+                    const int* start, int* ws, float* planes, int* q_idx, float* q_dist,
                     const unsigned long long* prev, unsigned long long* stats, hipStream_t stream)
 {
     if (NQ <= 0) return 0;
@@ -708,8 +710,8 @@ int launch_ann_tree(const float* points, const float* queries, int N, int NQ, in
                            start, q_rec, q_rank, cnt, cnt_shift, nullptr);
     // a bucket with c queries takes ceil(c / 16) work items: at most NQ / 16 + (buckets with queries) in all
     const int most_items = NQ / kQB + std::min(n_leaves, NQ) + 1;
-    const unsigned int share_q16 = ann_screen_share_q16(N, NQ, D, n_leaves);
-    AnnForm form = {K <= 64 && share_q16 != 0 && D <= kAnnScreenDims ? prev : nullptr, stats, share_q16, 0};
+    const unsigned int share_q16 = ann_screen_share_q16(N, NQ, D, K, n_leaves);
+    AnnForm form = {share_q16 != 0 ? prev : nullptr, stats, share_q16, 0};
     while ((most_items >> form.shift) > 512) ++form.shift;
     const unsigned g_scan = (unsigned)(rec_cap / kScanTile + 1);
     hipLaunchKernelGGL(k_ann_tile_sums, dim3(g_scan), dim3(256), 0, stream, cnt, cnt_shift, n_rec_dev, rec_cap, tile_sum, form);
@@ -718,7 +720,11 @@ int launch_ann_tree(const float* points, const float* queries, int N, int NQ, in
     hipLaunchKernelGGL(k_ann_fill, dim3(g_fill), dim3(256), 0, stream, NQ, q_rec, q_rank, n_rec_dev, rec_cap, recs, qoff, boff, qlist,
                        blk_desc, form);
     // (the form that is not taken finds out in every workgroup, hence few of them)
-    if (form.prev && launch_ann_screen(points, queries, D, K, perm, blk_desc, n_blocks, most_items, qlist, q_idx, q_dist, form, stream)) return 1;
+    if (form.prev && p_copy) {
+        if (launch_ann_screen_half(*q_copy, *p_copy, points, queries, D, K, perm, blk_desc, n_blocks, most_items, qlist, q_idx, q_dist, form, stream)) return 1;
+    } else if (form.prev) {
+        if (launch_ann_screen(points, queries, D, K, perm, blk_desc, n_blocks, most_items, qlist, q_idx, q_dist, form, stream)) return 1;
+    }
     const unsigned g_leaf = (unsigned)std::min(most_items, kLeafGrid);
     const bool vec = (D & 3) == 0 && ((reinterpret_cast<uintptr_t>(points) | reinterpret_cast<uintptr_t>(queries)) & 15) == 0;
 #define RSFK_ANN_CASE(SLV)                                                                                                   \

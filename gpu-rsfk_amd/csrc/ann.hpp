@@ -100,5 +100,9 @@ __device__ __forceinline__ uint16_t rounded_value(float nd, const RoundedPlane& 
 int launch_ann_screen(const float* points, const float* queries, int D, int K, const int* perm, const int4* blk_desc,
                       const int* n_blocks, int most_blocks, const int* qlist, int* q_idx, float* q_dist, const AnnForm& form,
                       hipStream_t stream);
+// ann_screen_half.hip: the same by copies of the queries and of the points with the same mu and s
+int launch_ann_screen_half(const JoinCopy& qc, const JoinCopy& pc, const float* points, const float* queries, int D, int K, const int* perm,
+                           const int4* blk_desc, const int* n_blocks, int most_blocks, const int* qlist, int* q_idx, float* q_dist,
+                           const AnnForm& form, hipStream_t stream);
 
 }  // namespace rsfk

@@ -15,6 +15,7 @@
 // trees 0.57 ms where k_ann_leaf takes 0.85 (vector ALUs); the first trees, where most pairs are left, 2.9 against 1.9.  Tried: the
 // members' rows of step 3 through a transposing tile in LDS (faster at D = 256 while many pairs are left, 0.65 ms here), K-NN
 // rows requested before the chains run (no change), two steps of 16 dimensions in flight in separate buffers (spills).
+// (Rows of 97 to 128 dimensions: ann_screen_half.hip, where there is room for copies of them.)
 // No barrier: the wavefronts of a workgroup share nothing but the cache lines of a bucket they may both work on.
 #include "forest.hpp"
 #include "ann.hpp"

@@ -635,18 +635,6 @@ __device__ __forceinline__ bool join_may(float least, float bar, float e_c)
     return !(least > w * w);
 }
 
-// squares of eight values of a row added up (lanes l and l + 32 have the values of a row in turns of eight)
-__device__ __forceinline__ float half_norm(f16x8 v, float acc)
-{
-    typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
-#pragma unroll
-    for (int i = 0; i < 8; i += 2) {
-        const f16x2 h = {v[i], v[i + 1]};
-        acc = __builtin_amdgcn_fdot2(h, h, acc, false);
-    }
-    return acc;
-}
-
 // One wavefront per q.  Per-wavefront LDS (ints): cq[KP] | pid[32] | pn[32] | pbar[32] | perr[32] | pper[32] | pe[32], KP = K rounded up to 32.
 // Workgroups (x, y): every gridDim.y-th tile of R(q), the y-th first.  (Five wavefronts per SIMD: 1M x 256 7.6 -> 7.0 ms against four
 // with the next 64 dimensions in flight.)
@@ -1214,8 +1202,7 @@ int launch_explore_join(ExploreWorkspace* w, const JoinCopy& jc, int N, int D, i
     const float kappa = (float)(ksteps * 16 + 16) * (1.0f / 2097152.0f);            // (Dp + 16) 2^-21
     const float one_minus_gamma = 1.0f - (float)(D + 8) * (1.0f / 4194304.0f);      // 1 - (D + 8) 2^-22
     RSFK_CHECK(one_minus_gamma > 0.5f, "exploration join: D too large");
-    // rounding of any row: 2^-11 of a value, 2^-14 of one set to zero, and errs' own terms (3e-3 covers these and the root)
-    const float any_rel = 1.003f / 2048.0f, any_abs = 1.001f * std::sqrt((float)D) / 16384.0f + 1e-6f;
+    const float any_rel = join_err_rel(), any_abs = join_err_abs(D);
     w->view.codes = w->bounds;
     w->view.bars = w->bars;
     w->view.norms = jc.norms;

@@ -502,24 +502,31 @@ int knn_ann_forest_device(int n_trees, int K, int N, int NQ, int D, int MIN, int
             if (ws_alloc(&pair_stats.p, sizeof(unsigned long long) * ann_stat_words(n_trees))) return 1;
             return launch_ann_ws_init(static_cast<int*>(aws.p), NQ, rec_cap, static_cast<unsigned long long*>(pair_stats.p), n_trees, stream);
         };
-        // trees that are searched one after the other: the copy of the queries, and for as many trees together as there is room for
-        // (512 MB at most) where every query goes on after the first levels; without these the queries are routed exactly
-        JoinCopyGuard q_copy;
+        // trees that are searched one after the other: the copy of the queries, that of the points where the screened bucket step reads copies, and for as
+        // many trees together as there is room for (512 MB at most) where every query goes on after the first levels; without these the
+        // queries are routed exactly, and the bucket step bounds the pairs by the fp32 rows
+        JoinCopyGuard q_copy, p_copy;
         DevBuf top_ws, top_start;
-        bool copied = false;
+        bool q_asked = false, p_asked = false;
         int top_trees = ann_top_wanted(NQ, D) ? (int)std::min<size_t>((size_t)B, ((size_t)512 << 20) / (sizeof(int) * (size_t)NQ)) : 0;
-        const auto room_routing = [&]() -> int {
-            if (copied || (top_trees <= 0 && !ann_low_wanted(N, NQ, D))) return 0;
-            if (join_copy_alloc(&q_copy.c, NQ, D, true)) {
-                join_copy_free(&q_copy.c);
-                top_trees = 0;
-                return 0;
+        const auto room_copies = [&](bool screened) -> int {
+            const bool points_too = screened && !p_asked, queries_too = (screened || top_trees > 0 || ann_low_wanted(N, NQ, D)) && !q_asked;
+            if (queries_too) {
+                q_asked = true;
+                if (join_copy_alloc(&q_copy.c, NQ, D, true)) join_copy_free(&q_copy.c);
+                if (q_copy.c.rows == nullptr ||
+                    (top_trees > 0 && (ws_try_alloc(&top_start.p, sizeof(int) * (size_t)NQ * (size_t)top_trees) ||
+                                       ws_try_alloc(&top_ws.p, ann_top_bytes(top_trees, D)))))
+                    top_trees = 0;
             }
-            copied = true;
-            if (top_trees > 0 && (ws_try_alloc(&top_start.p, sizeof(int) * (size_t)NQ * (size_t)top_trees) ||
-                                  ws_try_alloc(&top_ws.p, ann_top_bytes(top_trees, D))))
-                top_trees = 0;
-            return join_copy_fill(q_copy.c, d_queries, NQ, D, stream);
+            if (q_copy.c.rows == nullptr) return 0;
+            if (points_too) {
+                p_asked = true;
+                if (join_copy_alloc(&p_copy.c, N, D, true)) join_copy_free(&p_copy.c);
+                else if (join_copy_fill(p_copy.c, d_points, N, D, stream)) return 1;
+            }
+            if (p_copy.c.rows != nullptr && points_too) return join_copy_fill(q_copy.c, d_queries, NQ, D, stream, &p_copy.c);
+            return queries_too ? join_copy_fill(q_copy.c, d_queries, NQ, D, stream) : 0;
         };
         std::vector<int> stats((size_t)5 * B);
         std::vector<TimedEvent> ev((size_t)B + 1);          // ev[j]: the search in tree j of a batch begins, ev[nb]: the last ends
@@ -538,7 +545,9 @@ int knn_ann_forest_device(int n_trees, int K, int N, int NQ, int D, int MIN, int
             for (int j = 0; j < nb; ++j) max_bucket = std::max(max_bucket, stats[5 * j + 2]);
             int group = ann_forest_group(N, NQ, D, K, MAX, max_bucket, rec_cap, nb);
             if (group > 0 && !room_together(group)) group = 0;
-            if (group == 0 && (room_alone() || room_routing())) return 1;
+            bool screened = false;
+            for (int j = 0; j < nb; ++j) screened = screened || (ann_half_wanted(D) && ann_screen_share_q16(N, NQ, D, K, stats[5 * j]) != 0);
+            if (group == 0 && (room_alone() || room_copies(screened))) return 1;
             if (group > 0) (void)hipEventRecord(ev[0].e, stream);
             for (int j = 0; j < nb && rc == 0 && group > 0; j += group)
                 rc = launch_ann_forest(d_points, d_queries, N, NQ, D, K, std::min(group, nb - j), tree_ws_perm(ws.w, j),
@@ -552,7 +561,8 @@ int knn_ann_forest_device(int n_trees, int K, int N, int NQ, int D, int MIN, int
                     return 1;
                 const int* start = top_trees > 0 ? static_cast<const int*>(top_start.p) + (size_t)(j % top_trees) * (size_t)NQ : nullptr;
                 rc = launch_ann_tree(d_points, d_queries, N, NQ, D, K, tree_ws_perm(ws.w, j), tree_ws_recs(ws.w, j),
-                                     tree_ws_n_rec(ws.w, j), rec_cap, stats[5 * j + 0], copied ? &q_copy.c : nullptr, start, static_cast<int*>(aws.p),
+                                     tree_ws_n_rec(ws.w, j), rec_cap, stats[5 * j + 0], q_copy.c.rows ? &q_copy.c : nullptr,
+                                     p_copy.c.rows ? &p_copy.c : nullptr, start, static_cast<int*>(aws.p),
                                      static_cast<float*>(planes.p), d_qidx, d_qdist,
                                      tb0 + j > 0 ? static_cast<unsigned long long*>(pair_stats.p) + ann_stat_words(tb0 + j - 1) : nullptr,
                                      static_cast<unsigned long long*>(pair_stats.p) + ann_stat_words(tb0 + j), stream);

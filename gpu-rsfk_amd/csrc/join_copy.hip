@@ -136,6 +136,11 @@ __global__ __launch_bounds__(256) void k_col_mean(const float* __restrict__ poin
     }
 }
 
+__global__ __launch_bounds__(256) void k_col_take(const float* __restrict__ from, float* __restrict__ to, int n)
+{
+    for (int i = threadIdx.x; i < n; i += 256) to[i] = from[i];
+}
+
 // LPR lanes per row (64 / LPR rows per wavefront), each four dimensions at a time.  Streaming; 10M x 32 (8 lanes per row) 2.0 GB in
 // 0.35 ms, 5.7 TB/s (a wavefront per row, a value per lane: 1.13); 1M x 256 0.26 (0.42), 1M x 100 0.12 (0.22).
 template <int LPR, bool WHOLE>
@@ -232,17 +237,21 @@ void join_copy_free(JoinCopy* c)
     *c = JoinCopy();
 }
 
-int join_copy_fill(JoinCopy& c, const float* points, int N, int D, hipStream_t stream)
+int join_copy_fill(JoinCopy& c, const float* points, int N, int D, hipStream_t stream, const JoinCopy* like)
 {
     float* scale = c.mu + D;
     uint32_t* spread = reinterpret_cast<uint32_t*>(scale + 4);
-    hipLaunchKernelGGL(k_col_clear, dim3((2 * D + 4 + 255) / 256), dim3(256), 0, stream, reinterpret_cast<uint32_t*>(c.mu), 2 * D + 4);
-    // (a workgroup ends with two atomics per column, carried out one after the other: 123,457 x 37 with 64 rows each 0.062 ms, with 256
-    // 0.022)
-    const int g = std::max(1, std::min(N / (D <= 128 ? 256 : 64), 2048));
-    if (D <= 128) hipLaunchKernelGGL(k_col_sum_narrow, dim3(g), dim3(256), 0, stream, points, N, D, c.mu, spread);
-    else hipLaunchKernelGGL(k_col_sum, dim3(g), dim3(256), 0, stream, points, N, D, c.mu, spread);
-    hipLaunchKernelGGL(k_col_mean, dim3(1), dim3(256), 0, stream, points, c.mu, spread, scale, D, 1.0f / (float)N);
+    if (like) {
+        hipLaunchKernelGGL(k_col_take, dim3(1), dim3(256), 0, stream, like->mu, c.mu, D + 4);
+    } else {
+        hipLaunchKernelGGL(k_col_clear, dim3((2 * D + 4 + 255) / 256), dim3(256), 0, stream, reinterpret_cast<uint32_t*>(c.mu), 2 * D + 4);
+        // (a workgroup ends with two atomics per column, carried out one after the other: 123,457 x 37 with 64 rows each 0.062 ms, with 256
+        // 0.022)
+        const int g = std::max(1, std::min(N / (D <= 128 ? 256 : 64), 2048));
+        if (D <= 128) hipLaunchKernelGGL(k_col_sum_narrow, dim3(g), dim3(256), 0, stream, points, N, D, c.mu, spread);
+        else hipLaunchKernelGGL(k_col_sum, dim3(g), dim3(256), 0, stream, points, N, D, c.mu, spread);
+        hipLaunchKernelGGL(k_col_mean, dim3(1), dim3(256), 0, stream, points, c.mu, spread, scale, D, 1.0f / (float)N);
+    }
     const bool whole = (D & 3) == 0 && (reinterpret_cast<uintptr_t>(points) & 15) == 0;
     const int pitch = join_pitch(D);
 #define RSFK_TO_JOIN(L)                                                                                                            \

@@ -1,5 +1,5 @@
-// 16-bit copy of the points for the join of the exploration (explore_join.hip), and of the queries for the first levels of their
-// way through the trees (ann_top.hip).
+// 16-bit copy of the points for the join of the exploration (explore_join.hip), and of queries and points for the query-set search: the
+// way of the queries through the trees (ann_top.hip, k_route_low of ann.hip) and the bounds in their buckets (ann_screen.hip).
 //
 // Row p holds s (x - mu) in float16 (round to nearest; below 2^-14, the least normal number, zero), mu the column means and s a
 // power of two, padded with zeros to join_pitch(D) values; norms[p] = sum of the squares of the values as rounded, errs[p] >=
@@ -9,6 +9,7 @@
 // large.)  A row that is not finite has a norm that is not finite.
 #pragma once
 #include "rsfk_common.hpp"
+#include <cmath>
 
 namespace rsfk {
 
@@ -32,6 +33,24 @@ struct JoinCopy {
 // optional: as blocks the caller can do without (ws_try_alloc)
 int join_copy_alloc(JoinCopy* c, int N, int D, bool optional = false);
 void join_copy_free(JoinCopy* c);
-int join_copy_fill(JoinCopy& c, const float* points, int N, int D, hipStream_t stream);
+// like (null: none): the copy whose mu and s these rows take too; what overflows then is not finite
+int join_copy_fill(JoinCopy& c, const float* points, int N, int D, hipStream_t stream, const JoinCopy* like = nullptr);
+
+// Rounding of any row, errs <= rel |row| + abs: 2^-11 of a value, 2^-14 of one set to zero, and errs' own terms (3e-3 covers these and the
+// root).
+inline float join_err_rel() { return 1.003f / 2048.0f; }
+inline float join_err_abs(int D) { return 1.001f * std::sqrt((float)D) / 16384.0f + 1e-6f; }
+
+// acc + the squares of eight values of a row
+__device__ __forceinline__ float half_norm(__attribute__((ext_vector_type(8))) _Float16 v, float acc)
+{
+    typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
+#pragma unroll
+    for (int i = 0; i < 8; i += 2) {
+        const f16x2 h = {v[i], v[i + 1]};
+        acc = __builtin_amdgcn_fdot2(h, h, acc, false);
+    }
+    return acc;
+}
 
 }  // namespace rsfk

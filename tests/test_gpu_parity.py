@@ -1163,6 +1163,37 @@ def test_ann_batches_take_the_form_their_buckets_ask_for(gpu, capi, orc, rng, mo
     assert_knn_equal(di.cpu().numpy(), dd.cpu().numpy(), idx, dist)
 
 
+# the dimensions whose bounds are made from float16 copies, whole and ragged; one and two blocks of members, their remainders, and more; items of
+# one query, of 32 and more; few pairs that wait until the end and many
+@pytest.mark.parametrize("N,NQ,D,K,T,mn,mx", [(700, 900, 97, 64, 4, 65, 130), (2000, 2500, 100, 32, 6, 33, 66), (600, 333, 101, 5, 7, 6, 12), (40, 1, 104, 3, 3, 50, 100),
+                                              (1500, 1200, 112, 1, 5, 32, 64), (400, 65, 113, 10, 3, 150, 300), (900, 1000, 128, 20, 4, 21, 33)])
+@pytest.mark.parametrize("data", ["normal", "ties", "offset", "huge", "apart"])
+def test_ann_screened_by_copies_matches_oracle(gpu, capi, orc, rng, monkeypatch, N, NQ, D, K, T, mn, mx, data):
+    """The bucket step that bounds the pairs by float16 copies == the oracle, also into rows that hold something, with queries that the
+    copies' range does not hold, and without the memory for the copies."""
+    import torch
+    draw = {"normal": lambda n: rng.standard_normal((n, D)), "ties": lambda n: rng.integers(0, 3, (n, D)),
+            "offset": lambda n: rng.standard_normal((n, D)) * 1e-2 + 300.0,
+            "huge": lambda n: rng.standard_normal((n, D)) * np.where(rng.random((n, 1)) < 0.1, 3e18, 1.0),
+            "apart": lambda n: rng.standard_normal((n, D)) * (1.0 if n == N else np.where(rng.random((n, 1)) < 0.3, 1e5, 2.0))}[data]
+    X, Q = draw(N).astype(np.float32), draw(NQ).astype(np.float32)
+    dX, dQ = torch.from_numpy(X).cuda(), torch.from_numpy(Q).cuda()
+    oi, od = orc.ann_forest(X, Q, K, T, mn, mx, 5000, 5)
+    orc.ann_forest(X, Q, K, 2, mn, mx, 5000, 77, q_idx=oi, q_dist=od)
+    monkeypatch.setenv("RSFK_ANN_FOREST", "0")
+    monkeypatch.setenv("RSFK_ANN_SCREEN", "always")
+    for optional in (None, "0"):
+        if optional is not None:
+            monkeypatch.setenv("RSFK_OPTIONAL_MB", optional)
+        idx = torch.full((NQ, K), -1, dtype=torch.int32, device="cuda")
+        dist = torch.full((NQ, K), float("inf"), dtype=torch.float32, device="cuda")
+        _say("ann screened by copies", N, NQ, D, K, T, mn, mx, data, optional)
+        for trees, seed in ((T, 5), (2, 77)):
+            capi.knn_ann_device(trees, K, N, NQ, D, mn, mx, 5000, 0, seed, dX.data_ptr(), dQ.data_ptr(), idx.data_ptr(), dist.data_ptr())
+        torch.cuda.synchronize()
+        assert_knn_equal(idx.cpu().numpy(), dist.cpu().numpy(), oi, od)
+
+
 # one query, and the sizes around a wavefront's 64; every number of 16-dimension steps, rows that end inside one; trees that end within
 # the first seven levels (the first one at its root) and go on below; queries in no tree's cloud
 @pytest.mark.parametrize("N,NQ,D,K,T,mn,mx", [(40, 1, 3, 5, 3, 50, 100), (300, 63, 1, 4, 5, 5, 11), (2500, 64, 16, 3, 6, 4, 9), (5000, 65, 17, 2, 9, 3, 6),
