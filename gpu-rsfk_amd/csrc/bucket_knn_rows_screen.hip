@@ -8,15 +8,18 @@
 //
 //   1. the fp32 rows of the bucket are staged into LDS (pitch an odd number of 16-byte units).
 //   2. A wavefront takes 32 members at a time against all tiles of 32 candidates.  The rows minus a common point (the mean of 16 of
-//      them) are rounded to bfloat16 on the fly; v_mfma_f32_32x32x16_bf16 accumulates the products.  With x = a - m, y = b - m,
-//      S = |x|^2 + |y|^2 and G the accumulated product of the rounded vectors,
-//          | |a - b|^2 - (S - 2 G) |  <=  c S,
-//          c = 1.05 * 2^-7 + (4 D16 + 16) 2^-23      (D16 = D rounded up to 16):
-//      two roundings of at most 2^-8 per product give (2^-7 + 2^-16) S, the differences 2^-23 S, accumulation and norms at most
-//      1.7 (D16 + 2) 2^-23 S.  The fp32 chain returns at least (1 - gamma) times the real-number distance, gamma = (D + 8) 2^-22.
-//      The pair is dropped iff ((1 - c) S - 2 G) > last slot / (1 - gamma); for a lane that is one comparison per pair: the
-//      accumulator starts at -(1 - c)|y|^2 / 2 and is compared with ((1 - c)|x|^2 - last slot / (1 - gamma)) / 2.  A norm of
+//      them), times a power of two s that puts the longest of them between 2^13 and 2^14, are rounded to float16 on the fly;
+//      v_mfma_f32_32x32x16_f16 accumulates the products.  With x = s (a - m), y = s (b - m), S = |x|^2 + |y|^2, R the longest and G the
+//      accumulated product of the rounded vectors,
+//          | s^2 |a - b|^2 - (S - 2 G) |  <=  c S + z,
+//          c = 1.05 * 2^-10 + (4 D16 + 16) 2^-23,  z = 4.1 h sqrt(D) R + 2.1 h^2 D,  h = 2^-14     (D16 = D rounded up to 16):
+//      two roundings of at most 2^-11 per product give (2^-10 + 2^-22) S, the differences 2^-23 S, accumulation and norms at most
+//      1.7 (D16 + 2) 2^-23 S; z is for values below the least normal number h, wherever they end up.  The fp32 chain returns at least
+//      (1 - gamma) times the real-number distance, gamma = (D + 8) 2^-22.
+//      The pair is dropped iff ((1 - c) S - 2 G) > s^2 last slot / (1 - gamma) + z; for a lane that is one comparison per pair: the
+//      accumulator starts at -(1 - c)|y|^2 / 2 and is compared with ((1 - c)|x|^2 - s^2 last slot / (1 - gamma) - z) / 2.  A norm of
 //      1e37 or more, or NaN, drops nothing.  A lane holds the outcome for one member (a column of the tile) as bits.
+//      (bfloat16 needs no s, but its c is eight times as large and leaves more pairs to the exact chains: 10M x 32, trees 3 to 10 31.6 -> 30.5 ms.)
 //   3. The bits become a list of pairs ordered by member.  A turn takes up to 64 of them, whole members, one pair per lane: the exact
 //      chains from LDS, the members' K-NN rows (up to 256 slots) to LDS, then every lane counts the entries of its row below its
 //      candidate (one 64-bit comparison of (distance, index) each), sees whether the row holds the candidate already, and counts the member's
@@ -28,7 +31,7 @@
 // One workgroup per bucket, no barrier after the norms; a row is owned by one wavefront.  LDS for three workgroups per compute unit
 // (42 pieces of 1,280 bytes at D = 32: 128 bytes more mean two workgroups, and the last tree takes 4.1 ms instead of 2.8).
 //
-// 10M x 32, K = 32, buckets of 64..256, 10 trees, trees 3 to 10: 10.0 8.6 7.8 7.4 7.1 6.8 6.6 6.4 -> 7.8 5.1 4.1 3.5 3.2 3.0 2.9 2.8 ms;
+// 10M x 32, K = 32, buckets of 64..256, 10 trees, trees 3 to 10: 10.0 8.6 7.8 7.4 7.1 6.8 6.6 6.4 -> 7.4 4.9 3.9 3.4 3.1 2.9 2.8 2.7 ms;
 // loading and storing every row of a tree's buckets alone takes 2.1 ms, the rest is vector instructions (93 per row in the last tree, 244 in the
 // third; 400 and 600 before).  Requesting the rows of the next turn during this one: 12 % slower.
 #include "rsfk_common.hpp"
@@ -38,6 +41,7 @@
 #include "bucket_knn_stage.hpp"
 #include "bucket_knn_turn.hpp"
 #include <algorithm>
+#include <cmath>
 
 namespace rsfk {
 
@@ -60,7 +64,7 @@ __global__ __launch_bounds__(kRowsThreads, 3) void k_bucket_knn_rows_screen(cons
                                                                              const int* __restrict__ ids, const int* __restrict__ starts,
                                                                              const int* __restrict__ sizes, int min_size, int max_size,
                                                                              int* __restrict__ knn_idx, float* __restrict__ knn_dist,
-                                                                             int pitch, int per_k, uint32_t per_np, float c_err, float over)
+                                                                             int pitch, int per_k, uint32_t per_np, float c_err, float over, float lost)
 {
     extern __shared__ __align__(16) float lds_r[];
     float* rows = lds_r;                                          // 64 NT rows of `pitch` floats
@@ -107,7 +111,8 @@ __global__ __launch_bounds__(kRowsThreads, 3) void k_bucket_knn_rows_screen(cons
         if (half == 0 && c < 16 * KS) L.mean[c] = sum * 0.0625f;          // (zero beyond the last dimension)
     }
     wave_lds_sync();
-    // dimensions 16 k + 8 half .. of point r, minus the common point, and as operand of the matrix cores
+    // dimensions 16 k + 8 half .. of point r, minus the common point (times scale, once the mean is), and as operand of the matrix cores
+    float scale = 1.0f;
     auto centred = [&](int r, int k, float (&x)[8]) {
         const float* p = rows + r * pitch + 16 * k + 8 * half;
         float4 a = *reinterpret_cast<const float4*>(p);
@@ -119,15 +124,18 @@ __global__ __launch_bounds__(kRowsThreads, 3) void k_bucket_knn_rows_screen(cons
         }
         const float4 ma = *reinterpret_cast<const float4*>(&L.mean[16 * k + 8 * half]);
         const float4 mb = *reinterpret_cast<const float4*>(&L.mean[16 * k + 8 * half + 4]);
-        x[0] = a.x - ma.x; x[1] = a.y - ma.y; x[2] = a.z - ma.z; x[3] = a.w - ma.w;
-        x[4] = b.x - mb.x; x[5] = b.y - mb.y; x[6] = b.z - mb.z; x[7] = b.w - mb.w;
+        // (a power of two: s a - s m rounds as a - m does)
+        x[0] = __builtin_fmaf(a.x, scale, -ma.x); x[1] = __builtin_fmaf(a.y, scale, -ma.y);
+        x[2] = __builtin_fmaf(a.z, scale, -ma.z); x[3] = __builtin_fmaf(a.w, scale, -ma.w);
+        x[4] = __builtin_fmaf(b.x, scale, -mb.x); x[5] = __builtin_fmaf(b.y, scale, -mb.y);
+        x[6] = __builtin_fmaf(b.z, scale, -mb.z); x[7] = __builtin_fmaf(b.w, scale, -mb.w);
     };
     auto operand = [&](int r, int k) {
         float x[8];
         centred(r, k, x);
         typedef __attribute__((ext_vector_type(8))) float f32x8;
         const f32x8 v = {x[0], x[1], x[2], x[3], x[4], x[5], x[6], x[7]};
-        return __builtin_convertvector(v, bf16x8);
+        return __builtin_convertvector(v, f16x8);
     };
     for (int T = wave; 32 * T < s; T += kRowsWaves) {
         float n = 0.0f;
@@ -139,8 +147,30 @@ __global__ __launch_bounds__(kRowsThreads, 3) void k_bucket_knn_rows_screen(cons
             for (int u = 0; u < 8; ++u) n = __builtin_fmaf(x[u], x[u], n);
         }
         n += __shfl_xor(n, 32, 64);
-        if (half == 0) nhalf[32 * T + col] = n < 1e37f ? -0.5f * (1.0f - c_err) * n : INFINITY;
+        if (half == 0) nhalf[32 * T + col] = n;
     }
+    __syncthreads();
+    // s and R, the same for all wavefronts; from here on lengths are in units of s
+    float far = 0.0f;
+#pragma unroll
+    for (int u = 0; u < NT; ++u) {
+        const float n = 64 * u + lane < s ? nhalf[64 * u + lane] : 0.0f;
+        far = n < 1e37f ? fmaxf(far, n) : far;
+    }
+    far = wave_max(far);
+    const int e2 = (int)(__float_as_uint(far) >> 23) - 126;      // far < 2^e2
+    scale = __uint_as_float((uint32_t)(127 + max(-60, min(60, 14 - ((e2 + 1) >> 1)))) << 23);
+    const float scale2 = scale * scale;
+    const float z = lost * (4.1f * scale * sqrtf(far) + 2.1f * lost);
+    __syncthreads();                                              // the norms have been read
+#pragma unroll
+    for (int c0 = 0; c0 < 16 * KS; c0 += 64)
+        if (c0 + lane < 16 * KS) L.mean[c0 + lane] *= scale;
+    for (int T = wave; 32 * T < s; T += kRowsWaves)
+        if (half == 0) {
+            const float n = nhalf[32 * T + col];
+            nhalf[32 * T + col] = n < 1e37f ? -0.5f * (1.0f - c_err) * n * scale2 : INFINITY;
+        }
     __syncthreads();
 
     RowTurn turn(K, per_k);
@@ -149,10 +179,10 @@ __global__ __launch_bounds__(kRowsThreads, 3) void k_bucket_knn_rows_screen(cons
         const int i = 32 * T + col;
         const int gid = lids[i];
         const float tau = __shfl(T < kRowsWaves ? tau_of[0] : tau_of[NT > 2 ? 1 : 0], col, 64);
-        bf16x8 mem[KS];
+        f16x8 mem[KS];
 #pragma unroll
         for (int k = 0; k < KS; ++k) mem[k] = operand(i, k);
-        const float limit = -nhalf[i] - 0.5f * (tau * over + 1e-35f);
+        const float limit = -nhalf[i] - 0.5f * ((tau * over + 1e-35f) * scale2 + z);
         uint32_t bits[NT];
 #pragma unroll
         for (int w = 0; w < NT; ++w) {
@@ -169,7 +199,7 @@ __global__ __launch_bounds__(kRowsThreads, 3) void k_bucket_knn_rows_screen(cons
                 }
 #pragma unroll
                 for (int k = 0; k < KS; ++k)
-                    g = __builtin_amdgcn_mfma_f32_32x32x16_bf16(operand(32 * J + col, k), mem[k], g, 0, 0, 0);
+                    g = __builtin_amdgcn_mfma_f32_32x32x16_f16(operand(32 * J + col, k), mem[k], g, 0, 0, 0);
                 uint32_t b = 0;
 #pragma unroll
                 for (int r = 15; r >= 0; --r) b = b + b + (g[r] < limit ? 0u : 1u);
@@ -270,13 +300,14 @@ int launch_cfg(const float* points, int D, int K, const int* ids, const int* sta
 {
     const int pitch = bucket_rows_pitch(D);
     const size_t lds = (size_t)64 * NT * (pitch + 2) * sizeof(float) + kRowsWaves * sizeof(WaveLds<KS>);
-    const float c_err = 1.05f / 128.0f + (float)(64 * KS + 16) / 8388608.0f;
+    const float c_err = 1.05f / 1024.0f + (float)(64 * KS + 16) / 8388608.0f;
+    const float lost = std::sqrt((float)D) / 16384.0f;
     const double gamma = (double)(D + 8) / 4194304.0;
     const float over = (float)((1.0 + 1e-6) / (1.0 - gamma));
     auto kern = k_bucket_knn_rows_screen<NT, KS>;
     RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     hipLaunchKernelGGL(kern, dim3((unsigned)n_buckets), dim3(kRowsThreads), lds, stream, points, D, K, ids, starts, sizes, min_size,
-                       max_size, knn_idx, knn_dist, pitch, turn_per_k(K), rows_per_piece(D), c_err, over);
+                       max_size, knn_idx, knn_dist, pitch, turn_per_k(K), rows_per_piece(D), c_err, over, lost);
     RSFK_HIP(hipGetLastError());
     return 0;
 }
