@@ -743,29 +743,32 @@ __global__ __launch_bounds__(64 * WAVES, 5) void k_explore_join(JoinCopy jc, int
     }
 }
 
-// The join for rows of at most 32 neighbours and points of at most 128 dimensions (KS = steps of 16 dimensions, fixed
-// at compile time: 2, 4 or 8).  One word of marks per graph entry; the rows of the neighbours of q are loaded once
+// The join for points of at most 128 dimensions where no codes are kept (KS = steps of 16 dimensions, fixed
+// at compile time: 2, 4 or 8).  A wavefront takes 32 neighbours of q, one word of marks per graph entry; MANY: rows of more than 32
+// neighbours, MW wavefronts beside each other for a q, which find its tiles in the caches.  The rows of the neighbours are loaded once
 // and stay in registers for all tiles of R(q); the norm and last slot of the points of a tile travel while their rows
 // are fetched.  A wavefront then has three dependent trips to memory per q (row offsets and neighbours | their rows
 // and the elements of R(q) | the rows of those points) instead of five, and short rows leave room for twice the
-// wavefronts per SIMD.  The bound is that of k_explore_join.
-template <int WAVES, int KS>
+// wavefronts per SIMD.  The bound is that of k_explore_join.  (Against it: 1M x 100, K = 48 a
+// pass 39.6 -> 37.9 ms, 1M x 24, K = 36 7.63 -> 7.39, 123,457 x 37, K = 45 1.49 -> 1.44.)
+template <int WAVES, int KS, bool MANY>
 __global__ __launch_bounds__(64 * WAVES) void k_explore_join_short(JoinCopy jc, int N, int K, const int* __restrict__ old_idx,
                                                                     const float* __restrict__ bars,
                                                                     const int* __restrict__ offs, const int* __restrict__ rev,
-                                                                    uint32_t* __restrict__ pass, int bpitch, int ksteps,
+                                                                    uint32_t* __restrict__ pass, int MW, int bpitch, int ksteps,
                                                                     float kappa, float any_rel, float any_abs, uint32_t div_m, int div_s,
                                                                     const int* __restrict__ order)
 {
     __shared__ int pid_s[WAVES][32];
     __shared__ float pn_s[WAVES][32], pbar_s[WAVES][32];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int item = die_local_place(blockIdx.x, gridDim.x) * WAVES + wave;
+    const int unit = __builtin_amdgcn_readfirstlane(die_local_place(blockIdx.x, gridDim.x) * WAVES + wave);
+    const int item = MANY ? (int)((unsigned)unit / (unsigned)MW) : unit, ct = MANY ? unit - item * MW : 0;
     if (item >= N) return;                                // whole wavefront leaves together
     const int q = order ? order[item] : item;
     const int r0 = offs[q], R = offs[q + 1] - r0;
     const int col = lane & 31, hi = lane >> 5;
-    int cid = col < K ? old_idx[(size_t)q * K + col] : -1;
+    int cid = 32 * ct + col < K ? old_idx[(size_t)q * K + 32 * ct + col] : -1;
     if (R <= 32 * (int)blockIdx.y) return;
     if (cid < 0 || cid >= N) cid = -1;
     const uint16_t* rb = jc.rows + (size_t)(cid >= 0 ? cid : q) * (size_t)bpitch + 8 * hi;
@@ -832,7 +835,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_join_short(JoinCopy jc, 
             if (lane == m_lo + 4) mine = (uint32_t)(bm >> 32);
             if ((i & 3) == 3) __builtin_amdgcn_sched_barrier(0);   // four at a time: all sixteen at once take too many registers
         }
-        if (lane < np) pass[(size_t)my_e] = mine;
+        if (lane < np) pass[MANY ? (size_t)my_e * (size_t)MW + (size_t)ct : (size_t)my_e] = mine;
         wave_lds_sync();                                  // the tile's LDS values are read before the next tile writes them
     }
 }
@@ -842,20 +845,21 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_join_short(JoinCopy jc, 
 // points of R(q) and all neighbours of q pass through LDS together, 64 dimensions at a time (the next 64 are requested
 // while these are used), and the wavefronts share the pairs (tile of R(q), group of neighbours) among them, each
 // keeping the accumulators of its pairs: every row is read once per 96 points of R(q).  Bound and outputs are those
-// of k_explore_join.  NPW = pairs per wavefront (3: K <= 128, 6: K <= 256); the
-// first at three wavefronts per SIMD: 70,000 x 784, K = 90 6.9 -> 5.1 ms against two.
+// of k_explore_join.  K <= 128; at three wavefronts per SIMD
+// (70,000 x 784, K = 90 6.9 -> 5.1 ms against two).
 constexpr int kJwP = 96;                    // points of R(q) worked on together (three tiles)
 constexpr int kJwRowBytes = 144;            // 64 float16 values + 16 bytes: rows start in different banks
 
-template <bool BOUNDS, int NPW>
-__global__ __launch_bounds__(256, NPW == 3 ? 3 : 1) void k_explore_join_wg(JoinCopy jc, int N, int K, const int* __restrict__ old_idx,
+template <bool BOUNDS>
+__global__ __launch_bounds__(256, 3) void k_explore_join_wg(JoinCopy jc, int N, int K, const int* __restrict__ old_idx,
                                                          const float* __restrict__ bars, const int* __restrict__ offs,
                                                          const int* __restrict__ rev, uint32_t* __restrict__ pass,
                                                          uint16_t* __restrict__ bounds, int KP, int bpitch, int ksteps,
                                                          float kappa, float any_rel, float any_abs, uint32_t div_m, int div_s,
                                                          const int* __restrict__ order)
 {
-    constexpr int kPieces = (kJwP + (NPW == 3 ? 128 : 256)) * 8 / 256;      // 16-byte pieces a thread stages per step
+    constexpr int NPW = 3;                                                 // pairs per wavefront
+    constexpr int kPieces = (kJwP + 128) * 8 / 256;                        // 16-byte pieces a thread stages per step
     extern __shared__ __align__(16) unsigned char lds_jw[];
     unsigned char* rowsb = lds_jw;                                         // kJwP + KP rows of 144 bytes
     int* cq = reinterpret_cast<int*>(rowsb + (size_t)(kJwP + KP) * kJwRowBytes);
@@ -1214,32 +1218,39 @@ int launch_explore_join(ExploreWorkspace* w, const JoinCopy& jc, int N, int D, i
     hipLaunchKernelGGL(k_join_bars, dim3((unsigned)((N + 255) / 256) + 1), dim3(256), 0, stream, jc, jc.scale(), knn_dist, N, K,
                        one_minus_gamma, w->bars);
     RSFK_HIP(hipGetLastError());
-    if (!w->bounds && KP == 32 && ksteps <= 8) {
-        const dim3 grid(grid_for_dies(((size_t)N + kWaves - 1) / kWaves), parts), block(64 * kWaves);
-#define RSFK_JOIN_SHORT(KSV)                                                                                                \
-        hipLaunchKernelGGL((k_explore_join_short<kWaves, KSV>), grid, block, 0, stream, jc, N, K, old_idx, w->bars, w->offs, \
-                           w->rev, w->pass, join_pitch(D), ksteps, kappa, any_rel, any_abs, w->div_m, w->div_s, order)
-        if (ksteps <= 2) RSFK_JOIN_SHORT(2);
-        else if (ksteps <= 4) RSFK_JOIN_SHORT(4);
-        else RSFK_JOIN_SHORT(8);
-#undef RSFK_JOIN_SHORT
-    } else if (KP > 32 && join_wg_on()) {
-        // one workgroup per q: every row once per 96 points of R(q).  (Rows of at most 32 neighbours have one pair per
-        // tile of R(q): too little for four wavefronts; 1M x 256, K = 32: 8.1 ms against 12.6.)
+    const int MW = KP >> 5;
+    // One workgroup per q reads every row once per 96 points of R(q), one wavefront per q (and 32 neighbours) again for every group of 32
+    // neighbours, so the former pays with the bytes that are read again, D (K - 24) or so, sooner with more groups; up to 32 neighbours
+    // are one pair per tile of R(q), too little for four wavefronts (1M x 256, K = 32: 8.1 ms against 12.6).  A pass, a wavefront per q -> a
+    // workgroup: 123,457 x 37, K = 45 1.49 -> 2.08 ms, 300,000 x 64, K = 64 10.1 -> 11.6, x 200 16.7 -> 16.8, x 300 20.0 -> 18.5, 200,000 x 600, K = 40
+    // 10.9 -> 10.4, 300,000 x 64, K = 90 17.8 -> 19.0, x 100 20.8 -> 20.8, 100,000 x 128, K = 90 7.07 -> 6.89, x 400 12.3 -> 9.6, 200,000 x 16, K = 128 19.3
+    // -> 19.6, x 32 17.0 -> 16.9, 100,000 x 256, K = 128 15.0 -> 11.4.  Above 128 neighbours its accumulators leave one wavefront per SIMD: 100,000 x 32,
+    // K = 160 18.3 -> 29.7.
+    if (KP > 32 && KP <= 128 && join_wg_on() && D * (K - 24) > (MW == 2 ? 8000 : MW == 3 ? 6500 : 3000)) {
         const size_t lds_wg = (size_t)(kJwP + KP) * kJwRowBytes + (size_t)KP * 12 + (size_t)kJwP * 24;
-#define RSFK_JOIN_WG(BV, NV)                                                                                                \
+#define RSFK_JOIN_WG(BV)                                                                                                    \
         do {                                                                                                               \
-            RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_explore_join_wg<BV, NV>),                         \
+            RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_explore_join_wg<BV>),                             \
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_wg));                       \
-            hipLaunchKernelGGL((k_explore_join_wg<BV, NV>), dim3(grid_for_dies((size_t)N), parts), dim3(256), lds_wg, stream, jc, N, K,  \
+            hipLaunchKernelGGL((k_explore_join_wg<BV>), dim3(grid_for_dies((size_t)N), parts), dim3(256), lds_wg, stream, jc, N, K,  \
                                old_idx, w->bars, w->offs, w->rev, w->pass, w->bounds, KP, join_pitch(D), ksteps, kappa,  \
                                any_rel, any_abs, w->div_m, w->div_s, order);                                                \
         } while (0)
-        if (w->bounds && KP <= 128) RSFK_JOIN_WG(true, 3);
-        else if (w->bounds) RSFK_JOIN_WG(true, 6);
-        else if (KP <= 128) RSFK_JOIN_WG(false, 3);
-        else RSFK_JOIN_WG(false, 6);
+        if (w->bounds) RSFK_JOIN_WG(true);
+        else RSFK_JOIN_WG(false);
 #undef RSFK_JOIN_WG
+    } else if (!w->bounds && ksteps <= 8) {
+        const dim3 grid(grid_for_dies(((size_t)N * (size_t)MW + kWaves - 1) / kWaves), parts), block(64 * kWaves);
+#define RSFK_JOIN_SHORT(KSV, MANYV)                                                                                         \
+        hipLaunchKernelGGL((k_explore_join_short<kWaves, KSV, MANYV>), grid, block, 0, stream, jc, N, K, old_idx, w->bars, w->offs, \
+                           w->rev, w->pass, MW, join_pitch(D), ksteps, kappa, any_rel, any_abs, w->div_m, w->div_s, order)
+        if (MW == 1 && ksteps <= 2) RSFK_JOIN_SHORT(2, false);
+        else if (MW == 1 && ksteps <= 4) RSFK_JOIN_SHORT(4, false);
+        else if (MW == 1) RSFK_JOIN_SHORT(8, false);
+        else if (ksteps <= 2) RSFK_JOIN_SHORT(2, true);
+        else if (ksteps <= 4) RSFK_JOIN_SHORT(4, true);
+        else RSFK_JOIN_SHORT(8, true);
+#undef RSFK_JOIN_SHORT
     } else if (w->bounds)
         hipLaunchKernelGGL((k_explore_join<kWaves, true>), dim3(grid_for_dies(((size_t)N + kWaves - 1) / kWaves), parts), dim3(64 * kWaves), lds,
                            stream, jc, N, K, old_idx, w->bars, w->offs, w->rev, w->pass, w->bounds, KP, join_pitch(D), ksteps,

@@ -531,6 +531,31 @@ def test_explore_batches_merged_by_rank(gpu, orc, rng, N, D, K, values):
         assert_knn_equal(gi, gd, oi, od)
 
 
+# both sides of every line between the joins: neighbours in one to seven groups of 32, whole and with one over; dimensions around the
+# largest that stay in registers and around those from which a workgroup takes a point
+@pytest.mark.parametrize("N,D,K", [(900, 128, 33), (900, 129, 33), (700, 64, 64), (700, 200, 64), (600, 201, 64), (500, 500, 40), (500, 501, 40), (700, 32, 65),
+                                   (600, 98, 90), (600, 99, 90), (700, 90, 96), (600, 17, 97), (600, 28, 128), (600, 29, 128), (500, 16, 129), (400, 130, 200)])
+@pytest.mark.parametrize("data", ["normal", "notfinite", "no codes"])
+def test_explore_join_of_rows_of_many_neighbours(gpu, orc, rng, monkeypatch, N, D, K, data):
+    """A wavefront per 32 neighbours of a point, a wavefront per point, a workgroup per point, with and without room for the codes == the
+    oracle, two passes."""
+    if data == "no codes":
+        monkeypatch.setenv("RSFK_OPTIONAL_MB", "0")
+    X = rng.standard_normal((N, D)).astype(np.float32)
+    perm, ls, lz, _ = orc.build_tree(X, K + 1, 2 * K + 2, 5000, 0)
+    if data == "notfinite":
+        X[3, D // 2] = np.nan
+        X[N - 1, D - 1] = -np.inf
+    oi, od = orc.init_lists(N, K, self_in=True)
+    orc.bucket_knn(X, K, perm, lz, oi, od, starts=ls)
+    gi, gd = oi.copy(), od.copy()
+    _say("explore join", N, D, K, data)
+    for _ in range(2):
+        orc.explore(X, K, oi, od)
+        gpu.explore(X, K, gi, gd, 1)
+        assert_knn_equal(gi, gd, oi, od)
+
+
 @pytest.mark.parametrize("values", ["far", "tiny", "huge", "outlier", "spread", "notfinite"])
 @pytest.mark.parametrize("N,D,K", [(2500, 16, 8), (2500, 33, 32), (1500, 129, 20), (1500, 40, 70)])
 def test_explore_screens_rows_of_any_magnitude(gpu, orc, rng, N, D, K, values):
