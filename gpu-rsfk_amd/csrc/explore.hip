@@ -333,7 +333,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore(const float* __restrict_
 // the graph has the mask of neighbour slots at pass[p K + k] (entries without a valid neighbour have none).  One wavefront per point: gather
 // the marked ids, drop repeats and ids the row holds (hash set), exact distances, merge.  Points with
 // more marks than the LDS of this launch takes are appended to todo_out (for a launch with more LDS
-// per wavefront, or for the general kernel).  todo_in: the points to work on, or null for all.
+// per wavefront, or for the general kernel; share > 0: to the point's share of it, explore_ws_share_lists).  todo_in: the points to work on, or null for all.
 // Per-wavefront LDS (ints): tile[64*20] | xrow[dpad] | table[table_size] | srow[K] | marked[3/4 table_size].
 // Number of entry (p, k) of the graph snapshot, p K + k, or -1 when the slot holds no valid neighbour (the join writes
 // nothing for such an entry).
@@ -378,7 +378,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_merge(const float* __res
                                                                int wave_lds_ints, int dpad, int direct_max,
                                                                const uint32_t* __restrict__ pass, JoinBounds jb,
                                                                const int* __restrict__ todo_in, int n_in,
-                                                               int* __restrict__ todo_out, int* __restrict__ n_out,
+                                                               int* __restrict__ todo_out, int share, int* __restrict__ n_out,
                                                                unsigned long long* __restrict__ stat,
                                                                const int* __restrict__ order)
 {
@@ -422,7 +422,8 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_merge(const float* __res
     const int n_given = wave_sum_i(bits);
     if (n_given == 0) return;
     if (n_given + K + 1 > table_size / 4 * 3) {
-        if (lane == 0) todo_out[atomicAdd(n_out, 1)] = p;
+        const int s = share > 0 ? slot % kTodoShares : 0;
+        if (lane == 0) todo_out[(size_t)s * (size_t)share + (size_t)atomicAdd(n_out + 32 * s, 1)] = p;
         return;
     }
     ExploreLds L;
@@ -1054,7 +1055,7 @@ int next_pow2(int v)
 template <int SL, int WAVES>
 int launch_merge(const float* points, int N, int D, int K, const int* old_idx, int* knn_idx, float* knn_dist, int table,
                  int wave_ints, int dpad, const uint32_t* pass, const JoinBounds& bounds, const int* todo_in, int n_in,
-                 int* todo_out, int* n_out, unsigned long long* stat, const int* order, hipStream_t stream)
+                 int* todo_out, int share, int* n_out, unsigned long long* stat, const int* order, hipStream_t stream)
 {
     const size_t lds = (size_t)WAVES * (size_t)wave_ints * sizeof(int);
     const int n_work = todo_in ? n_in : N;
@@ -1063,13 +1064,13 @@ int launch_merge(const float* points, int N, int D, int K, const int* old_idx, i
         RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_explore_merge<SL, WAVES, false>),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         hipLaunchKernelGGL((k_explore_merge<SL, WAVES, false>), grid, block, lds, stream, points, N, D, K, old_idx, knn_idx,
-                           knn_dist, table, wave_ints, dpad, merge_direct_max(), pass, bounds, todo_in, n_in, todo_out, n_out,
+                           knn_dist, table, wave_ints, dpad, merge_direct_max(), pass, bounds, todo_in, n_in, todo_out, share, n_out,
                            stat, order);
     } else {
         RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_explore_merge<SL, WAVES, true>),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         hipLaunchKernelGGL((k_explore_merge<SL, WAVES, true>), grid, block, lds, stream, points, N, D, K, old_idx, knn_idx,
-                           knn_dist, table, wave_ints, dpad, merge_direct_max(), pass, bounds, todo_in, n_in, todo_out, n_out,
+                           knn_dist, table, wave_ints, dpad, merge_direct_max(), pass, bounds, todo_in, n_in, todo_out, share, n_out,
                            stat, order);
     }
     RSFK_HIP(hipGetLastError());
@@ -1088,18 +1089,27 @@ int merge_wave_ints(int table, int dpad, int K, bool with_bounds = false)
 
 int dispatch_merge(int sl, int waves, const float* points, int N, int D, int K, const int* old_idx, int* knn_idx,
                    float* knn_dist, int table, int dpad, const uint32_t* pass, const JoinBounds& bounds, const int* todo_in,
-                   int n_in, int* todo_out, int* n_out, unsigned long long* stat, const int* order, hipStream_t stream)
+                   int n_in, int* todo_out, int share, int* n_out, unsigned long long* stat, const int* order, hipStream_t stream)
 {
     const int wi = merge_wave_ints(table, dpad, K, bounds.codes != nullptr);
 #define RSFK_MERGE_CASE(SLV, WV)                                                                                        \
     if (sl == SLV && waves == WV)                                                                                       \
         return launch_merge<SLV, WV>(points, N, D, K, old_idx, knn_idx, knn_dist, table, wi, dpad, pass, bounds, \
-                                     todo_in, n_in, todo_out, n_out, stat, order, stream);
+                                     todo_in, n_in, todo_out, share, n_out, stat, order, stream);
     RSFK_MERGE_CASE(1, 4) RSFK_MERGE_CASE(1, 2) RSFK_MERGE_CASE(1, 1)
     RSFK_MERGE_CASE(2, 4) RSFK_MERGE_CASE(2, 2) RSFK_MERGE_CASE(2, 1)
     RSFK_MERGE_CASE(4, 4) RSFK_MERGE_CASE(4, 2) RSFK_MERGE_CASE(4, 1)
 #undef RSFK_MERGE_CASE
     RSFK_CHECK(false, "exploration: no merge kernel for this configuration");
+}
+
+// The shares of a list to one list (a workgroup each).
+__global__ __launch_bounds__(256) void k_todo_join(const int* __restrict__ lists, int share, const int* __restrict__ numbers, int* __restrict__ out)
+{
+    const int s = blockIdx.x, lane = threadIdx.x & 63;
+    const int mine = lane < kTodoShares ? numbers[32 * lane] : 0, n = read_lane_i(mine, s);
+    const int at = wave_sum_i(lane < s ? mine : 0);
+    for (int i = threadIdx.x; i < n; i += 256) out[at + i] = lists[(size_t)s * (size_t)share + i];
 }
 
 template <int SL, int WAVES>
@@ -1205,6 +1215,9 @@ int launch_explore(const float* points, const Bf16Copy* bf, const JoinCopy* jc, 
         const uint32_t* pass = explore_ws_pass(ws);
         int* listA = explore_ws_todo(ws, 0);
         int* listB = explore_ws_todo(ws, 1);
+        int* lists = explore_ws_share_lists(ws);          // what the small set hands back, in shares; listA once they are joined
+        int* numbers = explore_ws_shares(ws);
+        const int share = todo_share(N);
         int n_back = 0;
         // (the bounds of the join, when it kept them and the set with a bound per place still fits)
         JoinBounds wave_bounds = explore_ws_bounds(ws), no_bounds = wave_bounds;
@@ -1234,14 +1247,14 @@ int launch_explore(const float* points, const Bf16Copy* bf, const JoinCopy* jc, 
         // the order they are taken in): when it has to hand most of them back -- rows of many neighbours that are far
         // from done have thousands of marks each -- the launch over all points would only find that out for every
         // one of them (70,000 x 784, K = 90, 10 trees: all of them, 0.9 ms of a 25 ms pass).
-        constexpr int kSample = 2048;
+        constexpr int kSample = 2048;                      // (a multiple of kTodoShares: no share holds more than its part of N)
         int first = 0;                                    // points the small set has been tried on
         bool rest_per_wg = false;
         if (second && per_wg && order != nullptr && N > 2 * kSample) {
             if (dispatch_merge(sl, 4, points, N, D, K, old_idx, knn_idx, knn_dist, small_table, dpad, pass, wave_bounds, order,
-                               kSample, listA, listA + N, stat, nullptr, stream))
+                               kSample, lists, share, numbers, stat, nullptr, stream))
                 return 1;
-            if (fetch_words(listA + N, 1, &n_back, stream)) return 1;
+            if (fetch_total(numbers, kTodoShares, 32, &n_back, stream)) return 1;
             first = kSample;
             rest_per_wg = n_back > kSample / 2;
         }
@@ -1249,11 +1262,13 @@ int launch_explore(const float* points, const Bf16Copy* bf, const JoinCopy* jc, 
             // everything but the sample straight to the workgroup-per-point kernel (its list: the rest of the order)
             if (merge_wg(order + first, N - first)) return 1;
         } else if (dispatch_merge(sl, 4, points, N, D, K, old_idx, knn_idx, knn_dist, small_table, dpad, pass, wave_bounds,
-                                  first > 0 ? order + first : nullptr, first > 0 ? N - first : 0, listA, listA + N, stat,
+                                  first > 0 ? order + first : nullptr, first > 0 ? N - first : 0, lists, share, numbers, stat,
                                   first > 0 ? nullptr : order, stream)) {
             return 1;
         }
-        if (fetch_words(listA + N, 1, &n_back, stream)) return 1;
+        if (fetch_total(numbers, kTodoShares, 32, &n_back, stream)) return 1;
+        // (20,000 x 32 in 64 clusters, K = 32: 11,193 points come back, one counter took 0.10 of the launch's 0.136 ms)
+        if (n_back > 0) hipLaunchKernelGGL(k_todo_join, dim3(kTodoShares), dim3(256), 0, stream, lists, share, numbers, listA);
         n_todo = n_back;                                 // what the small set handed back (of the sample, or of all points)
         todo = listA;
         if (n_todo == 0 && !rest_per_wg) return 0;
@@ -1263,7 +1278,7 @@ int launch_explore(const float* points, const Bf16Copy* bf, const JoinCopy* jc, 
                 rc = 0;
             else if (!per_wg)
                 rc = dispatch_merge(sl, big_waves, points, N, D, K, old_idx, knn_idx, knn_dist, big_table, dpad, pass,
-                                    no_bounds, listA, n_todo, listB, listB + N, stat, nullptr, stream);
+                                    no_bounds, listA, n_todo, listB, 0, listB + N, stat, nullptr, stream);
             else
                 rc = merge_wg(listA, n_todo);
             if (rc)

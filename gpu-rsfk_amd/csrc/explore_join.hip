@@ -72,9 +72,16 @@ struct ExploreWorkspace {
     int* fine_size = nullptr;   // n_coarse << (cshift - fshift)
     int* fine_start = nullptr;  // the same + 1
     int* sub_off = nullptr;     // n_sub x fine bins per coarse bin
-    int* todo = nullptr;       // two lists of N+1 ints: points left over by a launch; entry N = their number
+    int* todo = nullptr;       // two lists of N+1 ints: points left over by a launch; entry N = their number; then the shares of such a list, and their numbers
 };
+int* explore_ws_shares(ExploreWorkspace* w)
+{
+    const size_t at = 2 * ((size_t)w->N + 1) + (size_t)kTodoShares * (size_t)todo_share(w->N);
+    return w->todo + ((at + 31) & ~(size_t)31);
+}
 namespace {
+
+size_t todo_ints(int N) { return 2 * ((size_t)N + 1) + (size_t)kTodoShares * (size_t)todo_share(N) + 32 + 32 * (size_t)kTodoShares; }
 
 typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
@@ -108,11 +115,12 @@ bool rev_bins(int N, int* shift, int* n_bins)
     return *n_bins <= kMaxBins;
 }
 
-__global__ void k_zero(int* a, int n, int* counter0, int* counter1)
+__global__ void k_zero(int* a, int n, int* counter0, int* counter1, int* shares)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) a[i] = 0;
     if (i == 0) { *counter0 = 0; *counter1 = 0; }
+    if (i < kTodoShares) shares[32 * i] = 0;
 }
 
 // exclusive scan of one value per thread over the workgroup (blockDim.x a multiple of 64, at most 1024); returns the
@@ -1085,7 +1093,7 @@ int explore_ws_alloc(ExploreWorkspace** out, int N, int K, bool with_bounds, boo
         dm(&w->offs, (size_t)N + 1) != hipSuccess || dm(&w->bin_size, (size_t)w->n_bins) != hipSuccess ||
         dm(&w->bin_start, (size_t)w->n_bins + 1) != hipSuccess ||
         dm(&w->part_off, (size_t)w->n_parts * (size_t)w->n_bins) != hipSuccess || (!graph_only && (dm(&w->pass, total * w->MW) != hipSuccess || dm(&w->bars, (size_t)N) != hipSuccess)) ||
-        dm(&w->todo, 2 * ((size_t)N + 1)) != hipSuccess) {
+        dm(&w->todo, todo_ints(N)) != hipSuccess) {
         explore_ws_free(w);
         if (!graph_only) set_last_error("exploration workspace: out of device memory");
         return 1;
@@ -1114,6 +1122,8 @@ void explore_ws_free(ExploreWorkspace* w)
 
 const uint32_t* explore_ws_pass(const ExploreWorkspace* w) { return w->pass; }
 const JoinBounds& explore_ws_bounds(const ExploreWorkspace* w) { return w->view; }
+// The shares: kTodoShares lists of todo_share(N) points, the number of each in a cache line of its own.
+int* explore_ws_share_lists(ExploreWorkspace* w) { return w->todo + 2 * ((size_t)w->N + 1); }
 int* explore_ws_todo(ExploreWorkspace* w, int which) { return w->todo + (size_t)which * ((size_t)w->N + 1); }
 
 bool explore_ws_takes(int N, int K)
@@ -1132,9 +1142,9 @@ int launch_reversed_graph(ExploreWorkspace* w, const int* old_idx, int N, int K,
     if (w->staged) {
         const int nc = w->n_coarse, per = 1 << (w->cshift - w->fshift);
         hipLaunchKernelGGL(k_zero, dim3((unsigned)((nc + 255) / 256)), dim3(256), 0, stream, w->bin_size, nc, w->todo + N,
-                           w->todo + 2 * (size_t)N + 1);
+                           w->todo + 2 * (size_t)N + 1, explore_ws_shares(w));
         hipLaunchKernelGGL(k_zero, dim3((unsigned)((w->n_fine + 255) / 256)), dim3(256), 0, stream, w->fine_size, w->n_fine,
-                           w->todo + N, w->todo + 2 * (size_t)N + 1);
+                           w->todo + N, w->todo + 2 * (size_t)N + 1, explore_ws_shares(w));
         hipLaunchKernelGGL(k_bin_count, dim3((unsigned)w->n_parts), dim3(256), (size_t)nc * sizeof(int), stream, old_idx, total,
                            w->per_part, N, w->cshift, nc, w->bin_size, w->part_off);
         hipLaunchKernelGGL(k_bin_scan, dim3(1), dim3(256), 0, stream, w->bin_size, nc, w->bin_start, w->offs + N);
@@ -1155,7 +1165,7 @@ int launch_reversed_graph(ExploreWorkspace* w, const int* old_idx, int N, int K,
     } else if (w->tiled) {
         const int nc = w->n_coarse;
         hipLaunchKernelGGL(k_zero, dim3((unsigned)((nc + 255) / 256)), dim3(256), 0, stream, w->bin_size, nc, w->todo + N,
-                           w->todo + 2 * (size_t)N + 1);
+                           w->todo + 2 * (size_t)N + 1, explore_ws_shares(w));
         hipLaunchKernelGGL(k_bin_count, dim3((unsigned)w->n_parts), dim3(1024), (size_t)nc * sizeof(int), stream, old_idx, total,
                            w->per_part, N, w->cshift, nc, w->bin_size, w->part_off);
         hipLaunchKernelGGL(k_bin_scan, dim3(1), dim3(256), 0, stream, w->bin_size, nc, w->bin_start, w->offs + N);
@@ -1171,7 +1181,7 @@ int launch_reversed_graph(ExploreWorkspace* w, const int* old_idx, int N, int K,
     const int nbins = w->n_bins;
     const size_t bin_lds = (size_t)nbins * sizeof(int);
     hipLaunchKernelGGL(k_zero, dim3((unsigned)((nbins + 255) / 256)), dim3(256), 0, stream, w->bin_size, nbins, w->todo + N,
-                       w->todo + 2 * (size_t)N + 1);
+                       w->todo + 2 * (size_t)N + 1, explore_ws_shares(w));
     hipLaunchKernelGGL(k_bin_count, dim3((unsigned)w->n_parts), dim3(256), bin_lds, stream, old_idx, total, w->per_part, N,
                        w->shift, nbins, w->bin_size, w->part_off);
     hipLaunchKernelGGL(k_bin_scan, dim3(1), dim3(256), 0, stream, w->bin_size, nbins, w->bin_start, w->offs + N);

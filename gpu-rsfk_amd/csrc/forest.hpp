@@ -208,6 +208,12 @@ const uint32_t* explore_ws_pass(const ExploreWorkspace* w);
 struct JoinBounds;
 const JoinBounds& explore_ws_bounds(const ExploreWorkspace* w);
 int* explore_ws_todo(ExploreWorkspace* w, int which);
+// A list that many points may go to at once is kept in shares, a counter each: additions to one cache line are carried out one after
+// the other, about 14 ns each.  Point number i of a launch (of at most N points) has share i % kTodoShares.
+constexpr int kTodoShares = 32;
+inline int todo_share(int N) { return (N + kTodoShares - 1) / kTodoShares; }
+int* explore_ws_share_lists(ExploreWorkspace* w);
+int* explore_ws_shares(ExploreWorkspace* w);               // numbers, 32 words apart
 // order: null, or a permutation of the points that keeps nearby points together (the buckets of a tree): the points
 // are then worked on in that order, a contiguous eighth of it per die (die_local_place)
 int launch_explore_join(ExploreWorkspace* w, const JoinCopy& jc, int N, int D, int K, const int* old_idx,

@@ -288,6 +288,14 @@ __global__ void k_fetch(const int* __restrict__ a, int na, const int* __restrict
     for (int i = 0; i < nb; ++i) out->word[na + i] = b[i];
     __hip_atomic_store(&out->seq, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
+__global__ void k_fetch_total(const int* __restrict__ a, int n, int pitch, Fetched* out)
+{
+    int v = (int)threadIdx.x < n ? a[(size_t)threadIdx.x * (size_t)pitch] : 0;
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    if (threadIdx.x != 0) return;
+    out->word[0] = v;
+    __hip_atomic_store(&out->seq, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 // One workgroup of 256 threads.
 __global__ void k_fetch_sum(const float* __restrict__ a, int n, Fetched* out)
 {
@@ -319,6 +327,22 @@ int fetch_words(const int* a, int na, const int* b, int nb, int* host, hipStream
     const int rc = e != hipSuccess ? 1 : wait_for_word(&f->seq, 1, stream);
     if (e != hipSuccess) set_last_error(std::string("fetch: ") + hipGetErrorString(e));
     for (int i = 0; i < n && !rc; ++i) host[i] = f->word[i];
+    pin_free(p);
+    return rc;
+}
+
+int fetch_total(const int* a, int n, int pitch, int* host, hipStream_t stream)
+{
+    RSFK_CHECK(n >= 1 && n <= 64, "fetch: too many words");
+    void* p = nullptr;
+    if (pin_alloc(&p, sizeof(Fetched))) return 1;
+    Fetched* f = static_cast<Fetched*>(p);
+    __atomic_store_n(&f->seq, 0, __ATOMIC_RELEASE);
+    hipLaunchKernelGGL(k_fetch_total, dim3(1), dim3(64), 0, stream, a, n, pitch, f);
+    const hipError_t e = hipGetLastError();
+    const int rc = e != hipSuccess ? 1 : wait_for_word(&f->seq, 1, stream);
+    if (e != hipSuccess) set_last_error(std::string("fetch: ") + hipGetErrorString(e));
+    if (!rc) *host = f->word[0];
     pin_free(p);
     return rc;
 }

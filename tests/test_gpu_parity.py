@@ -531,6 +531,22 @@ def test_explore_batches_merged_by_rank(gpu, orc, rng, N, D, K, values):
         assert_knn_equal(gi, gd, oi, od)
 
 
+# fewer points than shares of the list, one point in the last share, whole shares; a workgroup per point after it (K = 100)
+@pytest.mark.parametrize("N,D,K,T", [(20, 4, 9, 3), (65, 3, 20, 4), (1025, 8, 32, 8), (4224, 6, 30, 6), (4500, 12, 100, 5)])
+def test_explore_points_with_many_marks_are_handed_on(gpu, capi, orc, rng, N, D, K, T):
+    """Clusters little larger than a row: the neighbours of a point's neighbours are its own, so that most points have more marks than
+    the first launch has room for and go to the next one through a list kept in shares."""
+    import torch
+    X = (rng.standard_normal((max(1, N // (2 * K)), D))[rng.integers(0, max(1, N // (2 * K)), N)] * 20 + rng.standard_normal((N, D))).astype(np.float32)
+    oi, od = orc.forest(X, K, T, K + 1, 2 * K + 2, 5000, 3, 2)
+    gi, gd = orc.init_lists(N, K, self_in=True)
+    dX, di, dd = (torch.from_numpy(a).cuda() for a in (X, gi, gd))
+    _say("explore handed on", N, D, K, T)
+    capi.knn_forest_device(T, K, N, D, K + 1, 2 * K + 2, 5000, 0, 3, 2, dX.data_ptr(), di.data_ptr(), dd.data_ptr())
+    torch.cuda.synchronize()
+    assert_knn_equal(di.cpu().numpy(), dd.cpu().numpy(), oi, od)
+
+
 # both sides of every line between the joins: neighbours in one to seven groups of 32, whole and with one over; dimensions around the
 # largest that stay in registers and around those from which a workgroup takes a point
 @pytest.mark.parametrize("N,D,K", [(900, 128, 33), (900, 129, 33), (700, 64, 64), (700, 200, 64), (600, 201, 64), (500, 500, 40), (500, 501, 40), (700, 32, 65),
