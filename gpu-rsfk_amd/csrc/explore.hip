@@ -351,31 +351,44 @@ constexpr int kFewCandidates = 32;
 // kernel its second wavefront per SIMD: 39 ms.)
 constexpr int kChainGroup = 4;
 constexpr int kMergeTile = 64 * (kMergeChunk + 4);
-// Rows of at most this many (padded) dimensions are read by the lane that runs their chain, 32 dimensions at a time,
-// without the transposing tile in LDS (exact_direct): the LDS of a wavefront shrinks by the tile.
+// Short rows are read by the lane that runs their chain, 32 dimensions at a time, without the transposing tile in LDS
+// (exact_direct): the LDS of a wavefront shrinks by the tile.  This is the size of a wavefront's memory that the launches are
+// planned with; what a launch then takes is merge_direct's choice.
 __host__ __device__ inline int merge_tile_ints(int dpad, int direct_max) { return dpad <= direct_max ? 0 : kMergeTile; }
 __host__ __device__ inline int merge_rank_at(int table, int K, bool with_bounds)
 {
     return table + ((K + 3) & ~3) + (with_bounds ? table / 4 * 7 : 0);
 }
-int merge_direct_max()
+int merge_direct_env()
 {
     static const int v = [] {
-        // measured: 1M x 100 merge 4.4 -> 3.4 ms, 10M x 32 43 -> 27 ms; 1M x 256 slower (eight steps, each a trip)
         const char* e = std::getenv("RSFK_MERGE_DIRECT");
-        return e ? std::atoi(e) : 128;
+        return e ? std::atoi(e) : -1;
     }();
     return v;
 }
+int merge_direct_max() { return merge_direct_env() >= 0 ? merge_direct_env() : 128; }
+// Does a launch read rows of this many dimensions without the tile?  With all candidates of a point to be evaluated the trips to
+// memory of a long row weigh more than the wavefronts that the tile's 5 KB keep out (measured: 1M x 100 merge 4.4 -> 3.4 ms without,
+// 10M x 32 43 -> 27 ms, 1M x 256 slower), hence 128.  Where the join's codes leave a point few of them, most lanes of the tile's
+// loads carry nothing and the wavefronts count for longer: whole pass at 1M x 256, K = 32 in clusters 15.5 -> 14.0 ms, 500k x 132
+// 5.97 -> 4.98, 150k x 280, K = 44 4.65 -> 4.15; 150k x 320, K = 33 3.98 -> 4.24, x 384, K = 36 4.93 -> 5.18: 288.  Rows that are not
+// in whole 16-byte pieces take four times the loads: 150k x 161, K = 16 1.23 -> 1.18, x 231 1.41 -> 1.48, x 255 1.45 -> 1.58: 192.
+constexpr int kDirectCoded = 288, kDirectCodedOdd = 192;
+bool merge_direct(int D, int dpad, bool coded)
+{
+    if (!coded || merge_direct_env() >= 0) return dpad <= merge_direct_max();
+    return dpad <= ((D & 3) == 0 ? kDirectCoded : kDirectCodedOdd);
+}
 
 
-// TILE: the candidates' rows go through the transposing tile (rows longer than direct_max dimensions); the two forms
+// TILE: the candidates' rows go through the transposing tile (not merge_direct); the two forms
 // are kernels of their own, so that the shorter one does not carry the registers of the other.
 template <int SL, int WAVES, bool TILE>
 __global__ __launch_bounds__(64 * WAVES) void k_explore_merge(const float* __restrict__ points, int N, int D, int K,
                                                                const int* __restrict__ old_idx, int* __restrict__ knn_idx,
                                                                float* __restrict__ knn_dist, int table_size,
-                                                               int wave_lds_ints, int dpad, int direct_max,
+                                                               int wave_lds_ints, int dpad,
                                                                const uint32_t* __restrict__ pass, JoinBounds jb,
                                                                const int* __restrict__ todo_in, int n_in,
                                                                int* __restrict__ todo_out, int share, int* __restrict__ n_out,
@@ -404,7 +417,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_merge(const float* __res
         pw[0] = pass[at * MW];
         if (MW > 1) pw[1] = pass[at * MW + 1];
         const float* xp0 = points + (size_t)p * D;
-        float* xr = reinterpret_cast<float*>(base + merge_tile_ints(dpad, direct_max));
+        float* xr = reinterpret_cast<float*>(base + (TILE ? kMergeTile : 0));
         for (int d = lane; d < dpad; d += 64) xr[d] = d < D ? xp0[d] : 0.0f;
         if (lane >= K) { row.idx[0] = -2; row.dist[0] = INFINITY; q_own = -1; }
         if (!(q_own >= 0 && q_own < N)) { pw[0] = 0u; pw[1] = 0u; }          // the join writes nothing for such an entry
@@ -428,7 +441,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_merge(const float* __res
     }
     ExploreLds L;
     L.tile = reinterpret_cast<float*>(base);
-    const int tile_ints = merge_tile_ints(dpad, direct_max);
+    constexpr int tile_ints = TILE ? kMergeTile : 0;
     L.xrow = reinterpret_cast<float*>(base + tile_ints);
     L.queue2 = nullptr;
     L.table = base + tile_ints + dpad;
@@ -1054,23 +1067,23 @@ int next_pow2(int v)
 
 template <int SL, int WAVES>
 int launch_merge(const float* points, int N, int D, int K, const int* old_idx, int* knn_idx, float* knn_dist, int table,
-                 int wave_ints, int dpad, const uint32_t* pass, const JoinBounds& bounds, const int* todo_in, int n_in,
+                 int wave_ints, int dpad, bool direct, const uint32_t* pass, const JoinBounds& bounds, const int* todo_in, int n_in,
                  int* todo_out, int share, int* n_out, unsigned long long* stat, const int* order, hipStream_t stream)
 {
     const size_t lds = (size_t)WAVES * (size_t)wave_ints * sizeof(int);
     const int n_work = todo_in ? n_in : N;
     dim3 grid(grid_for_dies(((size_t)n_work + WAVES - 1) / WAVES)), block(64 * WAVES);
-    if (merge_tile_ints(dpad, merge_direct_max()) == 0) {
+    if (direct) {
         RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_explore_merge<SL, WAVES, false>),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         hipLaunchKernelGGL((k_explore_merge<SL, WAVES, false>), grid, block, lds, stream, points, N, D, K, old_idx, knn_idx,
-                           knn_dist, table, wave_ints, dpad, merge_direct_max(), pass, bounds, todo_in, n_in, todo_out, share, n_out,
+                           knn_dist, table, wave_ints, dpad, pass, bounds, todo_in, n_in, todo_out, share, n_out,
                            stat, order);
     } else {
         RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_explore_merge<SL, WAVES, true>),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         hipLaunchKernelGGL((k_explore_merge<SL, WAVES, true>), grid, block, lds, stream, points, N, D, K, old_idx, knn_idx,
-                           knn_dist, table, wave_ints, dpad, merge_direct_max(), pass, bounds, todo_in, n_in, todo_out, share, n_out,
+                           knn_dist, table, wave_ints, dpad, pass, bounds, todo_in, n_in, todo_out, share, n_out,
                            stat, order);
     }
     RSFK_HIP(hipGetLastError());
@@ -1079,22 +1092,26 @@ int launch_merge(const float* points, int N, int D, int K, const int* old_idx, i
 
 // ints of LDS a wavefront of the merge kernel needs for a set of `table` entries: tile | point | set | row | list of
 // marks | with_bounds: a bound per place of the set
-int merge_wave_ints(int table, int dpad, int K, bool with_bounds = false)
+int merge_wave_ints(int table, int dpad, int K, bool with_bounds, int tile)
 {
-    const int tile = merge_tile_ints(dpad, merge_direct_max());
     const int lists = table + K + table / 4 * 3 + (with_bounds ? table : 0);
     const int ranks = tile > 0 ? 0 : merge_rank_at(table, K, with_bounds) + rank_words(row_slots(K));
     return (tile + dpad + std::max(lists, ranks) + 3) / 4 * 4;
+}
+int merge_wave_ints(int table, int dpad, int K, bool with_bounds = false)
+{
+    return merge_wave_ints(table, dpad, K, with_bounds, merge_tile_ints(dpad, merge_direct_max()));
 }
 
 int dispatch_merge(int sl, int waves, const float* points, int N, int D, int K, const int* old_idx, int* knn_idx,
                    float* knn_dist, int table, int dpad, const uint32_t* pass, const JoinBounds& bounds, const int* todo_in,
                    int n_in, int* todo_out, int share, int* n_out, unsigned long long* stat, const int* order, hipStream_t stream)
 {
-    const int wi = merge_wave_ints(table, dpad, K, bounds.codes != nullptr);
+    const bool coded = bounds.codes != nullptr, direct = merge_direct(D, dpad, coded);
+    const int wi = merge_wave_ints(table, dpad, K, coded, direct ? 0 : kMergeTile);
 #define RSFK_MERGE_CASE(SLV, WV)                                                                                        \
     if (sl == SLV && waves == WV)                                                                                       \
-        return launch_merge<SLV, WV>(points, N, D, K, old_idx, knn_idx, knn_dist, table, wi, dpad, pass, bounds, \
+        return launch_merge<SLV, WV>(points, N, D, K, old_idx, knn_idx, knn_dist, table, wi, dpad, direct, pass, bounds, \
                                      todo_in, n_in, todo_out, share, n_out, stat, order, stream);
     RSFK_MERGE_CASE(1, 4) RSFK_MERGE_CASE(1, 2) RSFK_MERGE_CASE(1, 1)
     RSFK_MERGE_CASE(2, 4) RSFK_MERGE_CASE(2, 2) RSFK_MERGE_CASE(2, 1)
@@ -1226,9 +1243,13 @@ int launch_explore(const float* points, const Bf16Copy* bf, const JoinCopy* jc, 
         int big_table = want, big_waves = 4;
         while (big_waves > 1 && merge_wave_ints(big_table, dpad, K) > lds_ints / big_waves) big_waves >>= 1;
         // fewer than four wavefronts per workgroup would leave the compute units nearly empty: such sets get one
-        // workgroup per point instead
-        const bool per_wg = big_waves < 4;
+        // workgroup per point instead.  So do sets of 2048 places and more where the join kept its codes (at least one workgroup of
+        // four of them fits a compute unit, but they evaluate every candidate, and that kernel what the codes leave):
+        // whole pass with points that have most of their marks, D = 132, K = 40 5.4 -> 4.5 ms, K = 50 14.1 -> 6.0; D = 256, K = 32
+        // 9.2 -> 4.9, K = 60 28.6 -> 8.0; D = 960, K = 60 36.5 -> 5.9.  K = 32 is even at D = 192 and slower at D = 132 (3.9 -> 4.4).
         const WgSizes wg = merge_wg_sizes(dpad, K, sl);
+        const bool by_codes = explore_ws_bounds(ws).codes != nullptr && big_table >= 2048 && (K > 32 || D >= 192) && wg.cap > 0;
+        const bool per_wg = big_waves < 4 || by_codes;
         if (!per_wg)
             while (big_table > small_table && merge_wave_ints(big_table, dpad, K) > lds_ints / big_waves) big_table >>= 1;
         const bool second = per_wg ? wg.cap > 0 : big_table > small_table;

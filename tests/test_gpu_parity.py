@@ -629,6 +629,42 @@ def test_explore_with_a_workgroup_per_point(gpu, orc, rng, monkeypatch, N, D, K,
         assert_knn_equal(gi, gd, oi, od)
 
 
+@pytest.mark.parametrize("codes", [True, False])
+@pytest.mark.parametrize("D", [129, 191, 192, 193, 288, 292])
+@pytest.mark.parametrize("K", [31, 32, 33, 45, 63])
+def test_explore_of_long_vectors(gpu, orc, rng, monkeypatch, D, K, codes):
+    """More than 128 dimensions: with the join's codes up to 288 of them (192 where D is not a multiple of 4) are read without the tile,
+    and points of many marks (here: a first tree of small leaves, 500 clustered points) go to a workgroup each where the set has
+    2048 places (K >= 32) and K > 32 or D >= 192; without the codes neither."""
+    if not codes:
+        monkeypatch.setenv("RSFK_OPTIONAL_MB", "0")
+    N = 1500
+    X = rng.standard_normal((N, D)).astype(np.float32)
+    X[:500] = (X[rng.integers(0, 10, 500)] + np.float32(0.05) * X[:500]).astype(np.float32)
+    oi, od = orc.init_lists(N, K, self_in=True)
+    for seed, leaf in enumerate((K // 2, K + 1)):
+        perm, ls, lz, _ = orc.build_tree(X, leaf, 2 * leaf, 5000, seed)
+        orc.bucket_knn(X, K, perm, lz, oi, od, starts=ls)
+    gi, gd = oi.copy(), od.copy()
+    _say("explore long vectors", D, K, codes)
+    for _ in range(2):
+        orc.explore(X, K, oi, od)
+        gpu.explore(X, K, gi, gd, 1)
+        assert_knn_equal(gi, gd, oi, od)
+
+
+@pytest.mark.parametrize("D,K", [(192, 32), (129, 33), (400, 50)])
+def test_forest_of_long_vectors_with_many_marks(gpu, orc, rng, D, K):
+    """The same from a forest of two trees: the points that the small set is tried on first (more than 4,096 points in their order)."""
+    import gpu_rsfk
+    X = rng.standard_normal((5003, D)).astype(np.float32)
+    _say("forest of long vectors", D, K)
+    gi, gd = gpu_rsfk.RSFK(random_state=0).find_nearest_neighbors(X, K, n_trees=2, min_tree_children=K + 1, max_tree_children=2 * K + 2,
+                                                                    nn_exploring_factor=1)
+    oi, od, _ = orc.forest(X, K, 2, K + 1, 2 * K + 2, 5000, 0, 1, want_log=True)
+    assert_knn_equal(gi, gd, oi, od)
+
+
 # ---------------------------------------------------------------------------
 # the whole call, through the entry points the Python package binds
 # ---------------------------------------------------------------------------
