@@ -627,7 +627,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_merge(const float* __res
     if (row.changed) row.store(knn_idx + (size_t)p * K, knn_dist + (size_t)p * K);
 }
 
-// The same for rows so long that the set of one point takes most of the LDS a wavefront could get (K above about 45:
+// The same for rows so long that the set of one point takes much of a wavefront's LDS (K >= 64, or 32 with codes, launch_explore:
 // a point has up to K^2 marks): one workgroup of four wavefronts per point.
 //
 // A candidate can only end up in the row if its exact distance is at most the row's last slot at the end, and every exact distance is
