@@ -81,11 +81,13 @@ __global__ __launch_bounds__(kRowsThreads, 4) void k_bucket_knn_rows(const float
 #pragma unroll
     for (int t = 0; t < NT; ++t) cid[t] = lids[64 * t + lane];
 
-    auto load_row = [&](int m, int& ri, float& rd) {
+    // of member m: its id (the same in all lanes) and its row
+    auto load_row = [&](int m, int& id, int& ri, float& rd) {
+        id = __builtin_amdgcn_readfirstlane(lids[min(m, s - 1)]);
         ri = -2;
         rd = INFINITY;
         if (m < s && lane < K) {
-            const size_t at = (size_t)lids[m] * (size_t)K + lane;
+            const size_t at = (size_t)id * (size_t)K + lane;
             ri = knn_idx[at];
             rd = knn_dist[at];
         }
@@ -97,7 +99,7 @@ __global__ __launch_bounds__(kRowsThreads, 4) void k_bucket_knn_rows(const float
     // few others there.  Candidates that are points of the row already are found by a filter of 2,048 bits over the row's ids.
     // (10M x 32, buckets of 64..256: first tree 12.2 -> 10.6 ms, second, whose rows
     // used to take insertions, 14.1 -> 9.2; 530 and 470 vector instructions per point, 190 of them the chains.)
-    auto place_young = [&](int m, int ri, float rd, const KnnRow<1>& row, bool (&ok)[NT], const float (&acc)[NT]) -> bool {
+    auto place_young = [&](int id, const KnnRow<1>& row, bool (&ok)[NT], const float (&acc)[NT]) -> bool {
         bool in[NT];
         int n_in = 0;
 #pragma unroll
@@ -109,12 +111,15 @@ __global__ __launch_bounds__(kRowsThreads, 4) void k_bucket_knn_rows(const float
         if (n_in < kYoungLeast || row.changed) return false;          // (a row that had to be put in order is stored whole)
         const bool mine = lane < K && row.idx[0] >= 0 && row.dist[0] < INFINITY;
         const int n_row = __popcll(ballot64(mine));
-        const bool insert = n_row > 1 && D < kYoungDims;             // the histogram of the candidates alone, then insertions
+        // A row that holds nothing but, possibly, the point itself is new; any other entry may be a candidate too.  (Not told by the number
+        // of entries: after a bucket of two points, or from the caller, a row's only entry is another point.)
+        const bool new_row = ballot64(mine && row.idx[0] != id) == 0;
+        const bool insert = !new_row && D < kYoungDims;              // the histogram of the candidates alone, then insertions
         if (insert && n_in <= K + 16) return false;
         if (ballot64(lane < K && row.idx[0] >= 0 && !mine) != 0) return false;
         // the intervals: from the least of them to the last slot of a full row, or to the mean of the candidates (to the largest, where
         // fewer than K are below the mean); what is beyond is in the last one
-        float lo = n_row > 1 && lane > 0 && mine ? row.dist[0] : INFINITY, sum = 0.0f;      // (not the point itself, which is at 0)
+        float lo = !new_row && lane > 0 && mine ? row.dist[0] : INFINITY, sum = 0.0f;       // (not the point itself, which is at 0)
 #pragma unroll
         for (int t = 0; t < NT; ++t)
             if (in[t]) { lo = fminf(lo, acc[t]); sum += acc[t]; }
@@ -151,12 +156,12 @@ __global__ __launch_bounds__(kRowsThreads, 4) void k_bucket_knn_rows(const float
         const int h = hist[lane];
         const int before = wave_excl_scan_i(h);
         const int all = n_in + n_row;
-        const int need = insert ? K : min(all, K + (n_row > 1 ? 4 : 0));      // (some may be there twice)
+        const int need = insert ? K : min(all, K + (new_row ? 0 : 4));        // (some may be there twice)
         const int cross = first_lane(ballot64(before + h >= need));
         const int n_left = read_lane_i(before + h, cross);
         if (insert || n_left > 64) {
             // (insertions, of those that can stay)
-            if (insert || n_row <= 1)
+            if (insert || new_row)
 #pragma unroll
                 for (int t = 0; t < NT; ++t) ok[t] = in[t] && bin[t] <= cross;
             return false;
@@ -188,7 +193,7 @@ __global__ __launch_bounds__(kRowsThreads, 4) void k_bucket_knn_rows(const float
         }
         // candidates that are in the row: the filter first, then the row's ids
         bool twice = false;
-        if (n_row > 1) {
+        if (!new_row) {
             auto bit_of = [](int id) { return (id ^ (id >> 11)) & 2047; };
             wave_lds_sync();
             hist[lane] = 0;
@@ -212,13 +217,13 @@ __global__ __launch_bounds__(kRowsThreads, 4) void k_bucket_knn_rows(const float
             rank -= pair_above(d, c, read_lane_f(d, j), read_lane_i(c, j)) ? 1 : 0;
         }
         if (here && !twice && rank < K) {
-            const size_t to = (size_t)lids[m] * (size_t)K + rank;
+            const size_t to = (size_t)id * (size_t)K + rank;
             knn_idx[to] = c;
             knn_dist[to] = d;
         }
         return true;
     };
-    auto finish = [&](int m, int ri, float rd, const float (&acc)[NT]) {
+    auto finish = [&](int m, int id, int ri, float rd, const float (&acc)[NT]) {
         KnnRow<1> row;
         row.idx[0] = ri;
         row.dist[0] = rd;
@@ -227,26 +232,27 @@ __global__ __launch_bounds__(kRowsThreads, 4) void k_bucket_knn_rows(const float
         bool ok[NT];
 #pragma unroll
         for (int t = 0; t < NT; ++t) ok[t] = t < nt && cid[t] >= 0 && 64 * t + lane != m;
-        if (DENSE && place_young(m, ri, rd, row, ok, acc)) return;
+        if (DENSE && place_young(id, row, ok, acc)) return;
         // tile after tile: the last slot a tile leaves behind already turns away candidates of the next
 #pragma unroll
         for (int t = 0; t < NT; ++t)
             if (t < nt) row.merge(ok[t], cid[t], acc[t]);
         if (row.changed) {
-            const size_t at = (size_t)lids[m] * (size_t)K;
+            const size_t at = (size_t)id * (size_t)K;
             row.store(knn_idx + at, knn_dist + at);
         }
     };
 
     // members wave, wave + 4 (a pair), wave + 8, wave + 12 (the next pair), ...
+    int id0, id1, nid0, nid1;
     int ri0, ri1, nri0, nri1;
     float rd0, rd1, nrd0, nrd1;
-    load_row(wave, ri0, rd0);
-    load_row(wave + kRowsWaves, ri1, rd1);
+    load_row(wave, id0, ri0, rd0);
+    load_row(wave + kRowsWaves, id1, ri1, rd1);
     for (int m0 = wave; m0 < s; m0 += 2 * kRowsWaves) {
         const int m1 = m0 + kRowsWaves;
-        load_row(m0 + 2 * kRowsWaves, nri0, nrd0);
-        load_row(m1 + 2 * kRowsWaves, nri1, nrd1);
+        load_row(m0 + 2 * kRowsWaves, nid0, nri0, nrd0);
+        load_row(m1 + 2 * kRowsWaves, nid1, nri1, nrd1);
         const bool two = m1 < s;
         const float* r0 = rows + m0 * pitch;
         const float* r1 = rows + (two ? m1 : m0) * pitch;
@@ -288,10 +294,10 @@ __global__ __launch_bounds__(kRowsThreads, 4) void k_bucket_knn_rows(const float
                 }
             }
         }
-        finish(m0, ri0, rd0, acc0);
-        if (two) finish(m1, ri1, rd1, acc1);
-        ri0 = nri0; rd0 = nrd0;
-        ri1 = nri1; rd1 = nrd1;
+        finish(m0, id0, ri0, rd0, acc0);
+        if (two) finish(m1, id1, ri1, rd1, acc1);
+        id0 = nid0; ri0 = nri0; rd0 = nrd0;
+        id1 = nid1; ri1 = nri1; rd1 = nrd1;
     }
 }
 

@@ -377,6 +377,68 @@ def test_bucket_knn_resident_rows_merged_by_counting(gpu, orc, rng, K, MIN, MAX,
         assert rows_have_no_duplicates(gi)
 
 
+def _in_order_without_holes(idx, dist):
+    """Rows ascend, and no empty slot stands before a neighbour."""
+    return not ((idx[:, :-1] < 0) & (idx[:, 1:] >= 0)).any() and (dist[:, :-1] <= dist[:, 1:]).all()
+
+
+# rows counted by a wavefront (K + 4 at most 64) and longer ones; dimensions on both sides of the line between counting and insertions
+@pytest.mark.parametrize("data", ["continuous", "mixed"])
+@pytest.mark.parametrize("which", ["nearest", "any", "pairs"])
+@pytest.mark.parametrize("K,MIN,MAX,D", [(8, 40, 120, 9), (8, 80, 200, 4), (32, 64, 256, 9), (32, 64, 256, 5), (50, 74, 190, 7), (60, 61, 200, 6), (64, 70, 190, 12)])
+def test_bucket_knn_resident_rows_that_hold_one_other_point(gpu, orc, rng, K, MIN, MAX, D, which, data):
+    """A row whose only entry is a neighbour (with its distance) from the bucket the row meets next: the candidate that is that neighbour must
+    not be counted a second time.  The neighbour is the nearest, any other one of the bucket, or what a partition into pairs left in
+    rows that began empty; a fifth of the rows holds the point itself alone, or nothing."""
+    N = 4000
+    X = rng.standard_normal((N, D)).astype(np.float32)
+    if data == "mixed":
+        some = rng.random(N) < 0.1
+        X[some] = rng.integers(0, 2, (int(some.sum()), D)).astype(np.float32)
+    perm, ls, lz, _ = orc.build_tree(X, MIN, MAX, 5000, 3)
+    oi = np.full((N, K), -1, np.int32)
+    od = np.full((N, K), np.inf, np.float32)
+    parts = [(perm, ls, lz), orc.build_tree(X, MIN, MAX, 5000, 4)[:3]]
+    if which == "pairs":
+        parts.insert(0, (perm, np.arange(0, N, 2, dtype=np.int32), np.full(N // 2, 2, np.int32)))
+    else:
+        ti, td = np.full((N, MAX), -1, np.int32), np.full((N, MAX), np.inf, np.float32)
+        orc.bucket_knn(X, MAX, perm, lz, ti, td, starts=ls)
+        at = np.zeros(N, np.int64) if which == "nearest" else rng.integers(0, (ti >= 0).sum(1))
+        order = np.lexsort((ti, td), axis=1)[np.arange(N), at]
+        oi[:, 0], od[:, 0] = ti[np.arange(N), order], td[np.arange(N), order]
+        alone, nothing = rng.random(N) < 0.1, rng.random(N) < 0.1
+        oi[alone, 0], od[alone, 0] = np.flatnonzero(alone), 0.0
+        oi[nothing, 0], od[nothing, 0] = -1, np.inf
+    gi, gd = oi.copy(), od.copy()
+    for perm, ls, lz in parts:
+        _say("bucket_knn rows with one other point", K, MIN, MAX, D, which, data)
+        orc.bucket_knn(X, K, perm, lz, oi, od, starts=ls)
+        gpu.bucket_knn(X, K, perm, lz, gi, gd, starts=ls)
+        assert_knn_equal(gi, gd, oi, od)
+        assert rows_have_no_duplicates(gi)
+        assert _in_order_without_holes(gi, gd)
+
+
+@pytest.mark.parametrize("N,D,K,T", [(6000, 3, 32, 1), (6000, 9, 32, 1), (5000, 7, 45, 2), (4000, 6, 63, 1)])
+def test_extra_tree_after_buckets_of_two(gpu, orc, rng, N, D, K, T):
+    """Rows that begin empty and meet buckets of 2 to 4 points, then those of the extra tree of ensure_valid_indices: up to 3 (K + 1) points, so
+    that rows of a single neighbour are offered a resident bucket."""
+    import gpu_rsfk
+    mn, mx = 2, 4
+    X = rng.standard_normal((N, D)).astype(np.float32)
+    r = gpu_rsfk.RSFK(random_state=4)
+    for nnef in (0, 1):
+        _say("extra tree", N, D, K, T, nnef)
+        gi, gd = r.find_nearest_neighbors(X, K, n_trees=T, min_tree_children=mn, max_tree_children=mx, nn_exploring_factor=nnef,
+                                          point_in_self_neigh=False)
+        oi, od = orc.init_lists(N, K, self_in=False)
+        oi, od = orc.forest(X, K, T, mn, mx, 5000, 4, nnef, knn_idx=oi, knn_dist=od)
+        oi, od = orc.forest(X, K, 1, K + 1, 3 * (K + 1), 5000, 4, nnef, knn_idx=oi, knn_dist=od)
+        assert_knn_equal(gi, gd, oi, od)
+        assert _in_order_without_holes(gi, gd)
+
+
 def test_bucket_knn_single_bucket_is_exact_knn(gpu, rng):
     """One bucket holding every point: the kernel must return exact K-NN."""
     for N, D, K in [(300, 8, 16), (700, 20, 32)]:
