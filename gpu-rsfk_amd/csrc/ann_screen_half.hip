@@ -21,6 +21,7 @@
 #include "exact_batch.hpp"
 #include "join_bounds.hpp"
 #include <algorithm>
+#include <cstdlib>
 
 namespace rsfk {
 
@@ -309,7 +310,9 @@ int launch_ann_screen_half(const JoinCopy& qc, const JoinCopy& pc, const float* 
     const float kappa = (float)(16 * kSteps + 24) * (1.0f / 2097152.0f);            // (Dp + 24) 2^-21
     const float one_minus_gamma = 1.0f - (float)(D + 8) * (1.0f / 4194304.0f);
     RSFK_CHECK(one_minus_gamma > 0.5f, "query-set search: D too large for the screened form");
-    const unsigned grid = (unsigned)std::min(16384, most_blocks);
+    int most = 16384;
+    if (const char* e = std::getenv("RSFK_ANN_SCREEN_GROUPS")) most = std::max(1, std::atoi(e));       // for tests
+    const unsigned grid = (unsigned)std::min(most, most_blocks);
     const bool vec = (D & 3) == 0 && ((reinterpret_cast<uintptr_t>(points) | reinterpret_cast<uintptr_t>(queries)) & 15) == 0;
     hipLaunchKernelGGL(k_ann_screen_half, dim3(grid), dim3(64), 0, stream, qc, pc, points, queries, D, K, vec, perm, blk_desc, n_blocks, qlist,
                        q_idx, q_dist, pc.scale(), kappa, join_err_rel(), join_err_abs(D), one_minus_gamma, form);

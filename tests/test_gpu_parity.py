@@ -1333,6 +1333,33 @@ def test_ann_screened_by_copies_matches_oracle(gpu, capi, orc, rng, monkeypatch,
         assert_knn_equal(idx.cpu().numpy(), dist.cpu().numpy(), oi, od)
 
 
+# Workgroups with many items each, as they have them from about 16,384 items (a million queries) on: the items that follow an item are looked up while it is
+# worked on, and pairs of several items wait for each other.  Buckets of few members and queries (a pair or two of an item are
+# left, so that tens of items wait together), items of 32 queries and more than one block of members, items between these; one workgroup,
+# fewer than items, and as many as items of a tree or more.
+@pytest.mark.parametrize("N,NQ,D,K,T,mn,mx", [(3000, 2500, 97, 4, 5, 3, 6), (1200, 1600, 100, 32, 6, 33, 66), (500, 900, 128, 64, 4, 100, 200), (900, 700, 113, 1, 6, 9, 18),
+                                              (60, 200, 104, 7, 3, 8, 60)])
+@pytest.mark.parametrize("data", ["normal", "ties", "huge"])
+def test_ann_screened_by_copies_with_many_items_per_workgroup(gpu, capi, orc, rng, monkeypatch, N, NQ, D, K, T, mn, mx, data):
+    """The bucket step that bounds the pairs by float16 copies, from one workgroup for all items to one for each == the oracle."""
+    import torch
+    draw = {"normal": lambda n: rng.standard_normal((n, D)), "ties": lambda n: rng.integers(0, 3, (n, D)),
+            "huge": lambda n: rng.standard_normal((n, D)) * np.where(rng.random((n, 1)) < 0.1, 3e18, 1.0)}[data]
+    X, Q = draw(N).astype(np.float32), draw(NQ).astype(np.float32)
+    dX, dQ = torch.from_numpy(X).cuda(), torch.from_numpy(Q).cuda()
+    oi, od = orc.ann_forest(X, Q, K, T, mn, mx, 5000, 5)
+    monkeypatch.setenv("RSFK_ANN_FOREST", "0")
+    monkeypatch.setenv("RSFK_ANN_SCREEN", "always")
+    for groups in (1, 3, 50):
+        monkeypatch.setenv("RSFK_ANN_SCREEN_GROUPS", str(groups))
+        idx = torch.full((NQ, K), -1, dtype=torch.int32, device="cuda")
+        dist = torch.full((NQ, K), float("inf"), dtype=torch.float32, device="cuda")
+        _say("ann screened by copies, items per workgroup", N, NQ, D, K, T, mn, mx, data, groups)
+        capi.knn_ann_device(T, K, N, NQ, D, mn, mx, 5000, 0, 5, dX.data_ptr(), dQ.data_ptr(), idx.data_ptr(), dist.data_ptr())
+        torch.cuda.synchronize()
+        assert_knn_equal(idx.cpu().numpy(), dist.cpu().numpy(), oi, od)
+
+
 # one query, and the sizes around a wavefront's 64; every number of 16-dimension steps, rows that end inside one; trees that end within
 # the first seven levels (the first one at its root) and go on below; queries in no tree's cloud
 @pytest.mark.parametrize("N,NQ,D,K,T,mn,mx", [(40, 1, 3, 5, 3, 50, 100), (300, 63, 1, 4, 5, 5, 11), (2500, 64, 16, 3, 6, 4, 9), (5000, 65, 17, 2, 9, 3, 6),
