@@ -28,7 +28,6 @@
 #include "rsfk_common.hpp"
 #include "knn_list.hpp"
 #include "forest.hpp"
-#include "bucket_small_body.hpp"
 #include "bucket_knn_stage.hpp"
 #include <algorithm>
 

@@ -329,12 +329,6 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore(const float* __restrict_
     if (row.changed) row.store(knn_idx + (size_t)p * K, knn_dist + (size_t)p * K);
 }
 
-// Exploration of the points whose candidates the join has marked (explore_join.hip): entry (p, k) of
-// the graph has the mask of neighbour slots at pass[p K + k] (entries without a valid neighbour have none).  One wavefront per point: gather
-// the marked ids, drop repeats and ids the row holds (hash set), exact distances, merge.  Points with
-// more marks than the LDS of this launch takes are appended to todo_out (for a launch with more LDS
-// per wavefront, or for the general kernel; share > 0: to the point's share of it, explore_ws_share_lists).  todo_in: the points to work on, or null for all.
-// Per-wavefront LDS (ints): tile[64*20] | xrow[dpad] | table[table_size] | srow[K] | marked[3/4 table_size].
 // Number of entry (p, k) of the graph snapshot, p K + k, or -1 when the slot holds no valid neighbour (the join writes
 // nothing for such an entry).
 __device__ __forceinline__ int graph_entry(const int* __restrict__ old_idx, int N, int K, int p, int k)
@@ -381,7 +375,13 @@ bool merge_direct(int D, int dpad, bool coded)
     return dpad <= ((D & 3) == 0 ? kDirectCoded : kDirectCodedOdd);
 }
 
-
+// Exploration of the points whose candidates the join has marked (explore_join.hip): entry (p, k) of
+// the graph has the mask of neighbour slots at pass[p K + k] (entries without a valid neighbour have none).  One wavefront per point: gather
+// the marked ids, drop repeats and ids the row holds (hash set), exact distances, merge.  Points with
+// more marks than the LDS of this launch takes are appended to todo_out (for a launch with more LDS
+// per wavefront, or for the general kernel; share > 0: to the point's share of it, explore_ws_share_lists).  todo_in: the points to work on,
+// or null for all.  Per-wavefront LDS (ints): with TILE tile[64*20] | xrow[dpad] | table[table_size] | srow[K] | marked[3/4 table_size]
+// | with codes: tbound[table_size] | without TILE: the ranks (merge_rank_at).
 // TILE: the candidates' rows go through the transposing tile (not merge_direct); the two forms
 // are kernels of their own, so that the shorter one does not carry the registers of the other.
 template <int SL, int WAVES, bool TILE>
@@ -1018,14 +1018,14 @@ __global__ __launch_bounds__(256, 3) void k_explore_merge_wg(const float* __rest
     }
 }
 
-// Sizes of the workgroup-per-point merge with the LDS of a compute unit shared by two workgroups; no marks (cap) at all where it does
-// not fit.
-int merge_wg_ints(const WgSizes& sz, int dpad, int K, int sl)
+// Sizes of the workgroup-per-point merge, with the LDS of a compute unit shared by three workgroups where they have room for the marks a
+// point can have, else by two; no marks (cap) at all where it does not fit.
+int merge_wg_ints(const WgSizes& sz, int dpad, int K)
 {
     return (std::max(sz.set_size + sz.cap, 4 * kWgTile) + sz.most + sz.most / 2 + dpad + 5 * ((K + 3) & ~3) + 3 * kWgNew + 3) / 4 * 4;
 }
 
-WgSizes merge_wg_sizes(int dpad, int K, int sl)
+WgSizes merge_wg_sizes(int dpad, int K)
 {
     // three workgroups per compute unit where that leaves room for kWgMaxCap marks, else two
     for (int share = 3; share >= 2; --share) {
@@ -1035,9 +1035,9 @@ WgSizes merge_wg_sizes(int dpad, int K, int sl)
             sz.set_size = set;
             sz.most = std::min(kWgMost, (set / 8 * 7 - K - 1) & ~7);
             if (sz.most < kWgLeast) continue;
-            sz.cap = std::min({budget - merge_wg_ints({0, sz.most, set}, dpad, K, sl) + std::max(0, 4 * kWgTile - set), K * K + 3, kWgMaxCap}) & ~3;
+            sz.cap = std::min({budget - merge_wg_ints({0, sz.most, set}, dpad, K) + std::max(0, 4 * kWgTile - set), K * K + 3, kWgMaxCap}) & ~3;
             const int enough = share == 3 ? std::min((K * K + 3) & ~3, kWgMaxCap) : kWgMinCap;
-            if (sz.cap >= enough && sz.cap >= kWgMinCap && merge_wg_ints(sz, dpad, K, sl) <= budget) return sz;
+            if (sz.cap >= enough && sz.cap >= kWgMinCap && merge_wg_ints(sz, dpad, K) <= budget) return sz;
         }
     }
     return {0, 0, 0};
@@ -1048,7 +1048,7 @@ int launch_merge_wg(const float* points, int N, int D, int K, const int* old_idx
                     const WgSizes& sz, int dpad, const uint32_t* pass, const JoinBounds& bounds, const int* todo_in, int n_in,
                     int* todo_out, int* n_out, unsigned long long* stat, hipStream_t stream)
 {
-    const size_t lds = (size_t)merge_wg_ints(sz, dpad, K, SL) * sizeof(int);
+    const size_t lds = (size_t)merge_wg_ints(sz, dpad, K) * sizeof(int);
     RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_explore_merge_wg<SL>),
                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     const int n_work = todo_in ? n_in : N;
@@ -1150,8 +1150,9 @@ int launch_one(const float* points, const Bf16Copy& b, int N, int D, int K, cons
 // Does the join keep the lower bounds of the pairs it marks (N K KP 2-byte words)?  Yes for the rows that go to the
 // workgroup-per-point merge (below), and for rows of more than 128 dimensions while the array stays below 4 GB: the
 // wavefront-per-point merge then takes the candidates of a point nearer bounds first (their rows are long, and every
-// candidate that a tighter last slot turns away is a row not read; at 100 dimensions a point has fewer than 64
-// candidates, one batch, and the bounds only cost: merge 4.05 against 3.67 ms, join 6.0 against 3.6 ms at 1M x 100).
+// candidate that a tighter last slot turns away is a row not read).  Up to 128 dimensions they cost more than they give, without -> with:
+// 1M x 100, 50 trees, join 3.44 -> 4.81 ms and merge 2.74 -> 3.24, in 64 clusters 3.03 -> 4.50 and 2.62 -> 3.29; 1M x 128 3.53 -> 4.92 and
+// 2.79 -> 3.39; 300,000 x 64, K = 48, 12 trees 1.12 -> 2.35 and 1.46 -> 2.03, x 128, K = 60 2.27 -> 3.92 and 8.46 -> 7.70.
 // RSFK_MERGE_ORDER=0 switches the second case off.
 bool explore_join_keeps_bounds(int N, int D, int K)
 {
@@ -1168,16 +1169,12 @@ bool explore_merge_uses_bounds(int D, int K)
 {
     const int dpad = bf16_valid(D);
     const int lds_ints = 150 * 1024 / 4;
-    const int sl = K <= 64 ? 1 : (K <= 128 ? 2 : 4);
     const int want = std::max(next_pow2(K * K + K + 2), next_pow2(4 * K + 66));
     int big_waves = 4;
     while (big_waves > 1 && merge_wave_ints(want, dpad, K) > lds_ints / big_waves) big_waves >>= 1;
-    return big_waves < 4 && merge_wg_sizes(dpad, K, sl).cap > 0;
+    return big_waves < 4 && merge_wg_sizes(dpad, K).cap > 0;
 }
 
-
-// One exploration pass.  old_idx is scratch of N*K ints (receives the snapshot).
-// bf may be null (or hold null rows): every candidate then gets the exact distance.
 // Rows short enough for the LDS of the merge kernels: the exploration then takes its candidates from the join, and
 // the general kernel (the only user of the bfloat16 copy) only sees what the merge kernels hand back.
 bool explore_merge_fits(int D, int K)
@@ -1186,6 +1183,8 @@ bool explore_merge_fits(int D, int K)
     return K <= kMaxKJoin && 4 * merge_wave_ints(small_table, bf16_valid(D), K) <= 150 * 1024 / 4;
 }
 
+// One exploration pass.  old_idx is scratch of N*K ints (receives the snapshot).
+// bf may be null (or hold null rows): every candidate then gets the exact distance.
 // ws may be null; with a workspace and the copy for the join (jc)
 // the candidates come from the join over the reversed graph (explore_join.hip), which needs rows sorted by
 // distance.
@@ -1247,7 +1246,7 @@ int launch_explore(const float* points, const Bf16Copy* bf, const JoinCopy* jc, 
         // four of them fits a compute unit, but they evaluate every candidate, and that kernel what the codes leave):
         // whole pass with points that have most of their marks, D = 132, K = 40 5.4 -> 4.5 ms, K = 50 14.1 -> 6.0; D = 256, K = 32
         // 9.2 -> 4.9, K = 60 28.6 -> 8.0; D = 960, K = 60 36.5 -> 5.9.  K = 32 is even at D = 192 and slower at D = 132 (3.9 -> 4.4).
-        const WgSizes wg = merge_wg_sizes(dpad, K, sl);
+        const WgSizes wg = merge_wg_sizes(dpad, K);
         const bool by_codes = explore_ws_bounds(ws).codes != nullptr && big_table >= 2048 && (K > 32 || D >= 192) && wg.cap > 0;
         const bool per_wg = big_waves < 4 || by_codes;
         if (!per_wg)

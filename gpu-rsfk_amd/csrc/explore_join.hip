@@ -72,7 +72,8 @@ struct ExploreWorkspace {
     int* fine_size = nullptr;   // n_coarse << (cshift - fshift)
     int* fine_start = nullptr;  // the same + 1
     int* sub_off = nullptr;     // n_sub x fine bins per coarse bin
-    int* todo = nullptr;       // two lists of N+1 ints: points left over by a launch; entry N = their number; then the shares of such a list, and their numbers
+    int* todo = nullptr;       // two lists of N + 1 ints, points left over by a launch (entry N of the second: their number); then the
+                               // shares from which the first is joined, and their numbers
 };
 int* explore_ws_shares(ExploreWorkspace* w)
 {
@@ -115,11 +116,11 @@ bool rev_bins(int N, int* shift, int* n_bins)
     return *n_bins <= kMaxBins;
 }
 
-__global__ void k_zero(int* a, int n, int* counter0, int* counter1, int* shares)
+__global__ void k_zero(int* a, int n, int* counter, int* shares)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) a[i] = 0;
-    if (i == 0) { *counter0 = 0; *counter1 = 0; }
+    if (i == 0) *counter = 0;
     if (i < kTodoShares) shares[32 * i] = 0;
 }
 
@@ -1141,10 +1142,10 @@ int launch_reversed_graph(ExploreWorkspace* w, const int* old_idx, int N, int K,
     const int total = (int)((size_t)N * (size_t)K);
     if (w->staged) {
         const int nc = w->n_coarse, per = 1 << (w->cshift - w->fshift);
-        hipLaunchKernelGGL(k_zero, dim3((unsigned)((nc + 255) / 256)), dim3(256), 0, stream, w->bin_size, nc, w->todo + N,
+        hipLaunchKernelGGL(k_zero, dim3((unsigned)((nc + 255) / 256)), dim3(256), 0, stream, w->bin_size, nc,
                            w->todo + 2 * (size_t)N + 1, explore_ws_shares(w));
         hipLaunchKernelGGL(k_zero, dim3((unsigned)((w->n_fine + 255) / 256)), dim3(256), 0, stream, w->fine_size, w->n_fine,
-                           w->todo + N, w->todo + 2 * (size_t)N + 1, explore_ws_shares(w));
+                           w->todo + 2 * (size_t)N + 1, explore_ws_shares(w));
         hipLaunchKernelGGL(k_bin_count, dim3((unsigned)w->n_parts), dim3(256), (size_t)nc * sizeof(int), stream, old_idx, total,
                            w->per_part, N, w->cshift, nc, w->bin_size, w->part_off);
         hipLaunchKernelGGL(k_bin_scan, dim3(1), dim3(256), 0, stream, w->bin_size, nc, w->bin_start, w->offs + N);
@@ -1164,7 +1165,7 @@ int launch_reversed_graph(ExploreWorkspace* w, const int* old_idx, int N, int K,
                            w->fshift, N, w->offs, w->rev);
     } else if (w->tiled) {
         const int nc = w->n_coarse;
-        hipLaunchKernelGGL(k_zero, dim3((unsigned)((nc + 255) / 256)), dim3(256), 0, stream, w->bin_size, nc, w->todo + N,
+        hipLaunchKernelGGL(k_zero, dim3((unsigned)((nc + 255) / 256)), dim3(256), 0, stream, w->bin_size, nc,
                            w->todo + 2 * (size_t)N + 1, explore_ws_shares(w));
         hipLaunchKernelGGL(k_bin_count, dim3((unsigned)w->n_parts), dim3(1024), (size_t)nc * sizeof(int), stream, old_idx, total,
                            w->per_part, N, w->cshift, nc, w->bin_size, w->part_off);
@@ -1180,7 +1181,7 @@ int launch_reversed_graph(ExploreWorkspace* w, const int* old_idx, int N, int K,
     } else {
     const int nbins = w->n_bins;
     const size_t bin_lds = (size_t)nbins * sizeof(int);
-    hipLaunchKernelGGL(k_zero, dim3((unsigned)((nbins + 255) / 256)), dim3(256), 0, stream, w->bin_size, nbins, w->todo + N,
+    hipLaunchKernelGGL(k_zero, dim3((unsigned)((nbins + 255) / 256)), dim3(256), 0, stream, w->bin_size, nbins,
                        w->todo + 2 * (size_t)N + 1, explore_ws_shares(w));
     hipLaunchKernelGGL(k_bin_count, dim3((unsigned)w->n_parts), dim3(256), bin_lds, stream, old_idx, total, w->per_part, N,
                        w->shift, nbins, w->bin_size, w->part_off);
@@ -1207,7 +1208,9 @@ int launch_explore_join(ExploreWorkspace* w, const JoinCopy& jc, int N, int D, i
     const int KP = (K + 31) & ~31;
     // A few points are in hundreds of rows, and a launch over few points ends with the tiles of these, one after the other: they are
     // dealt out to several wavefronts (3,000 x 200, K = 30: 0.102 ms per pass with one, 0.029 with 16; 20,000 x 32 0.037, 0.038 with 3,
-    // 0.056 with 16; 1M x 256 7.0, 7.2 with 2).
+    // 0.056 with 16; 1M x 256 7.0, 7.2 with 2).  Between these a part more or less weighs little, microseconds with 1, 2, 3 and 4 parts: x 32 in
+    // 64 clusters 21,000 38 35 36 36, 26,000 45 42 42 44, 32,000 51 50 51 54, 45,000 67 68 73 76, 60,000 88 92 98 102; uniform x 100 21,000 70 71
+    // 75 77, 32,000 96 103 110 114, 60,000 164 184 200 213.
     const unsigned parts = (unsigned)std::max(1, std::min(16, 65536 / N));
     const int wave_ints = (KP + 192 + 3) & ~3;
     const size_t lds = (size_t)kWaves * (size_t)wave_ints * sizeof(int);

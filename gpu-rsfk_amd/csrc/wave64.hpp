@@ -80,7 +80,7 @@ __device__ __forceinline__ float half_butterfly_sum(float v)
     return lane_id() < 32 ? lo : hi;
 }
 
-// maximum over all 64 lanes, returned in every lane (wave-uniform value)
+// sum over all 64 lanes (in no order a caller may rely on), returned in every lane
 __device__ __forceinline__ float wave_total_f(float v)
 {
     v += dpp_f<kDppXor1>(v);
@@ -90,6 +90,7 @@ __device__ __forceinline__ float wave_total_f(float v)
     return (read_lane_f(v, 0) + read_lane_f(v, 16)) + (read_lane_f(v, 32) + read_lane_f(v, 48));
 }
 
+// maximum over all 64 lanes, returned in every lane (wave-uniform value)
 __device__ __forceinline__ float wave_max(float v)
 {
     v = fmaxf(v, dpp_f<kDppXor1>(v));
