@@ -837,14 +837,14 @@ __global__ __launch_bounds__(TB, CHAIN ? 4 : 6) void k_tail(const float* __restr
                                                  const uint16_t* __restrict__ pb16, const uint8_t* __restrict__ q8, TreeParams P,
                                                  const int* __restrict__ perm0, const int* __restrict__ perm1,
                                                  int* __restrict__ perm_out,
-                                                 const TreeNode* __restrict__ tasks, int n_tasks, int node_cap, int G,
+                                                 const TreeNode* __restrict__ tasks, int n_tasks, int leaf_most, int node_most, int G,
                                                  int leaf_cap, int* __restrict__ leaf_start, int* __restrict__ leaf_size,
                                                  TreeStats* stats, LevelCounters* ctr,
                                                  TreeRec* __restrict__ recs_all, int rec_cap,
                                                  unsigned long long* __restrict__ stat, TreeNode* __restrict__ chain_all, int chain_cap)
 {
-    // dynamic LDS: seg[small] | tmp[small] | nvec[G][nvec_len(D)] | lrec[node_cap] | level lists 2 x node_cap |
-    // nodes for the chain phase [node_cap] | fmap[small]
+    // dynamic LDS: seg[small] | tmp[small] | nvec[G][nvec_len(D)] | lrec[leaf_most] | level lists 2 x node_most |
+    // nodes for the chain phase [node_most] | fmap[small]
     extern __shared__ __align__(16) unsigned char lds_raw[];
     const int Dv = nvec_len(P.D);
     int* seg = reinterpret_cast<int*>(lds_raw);
@@ -853,10 +853,10 @@ __global__ __launch_bounds__(TB, CHAIN ? 4 : 6) void k_tail(const float* __restr
     // buckets of this subtree, written to the table of the tree together at the end (one reservation per
     // workgroup instead of one atomic round trip per bucket): x = start, y = size | rank among its kind << 16
     int2* lrec = reinterpret_cast<int2*>(nvec + (size_t)G * Dv);
-    SmallNode* cur = reinterpret_cast<SmallNode*>(lrec + node_cap);
-    SmallNode* nxt = cur + node_cap;
-    SmallNode* chain = nxt + node_cap;
-    unsigned char* fmap = reinterpret_cast<unsigned char*>(CHAIN ? chain + node_cap : chain);
+    SmallNode* cur = reinterpret_cast<SmallNode*>(lrec + leaf_most);
+    SmallNode* nxt = cur + node_most;
+    SmallNode* chain = nxt + node_most;
+    unsigned char* fmap = reinterpret_cast<unsigned char*>(CHAIN ? chain + node_most : chain);
     __shared__ float b_s[kMaxGroup], hp_s[kMaxGroup][3];
     __shared__ int left_s[kMaxGroup], pre_s[kMaxGroup + 1], start_s[kMaxGroup], pair_s[kMaxGroup][2];
     __shared__ int piece_s[CHAIN ? kMaxGroup + 1 : 1], lefts_s[CHAIN ? kTailMost / 64 + kMaxGroup : 1];      // pieces of 64 members before a node's, lefts of a piece
@@ -909,7 +909,7 @@ __global__ __launch_bounds__(TB, CHAIN ? 4 : 6) void k_tail(const float* __restr
         if (recs) index_bucket(recs, rec_cap, rec, tk.start + start, count, ctr);
         const int at = atomicAdd(&nrec_s, 1);
         const int rank = atomicAdd(&kind_s[count > kBucketSplit ? 1 : 0], 1);
-        if (at < node_cap) lrec[at] = make_int2(tk.start + start, count | (rank << 16)); else ctr->overflow = 1;
+        if (at < leaf_most) lrec[at] = make_int2(tk.start + start, count | (rank << 16)); else ctr->overflow = 1;
         atomicMax(&lev_s, depth + 1);
         atomicMax(&mx_s, count);
         atomicMin(&mn_s, count);
@@ -1103,7 +1103,7 @@ __global__ __launch_bounds__(TB, CHAIN ? 4 : 6) void k_tail(const float* __restr
                     } else {
                         const bool small = CHAIN && c.count <= P.chain_max;
                         const int at = atomicAdd(small ? &n_chain_all_s : &n_nxt_s, 1);
-                        if (at < node_cap) {
+                        if (at < node_most) {
                             SmallNode sn;
                             sn.start = c.start; sn.count = c.count; sn.dstart = c.dstart; sn.dcount = c.dcount;
                             sn.depth = c.depth;
@@ -1121,7 +1121,7 @@ __global__ __launch_bounds__(TB, CHAIN ? 4 : 6) void k_tail(const float* __restr
             }
             __syncthreads();
         }
-        if (tid == 0) { n_cur_s = min(n_nxt_s, node_cap); n_nxt_s = 0; }
+        if (tid == 0) { n_cur_s = min(n_nxt_s, node_most); n_nxt_s = 0; }
         SmallNode* t = cur; cur = nxt; nxt = t;
         __syncthreads();
     }
@@ -1141,13 +1141,13 @@ __global__ __launch_bounds__(TB, CHAIN ? 4 : 6) void k_tail(const float* __restr
         stat_add(stat, task, 1, unsure_s);
     }
     __syncthreads();
-    const int nrec = min(nrec_s, node_cap);
+    const int nrec = min(nrec_s, leaf_most);
     for (int i = tid; i < nrec; i += TB) {
         const int2 r = lrec[i];
         const int count = r.y & 0xffff, rank = r.y >> 16;
         store_leaf(tk.tree, r.x, count, base_s[count > kBucketSplit ? 1 : 0] + rank, leaf_cap, leaf_start, leaf_size, ctr);
     }
-    for (int i = tid; CHAIN && i < min(n_chain_all_s, node_cap); i += TB) {
+    for (int i = tid; CHAIN && i < min(n_chain_all_s, node_most); i += TB) {
         const SmallNode sn = chain[i];
         TreeNode c;
         c.tree = tk.tree; c.start = tk.start + sn.start; c.count = sn.count; c.dstart = tk.start + sn.dstart; c.dcount = sn.dcount;
@@ -2562,19 +2562,23 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
     if (mid) few = true;
     if (n_tail > 0) {
         // (the tail kernel keeps the bfloat16 screen: measured, it is not faster with the 8-bit one)
-        // nodes of a level of a subtree (and its buckets): at most small / MIN + 1; hyperplanes kept together:
-        // as many as 24 KB hold, at most kMaxGroup
-        const int node_cap = P.small / std::max(MIN, 1) + 4;
-        const int G = std::max(1, std::min(kMaxGroup, (int)(24 * 1024 / ((size_t)nvec_len(D) * 4))));
-        const size_t lds = (size_t)(2 * P.small) * 4 + (size_t)G * nvec_len(D) * 4 + (size_t)node_cap * sizeof(int2) +
-                           (few ? 3 : 2) * (size_t)node_cap * sizeof(SmallNode) + (size_t)P.small;
-        RSFK_CHECK(lds <= 150 * 1024, "tree batch: D too large for the tail kernel's LDS budget");
+        // buckets of a subtree: at most small / MIN + 1; nodes of a level that are no buckets, and those for the chain phase: MAX - 1 points
+        // or more each (split_rules), no two with a point in common.  Hyperplanes kept together: as many as 24 KB hold, at most kMaxGroup, and
+        // fewer where short buckets leave less
+        constexpr size_t kTailLds = 156 * 1024;           // (the kernel's own arrays: 1 KB)
+        const int leaf_most = P.small / std::max(MIN, 1) + 4, node_most = P.small / std::max({MIN, MAX - 1, 1}) + 4;
+        const size_t besides = (size_t)(2 * P.small) * 4 + (size_t)leaf_most * sizeof(int2) +
+                               (few ? 3 : 2) * (size_t)node_most * sizeof(SmallNode) + (size_t)P.small;
+        const size_t plane = (size_t)nvec_len(D) * 4;
+        RSFK_CHECK(besides + plane <= kTailLds, "tree batch: D too large for the tail kernel's LDS budget");
+        const int G = std::max(1, std::min(kMaxGroup, (int)(std::min<size_t>(24 * 1024, kTailLds - besides) / plane)));
+        const size_t lds = besides + (size_t)G * plane;
 #define RSFK_TAIL_LAUNCH(Q, T, C, L, U)                                                                                       \
         do {                                                                                                               \
             RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_tail<Q, T, C, L, U>),                                \
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));                          \
             hipLaunchKernelGGL((k_tail<Q, T, C, L, U>), dim3(n_tail), dim3(T), lds, stream, points, pb16, q8, P, w->perm[0],   \
-                               w->perm[1], w->perm[0], w->tail, n_tail, node_cap, G, w->leaf_cap, w->leaf_start,            \
+                               w->perm[1], w->perm[0], w->tail, n_tail, leaf_most, node_most, G, w->leaf_cap, w->leaf_start,            \
                                w->leaf_size, w->stats, w->ctr, w->recs, w->rec_cap, w->stat, w->chain, w->tail_cap);         \
         } while (0)
         // Lanes per point: as many as there are pieces of 16 coordinates, up to four; few subtrees wait for the loads of a point, and

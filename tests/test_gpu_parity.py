@@ -236,6 +236,43 @@ def test_tree_edge_cases(gpu, orc, rng):
     assert list(g[2]) == [20]
 
 
+# Buckets of a point or two: the tail kernel's lists of nodes and buckets leave room for few hyperplanes, down to one at a time (long rows)
+@pytest.mark.parametrize("N,D,MIN,MAX", [(45, 99, 2, 4), (3000, 49, 2, 4), (5000, 100, 2, 5), (2500, 784, 2, 4), (2100, 2050, 2, 9), (300, 11152, 2, 4),
+                                         (2600, 240, 2, 3), (3000, 100, 1, 4)])
+@pytest.mark.parametrize("screen", ["auto", "q8", "bf16", "q8-256"])
+def test_tree_of_buckets_of_two(gpu, orc, rng, monkeypatch, N, D, MIN, MAX, screen):
+    """A partition with the shortest buckets over rows of more than 48 dimensions == the oracle's."""
+    if screen == "q8-256":
+        monkeypatch.setenv("RSFK_TREE_SCREEN", "q8")
+        monkeypatch.setenv("RSFK_TAIL_BLOCK", "256")
+    elif screen != "auto":
+        monkeypatch.setenv("RSFK_TREE_SCREEN", screen)
+    X = rng.standard_normal((N, D)).astype(np.float32)
+    X[rng.random(N) < 0.1] = X[0]
+    for depth in (5000, 9):
+        _say("tree of buckets of two", N, D, MIN, MAX, screen, depth)
+        perm, ls, lz, st = orc.build_tree(X, MIN, MAX, depth, 3)
+        gperm, gls, glz, gst = gpu.build_tree(X, MIN, MAX, depth, 3)
+        assert np.array_equal(gperm, perm)
+        assert np.array_equal(gls, ls) and np.array_equal(glz, lz)
+        assert list(gst) == [len(ls), st[0], st[1], st[2]]
+
+
+@pytest.mark.parametrize("N,NQ,D,K,T,mn,mx", [(45, 30, 99, 7, 6, 2, 4), (4000, 500, 64, 5, 4, 2, 4), (1500, 200, 300, 10, 3, 2, 5)])
+def test_search_and_build_with_buckets_of_two(gpu, orc, rng, N, NQ, D, K, T, mn, mx):
+    """The trees of a K-NN build and those that carry an index, with the shortest buckets."""
+    import gpu_rsfk
+    X, Q = rng.standard_normal((N, D)).astype(np.float32), rng.standard_normal((NQ, D)).astype(np.float32)
+    r = gpu_rsfk.RSFK(random_state=4)
+    _say("build and search with buckets of two", N, NQ, D, K, T)
+    gi, gd = r.find_nearest_neighbors(X, K, n_trees=T, min_tree_children=mn, max_tree_children=mx, nn_exploring_factor=1, ensure_valid_indices=False)
+    oi, od = orc.forest(X, K, T, mn, mx, 5000, 4, 1)
+    assert_knn_equal(gi, gd, oi, od)
+    gi, gd = r.find_nearest_neighbors_ann(X, Q, K, n_trees=T, min_tree_children=mn, max_tree_children=mx, ensure_valid_indices=False)
+    oi, od = orc.ann_forest(X, Q, K, T, mn, mx, 5000, 4)
+    assert_knn_equal(gi, gd, oi, od)
+
+
 # ---------------------------------------------------------------------------
 # bucket K-NN on a fixed partition
 # ---------------------------------------------------------------------------
