@@ -690,7 +690,7 @@ __global__ __launch_bounds__(256, 3) void k_explore_merge_wg(const float* __rest
                                                           const int* __restrict__ old_idx, int* __restrict__ knn_idx,
                                                           float* __restrict__ knn_dist, WgSizes sz, int dpad,
                                                           const uint32_t* __restrict__ pass, JoinBounds jb,
-                                                          const int* __restrict__ todo_in, int n_in,
+                                                          const int* __restrict__ list, int n_in,
                                                           int* __restrict__ todo_out, int* __restrict__ n_out,
                                                           unsigned long long* __restrict__ stat)
 {
@@ -700,8 +700,8 @@ __global__ __launch_bounds__(256, 3) void k_explore_merge_wg(const float* __rest
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     // (the list of points a launch before this one left over is in the order in which that launch came to them)
     const int slot = die_local_place(blockIdx.x, gridDim.x);
-    if (slot >= (todo_in ? n_in : N)) return;
-    const int p = todo_in ? todo_in[slot] : slot;
+    if (slot >= n_in) return;
+    const int p = list[slot];
     const int MW = (K + 31) >> 5, KP = MW * 32, kq = (K + 3) & ~3;
     int* table = lds_w;
     uint32_t* marked = reinterpret_cast<uint32_t*>(table + sz.set_size);
@@ -1045,15 +1045,17 @@ WgSizes merge_wg_sizes(int dpad, int K)
 
 template <int SL>
 int launch_merge_wg(const float* points, int N, int D, int K, const int* old_idx, int* knn_idx, float* knn_dist,
-                    const WgSizes& sz, int dpad, const uint32_t* pass, const JoinBounds& bounds, const int* todo_in, int n_in,
+                    const WgSizes& sz, int dpad, const uint32_t* pass, const JoinBounds& bounds, const int* list, int n_in,
                     int* todo_out, int* n_out, unsigned long long* stat, hipStream_t stream)
 {
     const size_t lds = (size_t)merge_wg_ints(sz, dpad, K) * sizeof(int);
     RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_explore_merge_wg<SL>),
                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    const int n_work = todo_in ? n_in : N;
-    hipLaunchKernelGGL((k_explore_merge_wg<SL>), dim3(grid_for_dies((size_t)n_work)), dim3(256), lds, stream, points, N, D, K, old_idx,
-                       knn_idx, knn_dist, sz, dpad, pass, bounds, todo_in, n_in, todo_out, n_out, stat);
+    for (int off = 0; off < n_in; off += kMostGroups) {       // (as many points as a launch has threads for)
+        const int n = std::min(n_in - off, kMostGroups);
+        hipLaunchKernelGGL((k_explore_merge_wg<SL>), dim3(grid_for_dies((size_t)n)), dim3(256), lds, stream, points, N, D, K, old_idx,
+                           knn_idx, knn_dist, sz, dpad, pass, bounds, list + off, n, todo_out, n_out, stat);
+    }
     RSFK_HIP(hipGetLastError());
     return 0;
 }

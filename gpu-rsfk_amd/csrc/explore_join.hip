@@ -1232,6 +1232,10 @@ int launch_explore_join(ExploreWorkspace* w, const JoinCopy& jc, int N, int D, i
                        one_minus_gamma, w->bars);
     RSFK_HIP(hipGetLastError());
     const int MW = KP >> 5;
+    // More points than a launch has threads for take a wavefront per q: with a wavefront per 32 neighbours K = 33 from 33.5 million points on, 129
+    // from 13.4, 225 from 8.4, with a workgroup per q all from 16.8.
+    const unsigned short_groups = grid_for_dies(((size_t)N * (size_t)MW + kWaves - 1) / kWaves);
+    const bool short_fits = launch_fits(short_groups, 64 * kWaves), wg_fits = launch_fits(grid_for_dies((size_t)N), 256);
     // One workgroup per q reads every row once per 96 points of R(q), one wavefront per q (and 32 neighbours) again for every group of 32
     // neighbours, so the former pays with the bytes that are read again, D (K - 24) or so, sooner with more groups; up to 32 neighbours
     // are one pair per tile of R(q), too little for four wavefronts (1M x 256, K = 32: 8.1 ms against 12.6).  A pass, a wavefront per q -> a
@@ -1239,7 +1243,7 @@ int launch_explore_join(ExploreWorkspace* w, const JoinCopy& jc, int N, int D, i
     // 10.9 -> 10.4, 300,000 x 64, K = 90 17.8 -> 19.0, x 100 20.8 -> 20.8, 100,000 x 128, K = 90 7.07 -> 6.89, x 400 12.3 -> 9.6, 200,000 x 16, K = 128 19.3
     // -> 19.6, x 32 17.0 -> 16.9, 100,000 x 256, K = 128 15.0 -> 11.4.  Above 128 neighbours its accumulators leave one wavefront per SIMD: 100,000 x 32,
     // K = 160 18.3 -> 29.7.
-    if (KP > 32 && KP <= 128 && join_wg_on() && D * (K - 24) > (MW == 2 ? 8000 : MW == 3 ? 6500 : 3000)) {
+    if (KP > 32 && KP <= 128 && join_wg_on() && wg_fits && D * (K - 24) > (MW == 2 ? 8000 : MW == 3 ? 6500 : 3000)) {
         const size_t lds_wg = (size_t)(kJwP + KP) * kJwRowBytes + (size_t)KP * 12 + (size_t)kJwP * 24;
 #define RSFK_JOIN_WG(BV)                                                                                                    \
         do {                                                                                                               \
@@ -1252,8 +1256,8 @@ int launch_explore_join(ExploreWorkspace* w, const JoinCopy& jc, int N, int D, i
         if (w->bounds) RSFK_JOIN_WG(true);
         else RSFK_JOIN_WG(false);
 #undef RSFK_JOIN_WG
-    } else if (!w->bounds && ksteps <= 8) {
-        const dim3 grid(grid_for_dies(((size_t)N * (size_t)MW + kWaves - 1) / kWaves), parts), block(64 * kWaves);
+    } else if (!w->bounds && ksteps <= 8 && short_fits) {
+        const dim3 grid(short_groups, parts), block(64 * kWaves);
 #define RSFK_JOIN_SHORT(KSV, MANYV)                                                                                         \
         hipLaunchKernelGGL((k_explore_join_short<kWaves, KSV, MANYV>), grid, block, 0, stream, jc, N, K, old_idx, w->bars, w->offs, \
                            w->rev, w->pass, MW, join_pitch(D), ksteps, kappa, any_rel, any_abs, w->div_m, w->div_s, order)

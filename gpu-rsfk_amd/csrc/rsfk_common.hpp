@@ -69,6 +69,10 @@ constexpr int kDies = 8;
 __device__ __forceinline__ int die_local_place(int block, int grid) { return (block & (kDies - 1)) * (grid / kDies) + block / kDies; }
 inline unsigned grid_for_dies(size_t n_blocks) { return (unsigned)((n_blocks + kDies - 1) / kDies * kDies); }
 
+// A launch has fewer than 2^32 threads along x; what is beyond is cut off without an error.
+inline bool launch_fits(size_t groups, int threads) { return groups * (size_t)threads < ((size_t)1 << 32); }
+constexpr int kMostGroups = (1 << 24) - kDies;            // of 256 threads
+
 // ---------------------------------------------------------------------------
 // counter-based random numbers.  A node of a tree is identified by a 64-bit key
 // derived from the tree seed and the left/right path to the node, so a tree is

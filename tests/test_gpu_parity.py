@@ -671,6 +671,40 @@ def test_explore_join_of_rows_of_many_neighbours(gpu, orc, rng, monkeypatch, N, 
         assert_knn_equal(gi, gd, oi, od)
 
 
+# a wavefront for every 32 neighbours of a point, a workgroup for every point
+@pytest.mark.parametrize("N,D,K", [(13430000, 2, 129), (16800000, 201, 64)])
+def test_explore_of_more_points_than_a_launch_has_threads_for(gpu, N, D, K):
+    """The kernels that the size would take need 2^32 threads and more, which a launch cuts off without an error (about 100 GB of device
+    memory).  Every row holds the next point, so the exploration finds the one after that; coordinates are small integers, all
+    distances exact."""
+    import torch
+    torch.cuda.empty_cache()
+    gpu.lib().rsfk_release_workspace()
+    if torch.cuda.mem_get_info()[0] < 160 << 30:
+        pytest.skip("needs 160 GB of device memory")
+    X = torch.randint(0, 16, (N, D), device="cuda", dtype=torch.float32)
+    p = torch.arange(N, device="cuda")
+    one, two = (p + 1) % N, (p + 2) % N
+    d1 = torch.cat([((X[q] - X[(q + 1) % N]) ** 2).sum(1) for q in p.split(1 << 22)])
+    d2 = torch.cat([((X[q] - X[(q + 2) % N]) ** 2).sum(1) for q in p.split(1 << 22)])
+    idx = torch.full((N, K), -1, dtype=torch.int32, device="cuda")
+    dist = torch.full((N, K), float("inf"), device="cuda")
+    idx[:, 0] = one.int()
+    dist[:, 0] = d1
+    scratch = torch.empty((N, K), dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    _say("explore", N, D, K)
+    gpu.explore_device(X.data_ptr(), N, D, K, idx.data_ptr(), dist.data_ptr(), scratch.data_ptr())
+    del scratch
+    first = (d1 < d2) | ((d1 == d2) & (one < two))
+    assert torch.equal(idx[:, 0], torch.where(first, one, two).int()) and torch.equal(idx[:, 1], torch.where(first, two, one).int())
+    assert torch.equal(dist[:, 0], torch.minimum(d1, d2)) and torch.equal(dist[:, 1], torch.maximum(d1, d2))
+    assert bool((idx[:, 2] == -1).all()) and bool((idx[:, K - 1] == -1).all())
+    del idx, dist, X
+    torch.cuda.empty_cache()
+    gpu.lib().rsfk_release_workspace()
+
+
 @pytest.mark.parametrize("values", ["far", "tiny", "huge", "outlier", "spread", "notfinite"])
 @pytest.mark.parametrize("N,D,K", [(2500, 16, 8), (2500, 33, 32), (1500, 129, 20), (1500, 40, 70)])
 def test_explore_screens_rows_of_any_magnitude(gpu, orc, rng, N, D, K, values):
