@@ -520,12 +520,17 @@ int launch_sort_rows(int* knn_idx, float* knn_dist, int N, int K, hipStream_t st
 {
     if (N <= 0) return 0;
     RSFK_CHECK(K >= 1 && K <= kMaxK, "sort rows: K must be in 1..1024");
-    const dim3 grid((unsigned)((N + 3) / 4)), block(256);
-    if (K <= 64) hipLaunchKernelGGL(k_sort_rows<1>, grid, block, 0, stream, knn_idx, knn_dist, N, K);
-    else if (K <= 128) hipLaunchKernelGGL(k_sort_rows<2>, grid, block, 0, stream, knn_idx, knn_dist, N, K);
-    else if (K <= 256) hipLaunchKernelGGL(k_sort_rows<4>, grid, block, 0, stream, knn_idx, knn_dist, N, K);
-    else if (K <= 512) hipLaunchKernelGGL(k_sort_rows<8>, grid, block, 0, stream, knn_idx, knn_dist, N, K);
-    else hipLaunchKernelGGL(k_sort_rows<16>, grid, block, 0, stream, knn_idx, knn_dist, N, K);
+    for (int first = 0; first < N; first += std::min(kMostRows, N - first)) {
+        const int n = std::min(kMostRows, N - first);
+        int* idx = knn_idx + (size_t)first * (size_t)K;
+        float* dist = knn_dist + (size_t)first * (size_t)K;
+        const dim3 grid((unsigned)((n + 3) / 4)), block(256);
+        if (K <= 64) hipLaunchKernelGGL(k_sort_rows<1>, grid, block, 0, stream, idx, dist, n, K);
+        else if (K <= 128) hipLaunchKernelGGL(k_sort_rows<2>, grid, block, 0, stream, idx, dist, n, K);
+        else if (K <= 256) hipLaunchKernelGGL(k_sort_rows<4>, grid, block, 0, stream, idx, dist, n, K);
+        else if (K <= 512) hipLaunchKernelGGL(k_sort_rows<8>, grid, block, 0, stream, idx, dist, n, K);
+        else hipLaunchKernelGGL(k_sort_rows<16>, grid, block, 0, stream, idx, dist, n, K);
+    }
     RSFK_HIP(hipGetLastError());
     return 0;
 }

@@ -231,11 +231,11 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore(const float* __restrict_
                                                          const int* __restrict__ old_idx, int* __restrict__ knn_idx,
                                                          float* __restrict__ knn_dist, int table_size, int wave_lds_ints,
                                                          int dpad, int rows_per_group, const int* __restrict__ todo,
-                                                         int n_todo, unsigned long long* __restrict__ stat)
+                                                         int first, int n_todo, unsigned long long* __restrict__ stat)
 {
     extern __shared__ __align__(16) int lds_i[];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int slot = blockIdx.x * WAVES + wave;
+    const int slot = first + blockIdx.x * WAVES + wave;
     if (slot >= (todo ? n_todo : N)) return;              // whole wavefront leaves together
     const int p = todo ? todo[slot] : slot;               // all points, or the listed ones
     int* base = lds_i + (size_t)wave * (size_t)wave_lds_ints;
@@ -1140,9 +1140,11 @@ int launch_one(const float* points, const Bf16Copy& b, int N, int D, int K, cons
     RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_explore<SL, WAVES>),
                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     const int n_work = todo ? n_todo : N;
-    dim3 grid((unsigned)((n_work + WAVES - 1) / WAVES)), block(64 * WAVES);
-    hipLaunchKernelGGL((k_explore<SL, WAVES>), grid, block, lds, stream, points, b, N, D, K, old_idx, knn_idx, knn_dist,
-                       table, wave_ints, dpad, rows_per_group, todo, n_todo, stat);
+    for (int first = 0; first < n_work; first += std::min(kMostRows, n_work - first)) {
+        dim3 grid((unsigned)((std::min(kMostRows, n_work - first) + WAVES - 1) / WAVES)), block(64 * WAVES);
+        hipLaunchKernelGGL((k_explore<SL, WAVES>), grid, block, lds, stream, points, b, N, D, K, old_idx, knn_idx, knn_dist,
+                           table, wave_ints, dpad, rows_per_group, todo, first, n_todo, stat);
+    }
     RSFK_HIP(hipGetLastError());
     return 0;
 }

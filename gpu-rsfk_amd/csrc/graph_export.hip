@@ -38,14 +38,14 @@ __device__ __forceinline__ bool usable(int c, int p, int N, int drop_self) { ret
 
 // flag[p*K + k]: kNoEdge (empty slot, out of range, or a dropped self edge), kMutual (the neighbour stores p too),
 // kOneWay (it does not: the reverse edge has to be added).  n_own[p] = stored edges of p, extra[p] (zero on entry) =
-// reverse edges row p receives.
+// reverse edges row p receives.  One wavefront per point, from point `first` on.
 template <int SL>
-__global__ __launch_bounds__(256) void k_sym_flags(const int* __restrict__ idx, int N, int K, int drop_self,
+__global__ __launch_bounds__(256) void k_sym_flags(const int* __restrict__ idx, int first, int N, int K, int drop_self,
                                                    unsigned char* __restrict__ flag, int* __restrict__ n_own,
                                                    int* __restrict__ extra)
 {
     const int lane = threadIdx.x & 63;
-    const int p = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int p = first + blockIdx.x * 4 + (threadIdx.x >> 6);
     if (p >= N) return;
     int mine[SL];
 #pragma unroll
@@ -100,13 +100,13 @@ __global__ __launch_bounds__(256) void k_sym_len(const int* __restrict__ n_own, 
 // Lane k of the wavefront of p writes the stored edge k to its compacted place in row p and, for a one-way edge, the
 // reverse edge into the row of the neighbour behind that row's stored edges.
 template <int SL>
-__global__ __launch_bounds__(256) void k_sym_fill(const int* __restrict__ idx, const float* __restrict__ dist, int N, int K,
+__global__ __launch_bounds__(256) void k_sym_fill(const int* __restrict__ idx, const float* __restrict__ dist, int first, int N, int K,
                                                   const unsigned char* __restrict__ flag, const int* __restrict__ n_own,
                                                   int* __restrict__ cursor, const int* __restrict__ indptr,
                                                   int* __restrict__ cols, float* __restrict__ vals)
 {
     const int lane = threadIdx.x & 63;
-    const int p = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int p = first + blockIdx.x * 4 + (threadIdx.x >> 6);
     if (p >= N) return;
     const int row0 = indptr[p];
     int before = 0;
@@ -134,12 +134,14 @@ __global__ __launch_bounds__(256) void k_sym_fill(const int* __restrict__ idx, c
 
 int sym_launch_flags(const int* idx, int N, int K, int drop_self, unsigned char* flag, int* n_own, int* extra, hipStream_t stream)
 {
-    const dim3 grid((unsigned)((N + 3) / 4)), block(256);
-    if (K <= 64) hipLaunchKernelGGL(k_sym_flags<1>, grid, block, 0, stream, idx, N, K, drop_self, flag, n_own, extra);
-    else if (K <= 128) hipLaunchKernelGGL(k_sym_flags<2>, grid, block, 0, stream, idx, N, K, drop_self, flag, n_own, extra);
-    else if (K <= 256) hipLaunchKernelGGL(k_sym_flags<4>, grid, block, 0, stream, idx, N, K, drop_self, flag, n_own, extra);
-    else if (K <= 512) hipLaunchKernelGGL(k_sym_flags<8>, grid, block, 0, stream, idx, N, K, drop_self, flag, n_own, extra);
-    else hipLaunchKernelGGL(k_sym_flags<16>, grid, block, 0, stream, idx, N, K, drop_self, flag, n_own, extra);
+    for (int first = 0; first < N; first += std::min(kMostRows, N - first)) {
+        const dim3 grid((unsigned)((std::min(kMostRows, N - first) + 3) / 4)), block(256);
+        if (K <= 64) hipLaunchKernelGGL(k_sym_flags<1>, grid, block, 0, stream, idx, first, N, K, drop_self, flag, n_own, extra);
+        else if (K <= 128) hipLaunchKernelGGL(k_sym_flags<2>, grid, block, 0, stream, idx, first, N, K, drop_self, flag, n_own, extra);
+        else if (K <= 256) hipLaunchKernelGGL(k_sym_flags<4>, grid, block, 0, stream, idx, first, N, K, drop_self, flag, n_own, extra);
+        else if (K <= 512) hipLaunchKernelGGL(k_sym_flags<8>, grid, block, 0, stream, idx, first, N, K, drop_self, flag, n_own, extra);
+        else hipLaunchKernelGGL(k_sym_flags<16>, grid, block, 0, stream, idx, first, N, K, drop_self, flag, n_own, extra);
+    }
     RSFK_HIP(hipGetLastError());
     return 0;
 }
@@ -147,17 +149,19 @@ int sym_launch_flags(const int* idx, int N, int K, int drop_self, unsigned char*
 int sym_launch_fill(const int* idx, const float* dist, int N, int K, const unsigned char* flag, const int* n_own, int* cursor,
                     const int* indptr, int* cols, float* vals, hipStream_t stream)
 {
-    const dim3 grid((unsigned)((N + 3) / 4)), block(256);
-    if (K <= 64)
-        hipLaunchKernelGGL(k_sym_fill<1>, grid, block, 0, stream, idx, dist, N, K, flag, n_own, cursor, indptr, cols, vals);
-    else if (K <= 128)
-        hipLaunchKernelGGL(k_sym_fill<2>, grid, block, 0, stream, idx, dist, N, K, flag, n_own, cursor, indptr, cols, vals);
-    else if (K <= 256)
-        hipLaunchKernelGGL(k_sym_fill<4>, grid, block, 0, stream, idx, dist, N, K, flag, n_own, cursor, indptr, cols, vals);
-    else if (K <= 512)
-        hipLaunchKernelGGL(k_sym_fill<8>, grid, block, 0, stream, idx, dist, N, K, flag, n_own, cursor, indptr, cols, vals);
-    else
-        hipLaunchKernelGGL(k_sym_fill<16>, grid, block, 0, stream, idx, dist, N, K, flag, n_own, cursor, indptr, cols, vals);
+    for (int first = 0; first < N; first += std::min(kMostRows, N - first)) {
+        const dim3 grid((unsigned)((std::min(kMostRows, N - first) + 3) / 4)), block(256);
+        if (K <= 64)
+            hipLaunchKernelGGL(k_sym_fill<1>, grid, block, 0, stream, idx, dist, first, N, K, flag, n_own, cursor, indptr, cols, vals);
+        else if (K <= 128)
+            hipLaunchKernelGGL(k_sym_fill<2>, grid, block, 0, stream, idx, dist, first, N, K, flag, n_own, cursor, indptr, cols, vals);
+        else if (K <= 256)
+            hipLaunchKernelGGL(k_sym_fill<4>, grid, block, 0, stream, idx, dist, first, N, K, flag, n_own, cursor, indptr, cols, vals);
+        else if (K <= 512)
+            hipLaunchKernelGGL(k_sym_fill<8>, grid, block, 0, stream, idx, dist, first, N, K, flag, n_own, cursor, indptr, cols, vals);
+        else
+            hipLaunchKernelGGL(k_sym_fill<16>, grid, block, 0, stream, idx, dist, first, N, K, flag, n_own, cursor, indptr, cols, vals);
+    }
     RSFK_HIP(hipGetLastError());
     return 0;
 }
@@ -889,15 +893,18 @@ int symmetrize_flags(const int* d_idx, const float* d_dist, int N, int K, int dr
         return 1;
     int bits = 1;
     while (bits < 31 && (1ll << bits) < (long long)N) ++bits;          // columns are below N
+    // (the sort has a workgroup for a row: rows in pieces that a launch has threads for)
+    constexpr int kSortRows = 1 << 22;
     size_t sort_bytes = 0;
     RSFK_HIP(rocprim::segmented_radix_sort_pairs(nullptr, sort_bytes, static_cast<int*>(cols.p), d_cols,
-                                                 static_cast<float*>(vals.p), d_vals, (unsigned)n, (unsigned)N, d_indptr,
+                                                 static_cast<float*>(vals.p), d_vals, (unsigned)n, (unsigned)std::min(N, kSortRows), d_indptr,
                                                  d_indptr + 1, 0, (unsigned)bits, stream));
     Buf tmp;
     if (ws_alloc(&tmp.p, sort_bytes ? sort_bytes : 256)) return 1;
-    RSFK_HIP(rocprim::segmented_radix_sort_pairs(tmp.p, sort_bytes, static_cast<int*>(cols.p), d_cols,
-                                                 static_cast<float*>(vals.p), d_vals, (unsigned)n, (unsigned)N, d_indptr,
-                                                 d_indptr + 1, 0, (unsigned)bits, stream));
+    for (int first = 0; first < N; first += std::min(kSortRows, N - first))
+        RSFK_HIP(rocprim::segmented_radix_sort_pairs(tmp.p, sort_bytes, static_cast<int*>(cols.p), d_cols,
+                                                     static_cast<float*>(vals.p), d_vals, (unsigned)n, (unsigned)std::min(kSortRows, N - first),
+                                                     d_indptr + first, d_indptr + first + 1, 0, (unsigned)bits, stream));
     RSFK_HIP(hipStreamSynchronize(stream));
     return 0;
 }

@@ -72,6 +72,7 @@ inline unsigned grid_for_dies(size_t n_blocks) { return (unsigned)((n_blocks + k
 // A launch has fewer than 2^32 threads along x; what is beyond is cut off without an error.
 inline bool launch_fits(size_t groups, int threads) { return groups * (size_t)threads < ((size_t)1 << 32); }
 constexpr int kMostGroups = (1 << 24) - kDies;            // of 256 threads
+constexpr int kMostRows = 4 * kMostGroups;                // a wavefront each
 
 // ---------------------------------------------------------------------------
 // counter-based random numbers.  A node of a tree is identified by a 64-bit key

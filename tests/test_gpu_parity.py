@@ -705,6 +705,47 @@ def test_explore_of_more_points_than_a_launch_has_threads_for(gpu, N, D, K):
     gpu.lib().rsfk_release_workspace()
 
 
+def test_more_rows_than_a_launch_has_wavefronts_for(gpu):
+    """67.2 million points, 2^32 threads with a wavefront for every row: graph export by flags and exploration without the reversed graph (which takes
+    50 million).  Every row holds the next point, small integers for coordinates."""
+    import torch
+    N, D, K = 67200000, 2, 3
+    torch.cuda.empty_cache()
+    gpu.lib().rsfk_release_workspace()
+    if torch.cuda.mem_get_info()[0] < 60 << 30:
+        pytest.skip("needs 60 GB of device memory")
+    X = torch.randint(0, 256, (N, D), device="cuda", dtype=torch.float32)
+    p = torch.arange(N, device="cuda", dtype=torch.int32)
+    one, two, before = (p + 1) % N, (p + 2) % N, (p - 1) % N
+    d1, d2 = ((X[one] - X) ** 2).sum(1), ((X[two] - X) ** 2).sum(1)
+    idx = torch.full((N, K), -1, dtype=torch.int32, device="cuda")
+    dist = torch.full((N, K), float("inf"), device="cuda")
+    idx[:, 0] = one
+    dist[:, 0] = d1
+    indptr = torch.empty(N + 1, dtype=torch.int32, device="cuda")
+    cols = torch.empty((N, 2), dtype=torch.int32, device="cuda")
+    vals = torch.empty((N, 2), device="cuda")
+    torch.cuda.synchronize()
+    _say("symmetrize", N, K)
+    assert gpu.symmetrize_device(idx.data_ptr(), dist.data_ptr(), N, K, 1, indptr.data_ptr(), cols.data_ptr(), vals.data_ptr(), 2 * N) == 2 * N
+    assert torch.equal(indptr, 2 * torch.arange(N + 1, device="cuda", dtype=torch.int32))
+    swap = cols[:, 0] != one
+    assert torch.equal(torch.where(swap, cols[:, 1], cols[:, 0]), one) and torch.equal(torch.where(swap, cols[:, 0], cols[:, 1]), before)
+    assert torch.equal(torch.where(swap, vals[:, 1], vals[:, 0]), d1) and torch.equal(torch.where(swap, vals[:, 0], vals[:, 1]), d1[before])
+    del indptr, cols, vals, swap
+    scratch = torch.empty((N, K), dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    _say("explore", N, D, K)
+    gpu.explore_device(X.data_ptr(), N, D, K, idx.data_ptr(), dist.data_ptr(), scratch.data_ptr())
+    first = (d1 < d2) | ((d1 == d2) & (one < two))
+    assert torch.equal(idx[:, 0], torch.where(first, one, two)) and torch.equal(idx[:, 1], torch.where(first, two, one))
+    assert torch.equal(dist[:, 0], torch.minimum(d1, d2)) and torch.equal(dist[:, 1], torch.maximum(d1, d2))
+    assert bool((idx[:, 2] == -1).all())
+    del idx, dist, X, scratch
+    torch.cuda.empty_cache()
+    gpu.lib().rsfk_release_workspace()
+
+
 @pytest.mark.parametrize("values", ["far", "tiny", "huge", "outlier", "spread", "notfinite"])
 @pytest.mark.parametrize("N,D,K", [(2500, 16, 8), (2500, 33, 32), (1500, 129, 20), (1500, 40, 70)])
 def test_explore_screens_rows_of_any_magnitude(gpu, orc, rng, N, D, K, values):
