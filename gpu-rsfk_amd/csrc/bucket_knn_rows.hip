@@ -124,7 +124,7 @@ __global__ __launch_bounds__(kRowsThreads, 4) void k_bucket_knn_rows(const float
             if (in[t]) { lo = fminf(lo, acc[t]); sum += acc[t]; }
         lo = -wave_max(-lo);
         float hi = row.tau;
-        if (!(hi < INFINITY)) {
+        if (row.tau_i < 0) {                                         // (an empty last slot, whatever distance stands there)
             hi = wave_total_f(sum) * __builtin_amdgcn_rcpf((float)n_in);
             int n_below = n_row;
 #pragma unroll

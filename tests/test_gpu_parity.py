@@ -382,12 +382,12 @@ def test_bucket_knn_rows_that_start_new(gpu, orc, rng, start, data, K):
 
 
 @pytest.mark.parametrize("data", ["continuous", "grid", "mixed", "notfinite"])
-@pytest.mark.parametrize("start", ["self", "empty", "self_far"])
+@pytest.mark.parametrize("start", ["self", "empty", "self_far", "flt_max"])
 @pytest.mark.parametrize("K,MIN,MAX", [(8, 40, 120), (32, 64, 256), (60, 61, 200), (64, 33, 190)])
 def test_bucket_knn_resident_rows_merged_by_counting(gpu, orc, rng, K, MIN, MAX, start, data):
     """Buckets of 73..256 points whose rows are merged by counting: rows that are new, rows of which most points are in the bucket
     again (the same partition twice), rows that are neither new nor full, equal distances, duplicated points, points that are not
-    finite, and rows too long for one wavefront to count."""
+    finite, and rows too long for one wavefront to count.  Empty slots hold +inf, or FLT_MAX as the reference's CLI leaves them."""
     N, D = 4000, 5
     X = rng.standard_normal((N, D)).astype(np.float32)
     perm, ls, lz, _ = orc.build_tree(X, MIN, MAX, 5000, 3)
@@ -401,10 +401,10 @@ def test_bucket_knn_resident_rows_merged_by_counting(gpu, orc, rng, K, MIN, MAX,
         X[rng.integers(0, N, 30), rng.integers(0, D, 30)] = np.nan
         X[rng.integers(0, N, 30), 0] = np.inf
     oi = np.full((N, K), -1, np.int32)
-    od = np.full((N, K), np.inf, np.float32)
+    od = np.full((N, K), np.finfo(np.float32).max if start == "flt_max" else np.inf, np.float32)
     if start != "empty":
         oi[:, 0] = np.arange(N)
-        od[:, 0] = 0.0 if start == "self" else 0.3
+        od[:, 0] = 0.3 if start == "self_far" else 0.0
     gi, gd = oi.copy(), od.copy()
     for perm, ls, lz in parts:
         _say("bucket_knn by counting", K, MIN, MAX, start, data)
