@@ -670,11 +670,11 @@ int launch_ann_ws_init(int* ws, int NQ, int rec_cap, unsigned long long* stats, 
 // the tree has n_leaves buckets), groups them by bucket and offers the base points perm[..] of the bucket a query
 // reached to the query's row.  prev, stats: numbers of pairs of the tree before this one (null: the first) and of this one,
 // kAnnStatWords each.  q_copy, p_copy: null, or the copy of the queries, of the points
-// (with q_copy only: the screened bucket step reads them).  start: the records from which the queries go on (null: the root).  ws: ann_ws_ints(NQ, rec_cap) ints, prepared by launch_ann_ws_init; planes: rec_cap
+// (with q_copy only: the screened bucket step reads them).  n_trees: of the call.  start: the records from which the queries go on (null: the root).  ws: ann_ws_ints(NQ, rec_cap) ints, prepared by launch_ann_ws_init; planes: rec_cap
 // ann_plane_pitch(N, NQ, D) floats and 256 bytes.
 int launch_ann_tree(const float* points, const float* queries, int N, int NQ, int D, int K, const int* perm, const TreeRec* recs,
                     const int* n_rec_dev, int rec_cap, int n_leaves, const JoinCopy* q_copy, const JoinCopy* p_copy,
-                    const int* start, int* ws, float* planes, int* q_idx, float* q_dist,
+                    int n_trees, const int* start, int* ws, float* planes, int* q_idx, float* q_dist,
                     const unsigned long long* prev, unsigned long long* stats, hipStream_t stream)
 {
     if (NQ <= 0) return 0;
@@ -711,7 +711,7 @@ int launch_ann_tree(const float* points, const float* queries, int N, int NQ, in
     // a bucket with c queries takes ceil(c / 16) work items: at most NQ / 16 + (buckets with queries) in all
     const int most_items = NQ / kQB + std::min(n_leaves, NQ) + 1;
     const unsigned int share_q16 = ann_screen_share_q16(N, NQ, D, K, n_leaves);
-    AnnForm form = {share_q16 != 0 ? prev : nullptr, stats, share_q16, 0};
+    AnnForm form = {share_q16 != 0 ? prev : nullptr, stats, share_q16, p_copy ? ann_half_share_q16(N, NQ, D, n_trees, share_q16) : 0u, 0};
     while ((most_items >> form.shift) > 512) ++form.shift;
     const unsigned g_scan = (unsigned)(rec_cap / kScanTile + 1);
     hipLaunchKernelGGL(k_ann_tile_sums, dim3(g_scan), dim3(256), 0, stream, cnt, cnt_shift, n_rec_dev, rec_cap, tile_sum, form);
@@ -719,10 +719,11 @@ int launch_ann_tree(const float* points, const float* queries, int N, int NQ, in
     const unsigned g_fill = (unsigned)((std::max(NQ, rec_cap) + 255) / 256);
     hipLaunchKernelGGL(k_ann_fill, dim3(g_fill), dim3(256), 0, stream, NQ, q_rec, q_rank, n_rec_dev, rec_cap, recs, qoff, boff, qlist,
                        blk_desc, form);
-    // (the form that is not taken finds out in every workgroup, hence few of them)
-    if (form.prev && p_copy) {
-        if (launch_ann_screen_half(*q_copy, *p_copy, points, queries, D, K, perm, blk_desc, n_blocks, most_items, qlist, q_idx, q_dist, form, stream)) return 1;
-    } else if (form.prev) {
+    // (the forms that are not taken find out in every workgroup, hence few of them)
+    if (form.prev && form.half_q16 != 0 &&
+        launch_ann_screen_half(*q_copy, *p_copy, points, queries, D, K, perm, blk_desc, n_blocks, most_items, qlist, q_idx, q_dist, form, stream))
+        return 1;
+    if (form.prev && form.half_q16 != form.share_q16) {
         if (launch_ann_screen(points, queries, D, K, perm, blk_desc, n_blocks, most_items, qlist, q_idx, q_dist, form, stream)) return 1;
     }
     const unsigned g_leaf = (unsigned)std::min(most_items, kLeafGrid);

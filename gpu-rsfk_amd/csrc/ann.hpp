@@ -16,20 +16,23 @@ constexpr int kAnnStatWords = 8;      // of a tree: pairs << 32 | pairs that had
 struct AnnForm {
     const unsigned long long* prev;
     unsigned long long* stats;        // this tree's own (null: none are kept)
-    unsigned int share_q16;           // the screened form when fewer than share_q16 / 65536 of the pairs had to be evaluated
+    unsigned int share_q16;           // a screened form when fewer than share_q16 / 65536 of the pairs had to be evaluated,
+    unsigned int half_q16;            // the one by float16 copies when fewer than this (at most share_q16; 0: never)
     int shift;                        // one work item in 2^shift is counted
 
-    __device__ __forceinline__ bool screened() const
+    __device__ __forceinline__ bool screened() const { return below(share_q16); }
+    __device__ __forceinline__ bool by_copies() const { return half_q16 != 0 && below(half_q16); }
+    __device__ __forceinline__ bool below(unsigned int share) const
     {
         if (prev == nullptr) return false;
-        if (share_q16 == kScreenAlways) return true;
+        if (share == kScreenAlways) return true;
         unsigned long long pairs = 0, listed = 0;
 #pragma unroll
         for (int i = 0; i < kAnnStatWords; ++i) {
             pairs += prev[i] >> 32;
             listed += prev[i] & 0xffffffffull;
         }
-        return (listed << 16) < pairs * share_q16;
+        return (listed << 16) < pairs * share;
     }
     __device__ __forceinline__ bool counts(int item) const { return stats != nullptr && (item & ((1 << shift) - 1)) == 0; }
     __device__ __forceinline__ unsigned long long* word(int item) const { return &stats[(item >> shift) & (kAnnStatWords - 1)]; }
@@ -100,7 +103,7 @@ __device__ __forceinline__ uint16_t rounded_value(float nd, const RoundedPlane& 
 int launch_ann_screen(const float* points, const float* queries, int D, int K, const int* perm, const int4* blk_desc,
                       const int* n_blocks, int most_blocks, const int* qlist, int* q_idx, float* q_dist, const AnnForm& form,
                       hipStream_t stream);
-// ann_screen_half.hip: the same by copies of the queries and of the points with the same mu and s
+// ann_screen_half.hip: the same by copies of the queries and of the points with the same mu and s; only when form.by_copies(), when the one above leaves
 int launch_ann_screen_half(const JoinCopy& qc, const JoinCopy& pc, const float* points, const float* queries, int D, int K, const int* perm,
                            const int4* blk_desc, const int* n_blocks, int most_blocks, const int* qlist, int* q_idx, float* q_dist,
                            const AnnForm& form, hipStream_t stream);

@@ -15,7 +15,7 @@
 // trees 0.57 ms where k_ann_leaf takes 0.85 (vector ALUs); the first trees, where most pairs are left, 2.9 against 1.9.  Tried: the
 // members' rows of step 3 through a transposing tile in LDS (faster at D = 256 while many pairs are left, 0.65 ms here), K-NN
 // rows requested before the chains run (no change), two steps of 16 dimensions in flight in separate buffers (spills).
-// (Rows of 97 to 128 dimensions: ann_screen_half.hip, where there is room for copies of them.)
+// (Late trees of large inputs of 97 to 128 dimensions: ann_screen_half.hip, where there is room for copies of the rows.)
 // No barrier: the wavefronts of a workgroup share nothing but the cache lines of a bucket they may both work on.
 #include "forest.hpp"
 #include "ann.hpp"
@@ -44,7 +44,7 @@ __global__ __launch_bounds__(256, 4) void k_ann_screen(const float* __restrict__
                                                     int* __restrict__ q_idx, float* __restrict__ q_dist, float c_err,
                                                     float one_minus_gamma, AnnForm form)
 {
-    if (!form.screened()) return;
+    if (!form.screened() || form.by_copies()) return;
     __shared__ AnnScreenLds lds_s[4];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int half = lane >> 5, r = lane & 31;

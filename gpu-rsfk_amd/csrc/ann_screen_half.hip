@@ -1,5 +1,5 @@
-// The screened bucket step of the query-set search (ann_screen.hip) for rows of 97 to 128 dimensions, by float16 copies of the queries and the
-// points (join_copy.hpp, the same mu and s for both): same results.
+// The screened bucket step of the query-set search (ann_screen.hip) for late trees over many rows of 97 to 128 dimensions, by float16 copies of the
+// queries and the points (join_copy.hpp, the same mu and s for both): same results.
 //
 // In ann_screen.hip a lane reads "its" fp32 row 16 bytes at a time: a load touches up to 64 rows, comes back to a cache line seven times
 // while the line is still on its way, and rows of 400 bytes straddle lines, so that the address units are busy 82 % of the time and
@@ -12,9 +12,9 @@
 //   3. the pairs that are left wait until there are 64 of them, over several items: rows of the queries, then of the members, 128 bytes at a
 //      time through the tile; a lane runs the sequential chain of its pair;
 //   4. the pairs whose distance is not above the last slot (as it was when the pair was listed) are merged into the rows.
-// Bound by the lines it fetches: the last of 50 trees 0.565 -> 0.42 ms (14 million lines, 4.3 TB/s), all 47 screened ones 31.9 -> 26.2.  Where rows
-// are shorter or aligned to lines the form above is the faster one (300,000 / 500,000, 30 trees of K = 32, ann_screen.hip -> here: x 128 24.6 -> 23.6
-// ms, x 100 22.7 -> 22.1, x 80 19.7 -> 20.4, x 64 17.1 -> 17.7, x 40 15.7 -> 17.1).  One wavefront per workgroup, 11 of them per compute unit (LDS);
+// Bound by the lines it fetches: the last of 50 trees 0.565 -> 0.42 ms (14 million lines, 4.3 TB/s).  Where rows are shorter or aligned to lines the
+// form above is the faster one (300,000 / 500,000, 30 trees of K = 32, ann_screen.hip -> here for all screened trees: x 80 19.7 -> 20.4, x 64 17.1
+// -> 17.7, x 40 15.7 -> 17.1), and so it is in early trees and where the rows stay in the last cache (ann_half_share_q16).  One wavefront per workgroup, 11 of them per compute unit (LDS);
 // 16,384 workgroups at most: 8,192 end with a tail (28.2), one item each leaves the waiting list half empty (27.1).
 #include "forest.hpp"
 #include "ann.hpp"
@@ -146,7 +146,7 @@ __global__ __launch_bounds__(64, 3) void k_ann_screen_half(JoinCopy qc, JoinCopy
                                                        int* __restrict__ q_idx, float* __restrict__ q_dist, const float* __restrict__ scale, float kappa,
                                                        float err_rel, float err_abs, float one_minus_gamma, AnnForm form)
 {
-    if (!form.screened()) return;
+    if (!form.by_copies()) return;
     __shared__ AnnHalfLds L;
     const int lane = threadIdx.x, half = lane >> 5, r = lane & 31, sub = lane & 7, grp = lane >> 3;
     const int n_items = *n_blocks, pitch = 16 * kSteps;
@@ -298,8 +298,21 @@ __global__ __launch_bounds__(64, 3) void k_ann_screen_half(JoinCopy qc, JoinCopy
 
 }  // namespace
 
-// Rows whose bounds are made from the copies (measured at the top).
-bool ann_half_wanted(int D) { return D > 96 && D <= 128; }
+// The share of pairs (as ann_screen_share_q16) below which the bounds are made from the copies, 0: never.  The rows of the copies come in whole lines,
+// but a pair that is left is one of 64 that wait together and costs more than in ann_screen.hip: trees late in a call, and rows that do not
+// stay in the last cache (256 MB).  Per tree, fp32 rows -> copies, with the share that was left: 1M / 1M x 100 1797 -> 1895 us at 14 %, 1675 -> 1649 at
+// 10 %, 1397 -> 1199 at 3.8 %; 500,000 / 500,000 x 128 785 -> 812 at 7.8 %, 724 -> 712 at 5.0 %, 671 -> 635 at 3 %; 300,000 / 500,000 x 100 702 -> 781 at 10 %,
+// 617 -> 617 at 5.0 %, 550 -> 514 at 2.5 %; 200,000 / 300,000 x 100 405 -> 495, 330 -> 356, 311 -> 324; 60,000 / 250,000 x 128 276 -> 309, 230 -> 247, 216 -> 227.
+// Tree t leaves about 72 / t per cent, and the copies take as long as two or three trees gain (300,000 / 500,000: seven): calls of fewer trees make none.
+unsigned int ann_half_share_q16(int N, int NQ, int D, int n_trees, unsigned int share_q16)
+{
+    if (D <= 96 || D > 128 || share_q16 == 0) return 0;
+    if (share_q16 == kScreenAlways) return n_trees > 1 ? kScreenAlways : 0;
+    const size_t bytes = ((size_t)N + (size_t)NQ) * (size_t)D * sizeof(float);
+    const bool beyond = bytes >= (size_t)640 << 20;
+    if (bytes < (size_t)256 << 20 || n_trees < (beyond ? 12 : 30)) return 0;
+    return std::min(share_q16, (unsigned int)((beyond ? 0.12 : 0.055) * 65536.0));
+}
 
 int launch_ann_screen_half(const JoinCopy& qc, const JoinCopy& pc, const float* points, const float* queries, int D, int K, const int* perm,
                            const int4* blk_desc, const int* n_blocks, int most_blocks, const int* qlist, int* q_idx, float* q_dist,

@@ -546,7 +546,7 @@ int knn_ann_forest_device(int n_trees, int K, int N, int NQ, int D, int MIN, int
             int group = ann_forest_group(N, NQ, D, K, MAX, max_bucket, rec_cap, nb);
             if (group > 0 && !room_together(group)) group = 0;
             bool screened = false;
-            for (int j = 0; j < nb; ++j) screened = screened || (ann_half_wanted(D) && ann_screen_share_q16(N, NQ, D, K, stats[5 * j]) != 0);
+            for (int j = 0; j < nb; ++j) screened = screened || ann_half_share_q16(N, NQ, D, n_trees, ann_screen_share_q16(N, NQ, D, K, stats[5 * j])) != 0;
             if (group == 0 && (room_alone() || room_copies(screened))) return 1;
             if (group > 0) (void)hipEventRecord(ev[0].e, stream);
             for (int j = 0; j < nb && rc == 0 && group > 0; j += group)
@@ -562,7 +562,7 @@ int knn_ann_forest_device(int n_trees, int K, int N, int NQ, int D, int MIN, int
                 const int* start = top_trees > 0 ? static_cast<const int*>(top_start.p) + (size_t)(j % top_trees) * (size_t)NQ : nullptr;
                 rc = launch_ann_tree(d_points, d_queries, N, NQ, D, K, tree_ws_perm(ws.w, j), tree_ws_recs(ws.w, j),
                                      tree_ws_n_rec(ws.w, j), rec_cap, stats[5 * j + 0], q_copy.c.rows ? &q_copy.c : nullptr,
-                                     p_copy.c.rows ? &p_copy.c : nullptr, start, static_cast<int*>(aws.p),
+                                     p_copy.c.rows ? &p_copy.c : nullptr, n_trees, start, static_cast<int*>(aws.p),
                                      static_cast<float*>(planes.p), d_qidx, d_qdist,
                                      tb0 + j > 0 ? static_cast<unsigned long long*>(pair_stats.p) + ann_stat_words(tb0 + j - 1) : nullptr,
                                      static_cast<unsigned long long*>(pair_stats.p) + ann_stat_words(tb0 + j), stream);

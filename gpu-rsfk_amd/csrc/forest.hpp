@@ -243,13 +243,13 @@ int symmetrize_host(const int* idx, const float* dist, int N, int K, int drop_se
 size_t ann_ws_ints(int NQ, int rec_cap);
 int ann_plane_pitch(int N, int NQ, int D);
 bool ann_low_wanted(int N, int NQ, int D);
-bool ann_half_wanted(int D);
+unsigned int ann_half_share_q16(int N, int NQ, int D, int n_trees, unsigned int share_q16);
 unsigned int ann_screen_share_q16(int N, int NQ, int D, int K, int n_leaves);
 size_t ann_stat_words(int n_trees);
 int launch_ann_ws_init(int* ws, int NQ, int rec_cap, unsigned long long* stats, int n_trees, hipStream_t stream);
 int launch_ann_tree(const float* points, const float* queries, int N, int NQ, int D, int K, const int* perm, const TreeRec* recs,
                     const int* n_rec_dev, int rec_cap, int n_leaves, const JoinCopy* q_copy, const JoinCopy* p_copy,
-                    const int* start, int* ws, float* planes, int* q_idx, float* q_dist,
+                    int n_trees, const int* start, int* ws, float* planes, int* q_idx, float* q_dist,
                     const unsigned long long* prev, unsigned long long* stats, hipStream_t stream);
 // ann_top.hip: the first levels of the trees of a batch
 bool ann_top_wanted(int NQ, int D);

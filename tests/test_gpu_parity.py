@@ -1445,6 +1445,26 @@ def test_ann_screened_by_copies_matches_oracle(gpu, capi, orc, rng, monkeypatch,
         assert_knn_equal(idx.cpu().numpy(), dist.cpu().numpy(), oi, od)
 
 
+# calls whose early screened trees bound the pairs by the fp32 rows and whose late ones by the copies: from 256 MB and from 640 MB of rows on
+@pytest.mark.parametrize("N,NQ,D,K,T", [(300000, 500001, 97, 10, 30), (700001, 900000, 104, 6, 14)])
+def test_ann_screened_by_fp32_rows_then_by_copies(gpu, capi, monkeypatch, N, NQ, D, K, T):
+    """== the search without room for copies (which the oracle has confirmed at small sizes)."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(3)
+    X, Q = torch.randn(N, D, device="cuda", generator=g), torch.randn(NQ, D, device="cuda", generator=g)
+    out = []
+    for room in (None, "0"):
+        if room is not None:
+            monkeypatch.setenv("RSFK_OPTIONAL_MB", room)
+        idx = torch.full((NQ, K), -1, dtype=torch.int32, device="cuda")
+        dist = torch.full((NQ, K), float("inf"), device="cuda")
+        torch.cuda.synchronize()
+        _say("ann screened twice", N, NQ, D, K, T, room)
+        capi.knn_ann_device(T, K, N, NQ, D, K + 1, 2 * K + 2, 5000, 0, 3, X.data_ptr(), Q.data_ptr(), idx.data_ptr(), dist.data_ptr())
+        out.append((idx, dist))
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
+
+
 # Workgroups with many items each, as they have them from about 16,384 items (a million queries) on: the items that follow an item are looked up while it is
 # worked on, and pairs of several items wait for each other.  Buckets of few members and queries (a pair or two of an item are
 # left, so that tens of items wait together), items of 32 queries and more than one block of members, items between these; one workgroup,
