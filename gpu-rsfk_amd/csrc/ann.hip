@@ -618,7 +618,11 @@ int count_shift(int rec_cap)
 
 // floats of working memory a record of a tree takes (both tables of hyperplanes)
 int ann_plane_pitch(int N, int NQ, int D) { return plane_pitch(D) + low_plane_pitch(N, NQ, D); }
-bool ann_low_wanted(int N, int NQ, int D) { return low_plane_pitch(N, NQ, D) > 0; }
+bool ann_low_wanted(int n_trees, int N, int NQ, int D)
+{
+    const char* e = std::getenv("RSFK_ANN_ROUTE_LOW");
+    return low_plane_pitch(N, NQ, D) > 0 && ((e && *e) || ann_copy_pays(n_trees, NQ));
+}
 
 size_t ann_ws_ints(int NQ, int rec_cap)
 {

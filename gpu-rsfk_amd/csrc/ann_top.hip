@@ -187,14 +187,14 @@ __global__ __launch_bounds__(256) void k_route_top(JoinCopy jc, int NQ, int n_tr
 
 // 20 trees, all levels by k_route or k_route_low -> the first seven here: 300,000 / 300,000 x 8 7.82 -> 7.67 ms, x 100 12.6 -> 12.4; 60,000
 // points, 1M queries x 8 15.4 -> 14.7, x 128 26.1 -> 25.6; 20,000 / 100,000 x 50 3.21 -> 3.18; 1M / 100,000 x 8 to x 128 the same, and so are 50,000
-// queries and fewer.  RSFK_ANN_TOP=1 / 0 says yes or no.
-bool ann_top_wanted(int NQ, int D)
+// queries and fewer.  Few trees do not pay for the copy of the queries (ann_copy_pays).  RSFK_ANN_TOP=1 / 0 says yes or no.
+bool ann_top_wanted(int n_trees, int NQ, int D)
 {
     const char* e = std::getenv("RSFK_ANN_TOP");
     if (e && e[0] == '0') return false;
     if (D > 128) return false;
     if (e && e[0] == '1') return true;
-    return NQ >= 100000;
+    return NQ >= 100000 && ann_copy_pays(n_trees, NQ);
 }
 
 size_t ann_top_bytes(int n_trees, int D)

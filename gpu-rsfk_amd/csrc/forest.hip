@@ -508,9 +508,9 @@ int knn_ann_forest_device(int n_trees, int K, int N, int NQ, int D, int MIN, int
         JoinCopyGuard q_copy, p_copy;
         DevBuf top_ws, top_start;
         bool q_asked = false, p_asked = false;
-        int top_trees = ann_top_wanted(NQ, D) ? (int)std::min<size_t>((size_t)B, ((size_t)512 << 20) / (sizeof(int) * (size_t)NQ)) : 0;
+        int top_trees = ann_top_wanted(n_trees, NQ, D) ? (int)std::min<size_t>((size_t)B, ((size_t)512 << 20) / (sizeof(int) * (size_t)NQ)) : 0;
         const auto room_copies = [&](bool screened) -> int {
-            const bool points_too = screened && !p_asked, queries_too = (screened || top_trees > 0 || ann_low_wanted(N, NQ, D)) && !q_asked;
+            const bool points_too = screened && !p_asked, queries_too = (screened || top_trees > 0 || ann_low_wanted(n_trees, N, NQ, D)) && !q_asked;
             if (queries_too) {
                 q_asked = true;
                 if (join_copy_alloc(&q_copy.c, NQ, D, true)) join_copy_free(&q_copy.c);

@@ -242,8 +242,12 @@ int symmetrize_host(const int* idx, const float* dist, int N, int K, int drop_se
 // ann.hip
 size_t ann_ws_ints(int NQ, int rec_cap);
 int ann_plane_pitch(int N, int NQ, int D);
-bool ann_low_wanted(int N, int NQ, int D);
+bool ann_low_wanted(int n_trees, int N, int NQ, int D);
 unsigned int ann_half_share_q16(int N, int NQ, int D, int n_trees, unsigned int share_q16);
+// Does the float16 copy of the queries, for their way through the trees, take less than what it gives?  (x 50 300,000 / 120,000 3 trees 1.94 -> 1.99 ms
+// with it, 8 3.44 -> 3.43, 20 6.52 -> 6.37; 100,000 / 100,000 x 100 1.54 -> 1.57, 2.63 -> 2.63, 5.14 -> 4.95; 300,000 / 600,000 x 80 one tree 2.35 -> 2.46, 3
+// 4.83 -> 4.77, 8 9.16 -> 8.75.)
+inline bool ann_copy_pays(int n_trees, int NQ) { return (long long)n_trees * NQ >= 1500000; }
 unsigned int ann_screen_share_q16(int N, int NQ, int D, int K, int n_leaves);
 size_t ann_stat_words(int n_trees);
 int launch_ann_ws_init(int* ws, int NQ, int rec_cap, unsigned long long* stats, int n_trees, hipStream_t stream);
@@ -252,7 +256,7 @@ int launch_ann_tree(const float* points, const float* queries, int N, int NQ, in
                     int n_trees, const int* start, int* ws, float* planes, int* q_idx, float* q_dist,
                     const unsigned long long* prev, unsigned long long* stats, hipStream_t stream);
 // ann_top.hip: the first levels of the trees of a batch
-bool ann_top_wanted(int NQ, int D);
+bool ann_top_wanted(int n_trees, int NQ, int D);
 size_t ann_top_bytes(int n_trees, int D);
 int launch_ann_top(const float* points, const JoinCopy& jc, int NQ, int D, int n_trees, const TreeRec* recs, const int* n_rec_dev, int rec_cap,
                    void* ws, int* start, hipStream_t stream);
