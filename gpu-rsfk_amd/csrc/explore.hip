@@ -1194,7 +1194,7 @@ bool explore_merge_fits(int D, int K)
 // distance.
 int launch_explore(const float* points, const Bf16Copy* bf, const JoinCopy* jc, int N, int D, int K, int* knn_idx,
                    float* knn_dist, int* old_idx, ExploreWorkspace* ws, hipStream_t stream, bool rows_sorted,
-                   unsigned long long* stat, const int* order)
+                   unsigned long long* stat, const int* order, bool one_tree)
 {
     if (N <= 0) return 0;
     RSFK_CHECK(K >= 1 && K <= kMaxK, "exploration: K must be in 1..1024");
@@ -1249,9 +1249,13 @@ int launch_explore(const float* points, const Bf16Copy* bf, const JoinCopy* jc, 
         // workgroup per point instead.  So do sets of 2048 places and more where the join kept its codes (at least one workgroup of
         // four of them fits a compute unit, but they evaluate every candidate, and that kernel what the codes leave):
         // whole pass with points that have most of their marks, D = 132, K = 40 5.4 -> 4.5 ms, K = 50 14.1 -> 6.0; D = 256, K = 32
-        // 9.2 -> 4.9, K = 60 28.6 -> 8.0; D = 960, K = 60 36.5 -> 5.9.  K = 32 is even at D = 192 and slower at D = 132 (3.9 -> 4.4).
+        // 9.2 -> 4.9, K = 60 28.6 -> 8.0; D = 960, K = 60 36.5 -> 5.9.  Not with K = 32 while two workgroups fit (120,000 points after two trees, by
+        // wavefronts -> by workgroups: D = 192 3.21 -> 3.55 ms, 224 3.56 -> 3.82, 256 6.38 -> 3.89, in clusters after four 192 2.93 -> 3.33, 224 3.29 ->
+        // 3.66, 256 5.51 -> 3.79), and not after one tree, when the many marks of a point are the few points of its bucket (D = 132, K = 38 2.36 ->
+        // 5.13, D = 192, K = 32 1.75 -> 3.99, K = 60 7.48 -> 8.98, D = 420, K = 60 9.79 -> 10.16).
         const WgSizes wg = merge_wg_sizes(dpad, K);
-        const bool by_codes = explore_ws_bounds(ws).codes != nullptr && big_table >= 2048 && (K > 32 || D >= 192) && wg.cap > 0;
+        const bool by_codes = explore_ws_bounds(ws).codes != nullptr && big_table >= 2048 && !one_tree && wg.cap > 0 &&
+                              (K > 32 || merge_wave_ints(big_table, dpad, K) > 80 * 1024 / 16);
         const bool per_wg = big_waves < 4 || by_codes;
         if (!per_wg)
             while (big_table > small_table && merge_wave_ints(big_table, dpad, K) > lds_ints / big_waves) big_table >>= 1;

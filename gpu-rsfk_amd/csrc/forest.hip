@@ -433,7 +433,8 @@ int knn_forest_device(int n_trees, int K, int N, int D, int MIN, int MAX, int MA
         for (int it = 0; it < nnef; ++it) {
             // (the bucket step of the forest, and every exploration pass, leave all rows in order)
             if (launch_explore(d_points, plain_copy ? &bf.c : nullptr, &jc.c, N, D, K, d_idx, d_dist, static_cast<int*>(old.p), ews.w, stream,
-                               n_trees > 0 || it > 0, static_cast<unsigned long long*>(stat.p), static_cast<const int*>(order.p)))
+                               n_trees > 0 || it > 0, static_cast<unsigned long long*>(stat.p), static_cast<const int*>(order.p),
+                               n_trees == 1 && it == 0))
                 return 1;
         }
         std::vector<unsigned long long> h_stat((size_t)kExploreStatWords);

@@ -227,7 +227,8 @@ bool explore_join_keeps_bounds(int N, int D, int K);
 int launch_explore(const float* points, const Bf16Copy* bf, const JoinCopy* jc, int N, int D, int K, int* knn_idx,
                    float* knn_dist, int* old_idx, ExploreWorkspace* ws, hipStream_t stream, bool rows_sorted = false,
                    unsigned long long* stat = nullptr,       // stat: kExploreStatWords words, or null (count_exact)
-                   const int* order = nullptr);              // order: see launch_explore_join
+                   const int* order = nullptr,               // order: see launch_explore_join
+                   bool one_tree = false);                   // the rows come from the buckets of one tree (which kernels are faster)
 constexpr int kExploreStatWords = 32 * 256;
 
 // graph_export.hip
