@@ -854,21 +854,20 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_join_short(JoinCopy jc, 
 // points of R(q) and all neighbours of q pass through LDS together, 64 dimensions at a time (the next 64 are requested
 // while these are used), and the wavefronts share the pairs (tile of R(q), group of neighbours) among them, each
 // keeping the accumulators of its pairs: every row is read once per 96 points of R(q).  Bound and outputs are those
-// of k_explore_join.  K <= 128; at three wavefronts per SIMD
-// (70,000 x 784, K = 90 6.9 -> 5.1 ms against two).
+// of k_explore_join.  NPW = pairs per wavefront (3: K <= 128, at three wavefronts per SIMD, 70,000 x 784, K = 90 6.9 -> 5.1 ms against two; 6: K <= 256, at
+// one).
 constexpr int kJwP = 96;                    // points of R(q) worked on together (three tiles)
 constexpr int kJwRowBytes = 144;            // 64 float16 values + 16 bytes: rows start in different banks
 
-template <bool BOUNDS>
-__global__ __launch_bounds__(256, 3) void k_explore_join_wg(JoinCopy jc, int N, int K, const int* __restrict__ old_idx,
+template <bool BOUNDS, int NPW>
+__global__ __launch_bounds__(256, NPW == 3 ? 3 : 1) void k_explore_join_wg(JoinCopy jc, int N, int K, const int* __restrict__ old_idx,
                                                          const float* __restrict__ bars, const int* __restrict__ offs,
                                                          const int* __restrict__ rev, uint32_t* __restrict__ pass,
                                                          uint16_t* __restrict__ bounds, int KP, int bpitch, int ksteps,
                                                          float kappa, float any_rel, float any_abs, uint32_t div_m, int div_s,
                                                          const int* __restrict__ order)
 {
-    constexpr int NPW = 3;                                                 // pairs per wavefront
-    constexpr int kPieces = (kJwP + 128) * 8 / 256;                        // 16-byte pieces a thread stages per step
+    constexpr int kPieces = (kJwP + (NPW == 3 ? 128 : 256)) * 8 / 256;     // 16-byte pieces a thread stages per step
     extern __shared__ __align__(16) unsigned char lds_jw[];
     unsigned char* rowsb = lds_jw;                                         // kJwP + KP rows of 144 bytes
     int* cq = reinterpret_cast<int*>(rowsb + (size_t)(kJwP + KP) * kJwRowBytes);
@@ -1241,20 +1240,23 @@ int launch_explore_join(ExploreWorkspace* w, const JoinCopy& jc, int N, int D, i
     // are one pair per tile of R(q), too little for four wavefronts (1M x 256, K = 32: 8.1 ms against 12.6).  A pass, a wavefront per q -> a
     // workgroup: 123,457 x 37, K = 45 1.49 -> 2.08 ms, 300,000 x 64, K = 64 10.1 -> 11.6, x 200 16.7 -> 16.8, x 300 20.0 -> 18.5, 200,000 x 600, K = 40
     // 10.9 -> 10.4, 300,000 x 64, K = 90 17.8 -> 19.0, x 100 20.8 -> 20.8, 100,000 x 128, K = 90 7.07 -> 6.89, x 400 12.3 -> 9.6, 200,000 x 16, K = 128 19.3
-    // -> 19.6, x 32 17.0 -> 16.9, 100,000 x 256, K = 128 15.0 -> 11.4.  Above 128 neighbours its accumulators leave one wavefront per SIMD: 100,000 x 32,
-    // K = 160 18.3 -> 29.7.
-    if (KP > 32 && KP <= 128 && join_wg_on() && wg_fits && D * (K - 24) > (MW == 2 ? 8000 : MW == 3 ? 6500 : 3000)) {
+    // -> 19.6, x 32 17.0 -> 16.9, 100,000 x 256, K = 128 15.0 -> 11.4.  Above 128 neighbours its accumulators leave one wavefront per SIMD, and the
+    // line is far up: 8,000 points after one tree, x 400, K = 256 21.33 -> 21.38, x 550, K = 190 14.04 -> 13.99, K = 220 18.1 -> 17.7, x 784, K = 130 8.03 -> 8.08,
+    // K = 160 10.1 -> 9.8, K = 256 28.4 -> 26.1, x 100, K = 256 17.2 -> 18.6; 100,000 x 32, K = 160 18.3 -> 29.7.
+    if (KP > 32 && join_wg_on() && wg_fits && D * (K - 24) > (MW == 2 ? 8000 : MW == 3 ? 6500 : MW == 4 ? 3000 : 95000)) {
         const size_t lds_wg = (size_t)(kJwP + KP) * kJwRowBytes + (size_t)KP * 12 + (size_t)kJwP * 24;
-#define RSFK_JOIN_WG(BV)                                                                                                    \
+#define RSFK_JOIN_WG(BV, NV)                                                                                                    \
         do {                                                                                                               \
-            RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_explore_join_wg<BV>),                             \
+            RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_explore_join_wg<BV, NV>),                         \
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_wg));                       \
-            hipLaunchKernelGGL((k_explore_join_wg<BV>), dim3(grid_for_dies((size_t)N), parts), dim3(256), lds_wg, stream, jc, N, K,  \
+            hipLaunchKernelGGL((k_explore_join_wg<BV, NV>), dim3(grid_for_dies((size_t)N), parts), dim3(256), lds_wg, stream, jc, N, K,  \
                                old_idx, w->bars, w->offs, w->rev, w->pass, w->bounds, KP, join_pitch(D), ksteps, kappa,  \
                                any_rel, any_abs, w->div_m, w->div_s, order);                                                \
         } while (0)
-        if (w->bounds) RSFK_JOIN_WG(true);
-        else RSFK_JOIN_WG(false);
+        if (w->bounds && KP <= 128) RSFK_JOIN_WG(true, 3);
+        else if (w->bounds) RSFK_JOIN_WG(true, 6);
+        else if (KP <= 128) RSFK_JOIN_WG(false, 3);
+        else RSFK_JOIN_WG(false, 6);
 #undef RSFK_JOIN_WG
     } else if (!w->bounds && ksteps <= 8 && short_fits) {
         const dim3 grid(short_groups, parts), block(64 * kWaves);

@@ -649,7 +649,7 @@ def test_explore_points_with_many_marks_are_handed_on(gpu, capi, orc, rng, N, D,
 # both sides of every line between the joins: neighbours in one to seven groups of 32, whole and with one over; dimensions around the
 # largest that stay in registers and around those from which a workgroup takes a point
 @pytest.mark.parametrize("N,D,K", [(900, 128, 33), (900, 129, 33), (700, 64, 64), (700, 200, 64), (600, 201, 64), (500, 500, 40), (500, 501, 40), (700, 32, 65),
-                                   (600, 98, 90), (600, 99, 90), (700, 90, 96), (600, 17, 97), (600, 28, 128), (600, 29, 128), (500, 16, 129), (400, 130, 200)])
+                                   (600, 98, 90), (600, 99, 90), (700, 90, 96), (600, 17, 97), (600, 28, 128), (600, 29, 128), (500, 16, 129), (400, 130, 200), (300, 698, 160), (300, 700, 160), (400, 411, 256)])
 @pytest.mark.parametrize("data", ["normal", "notfinite", "no codes"])
 def test_explore_join_of_rows_of_many_neighbours(gpu, orc, rng, monkeypatch, N, D, K, data):
     """A wavefront per 32 neighbours of a point, a wavefront per point, a workgroup per point, with and without room for the codes == the
