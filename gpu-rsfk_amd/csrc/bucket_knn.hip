@@ -371,23 +371,28 @@ int launch_general(const float* points, int D, int K, const int* ids, const int*
     const int max_tiles = max_bucket > 0 ? (max_bucket + kTile - 1) / kTile : 0;
     const char* env = std::getenv("RSFK_BUCKET_STRIP");        // 0 / 1 overrides the choice (the results are the same)
     const bool strip = max_tiles > 1 && (env && *env ? env[0] == '1' : n_buckets <= kStripBuckets);
-    dim3 grid((unsigned)n_buckets * (unsigned)(strip ? max_tiles : 1)), block(256);
     if (launched) *launched |= strip ? kBucketKernelStrip : kBucketKernelTiled;
+    const int most = strip ? std::max(1, kMostGroups / max_tiles) : n_buckets;      // (as many buckets as a launch has threads for)
+    for (int b0 = 0; b0 < n_buckets; b0 += std::min(most, n_buckets - b0)) {
+        const int* ids_c = starts ? ids : ids + (size_t)b0 * (size_t)stride;
+        const int* starts_c = starts ? starts + b0 : nullptr;
+        const dim3 grid((unsigned)std::min(most, n_buckets - b0) * (unsigned)(strip ? max_tiles : 1)), block(256);
 #define RSFK_GENERAL_CASE(SLV)                                                                                              \
-    do {                                                                                                                    \
-        if (strip)                                                                                                          \
-            hipLaunchKernelGGL((k_bucket_knn<SLV, true>), grid, block, 0, stream, points, D, K, ids, starts, sizes, stride,  \
-                               skip_upto, knn_idx, knn_dist, rs, max_tiles);                                                \
-        else                                                                                                                \
-            hipLaunchKernelGGL((k_bucket_knn<SLV, false>), grid, block, 0, stream, points, D, K, ids, starts, sizes, stride, \
-                               skip_upto, knn_idx, knn_dist, rs, 1);                                                        \
-    } while (0)
-    if (K <= 64) RSFK_GENERAL_CASE(1);
-    else if (K <= 128) RSFK_GENERAL_CASE(2);
-    else if (K <= 256) RSFK_GENERAL_CASE(4);
-    else if (K <= 512) RSFK_GENERAL_CASE(8);
-    else RSFK_GENERAL_CASE(16);
+        do {                                                                                                                \
+            if (strip)                                                                                                      \
+                hipLaunchKernelGGL((k_bucket_knn<SLV, true>), grid, block, 0, stream, points, D, K, ids_c, starts_c, sizes + b0, \
+                                   stride, skip_upto, knn_idx, knn_dist, rs, max_tiles);                                    \
+            else                                                                                                            \
+                hipLaunchKernelGGL((k_bucket_knn<SLV, false>), grid, block, 0, stream, points, D, K, ids_c, starts_c, sizes + b0, \
+                                   stride, skip_upto, knn_idx, knn_dist, rs, 1);                                            \
+        } while (0)
+        if (K <= 64) RSFK_GENERAL_CASE(1);
+        else if (K <= 128) RSFK_GENERAL_CASE(2);
+        else if (K <= 256) RSFK_GENERAL_CASE(4);
+        else if (K <= 512) RSFK_GENERAL_CASE(8);
+        else RSFK_GENERAL_CASE(16);
 #undef RSFK_GENERAL_CASE
+    }
     RSFK_HIP(hipGetLastError());
     return 0;
 }
@@ -495,6 +500,13 @@ int launch_bucket_knn(const float* points, int N, int D, int K, const int* ids, 
     if (n_buckets <= 0) return 0;
     RSFK_CHECK(K >= 1 && K <= kMaxK, "bucket K-NN: K must be in 1..1024");
     RSFK_CHECK(D >= 1, "bucket K-NN: D must be positive");
+    if (n_buckets > kMostGroups) {                            // (as many buckets as a launch has threads for)
+        for (int b0 = 0; b0 < n_buckets; b0 += std::min(kMostGroups, n_buckets - b0))
+            if (launch_bucket_knn(points, N, D, K, starts ? ids : ids + (size_t)b0 * (size_t)stride, starts ? starts + b0 : nullptr, sizes + b0,
+                                  std::min(kMostGroups, n_buckets - b0), stride, max_bucket, knn_idx, knn_dist, stream))
+                return 1;
+        return 0;
+    }
     if (bucket_gram_from() == 0 && K <= kMaxKJoin) {
         // RSFK_GRAM_FROM=0: the screened kernel for every call; it needs sorted rows and the size of the largest bucket
         if (launch_sort_rows(knn_idx, knn_dist, N, K, stream)) return 1;
@@ -562,6 +574,13 @@ int launch_bucket_knn_tree(const float* points, const SmallBucketForm* form,
 {
     RSFK_CHECK(K >= 1 && K <= kMaxK, "bucket K-NN: K must be in 1..1024");
     RSFK_CHECK(D >= 1, "bucket K-NN: D must be positive");
+    if (n_small > kMostGroups && part != 2) {                 // (as many buckets as a launch has threads for)
+        for (int b0 = 0; b0 < n_small; b0 += std::min(kMostGroups, n_small - b0))
+            if (launch_bucket_knn_tree(points, form, rows_sorted, gram, D, K, ids, starts + b0, sizes + b0, leaf_cap,
+                                       std::min(kMostGroups, n_small - b0), 0, max_bucket, knn_idx, knn_dist, stream, 1, trees_before, launched, pairs))
+                return 1;
+        n_small = 0;
+    }
     int none = 0;
     int& used = launched ? *launched : none;              // which kernels this tree's buckets went to (kBucketKernel...)
     if (gram && rows_sorted && K <= kMaxKJoin) {

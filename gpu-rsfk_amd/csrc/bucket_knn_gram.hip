@@ -362,7 +362,7 @@ int launch_bucket_knn_gram(const float* points, int D, int K, const int* ids, co
 {
     if (n_buckets <= 0 || max_size < 2) return 0;
     const int max_tiles = (max_size + kGT - 1) / kGT;
-    RSFK_CHECK((long long)n_buckets * max_tiles < (1ll << 31), "screened bucket kernel: too many workgroups");
+    RSFK_CHECK((long long)n_buckets * max_tiles <= kMostGroups, "screened bucket kernel: too many workgroups");
     RSFK_CHECK(K >= 1 && K <= 256 && D >= 1, "screened bucket kernel: K must be in 1..256 and D positive");
     min_size = std::max(min_size, 2);
     const int d16 = (D + 15) & ~15;

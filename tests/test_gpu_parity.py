@@ -746,6 +746,29 @@ def test_more_rows_than_a_launch_has_wavefronts_for(gpu):
     gpu.lib().rsfk_release_workspace()
 
 
+@pytest.mark.parametrize("padded", [False, True])
+def test_more_buckets_than_a_launch_has_threads_for(gpu, padded):
+    """17 million buckets of two points, by a table of starts and as rows of a padded matrix."""
+    import torch
+    nb, D, K = 17000000, 2, 2
+    N = 2 * nb
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < 20 << 30:
+        pytest.skip("needs 20 GB of device memory")
+    X = torch.randint(0, 256, (N, D), device="cuda", dtype=torch.float32)
+    ids = torch.arange(N, dtype=torch.int32, device="cuda")
+    starts = 2 * torch.arange(nb, dtype=torch.int32, device="cuda")
+    sizes = torch.full((nb,), 2, dtype=torch.int32, device="cuda")
+    idx = torch.full((N, K), -1, dtype=torch.int32, device="cuda")
+    dist = torch.full((N, K), float("inf"), device="cuda")
+    torch.cuda.synchronize()
+    _say("buckets of two", N, padded)
+    gpu.bucket_knn_device(X.data_ptr(), N, D, K, ids.data_ptr(), 0 if padded else starts.data_ptr(), sizes.data_ptr(), nb, 2,
+                          idx.data_ptr(), dist.data_ptr())
+    assert torch.equal(idx[:, 0], ids ^ 1) and bool((idx[:, 1] == -1).all())
+    assert torch.equal(dist[:, 0], ((X - X[(ids ^ 1).long()]) ** 2).sum(1)) and bool(torch.isinf(dist[:, 1]).all())
+
+
 @pytest.mark.parametrize("values", ["far", "tiny", "huge", "outlier", "spread", "notfinite"])
 @pytest.mark.parametrize("N,D,K", [(2500, 16, 8), (2500, 33, 32), (1500, 129, 20), (1500, 40, 70)])
 def test_explore_screens_rows_of_any_magnitude(gpu, orc, rng, N, D, K, values):
