@@ -33,6 +33,18 @@ __global__ __launch_bounds__(256) void k_to_bf16(const float* __restrict__ point
     }
 }
 
+// e1 of a row (bf16.hpp) from the largest error of its coordinates and the sum of their squares.  Both were measured against
+// fl(lo + scale q); the screen evaluates lo sum n + scale sum n q in fp32 and is compared with an fp32 evaluation of n.x: all of that
+// stays below ev = c_d (|lo| + 255 scale) per unit of ||n||_1, so below sqrt(D) ev per unit of ||n||_2 (the factors above one: the
+// rounding of the sums and norms themselves).  Where the squares may underflow, the largest error stands for all of them.
+__device__ __forceinline__ float row_bound(float err, float sq, float lo, float scale, float range, int D, float c_d, bool bad)
+{
+    if (bad || !(range <= 3.0e38f)) return __builtin_nanf("");      // the screen never decides for such a row
+    const float ev = 1.0011f * (c_d * (fabsf(lo) + 255.0f * scale));
+    const float rms = range > 1e-12f ? __builtin_sqrtf(sq / (float)D) + 2e-19f : err;
+    return fmaxf(1.0111f * err + ev, (1.0111f * rms + ev) * (1.0f / kRmsShare)) + kQ8Least;
+}
+
 // one wavefront per row of the 8-bit copy
 __global__ __launch_bounds__(256) void k_to_q8(const float* __restrict__ points, uint8_t* __restrict__ out,
                                                float* __restrict__ rho_parts, int N, int D, int pitch, float c_d, float most)
@@ -63,7 +75,7 @@ __global__ __launch_bounds__(256) void k_to_q8(const float* __restrict__ points,
         const float range = hi - lo;
         const float scale = range * (1.0f / 255.0f);
         const float inv = range > 0.0f ? 255.0f / range : 0.0f;
-        float err = 0.0f;
+        float err = 0.0f, sq = 0.0f;
         // four coordinates per lane and step: one 4-byte store instead of four 1-byte stores
         for (int d0 = 4 * lane; d0 < pitch - 16; d0 += 256) {
             uint32_t packed = 0u;
@@ -75,19 +87,19 @@ __global__ __launch_bounds__(256) void k_to_q8(const float* __restrict__ points,
                     float t = __builtin_rintf((x - lo) * inv);
                     t = fminf(fmaxf(t, 0.0f), 255.0f);
                     packed |= (uint32_t)t << (8 * k);
-                    err = fmaxf(err, fabsf(x - __builtin_fmaf(scale, t, lo)));
+                    const float off = x - __builtin_fmaf(scale, t, lo);
+                    err = fmaxf(err, fabsf(off));
+                    sq = __builtin_fmaf(off, off, sq);
                 }
             }
             *reinterpret_cast<uint32_t*>(dst + 16 + d0) = packed;
         }
 #pragma unroll
-        for (int o = 1; o < 64; o <<= 1) err = fmaxf(err, __shfl_xor(err, o, 64));
-        // err was measured against fl(lo + scale q); the screen evaluates lo sum n + scale sum n q in fp32 and is
-        // compared with an fp32 evaluation of n.x: all of that stays below c_d (|lo| + 255 scale) per unit of ||n||_1
-        // (1.001 for the rounding of ||n||_1 itself)
-        const float mag = fabsf(lo) + 255.0f * scale;
-        float e1 = 1.0111f * err + 1.0011f * (c_d * mag) + kQ8Least;
-        if (bad || !(range <= 3.0e38f)) e1 = __builtin_nanf("");      // the screen never decides for such a row
+        for (int o = 1; o < 64; o <<= 1) {
+            err = fmaxf(err, __shfl_xor(err, o, 64));
+            sq += __shfl_xor(sq, o, 64);
+        }
+        const float e1 = row_bound(err, sq, lo, scale, range, D, c_d, bad);
         if (lane == 0) {
             float* head = reinterpret_cast<float*>(dst);
             head[0] = 0.0f;
@@ -161,7 +173,7 @@ __global__ __launch_bounds__(256) void k_to_q8_regs(const float* __restrict__ po
         const float range = hi - lo;
         const float scale = range * (1.0f / 255.0f);
         const float inv = range > 0.0f ? 255.0f / range : 0.0f;
-        float err = 0.0f;
+        float err = 0.0f, sq = 0.0f;
         uint8_t* dst = out + (size_t)(row_ok ? r : 0) * (size_t)pitch;
 #pragma unroll
         for (int k = 0; k < PPL; ++k) {
@@ -176,17 +188,20 @@ __global__ __launch_bounds__(256) void k_to_q8_regs(const float* __restrict__ po
                         float t = __builtin_rintf((v[c] - lo) * inv);
                         t = fminf(fmaxf(t, 0.0f), 255.0f);
                         packed |= (uint32_t)t << (8 * c);
-                        err = fmaxf(err, fabsf(v[c] - __builtin_fmaf(scale, t, lo)));
+                        const float off = v[c] - __builtin_fmaf(scale, t, lo);
+                        err = fmaxf(err, fabsf(off));
+                        sq = __builtin_fmaf(off, off, sq);
                     }
                 }
                 *reinterpret_cast<uint32_t*>(dst + 16 + 4 * pc) = packed;
             }
         }
 #pragma unroll
-        for (int o = 1; o < LPR; o <<= 1) err = fmaxf(err, __shfl_xor(err, o, 64));
-        const float mag = fabsf(lo) + 255.0f * scale;
-        float e1 = 1.0111f * err + 1.0011f * (c_d * mag) + kQ8Least;
-        if (badi || !(range <= 3.0e38f)) e1 = __builtin_nanf("");      // the screen never decides for such a row
+        for (int o = 1; o < LPR; o <<= 1) {
+            err = fmaxf(err, __shfl_xor(err, o, 64));
+            sq += __shfl_xor(sq, o, 64);
+        }
+        const float e1 = row_bound(err, sq, lo, scale, range, D, c_d, badi != 0);
         if (row_ok && l == 0) {
             *reinterpret_cast<float4*>(dst) = make_float4(0.0f, lo, scale, e1);
             const float bf = sabs / (float)D * (1.0f / 256.0f);

@@ -29,9 +29,13 @@ struct Bf16Copy {
 //
 // Row p, q8_pitch(D) bytes on a 64-byte boundary: a 16-byte header (pad, lo, scale, e1 as four floats), then one
 // byte per coordinate, q_d = round((x_d - lo) / scale) in 0..255 with lo = min_d x_d and scale = (max_d x_d - lo) / 255,
-// zeros up to the end of the row.  e1 bounds what the quantisation can do to a dot product per unit of the
-// 1-norm of the other vector: for any n, |n.x - (lo sum_d n_d + scale sum_d n_d q_d)| <= e1 ||n||_1, including
-// the fp32 evaluation of either side with at most D/8-term chains (see k_to_q8).  mean_rho (host, after
+// zeros up to the end of the row.  e1 bounds what the quantisation can do to a dot product per unit of a
+// length L(n) of the other vector: for any n, |n.x - (lo sum_d n_d + scale sum_d n_d q_d)| <= e1 L(n), including
+// the fp32 evaluation of either side with at most D/8-term chains (see k_to_q8).  L(n) = min(||n||_1, kRmsShare sqrt(D) ||n||_2):
+// the first factor goes with the largest error of a coordinate, the second (Cauchy and Schwarz) with the root of their mean square,
+// which is 1 / sqrt(3) of the largest where coordinates fall anywhere between two steps; e1 is the larger of the largest error and
+// 1 / kRmsShare of that root, so either holds.  For normals whose components spread like those of a uniform or a normal distribution
+// L(n) is 0.71..0.73 ||n||_1 (points left to the exact test: 1M x 100 uniform 3.77 -> 2.74 %, 1M x 256 in clusters 12.3 -> 9.1 %; trees of the former 24.4 -> 23.5 ms for 50, of the latter 29.4 -> 26.4 for 20).  mean_rho (host, after
 // q8_copy_fill has completed) compares e1 with the corresponding quantity of the bfloat16 copy,
 // 2^-8 mean_d |x_d|, averaged over the rows: the 8-bit copy pays off while it is below about 6.
 __host__ __device__ inline int q8_pitch(int D) { return (16 + D + 63) & ~63; }
@@ -54,6 +58,7 @@ struct Q8Copy {
 // bfloat16 copy: sum |n_d||x_d|, which is part of the band, is compared with 1e38 at every point.  (The same for the 8-bit copy, or
 // limits per row and per hyperplane: tail kernel and chains of 20,000 x 64, 50 trees 1.02 -> 1.06 and 1.04 ms.)
 constexpr float kQ8Least = 1e-21f, kNormalLeast = 1e-18f;
+constexpr float kRmsShare = 0.58f;
 inline float q8_most(int D) { return 7.07e18f / __builtin_sqrtf((float)D); }
 
 int q8_copy_alloc(Q8Copy* c, int N, int D);

@@ -103,8 +103,8 @@ __host__ __device__ inline int nvec_len(int D) { return (D + 15) & ~15; }
 
 // Hyperplane of (x1,x2) by one wavefront (all 64 lanes call): normal into LDS nvec[0..nvec_len(D)), and
 // hp[0] = offset (order of create_node.cu:122-135: 32 lane-strided partial sums + xor butterfly),
-// hp[1] = the 1-norm of the normal (kNormalLeast added: bf16.hpp), hp[2] = the sum of its components (any order: only the
-// screens use them, with a margin).  A pair with the same coordinates has the normal 0 and every point on its left (0 < 0):
+// hp[1] = the length L of the normal that the 8-bit rows' bounds are for (kNormalLeast added: bf16.hpp), hp[2] = the sum of its components (any
+// order: only the screens use them, with a margin).  The sum of squares in it is used where the squares neither underflow nor overflow.  A pair with the same coordinates has the normal 0 and every point on its left (0 < 0):
 // its hp[1] is kZeroNormal, which makes the bounds of the screens negative, so that no point is left to the exact test
 // (100,000 x 32, a tenth of the points in groups of 2,000 equal rows, 10 trees: 947 -> 220 ms).
 constexpr float kZeroNormal = -1e30f;
@@ -116,8 +116,8 @@ __device__ __forceinline__ void make_hyperplane_wave(const float* __restrict__ x
     const int hl = lane & 31;
     const bool lowh = lane < 32;
     // Both halves of the wavefront walk the dimensions hl, hl + 32, ... (the loads of eight steps are requested
-    // together): the lower half forms the offset with the arithmetic of create_node.cu:122-135 and writes the normal,
-    // the upper half the 1-norm and the sum of the components.
+    // together): the lower half forms the offset with the arithmetic of create_node.cu:122-135, the normal
+    // and the sum of its squares, the upper half the 1-norm and the sum of the components.
     float s = 0.0f, s2 = 0.0f;
     for (int d0 = hl; d0 < D; d0 += 256) {
         float t1[8], t2[8];
@@ -136,6 +136,7 @@ __device__ __forceinline__ void make_hyperplane_wave(const float* __restrict__ x
                     nvec[d] = nd;
                     const float prod = nd * (t1[k] + t2[k]);
                     s = s + prod * 0.5f;
+                    s2 = __builtin_fmaf(nd, nd, s2);
                 } else {
                     s += fabsf(nd);
                     s2 += nd;
@@ -146,8 +147,13 @@ __device__ __forceinline__ void make_hyperplane_wave(const float* __restrict__ x
     for (int d = D + lane; d < Dn; d += 64) nvec[d] = 0.0f;
     s = half_butterfly_sum(s);
     s2 = half_butterfly_sum(s2);
+    const float sq = read_lane_f(s2, 0);
     if (lane == 0) hp[0] = s;
-    if (lane == 32) { hp[1] = s == 0.0f ? kZeroNormal : s + kNormalLeast; hp[2] = s2; }
+    if (lane == 32) {
+        const float l2 = __builtin_sqrtf(sq * (kRmsShare * kRmsShare * 1.0005f * (float)D));
+        hp[1] = s == 0.0f ? kZeroNormal : (s > 1e-9f ? fminf(s, l2) : s) + kNormalLeast;
+        hp[2] = s2;
+    }
 }
 
 // Screen of the side test for eight points per wavefront (right = n.x < b): lanes 8g..8g+7 work on
@@ -169,7 +175,7 @@ __device__ __forceinline__ void make_hyperplane_wave(const float* __restrict__ x
 // first is needed (the loop over points is bound by the latency of these gathers otherwise).
 //
 // With the 8-bit copy (bf16.hpp) the row is 16 header bytes + one byte per coordinate: approx = lo sum_d n_d +
-// scale sum_d n_d q_d, undecided band e1 ||n||_1 (hp1 = bound of the 1-norm, hp2 = sum of the components of the
+// scale sum_d n_d q_d, undecided band e1 L(n) (hp1 = L(n), hp2 = sum of the components of the
 // normal of the point's node).  Only lane 0 of a group holds the header, so only its right / redo are meaningful
 // (with either copy the callers use lane 0 only).
 // (KU: pieces of a row a lane has in flight, 8-bit copy)
@@ -504,7 +510,7 @@ __global__ __launch_bounds__(256) void k_tree_init(int* __restrict__ perm, NodeQ
 }
 
 // A wide level begins: hyperplanes of its nodes, one wavefront per node -- record ni of the table is
-// [offset, bound of the 1-norm, sum of the components, 0 | normal, nvec_len(D) floats]; the workgroups of a node (one per
+// [offset, L(n) (bf16.hpp), sum of the components, 0 | normal, nvec_len(D) floats]; the workgroups of a node (one per
 // chunk, up to a thousand at the first levels) fetch the record instead of each making the hyperplane again --, the
 // chunks of the nodes, and the level's counts for the host, which has queued this level from bounds on them.
 __global__ __launch_bounds__(256) void k_level_planes(const float* __restrict__ points, TreeParams P,
@@ -558,7 +564,7 @@ __global__ __launch_bounds__(kBlock) void k_side(const float* __restrict__ point
                                                  const float* __restrict__ planes, unsigned long long* __restrict__ stat)
 {
     extern __shared__ __align__(16) float side_lds[];      // record of the node's hyperplane (k_level_planes)
-    float* hp_s = side_lds;                                 // offset, bound of the 1-norm, sum of the components
+    float* hp_s = side_lds;                                 // offset, L(n) (bf16.hpp), sum of the components
     float* nvec = side_lds + 4;                             // nvec_len(D) floats
     __shared__ int left_s, n_def_s;
     __shared__ int deferred[1024];                          // points of the chunk left to the exact test (chunk <= 1024)

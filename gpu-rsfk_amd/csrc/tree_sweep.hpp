@@ -13,7 +13,7 @@
 //     hyperplanes at a time by v_mfma_i32_32x32x32_i8: exact integer sums I1 = sum m1_d (q_d - 128),
 //     I2 = sum m2_d (q_d - 128);
 //   * n.x ~ lo sum n_d + scale s2 (254 I1 + I2 + 128 (254 sum m1 + sum m2)); the row's quantisation error is
-//     bounded by e1 ||n||_1 (header of the 8-bit row, bf16.hpp), the residual by (|lo| + 255 scale) sum |r_d|; a
+//     bounded by e1 L(n) (header of the 8-bit row, bf16.hpp), the residual by (|lo| + 255 scale) sum |r_d|; a
 //     point whose value is farther from the offset than these bounds has the side the exact fp32 test would give
 //     it, the others (one or two per cent) are marked and get the exact test (k_pm_resolve: the arithmetic of
 //     resolve_exact in tree_build.hip);
@@ -42,7 +42,7 @@ constexpr int kMaxGroups = kPaths / kSlots;
 
 // One hyperplane as the sweep needs it.
 struct PlaneQ {
-    float b, hp1, hp2, s2;      // offset, bound of ||n||_1 (or kZeroNormal), sum of the components, scale of the second 8-bit part
+    float b, hp1, hp2, s2;      // offset, L(n) (bf16.hpp; or kZeroNormal), sum of the components, scale of the second 8-bit part
     float c0, rres, pad;        // 128 s2 (254 sum m1 + sum m2), bound of sum |r_d| (and of what 254 s2 != s1 does)
     int ni;                     // node of the level's queue, or -1: the points with this path are not split any more
 };
@@ -77,7 +77,7 @@ __global__ void k_pm_next_map(const int* __restrict__ pmap, int* __restrict__ pm
 }
 
 // 8-bit parts and scalars of the hyperplanes of a level, one wavefront per (tree, path).  planes: records of
-// k_level_planes ([offset, bound of the 1-norm, sum of the components, 0 | normal]), rec floats each.
+// k_level_planes ([offset, L(n) (bf16.hpp), sum of the components, 0 | normal]), rec floats each.
 // Aq: [tree][group] blocks of 32 rows x rowbytes, row j of a block = first part of the group's path j, row 16 + j =
 // second part, stored in the order the sweep's lanes read them: bytes 32 k + 16 h .. + 15 of row r are the 16-byte
 // piece number 64 k + 32 h + r of the block (a wavefront's load of step k is one contiguous kilobyte).
@@ -131,8 +131,8 @@ __global__ __launch_bounds__(256) void k_pm_planes(const float* __restrict__ pla
         q.b = r[0]; q.hp1 = r[1]; q.hp2 = r[2]; q.s2 = s2;
         q.c0 = s2 * (float)(128 * M);                     // |128 M| <= 128 x 127 x 255 D < 2^31 for D <= 256
         // the residuals are known to a relative 2^-7 or so of their size (they are differences of fp32 numbers of
-        // the size of s1); 2^-18 of the 1-norm covers that, the rounding of their sum and of c0, and s1 != 254 s2
-        q.rres = 1.01f * rs + r[1] * (1.0f / 262144.0f);
+        // the size of s1); 2^-18 of the 1-norm (which is at most L(n) / kRmsShare) covers that, the rounding of their sum and of c0, and s1 != 254 s2
+        q.rres = 1.01f * rs + r[1] * (1.0f / (262144.0f * kRmsShare));
         q.pad = 0.0f;
         q.ni = ni;
         *out = q;

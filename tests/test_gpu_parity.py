@@ -138,6 +138,39 @@ def test_tree_of_rows_whose_sums_leave_fp32(gpu, orc, rng, monkeypatch, kind, en
         assert list(gst) == [len(ls), st[0], st[1], st[2]]
 
 
+# The bound of the 8-bit rows goes with the largest error of a coordinate or with the root of their mean square, whichever is smaller: a column that
+# dwarfs the others (1-norm and 2-norm of a normal nearly the same), coordinates that all lie halfway between two steps (every error as large
+# as the largest), all but a few exact, ranges around where squares may underflow, and rows of one value.
+@pytest.mark.parametrize("kind", ["column", "halfway", "few_off", "tiny", "tinier", "one_value"])
+@pytest.mark.parametrize("D", [3, 48, 100, 260])
+@pytest.mark.parametrize("env", [dict(PM="7"), dict(PM="0", TAIL="256")], ids=lambda e: "-".join(e.values()))
+def test_tree_bounds_by_largest_and_mean_error(gpu, orc, rng, monkeypatch, kind, D, env):
+    monkeypatch.setenv("RSFK_TREE_SCREEN", "q8")
+    monkeypatch.setenv("RSFK_PM_LEVELS", env["PM"])
+    if "TAIL" in env:
+        monkeypatch.setenv("RSFK_TAIL_BLOCK", env["TAIL"])
+    N, MIN, MAX = 6000, 17, 34
+    X = rng.standard_normal((N, D))
+    if kind == "column":
+        X[:, 0] *= 1000.0
+    if kind == "halfway":                                       # 0, 255 and values k + 1/2 of a scale that is 1
+        X = rng.integers(0, 255, (N, D)) + 0.5
+        X[:, 0], X[:, 1] = 0.0, 255.0
+    if kind == "few_off":
+        X = rng.integers(0, 256, (N, D)) + np.where(rng.random((N, D)) < 0.02, 0.49, 0.0)
+        X[:, 0], X[:, 1] = 0.0, 255.0
+    if kind in ("tiny", "tinier"):
+        X *= 1e-12 if kind == "tiny" else 1e-18
+    if kind == "one_value":
+        X[: N // 2] = rng.standard_normal((N // 2, 1))
+    X = X.astype(np.float32)
+    _say("tree bounds", kind, D, env)
+    perm, ls, lz, st = orc.build_tree(X, MIN, MAX, 300, 1)
+    gperm, gls, glz, gst = gpu.build_tree(X, MIN, MAX, 300, 1)
+    assert np.array_equal(gperm, perm)
+    assert np.array_equal(gls, ls) and np.array_equal(glz, lz)
+
+
 # The forms of the tail and of the chain phase: leaf limits on either side of the sizes of the chain's matrix (nodes of up to 64, 128
 # and 256 points, and none), rows on either side of the lanes that share one, many subtrees (nodes above `small` points are wide) and
 # few; rows without distances (NaN, and a few far longer than the others), clusters within one node, the index that query points
