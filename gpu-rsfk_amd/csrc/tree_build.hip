@@ -339,6 +339,7 @@ __device__ __forceinline__ void resolve_exact(int halves, int h, const Entry* li
     }
 }
 
+constexpr int kWideChunk = 1024;     // points per workgroup in the wide passes (the side tests keep a chunk's undecided points in LDS)
 constexpr int kSideBatch = 4;        // points per group and call of the screen in the wide phase
 
 // The queues nodes go to: the next wide level (entry `slot` of the counters) and the tail kernel (one workgroup per node).
@@ -509,6 +510,9 @@ __global__ __launch_bounds__(256) void k_tree_init(int* __restrict__ perm, NodeQ
     if (pmap) pmap[t * pm::kPaths] = at[0];      // path 0 of level 0 = the root, if it is split at all
 }
 
+// bytes of a node's record for k_side_q8: [scale of the second part, 128 x it x (254 sum m1 + sum m2), bound of the residuals, 0 | first part | second part]
+__host__ __device__ inline size_t side_op_bytes(int D) { return 16 + 2 * (size_t)q8_pitch(D); }
+
 // A wide level begins: hyperplanes of its nodes, one wavefront per node -- record ni of the table is
 // [offset, L(n) (bf16.hpp), sum of the components, 0 | normal, nvec_len(D) floats]; the workgroups of a node (one per
 // chunk, up to a thousand at the first levels) fetch the record instead of each making the hyperplane again --, the
@@ -516,8 +520,8 @@ __global__ __launch_bounds__(256) void k_tree_init(int* __restrict__ perm, NodeQ
 __global__ __launch_bounds__(256) void k_level_planes(const float* __restrict__ points, TreeParams P,
                                                       const int* __restrict__ perm0, const int* __restrict__ perm1,
                                                       const TreeNode* __restrict__ nodes, int level, int node_cap,
-                                                      float* __restrict__ table, int* __restrict__ chunk2node, LevelCounters* ctr,
-                                                      unsigned long long* __restrict__ stat, LevelNote* note, int seq)
+                                                      float* __restrict__ table, uint8_t* __restrict__ ops, int* __restrict__ chunk2node,
+                                                      LevelCounters* ctr, unsigned long long* __restrict__ stat, LevelNote* note, int seq)
 {
     extern __shared__ __align__(16) float lds_p[];          // per wavefront: 4 + nvec_len(D) floats
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -550,13 +554,41 @@ __global__ __launch_bounds__(256) void k_level_planes(const float* __restrict__ 
     wave_lds_sync();
     float* out = table + (size_t)ni * rec;
     for (int i = lane; i < rec; i += 64) out[i] = mine[i];
+    if (!ops) return;
+    // operand rows of k_side_q8: the two 8-bit parts of the normal, byte for byte below a row of the 8-bit copy (zeros below its header)
+    float most = 0.0f;
+    for (int d = lane; d < P.D; d += 64) most = fmaxf(most, fabsf(mine[4 + d]));
+    const pm::NormalParts parts(wave_max(most));
+    const int pitch = q8_pitch(P.D);
+    uint8_t* op = ops + (size_t)ni * side_op_bytes(P.D);
+    float rs = 0.0f;
+    int M = 0;
+    for (int at = 4 * lane; at < pitch; at += 256) {
+        uint32_t w1 = 0u, w2 = 0u;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int d = at + k - 16;
+            if (d >= 0 && d < P.D) {
+                int i1, i2;
+                rs += parts.split(mine[4 + d], i1, i2);
+                M += 254 * i1 + i2;
+                w1 |= (uint32_t)(i1 & 0xff) << (8 * k);
+                w2 |= (uint32_t)(i2 & 0xff) << (8 * k);
+            }
+        }
+        *reinterpret_cast<uint32_t*>(op + 16 + at) = w1;
+        *reinterpret_cast<uint32_t*>(op + 16 + pitch + at) = w2;
+    }
+    rs = pm::wave_sum_f(rs);
+    M = wave_sum_i(M);
+    if (lane == 0)
+        *reinterpret_cast<float4*>(op) = make_float4(parts.s2, parts.s2 * (128.0f * (float)M), pm::NormalParts::residual(rs, mine[1]), 0.0f);
 }
 
 // Side test of one chunk of one node: sets bit 31 of the permutation entry of
-// every member on the right side and counts the members on the left.
-template <bool Q8, int LPP>
-__global__ __launch_bounds__(kBlock) void k_side(const float* __restrict__ points,
-                                                 const uint16_t* __restrict__ pb16, const uint8_t* __restrict__ q8,
+// every member on the right side and counts the members on the left.  (By the bfloat16 copy, or by the fp32 rows alone; with the 8-bit copy
+// k_side_q8 takes its place.)
+__global__ __launch_bounds__(kBlock) void k_side(const float* __restrict__ points, const uint16_t* __restrict__ pb16,
                                                  TreeParams P,
                                                  int* __restrict__ perm0, int* __restrict__ perm1,
                                                  const TreeNode* __restrict__ nodes, int slot, LevelCounters* ctr,
@@ -585,8 +617,8 @@ __global__ __launch_bounds__(kBlock) void k_side(const float* __restrict__ point
     const float b = hp_s[0], n1 = hp_s[1], sn = hp_s[2];
     const int pos0 = nd.start + k * P.chunk;
     const int pos1 = min(nd.start + nd.count, pos0 + P.chunk);
-    constexpr int kGroupsL = kBlock / LPP;                           // groups of LPP lanes, one point each
-    const int grp = threadIdx.x / LPP, sub8 = threadIdx.x & (LPP - 1);
+    constexpr int kGroupsL = kBlock / 8;                             // groups of eight lanes, one point each
+    const int grp = threadIdx.x >> 3, sub8 = threadIdx.x & 7;
     const int iters = (pos1 - pos0 + kGroupsL - 1) / kGroupsL;
     int lefts = 0;
     for (int it = 0; it < iters; it += kSideBatch) {
@@ -603,7 +635,7 @@ __global__ __launch_bounds__(kBlock) void k_side(const float* __restrict__ point
             h1[u] = n1;
             h2[u] = sn;
         }
-        side_screen8<kSideBatch, Q8, LPP>(nvec, 0, jz, bb, h1, h2, pb16, q8, id, P.D, P.band, valid, right, redo);
+        side_screen8<kSideBatch, false>(nvec, 0, jz, bb, h1, h2, pb16, nullptr, id, P.D, P.band, valid, right, redo);
 #pragma unroll
         for (int u = 0; u < kSideBatch; ++u) {
             if (valid[u] && sub8 == 0) {
@@ -629,6 +661,133 @@ __global__ __launch_bounds__(kBlock) void k_side(const float* __restrict__ point
     if (threadIdx.x == 0) {
         chunk_left[c] = left_s;
         stat_add(stat, c, 1, n_def_s);
+    }
+}
+
+// The same by the 8-bit copy.  What bounds it is the rows, a cache line or more each from anywhere in the copy: the device delivers 55 to 59 G
+// lines a second, 6.3 TB/s of rows of several lines.  So that nothing else does, a wavefront has 64 rows on their way at a time, their places are
+// known before the first is asked for, no line of a short row is asked for twice (a load takes lines, and the headers come with them), and the products come from
+// the matrix cores: all points of a chunk meet the same hyperplane, whose two 8-bit parts (pm::NormalParts) are rows of one operand; the bytes of the
+// points' rows as they lie in memory, header and all, above zeros of the normal, are columns of the other.
+//   LINE false, rows of 64 bytes: a load is 16 rows, lane (row % 16, piece / 16) has a piece of 16 bytes.  Even and odd rows of the first operand repeat
+//   the two parts, so every lane holds both sums of row lane % 16 of each of four tiles.
+//   LINE true, longer rows: a load is 128 bytes of 8 rows, so columns 0..7 of the operand are the even pieces of the eight rows and 8..15 the odd ones; rows 4 i,
+//   4 i + 1 of the first operand are the parts below even pieces, 4 i + 2, 4 i + 3 those below odd ones, and a row's sums are added up over lanes c and c + 8.
+// Either way lane l then decides point l of the 64.  A level of 1M x 100, 50 trees: 1.49 -> 0.99 ms, of 10M x 32, 10 trees: 2.53 -> 2.15, of 1M x 256, 20 trees:
+// 1.52 -> 1.31 (a few per cent of it by the tighter bound of bf16.hpp), against eight (or two) lanes per point that multiply byte by byte, two vector instructions
+// each, and ask for a point's place, its row and its header in turn.  Headers by loads of their own: 1.11, 2.38; rows on multiples of 128 bytes: 1.35 for 256 dimensions.
+template <bool LINE>
+__global__ __launch_bounds__(kBlock) void k_side_q8(const float* __restrict__ points, const uint8_t* __restrict__ q8, TreeParams P,
+                                                    int* __restrict__ perm0, int* __restrict__ perm1,
+                                                    const TreeNode* __restrict__ nodes, int slot, LevelCounters* ctr,
+                                                    const int* __restrict__ chunk2node, int* __restrict__ chunk_left,
+                                                    const float* __restrict__ planes, const uint8_t* __restrict__ ops,
+                                                    unsigned long long* __restrict__ stat)
+{
+    extern __shared__ __align__(16) float side_lds[];      // record of the node's hyperplane (k_level_planes)
+    constexpr int kRounds = kWideChunk / kBlock;
+    constexpr int kTiles = LINE ? 8 : 4, kRows = 64 / kTiles;       // of the 64 points of a wavefront; lanes of a row
+    __shared__ float4 head_s[kBlock / 64][64];
+    __shared__ int ids[kWideChunk];                         // members of the chunk, bit 31 as it will be stored
+    __shared__ uint16_t undecided[kWideChunk];
+    __shared__ int left_s, n_und_s;
+    const int c = blockIdx.x;
+    if (c >= ctr->queue[slot].chunks) return;
+    if (c == 0 && threadIdx.x == 0) phase_tick(ctr, 0);
+    const int ni = chunk2node[c];
+    const TreeNode nd = nodes[ni];
+    const int tid = threadIdx.x, lane = tid & 63, row = lane % kRows, piece = lane / kRows;
+    int* perm = (nd.buf ? perm1 : perm0) + (size_t)nd.tree * (size_t)P.N;
+    const int pos0 = nd.start + (c - nd.chunk0) * kWideChunk;
+    const int n = min(nd.start + nd.count - pos0, kWideChunk);
+    int id[kRounds];
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) id[r] = r * kBlock + tid < n ? (perm[pos0 + r * kBlock + tid] & kIdMask) : 0;
+    const float* rec = planes + (size_t)ni * (size_t)(4 + nvec_len(P.D));
+    for (int i = tid; i < (4 + nvec_len(P.D)) >> 2; i += kBlock)
+        reinterpret_cast<float4*>(side_lds)[i] = reinterpret_cast<const float4*>(rec)[i];
+    if (tid == 0) { left_s = 0; n_und_s = 0; }
+    const float b = rec[0], length = rec[1], sum = rec[2];
+    const size_t pitch = (size_t)q8_pitch(P.D);
+    const uint8_t* op = ops + (size_t)ni * side_op_bytes(P.D);
+    const float4 scales = *reinterpret_cast<const float4*>(op);
+    const int below_at = 16 * (LINE ? 2 * (lane >> 4) + ((lane >> 1) & 1) : lane >> 4);
+    const uint8_t* part = op + 16 + (lane & 1) * pitch + below_at;
+    const int steps = LINE ? (int)((pitch + 127) >> 7) : 1;
+    float4* heads = head_s[tid >> 6];
+    pm::v4i normal = *reinterpret_cast<const pm::v4i*>(part);       // of the first step, which is the only one of most rows
+    __syncthreads();
+    int lefts = 0;
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) {
+        if (r * kBlock + (tid & ~63) >= n) break;
+        const uint8_t* src[kTiles];
+        pm::v4i acc[kTiles], w[kTiles];
+#pragma unroll
+        for (int t = 0; t < kTiles; ++t) {
+            src[t] = q8 + (size_t)__shfl(id[r], kRows * t + row, 64) * pitch + 16 * piece;
+            w[t] = *reinterpret_cast<const pm::v4i*>(src[t]);
+            acc[t] = pm::v4i{0, 0, 0, 0};
+        }
+        if (piece == 0) {
+#pragma unroll
+            for (int t = 0; t < kTiles; ++t) *reinterpret_cast<pm::v4i*>(&heads[kRows * t + row]) = w[t];
+        }
+        pm::v4i below = normal;
+        for (int k = 1;; ++k) {
+#pragma unroll
+            for (int t = 0; t < kTiles; ++t)
+                acc[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(below, w[t] ^ (int)0x80808080, acc[t], 0, 0, 0);
+            if (!LINE || k >= steps) break;
+            below = pm::v4i{0, 0, 0, 0};
+            if (128 * k + below_at < (int)pitch) below = *reinterpret_cast<const pm::v4i*>(part + 128 * k);
+#pragma unroll
+            for (int t = 0; t < kTiles; ++t)
+                if (128 * k + 16 * piece < (int)pitch) w[t] = *reinterpret_cast<const pm::v4i*>(src[t] + 128 * k);
+        }
+        int i1 = 0, i2 = 0;
+#pragma unroll
+        for (int t = 0; t < kTiles; ++t) {
+            int s1 = acc[t][0], s2 = acc[t][1];
+            if (LINE) {
+                s1 = lane & 8 ? acc[t][2] : s1;
+                s2 = lane & 8 ? acc[t][3] : s2;
+                s1 += dpp_i<kDppRor8>(s1);
+                s2 += dpp_i<kDppRor8>(s2);
+            }
+            i1 = piece == t ? s1 : i1;
+            i2 = piece == t ? s2 : i2;
+        }
+        wave_lds_sync();
+        const float4 head = heads[lane];
+        const float lo = head.y, scale = head.z, e1 = head.w;
+        const float product = __builtin_fmaf(scales.x, __builtin_fmaf(254.0f, (float)i1, (float)i2), scales.y);
+        const float approx = __builtin_fmaf(scale, product, lo * sum);
+        const float band = __builtin_fmaf(e1, length, (fabsf(lo) + 255.0f * scale) * scales.z);
+        const bool valid = r * kBlock + tid < n;
+        const bool certain = fabsf(approx - b) > band;                     // false if anything is NaN
+        const bool right = certain && approx < b;
+        ids[r * kBlock + tid] = right ? id[r] | (int)0x80000000 : id[r];
+        lefts += valid && certain && !right ? 1 : 0;
+        if (valid && !certain) undecided[atomicAdd(&n_und_s, 1)] = (uint16_t)(r * kBlock + tid);
+        wave_lds_sync();
+    }
+    __syncthreads();
+    resolve_exact(kBlock >> 5, tid >> 5, undecided, n_und_s, side_lds + 4, 0, side_lds, points, P.D,
+                  [&](int local) { return ids[local] & kIdMask; },
+                  [&](int local, bool right) {
+                      if (right) ids[local] |= (int)0x80000000;            // build_tree_check_points_side.cu:149
+                      lefts += right ? 0 : 1;
+                  });
+    lefts = wave_sum_i(lefts);
+    if (lane == 0 && lefts) atomicAdd(&left_s, lefts);
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r)
+        if (r * kBlock + tid < n) perm[pos0 + r * kBlock + tid] = ids[r * kBlock + tid];
+    if (tid == 0) {
+        chunk_left[c] = left_s;
+        stat_add(stat, c, 1, n_und_s);
     }
 }
 
@@ -2214,6 +2373,7 @@ struct TreeBatchWorkspace {
     int* chunk2node = nullptr;
     int* chunk_left = nullptr;
     float* planes = nullptr;             // hyperplanes of the nodes of the current wide level: node_cap x (4 + nvec_len(D))
+    uint8_t* side_ops = nullptr;         // ... and their records for the side tests by the 8-bit copy
     int* leaf_start = nullptr;
     int* leaf_size = nullptr;
     TreeStats* stats = nullptr;
@@ -2243,7 +2403,7 @@ struct TreeBatchWorkspace {
 static void free_ws(TreeBatchWorkspace& w)
 {
     void* dev[] = {w.perm[0], w.perm[1], w.nodes[0], w.nodes[1], w.tail, w.chain, w.mid, w.chunk2node,
-                   w.chunk_left, w.leaf_start, w.leaf_size, w.stats, w.ctr, w.recs, w.planes,
+                   w.chunk_left, w.leaf_start, w.leaf_size, w.stats, w.ctr, w.recs, w.planes, w.side_ops,
                    w.pm_path, w.pm_side, w.pm_undec, w.pm_map[0], w.pm_map[1], w.pm_sc, w.pm_aq, w.pm_child, w.stat};
     for (void* p : dev) ws_free(p);
     pin_free(w.notes.block());
@@ -2306,13 +2466,12 @@ int tree_mid_most(int D, int N, int B, int small)
     }
     return n >= least && N > small ? n : 0;
 }
-constexpr int kWideChunk = 1024;         // points per workgroup in the wide passes (k_side keeps a chunk's undecided points in LDS)
 
 // bytes of device memory a batch of B trees needs
 size_t tree_ws_bytes(int N, int D, int MIN, int B)
 {
     const size_t lc = (size_t)N / (size_t)std::max(MIN, 1) + 2;
-    return bf16_copy_bytes(N, D) + (size_t)B * ((size_t)N * 8 + (size_t)N * 2 + 512 * 1024 + lc * (8 + 3 * sizeof(TreeNode)) + ((size_t)N / 1024 + 2) * (2 * sizeof(TreeNode) + 24 + (size_t)(4 + nvec_len(D)) * 4));
+    return bf16_copy_bytes(N, D) + (size_t)B * ((size_t)N * 8 + (size_t)N * 2 + 512 * 1024 + lc * (8 + 3 * sizeof(TreeNode)) + ((size_t)N / 1024 + 2) * (2 * sizeof(TreeNode) + 24 + (size_t)(4 + nvec_len(D)) * 4 + side_op_bytes(D)));
 }
 
 // From now on every build with this workspace also writes the index of each tree (TreeRec records).
@@ -2352,6 +2511,7 @@ int tree_ws_alloc(TreeBatchWorkspace** out, int N, int D, int MIN, int B)
     if (dmalloc(&w->chunk2node, (size_t)w->chunk_cap)) return 1;
     if (dmalloc(&w->chunk_left, (size_t)w->chunk_cap)) return 1;
     if (dmalloc(&w->planes, (size_t)w->node_cap * (size_t)(4 + nvec_len(D)))) return 1;
+    if (dmalloc(&w->side_ops, (size_t)w->node_cap * side_op_bytes(D))) return 1;
     if (dmalloc(&w->leaf_start, (size_t)B * w->leaf_cap)) return 1;
     if (dmalloc(&w->leaf_size, (size_t)B * w->leaf_cap)) return 1;
     if (dmalloc(&w->stats, (size_t)B)) return 1;
@@ -2447,13 +2607,8 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
     if (side_lds > 48 * 1024) {
         RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_level_planes), hipFuncAttributeMaxDynamicSharedMemorySize,
                                      (int)side_lds));
-        if (q8) {
-            RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_side<true, 8>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                         (int)side_lds));
-        } else {
-            RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_side<false, 8>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                         (int)side_lds));
-        }
+        RSFK_HIP(hipFuncSetAttribute(q8 ? reinterpret_cast<const void*>(k_side_q8<true>) : reinterpret_cast<const void*>(k_side),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)side_lds));
     }
     for (float& v : w->phase_s) v = 0.0f;
     // Wide levels.  A level is three launches over bounds on its counts, which follow from the counts of the level before:
@@ -2479,10 +2634,11 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
         const int slot = level & 3;
         const int n_chunks = (int)std::min<size_t>(most_chunks, (size_t)w->chunk_cap);
         int* ctr_chunks = &w->ctr->queue[slot].chunks;
+        const bool swept = level < pm_levels;
         hipLaunchKernelGGL(k_level_planes, dim3((unsigned)((most_nodes + plane_waves - 1) / plane_waves)), dim3(64 * plane_waves),
                            plane_waves * side_lds, stream, points, PW, w->perm[0], w->perm[1], w->nodes[cur], level, w->node_cap,
-                           w->planes, w->chunk2node, w->ctr, w->stat, w->notes.of(level), LevelNotes::seq(level));
-        const bool swept = level < pm_levels;
+                           w->planes, q8 && !swept ? w->side_ops : nullptr, w->chunk2node, w->ctr, w->stat, w->notes.of(level),
+                           LevelNotes::seq(level));
         if (swept) {
             // the sides of every point in all trees of the batch, then their marks in the permutations
             const int n_paths = 1 << level, ks = w->pm_ks, W = w->pm_W;
@@ -2504,15 +2660,14 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
             hipLaunchKernelGGL(k_pm_mark, dim3(n_chunks), dim3(kBlock), 0, stream, P, w->perm[0], w->perm[1], w->nodes[cur],
                                ctr_chunks, w->chunk2node, w->chunk_left, w->pm_side, W);
         } else {
-        // lanes per point in the 8-bit screen: a lane takes 16 coordinates per step
-        const int q8_pieces = q8_padded(D) >> 4;
-#define RSFK_SIDE_LAUNCH(Q, L)                                                                                              \
-        hipLaunchKernelGGL((k_side<Q, L>), dim3(n_chunks), dim3(kBlock), side_lds, stream, points, pb16, q8, P, w->perm[0],    \
-                           w->perm[1], w->nodes[cur], slot, w->ctr, w->chunk2node, w->chunk_left, w->planes, w->stat)
-        if (!q8) RSFK_SIDE_LAUNCH(false, 8);
-        else if (q8_pieces <= 2) RSFK_SIDE_LAUNCH(true, 2);
-        else if (q8_pieces <= 4) RSFK_SIDE_LAUNCH(true, 4);
-        else RSFK_SIDE_LAUNCH(true, 8);
+#define RSFK_SIDE_LAUNCH(LINE)                                                                                                 \
+            hipLaunchKernelGGL(k_side_q8<LINE>, dim3(n_chunks), dim3(kBlock), side_lds, stream, points, q8, P, w->perm[0], w->perm[1], \
+                               w->nodes[cur], slot, w->ctr, w->chunk2node, w->chunk_left, w->planes, w->side_ops, w->stat)
+            if (!q8)
+                hipLaunchKernelGGL(k_side, dim3(n_chunks), dim3(kBlock), side_lds, stream, points, pb16, P, w->perm[0], w->perm[1],
+                                   w->nodes[cur], slot, w->ctr, w->chunk2node, w->chunk_left, w->planes, w->stat);
+            else if (q8_pitch(D) == 64) RSFK_SIDE_LAUNCH(false);
+            else RSFK_SIDE_LAUNCH(true);
 #undef RSFK_SIDE_LAUNCH
         }
         const bool map_next = level + 1 < pm_levels;

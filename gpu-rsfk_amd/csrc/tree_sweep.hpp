@@ -76,14 +76,39 @@ __global__ void k_pm_next_map(const int* __restrict__ pmap, int* __restrict__ pm
     pmap_next[t * kPaths + 2 * v + 1] = c.y;
 }
 
+// A normal in two signed 8-bit parts.  With s2 about max|n| / (127 x 254) and s1 = fl(254 s2): m1 = round(n / s1), m2 =
+// round((n - s1 m1) / s2), both clamped to +-127, r = n - s1 m1 - s2 m2 as computed.  The products are evaluated as s2 (254 I1 + I2),
+// which takes 254 s2 for s1: that is off by a relative 2^-24, far below the 2^-18 ||n||_1 added to the bound of the residuals.
+struct NormalParts {
+    float s1, s2, inv1, inv2;
+    __device__ __forceinline__ explicit NormalParts(float most)          // of the normal's components, by absolute value
+    {
+        s2 = most * (1.000001f / 32258.0f);
+        s1 = 254.0f * s2;
+        inv1 = s1 > 1e-30f ? 1.0f / s1 : 0.0f;
+        inv2 = s2 > 1e-30f ? 1.0f / s2 : 0.0f;
+    }
+    // the parts of a component; returns |r| (NaN, of a normal with NaN or infinite components, stays NaN)
+    __device__ __forceinline__ float split(float n, int& i1, int& i2) const
+    {
+        const float m1 = fminf(fmaxf(__builtin_rintf(n * inv1), -127.0f), 127.0f);
+        const float e = __builtin_fmaf(-s1, m1, n);
+        const float m2 = fminf(fmaxf(__builtin_rintf(e * inv2), -127.0f), 127.0f);
+        i1 = (int)m1;
+        i2 = (int)m2;
+        return fabsf(__builtin_fmaf(-s2, m2, e));
+    }
+    // bound of the residuals of a dot product per unit of a row's magnitude (|lo| + 255 scale): their sum rs is known to a relative 2^-7 or
+    // so (they are differences of fp32 numbers of the size of s1); 2^-18 of the 1-norm, which is at most L(n) / kRmsShare, covers that, the rounding of
+    // their sum and of the products, and s1 != 254 s2
+    __device__ static __forceinline__ float residual(float rs, float length) { return 1.01f * rs + length * (1.0f / (262144.0f * kRmsShare)); }
+};
+
 // 8-bit parts and scalars of the hyperplanes of a level, one wavefront per (tree, path).  planes: records of
 // k_level_planes ([offset, L(n) (bf16.hpp), sum of the components, 0 | normal]), rec floats each.
 // Aq: [tree][group] blocks of 32 rows x rowbytes, row j of a block = first part of the group's path j, row 16 + j =
 // second part, stored in the order the sweep's lanes read them: bytes 32 k + 16 h .. + 15 of row r are the 16-byte
 // piece number 64 k + 32 h + r of the block (a wavefront's load of step k is one contiguous kilobyte).
-// With s2 about max|n| / (127 x 254) and s1 = fl(254 s2): m1 = round(n / s1), m2 = round((n - s1 m1) / s2), both
-// clamped to +-127, r = n - s1 m1 - s2 m2 as computed.  The sweep evaluates s2 (254 I1 + I2), i.e. it takes
-// 254 s2 for s1: that is off by a relative 2^-24, far below the 2^-18 ||n||_1 added to the bound of the residuals.
 __global__ __launch_bounds__(256) void k_pm_planes(const float* __restrict__ planes, int rec, int D, int rowbytes,
                                                    const int* __restrict__ pmap, int n_paths, int nb,
                                                    PlaneQ* __restrict__ sc, int8_t* __restrict__ Aq)
@@ -103,22 +128,15 @@ __global__ __launch_bounds__(256) void k_pm_planes(const float* __restrict__ pla
     float mx = 0.0f;
     for (int d = lane; d < D; d += 64) mx = fmaxf(mx, fabsf(nvec[d]));
     mx = wave_max(mx);
-    const float s2 = mx * (1.000001f / 32258.0f);
-    const float s1 = 254.0f * s2;
-    const float inv1 = s1 > 1e-30f ? 1.0f / s1 : 0.0f;
-    const float inv2 = s2 > 1e-30f ? 1.0f / s2 : 0.0f;
+    const NormalParts parts(mx);
     int8_t* block = Aq + (size_t)(t * kMaxGroups + v / kSlots) * 32 * rowbytes;
     const int r1 = v % kSlots, r2 = r1 + kSlots;
     float rs = 0.0f;
     int M = 0;
     for (int d = lane; d < rowbytes; d += 64) {
         const float n = d < D ? nvec[d] : 0.0f;
-        const float m1 = fminf(fmaxf(__builtin_rintf(n * inv1), -127.0f), 127.0f);
-        const float e = __builtin_fmaf(-s1, m1, n);
-        const float m2 = fminf(fmaxf(__builtin_rintf(e * inv2), -127.0f), 127.0f);
-        const float rr = __builtin_fmaf(-s2, m2, e);
-        rs += fabsf(rr);                                  // NaN (a normal with NaN or infinite components) stays NaN
-        const int i1 = (int)m1, i2 = (int)m2;
+        int i1, i2;
+        rs += parts.split(n, i1, i2);
         M += 254 * i1 + i2;
         const int piece = 64 * (d >> 5) + 32 * ((d >> 4) & 1);
         block[(piece + r1) * 16 + (d & 15)] = (int8_t)i1;
@@ -128,11 +146,9 @@ __global__ __launch_bounds__(256) void k_pm_planes(const float* __restrict__ pla
     M = wave_sum_i(M);
     if (lane == 0) {
         PlaneQ q;
-        q.b = r[0]; q.hp1 = r[1]; q.hp2 = r[2]; q.s2 = s2;
-        q.c0 = s2 * (float)(128 * M);                     // |128 M| <= 128 x 127 x 255 D < 2^31 for D <= 256
-        // the residuals are known to a relative 2^-7 or so of their size (they are differences of fp32 numbers of
-        // the size of s1); 2^-18 of the 1-norm (which is at most L(n) / kRmsShare) covers that, the rounding of their sum and of c0, and s1 != 254 s2
-        q.rres = 1.01f * rs + r[1] * (1.0f / (262144.0f * kRmsShare));
+        q.b = r[0]; q.hp1 = r[1]; q.hp2 = r[2]; q.s2 = parts.s2;
+        q.c0 = parts.s2 * (float)(128 * M);                     // |128 M| <= 128 x 127 x 255 D < 2^31 for D <= 256
+        q.rres = NormalParts::residual(rs, r[1]);
         q.pad = 0.0f;
         q.ni = ni;
         *out = q;

@@ -37,6 +37,7 @@ __device__ __forceinline__ int read_lane_i(int v, int lane) { return __builtin_a
 constexpr int kDppXor1 = 0xB1;          // quad_perm:[1,0,3,2]
 constexpr int kDppXor2 = 0x4E;          // quad_perm:[2,3,0,1]
 constexpr int kDppHalfMirror = 0x141;   // lane i <-> 7-i inside each group of 8
+constexpr int kDppRor8 = 0x128;         // lane i <- i^8 inside each row of 16
 constexpr int kDppMirror = 0x140;       // lane i <-> 15-i inside each row of 16
 
 template <int CTRL>

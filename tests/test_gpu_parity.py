@@ -171,6 +171,29 @@ def test_tree_bounds_by_largest_and_mean_error(gpu, orc, rng, monkeypatch, kind,
     assert np.array_equal(gls, ls) and np.array_equal(glz, lz)
 
 
+# Side tests of the wide levels by the 8-bit copy: rows of 64 bytes and of one line to several, whole or ending in half a line; chunks of any size; rows of NaN,
+# equal rows, and a common offset that leaves every point to the exact test.
+@pytest.mark.parametrize("D", [1, 47, 48, 49, 111, 112, 113, 176, 240, 241, 305, 1100])
+@pytest.mark.parametrize("kind", ["n", "nan", "dup", "offset"])
+def test_tree_wide_levels_by_the_8_bit_copy(gpu, orc, rng, monkeypatch, D, kind):
+    for name, v in (("SCREEN", "q8"), ("MID", "0"), ("SMALL", "64")):
+        monkeypatch.setenv("RSFK_TREE_" + name, v)
+    monkeypatch.setenv("RSFK_PM_LEVELS", "0")
+    N, MIN, MAX = 5000 if D < 300 else 2500, 17, 34
+    X = rng.standard_normal((N, D)).astype(np.float32)
+    if kind == "nan":
+        X[rng.random(N) < 0.02, D // 2] = np.nan
+    if kind == "dup":
+        X[: N // 3] = X[0]
+    if kind == "offset":
+        X = (X * 1e-3 + 1000.0).astype(np.float32)
+    _say("tree wide levels", D, kind)
+    perm, ls, lz, st = orc.build_tree(X, MIN, MAX, 100, 5)
+    gperm, gls, glz, gst = gpu.build_tree(X, MIN, MAX, 100, 5)
+    assert np.array_equal(gperm, perm)
+    assert np.array_equal(gls, ls) and np.array_equal(glz, lz)
+
+
 # The forms of the tail and of the chain phase: leaf limits on either side of the sizes of the chain's matrix (nodes of up to 64, 128
 # and 256 points, and none), rows on either side of the lanes that share one, many subtrees (nodes above `small` points are wide) and
 # few; rows without distances (NaN, and a few far longer than the others), clusters within one node, the index that query points
