@@ -2571,11 +2571,14 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
     RSFK_CHECK(nb <= 64, "tree batch: at most 64 trees at a time");
     // Levels whose side tests are taken point by point (needs the 8-bit copy).  RSFK_PM_LEVELS overrides (0 = none).
     // The sweep multiplies every tile of points with every block of 16 hyperplanes of a tree, so its cost doubles
-    // per level from the fifth on; measured, the seventh level is the last one it takes faster than k_side.  Batches of
-    // less than 2^22 points do not fill the device either way, and k_side is one launch instead of four.
+    // per level from the fifth on; measured, the seventh level is the last one it takes faster than k_side_q8 (with six: trees of 10M x 32 37.9 -> 38.7 ms,
+    // of 1M x 256 26.4 -> 26.9), the sixth where a row is a single line and the sweep's operands are those of 128 dimensions (1M x 72, 96, 112, 25 trees:
+    // 11.5, 11.6, 12.3 -> 11.2, 11.5, 12.0; 64, 120 dimensions 9.8, 15.0 -> 9.8, 15.2).  Batches of
+    // less than 2^22 points do not fill the device either way, and k_side_q8 is one launch instead of four.
     int pm_levels = 0;
     if (q8 && w->pm_ks) {
-        pm_levels = (size_t)N * (size_t)nb >= ((size_t)1 << 22) ? pm::kMaxLevels - 1 : 0;
+        const int last = D > 64 && q8_pitch(D) == 128 ? pm::kMaxLevels - 2 : pm::kMaxLevels - 1;
+        pm_levels = (size_t)N * (size_t)nb >= ((size_t)1 << 22) ? last : 0;
         if (const char* e = std::getenv("RSFK_PM_LEVELS")) pm_levels = std::max(0, std::min(pm::kMaxLevels, std::atoi(e)));
     }
     NodeQueues Q;
