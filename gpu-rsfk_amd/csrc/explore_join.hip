@@ -28,6 +28,13 @@
 // merges them.  Nothing is decided here that the exact arithmetic would decide
 // otherwise; no atomics on shared counters, no buffer that can overflow.
 //
+// What the row certainly holds is not marked: q itself (in its own row as a rule, and in row p for every p in R(q)), and everything where p is q.
+// That is half of what passes the bound or more, and in every word: each such mark was an id gathered by the merge, and the words that are
+// left without marks are not stored (k_join_bars clears them).  (Their norms are taken for kNever, so a row with an infinite bar keeps such marks, and the
+// merge drops them.)  p among the neighbours of q, which the merge would drop too, is found by JoinSelf.
+// 10M x 32: join 24.7 -> 23.1 ms, merge 20.3 -> 18.9; 1M x 100 3.39 -> 3.21, 2.76 -> 2.56; 1M x 256 7.14 -> 7.05, 6.04 -> 5.93; 20,000 x 32 merge 0.086 -> 0.046;
+// 70,000 x 784, K = 90 the same.  (A fifth of the words is left without marks at 10M x 32: most others hold points that row p has from elsewhere.)
+//
 // For the merge kernel that works through a point's candidates in the order of their
 // bounds (explore.hip: rows with many candidates), the bound is kept for every marked
 // pair as a 16-bit code (join_bounds.hpp).
@@ -598,8 +605,10 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_rows(const int2* __restri
 // and the comparison.  1e-30 under the root covers what underflow takes from the chain.  An infinite or NaN last slot makes the bar
 // infinite or NaN, a row that is not finite makes d~ - E1 NaN, and a comparison with that drops nothing.
 // The last workgroup has no points: it takes the largest norm and error of any finite row from the parts of them (join_copy.hip).
+// The others also clear the marks (words of them): the join stores the words that are not zero only.  A word stored somewhere in a large array is a
+// memory write of its own, twice the time of a line read (26 G a second; 87 G while the array fits the last cache).
 __global__ __launch_bounds__(256) void k_join_bars(JoinCopy jc, float* __restrict__ scale, const float* __restrict__ knn_dist, int N, int K,
-                                                   float one_minus_gamma, float* __restrict__ out)
+                                                   float one_minus_gamma, float* __restrict__ out, uint32_t* __restrict__ pass, size_t words)
 {
     if (blockIdx.x + 1 == gridDim.x) {
         __shared__ float2 part[256];
@@ -625,6 +634,11 @@ __global__ __launch_bounds__(256) void k_join_bars(JoinCopy jc, float* __restric
         }
         return;
     }
+    {
+        const size_t pieces = words >> 2, stride = (size_t)(gridDim.x - 1) * 256, first = (size_t)blockIdx.x * 256 + threadIdx.x;
+        for (size_t i = first; i < pieces; i += stride) reinterpret_cast<uint4*>(pass)[i] = make_uint4(0u, 0u, 0u, 0u);
+        if (first < (words & 3)) pass[4 * pieces + first] = 0u;
+    }
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= N) return;
     const float tau = knn_dist[(size_t)p * K + (K - 1)];
@@ -644,7 +658,20 @@ __device__ __forceinline__ bool join_may(float least, float bar, float e_c)
     return !(least > w * w);
 }
 
-// One wavefront per q.  Per-wavefront LDS (ints): cq[KP] | pid[32] | pn[32] | pbar[32] | perr[32] | pper[32] | pe[32], KP = K rounded up to 32.
+// In place of the norm of a point whose pairs are not marked: above the square of any bar of a full row
+// (the finite rows' coordinates are below 2^15), and no sum with it overflows.
+constexpr float kNever = 1e37f;
+
+// Where a point is among the neighbours of q, if it is: a table in LDS by the low bits of the ids, in which a later neighbour hides an
+// earlier one (a mark too many, which the merge drops).
+template <int SIZE>
+struct JoinSelf {
+    uint8_t* at;
+    __device__ __forceinline__ void put(int c, int col) const { if (c >= 0) at[c & (SIZE - 1)] = (uint8_t)col; }
+    __device__ __forceinline__ int find(int p) const { return at[p & (SIZE - 1)]; }     // (a column that may hold p, to be compared)
+};
+
+// One wavefront per q.  Per-wavefront LDS (ints): cq[KP] | pid[32] | pn[32] | pbar[32] | perr[32] | pper[32] | pe[32] | self[64], KP = K rounded up to 32.
 // Workgroups (x, y): every gridDim.y-th tile of R(q), the y-th first.  (Five wavefronts per SIMD: 1M x 256 7.6 -> 7.0 ms against four
 // with the next 64 dimensions in flight.)
 template <int WAVES, bool BOUNDS>
@@ -669,6 +696,7 @@ __global__ __launch_bounds__(64 * WAVES, 5) void k_explore_join(JoinCopy jc, int
     float* perr = pbar + 32;
     float* pper = perr + 32;
     int* pe = reinterpret_cast<int*>(pper + 32);
+    const JoinSelf<256> self{reinterpret_cast<uint8_t*>(pe + 32)};
     const int MW = KP >> 5;
     const float most_norm = jc.mu[jc.D + 1], most_err = jc.mu[jc.D + 2];
 
@@ -676,6 +704,7 @@ __global__ __launch_bounds__(64 * WAVES, 5) void k_explore_join(JoinCopy jc, int
         int c = k < K ? old_idx[(size_t)q * K + k] : -1;
         if (c < 0 || c >= N) c = -1;
         cq[k] = c;
+        self.put(c, k);
     }
 
     for (int pt0 = 32 * (int)blockIdx.y; pt0 < R; pt0 += 32 * (int)gridDim.y) {
@@ -694,6 +723,7 @@ __global__ __launch_bounds__(64 * WAVES, 5) void k_explore_join(JoinCopy jc, int
         wave_lds_sync();
 
         const int pm = pid[lane & 31];
+        const int own = pm >= 0 ? self.find(pm) % KP : 0, own_at = cq[own] == pm ? own : -1;    // place of p among the neighbours
         const uint16_t* ra = jc.rows + (size_t)(pm >= 0 ? pm : q) * (size_t)bpitch + 8 * (lane >> 5);
         const int mbase = 4 * (lane >> 5);
         for (int ct = 0; ct < MW; ++ct) {
@@ -724,9 +754,10 @@ __global__ __launch_bounds__(64 * WAVES, 5) void k_explore_join(JoinCopy jc, int
             an += __shfl_xor(an, 32, 64);
             cn += __shfl_xor(cn, 32, 64);
             const float ce = join_err(cn, any_rel, any_abs, most_err);
+            if (cid == q) cn = kNever;
             wave_lds_sync();
             if (lane < 32) {
-                pn[lane] = an;
+                pn[lane] = pm == q ? kNever : an;
                 if (BOUNDS) perr[lane] = join_err(an, any_rel, any_abs, most_err);
             }
             wave_lds_sync();
@@ -747,7 +778,8 @@ __global__ __launch_bounds__(64 * WAVES, 5) void k_explore_join(JoinCopy jc, int
                 if (lane == m_lo) mine = (uint32_t)bm;
                 if (lane == m_lo + 4) mine = (uint32_t)(bm >> 32);
             }
-            if (lane < np) pass[(size_t)my_e * MW + ct] = mine;
+            if ((own_at >> 5) == ct) mine &= ~(1u << (own_at & 31));
+            if (lane < np && mine) pass[(size_t)my_e * MW + ct] = mine;
         }
     }
 }
@@ -770,6 +802,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_join_short(JoinCopy jc, 
 {
     __shared__ int pid_s[WAVES][32];
     __shared__ float pn_s[WAVES][32], pbar_s[WAVES][32];
+    __shared__ uint8_t self_s[WAVES][128];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int unit = __builtin_amdgcn_readfirstlane(die_local_place(blockIdx.x, gridDim.x) * WAVES + wave);
     const int item = MANY ? (int)((unsigned)unit / (unsigned)MW) : unit, ct = MANY ? unit - item * MW : 0;
@@ -793,6 +826,9 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_join_short(JoinCopy jc, 
     for (int u = 0; u < KS; ++u) cn = half_norm(b[u], cn);
     cn += __shfl_xor(cn, 32, 64);
     const float ce = join_err(cn, any_rel, any_abs, jc.mu[jc.D + 2]);
+    if (cid == q) cn = kNever;
+    const JoinSelf<128> self{self_s[wave]};
+    self.put(cid, col);
     const int mbase = 4 * hi;
     int* pid = pid_s[wave];
     float* pn = pn_s[wave];
@@ -810,6 +846,8 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_join_short(JoinCopy jc, 
         }
         wave_lds_sync();
         const int pm = pid[col];
+        const int own = pm >= 0 ? self.find(pm) & 31 : 0;
+        const bool own_there = __shfl(cid, own, 64) == pm && pm >= 0;                       // p is neighbour `own` of these
         const uint16_t* ra = jc.rows + (size_t)(pm >= 0 ? pm : q) * (size_t)bpitch + 8 * hi;
         f16x8 a[KS];
 #pragma unroll
@@ -828,7 +866,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_join_short(JoinCopy jc, 
         for (int u = 0; u < KS; ++u) an = half_norm(a[u], an);
         an += __shfl_xor(an, 32, 64);
         if (lane < 32) {
-            pn[lane] = an;
+            pn[lane] = pm == q ? kNever : an;
             pbar[lane] = bar;
         }
         wave_lds_sync();
@@ -844,7 +882,8 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_join_short(JoinCopy jc, 
             if (lane == m_lo + 4) mine = (uint32_t)(bm >> 32);
             if ((i & 3) == 3) __builtin_amdgcn_sched_barrier(0);   // four at a time: all sixteen at once take too many registers
         }
-        if (lane < np) pass[MANY ? (size_t)my_e * (size_t)MW + (size_t)ct : (size_t)my_e] = mine;
+        if (own_there) mine &= ~(1u << own);
+        if (lane < np && mine) pass[MANY ? (size_t)my_e * (size_t)MW + (size_t)ct : (size_t)my_e] = mine;
         wave_lds_sync();                                  // the tile's LDS values are read before the next tile writes them
     }
 }
@@ -869,6 +908,7 @@ __global__ __launch_bounds__(256, NPW == 3 ? 3 : 1) void k_explore_join_wg(JoinC
 {
     constexpr int kPieces = (kJwP + (NPW == 3 ? 128 : 256)) * 8 / 256;     // 16-byte pieces a thread stages per step
     extern __shared__ __align__(16) unsigned char lds_jw[];
+    __shared__ uint8_t self_s[512];
     unsigned char* rowsb = lds_jw;                                         // kJwP + KP rows of 144 bytes
     int* cq = reinterpret_cast<int*>(rowsb + (size_t)(kJwP + KP) * kJwRowBytes);
     float* cn = reinterpret_cast<float*>(cq + KP);
@@ -889,12 +929,14 @@ __global__ __launch_bounds__(256, NPW == 3 ? 3 : 1) void k_explore_join_wg(JoinC
     const int MW = KP >> 5;
     const int nrows = kJwP + KP;
     const float most_norm = jc.mu[jc.D + 1], most_err = jc.mu[jc.D + 2];
+    const JoinSelf<512> self{self_s};
     for (int k = tid; k < KP; k += 256) {
         int c = k < K ? old_idx[(size_t)q * K + k] : -1;
         if (c < 0 || c >= N) c = -1;
         cq[k] = c;
         const float n_c = c >= 0 ? jc.norms[c] : 0.0f;
-        cn[k] = n_c;
+        self.put(c, k);
+        cn[k] = c == q ? kNever : n_c;
         cerr[k] = join_err(n_c, any_rel, any_abs, most_err);
     }
     for (int pg = kJwP * (int)blockIdx.y; pg < R; pg += kJwP * (int)gridDim.y) {
@@ -907,7 +949,7 @@ __global__ __launch_bounds__(256, NPW == 3 ? 3 : 1) void k_explore_join_wg(JoinC
             const float n_p = p >= 0 ? jc.norms[p] : 0.0f, bar = p >= 0 ? bars[p] : 0.0f;
             pid[tid] = p;
             pe[tid] = e;
-            pn[tid] = n_p;
+            pn[tid] = p == q ? kNever : n_p;
             pbar[tid] = bar;
             if (BOUNDS) {
                 perr[tid] = join_err(n_p, any_rel, any_abs, most_err);
@@ -988,7 +1030,9 @@ __global__ __launch_bounds__(256, NPW == 3 ? 3 : 1) void k_explore_join_wg(JoinC
                     if (lane == m_lo + 4) mine = (uint32_t)(bm >> 32);
                     if ((j & 3) == 3) __builtin_amdgcn_sched_barrier(0);   // four at a time (registers)
                 }
-                if (lane < 32 && pt * 32 + lane < npg) pass[(size_t)pe[pt * 32 + lane] * MW + ct] = mine;
+                const int p = pid[pt * 32 + (lane & 31)], own = p >= 0 ? self.find(p) : 0;
+                if (p >= 0 && (own >> 5) == ct && cq[own] == p) mine &= ~(1u << (own & 31));
+                if (lane < 32 && pt * 32 + lane < npg && mine) pass[(size_t)pe[pt * 32 + lane] * MW + ct] = mine;
             }
         }
     }
@@ -1211,7 +1255,7 @@ int launch_explore_join(ExploreWorkspace* w, const JoinCopy& jc, int N, int D, i
     // 64 clusters 21,000 38 35 36 36, 26,000 45 42 42 44, 32,000 51 50 51 54, 45,000 67 68 73 76, 60,000 88 92 98 102; uniform x 100 21,000 70 71
     // 75 77, 32,000 96 103 110 114, 60,000 164 184 200 213.
     const unsigned parts = (unsigned)std::max(1, std::min(16, 65536 / N));
-    const int wave_ints = (KP + 192 + 3) & ~3;
+    const int wave_ints = (KP + 256 + 3) & ~3;
     const size_t lds = (size_t)kWaves * (size_t)wave_ints * sizeof(int);
     const int ksteps = (D + 15) / 16;
     RSFK_CHECK(ksteps * 16 <= join_pitch(D), "exploration join: rows of the copy too short");
@@ -1228,7 +1272,7 @@ int launch_explore_join(ExploreWorkspace* w, const JoinCopy& jc, int N, int D, i
     w->view.any_rel = any_rel;
     w->view.any_abs = any_abs;
     hipLaunchKernelGGL(k_join_bars, dim3((unsigned)((N + 255) / 256) + 1), dim3(256), 0, stream, jc, jc.scale(), knn_dist, N, K,
-                       one_minus_gamma, w->bars);
+                       one_minus_gamma, w->bars, w->pass, (size_t)N * (size_t)K * (size_t)(KP >> 5));
     RSFK_HIP(hipGetLastError());
     const int MW = KP >> 5;
     // More points than a launch has threads for take a wavefront per q: with a wavefront per 32 neighbours K = 33 from 33.5 million points on, 129
