@@ -651,11 +651,38 @@ __device__ __forceinline__ float join_least(float S, float g, float kappa)
     return __builtin_fmaf(-kappa, S, __builtin_fmaf(-2.0f, g, S));
 }
 
-// May the pair enter row p?  (true when anything is NaN; a tie at the last slot may still enter: smaller index)
-__device__ __forceinline__ bool join_may(float least, float bar, float e_c)
+// May the pair enter row p?  Not when d~ - E1 is above w^2, w = bar_p + e, e the largest e_c of the 32 neighbours tested together; that is, when
+//   g + join_reach(n_p, bar_p + e) < join_floor(n_c),   the halves of w^2 - (1 - kappa) n_p and of (1 - kappa) n_c:
+// one addition and one comparison per pair where S, d~ - E1, w and its square for each took six instructions, with branches around them.  The roundings
+// of both and of the sum are below 2^-23 (w^2 + S): kJoinWide, and 2^-19 more for kappa.  (True when anything is NaN; a tie at the last
+// slot may still enter: smaller index.)
+constexpr float kJoinWide = 1.0f + 1.0f / 1048576.0f;
+__device__ __forceinline__ float join_reach(float n_p, float w, float kappa)
 {
-    const float w = bar + e_c;
-    return !(least > w * w);
+    return 0.5f * __builtin_fmaf(kappa + 1.0f / 524288.0f - 1.0f, n_p, w * w * kJoinWide);
+}
+__device__ __forceinline__ float join_floor(float n_c, float kappa) { return 0.5f * (1.0f - (kappa + 1.0f / 524288.0f)) * n_c; }
+
+// The marks of a tile of 32 points: accumulator i of lane l holds point m = 4 (l / 32) + 8 (i / 4) + i % 4 of the tile and neighbour l % 32, so the
+// ballot over the wavefront holds the 32-bit masks of two points, low half for m = 8 (i / 4) + i % 4, high half for m + 4.  Lane m < 32 is left with
+// the mask of point m.  reach: join_reach of the tile's points (LDS).  No branch and no wait for LDS between the sixteen, and a mask goes to its lane in
+// one instruction: 10M x 32 23.06 -> 21.96 ms, 1M x 100 3.23 -> 2.86, 123,457 x 37 with K = 45 0.443 -> 0.367, 70,000 x 784 with K = 90 5.36 -> 5.05, 1M x 256
+// (whose codes are stored pair by pair) 7.0 either way.
+__device__ __forceinline__ uint32_t join_masks(const f32x16& g, const float* reach, int mbase, float floor_c)
+{
+    uint32_t mine = 0;
+#pragma unroll
+    for (int i = 0; i < 16; i += 4) {
+        const float4 r = *reinterpret_cast<const float4*>(reach + mbase + 2 * i);
+        const float at[4] = {r.x, r.y, r.z, r.w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const uint64_t bm = ballot64(!(g[i + j] + at[j] < floor_c));
+            mine = write_lane_u32((uint32_t)bm, 2 * i + j, mine);
+            mine = write_lane_u32((uint32_t)(bm >> 32), 2 * i + j + 4, mine);
+        }
+    }
+    return mine;
 }
 
 // In place of the norm of a point whose pairs are not marked: above the square of any bar of a full row
@@ -671,7 +698,7 @@ struct JoinSelf {
     __device__ __forceinline__ int find(int p) const { return at[p & (SIZE - 1)]; }     // (a column that may hold p, to be compared)
 };
 
-// One wavefront per q.  Per-wavefront LDS (ints): cq[KP] | pid[32] | pn[32] | pbar[32] | perr[32] | pper[32] | pe[32] | self[64], KP = K rounded up to 32.
+// One wavefront per q.  Per-wavefront LDS (ints): cq[KP] | pid[32] | reach[32] | pn[32] | perr[32] | pper[32] | pe[32] | self[64], KP = K rounded up to 32.
 // Workgroups (x, y): every gridDim.y-th tile of R(q), the y-th first.  (Five wavefronts per SIMD: 1M x 256 7.6 -> 7.0 ms against four
 // with the next 64 dimensions in flight.)
 template <int WAVES, bool BOUNDS>
@@ -691,9 +718,9 @@ __global__ __launch_bounds__(64 * WAVES, 5) void k_explore_join(JoinCopy jc, int
     if (R <= 32 * (int)blockIdx.y) return;
     int* cq = lds_join + (size_t)wave * (size_t)wave_lds_ints;
     int* pid = cq + KP;
-    float* pn = reinterpret_cast<float*>(pid + 32);
-    float* pbar = pn + 32;
-    float* perr = pbar + 32;
+    float* reach = reinterpret_cast<float*>(pid + 32);
+    float* pn = reach + 32;
+    float* perr = pn + 32;
     float* pper = perr + 32;
     int* pe = reinterpret_cast<int*>(pper + 32);
     const JoinSelf<256> self{reinterpret_cast<uint8_t*>(pe + 32)};
@@ -711,14 +738,14 @@ __global__ __launch_bounds__(64 * WAVES, 5) void k_explore_join(JoinCopy jc, int
         const int np = min(32, R - pt0);
         wave_lds_sync();                                  // reads of the previous tile are done (and cq is written)
         int my_e = -1;                                    // lanes 0..31: the graph entry (p, k) with q = neighbour k of p
+        float pbar = 0.0f;
         if (lane < 32) {
             my_e = lane < np ? rev[(size_t)r0 + pt0 + lane] : -1;
             const int p = my_e >= 0 ? (int)(((uint64_t)div_m * (uint64_t)(uint32_t)my_e) >> div_s) : -1;
             pid[lane] = p;
             pe[lane] = my_e;
-            const float bar = p >= 0 ? bars[p] : 0.0f;
-            pbar[lane] = bar;
-            if (BOUNDS) pper[lane] = 65534.0f / join_span(bar, most_norm);
+            if (p >= 0) pbar = bars[p];
+            if (BOUNDS) pper[lane] = 65534.0f / join_span(pbar, most_norm);
         }
         wave_lds_sync();
 
@@ -754,29 +781,29 @@ __global__ __launch_bounds__(64 * WAVES, 5) void k_explore_join(JoinCopy jc, int
             an += __shfl_xor(an, 32, 64);
             cn += __shfl_xor(cn, 32, 64);
             const float ce = join_err(cn, any_rel, any_abs, most_err);
+            const float e = wave_max(cid >= 0 ? ce : 0.0f);
             if (cid == q) cn = kNever;
             wave_lds_sync();
             if (lane < 32) {
-                pn[lane] = pm == q ? kNever : an;
-                if (BOUNDS) perr[lane] = join_err(an, any_rel, any_abs, most_err);
+                const float n_p = pm == q ? kNever : an;
+                reach[lane] = join_reach(n_p, pbar + e, kappa);
+                if (BOUNDS) {
+                    pn[lane] = n_p;
+                    perr[lane] = join_err(an, any_rel, any_abs, most_err);
+                }
             }
             wave_lds_sync();
-            // Accumulator i of lane l: point m = 4 (l / 32) + 8 (i / 4) + i % 4 of the tile, column = neighbour l % 32
-            // of this group of 32.  The ballot over the wavefront therefore holds the 32-bit masks of two points:
-            // low half for m = 8 (i / 4) + i % 4, high half for m + 4.
-            uint32_t mine = 0;                            // mask of the point this lane stores (lanes 0..31)
+            const float floor_c = join_floor(cn, kappa);
+            uint32_t mine = join_masks(g, reach, mbase, floor_c) & (uint32_t)ballot64(cid >= 0);   // mask of the point this lane stores (lanes 0..31)
+            if (BOUNDS && cid >= 0) {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const int m = mbase + 8 * (i >> 2) + (i & 3);
-                const float least = join_least(pn[m] + cn, g[i], kappa);
-                const bool marked = cid >= 0 && join_may(least, pbar[m], ce);
-                const uint64_t bm = ballot64(marked);
-                if (BOUNDS && marked && m < np)
-                    bounds[(size_t)pe[m] * (size_t)KP + ct * 32 + (lane & 31)] =
-                        (uint16_t)join_code(least, perr[m], ce, pper[m]);
-                const int m_lo = 8 * (i >> 2) + (i & 3);
-                if (lane == m_lo) mine = (uint32_t)bm;
-                if (lane == m_lo + 4) mine = (uint32_t)(bm >> 32);
+                for (int i = 0; i < 16; ++i) {
+                    const int m = mbase + 8 * (i >> 2) + (i & 3);
+                    if (m < np && !(g[i] + reach[m] < floor_c))
+                        bounds[(size_t)pe[m] * (size_t)KP + ct * 32 + (lane & 31)] =
+                            (uint16_t)join_code(join_least(pn[m] + cn, g[i], kappa), perr[m], ce, pper[m]);
+                    if ((i & 3) == 3) __builtin_amdgcn_sched_barrier(0);   // four at a time (registers)
+                }
             }
             if ((own_at >> 5) == ct) mine &= ~(1u << (own_at & 31));
             if (lane < np && mine) pass[(size_t)my_e * MW + ct] = mine;
@@ -801,7 +828,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_join_short(JoinCopy jc, 
                                                                     const int* __restrict__ order)
 {
     __shared__ int pid_s[WAVES][32];
-    __shared__ float pn_s[WAVES][32], pbar_s[WAVES][32];
+    __shared__ __align__(16) float reach_s[WAVES][32];
     __shared__ uint8_t self_s[WAVES][128];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int unit = __builtin_amdgcn_readfirstlane(die_local_place(blockIdx.x, gridDim.x) * WAVES + wave);
@@ -819,20 +846,20 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_join_short(JoinCopy jc, 
     for (int u = 0; u < KS; ++u) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) b[u][i] = (_Float16)0.0f;
-        if (u < ksteps) b[u] = *reinterpret_cast<const f16x8*>(rb + 16 * u);
+        if (KS <= 4 || u < ksteps) b[u] = *reinterpret_cast<const f16x8*>(rb + 16 * u);
     }
     float cn = 0.0f;
 #pragma unroll
     for (int u = 0; u < KS; ++u) cn = half_norm(b[u], cn);
     cn += __shfl_xor(cn, 32, 64);
-    const float ce = join_err(cn, any_rel, any_abs, jc.mu[jc.D + 2]);
-    if (cid == q) cn = kNever;
+    const float e = wave_max(cid >= 0 ? join_err(cn, any_rel, any_abs, jc.mu[jc.D + 2]) : 0.0f);
+    const float floor_c = join_floor(cid == q ? kNever : cn, kappa);
+    const uint32_t there = (uint32_t)ballot64(cid >= 0);
     const JoinSelf<128> self{self_s[wave]};
     self.put(cid, col);
     const int mbase = 4 * hi;
     int* pid = pid_s[wave];
-    float* pn = pn_s[wave];
-    float* pbar = pbar_s[wave];
+    float* reach = reach_s[wave];
 
     for (int pt0 = 32 * (int)blockIdx.y; pt0 < R; pt0 += 32 * (int)gridDim.y) {
         const int np = min(32, R - pt0);
@@ -854,7 +881,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_join_short(JoinCopy jc, 
         for (int u = 0; u < KS; ++u) {
 #pragma unroll
             for (int i = 0; i < 8; ++i) a[u][i] = (_Float16)0.0f;
-            if (u < ksteps) a[u] = *reinterpret_cast<const f16x8*>(ra + 16 * u);
+            if (KS <= 4 || u < ksteps) a[u] = *reinterpret_cast<const f16x8*>(ra + 16 * u);
         }
         f32x16 g;
 #pragma unroll
@@ -865,23 +892,9 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_join_short(JoinCopy jc, 
 #pragma unroll
         for (int u = 0; u < KS; ++u) an = half_norm(a[u], an);
         an += __shfl_xor(an, 32, 64);
-        if (lane < 32) {
-            pn[lane] = pm == q ? kNever : an;
-            pbar[lane] = bar;
-        }
+        if (lane < 32) reach[lane] = join_reach(pm == q ? kNever : an, bar + e, kappa);
         wave_lds_sync();
-        // Accumulator i of lane l: point m = 4 (l / 32) + 8 (i / 4) + i % 4 of the tile, column = neighbour l % 32.
-        uint32_t mine = 0;                                // mask of the point this lane stores (lanes 0..31)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int m = mbase + 8 * (i >> 2) + (i & 3);
-            const float least = join_least(pn[m] + cn, g[i], kappa);
-            const uint64_t bm = ballot64(cid >= 0 && join_may(least, pbar[m], ce));
-            const int m_lo = 8 * (i >> 2) + (i & 3);
-            if (lane == m_lo) mine = (uint32_t)bm;
-            if (lane == m_lo + 4) mine = (uint32_t)(bm >> 32);
-            if ((i & 3) == 3) __builtin_amdgcn_sched_barrier(0);   // four at a time: all sixteen at once take too many registers
-        }
+        uint32_t mine = join_masks(g, reach, mbase, floor_c) & there;    // mask of the point this lane stores (lanes 0..31)
         if (own_there) mine &= ~(1u << own);
         if (lane < np && mine) pass[MANY ? (size_t)my_e * (size_t)MW + (size_t)ct : (size_t)my_e] = mine;
         wave_lds_sync();                                  // the tile's LDS values are read before the next tile writes them
@@ -909,6 +922,7 @@ __global__ __launch_bounds__(256, NPW == 3 ? 3 : 1) void k_explore_join_wg(JoinC
     constexpr int kPieces = (kJwP + (NPW == 3 ? 128 : 256)) * 8 / 256;     // 16-byte pieces a thread stages per step
     extern __shared__ __align__(16) unsigned char lds_jw[];
     __shared__ uint8_t self_s[512];
+    __shared__ float wave_e[4];
     unsigned char* rowsb = lds_jw;                                         // kJwP + KP rows of 144 bytes
     int* cq = reinterpret_cast<int*>(rowsb + (size_t)(kJwP + KP) * kJwRowBytes);
     float* cn = reinterpret_cast<float*>(cq + KP);
@@ -916,8 +930,8 @@ __global__ __launch_bounds__(256, NPW == 3 ? 3 : 1) void k_explore_join_wg(JoinC
     int* pid = reinterpret_cast<int*>(cerr + KP);
     int* pe = pid + kJwP;
     float* pn = reinterpret_cast<float*>(pe + kJwP);
-    float* pbar = pn + kJwP;
-    float* perr = pbar + kJwP;
+    float* reach = pn + kJwP;
+    float* perr = reach + kJwP;
     float* pper = perr + kJwP;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int n = lane & 31, h = lane >> 5;
@@ -930,6 +944,7 @@ __global__ __launch_bounds__(256, NPW == 3 ? 3 : 1) void k_explore_join_wg(JoinC
     const int nrows = kJwP + KP;
     const float most_norm = jc.mu[jc.D + 1], most_err = jc.mu[jc.D + 2];
     const JoinSelf<512> self{self_s};
+    float e_most = 0.0f;                                                   // the largest e_c of all the neighbours
     for (int k = tid; k < KP; k += 256) {
         int c = k < K ? old_idx[(size_t)q * K + k] : -1;
         if (c < 0 || c >= N) c = -1;
@@ -937,8 +952,14 @@ __global__ __launch_bounds__(256, NPW == 3 ? 3 : 1) void k_explore_join_wg(JoinC
         const float n_c = c >= 0 ? jc.norms[c] : 0.0f;
         self.put(c, k);
         cn[k] = c == q ? kNever : n_c;
-        cerr[k] = join_err(n_c, any_rel, any_abs, most_err);
+        const float ce = join_err(n_c, any_rel, any_abs, most_err);
+        cerr[k] = ce;
+        if (c >= 0) e_most = fmaxf(e_most, ce);
     }
+    e_most = wave_max(e_most);
+    if (lane == 0) wave_e[wave] = e_most;
+    __syncthreads();
+    e_most = fmaxf(fmaxf(wave_e[0], wave_e[1]), fmaxf(wave_e[2], wave_e[3]));
     for (int pg = kJwP * (int)blockIdx.y; pg < R; pg += kJwP * (int)gridDim.y) {
         const int npg = min(kJwP, R - pg);
         const int npairs = ((npg + 31) >> 5) * MW;
@@ -949,8 +970,9 @@ __global__ __launch_bounds__(256, NPW == 3 ? 3 : 1) void k_explore_join_wg(JoinC
             const float n_p = p >= 0 ? jc.norms[p] : 0.0f, bar = p >= 0 ? bars[p] : 0.0f;
             pid[tid] = p;
             pe[tid] = e;
-            pn[tid] = p == q ? kNever : n_p;
-            pbar[tid] = bar;
+            const float n_m = p == q ? kNever : n_p;
+            pn[tid] = n_m;
+            reach[tid] = join_reach(n_m, bar + e_most, kappa);
             if (BOUNDS) {
                 perr[tid] = join_err(n_p, any_rel, any_abs, most_err);
                 pper[tid] = 65534.0f / join_span(bar, most_norm);
@@ -1015,20 +1037,17 @@ __global__ __launch_bounds__(256, NPW == 3 ? 3 : 1) void k_explore_join_wg(JoinC
                 const int pt = pair / MW, ct = pair - pt * MW;
                 const int col = ct * 32 + n;
                 const int cid = cq[col];
-                const float cnv = cn[col], ce = cerr[col];
-                uint32_t mine = 0;
+                const float cnv = cn[col], ce = cerr[col], floor_c = join_floor(cnv, kappa);
+                uint32_t mine = join_masks(acc[i], reach + pt * 32, 4 * h, floor_c) & (uint32_t)ballot64(cid >= 0);
+                if (BOUNDS && cid >= 0) {
 #pragma unroll
-                for (int j = 0; j < 16; ++j) {
-                    const int m = pt * 32 + 4 * h + 8 * (j >> 2) + (j & 3);
-                    const float least = join_least(pn[m] + cnv, acc[i][j], kappa);
-                    const bool marked = cid >= 0 && join_may(least, pbar[m], ce);
-                    const uint64_t bm = ballot64(marked);
-                    if (BOUNDS && marked && m < npg)
-                        bounds[(size_t)pe[m] * (size_t)KP + col] = (uint16_t)join_code(least, perr[m], ce, pper[m]);
-                    const int m_lo = 8 * (j >> 2) + (j & 3);
-                    if (lane == m_lo) mine = (uint32_t)bm;
-                    if (lane == m_lo + 4) mine = (uint32_t)(bm >> 32);
-                    if ((j & 3) == 3) __builtin_amdgcn_sched_barrier(0);   // four at a time (registers)
+                    for (int j = 0; j < 16; ++j) {
+                        const int m = pt * 32 + 4 * h + 8 * (j >> 2) + (j & 3);
+                        if (m < npg && !(acc[i][j] + reach[m] < floor_c))
+                            bounds[(size_t)pe[m] * (size_t)KP + col] =
+                                (uint16_t)join_code(join_least(pn[m] + cnv, acc[i][j], kappa), perr[m], ce, pper[m]);
+                        if ((j & 3) == 3) __builtin_amdgcn_sched_barrier(0);   // four at a time (registers)
+                    }
                 }
                 const int p = pid[pt * 32 + (lane & 31)], own = p >= 0 ? self.find(p) : 0;
                 if (p >= 0 && (own >> 5) == ct && cq[own] == p) mine &= ~(1u << (own & 31));
