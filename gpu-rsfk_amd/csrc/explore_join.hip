@@ -59,6 +59,7 @@ struct ExploreWorkspace {
     uint32_t div_m = 0;        // e / K == (div_m * e) >> div_s for 0 <= e < 2^31
     int div_s = 0;
     int* rev = nullptr;        // N*K: R lists in compressed rows; an element is the number p K + k of a graph entry
+    uint16_t* rev_bars = nullptr;   // N*K: code of the bar of the point of each element of rev (bar_code), or null
     int* offs = nullptr;       // N+1: start of R(q)
     int2* bin_eq = nullptr;    // N*K: (entry number, neighbour minus the first point of its bin), grouped by the bin of
                                // the neighbour; one 8-byte store per entry
@@ -122,6 +123,28 @@ bool rev_bins(int N, int* shift, int* n_bins)
     *n_bins = N > 0 ? ((N - 1) >> s) + 1 : 1;
     return *n_bins <= kMaxBins;
 }
+
+// A bar in 16 bits, rounded up: 11 bits behind the leading one, from 2^-9 to 2^23 (in the units of the copy, whose coordinates are below 2^15 and
+// not all below 2^12); what is not below that, or NaN, is infinite.  A candidate more passes for it, none less.  (10M x 32: 0.8 % more marks.)
+// The staged builder of the reversed graph carries it beside the entries, in the half of a record that the place in its bin leaves, because it
+// reads the graph point by point: gathered by the join, the bars are a line read for every element of R(q), and a trip after it.
+// 10M x 32: join 15.54 -> 12.02 ms, last step of the builder 2.24 -> 2.54.  (Smaller graphs, whose bars stay in the L2, gain nothing: 1M x 100 join 2.86 ->
+// 2.85 ms, last step of the builder 0.18 -> 0.25.)
+constexpr uint32_t kBarBase = 118u << 11;
+__device__ __forceinline__ uint32_t bar_code(float bar)
+{
+    if (!(bar < 8388608.0f)) return 0xffffu;
+    return min(((__float_as_uint(fmaxf(bar, 1.0f / 512.0f)) + 0xfffu) >> 12) - kBarBase, 0xffffu);
+}
+__device__ __forceinline__ float bar_of(uint32_t code) { return code == 0xffffu ? INFINITY : __uint_as_float((code + kBarBase) << 12); }
+
+// What a builder needs for it.  With bars a record's second word is the place in its bin (16 bits) and the code above it.
+struct RevBars {
+    const float* bars = nullptr;
+    uint32_t div_m = 0;
+    int div_s = 0;
+    __device__ __forceinline__ float of_entry(int e) const { return bars[(int)(((uint64_t)div_m * (uint64_t)(uint32_t)e) >> div_s)]; }
+};
 
 __global__ void k_zero(int* a, int n, int* counter, int* shares)
 {
@@ -324,9 +347,10 @@ constexpr size_t staged_lds_bytes(int n_bins)
 }
 
 // (1) a part of the graph to the coarse bins.  part_off / bin_start as left by k_bin_count / k_bin_scan at shift = cshift.
+template <bool BARS>
 __global__ __launch_bounds__(256) void k_staged_scatter1(const int* __restrict__ old_idx, int total, int per_part, int N, int cshift,
                                                          int n_coarse, const int* __restrict__ bin_start,
-                                                         const int* __restrict__ part_off, int2* __restrict__ out)
+                                                         const int* __restrict__ part_off, int2* __restrict__ out, RevBars rb)
 {
     extern __shared__ __align__(16) int lds_st[];
     __shared__ int wave_lds[4];
@@ -339,17 +363,29 @@ __global__ __launch_bounds__(256) void k_staged_scatter1(const int* __restrict__
     __syncthreads();
     const long long begin = (long long)blockIdx.x * per_part;
     const int e0 = (int)min((long long)total, begin), e1 = (int)min((long long)total, begin + per_part);
+    // (the neighbours of the next tile travel while this one is sorted)
+    int q[16];
+    float bar[16];
+    auto request = [&](int t0) {
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            const int e = t0 + 256 * u + (int)threadIdx.x;
+            q[u] = e < e1 ? old_idx[e] : -1;
+            if (BARS) bar[u] = rb.of_entry(min(e, e1 - 1));
+        }
+    };
+    if (e0 < e1) request(e0);
     for (int t0 = e0; t0 < e1; t0 += kStTile) {
         int2 rec[16];
         int bin[16];
 #pragma unroll
         for (int u = 0; u < 16; ++u) {
-            const int e = t0 + 256 * u + (int)threadIdx.x;
-            const int q = e < e1 ? old_idx[e] : -1;
-            const bool ok = q >= 0 && q < N;
-            rec[u] = make_int2(e, q);
-            bin[u] = ok ? q >> cshift : -1;
+            const bool ok = q[u] >= 0 && q[u] < N;
+            rec[u] = make_int2(t0 + 256 * u + (int)threadIdx.x,
+                               BARS ? (int)(((uint32_t)q[u] & ((1u << cshift) - 1u)) | bar_code(bar[u]) << 16) : q[u]);
+            bin[u] = ok ? q[u] >> cshift : -1;
         }
+        if (t0 + kStTile < e1) request(t0 + kStTile);
         staged_tile_out(rec, bin, n_coarse, cnt, first, stage, sbin, cursor, wave_lds, out);
     }
 }
@@ -419,15 +455,18 @@ __global__ __launch_bounds__(256) void k_staged_scatter2(const int2* __restrict_
 }
 
 // (3) one workgroup per fine bin: row offsets of its points, and its rows -- assembled in LDS and written whole when the
-// bin has at most kStRowsCap entries, entry by entry otherwise.  LDS: cnt[2^fshift] | stage[kStRowsCap].
+// bin has at most kStRowsCap entries, entry by entry otherwise.  LDS: cnt[2^fshift] | stage[kStRowsCap] | codes[kStRowsCap] (16 bits; with bars).
+template <bool BARS>
 __global__ __launch_bounds__(kRowsBlock) void k_staged_rows(const int2* __restrict__ rec2, const int* __restrict__ fine_start,
-                                                            int fshift, int N, int* __restrict__ offs, int* __restrict__ rev)
+                                                            int fshift, int N, int* __restrict__ offs, int* __restrict__ rev,
+                                                            uint16_t* __restrict__ rev_bars)
 {
     extern __shared__ int lds_rows[];
     __shared__ int wave_lds[kRowsBlock / 64];
     const int R = 1 << fshift;
     int* cnt = lds_rows;
     int* stage = cnt + R;
+    uint16_t* codes = reinterpret_cast<uint16_t*>(stage + kStRowsCap);
     const int b = blockIdx.x;
     const int s0 = fine_start[b], s1 = fine_start[b + 1];
     const int q0 = b << fshift;
@@ -456,10 +495,14 @@ __global__ __launch_bounds__(kRowsBlock) void k_staged_rows(const int2* __restri
         const int at = atomicAdd(&cnt[eq.y & low], 1);
         if (in_lds) stage[at] = eq.x;
         else rev[s0 + at] = eq.x;
+        if (BARS) (in_lds ? codes[at] : rev_bars[s0 + at]) = (uint16_t)((uint32_t)eq.y >> 16);
     }
     if (in_lds) {
         __syncthreads();
-        for (int i = threadIdx.x; i < s1 - s0; i += kRowsBlock) rev[s0 + i] = stage[i];
+        for (int i = threadIdx.x; i < s1 - s0; i += kRowsBlock) {
+            rev[s0 + i] = stage[i];
+            if (BARS) rev_bars[s0 + i] = codes[i];
+        }
     }
 }
 
@@ -600,12 +643,127 @@ __global__ __launch_bounds__(kTileThreads) void k_tile_rows(const int2* __restri
     }
 }
 
+// The marks of graphs of 2^26 entries and more (those of the staged builder) with up to 32 neighbours.  A word stored somewhere in an array
+// beyond the last cache is a memory write of its own, about 26 G a second whatever else goes on, and the join of 10M x 32 stored 256 M of them.
+// It now writes its words in the order of R, whole lines, and they go to their places as the entries came: sorted by window of 2^21 words, 8192 words at a time in LDS, leaving as records (entry, word) in runs, each window's share reserved by one
+// addition per tile and window; the same again inside a window to pieces of 2^14 words; a piece is put together in LDS and written whole, with the zeros.
+// 10M x 32: join 21.96 -> 15.54 ms, the three steps 1.22 + 1.23 + 0.63, and 0.24 less for words not cleared.  (One sort by windows of 2^19 words
+// and stores from there, although they meet in the L2: 1.76 + 3.04, by 2^21 1.21 + 3.54.)  Smaller graphs: 1M x 100, whose words fit the last cache, 2.85 ms of which 0.47 are the stores; the steps would
+// take 0.3 of that.
+constexpr int kMarkThreads = 512, kMarkPer = 16, kMarkTile = kMarkThreads * kMarkPer;
+constexpr int kMarkWindow = 21, kMarkPiece = 14;          // bits
+
+__host__ __device__ inline size_t mark_lds_bytes(int n_bins) { return (size_t)3 * ((n_bins + 3) & ~3) * sizeof(int) + (size_t)kMarkTile * sizeof(int2); }
+inline int mark_windows(size_t total) { return (int)((total - 1) >> kMarkWindow) + 1; }
+// counters: a line for each window, an int for each piece
+inline size_t mark_ints(size_t total) { return (size_t)mark_windows(total) * (32 + ((size_t)1 << (kMarkWindow - kMarkPiece))); }
+
+// FIRST: word i of marks belongs to entry rev[i], i < *n_in, and goes to its window; otherwise the records of window blockIdx.y (n_in[32 y] of them) to
+// their pieces.  taken[stride b]: words of bin b so far (zero before the launch).  Record i of bin b of out: one of its words, in no order.
+template <bool FIRST>
+__global__ __launch_bounds__(kMarkThreads) void k_mark_scatter(const int* __restrict__ rev, const uint32_t* __restrict__ marks,
+                                                               const int2* __restrict__ rec, const int* __restrict__ n_in, int n_bins,
+                                                               int stride, int* __restrict__ taken, int2* __restrict__ out)
+{
+    constexpr int kBits = FIRST ? kMarkWindow : kMarkPiece;
+    extern __shared__ __align__(16) int lds_mark[];
+    __shared__ int wave_lds[kMarkThreads / 64];
+    const int nb = (n_bins + 3) & ~3, tid = threadIdx.x;
+    int* cnt = lds_mark;
+    int* first = cnt + nb;
+    int* base = first + nb;
+    int2* stage = reinterpret_cast<int2*>(base + nb);
+    if (!FIRST) {
+        rec += (size_t)blockIdx.y << kMarkWindow;
+        out += (size_t)blockIdx.y << kMarkWindow;
+        taken += (size_t)blockIdx.y * (size_t)n_bins;
+    }
+    const size_t n = (size_t)(FIRST ? *n_in : n_in[32 * blockIdx.y]), step = (size_t)gridDim.x * kMarkTile;
+    const int low = FIRST ? 0x7fffffff : (1 << kMarkWindow) - 1;
+    int2 r[kMarkPer];
+    auto request = [&](size_t t0) {
+#pragma unroll
+        for (int u = 0; u < kMarkPer; ++u) {
+            const size_t i = t0 + (size_t)(kMarkThreads * u + tid);
+            r[u] = make_int2(0, 0);
+            if (FIRST && i < n) r[u] = make_int2(rev[i], (int)marks[i]);
+            if (!FIRST && i < n) r[u] = rec[i];
+        }
+    };
+    const size_t t_first = (size_t)blockIdx.x * kMarkTile;
+    request(t_first);
+    for (size_t t0 = t_first; t0 < n; t0 += step) {
+        for (int b = tid; b < n_bins; b += kMarkThreads) cnt[b] = 0;
+        __syncthreads();
+        int rank[kMarkPer];
+#pragma unroll
+        for (int u = 0; u < kMarkPer; ++u) rank[u] = r[u].y ? atomicAdd(&cnt[(r[u].x & low) >> kBits], 1) : 0;
+        __syncthreads();
+        // (at most 1024 bins: two per thread)
+        const int b0 = 2 * tid, c0 = b0 < n_bins ? cnt[b0] : 0, c1 = b0 + 1 < n_bins ? cnt[b0 + 1] : 0;
+        if (c0) base[b0] = atomicAdd(&taken[stride * b0], c0);
+        if (c1) base[b0 + 1] = atomicAdd(&taken[stride * (b0 + 1)], c1);
+        int n_tile;
+        const int ex = block_excl_scan(c0 + c1, &n_tile, wave_lds);
+        if (b0 < n_bins) first[b0] = ex;
+        if (b0 + 1 < n_bins) first[b0 + 1] = ex + c0;
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < kMarkPer; ++u)
+            if (r[u].y) stage[first[(r[u].x & low) >> kBits] + rank[u]] = r[u];
+        __syncthreads();
+        if (t0 + step < n) request(t0 + step);
+        for (int i = tid; i < n_tile; i += kMarkThreads) {
+            const int2 x = stage[i];
+            const int b = (x.x & low) >> kBits;
+            out[((size_t)b << kBits) + (size_t)(base[b] + i - first[b])] = x;
+        }
+        __syncthreads();
+    }
+}
+
+// One workgroup per piece: its words, taken[blockIdx.x] of them in records, and zeros.
+__global__ __launch_bounds__(kMarkThreads) void k_mark_place(const int2* __restrict__ rec, const int* __restrict__ taken, size_t total,
+                                                             uint32_t* __restrict__ pass)
+{
+    extern __shared__ __align__(16) int lds_mark[];
+    uint4* words = reinterpret_cast<uint4*>(lds_mark);
+    const size_t first = (size_t)blockIdx.x << kMarkPiece;
+    const int n = taken[blockIdx.x], tid = threadIdx.x;
+    rec += first;
+    pass += first;
+    int2 r[8];
+    auto request = [&](int i) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) r[u] = i + kMarkThreads * u < n ? rec[i + kMarkThreads * u] : make_int2(-1, 0);
+    };
+    request(tid);
+    for (int i = tid; i < (1 << kMarkPiece) / 4; i += kMarkThreads) words[i] = make_uint4(0u, 0u, 0u, 0u);
+    __syncthreads();
+    for (int i = tid; i < n; i += 8 * kMarkThreads) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (r[u].x >= 0) lds_mark[r[u].x & ((1 << kMarkPiece) - 1)] = r[u].y;
+        if (i + 8 * kMarkThreads < n) request(i + 8 * kMarkThreads);
+    }
+    __syncthreads();
+    const int there = (int)min((size_t)1 << kMarkPiece, total - first);
+    for (int i = tid; i < there / 4; i += kMarkThreads) reinterpret_cast<uint4*>(pass)[i] = words[i];
+    if (tid < (there & 3)) pass[(there & ~3) + tid] = (uint32_t)lds_mark[(there & ~3) + tid];
+}
+
+__global__ __launch_bounds__(256) void k_mark_clear(int* __restrict__ taken, int n)
+{
+    const int b = blockIdx.x * 256 + threadIdx.x;
+    if (b < n) taken[b] = 0;
+}
+
 // The bar of a point: s sqrt(last slot of its row / (1 - gamma)) + e_p.
 // A sum bar + e_c is at least 1 + 2^-21 times the sum of the values it stands for, which covers the roundings of the sum, its square
 // and the comparison.  1e-30 under the root covers what underflow takes from the chain.  An infinite or NaN last slot makes the bar
 // infinite or NaN, a row that is not finite makes d~ - E1 NaN, and a comparison with that drops nothing.
 // The last workgroup has no points: it takes the largest norm and error of any finite row from the parts of them (join_copy.hip).
-// The others also clear the marks (words of them): the join stores the words that are not zero only.  A word stored somewhere in a large array is a
+// The others also clear the marks (words of them, none where they are put together: k_mark_place): the join stores the words that are not zero only.  A word stored somewhere in a large array is a
 // memory write of its own, twice the time of a line read (26 G a second; 87 G while the array fits the last cache).
 __global__ __launch_bounds__(256) void k_join_bars(JoinCopy jc, float* __restrict__ scale, const float* __restrict__ knn_dist, int N, int K,
                                                    float one_minus_gamma, float* __restrict__ out, uint32_t* __restrict__ pass, size_t words)
@@ -823,7 +981,8 @@ template <int WAVES, int KS, bool MANY>
 __global__ __launch_bounds__(64 * WAVES) void k_explore_join_short(JoinCopy jc, int N, int K, const int* __restrict__ old_idx,
                                                                     const float* __restrict__ bars,
                                                                     const int* __restrict__ offs, const int* __restrict__ rev,
-                                                                    uint32_t* __restrict__ pass, int MW, int bpitch, int ksteps,
+                                                                    const uint16_t* __restrict__ rev_bars,
+                                                                    uint32_t* __restrict__ pass, uint32_t* __restrict__ marks, int MW, int bpitch, int ksteps,
                                                                     float kappa, float any_rel, float any_abs, uint32_t div_m, int div_s,
                                                                     const int* __restrict__ order)
 {
@@ -869,7 +1028,8 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_join_short(JoinCopy jc, 
             my_e = lane < np ? rev[(size_t)r0 + pt0 + lane] : -1;
             const int p = my_e >= 0 ? (int)(((uint64_t)div_m * (uint64_t)(uint32_t)my_e) >> div_s) : -1;
             pid[lane] = p;
-            if (p >= 0) bar = bars[p];
+            if (lane < np && rev_bars) bar = bar_of(rev_bars[(size_t)r0 + pt0 + lane]);
+            else if (p >= 0) bar = bars[p];
         }
         wave_lds_sync();
         const int pm = pid[col];
@@ -896,7 +1056,9 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_join_short(JoinCopy jc, 
         wave_lds_sync();
         uint32_t mine = join_masks(g, reach, mbase, floor_c) & there;    // mask of the point this lane stores (lanes 0..31)
         if (own_there) mine &= ~(1u << own);
-        if (lane < np && mine) pass[MANY ? (size_t)my_e * (size_t)MW + (size_t)ct : (size_t)my_e] = mine;
+        if (!MANY && marks) {
+            if (lane < np) marks[(size_t)r0 + pt0 + lane] = mine;          // (in the order of R: k_mark_scatter)
+        } else if (lane < np && mine) pass[MANY ? (size_t)my_e * (size_t)MW + (size_t)ct : (size_t)my_e] = mine;
         wave_lds_sync();                                  // the tile's LDS values are read before the next tile writes them
     }
 }
@@ -1147,7 +1309,7 @@ int explore_ws_alloc(ExploreWorkspace** out, int N, int K, bool with_bounds, boo
     if (w->staged &&
         (dm(&w->bin_eq2, 2 * total) != hipSuccess || dm(&w->fine_size, (size_t)w->n_fine) != hipSuccess ||
          dm(&w->fine_start, (size_t)w->n_fine + 1) != hipSuccess ||
-         dm(&w->sub_off, (size_t)w->n_sub << (w->cshift - w->fshift)) != hipSuccess)) {
+         dm(&w->sub_off, std::max((size_t)w->n_sub << (w->cshift - w->fshift), mark_ints(total))) != hipSuccess)) {
         explore_ws_free(w);
         if (!graph_only) set_last_error("exploration workspace: out of device memory");
         return 1;
@@ -1169,6 +1331,9 @@ int explore_ws_alloc(ExploreWorkspace** out, int N, int K, bool with_bounds, boo
         void* b = nullptr;
         if (bytes <= ((size_t)16 << 30) && ws_try_alloc(&b, bytes) == 0) w->bounds = static_cast<uint16_t*>(b);
     }
+    // The codes of the bars beside the reversed graph, in the records of the first scatter, which are done with when the rows are made.
+    // Bins of more than 2^16 points leave no room in a record, rows of more than 2^11 points at a time none in LDS.
+    if (!graph_only && !w->bounds && w->staged && w->cshift <= 16 && w->fshift <= 11) w->rev_bars = reinterpret_cast<uint16_t*>(w->bin_eq);
     *out = w;
     return 0;
 }
@@ -1197,11 +1362,15 @@ bool explore_ws_takes(int N, int K)
 const int* explore_ws_offs(const ExploreWorkspace* w) { return w->offs; }
 int* explore_ws_rev(const ExploreWorkspace* w) { return w->rev; }
 
-// The reversed graph of idx (offs, rev).
-int launch_reversed_graph(ExploreWorkspace* w, const int* old_idx, int N, int K, hipStream_t stream)
+namespace {
+
+// with_bars: rev_bars too, from bars
+int launch_rev(ExploreWorkspace* w, const int* old_idx, int N, int K, hipStream_t stream, bool with_bars)
 {
     RSFK_CHECK(w && w->N == N && w->K == K, "reversed graph: workspace does not match");
     const int total = (int)((size_t)N * (size_t)K);
+    const RevBars rb{w->bars, w->div_m, w->div_s};
+    const size_t rows_lds = ((size_t)(1 << w->fshift) + kStRowsCap) * sizeof(int) + (with_bars ? kStRowsCap * sizeof(uint16_t) : 0);
     if (w->staged) {
         const int nc = w->n_coarse, per = 1 << (w->cshift - w->fshift);
         hipLaunchKernelGGL(k_zero, dim3((unsigned)((nc + 255) / 256)), dim3(256), 0, stream, w->bin_size, nc,
@@ -1211,8 +1380,9 @@ int launch_reversed_graph(ExploreWorkspace* w, const int* old_idx, int N, int K,
         hipLaunchKernelGGL(k_bin_count, dim3((unsigned)w->n_parts), dim3(256), (size_t)nc * sizeof(int), stream, old_idx, total,
                            w->per_part, N, w->cshift, nc, w->bin_size, w->part_off);
         hipLaunchKernelGGL(k_bin_scan, dim3(1), dim3(256), 0, stream, w->bin_size, nc, w->bin_start, w->offs + N);
-        hipLaunchKernelGGL(k_staged_scatter1, dim3((unsigned)w->n_parts), dim3(256), staged_lds_bytes(nc), stream, old_idx, total,
-                           w->per_part, N, w->cshift, nc, w->bin_start, w->part_off, w->bin_eq);
+        auto* scatter1 = with_bars ? k_staged_scatter1<true> : k_staged_scatter1<false>;
+        hipLaunchKernelGGL(scatter1, dim3((unsigned)w->n_parts), dim3(256), staged_lds_bytes(nc), stream, old_idx, total,
+                           w->per_part, N, w->cshift, nc, w->bin_start, w->part_off, w->bin_eq, rb);
         // sub-parts of a coarse bin walked by a few workgroups each (four times the mean number of sub-parts per bin)
         const unsigned walkers = (unsigned)std::max<size_t>(1, std::min<size_t>(64, 4 * ((size_t)total / kStSub / (size_t)nc + 1)));
         hipLaunchKernelGGL(k_staged_count2, dim3(walkers, (unsigned)nc), dim3(256), (size_t)per * sizeof(int), stream, w->bin_eq,
@@ -1220,11 +1390,10 @@ int launch_reversed_graph(ExploreWorkspace* w, const int* old_idx, int N, int K,
         hipLaunchKernelGGL(k_bin_scan, dim3(1), dim3(256), 0, stream, w->fine_size, w->n_fine, w->fine_start, w->offs + N);
         hipLaunchKernelGGL(k_staged_scatter2, dim3(walkers, (unsigned)nc), dim3(256), staged_lds_bytes(per), stream, w->bin_eq,
                            w->bin_start, w->cshift, w->fshift, w->fine_start, w->sub_off, w->bin_eq2);
-        const size_t rows_lds = ((size_t)(1 << w->fshift) + kStRowsCap) * sizeof(int);
-        RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_staged_rows), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     (int)rows_lds));
-        hipLaunchKernelGGL(k_staged_rows, dim3((unsigned)w->n_fine), dim3(kRowsBlock), rows_lds, stream, w->bin_eq2, w->fine_start,
-                           w->fshift, N, w->offs, w->rev);
+        auto* rows = with_bars ? k_staged_rows<true> : k_staged_rows<false>;
+        RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(rows), hipFuncAttributeMaxDynamicSharedMemorySize, (int)rows_lds));
+        hipLaunchKernelGGL(rows, dim3((unsigned)w->n_fine), dim3(kRowsBlock), rows_lds, stream, w->bin_eq2, w->fine_start,
+                           w->fshift, N, w->offs, w->rev, w->rev_bars);
     } else if (w->tiled) {
         const int nc = w->n_coarse;
         hipLaunchKernelGGL(k_zero, dim3((unsigned)((nc + 255) / 256)), dim3(256), 0, stream, w->bin_size, nc,
@@ -1236,7 +1405,6 @@ int launch_reversed_graph(ExploreWorkspace* w, const int* old_idx, int N, int K,
                                      (int)tile_lds_bytes(nc)));
         hipLaunchKernelGGL(k_tile_scatter, dim3((unsigned)w->n_parts), dim3(kTileThreads), tile_lds_bytes(nc), stream, old_idx, total,
                            w->per_part, N, w->cshift, nc, w->bin_start, w->part_off, w->bin_eq);
-        const size_t rows_lds = ((size_t)(1 << w->fshift) + kStRowsCap) * sizeof(int);
         RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_tile_rows), hipFuncAttributeMaxDynamicSharedMemorySize, (int)rows_lds));
         hipLaunchKernelGGL(k_tile_rows, dim3((unsigned)(nc << (w->cshift - w->fshift))), dim3(kTileThreads), rows_lds, stream, w->bin_eq,
                            w->bin_start, w->cshift, w->fshift, N, w->offs, w->rev);
@@ -1257,6 +1425,14 @@ int launch_reversed_graph(ExploreWorkspace* w, const int* old_idx, int N, int K,
     return 0;
 }
 
+}  // namespace
+
+// The reversed graph of idx (offs, rev).
+int launch_reversed_graph(ExploreWorkspace* w, const int* old_idx, int N, int K, hipStream_t stream)
+{
+    return launch_rev(w, old_idx, N, K, stream, false);
+}
+
 // Fill pass (and bounds) from the snapshot old_idx and the current last slots of knn_dist (rows sorted by distance).
 int launch_explore_join(ExploreWorkspace* w, const JoinCopy& jc, int N, int D, int K, const int* old_idx,
                         const float* knn_dist, hipStream_t stream, const int* order)
@@ -1264,7 +1440,6 @@ int launch_explore_join(ExploreWorkspace* w, const JoinCopy& jc, int N, int D, i
     RSFK_CHECK(w && w->N == N && w->K == K, "exploration join: workspace does not match");
     RSFK_CHECK(K >= 1 && K <= 256, "exploration join: K must be in 1..256");
     RSFK_CHECK((size_t)N * (size_t)K < kMaxEntries, "exploration join: N*K must be below 2^31 - 4096");
-    if (launch_reversed_graph(w, old_idx, N, K, stream)) return 1;
 
     constexpr int kWaves = 4;
     const int KP = (K + 31) & ~31;
@@ -1290,14 +1465,18 @@ int launch_explore_join(ExploreWorkspace* w, const JoinCopy& jc, int N, int D, i
     w->view.one_minus_gamma = one_minus_gamma;
     w->view.any_rel = any_rel;
     w->view.any_abs = any_abs;
-    hipLaunchKernelGGL(k_join_bars, dim3((unsigned)((N + 255) / 256) + 1), dim3(256), 0, stream, jc, jc.scale(), knn_dist, N, K,
-                       one_minus_gamma, w->bars, w->pass, (size_t)N * (size_t)K * (size_t)(KP >> 5));
-    RSFK_HIP(hipGetLastError());
     const int MW = KP >> 5;
+    const unsigned short_groups = grid_for_dies(((size_t)N * (size_t)MW + kWaves - 1) / kWaves);
+    const bool use_short = !w->bounds && ksteps <= 8 && launch_fits(short_groups, 64 * kWaves);
+    // (the records of the reversed graph's builder are done with: the words take the place of the last ones, and are sorted from there)
+    uint32_t* marks = use_short && w->staged && MW == 1 ? reinterpret_cast<uint32_t*>(w->bin_eq2) : nullptr;
+    hipLaunchKernelGGL(k_join_bars, dim3((unsigned)((N + 255) / 256) + 1), dim3(256), 0, stream, jc, jc.scale(), knn_dist, N, K,
+                       one_minus_gamma, w->bars, w->pass, marks ? 0 : (size_t)N * (size_t)K * (size_t)MW);
+    RSFK_HIP(hipGetLastError());
+    if (launch_rev(w, old_idx, N, K, stream, w->rev_bars && use_short)) return 1;
     // More points than a launch has threads for take a wavefront per q: with a wavefront per 32 neighbours K = 33 from 33.5 million points on, 129
     // from 13.4, 225 from 8.4, with a workgroup per q all from 16.8.
-    const unsigned short_groups = grid_for_dies(((size_t)N * (size_t)MW + kWaves - 1) / kWaves);
-    const bool short_fits = launch_fits(short_groups, 64 * kWaves), wg_fits = launch_fits(grid_for_dies((size_t)N), 256);
+    const bool wg_fits = launch_fits(grid_for_dies((size_t)N), 256);
     // One workgroup per q reads every row once per 96 points of R(q), one wavefront per q (and 32 neighbours) again for every group of 32
     // neighbours, so the former pays with the bytes that are read again, D (K - 24) or so, sooner with more groups; up to 32 neighbours
     // are one pair per tile of R(q), too little for four wavefronts (1M x 256, K = 32: 8.1 ms against 12.6).  A pass, a wavefront per q -> a
@@ -1321,11 +1500,11 @@ int launch_explore_join(ExploreWorkspace* w, const JoinCopy& jc, int N, int D, i
         else if (KP <= 128) RSFK_JOIN_WG(false, 3);
         else RSFK_JOIN_WG(false, 6);
 #undef RSFK_JOIN_WG
-    } else if (!w->bounds && ksteps <= 8 && short_fits) {
+    } else if (use_short) {
         const dim3 grid(short_groups, parts), block(64 * kWaves);
 #define RSFK_JOIN_SHORT(KSV, MANYV)                                                                                         \
         hipLaunchKernelGGL((k_explore_join_short<kWaves, KSV, MANYV>), grid, block, 0, stream, jc, N, K, old_idx, w->bars, w->offs, \
-                           w->rev, w->pass, MW, join_pitch(D), ksteps, kappa, any_rel, any_abs, w->div_m, w->div_s, order)
+                           w->rev, w->rev_bars, w->pass, marks, MW, join_pitch(D), ksteps, kappa, any_rel, any_abs, w->div_m, w->div_s, order)
         if (MW == 1 && ksteps <= 2) RSFK_JOIN_SHORT(2, false);
         else if (MW == 1 && ksteps <= 4) RSFK_JOIN_SHORT(4, false);
         else if (MW == 1) RSFK_JOIN_SHORT(8, false);
@@ -1333,6 +1512,24 @@ int launch_explore_join(ExploreWorkspace* w, const JoinCopy& jc, int N, int D, i
         else if (ksteps <= 4) RSFK_JOIN_SHORT(4, true);
         else RSFK_JOIN_SHORT(8, true);
 #undef RSFK_JOIN_SHORT
+        if (marks) {
+            const size_t total = (size_t)N * (size_t)K;
+            const int n_win = mark_windows(total), per = 1 << (kMarkWindow - kMarkPiece);
+            const unsigned pieces = (unsigned)(((total - 1) >> kMarkPiece) + 1);
+            int *by_window = w->sub_off, *by_piece = by_window + 32 * (size_t)n_win;
+            hipLaunchKernelGGL(k_mark_clear, dim3((unsigned)((mark_ints(total) + 255) / 256)), dim3(256), 0, stream, by_window, (int)mark_ints(total));
+            auto *to_windows = k_mark_scatter<true>, *to_pieces = k_mark_scatter<false>;
+            RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(to_windows), hipFuncAttributeMaxDynamicSharedMemorySize, (int)mark_lds_bytes(n_win)));
+            RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(to_pieces), hipFuncAttributeMaxDynamicSharedMemorySize, (int)mark_lds_bytes(per)));
+            // (two workgroups fit a compute unit)
+            const size_t tiles = (total + kMarkTile - 1) / kMarkTile;
+            hipLaunchKernelGGL(to_windows, dim3((unsigned)std::min<size_t>(tiles, 512)), dim3(kMarkThreads), mark_lds_bytes(n_win), stream,
+                               w->rev, marks, (const int2*)nullptr, w->offs + N, n_win, 32, by_window, w->bin_eq);
+            hipLaunchKernelGGL(to_pieces, dim3((unsigned)(1024 / n_win + 1), (unsigned)n_win), dim3(kMarkThreads), mark_lds_bytes(per), stream,
+                               (const int*)nullptr, (const uint32_t*)nullptr, w->bin_eq, by_window, per, 1, by_piece, w->bin_eq2);
+            RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_mark_place), hipFuncAttributeMaxDynamicSharedMemorySize, 4 << kMarkPiece));
+            hipLaunchKernelGGL(k_mark_place, dim3(pieces), dim3(kMarkThreads), 4 << kMarkPiece, stream, w->bin_eq2, by_piece, total, w->pass);
+        }
     } else if (w->bounds)
         hipLaunchKernelGGL((k_explore_join<kWaves, true>), dim3(grid_for_dies(((size_t)N + kWaves - 1) / kWaves), parts), dim3(64 * kWaves), lds,
                            stream, jc, N, K, old_idx, w->bars, w->offs, w->rev, w->pass, w->bounds, KP, join_pitch(D), ksteps,

@@ -664,6 +664,29 @@ def test_explore_with_the_reversed_graph_by_tiles(gpu, orc, rng, monkeypatch, N,
     assert_knn_equal(gi, gd, oi, od)
 
 
+@pytest.mark.parametrize("N,D,K", [(70001, 6, 31), (66000, 20, 32), (9001, 12, 3), (5000, 40, 1), (700, 33, 32), (2000, 20, 45)])
+def test_explore_with_the_staged_reversed_graph(gpu, orc, rng, monkeypatch, N, D, K):
+    """RSFK_REV_STAGED=1: marks put in place window by window (more than 2^21 of them, a last piece of any length, few), bars as 16-bit codes beside
+    the entries and, with few neighbours, gathered; rows that are not full; points far out, whose rounding errors are large.  More than 32
+    neighbours: marks stored one by one."""
+    monkeypatch.setenv("RSFK_REV_STAGED", "1")
+    X = rng.random((N, D), dtype=np.float32)
+    X[::97] *= 1000.0
+    oi, od = orc.init_lists(N, K, self_in=True)
+    perm, ls, lz, _ = orc.build_tree(X, K + 1, 2 * K + 2, 5000, 0)
+    orc.bucket_knn(X, K, perm, lz, oi, od, starts=ls)
+    if K > 2:
+        far = np.argsort(od, axis=1)[::7, -(K // 2):]
+        rows = np.arange(0, N, 7)[:, None]
+        oi[rows, far], od[rows, far] = -1, np.inf
+    gi, gd = oi.copy(), od.copy()
+    for _ in range(2):
+        _say("explore staged", N, D, K)
+        orc.explore(X, K, oi, od)
+        gpu.explore(X, K, gi, gd, 1)
+        assert_knn_equal(gi, gd, oi, od)
+
+
 @pytest.mark.parametrize("values", ["any", "whole", "near"])
 @pytest.mark.parametrize("N,D,K", [(1500, 6, 1), (3000, 3, 32), (3000, 33, 33), (2500, 130, 31), (2000, 8, 64), (1500, 200, 64), (1800, 20, 65),
                                    (1500, 12, 128), (1500, 140, 90), (1600, 10, 200)])
