@@ -550,7 +550,7 @@ __global__ __launch_bounds__(256) void k_ann_forest(const float* __restrict__ po
             n += __popcll(m);
             wave_lds_sync();
             if (n >= 64) {
-                exact_direct<SL>(L, list, 64, points, D, vec_ok, row);
+                exact_direct<SL>(L, list, 64, points, D, row);
                 n -= 64;
                 const int rest = lane < n ? list[64 + lane] : -1;
                 wave_lds_sync();
@@ -559,7 +559,7 @@ __global__ __launch_bounds__(256) void k_ann_forest(const float* __restrict__ po
             }
         }
     }
-    if (n > 0) exact_direct<SL>(L, list, n, points, D, vec_ok, row);
+    if (n > 0) exact_direct<SL>(L, list, n, points, D, row);
     if (wave > 0) {
 #pragma unroll
         for (int s = 0; s < SL; ++s) {

@@ -380,12 +380,14 @@ bool merge_direct(int D, int dpad, bool coded)
 // the marked ids, drop repeats and ids the row holds (hash set), exact distances, merge.  Points with
 // more marks than the LDS of this launch takes are appended to todo_out (for a launch with more LDS
 // per wavefront, or for the general kernel; share > 0: to the point's share of it, explore_ws_share_lists).  todo_in: the points to work on,
-// or null for all.  Per-wavefront LDS (ints): with TILE tile[64*20] | xrow[dpad] | table[table_size] | srow[K] | marked[3/4 table_size]
-// | with codes: tbound[table_size] | without TILE: the ranks (merge_rank_at).
-// TILE: the candidates' rows go through the transposing tile (not merge_direct); the two forms
-// are kernels of their own, so that the shorter one does not carry the registers of the other.
-template <int SL, int WAVES, bool TILE>
-__global__ __launch_bounds__(64 * WAVES) void k_explore_merge(const float* __restrict__ points, int N, int D, int K,
+// or null for all.  Per-wavefront LDS (ints): with the tile tile[64*20] | xrow[dpad] | table[table_size] | srow[K] | marked[3/4 table_size]
+// | with codes: tbound[table_size] | without the tile: the ranks (merge_rank_at).
+// kFormTile: the candidates' rows go through the transposing tile (not merge_direct).  The forms are kernels of their own, so that none carries
+// the registers of another: without the tile 75 without codes, held to the 72 of seven wavefronts per SIMD, 85 with codes, held to the 80 of six
+// (10M x 32 17.33 ms, 17.98 with six wavefronts, 24.2 with the 99 registers of code of its own choice; 1M x 256 5.65, 6.33 with seven).
+enum { kFormTile, kFormDirect, kFormDirectCoded };
+template <int SL, int WAVES, int FORM>
+__global__ __launch_bounds__(64 * WAVES, FORM == kFormTile || SL > 1 ? 1 : FORM == kFormDirect ? 7 : 6) void k_explore_merge(const float* __restrict__ points, int N, int D, int K,
                                                                const int* __restrict__ old_idx, int* __restrict__ knn_idx,
                                                                float* __restrict__ knn_dist, int table_size,
                                                                int wave_lds_ints, int dpad,
@@ -405,7 +407,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_merge(const float* __res
     // Rows of at most 64 neighbours (one slot per lane): everything the point needs from memory before its candidates
     // are known -- its K-NN row, the snapshot of its neighbours, its mark words, its coordinates -- is requested at once;
     // none of these addresses depends on another's data.  (Longer rows: one after the other, as they are needed.)
-    constexpr bool kEarly = SL == 1;
+    constexpr bool kEarly = SL == 1, TILE = FORM == kFormTile;
     KnnRow<SL> row;
     int q_own = -1;
     uint32_t pw[2] = {0u, 0u};
@@ -446,7 +448,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_merge(const float* __res
     L.queue2 = nullptr;
     L.table = base + tile_ints + dpad;
     L.srow = L.table + table_size;
-    const uint16_t* __restrict__ bounds = jb.codes;
+    const uint16_t* __restrict__ bounds = FORM == kFormDirect ? nullptr : jb.codes;
     // with bounds: the code of the id in the same place of the set, behind the list of marks
     int* tbound = bounds ? L.srow + K + table_size / 4 * 3 : nullptr;
     // without the tile: the ranks' working memory, in place of the list of marks or behind the bounds
@@ -549,7 +551,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_merge(const float* __res
     float reach = INFINITY;                               // what the row's last slot will be at most
     auto batch = [&](const int* list, int n) {
         n_exact += n;
-        if (!TILE) exact_direct<SL, true>(L, list, n, points, D, vec_ok, row, reach);
+        if (!TILE) exact_direct<SL, true>(L, list, n, points, D, row, reach);
         else exact_batch<SL, kMergeChunk, true, kChainGroup, true>(L, list, n, points, D, vec_ok, row, reach);    // two steps of gathers in flight
     };
     if (tbound == nullptr || U <= kFewCandidates) {
@@ -1075,19 +1077,11 @@ int launch_merge(const float* points, int N, int D, int K, const int* old_idx, i
     const size_t lds = (size_t)WAVES * (size_t)wave_ints * sizeof(int);
     const int n_work = todo_in ? n_in : N;
     dim3 grid(grid_for_dies(((size_t)n_work + WAVES - 1) / WAVES)), block(64 * WAVES);
-    if (direct) {
-        RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_explore_merge<SL, WAVES, false>),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        hipLaunchKernelGGL((k_explore_merge<SL, WAVES, false>), grid, block, lds, stream, points, N, D, K, old_idx, knn_idx,
-                           knn_dist, table, wave_ints, dpad, pass, bounds, todo_in, n_in, todo_out, share, n_out,
-                           stat, order);
-    } else {
-        RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_explore_merge<SL, WAVES, true>),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        hipLaunchKernelGGL((k_explore_merge<SL, WAVES, true>), grid, block, lds, stream, points, N, D, K, old_idx, knn_idx,
-                           knn_dist, table, wave_ints, dpad, pass, bounds, todo_in, n_in, todo_out, share, n_out,
-                           stat, order);
-    }
+    auto* kernel = !direct ? k_explore_merge<SL, WAVES, kFormTile> : bounds.codes ? k_explore_merge<SL, WAVES, kFormDirectCoded>
+                                                                                 : k_explore_merge<SL, WAVES, kFormDirect>;
+    RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(kernel, grid, block, lds, stream, points, N, D, K, old_idx, knn_idx, knn_dist, table, wave_ints, dpad, pass,
+                       bounds, todo_in, n_in, todo_out, share, n_out, stat, order);
     RSFK_HIP(hipGetLastError());
     return 0;
 }
