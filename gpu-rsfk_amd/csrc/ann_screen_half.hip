@@ -47,15 +47,6 @@ struct alignas(16) AnnHalfLds {
 };
 __device__ __forceinline__ int tile_at(int row, int piece) { return 8 * row + (piece ^ (row & 7)); }
 
-// 16 bytes per lane straight to LDS: lane l's to to[l] (to is the same for all lanes; lanes that are not active write nothing).
-__device__ __forceinline__ void load_to_lds(const void* from, u32x4* to)
-{
-    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)from, (__attribute__((address_space(3))) void*)to, 16, 0, 0);
-}
-// Waits for this wavefront's LDS operations, for its loads.
-__device__ __forceinline__ void wave_lds_drain() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
-__device__ __forceinline__ void wave_vm_drain() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-
 // The first n <= 64 pairs that wait: their distances, and those not above the last slot into the rows.
 __device__ __forceinline__ void evaluate(AnnHalfLds& L, int n, const float* __restrict__ points, const float* __restrict__ queries, int D, int K,
                                          bool vec, int* __restrict__ q_idx, float* __restrict__ q_dist)

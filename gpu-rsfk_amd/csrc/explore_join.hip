@@ -93,6 +93,7 @@ namespace {
 size_t todo_ints(int N) { return 2 * ((size_t)N + 1) + (size_t)kTodoShares * (size_t)todo_share(N) + 32 + 32 * (size_t)kTodoShares; }
 
 typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
+typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 
 constexpr int kMaxBins = 6144;
@@ -856,11 +857,13 @@ struct JoinSelf {
     __device__ __forceinline__ int find(int p) const { return at[p & (SIZE - 1)]; }     // (a column that may hold p, to be compared)
 };
 
-// One wavefront per q.  Per-wavefront LDS (ints): cq[KP] | pid[32] | reach[32] | pn[32] | perr[32] | pper[32] | pe[32] | self[64], KP = K rounded up to 32.
-// Workgroups (x, y): every gridDim.y-th tile of R(q), the y-th first.  (Five wavefronts per SIMD: 1M x 256 7.6 -> 7.0 ms against four
-// with the next 64 dimensions in flight.)
-template <int WAVES, bool BOUNDS>
-__global__ __launch_bounds__(64 * WAVES, 5) void k_explore_join(JoinCopy jc, int N, int K, const int* __restrict__ old_idx,
+// One wavefront per q.  Per-wavefront LDS (ints): cq[KP] | pid[32] | reach[32] | pn[32] | perr[32] | pper[32] | pe[32] | self[64] | LINES: rows[2][32] of 128 bytes, KP = K rounded up to 32.
+// Workgroups (x, y): every gridDim.y-th tile of R(q), the y-th first.
+// LINES: rows through LDS.  A lane that loads its 16 bytes of a row by itself asks for a line eight times, and the address units were busy 79 % of the
+// time; lines loaded whole cost a wavefront per SIMD and its LDS.  1M x 256 7.0 -> 6.57 ms, 300,000 x 200 1.64 -> 1.60, 100,000 x 784 1.97 -> 1.70, 60,000 x 200 with
+// K = 130 5.3 -> 4.6, 20,000 x 300 with K = 250 7.4 -> 5.3; 200,000 x 130 0.88 -> 0.95: from 161 dimensions on.
+template <int WAVES, bool BOUNDS, bool LINES>
+__global__ __launch_bounds__(64 * WAVES, LINES ? 4 : 5) void k_explore_join(JoinCopy jc, int N, int K, const int* __restrict__ old_idx,
                                                               const float* __restrict__ bars,
                                                               const int* __restrict__ offs, const int* __restrict__ rev,
                                                               uint32_t* __restrict__ pass, uint16_t* __restrict__ bounds, int KP, int bpitch, int ksteps,
@@ -882,6 +885,7 @@ __global__ __launch_bounds__(64 * WAVES, 5) void k_explore_join(JoinCopy jc, int
     float* pper = perr + 32;
     int* pe = reinterpret_cast<int*>(pper + 32);
     const JoinSelf<256> self{reinterpret_cast<uint8_t*>(pe + 32)};
+    u32x4* rows = reinterpret_cast<u32x4*>(pe + 32 + 64);
     const int MW = KP >> 5;
     const float most_norm = jc.mu[jc.D + 1], most_err = jc.mu[jc.D + 2];
 
@@ -909,23 +913,52 @@ __global__ __launch_bounds__(64 * WAVES, 5) void k_explore_join(JoinCopy jc, int
 
         const int pm = pid[lane & 31];
         const int own = pm >= 0 ? self.find(pm) % KP : 0, own_at = cq[own] == pm ? own : -1;    // place of p among the neighbours
-        const uint16_t* ra = jc.rows + (size_t)(pm >= 0 ? pm : q) * (size_t)bpitch + 8 * (lane >> 5);
         const int mbase = 4 * (lane >> 5);
         for (int ct = 0; ct < MW; ++ct) {
             const int cid = cq[ct * 32 + (lane & 31)];
+            const uint16_t* ra = jc.rows + (size_t)(pm >= 0 ? pm : q) * (size_t)bpitch + 8 * (lane >> 5);
             const uint16_t* rb = jc.rows + (size_t)(cid >= 0 ? cid : q) * (size_t)bpitch + 8 * (lane >> 5);
+            // LINES: 64 dimensions of the rows of the tile's points and of these neighbours at a time, eight lanes per row, whole lines (piece d of row r in
+            // place d ^ r % 8: eight lanes that read the same piece of eight rows meet no bank twice); the next 64 travel while the products are made
+            int id[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                if (!LINES) break;
+                id[i] = i < 4 ? pid[8 * i + (lane >> 3)] : cq[ct * 32 + 8 * (i - 4) + (lane >> 3)];
+                if (id[i] < 0) id[i] = q;
+            }
+            const int at = 8 * ((lane & 7) ^ (lane >> 3));
+            const auto fetch = [&](int k0) {
+                if (16 * k0 + at < bpitch) {
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) load_to_lds(jc.rows + (size_t)id[i] * (size_t)bpitch + 16 * k0 + at, rows + 64 * i);
+                }
+            };
             float an = 0.0f, cn = 0.0f;                   // norms of the row of point l % 32 of the tile and of neighbour l % 32
             f32x16 g;
 #pragma unroll
             for (int i = 0; i < 16; ++i) g[i] = 0.0f;
+            if (LINES) {
+                wave_lds_drain();
+                fetch(0);
+            }
             for (int k0 = 0; k0 < ksteps; k0 += 4) {
                 f16x8 a[4], b[4];
+                if (LINES) wave_vm_drain();
 #pragma unroll
                 for (int u = 0; u < 4; ++u) {
-                    if (k0 + u < ksteps) {
+                    if (LINES) {
+                        const int from = 8 * (lane & 31) + ((2 * u + (lane >> 5)) ^ (lane & 7));
+                        a[u] = *reinterpret_cast<const f16x8*>(rows + from);
+                        b[u] = *reinterpret_cast<const f16x8*>(rows + 256 + from);
+                    } else if (k0 + u < ksteps) {
                         a[u] = *reinterpret_cast<const f16x8*>(ra + 16 * (k0 + u));
                         b[u] = *reinterpret_cast<const f16x8*>(rb + 16 * (k0 + u));
                     }
+                }
+                if (LINES) {
+                    wave_lds_drain();
+                    if (k0 + 4 < ksteps) fetch(k0 + 4);
                 }
 #pragma unroll
                 for (int u = 0; u < 4; ++u) {
@@ -975,10 +1008,12 @@ __global__ __launch_bounds__(64 * WAVES, 5) void k_explore_join(JoinCopy jc, int
 // and stay in registers for all tiles of R(q); the norm and last slot of the points of a tile travel while their rows
 // are fetched.  A wavefront then has three dependent trips to memory per q (row offsets and neighbours | their rows
 // and the elements of R(q) | the rows of those points) instead of five, and short rows leave room for twice the
-// wavefronts per SIMD.  The bound is that of k_explore_join.  (Against it: 1M x 100, K = 48 a
+// wavefronts per SIMD.  With more than 32 dimensions the rows come by whole lines through LDS (as in k_explore_join: the address units were busy 72 % of the time
+// at 100 dimensions): 123,457 x 37, K = 45 0.367 -> 0.287 ms, 400,000 x 64 0.78 -> 0.59, 400,000 x 48, K = 60 1.80 -> 1.37, 200,000 x 100, K = 48 1.19 -> 0.96, 1M x
+// 100 2.86 -> 2.79; 10M x 32, which is at the rate of its lines, 12.0 -> 13.1 with a wavefront per SIMD less.  The bound is that of k_explore_join.  (Against it: 1M x 100, K = 48 a
 // pass 39.6 -> 37.9 ms, 1M x 24, K = 36 7.63 -> 7.39, 123,457 x 37, K = 45 1.49 -> 1.44.)
 template <int WAVES, int KS, bool MANY>
-__global__ __launch_bounds__(64 * WAVES) void k_explore_join_short(JoinCopy jc, int N, int K, const int* __restrict__ old_idx,
+__global__ __launch_bounds__(64 * WAVES, KS == 4 ? 7 : 1) void k_explore_join_short(JoinCopy jc, int N, int K, const int* __restrict__ old_idx,
                                                                     const float* __restrict__ bars,
                                                                     const int* __restrict__ offs, const int* __restrict__ rev,
                                                                     const uint16_t* __restrict__ rev_bars,
@@ -986,6 +1021,9 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_join_short(JoinCopy jc, 
                                                                     float kappa, float any_rel, float any_abs, uint32_t div_m, int div_s,
                                                                     const int* __restrict__ order)
 {
+    constexpr bool LINES = KS > 2;
+    constexpr int P = 2 * KS;                             // 16-byte pieces of a row in LDS
+    __shared__ u32x4 rows_s[WAVES][LINES ? 32 * P : 1];
     __shared__ int pid_s[WAVES][32];
     __shared__ __align__(16) float reach_s[WAVES][32];
     __shared__ uint8_t self_s[WAVES][128];
@@ -999,13 +1037,31 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_join_short(JoinCopy jc, 
     int cid = 32 * ct + col < K ? old_idx[(size_t)q * K + 32 * ct + col] : -1;
     if (R <= 32 * (int)blockIdx.y) return;
     if (cid < 0 || cid >= N) cid = -1;
+    int* pid = pid_s[wave];
+    u32x4* rows = rows_s[wave];
+    // LINES: the rows of the points in pid go to LDS, whole lines at a time (P lanes per row, KS loads): piece d of row r in place d ^ r % 8, so that eight
+    // lanes that read the same piece of eight rows meet no bank twice.
+    const auto fetch = [&]() {
+#pragma unroll
+        for (int i = 0; i < KS; ++i) {
+            const int r = (64 / P) * i + lane / P, piece = (lane % P) ^ (r & 7), id = pid[r];
+            if (KS <= 4 || 8 * piece < bpitch) load_to_lds(jc.rows + (size_t)(id >= 0 ? id : q) * (size_t)bpitch + 8 * piece, rows + 64 * i);
+        }
+    };
+    const auto from_lds = [&](int u) { return *reinterpret_cast<const f16x8*>(rows + col * P + ((2 * u + hi) ^ (col & 7))); };
     const uint16_t* rb = jc.rows + (size_t)(cid >= 0 ? cid : q) * (size_t)bpitch + 8 * hi;
+    if (LINES) {
+        if (lane < 32) pid[lane] = cid;
+        wave_lds_sync();
+        fetch();
+        wave_vm_drain();
+    }
     f16x8 b[KS];
 #pragma unroll
     for (int u = 0; u < KS; ++u) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) b[u][i] = (_Float16)0.0f;
-        if (KS <= 4 || u < ksteps) b[u] = *reinterpret_cast<const f16x8*>(rb + 16 * u);
+        if (KS <= 4 || u < ksteps) b[u] = LINES ? from_lds(u) : *reinterpret_cast<const f16x8*>(rb + 16 * u);
     }
     float cn = 0.0f;
 #pragma unroll
@@ -1017,7 +1073,6 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_join_short(JoinCopy jc, 
     const JoinSelf<128> self{self_s[wave]};
     self.put(cid, col);
     const int mbase = 4 * hi;
-    int* pid = pid_s[wave];
     float* reach = reach_s[wave];
 
     for (int pt0 = 32 * (int)blockIdx.y; pt0 < R; pt0 += 32 * (int)gridDim.y) {
@@ -1036,21 +1091,24 @@ __global__ __launch_bounds__(64 * WAVES) void k_explore_join_short(JoinCopy jc, 
         const int own = pm >= 0 ? self.find(pm) & 31 : 0;
         const bool own_there = __shfl(cid, own, 64) == pm && pm >= 0;                       // p is neighbour `own` of these
         const uint16_t* ra = jc.rows + (size_t)(pm >= 0 ? pm : q) * (size_t)bpitch + 8 * hi;
-        f16x8 a[KS];
-#pragma unroll
-        for (int u = 0; u < KS; ++u) {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) a[u][i] = (_Float16)0.0f;
-            if (KS <= 4 || u < ksteps) a[u] = *reinterpret_cast<const f16x8*>(ra + 16 * u);
+        if (LINES) {
+            wave_lds_drain();                             // (the rows before have been read)
+            fetch();
+            wave_vm_drain();
         }
         f32x16 g;
 #pragma unroll
         for (int i = 0; i < 16; ++i) g[i] = 0.0f;
-#pragma unroll
-        for (int u = 0; u < KS; ++u) g = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[u], b[u], g, 0, 0, 0);
         float an = 0.0f;
 #pragma unroll
-        for (int u = 0; u < KS; ++u) an = half_norm(a[u], an);
+        for (int u = 0; u < KS; ++u) {
+            if (KS <= 4 || u < ksteps) {
+                const f16x8 a = LINES ? from_lds(u) : *reinterpret_cast<const f16x8*>(ra + 16 * u);
+                g = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b[u], g, 0, 0, 0);
+                an = half_norm(a, an);
+            }
+            if ((u & 1) == 1) __builtin_amdgcn_sched_barrier(0);       // two steps at a time (registers)
+        }
         an += __shfl_xor(an, 32, 64);
         if (lane < 32) reach[lane] = join_reach(pm == q ? kNever : an, bar + e, kappa);
         wave_lds_sync();
@@ -1449,7 +1507,8 @@ int launch_explore_join(ExploreWorkspace* w, const JoinCopy& jc, int N, int D, i
     // 64 clusters 21,000 38 35 36 36, 26,000 45 42 42 44, 32,000 51 50 51 54, 45,000 67 68 73 76, 60,000 88 92 98 102; uniform x 100 21,000 70 71
     // 75 77, 32,000 96 103 110 114, 60,000 164 184 200 213.
     const unsigned parts = (unsigned)std::max(1, std::min(16, 65536 / N));
-    const int wave_ints = (KP + 256 + 3) & ~3;
+    const bool lines = D > 160;
+    const int wave_ints = KP + 256 + (lines ? 2 * 32 * 32 : 0);
     const size_t lds = (size_t)kWaves * (size_t)wave_ints * sizeof(int);
     const int ksteps = (D + 15) / 16;
     RSFK_CHECK(ksteps * 16 <= join_pitch(D), "exploration join: rows of the copy too short");
@@ -1530,14 +1589,13 @@ int launch_explore_join(ExploreWorkspace* w, const JoinCopy& jc, int N, int D, i
             RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_mark_place), hipFuncAttributeMaxDynamicSharedMemorySize, 4 << kMarkPiece));
             hipLaunchKernelGGL(k_mark_place, dim3(pieces), dim3(kMarkThreads), 4 << kMarkPiece, stream, w->bin_eq2, by_piece, total, w->pass);
         }
-    } else if (w->bounds)
-        hipLaunchKernelGGL((k_explore_join<kWaves, true>), dim3(grid_for_dies(((size_t)N + kWaves - 1) / kWaves), parts), dim3(64 * kWaves), lds,
-                           stream, jc, N, K, old_idx, w->bars, w->offs, w->rev, w->pass, w->bounds, KP, join_pitch(D), ksteps,
-                           kappa, any_rel, any_abs, wave_ints, w->div_m, w->div_s, order);
-    else
-        hipLaunchKernelGGL((k_explore_join<kWaves, false>), dim3(grid_for_dies(((size_t)N + kWaves - 1) / kWaves), parts), dim3(64 * kWaves), lds,
-                           stream, jc, N, K, old_idx, w->bars, w->offs, w->rev, w->pass, w->bounds, KP, join_pitch(D), ksteps,
-                           kappa, any_rel, any_abs, wave_ints, w->div_m, w->div_s, order);
+    } else {
+        auto* join = w->bounds ? (lines ? k_explore_join<kWaves, true, true> : k_explore_join<kWaves, true, false>)
+                               : (lines ? k_explore_join<kWaves, false, true> : k_explore_join<kWaves, false, false>);
+        hipLaunchKernelGGL(join, dim3(grid_for_dies(((size_t)N + kWaves - 1) / kWaves), parts), dim3(64 * kWaves), lds, stream, jc, N, K, old_idx,
+                           w->bars, w->offs, w->rev, w->pass, w->bounds, KP, join_pitch(D), ksteps, kappa, any_rel, any_abs, wave_ints,
+                           w->div_m, w->div_s, order);
+    }
     RSFK_HIP(hipGetLastError());
     return 0;
 }

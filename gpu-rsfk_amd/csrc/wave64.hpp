@@ -133,6 +133,15 @@ __device__ __forceinline__ void wave_lds_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// 16 bytes per lane straight to LDS: lane l's to 16 bytes from 16 l on (to is the same for all lanes; lanes that are not active write nothing).
+__device__ __forceinline__ void load_to_lds(const void* from, void* to)
+{
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)from, (__attribute__((address_space(3))) void*)to, 16, 0, 0);
+}
+// Waits for this wavefront's LDS operations, for its loads.
+__device__ __forceinline__ void wave_lds_drain() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+__device__ __forceinline__ void wave_vm_drain() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
 __device__ __forceinline__ int wave_sum_i(int v)
 {
     v += dpp_i<kDppXor1>(v);
