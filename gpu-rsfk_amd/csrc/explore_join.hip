@@ -407,7 +407,7 @@ __global__ __launch_bounds__(256) void k_staged_count2(const int2* __restrict__ 
     for (int s = blockIdx.x; s0 + (long long)s * kStSub < s1; s += gridDim.x) {
         for (int b = threadIdx.x; b < per; b += 256) hist2[b] = 0;
         __syncthreads();
-        const int a = s0 + s * kStSub, z = min(s1, a + kStSub);
+        const int a = s0 + s * kStSub, z = a + min(s1 - a, kStSub);
         for (int i = a + (int)threadIdx.x; i < z; i += 256) atomicAdd(&hist2[(rec1[i].y & low) >> fshift], 1);
         __syncthreads();
         const size_t row = (size_t)staged_sub_id(s0, cb, s) * per;
@@ -441,17 +441,17 @@ __global__ __launch_bounds__(kSt2Threads) void k_staged_scatter2(const int2* __r
     for (int s = blockIdx.x; s0 + (long long)s * kStSub < s1; s += gridDim.x) {
         const size_t row = (size_t)staged_sub_id(s0, cb, s) * per;
         for (int b = tid; b < per; b += kSt2Threads) cursor[b] = fine_start[(size_t)cb * per + b] + sub_off[row + b];
-        const int a = s0 + s * kStSub, z = min(s1, a + kStSub);
+        const int a = s0 + s * kStSub, n = min(s1 - a, kStSub);
         int2 r[kSt2Per];
         auto request = [&](int t0) {
 #pragma unroll
             for (int u = 0; u < kSt2Per; ++u) {
                 const int i = t0 + kSt2Threads * u + tid;
-                r[u] = i < z ? rec1[i] : make_int2(-1, 0);
+                r[u] = i < n ? rec1[(size_t)a + (size_t)i] : make_int2(-1, 0);
             }
         };
-        request(a);
-        for (int t0 = a; t0 < z; t0 += kSt2Tile) {
+        request(0);
+        for (int t0 = 0; t0 < n; t0 += kSt2Tile) {
             for (int b = tid; b < per; b += kSt2Threads) cnt[b] = 0;
             __syncthreads();
             int rank[kSt2Per];
@@ -468,7 +468,7 @@ __global__ __launch_bounds__(kSt2Threads) void k_staged_scatter2(const int2* __r
             for (int u = 0; u < kSt2Per; ++u)
                 if (r[u].x >= 0) stage[first[(r[u].y & low) >> fshift] + rank[u]] = r[u];
             __syncthreads();
-            if (t0 + kSt2Tile < z) request(t0 + kSt2Tile);
+            if (t0 + kSt2Tile < n) request(t0 + kSt2Tile);
             for (int i = tid; i < n_tile; i += kSt2Threads) {
                 const int2 x = stage[i];
                 const int b = (x.y & low) >> fshift;
