@@ -70,6 +70,7 @@ struct ExploreWorkspace {
     float* bars = nullptr;     // N: the bar the candidates of a point have to pass (k_join_bars)
     JoinBounds view;           // what the merge kernels read (set by launch_explore_join)
     uint16_t* bounds = nullptr; // N*K*32*MW codes of the marked pairs (join_bounds.hpp), or null
+    int direct = 0;             // the builder of small graphs: points of a workgroup, or 0
     bool tiled = false;         // the builder of medium graphs: bins of 2^cshift points, rows of 2^fshift of them at a time
     // the builder for large graphs (staged_rev_*): two scatters through LDS instead of one straight to memory
     bool staged = false;
@@ -99,6 +100,7 @@ typedef __attribute__((ext_vector_type(16))) float f32x16;
 constexpr int kMaxBins = 6144;
 constexpr int kMaxShift = 13;
 // entry numbers are ints, and the passes over the graph look 768 entries ahead of the one they test
+constexpr size_t kDirectMost = (size_t)1 << 18;
 constexpr size_t kMaxEntries = ((size_t)1 << 31) - 4096;
 constexpr int kRowsBlock = 512;             // threads of k_bin_rows
 
@@ -280,6 +282,95 @@ __global__ __launch_bounds__(kRowsBlock) void k_bin_rows(const int2* __restrict_
         const int at = atomicAdd(&cnt[eq.y], 1);
         rev[s0 + at] = eq.x;
     }
+}
+
+// ---------------------------------------------------------------------------
+// The same reversed graph for small inputs, in one launch.  What bounds the five above there is their launches.  A workgroup has `per` points and goes
+// through the whole graph (from the L2): it counts the entries of the points before its own, which is where its rows begin, and lists the numbers of its
+// own in LDS, which are then counted, scanned and placed; if they are more than fit, it goes through the graph twice more.
+// 3,000 x 30 13.4 us against 22 in five launches, the call (two passes) 748 -> 705; 10,000 x 32 17.2 against 25, 592 -> 579; 20,000 x 32 54 against 24, the call 1.72
+// ms with the five and 1.76 with the one: up to 2^18 entries.  (Bound by its instructions, six per entry in every workgroup: a branch and an addition per
+// entry 15.1, 20.6, 60 us; the next entries on their way, or workgroups that begin in different places, the same.)
+constexpr int kDirectThreads = 1024, kDirectCap = 8192, kDirectMostPer = 4096;
+typedef int i32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+
+__global__ __launch_bounds__(kDirectThreads) void k_rev_direct(const int* __restrict__ old_idx, int total, int N, int per, int* __restrict__ offs,
+                                                               int* __restrict__ rev, int* counter, int* shares)
+{
+    extern __shared__ int cnt[];                          // entries of each point, then where its next one goes
+    __shared__ int own[kDirectCap];
+    __shared__ int wave_lds[kDirectThreads / 64];
+    __shared__ int n_own;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int lo = blockIdx.x * per, n = min(N - lo, per);
+    if (blockIdx.x == 0) {
+        if (tid == 0) *counter = 0;
+        if (tid < kTodoShares) shares[32 * tid] = 0;
+    }
+    for (int i = tid; i < n; i += kDirectThreads) cnt[i] = 0;
+    if (tid == 0) n_own = 0;
+    __syncthreads();
+    int below = 0;
+    for (int t0 = 4 * tid; t0 < total; t0 += 16 * kDirectThreads) {
+        i32x4_a4 q[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int e = t0 + 4 * kDirectThreads * u;
+            if (e + 4 <= total) {
+                q[u] = *reinterpret_cast<const i32x4_a4*>(old_idx + e);
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) q[u][j] = e + j < total ? old_idx[e + j] : -1;
+            }
+        }
+        // (no branch per entry: one in `per` of N is this workgroup's, a few of the thousand of a wavefront)
+        uint32_t hits = 0;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const int c = q[i >> 2][i & 3];
+            below += (unsigned)c < (unsigned)lo ? 1 : 0;
+            hits |= (unsigned)(c - lo) < (unsigned)n ? 1u << i : 0u;
+        }
+        while (hits) {
+            const int i = __builtin_ctz(hits);
+            hits &= hits - 1;
+            const int at = atomicAdd(&n_own, 1);
+            if (at < kDirectCap) own[at] = t0 + 4 * kDirectThreads * (i >> 2) + (i & 3);
+        }
+    }
+    below = wave_sum_i(below);
+    if (lane == 0) wave_lds[wave] = below;
+    __syncthreads();
+    int begin = 0;
+    for (int w = 0; w < kDirectThreads / 64; ++w) begin += wave_lds[w];
+    const int m = n_own;
+    // calls f(entry, place of its point) for the workgroup's entries
+    const auto for_own = [&](auto f) {
+        if (m <= kDirectCap) {
+            for (int i = tid; i < m; i += kDirectThreads) f(own[i], old_idx[own[i]] - lo);
+        } else {
+            for (int e = tid; e < total; e += kDirectThreads) {
+                const int c = old_idx[e] - lo;
+                if ((unsigned)c < (unsigned)n) f(e, c);
+            }
+        }
+    };
+    for_own([&](int, int c) { atomicAdd(&cnt[c], 1); });
+    __syncthreads();
+    int carry = begin;
+    for (int c0 = 0; c0 < n; c0 += kDirectThreads) {
+        const int c = c0 + tid, v = c < n ? cnt[c] : 0;
+        int all;
+        const int ex = block_excl_scan(v, &all, wave_lds);
+        if (c < n) {
+            cnt[c] = carry + ex;
+            offs[lo + c] = carry + ex;
+        }
+        carry += all;
+    }
+    if (lo + n == N && tid == 0) offs[N] = carry;
+    __syncthreads();
+    for_own([&](int e, int c) { rev[atomicAdd(&cnt[c], 1)] = e; });
 }
 
 // ---------------------------------------------------------------------------
@@ -1356,6 +1447,12 @@ int explore_ws_alloc(ExploreWorkspace** out, int N, int K, bool with_bounds, boo
     while ((1 << l) < K) ++l;
     w->div_s = 31 + l;
     w->div_m = (uint32_t)((((uint64_t)1 << w->div_s) + (uint64_t)K - 1) / (uint64_t)K);
+    // Graphs of up to 2^18 entries (RSFK_REV_STAGED=3: of up to 2^21) take the builder of one launch.
+    {
+        const char* e = std::getenv("RSFK_REV_STAGED");
+        const int per = std::max(1, (N + 255) / 256);
+        if ((e && *e ? e[0] == '3' && total <= ((size_t)1 << 21) : total <= kDirectMost) && per <= kDirectMostPer) w->direct = per;
+    }
     // Graphs of 2^21 to 2^26 entries (RSFK_REV_STAGED=2: whenever the bins allow it) take the builder that sorts tiles in LDS.
     {
         const char* e = std::getenv("RSFK_REV_STAGED");
@@ -1470,7 +1567,10 @@ int launch_rev(ExploreWorkspace* w, const int* old_idx, int N, int K, hipStream_
     const int total = (int)((size_t)N * (size_t)K);
     const RevBars rb{w->bars, w->div_m, w->div_s};
     const size_t rows_lds = ((size_t)(1 << w->fshift) + kStRowsCap) * sizeof(int) + (with_bars ? kStRowsCap * sizeof(uint16_t) : 0);
-    if (w->staged) {
+    if (w->direct) {
+        hipLaunchKernelGGL(k_rev_direct, dim3((unsigned)((N + w->direct - 1) / w->direct)), dim3(kDirectThreads), (size_t)w->direct * sizeof(int), stream,
+                           old_idx, total, N, w->direct, w->offs, w->rev, w->todo + 2 * (size_t)N + 1, explore_ws_shares(w));
+    } else if (w->staged) {
         const int nc = w->n_coarse, per = 1 << (w->cshift - w->fshift);
         hipLaunchKernelGGL(k_zero, dim3((unsigned)((nc + 255) / 256)), dim3(256), 0, stream, w->bin_size, nc,
                            w->todo + 2 * (size_t)N + 1, explore_ws_shares(w));

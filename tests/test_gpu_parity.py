@@ -1822,6 +1822,13 @@ def test_symmetric_graph_forms(gpu, orc, rng, monkeypatch, N, K, hubs, staged):
     assert np.array_equal(gp, op) and np.array_equal(gc, oc) and np.array_equal(gv, ov)
 
 
+# The reversed graph in one launch (RSFK_REV_STAGED=3): a point per workgroup and many, a last workgroup with few, entries that are no multiple of four,
+# hubs with more entries than a workgroup keeps.
+@pytest.mark.parametrize("N,K,hubs", [(100, 7, 1), (257, 3, 0), (4003, 31, 2), (40000, 8, 5), (16500, 127, 0), (65537, 1, 0)])
+def test_symmetric_graph_of_one_launch(gpu, orc, rng, monkeypatch, N, K, hubs):
+    test_symmetric_graph_forms(gpu, orc, rng, monkeypatch, N, K, hubs, "3")
+
+
 # Points per wavefront by the points and the neighbours: two and four with rows of many neighbours, on either side of the lines.
 @pytest.mark.parametrize("N,K,hubs", [(31999, 32, 0), (32003, 32, 2), (31003, 31, 0), (15999, 32, 0), (16001, 32, 2), (16497, 33, 0), (16503, 33, 3), (32003, 64, 2)])
 def test_symmetric_graph_points_per_wavefront(gpu, orc, rng, monkeypatch, N, K, hubs):
