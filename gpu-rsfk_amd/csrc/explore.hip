@@ -1198,7 +1198,7 @@ int launch_explore(const float* points, const Bf16Copy* bf, const JoinCopy* jc, 
     const bool join = ws != nullptr && jc != nullptr && jc->rows != nullptr && explore_merge_fits(D, K);
     // (rows_sorted: the caller knows that every row is in order, e.g. after the bucket step of a forest)
     if (join && !rows_sorted && launch_sort_rows(knn_idx, knn_dist, N, K, stream)) return 1;
-    RSFK_HIP(hipMemcpyAsync(old_idx, knn_idx, sizeof(int) * (size_t)N * (size_t)K, hipMemcpyDeviceToDevice, stream));
+    if (!join) RSFK_HIP(hipMemcpyAsync(old_idx, knn_idx, sizeof(int) * (size_t)N * (size_t)K, hipMemcpyDeviceToDevice, stream));
     const int fixed = 64 * kPitch + dpad + kQueue2 + K;                 // ints per wavefront besides the set
     const int lds_ints = 150 * 1024 / 4;                                // usable LDS per workgroup
     // The set must hold the seeds (K+1) and all candidates of a group of neighbours with room to
@@ -1225,7 +1225,7 @@ int launch_explore(const float* points, const Bf16Copy* bf, const JoinCopy* jc, 
         // Marks from the join, then the merge kernel with a small set (little LDS, many wavefronts per CU).
         // The points it cannot take come back in a list and get a second launch with the largest set that
         // fits; what is left after that goes to the general kernel below.
-        if (launch_explore_join(ws, *jc, N, D, K, old_idx, knn_dist, stream, order)) return 1;
+        if (launch_explore_join(ws, *jc, N, D, K, knn_idx, old_idx, knn_dist, stream, order)) return 1;
         const uint32_t* pass = explore_ws_pass(ws);
         int* listA = explore_ws_todo(ws, 0);
         int* listB = explore_ws_todo(ws, 1);

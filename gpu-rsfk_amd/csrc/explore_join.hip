@@ -898,8 +898,10 @@ __global__ __launch_bounds__(256) void k_mark_clear(int* __restrict__ taken, int
 // The last workgroup has no points: it takes the largest norm and error of any finite row from the parts of them (join_copy.hip).
 // The others also clear the marks (words of them, none where they are put together: k_mark_place): the join stores the words that are not zero only.  A word stored somewhere in a large array is a
 // memory write of its own, twice the time of a line read (26 G a second; 87 G while the array fits the last cache).
+// And they take the snapshot of the neighbours: a launch less per pass (10M x 32 0.80 -> 0.77 ms for both, 1M x 100 0.094 either way; 10,000 x 32 the call 579 -> 573 us).
 __global__ __launch_bounds__(256) void k_join_bars(JoinCopy jc, float* __restrict__ scale, const float* __restrict__ knn_dist, int N, int K,
-                                                   float one_minus_gamma, float* __restrict__ out, uint32_t* __restrict__ pass, size_t words)
+                                                   float one_minus_gamma, float* __restrict__ out, uint32_t* __restrict__ pass, size_t words,
+                                                   const int* __restrict__ knn_idx, int* __restrict__ old_idx)
 {
     if (blockIdx.x + 1 == gridDim.x) {
         __shared__ float2 part[256];
@@ -929,6 +931,9 @@ __global__ __launch_bounds__(256) void k_join_bars(JoinCopy jc, float* __restric
         const size_t pieces = words >> 2, stride = (size_t)(gridDim.x - 1) * 256, first = (size_t)blockIdx.x * 256 + threadIdx.x;
         for (size_t i = first; i < pieces; i += stride) reinterpret_cast<uint4*>(pass)[i] = make_uint4(0u, 0u, 0u, 0u);
         if (first < (words & 3)) pass[4 * pieces + first] = 0u;
+        const size_t ids = (size_t)N * (size_t)K;
+        for (size_t i = first; i < ids >> 2; i += stride) reinterpret_cast<i32x4_a4*>(old_idx)[i] = reinterpret_cast<const i32x4_a4*>(knn_idx)[i];
+        if (first < (ids & 3)) old_idx[(ids & ~(size_t)3) + first] = knn_idx[(ids & ~(size_t)3) + first];
     }
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= N) return;
@@ -1634,8 +1639,8 @@ int launch_reversed_graph(ExploreWorkspace* w, const int* old_idx, int N, int K,
     return launch_rev(w, old_idx, N, K, stream, false);
 }
 
-// Fill pass (and bounds) from the snapshot old_idx and the current last slots of knn_dist (rows sorted by distance).
-int launch_explore_join(ExploreWorkspace* w, const JoinCopy& jc, int N, int D, int K, const int* old_idx,
+// Fill pass (and bounds) from the snapshot old_idx, which is made here, and the current last slots of knn_dist (rows sorted by distance).
+int launch_explore_join(ExploreWorkspace* w, const JoinCopy& jc, int N, int D, int K, const int* knn_idx, int* old_idx,
                         const float* knn_dist, hipStream_t stream, const int* order)
 {
     RSFK_CHECK(w && w->N == N && w->K == K, "exploration join: workspace does not match");
@@ -1673,7 +1678,7 @@ int launch_explore_join(ExploreWorkspace* w, const JoinCopy& jc, int N, int D, i
     // (the records of the reversed graph's builder are done with: the words take the place of the last ones, and are sorted from there)
     uint32_t* marks = use_short && w->staged && MW == 1 ? reinterpret_cast<uint32_t*>(w->bin_eq2) : nullptr;
     hipLaunchKernelGGL(k_join_bars, dim3((unsigned)((N + 255) / 256) + 1), dim3(256), 0, stream, jc, jc.scale(), knn_dist, N, K,
-                       one_minus_gamma, w->bars, w->pass, marks ? 0 : (size_t)N * (size_t)K * (size_t)MW);
+                       one_minus_gamma, w->bars, w->pass, marks ? 0 : (size_t)N * (size_t)K * (size_t)MW, knn_idx, old_idx);
     RSFK_HIP(hipGetLastError());
     if (launch_rev(w, old_idx, N, K, stream, w->rev_bars && use_short)) return 1;
     // More points than a launch has threads for take a wavefront per q: with a wavefront per 32 neighbours K = 33 from 33.5 million points on, 129

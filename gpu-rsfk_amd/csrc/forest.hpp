@@ -216,7 +216,7 @@ int* explore_ws_share_lists(ExploreWorkspace* w);
 int* explore_ws_shares(ExploreWorkspace* w);               // numbers, 32 words apart
 // order: null, or a permutation of the points that keeps nearby points together (the buckets of a tree): the points
 // are then worked on in that order, a contiguous eighth of it per die (die_local_place)
-int launch_explore_join(ExploreWorkspace* w, const JoinCopy& jc, int N, int D, int K, const int* old_idx,
+int launch_explore_join(ExploreWorkspace* w, const JoinCopy& jc, int N, int D, int K, const int* knn_idx, int* old_idx,
                         const float* knn_dist, hipStream_t stream, const int* order = nullptr);
 
 // explore.hip
