@@ -264,8 +264,8 @@ int knn_forest_device(int n_trees, int K, int N, int D, int MIN, int MAX, int MA
         DevBuf pair_stats;
         const size_t stat_words = (size_t)kFormWords * (size_t)n_trees;
         if (ws_alloc(&pair_stats.p, sizeof(unsigned long long) * stat_words)) return 1;
-        RSFK_HIP(hipMemsetAsync(pair_stats.p, 0, sizeof(unsigned long long) * stat_words, stream));
         unsigned long long* d_pairs = static_cast<unsigned long long*>(pair_stats.p);
+        bool pairs_counted = false;                      // (trees taken together leave no numbers: nothing to clear or to fetch)
         rep.screen_share_q16 = bucket_screen_share_q16();
         rep.rules.assign((size_t)n_trees, BucketFormRule{rep.screen_share_q16, 0, 0, 0});
         const int gram_from = bucket_gram_from();
@@ -330,7 +330,11 @@ int knn_forest_device(int n_trees, int K, int N, int D, int MIN, int MAX, int MA
                 }
                 if (rc) break;
                 rows_in_order = true;
-            } else if (!rows_in_order) {
+            } else if (!pairs_counted) {
+                RSFK_HIP(hipMemsetAsync(pair_stats.p, 0, sizeof(unsigned long long) * stat_words, stream));
+                pairs_counted = true;
+            }
+            if (!rows_in_order) {
                 // the bucket kernels read a row's maximum from its last slot: rows the caller passed in unsorted are
                 // put in order once
                 if (launch_sort_rows(d_idx, d_dist, N, K, stream)) return 1;
@@ -375,6 +379,9 @@ int knn_forest_device(int n_trees, int K, int N, int D, int MIN, int MAX, int MA
             if (big_pending) (void)hipStreamWaitEvent(stream, sync.big, 0);
             (void)hipEventRecord(ev[nb].e, stream);
             if (rc) break;
+            // (finished before the tree workspace goes back to the pool)
+            if (order.p && t0 + nb == n_trees)
+                RSFK_HIP(hipMemcpyAsync(order.p, tree_ws_perm(ws.w, (n_trees - 1) % B), sizeof(int) * (size_t)N, hipMemcpyDeviceToDevice, stream));
             RSFK_HIP(hipStreamSynchronize(stream));
             for (int j = 0; j < nb; ++j) {
                 float ms = 0.0f;
@@ -406,13 +413,9 @@ int knn_forest_device(int n_trees, int K, int N, int D, int MIN, int MAX, int MA
             }
         }
         if (rc) return rc;
-        if (order.p) {
-            // (finished before the tree workspace goes back to the pool)
-            RSFK_HIP(hipMemcpyAsync(order.p, tree_ws_perm(ws.w, (n_trees - 1) % B), sizeof(int) * (size_t)N, hipMemcpyDeviceToDevice, stream));
-            RSFK_HIP(hipStreamSynchronize(stream));
-        }
-        rep.form_words.resize(stat_words);
-        RSFK_HIP(hipMemcpy(rep.form_words.data(), d_pairs, sizeof(unsigned long long) * stat_words, hipMemcpyDeviceToHost));
+        rep.form_words.assign(stat_words, 0);
+        if (pairs_counted)
+            RSFK_HIP(hipMemcpy(rep.form_words.data(), d_pairs, sizeof(unsigned long long) * stat_words, hipMemcpyDeviceToHost));
     }
     const double t_forest = now_s() - t_forest0;
     if (verbose >= 1) std::printf("Creating RSFK forest takes %lf seconds\n", t_forest);
@@ -437,10 +440,10 @@ int knn_forest_device(int n_trees, int K, int N, int D, int MIN, int MAX, int MA
                                n_trees == 1 && it == 0))
                 return 1;
         }
-        std::vector<unsigned long long> h_stat((size_t)kExploreStatWords);
-        RSFK_HIP(hipMemcpyAsync(h_stat.data(), stat.p, sizeof(unsigned long long) * kExploreStatWords, hipMemcpyDeviceToHost, stream));
-        RSFK_HIP(hipStreamSynchronize(stream));
-        for (int i = 0; i < kExploreStatWords; i += 32) rep.exact += h_stat[(size_t)i];
+        // (one word in pinned memory: a copy of the counters' 64 KB is a trip of its own)
+        unsigned long long exact = 0;
+        if (fetch_total(static_cast<const unsigned long long*>(stat.p), kExploreStatWords / 32, 32, &exact, stream)) return 1;
+        rep.exact += exact;
     }
     const double t_exp = now_s() - t_exp0;
     if (verbose >= 1) std::printf("Nearest Neighbors Exploring computation Kernel takes %lf seconds\n", t_exp);

@@ -33,6 +33,7 @@ constexpr int kFetchMost = 8;
 int fetch_words(const int* a, int na, const int* b, int nb, int* host, hipStream_t stream);
 // *host = sum of the n <= 64 words a[0], a[pitch], ..
 int fetch_total(const int* a, int n, int pitch, int* host, hipStream_t stream);
+int fetch_total(const unsigned long long* a, int n, int pitch, unsigned long long* host, hipStream_t stream);
 inline int fetch_words(const int* dev, int n, int* host, hipStream_t stream) { return fetch_words(dev, n, nullptr, 0, host, stream); }
 // ... the sum of n numbers there.
 int fetch_sum(const float* a, int n, float* host, hipStream_t stream);

@@ -297,6 +297,23 @@ __global__ void k_fetch_total(const int* __restrict__ a, int n, int pitch, Fetch
     __hip_atomic_store(&out->seq, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 // One workgroup of 256 threads.
+__global__ void k_fetch_total64(const unsigned long long* __restrict__ a, int n, int pitch, Fetched* out)
+{
+    __shared__ unsigned long long part[256];
+    unsigned long long t = 0;
+    for (int i = threadIdx.x; i < n; i += 256) t += a[(size_t)i * (size_t)pitch];
+    part[threadIdx.x] = t;
+    __syncthreads();
+    for (int o = 128; o > 0; o >>= 1) {
+        if ((int)threadIdx.x < o) part[threadIdx.x] += part[threadIdx.x + o];
+        __syncthreads();
+    }
+    if (threadIdx.x != 0) return;
+    out->word[0] = (int)(unsigned)part[0];
+    out->word[1] = (int)(unsigned)(part[0] >> 32);
+    __hip_atomic_store(&out->seq, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+// One workgroup of 256 threads.
 __global__ void k_fetch_sum(const float* __restrict__ a, int n, Fetched* out)
 {
     __shared__ float part[256];
@@ -343,6 +360,21 @@ int fetch_total(const int* a, int n, int pitch, int* host, hipStream_t stream)
     const int rc = e != hipSuccess ? 1 : wait_for_word(&f->seq, 1, stream);
     if (e != hipSuccess) set_last_error(std::string("fetch: ") + hipGetErrorString(e));
     if (!rc) *host = f->word[0];
+    pin_free(p);
+    return rc;
+}
+
+int fetch_total(const unsigned long long* a, int n, int pitch, unsigned long long* host, hipStream_t stream)
+{
+    void* p = nullptr;
+    if (pin_alloc(&p, sizeof(Fetched))) return 1;
+    Fetched* f = static_cast<Fetched*>(p);
+    __atomic_store_n(&f->seq, 0, __ATOMIC_RELEASE);
+    hipLaunchKernelGGL(k_fetch_total64, dim3(1), dim3(256), 0, stream, a, n, pitch, f);
+    const hipError_t e = hipGetLastError();
+    const int rc = e != hipSuccess ? 1 : wait_for_word(&f->seq, 1, stream);
+    if (e != hipSuccess) set_last_error(std::string("fetch: ") + hipGetErrorString(e));
+    if (!rc) *host = (unsigned)f->word[0] | (unsigned long long)(unsigned)f->word[1] << 32;
     pin_free(p);
     return rc;
 }
