@@ -64,6 +64,7 @@ struct LevelCounters {
     } queue[4];
     int n_tail;        // tail tasks appended so far
     int n_mid;         // ... and tasks of the middle phase
+    int n_mid_next[2]; // ... of its second and its third launch
     int n_chain;       // nodes for the chain phase appended so far, at the front of their queue
     int n_chain_back;  // ... and at its back: those that are hardly split in vain
     int overflow;      // set when a queue capacity is exceeded
@@ -1355,9 +1356,10 @@ __global__ __launch_bounds__(TB, CHAIN ? 4 : 6) void k_tail(const float* __restr
 constexpr int kMidMost = 12288;          // points (LDS: 4 bytes of permutation and 2 of the list of undecided points each)
 constexpr int kMidThreads = 1024, kMidPer = kMidMost / kMidThreads;
 constexpr int kMidOut = 64;              // nodes for the tail kernel kept before they are given a place in its queue
+constexpr int kMidNext = 2;
 
 struct MidNode : SmallNode {
-    int leaf;                             // a bucket, or to be one at the depth limit
+    int leaf;                             // 1: a bucket, or to be one at the depth limit; kMidNext: for the next launch
 };
 
 template <int LPP, int KU>
@@ -1365,7 +1367,8 @@ __global__ __launch_bounds__(kMidThreads, 4) void k_mid(const float* __restrict_
                                                         const int* __restrict__ perm0, const int* __restrict__ perm1, int* __restrict__ perm_out,
                                                         const TreeNode* __restrict__ tasks, TreeNode* __restrict__ tail, int tail_cap, int stack_cap,
                                                         TreeStats* stats, LevelCounters* ctr, TreeRec* __restrict__ recs_all, int rec_cap,
-                                                        unsigned long long* __restrict__ stat)
+                                                        unsigned long long* __restrict__ stat, const int* n_tasks, TreeNode* __restrict__ next,
+                                                        int* n_next, int next_cap)
 {
     // dynamic LDS: seg[most] | nvec[nvec_len(D)] | nodes to split [stack_cap] | nodes for the tail [kMidOut] | undecided points [most]
     extern __shared__ __align__(16) unsigned char mid_lds[];
@@ -1376,8 +1379,9 @@ __global__ __launch_bounds__(kMidThreads, 4) void k_mid(const float* __restrict_
     uint16_t* list = reinterpret_cast<uint16_t*>(out + kMidOut);
     constexpr int kWaves = kMidThreads / 64;
     __shared__ float hp_s[4];
-    __shared__ int count_s[kMidPer * kWaves], all_s, n_def_s, n_stack_s, n_out_s, out_base_s;
+    __shared__ int count_s[kMidPer * kWaves], all_s, n_def_s, n_stack_s, n_out_s;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (n_tasks && (int)blockIdx.x >= *n_tasks) return;
     if (blockIdx.x == 0 && tid == 0) phase_tick(ctr, 2);
     const TreeNode tk = tasks[blockIdx.x];
     if (tk.leaf || tk.count <= P.small) {
@@ -1400,19 +1404,24 @@ __global__ __launch_bounds__(kMidThreads, 4) void k_mid(const float* __restrict_
         n_out_s = 0;
     }
     __syncthreads();
-    // the nodes that wait for the tail kernel get their places (all threads call)
+    // the nodes that wait for the tail kernel, or for the next launch, get their places (all threads call)
     auto give_out = [&]() {
         const int n = n_out_s;
-        if (tid == 0) out_base_s = n ? atomicAdd(&ctr->n_tail, n) : 0;
-        __syncthreads();
-        for (int i = tid; i < n; i += kMidThreads) {
-            const MidNode sn = out[i];
+        if (tid < n) {
+            const MidNode sn = out[tid];
             TreeNode c;
             c.tree = tk.tree; c.start = tk.start + sn.start; c.count = sn.count; c.dstart = tk.start + sn.dstart; c.dcount = sn.dcount;
             c.depth = sn.depth; c.buf = 0; c.leaf = sn.leaf; c.rec = sn.rec; c.chunk0 = 0; c.key = sn.key;
-            const int at = out_base_s + i;
-            if (at < tail_cap) tail[at] = c; else ctr->overflow = 1;
+            if (sn.leaf == kMidNext) {
+                c.leaf = 0;
+                const int at = atomicAdd(n_next, 1);
+                if (at < next_cap) next[at] = c; else ctr->overflow = 1;
+            } else {
+                const int at = atomicAdd(&ctr->n_tail, 1);
+                if (at < tail_cap) tail[at] = c; else ctr->overflow = 1;
+            }
         }
+        __syncthreads();
         if (tid == 0) n_out_s = 0;
         __syncthreads();
     };
@@ -1524,7 +1533,8 @@ __global__ __launch_bounds__(kMidThreads, 4) void k_mid(const float* __restrict_
                 MidNode x;
                 x.start = c.start; x.count = c.count; x.dstart = c.dstart; x.dcount = c.dcount;
                 x.depth = c.depth; x.leaf = c.leaf || forced ? 1 : 0; x.rec = c.rec; x.key = c.key;
-                if (!split) out[n_out++] = x;
+                if (split && next) x.leaf = kMidNext;
+                if (!split || next) out[n_out++] = x;
                 else if (n_left < stack_cap) stack[n_left++] = x;
                 else ctr->overflow = 1;
             };
@@ -2378,6 +2388,7 @@ struct TreeBatchWorkspace {
     TreeNode* chain = nullptr;           // nodes for the chain phase
     TreeNode* mid = nullptr;             // nodes for the middle phase (when there is one)
     int mid_most = 0;                    // points of the largest of them
+    TreeNode* mid_next = nullptr;        // nodes for its second launch, and for its third: tail_cap each
     int* chunk2node = nullptr;
     int* chunk_left = nullptr;
     float* planes = nullptr;             // hyperplanes of the nodes of the current wide level: node_cap x (4 + nvec_len(D))
@@ -2410,7 +2421,7 @@ struct TreeBatchWorkspace {
 
 static void free_ws(TreeBatchWorkspace& w)
 {
-    void* dev[] = {w.perm[0], w.perm[1], w.nodes[0], w.nodes[1], w.tail, w.chain, w.mid, w.chunk2node,
+    void* dev[] = {w.perm[0], w.perm[1], w.nodes[0], w.nodes[1], w.tail, w.chain, w.mid, w.mid_next, w.chunk2node,
                    w.chunk_left, w.leaf_start, w.leaf_size, w.stats, w.ctr, w.recs, w.planes, w.side_ops,
                    w.pm_path, w.pm_side, w.pm_undec, w.pm_map[0], w.pm_map[1], w.pm_sc, w.pm_aq, w.pm_child, w.stat};
     for (void* p : dev) ws_free(p);
@@ -2515,7 +2526,7 @@ int tree_ws_alloc(TreeBatchWorkspace** out, int N, int D, int MIN, int B)
     if (dmalloc(&w->tail, (size_t)w->tail_cap)) return 1;
     if (dmalloc(&w->chain, (size_t)w->tail_cap)) return 1;
     w->mid_most = tree_mid_most(D, N, B, small);
-    if (w->mid_most && dmalloc(&w->mid, (size_t)w->tail_cap)) return 1;
+    if (w->mid_most && (dmalloc(&w->mid, (size_t)w->tail_cap) || dmalloc(&w->mid_next, 2 * (size_t)w->tail_cap))) return 1;
     if (dmalloc(&w->chunk2node, (size_t)w->chunk_cap)) return 1;
     if (dmalloc(&w->chunk_left, (size_t)w->chunk_cap)) return 1;
     if (dmalloc(&w->planes, (size_t)w->node_cap * (size_t)(4 + nvec_len(D)))) return 1;
@@ -2712,20 +2723,36 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
         const int stack_cap = w->mid_most / std::max(P.small, 1) + 4;
         const size_t lds = (size_t)w->mid_most * 6 + (size_t)nvec_len(D) * 4 + (size_t)(stack_cap + kMidOut) * sizeof(MidNode);
         const int pieces = q8_padded(D) / 16;
+        // A workgroup splits one node after the other, about 10 us each; while several of its descendants will be larger than P.small, a launch ends
+        // with the children, which the next one takes side by side.
+        // One tree of 10,000 x 2 73 us in one launch, 19 + 15 + 25 in three, the call 187 -> 178; 10,000 x 32, 4 trees 86 -> 78, the call the same; with
+        // two launches 72 and 81 (the halves are rarely alike).  Not with many nodes, when those of the last launch wait for each other's compute units: 20,000 x
+        // 32, 50 trees 111 -> 125 us.
+        int hand = 0;
+        if (n_tail <= 64)
+            for (int m = std::min(N, w->mid_most); m > 2 * P.small && hand < 2; m /= 2) ++hand;
+        for (int pass = 0; pass <= hand; ++pass) {
+            const TreeNode* tasks = pass == 0 ? w->mid : w->mid_next + (size_t)(pass - 1) * (size_t)w->tail_cap;
+            const int* n_tasks = pass == 0 ? nullptr : &w->ctr->n_mid_next[pass - 1];
+            TreeNode* next = pass == hand ? nullptr : w->mid_next + (size_t)pass * (size_t)w->tail_cap;
+            // (nodes above P.small, no two with a point in common; two at most from each of the launch before)
+            const unsigned grid = pass == 0 ? (unsigned)n_tail
+                                            : (unsigned)std::max<size_t>(1, std::min((size_t)n_tail << pass, (size_t)N * (size_t)nb / (size_t)(P.small + 1)));
 #define RSFK_MID_LAUNCH(L, U)                                                                                               \
         do {                                                                                                               \
             RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_mid<L, U>),                                       \
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));                          \
-            hipLaunchKernelGGL((k_mid<L, U>), dim3(n_tail), dim3(kMidThreads), lds, stream, points, q8, P, w->mid_most,     \
-                               w->perm[0], w->perm[1], w->perm[0], w->mid, w->tail, w->tail_cap, stack_cap, w->stats, w->ctr,  \
-                               w->recs, w->rec_cap, w->stat);                                                               \
+            hipLaunchKernelGGL((k_mid<L, U>), dim3(grid), dim3(kMidThreads), lds, stream, points, q8, P, w->mid_most,     \
+                               w->perm[0], w->perm[1], w->perm[0], tasks, w->tail, w->tail_cap, stack_cap, w->stats, w->ctr,  \
+                               w->recs, w->rec_cap, w->stat, n_tasks, next, pass < hand ? &w->ctr->n_mid_next[pass] : nullptr, w->tail_cap); \
         } while (0)
-        if (pieces <= 2) RSFK_MID_LAUNCH(2, 1);
-        else if (pieces <= 4) RSFK_MID_LAUNCH(4, 1);
-        else if (pieces <= 16) RSFK_MID_LAUNCH(4, 4);
-        else RSFK_MID_LAUNCH(8, 4);
+            if (pieces <= 2) RSFK_MID_LAUNCH(2, 1);
+            else if (pieces <= 4) RSFK_MID_LAUNCH(4, 1);
+            else if (pieces <= 16) RSFK_MID_LAUNCH(4, 4);
+            else RSFK_MID_LAUNCH(8, 4);
 #undef RSFK_MID_LAUNCH
-        RSFK_HIP(hipGetLastError());
+            RSFK_HIP(hipGetLastError());
+        }
         // (how many nodes it leaves to the tail only the device knows; that many are usual, and the tail kernel takes any number)
         n_tail = (int)std::min<size_t>((size_t)N * (size_t)nb * 5 / (size_t)(3 * P.small) + (size_t)nb, (size_t)w->tail_cap);
     }

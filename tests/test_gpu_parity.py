@@ -194,6 +194,23 @@ def test_tree_wide_levels_by_the_8_bit_copy(gpu, orc, rng, monkeypatch, D, kind)
     assert np.array_equal(gls, ls) and np.array_equal(glz, lz)
 
 
+# The middle phase in one, two and three launches: largest nodes of up to twice the tail's, of one point more, of more than four times as many; nodes
+# of a tree that stay above the tail's size after the last of them; many equal rows, whose nodes lose a few points at a time.
+@pytest.mark.parametrize("N", [512, 513, 1025, 1100, 4000, 12000])
+@pytest.mark.parametrize("D,kind", [(2, "n"), (40, "n"), (70, "n"), (300, "n"), (5, "dup")])
+def test_tree_middle_phase_by_launches(gpu, orc, rng, monkeypatch, N, D, kind):
+    for name, v in (("SCREEN", "q8"), ("SMALL", "256")):
+        monkeypatch.setenv("RSFK_TREE_" + name, v)
+    X = rng.standard_normal((N, D)).astype(np.float32)
+    if kind == "dup":
+        X[: N // 3] = X[0]
+    _say("tree middle phase", N, D, kind)
+    perm, ls, lz, st = orc.build_tree(X, 17, 34, 100, 5)
+    gperm, gls, glz, gst = gpu.build_tree(X, 17, 34, 100, 5)
+    assert np.array_equal(gperm, perm)
+    assert np.array_equal(gls, ls) and np.array_equal(glz, lz)
+
+
 # The forms of the tail and of the chain phase: leaf limits on either side of the sizes of the chain's matrix (nodes of up to 64, 128
 # and 256 points, and none), rows on either side of the lanes that share one, many subtrees (nodes above `small` points are wide) and
 # few; rows without distances (NaN, and a few far longer than the others), clusters within one node, the index that query points
