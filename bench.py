@@ -448,7 +448,7 @@ def main():
         R = report["tree_screen_row_bytes"]
         tb = (report["tree_points_tested"] * (R + 16.0) + report["tree_points_undecided"] * 4.0 * D) / T + 4.0 * N
         ach = tb / tree_s / 1e9 if tree_s > 0 else 0.0
-        roofline_tree = {"kernel": "tree build of one tree (k_pm_sweep / k_side, k_scatter, k_tail; trees are built in batches, level by level)",
+        roofline_tree = {"kernel": "tree build of one tree (k_pm_sweep / k_side_q8, k_scatter, k_tail; trees are built in batches, level by level)",
                          "bound": "hbm", "achieved": round(ach, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                          "frac": round(ach / HBM_PEAK_GBS, 4), "traffic": None, "algorithmic_bytes_per_launch": round(tb),
                          "avg_launch_ms": round(tree_s * 1e3, 4), "launches_per_step": T,

@@ -401,7 +401,7 @@ int knn_forest_device(int n_trees, int K, int N, int D, int MIN, int MAX, int MA
                     log_forest[(size_t)5 * n_trees + t] = (float)(tb / nb);          // Total Tree Building Time
                     // the trees of a batch are built together, level by level: a tree's share of the batch's kernels
                     const float* ph = tree_ws_phase_seconds(ws.w);
-                    log_forest[(size_t)7 * n_trees + t] = ph[0] / nb;                // Check Points Side Time (k_side)
+                    log_forest[(size_t)7 * n_trees + t] = ph[0] / nb;                // Check Points Side Time (k_side_q8)
                     log_forest[(size_t)11 * n_trees + t] = ph[1] / nb;               // Create Nodes Time (k_level_planes)
                     log_forest[(size_t)12 * n_trees + t] = ph[2] / nb;               // Update Nodes Time (k_scatter)
                     log_forest[(size_t)13 * n_trees + t] = ph[3] / nb;               // Bucket Creation Time (k_tail)

@@ -900,7 +900,7 @@ __global__ __launch_bounds__(kBlock) void k_scatter(TreeParams P, int* __restric
     }
 }
 
-// What k_side leaves behind, from sides that are already known (one bit per point of the tree, pm::k_pm_sweep and
+// What k_side_q8 leaves behind, from sides that are already known (one bit per point of the tree, pm::k_pm_sweep and
 // pm::k_pm_resolve): bit 31 of the permutation entries of a chunk and the number of its left members.
 __global__ __launch_bounds__(kBlock) void k_pm_mark(TreeParams P, int* __restrict__ perm0, int* __restrict__ perm1,
                                                     const TreeNode* __restrict__ nodes, const int* __restrict__ n_chunks,
@@ -1004,7 +1004,7 @@ constexpr int kMaxGroup = 16;        // nodes of one level of a subtree worked o
 // most of the device idle (the phases of a level then have more lanes).  CHAIN: nodes of at most P.chain_max points go
 // to the queue of the chain phase; otherwise those of them that have been split in vain kVainMost times in a row.  The form of 256 threads is for many subtrees and lives by six wavefronts per SIMD, for which
 // it has to stay within 80 registers (81 and five wavefronts: 1M x 100, 50 trees 10.8 -> 12.3 ms).
-// LPP: lanes per point in the screen (k_side), eight with the bfloat16 copy; KU: 16-byte pieces of a point's row each of them has in
+// LPP: lanes per point in the screen (side_screen8), eight with the bfloat16 copy; KU: 16-byte pieces of a point's row each of them has in
 // flight.
 template <bool Q8, int TB, bool CHAIN, int LPP, int KU>
 __global__ __launch_bounds__(TB, CHAIN ? 4 : 6) void k_tail(const float* __restrict__ points,

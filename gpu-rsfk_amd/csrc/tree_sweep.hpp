@@ -2,7 +2,7 @@
 //
 // At the first levels of a tree every point is a member of a node that is still being split
 // (build_tree_check_points_side.cu:131-149 tests each of them against the hyperplane of its node), and a batch of
-// trees has few nodes per level: 2^l per tree.  The node-by-node kernel (k_side) gathers the screening row of every
+// trees has few nodes per level: 2^l per tree.  The node-by-node kernel (k_side_q8) gathers the screening row of every
 // point once per tree and level, in the order of the tree's permutation.  Here the rows are streamed once per level
 // in their natural order for all trees of the batch, and the tests become small integer matrix products on the
 // matrix cores:
@@ -22,7 +22,7 @@
 //     to the tail queue need no special case in the sweep.
 //
 // The sides are left as one bit per point and tree; k_pm_mark writes them into the permutation entries and counts
-// the left members of every chunk, which is what k_side leaves for k_scatter.
+// the left members of every chunk, which is what k_side_q8 leaves for k_scatter.
 #pragma once
 #include "rsfk_common.hpp"
 #include "wave64.hpp"
