@@ -502,7 +502,8 @@ __global__ __launch_bounds__(256) void k_ann_leaf(const float* __restrict__ poin
 // k_planes and k_route (six launches a tree before: 1,780 us).
 constexpr int kAnnSeen = 1024;
 constexpr int kAnnList = 128;         // of a wavefront: fewer than 64 waiting and up to 64 new ones
-template <int SL>
+// QUADS: how the rows are read (exact_direct; the rule is at the launch).
+template <int SL, bool QUADS>
 __global__ __launch_bounds__(256) void k_ann_forest(const float* __restrict__ points, const float* __restrict__ queries, int N, int D,
                                                     int K, int T, const int* __restrict__ perm, const int2* __restrict__ reached,
                                                     bool vec_ok, int dpad, int* __restrict__ q_idx, float* __restrict__ q_dist)
@@ -550,7 +551,7 @@ __global__ __launch_bounds__(256) void k_ann_forest(const float* __restrict__ po
             n += __popcll(m);
             wave_lds_sync();
             if (n >= 64) {
-                exact_direct<SL>(L, list, 64, points, D, row);
+                exact_direct<SL, QUADS>(L, list, 64, points, D, vec_ok, row);
                 n -= 64;
                 const int rest = lane < n ? list[64 + lane] : -1;
                 wave_lds_sync();
@@ -559,7 +560,7 @@ __global__ __launch_bounds__(256) void k_ann_forest(const float* __restrict__ po
             }
         }
     }
-    if (n > 0) exact_direct<SL>(L, list, n, points, D, row);
+    if (n > 0) exact_direct<SL, QUADS>(L, list, n, points, D, vec_ok, row);
     if (wave > 0) {
 #pragma unroll
         for (int s = 0; s < SL; ++s) {
@@ -804,9 +805,17 @@ int launch_ann_forest(const float* points, const float* queries, int N, int NQ, 
     const bool vec_p = (D & 3) == 0 && (reinterpret_cast<uintptr_t>(points) & 15) == 0;
     const int dpad = (D + 31) & ~31;
     const size_t lds = ann_forest_lds(D, K);
+    // Rows of a few lines in an L2 are read sooner by a lane each: four lanes that exchange what they load take more instructions, and save
+    // requests that only count where there are many, from farther away.  A call, own rows -> quads, K = 16, 50 trees, 10,000 queries: 5,000 x 24 +7 %, x 48 -1,
+    // x 60 -7, x 96 -14; 40,000 x 24 +2, x 48 -9, x 96 -16; 1,000 x 64 0; K = 10, 12 trees, 10,000 queries: 5,000 x 24 +4, x 72 +3, 3,000 x 150 -6; K = 16, 20
+    // trees, 8,000 queries: 3,000 x 56 +4, 20,000 x 56 -4, 20,000 x 112 -14; K = 10, 20 trees: 2,000 x 100 +3 to +5; K = 107, 50 trees, 62,271 queries: 1,909 x 3 +29.
+    const bool quads = D > 128 || (D > 48 && T * K >= 250 && (size_t)N * (size_t)D >= (size_t)1 << 18);
 #define RSFK_ANN_CASE(SLV)                                                                                                    \
-    hipLaunchKernelGGL(k_ann_forest<SLV>, dim3((unsigned)NQ), dim3(256), lds, stream, points, queries, N, D, K, T, perm, where,  \
-                       vec_p, dpad, q_idx, q_dist)
+    do {                                                                                                                     \
+        auto* kernel = quads ? k_ann_forest<SLV, true> : k_ann_forest<SLV, false>;                                            \
+        hipLaunchKernelGGL(kernel, dim3((unsigned)NQ), dim3(256), lds, stream, points, queries, N, D, K, T, perm, where, vec_p, dpad, \
+                           q_idx, q_dist);                                                                                   \
+    } while (0)
     switch (row_slots(K)) {
     case 1: RSFK_ANN_CASE(1); break;
     case 2: RSFK_ANN_CASE(2); break;

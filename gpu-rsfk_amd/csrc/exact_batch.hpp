@@ -159,50 +159,62 @@ __device__ __forceinline__ void quad_swap(float4& a, float4& b, bool bit)
 
 // The same without the tile: the chain of candidate l runs in the registers of lane l, 32 dimensions (eight 16-byte pieces) per step; the point's
 // coordinates come from L.xrow (every lane reads the same word).  For short rows: no LDS besides xrow, no synchronisation inside the batch.
-// Four lanes load 64 bytes of the row of each of them in turn and exchange the pieces.  (A lane loading its own row asks for every line eight times, and
+// QUADS: four lanes load 64 bytes of the row of each of them in turn and exchange the pieces; else a lane reads its own row, which the query-set search does
+// where rows are short or few (ann.hip).  (A lane loading its own row asks for every line eight times, and
 // a request of one lane takes the address units as long as one of four lanes in a row: they were busy 67 to 76 % of the exploration merge's time.  10M x 32
 // 18.95 -> 17.33 ms, 1M x 100 2.56 -> 2.44, 1M x 256 5.95 -> 5.65, 123,457 x 37, K = 45 0.838 -> 0.660.  Whole lines by eight lanes each through 4 KB of LDS:
 // 26.3, 3.57, 8.1, 1.11: 97 registers, and the LDS of four more wavefronts.)
-template <int SL, bool RANK = false>
+template <int SL, bool QUADS, bool RANK = false>
 __device__ __forceinline__ void exact_direct(const ExploreLds& L, const int* list, int n, const float* __restrict__ points,
-                                             int D, KnnRow<SL>& row, float tau_cap = INFINITY)
+                                             int D, bool vec_ok, KnnRow<SL>& row, float tau_cap = INFINITY)
 {
     const int lane = lane_id();
     const int my_c = lane < n ? list[lane] : -1;
+    const float* rp = points + (size_t)(my_c >= 0 ? my_c : 0) * (size_t)D;
     float acc = 0.0f;
     const float tau0 = fminf(row.tau, tau_cap);
     bool finished = true;
-    // instruction k of 16 dimensions loads 64 bytes of the row of lane k of every four lanes, and the four exchange them
+    // QUADS: instruction k of 16 dimensions loads 64 bytes of the row of lane k of every four lanes, and the four exchange them
     const int quarter = 4 * (lane & 3);
     const bool odd = (lane & 1) != 0, upper = (lane & 2) != 0;
     const int id[4] = {dpp_i<0x00>(my_c), dpp_i<0x55>(my_c), dpp_i<0xAA>(my_c), dpp_i<0xFF>(my_c)};
+    // the four dimensions from d on, of this lane's candidate (xrow is zero beyond D like the pieces)
+    const auto chain = [&](int d, const float4& v) {
+        const float4 x = *reinterpret_cast<const float4*>(&L.xrow[d]);
+        float df;
+        df = v.x - x.x; acc = __builtin_fmaf(df, df, acc);
+        df = v.y - x.y; acc = __builtin_fmaf(df, df, acc);
+        df = v.z - x.z; acc = __builtin_fmaf(df, df, acc);
+        df = v.w - x.w; acc = __builtin_fmaf(df, df, acc);
+    };
     for (int d0 = 0; d0 < D; d0 += 32) {
         float4 v[8];
+        if (!QUADS) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int d = d0 + 16 * (i >> 2) + quarter, k = id[i & 3];
-            v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (k >= 0 && d < D) v[i] = load_dims(points + (size_t)(uint32_t)k * (size_t)(uint32_t)D + (size_t)(uint32_t)d, D - d, false);
-        }
+            for (int i = 0; i < 8; ++i)
+                v[i] = my_c >= 0 ? load_piece(rp, d0 + 4 * i, D, vec_ok) : make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
-        for (int h = 0; h < 8; h += 4) {
-            quad_swap<kDppXor1>(v[h], v[h + 1], odd);
-            quad_swap<kDppXor1>(v[h + 2], v[h + 3], odd);
-            quad_swap<kDppXor2>(v[h], v[h + 2], upper);
-            quad_swap<kDppXor2>(v[h + 1], v[h + 3], upper);
-            __builtin_amdgcn_sched_barrier(0);
+            for (int i = 0; i < 8; ++i)
+                if (d0 + 4 * i < D) chain(d0 + 4 * i, v[i]);              // (wave-uniform)
+        } else {
 #pragma unroll
-            for (int i = h; i < h + 4; ++i) {
-                if (d0 + 4 * i < D) {                         // (wave-uniform; xrow is zero beyond D like the pieces)
-                    const float4 x = *reinterpret_cast<const float4*>(&L.xrow[d0 + 4 * i]);
-                    float df;
-                    df = v[i].x - x.x; acc = __builtin_fmaf(df, df, acc);
-                    df = v[i].y - x.y; acc = __builtin_fmaf(df, df, acc);
-                    df = v[i].z - x.z; acc = __builtin_fmaf(df, df, acc);
-                    df = v[i].w - x.w; acc = __builtin_fmaf(df, df, acc);
-                }
+            for (int i = 0; i < 8; ++i) {
+                const int d = d0 + 16 * (i >> 2) + quarter, k = id[i & 3];
+                v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (k >= 0 && d < D) v[i] = load_dims(points + (size_t)(uint32_t)k * (size_t)(uint32_t)D + (size_t)(uint32_t)d, D - d, false);
             }
-            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int h = 0; h < 8; h += 4) {
+                quad_swap<kDppXor1>(v[h], v[h + 1], odd);
+                quad_swap<kDppXor1>(v[h + 2], v[h + 3], odd);
+                quad_swap<kDppXor2>(v[h], v[h + 2], upper);
+                quad_swap<kDppXor2>(v[h + 1], v[h + 3], upper);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int i = h; i < h + 4; ++i)
+                    if (d0 + 4 * i < D) chain(d0 + 4 * i, v[i]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
         // partial sums only grow: once all of them are above the row maximum nothing can enter
         if (ballot64(lane < n && acc <= tau0) == 0) { finished = false; break; }

@@ -551,7 +551,7 @@ __global__ __launch_bounds__(64 * WAVES, FORM == kFormTile || SL > 1 ? 1 : FORM 
     float reach = INFINITY;                               // what the row's last slot will be at most
     auto batch = [&](const int* list, int n) {
         n_exact += n;
-        if (!TILE) exact_direct<SL, true>(L, list, n, points, D, row, reach);
+        if (!TILE) exact_direct<SL, true, true>(L, list, n, points, D, vec_ok, row, reach);
         else exact_batch<SL, kMergeChunk, true, kChainGroup, true>(L, list, n, points, D, vec_ok, row, reach);    // two steps of gathers in flight
     };
     if (tbound == nullptr || U <= kFewCandidates) {

@@ -1478,10 +1478,11 @@ def test_find_nearest_neighbors_ann_matches_oracle(gpu, orc, rng, N, NQ, D, K, T
 
 
 # one query; one tree more than the wavefronts take in turn; buckets on both sides of 64 and 128; rows of one, two and
-# more slots per lane; rows that end inside a 16-byte piece; more trees than go together
+# more slots per lane; rows that end inside a 16-byte piece; more trees than go together; rows read by four lanes (from 129 dimensions on, and of 53) and by one
 @pytest.mark.parametrize("N,NQ,D,K,T,mn,mx", [(300, 1, 1, 1, 2, 3, 6), (2000, 37, 33, 64, 5, 65, 65 * 2), (1500, 300, 64, 65, 9, 66, 128),
                                               (900, 130, 31, 16, 3, 17, 64), (700, 65, 100, 300, 4, 301, 700), (4000, 90, 7, 5, 70, 6, 12),
-                                              (50, 20, 12, 8, 6, 60, 120), (1200, 33, 260, 20, 8, 21, 65)])
+                                              (50, 20, 12, 8, 6, 60, 120), (1200, 33, 260, 20, 8, 21, 65), (5300, 60, 53, 30, 9, 31, 62),
+                                              (700, 40, 129, 70, 3, 71, 150)])
 @pytest.mark.parametrize("data", ["normal", "ties", "tiny"])
 def test_ann_trees_together_match_oracle(gpu, capi, orc, rng, monkeypatch, N, NQ, D, K, T, mn, mx, data):
     """All trees of a query in one workgroup == one tree after the other == the oracle, also into rows that hold something."""
