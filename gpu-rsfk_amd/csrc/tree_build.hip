@@ -2723,14 +2723,16 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
         const int stack_cap = w->mid_most / std::max(P.small, 1) + 4;
         const size_t lds = (size_t)w->mid_most * 6 + (size_t)nvec_len(D) * 4 + (size_t)(stack_cap + kMidOut) * sizeof(MidNode);
         const int pieces = q8_padded(D) / 16;
-        // A workgroup splits one node after the other, about 10 us each; while several of its descendants will be larger than P.small, a launch ends
-        // with the children, which the next one takes side by side.
-        // One tree of 10,000 x 2 73 us in one launch, 19 + 15 + 25 in three, the call 187 -> 178; 10,000 x 32, 4 trees 86 -> 78, the call the same; with
-        // two launches 72 and 81 (the halves are rarely alike).  Not with many nodes, when those of the last launch wait for each other's compute units: 20,000 x
-        // 32, 50 trees 111 -> 125 us.
+        // A workgroup splits one node after the other, about 10 us each; where several of its descendants will be larger than P.small, a launch ends
+        // with the children, which the next one takes side by side.  A launch more is about 10 us too, so not below four times P.small, but of
+        // one or two nodes from three times on (there into two launches).  Calls of trees alone, one launch -> with the children handed on: one tree of 4,300 x 2
+        // 243 -> 247 us, 5,000 x 20 263 -> 267, 6,500 x 100 359 -> 338, 8,100 x 20 307 -> 299, 12,000 x 2 324 -> 311, 18,500 x 20 403 -> 385; four trees of 5,000 x 32
+        // 235 -> 244, 8,000 x 4 278 -> 286, 12,000 x 4 322 -> 301; 2 to 50 trees of 7,000 points 0.95 to 1.03 (mean 1.00), of 8,500 to 22,000 0.94 to 1.05 (0.985).
+        // Not with many nodes, when those of the last launch wait for each other's compute units: 20,000 x 32, 50 trees 111 -> 125 us.
+        const int largest = std::min(N, w->mid_most);
         int hand = 0;
-        if (n_tail <= 64)
-            for (int m = std::min(N, w->mid_most); m > 2 * P.small && hand < 2; m /= 2) ++hand;
+        if (n_tail <= 64 && largest > 4 * P.small) hand = 2;
+        else if (n_tail <= 2 && largest > 3 * P.small) hand = 1;
         for (int pass = 0; pass <= hand; ++pass) {
             const TreeNode* tasks = pass == 0 ? w->mid : w->mid_next + (size_t)(pass - 1) * (size_t)w->tail_cap;
             const int* n_tasks = pass == 0 ? nullptr : &w->ctr->n_mid_next[pass - 1];

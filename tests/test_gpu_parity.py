@@ -194,9 +194,9 @@ def test_tree_wide_levels_by_the_8_bit_copy(gpu, orc, rng, monkeypatch, D, kind)
     assert np.array_equal(gls, ls) and np.array_equal(glz, lz)
 
 
-# The middle phase in one, two and three launches: largest nodes of up to twice the tail's, of one point more, of more than four times as many; nodes
-# of a tree that stay above the tail's size after the last of them; many equal rows, whose nodes lose a few points at a time.
-@pytest.mark.parametrize("N", [512, 513, 1025, 1100, 4000, 12000])
+# The middle phase in one, two and three launches: largest nodes of up to three times the tail's, of one point more, of up to four times as many and of one
+# point more; nodes of a tree that stay above the tail's size after the last of them; many equal rows, whose nodes lose a few points at a time.
+@pytest.mark.parametrize("N", [512, 513, 768, 769, 1024, 1025, 1100, 4000, 12000])
 @pytest.mark.parametrize("D,kind", [(2, "n"), (40, "n"), (70, "n"), (300, "n"), (5, "dup")])
 def test_tree_middle_phase_by_launches(gpu, orc, rng, monkeypatch, N, D, kind):
     for name, v in (("SCREEN", "q8"), ("SMALL", "256")):
