@@ -180,7 +180,14 @@ __device__ __forceinline__ void make_hyperplane_wave(const float* __restrict__ x
 // normal of the point's node).  Only lane 0 of a group holds the header, so only its right / redo are meaningful
 // (with either copy the callers use lane 0 only).
 // (KU: pieces of a row a lane has in flight, 8-bit copy)
-template <int NB, bool Q8, int LPP = 8, int KU = 1>
+// INSIDE: the header comes with the row, as its first piece, above nothing of the normal (header_inside says where; 16 floats that can be read have to be before
+// nvec0): the row then comes in loads of whole lines, each once, where a load of its own asks for the first line again while it is on its way.  Middle phase
+// of 123,457 x 37, 12 trees 0.202 -> 0.182 ms, of 3,000 x 200, 10 trees 0.046 -> 0.043.  Not in the tail kernel, which is bound by its instructions: 5,000 x 24, 50
+// trees 135 -> 138 us, 8,000 x 32, 8 trees 114 -> 117, 5,000 x 52, 50 trees 156 -> 160, 200,000 x 32, 12 trees 363 -> 367.
+template <int LPP>
+bool header_inside(int D) { return (q8_padded(D) >> 4) % LPP != 0; }      // (the last step has a lane to spare)
+
+template <int NB, bool Q8, int LPP = 8, int KU = 1, bool INSIDE = false>
 __device__ __forceinline__ void side_screen8(const float* nvec0, int nstride, const int (&j)[NB], const float (&b)[NB],
                                              const float (&hp1)[NB], const float (&hp2)[NB],
                                              const uint16_t* __restrict__ pb16, const uint8_t* __restrict__ q8,
@@ -193,21 +200,16 @@ __device__ __forceinline__ void side_screen8(const float* nvec0, int nstride, co
 #pragma unroll
         for (int u = 0; u < NB; ++u) { right[u] = false; redo[u] = valid[u]; }
         const size_t pitch = (size_t)q8_pitch(D);
-        // Where the header takes no step more (the last step has a lane to spare) it is the first piece, above nothing of the normal: the
-        // row then comes in loads of whole lines, each once (a load of its own asks for the first line again while it is on its way: middle phase of
-        // 123,457 x 37, 12 trees 0.202 -> 0.182 ms, of 3,000 x 200, 10 trees 0.046 -> 0.043; the tail kernel, bound by its instructions, the same).
-        const int all = (q8_padded(D) >> 4) + 1;
-        const bool inside = (all - 1) % LPP != 0;
-        const int skip = inside ? 0 : 1, pieces = all - skip;
-        q8 += 16 * skip;
-        nvec0 -= 16 * (1 - skip);
+        const int pieces = (q8_padded(D) >> 4) + (INSIDE ? 1 : 0);
+        if (!INSIDE) q8 += 16;
+        else nvec0 -= 16;
         float da[NB];
         uint4 head[NB];
 #pragma unroll
         for (int u = 0; u < NB; ++u) {
             da[u] = 0.0f;
             head[u] = make_uint4(0u, 0u, 0u, 0u);
-            if (!inside && valid[u] && sub == 0) head[u] = *reinterpret_cast<const uint4*>(q8 - 16 + (size_t)id[u] * pitch);
+            if (!INSIDE && valid[u] && sub == 0) head[u] = *reinterpret_cast<const uint4*>(q8 - 16 + (size_t)id[u] * pitch);
         }
         for (int k0 = sub; k0 < pieces; k0 += KU * LPP) {
             uint4 w[KU][NB];
@@ -235,7 +237,7 @@ __device__ __forceinline__ void side_screen8(const float* nvec0, int nstride, co
                         da[u] = __builtin_fmaf(nq.z, (float)((ww[q] >> 16) & 0xffu), da[u]);
                         da[u] = __builtin_fmaf(nq.w, (float)((ww[q] >> 24) & 0xffu), da[u]);
                     }
-                    if (y == 0 && inside && k == 0) { head[u] = w[0][u]; da[u] = 0.0f; }
+                    if (INSIDE && y == 0 && k == 0) { head[u] = w[0][u]; da[u] = 0.0f; }
                 }
             }
         }
@@ -1362,7 +1364,7 @@ struct MidNode : SmallNode {
     int leaf;                             // 1: a bucket, or to be one at the depth limit; kMidNext: for the next launch
 };
 
-template <int LPP, int KU>
+template <int LPP, int KU, bool INSIDE>
 __global__ __launch_bounds__(kMidThreads, 4) void k_mid(const float* __restrict__ points, const uint8_t* __restrict__ q8, TreeParams P, int most,
                                                         const int* __restrict__ perm0, const int* __restrict__ perm1, int* __restrict__ perm_out,
                                                         const TreeNode* __restrict__ tasks, TreeNode* __restrict__ tail, int tail_cap, int stack_cap,
@@ -1465,7 +1467,7 @@ __global__ __launch_bounds__(kMidThreads, 4) void k_mid(const float* __restrict_
                 h1[u] = n1;
                 h2[u] = sn;
             }
-            side_screen8<kBatch, true, LPP, KU>(nvec, 0, jz, bb, h1, h2, nullptr, q8, id, P.D, P.band, valid, right, redo);
+            side_screen8<kBatch, true, LPP, KU, INSIDE>(nvec, 0, jz, bb, h1, h2, nullptr, q8, id, P.D, P.band, valid, right, redo);
 #pragma unroll
             for (int u = 0; u < kBatch; ++u) {
                 if (valid[u] && sub == 0) {
@@ -2741,13 +2743,13 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
             const unsigned grid = pass == 0 ? (unsigned)n_tail
                                             : (unsigned)std::max<size_t>(1, std::min((size_t)n_tail << pass, (size_t)N * (size_t)nb / (size_t)(P.small + 1)));
 #define RSFK_MID_LAUNCH(L, U)                                                                                               \
-        do {                                                                                                               \
-            RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_mid<L, U>),                                       \
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));                          \
-            hipLaunchKernelGGL((k_mid<L, U>), dim3(grid), dim3(kMidThreads), lds, stream, points, q8, P, w->mid_most,     \
-                               w->perm[0], w->perm[1], w->perm[0], tasks, w->tail, w->tail_cap, stack_cap, w->stats, w->ctr,  \
-                               w->recs, w->rec_cap, w->stat, n_tasks, next, pass < hand ? &w->ctr->n_mid_next[pass] : nullptr, w->tail_cap); \
-        } while (0)
+            do {                                                                                                           \
+                auto* kernel = header_inside<L>(D) ? k_mid<L, U, true> : k_mid<L, U, false>;                                   \
+                RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)); \
+                hipLaunchKernelGGL(kernel, dim3(grid), dim3(kMidThreads), lds, stream, points, q8, P, w->mid_most, w->perm[0], w->perm[1], \
+                                   w->perm[0], tasks, w->tail, w->tail_cap, stack_cap, w->stats, w->ctr, w->recs, w->rec_cap, w->stat, n_tasks, \
+                                   next, pass < hand ? &w->ctr->n_mid_next[pass] : nullptr, w->tail_cap);                       \
+            } while (0)
             if (pieces <= 2) RSFK_MID_LAUNCH(2, 1);
             else if (pieces <= 4) RSFK_MID_LAUNCH(4, 1);
             else if (pieces <= 16) RSFK_MID_LAUNCH(4, 4);
