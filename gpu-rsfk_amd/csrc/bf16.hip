@@ -37,12 +37,16 @@ __global__ __launch_bounds__(256) void k_to_bf16(const float* __restrict__ point
 // fl(lo + scale q); the screen evaluates lo sum n + scale sum n q in fp32 and is compared with an fp32 evaluation of n.x: all of that
 // stays below ev = c_d (|lo| + 255 scale) per unit of ||n||_1, so below sqrt(D) ev per unit of ||n||_2 (the factors above one: the
 // rounding of the sums and norms themselves).  Where the squares may underflow, the largest error stands for all of them.
-__device__ __forceinline__ float row_bound(float err, float sq, float lo, float scale, float range, int D, float c_d, bool bad)
+struct RowBound {
+    float e1, by_largest;       // the bound, and what it would be per unit of ||n||_1 alone (mean_rho)
+};
+__device__ __forceinline__ RowBound row_bound(float err, float sq, float lo, float scale, float range, int D, float c_d, bool bad)
 {
-    if (bad || !(range <= 3.0e38f)) return __builtin_nanf("");      // the screen never decides for such a row
+    if (bad || !(range <= 3.0e38f)) return {__builtin_nanf(""), __builtin_nanf("")};      // the screen never decides for such a row
     const float ev = 1.0011f * (c_d * (fabsf(lo) + 255.0f * scale));
     const float rms = range > 1e-12f ? __builtin_sqrtf(sq / (float)D) + 2e-19f : err;
-    return fmaxf(1.0111f * err + ev, (1.0111f * rms + ev) * (1.0f / kRmsShare)) + kQ8Least;
+    const float largest = 1.0111f * err + ev;
+    return {fmaxf(largest, (1.0111f * rms + ev) * (1.0f / kRmsShare)) + kQ8Least, largest + kQ8Least};
 }
 
 // one wavefront per row of the 8-bit copy
@@ -99,15 +103,15 @@ __global__ __launch_bounds__(256) void k_to_q8(const float* __restrict__ points,
             err = fmaxf(err, __shfl_xor(err, o, 64));
             sq += __shfl_xor(sq, o, 64);
         }
-        const float e1 = row_bound(err, sq, lo, scale, range, D, c_d, bad);
+        const RowBound bound = row_bound(err, sq, lo, scale, range, D, c_d, bad);
         if (lane == 0) {
             float* head = reinterpret_cast<float*>(dst);
             head[0] = 0.0f;
             head[1] = lo;
             head[2] = scale;
-            head[3] = e1;
+            head[3] = bound.e1;
             const float bf = sabs / (float)D * (1.0f / 256.0f);
-            rho_acc += (e1 == e1 && bf > 0.0f) ? fminf(e1 / bf, 1000.0f) : 1000.0f;
+            rho_acc += (bound.by_largest == bound.by_largest && bf > 0.0f) ? fminf(bound.by_largest / bf, 1000.0f) : 1000.0f;
             if (!bad && fmaxf(fabsf(lo), fabsf(hi)) > most) rho_acc = INFINITY;
         }
     }
@@ -201,11 +205,11 @@ __global__ __launch_bounds__(256) void k_to_q8_regs(const float* __restrict__ po
             err = fmaxf(err, __shfl_xor(err, o, 64));
             sq += __shfl_xor(sq, o, 64);
         }
-        const float e1 = row_bound(err, sq, lo, scale, range, D, c_d, badi != 0);
+        const RowBound bound = row_bound(err, sq, lo, scale, range, D, c_d, badi != 0);
         if (row_ok && l == 0) {
-            *reinterpret_cast<float4*>(dst) = make_float4(0.0f, lo, scale, e1);
+            *reinterpret_cast<float4*>(dst) = make_float4(0.0f, lo, scale, bound.e1);
             const float bf = sabs / (float)D * (1.0f / 256.0f);
-            rho_acc += (e1 == e1 && bf > 0.0f) ? fminf(e1 / bf, 1000.0f) : 1000.0f;
+            rho_acc += (bound.by_largest == bound.by_largest && bf > 0.0f) ? fminf(bound.by_largest / bf, 1000.0f) : 1000.0f;
             if (!badi && fmaxf(fabsf(lo), fabsf(hi)) > most) rho_acc = INFINITY;
         }
     }

@@ -36,8 +36,10 @@ struct Bf16Copy {
 // which is 1 / sqrt(3) of the largest where coordinates fall anywhere between two steps; e1 is the larger of the largest error and
 // 1 / kRmsShare of that root, so either holds.  For normals whose components spread like those of a uniform or a normal distribution
 // L(n) is 0.71..0.73 ||n||_1 (points left to the exact test: 1M x 100 uniform 3.77 -> 2.74 %, 1M x 256 in clusters 12.3 -> 9.1 %; trees of the former 24.4 -> 23.5 ms for 50, of the latter 29.4 -> 26.4 for 20).  mean_rho (host, after
-// q8_copy_fill has completed) compares e1 with the corresponding quantity of the bfloat16 copy,
-// 2^-8 mean_d |x_d|, averaged over the rows: the 8-bit copy pays off while it is below about 6.
+// q8_copy_fill has completed) compares the bound by the largest error, per unit of ||n||_1, with the corresponding quantity of the bfloat16 copy,
+// 2^-8 mean_d |x_d|, averaged over the rows: the 8-bit copy pays off while it is below about 6.  (Not e1, which can be 1.72 times that where
+// L(n) makes up for it.  One tree of 5,000 x 4096 normal points, 5.9 by the one and 6.0 by the other: 13.3 ms by the 8-bit copy, 14.9 by the bfloat16 copy.  Since
+// L(n) the times of the two meet at 6 to 7 for 784 dimensions, 10 for 256, beyond 12 for 100 and fewer.)
 __host__ __device__ inline int q8_pitch(int D) { return (16 + D + 63) & ~63; }
 __host__ __device__ inline int q8_padded(int D) { return (D + 15) & ~15; }      // coordinates in whole 16-byte pieces
 

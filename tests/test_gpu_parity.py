@@ -171,6 +171,22 @@ def test_tree_bounds_by_largest_and_mean_error(gpu, orc, rng, monkeypatch, kind,
     assert np.array_equal(gls, ls) and np.array_equal(glz, lz)
 
 
+# The 8-bit copy is the screen while the largest rounding error of its coordinates is below six of bfloat16's mean one, however the errors spread: here
+# all coordinates but two lie half a step off, where the bound by the mean square is 1.7 times that by the largest.  Between 0 and 255 the error
+# is 0.5, and bfloat16's the mean of the coordinates / 256: 5.0 of it with coordinates of up to 43.5, 10 with up to 15.5.
+@pytest.mark.parametrize("top,row_bytes", [(44, 128), (16, 256)])
+def test_screen_is_chosen_by_the_largest_error(gpu, orc, rng, top, row_bytes):
+    import gpu_rsfk
+    N, D, K = 1500, 100, 8
+    X = (rng.integers(0, top, (N, D)) + 0.5).astype(np.float32)
+    X[:, 3], X[:, 70] = 0.0, 255.0
+    _say("screen by the largest error", top)
+    gi, gd = gpu_rsfk.RSFK(random_state=2).find_nearest_neighbors(X, K, n_trees=2, nn_exploring_factor=0)
+    assert gpu.last_build_report()["tree_screen_row_bytes"] == row_bytes
+    oi, od = orc.forest(X, K, 2, K + 1, 2 * (K + 1), 5000, 2, 0)
+    assert_knn_equal(gi, gd, oi, od)
+
+
 # Side tests of the wide levels by the 8-bit copy: rows of 64 bytes and of one line to several, whole or ending in half a line; chunks of any size; rows of NaN,
 # equal rows, and a common offset that leaves every point to the exact test.
 @pytest.mark.parametrize("D", [1, 47, 48, 49, 111, 112, 113, 176, 240, 241, 305, 1100])
