@@ -108,7 +108,9 @@ __host__ __device__ inline int nvec_len(int D) { return (D + 15) & ~15; }
 // order: only the screens use them, with a margin).  The sum of squares in it is used where the squares neither underflow nor overflow.  A pair with the same coordinates has the normal 0 and every point on its left (0 < 0):
 // its hp[1] is kZeroNormal, which makes the bounds of the screens negative, so that no point is left to the exact test
 // (100,000 x 32, a tenth of the points in groups of 2,000 equal rows, 10 trees: 947 -> 220 ms).
+// SCREEN8 false: hp[1] is the 1-norm, of which the bfloat16 screen takes the sign (tail of 3,000 x 9000 22.0 ms with the sum of squares, 21.8 without, of 1,200 x 20000 89.7 and 88.4).
 constexpr float kZeroNormal = -1e30f;
+template <bool SCREEN8 = true>
 __device__ __forceinline__ void make_hyperplane_wave(const float* __restrict__ x1, const float* __restrict__ x2,
                                                      int D, float* nvec, float* hp)
 {
@@ -137,7 +139,7 @@ __device__ __forceinline__ void make_hyperplane_wave(const float* __restrict__ x
                     nvec[d] = nd;
                     const float prod = nd * (t1[k] + t2[k]);
                     s = s + prod * 0.5f;
-                    s2 = __builtin_fmaf(nd, nd, s2);
+                    if (SCREEN8) s2 = __builtin_fmaf(nd, nd, s2);
                 } else {
                     s += fabsf(nd);
                     s2 += nd;
@@ -148,11 +150,11 @@ __device__ __forceinline__ void make_hyperplane_wave(const float* __restrict__ x
     for (int d = D + lane; d < Dn; d += 64) nvec[d] = 0.0f;
     s = half_butterfly_sum(s);
     s2 = half_butterfly_sum(s2);
-    const float sq = read_lane_f(s2, 0);
+    const float sq = SCREEN8 ? read_lane_f(s2, 0) : 0.0f;
     if (lane == 0) hp[0] = s;
     if (lane == 32) {
         const float l2 = __builtin_sqrtf(sq * (kRmsShare * kRmsShare * 1.0005f * (float)D));
-        hp[1] = s == 0.0f ? kZeroNormal : (s > 1e-9f ? fminf(s, l2) : s) + kNormalLeast;
+        hp[1] = s == 0.0f ? kZeroNormal : (SCREEN8 && s > 1e-9f ? fminf(s, l2) : s) + kNormalLeast;
         hp[2] = s2;
     }
 }
@@ -1125,8 +1127,8 @@ __global__ __launch_bounds__(TB, CHAIN ? 4 : 6) void k_tail(const float* __restr
             }
             __syncthreads();
             for (int j = wave; j < nb; j += TB / 64) {
-                make_hyperplane_wave(points + (size_t)pair_s[j][0] * P.D, points + (size_t)pair_s[j][1] * P.D, P.D,
-                                     nvec + (size_t)j * Dv, hp_s[j]);
+                make_hyperplane_wave<Q8>(points + (size_t)pair_s[j][0] * P.D, points + (size_t)pair_s[j][1] * P.D, P.D,
+                                         nvec + (size_t)j * Dv, hp_s[j]);
                 if (lane == 0) b_s[j] = hp_s[j][0];       // written by this lane just above
             }
             for (int j = 0; j < nb; ++j) {
