@@ -1673,17 +1673,8 @@ int launch_explore_join(ExploreWorkspace* w, const JoinCopy& jc, int N, int D, i
     w->view.any_rel = any_rel;
     w->view.any_abs = any_abs;
     const int MW = KP >> 5;
-    const unsigned short_groups = grid_for_dies(((size_t)N * (size_t)MW + kWaves - 1) / kWaves);
-    const bool use_short = !w->bounds && ksteps <= 8 && launch_fits(short_groups, 64 * kWaves);
-    // (the records of the reversed graph's builder are done with: the words take the place of the last ones, and are sorted from there)
-    uint32_t* marks = use_short && w->staged && MW == 1 ? reinterpret_cast<uint32_t*>(w->bin_eq2) : nullptr;
-    hipLaunchKernelGGL(k_join_bars, dim3((unsigned)((N + 255) / 256) + 1), dim3(256), 0, stream, jc, jc.scale(), knn_dist, N, K,
-                       one_minus_gamma, w->bars, w->pass, marks ? 0 : (size_t)N * (size_t)K * (size_t)MW, knn_idx, old_idx);
-    RSFK_HIP(hipGetLastError());
-    if (launch_rev(w, old_idx, N, K, stream, w->rev_bars && use_short)) return 1;
     // More points than a launch has threads for take a wavefront per q: with a wavefront per 32 neighbours K = 33 from 33.5 million points on, 129
     // from 13.4, 225 from 8.4, with a workgroup per q all from 16.8.
-    const bool wg_fits = launch_fits(grid_for_dies((size_t)N), 256);
     // One workgroup per q reads every row once per 96 points of R(q), one wavefront per q (and 32 neighbours) again for every group of 32
     // neighbours, so the former pays with the bytes that are read again, D (K - 24) or so, sooner with more groups; up to 32 neighbours
     // are one pair per tile of R(q), too little for four wavefronts (1M x 256, K = 32: 8.1 ms against 12.6).  A pass, a wavefront per q -> a
@@ -1692,7 +1683,18 @@ int launch_explore_join(ExploreWorkspace* w, const JoinCopy& jc, int N, int D, i
     // -> 19.6, x 32 17.0 -> 16.9, 100,000 x 256, K = 128 15.0 -> 11.4.  Above 128 neighbours its accumulators leave one wavefront per SIMD, and the
     // line is far up: 8,000 points after one tree, x 400, K = 256 21.33 -> 21.38, x 550, K = 190 14.04 -> 13.99, K = 220 18.1 -> 17.7, x 784, K = 130 8.03 -> 8.08,
     // K = 160 10.1 -> 9.8, K = 256 28.4 -> 26.1, x 100, K = 256 17.2 -> 18.6; 100,000 x 32, K = 160 18.3 -> 29.7.
-    if (KP > 32 && join_wg_on() && wg_fits && D * (K - 24) > (MW == 2 ? 8000 : MW == 3 ? 6500 : MW == 4 ? 3000 : 95000)) {
+    const bool use_wg = KP > 32 && join_wg_on() && launch_fits(grid_for_dies((size_t)N), 256) &&
+                        D * (K - 24) > (MW == 2 ? 8000 : MW == 3 ? 6500 : MW == 4 ? 3000 : 95000);
+    const unsigned short_groups = grid_for_dies(((size_t)N * (size_t)MW + kWaves - 1) / kWaves);
+    const bool use_short = !use_wg && !w->bounds && ksteps <= 8 && launch_fits(short_groups, 64 * kWaves);
+    // (the records of the reversed graph's builder are done with: the words take the place of the last ones, and are sorted from there)
+    uint32_t* marks = use_short && w->staged && MW == 1 ? reinterpret_cast<uint32_t*>(w->bin_eq2) : nullptr;
+    hipLaunchKernelGGL(k_join_bars, dim3((unsigned)((N + 255) / 256) + 1), dim3(256), 0, stream, jc, jc.scale(), knn_dist, N, K,
+                       one_minus_gamma, w->bars, w->pass, marks ? 0 : (size_t)N * (size_t)K * (size_t)MW, knn_idx, old_idx);
+    RSFK_HIP(hipGetLastError());
+    // (the other forms read bars, not their codes)
+    if (launch_rev(w, old_idx, N, K, stream, w->rev_bars && use_short)) return 1;
+    if (use_wg) {
         const size_t lds_wg = (size_t)(kJwP + KP) * kJwRowBytes + (size_t)KP * 12 + (size_t)kJwP * 24;
 #define RSFK_JOIN_WG(BV, NV)                                                                                                    \
         do {                                                                                                               \

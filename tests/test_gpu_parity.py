@@ -697,12 +697,15 @@ def test_explore_with_the_reversed_graph_by_tiles(gpu, orc, rng, monkeypatch, N,
     assert_knn_equal(gi, gd, oi, od)
 
 
-@pytest.mark.parametrize("N,D,K", [(70001, 6, 31), (66000, 20, 32), (9001, 12, 3), (5000, 40, 1), (700, 33, 32), (2000, 20, 45)])
+@pytest.mark.parametrize("N,D,K", [(70001, 6, 31), (66000, 20, 32), (9001, 12, 3), (5000, 40, 1), (700, 33, 32), (2000, 20, 45), (3000, 65, 31),
+                                   (2300, 100, 32), (2500, 128, 20), (600, 110, 90)])
 def test_explore_with_the_staged_reversed_graph(gpu, orc, rng, monkeypatch, N, D, K):
     """RSFK_REV_STAGED=1: marks put in place window by window (more than 2^21 of them, a last piece of any length, few), bars as 16-bit codes beside
     the entries and, with few neighbours, gathered; rows that are not full; points far out, whose rounding errors are large.  More than 32
-    neighbours: marks stored one by one."""
+    neighbours: marks stored one by one, and, by the workgroups of rows without codes, from the bars themselves."""
     monkeypatch.setenv("RSFK_REV_STAGED", "1")
+    if K > 64:
+        monkeypatch.setenv("RSFK_OPTIONAL_MB", "0")
     X = rng.random((N, D), dtype=np.float32)
     X[::97] *= 1000.0
     oi, od = orc.init_lists(N, K, self_in=True)
