@@ -2392,7 +2392,8 @@ struct TreeBatchWorkspace {
     TreeNode* chain = nullptr;           // nodes for the chain phase
     TreeNode* mid = nullptr;             // nodes for the middle phase (when there is one)
     int mid_most = 0;                    // points of the largest of them
-    TreeNode* mid_next = nullptr;        // nodes for its second launch, and for its third: tail_cap each
+    TreeNode* mid_next = nullptr;        // nodes for its second launch, and for its third: mid_next_cap each
+    int mid_next_cap = 0;
     int* chunk2node = nullptr;
     int* chunk_left = nullptr;
     float* planes = nullptr;             // hyperplanes of the nodes of the current wide level: node_cap x (4 + nvec_len(D))
@@ -2490,7 +2491,7 @@ int tree_mid_most(int D, int N, int B, int small)
     return n >= least && N > small ? n : 0;
 }
 
-// bytes of device memory a batch of B trees needs
+// bytes of device memory a batch of B trees needs (three lists of nodes: tail, chain phase, middle phase)
 size_t tree_ws_bytes(int N, int D, int MIN, int B)
 {
     const size_t lc = (size_t)N / (size_t)std::max(MIN, 1) + 2;
@@ -2530,7 +2531,9 @@ int tree_ws_alloc(TreeBatchWorkspace** out, int N, int D, int MIN, int B)
     if (dmalloc(&w->tail, (size_t)w->tail_cap)) return 1;
     if (dmalloc(&w->chain, (size_t)w->tail_cap)) return 1;
     w->mid_most = tree_mid_most(D, N, B, small);
-    if (w->mid_most && (dmalloc(&w->mid, (size_t)w->tail_cap) || dmalloc(&w->mid_next, 2 * (size_t)w->tail_cap))) return 1;
+    // (nodes above `small`, no two with a point in common, are handed on; a few kilobytes)
+    w->mid_next_cap = (int)((size_t)N * (size_t)B / (size_t)(small + 1)) + 1;
+    if (w->mid_most && (dmalloc(&w->mid, (size_t)w->tail_cap) || dmalloc(&w->mid_next, 2 * (size_t)w->mid_next_cap))) return 1;
     if (dmalloc(&w->chunk2node, (size_t)w->chunk_cap)) return 1;
     if (dmalloc(&w->chunk_left, (size_t)w->chunk_cap)) return 1;
     if (dmalloc(&w->planes, (size_t)w->node_cap * (size_t)(4 + nvec_len(D)))) return 1;
@@ -2738,9 +2741,9 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
         if (n_tail <= 64 && largest > 4 * P.small) hand = 2;
         else if (n_tail <= 2 && largest > 3 * P.small) hand = 1;
         for (int pass = 0; pass <= hand; ++pass) {
-            const TreeNode* tasks = pass == 0 ? w->mid : w->mid_next + (size_t)(pass - 1) * (size_t)w->tail_cap;
+            const TreeNode* tasks = pass == 0 ? w->mid : w->mid_next + (size_t)(pass - 1) * (size_t)w->mid_next_cap;
             const int* n_tasks = pass == 0 ? nullptr : &w->ctr->n_mid_next[pass - 1];
-            TreeNode* next = pass == hand ? nullptr : w->mid_next + (size_t)pass * (size_t)w->tail_cap;
+            TreeNode* next = pass == hand ? nullptr : w->mid_next + (size_t)pass * (size_t)w->mid_next_cap;
             // (nodes above P.small, no two with a point in common; two at most from each of the launch before)
             const unsigned grid = pass == 0 ? (unsigned)n_tail
                                             : (unsigned)std::max<size_t>(1, std::min((size_t)n_tail << pass, (size_t)N * (size_t)nb / (size_t)(P.small + 1)));
@@ -2750,7 +2753,7 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
                 RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)); \
                 hipLaunchKernelGGL(kernel, dim3(grid), dim3(kMidThreads), lds, stream, points, q8, P, w->mid_most, w->perm[0], w->perm[1], \
                                    w->perm[0], tasks, w->tail, w->tail_cap, stack_cap, w->stats, w->ctr, w->recs, w->rec_cap, w->stat, n_tasks, \
-                                   next, pass < hand ? &w->ctr->n_mid_next[pass] : nullptr, w->tail_cap);                       \
+                                   next, pass < hand ? &w->ctr->n_mid_next[pass] : nullptr, w->mid_next_cap);                   \
             } while (0)
             if (pieces <= 2) RSFK_MID_LAUNCH(2, 1);
             else if (pieces <= 4) RSFK_MID_LAUNCH(4, 1);

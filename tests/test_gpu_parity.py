@@ -2065,6 +2065,30 @@ def test_points_with_nan_coordinates_in_large_buckets(gpu, orc, rng, K, D):
     assert_knn_equal(gi, gd, oi, od)
 
 
+def test_middle_phase_needs_one_more_list_of_nodes(gpu, monkeypatch):
+    """The number of trees built together is chosen by an estimate with one list of nodes (48 bytes for each bucket there may be) for the middle phase;
+    what its later launches take is a few kilobytes."""
+    import torch
+    N, D, K, T, MIN = 40000, 4, 4, 50, 2
+    X = torch.rand((N, D), device="cuda")
+    held = {}
+    for mid in ("0", None, "0", None):                     # (the first calls also load the kernels)
+        if mid is None:
+            monkeypatch.delenv("RSFK_TREE_MID")
+        else:
+            monkeypatch.setenv("RSFK_TREE_MID", mid)
+        idx = dist = None
+        gpu.lib().rsfk_release_workspace()
+        idx = torch.full((N, K), -1, dtype=torch.int32, device="cuda")
+        dist = torch.full((N, K), float("inf"), device="cuda")
+        torch.cuda.synchronize()
+        before = torch.cuda.mem_get_info()[0]
+        _say("memory of the middle phase", mid)
+        gpu.knn_forest_device(T, K, N, D, MIN, 2 * MIN, 5000, 0, 0, 0, X.data_ptr(), idx.data_ptr(), dist.data_ptr())
+        held[mid] = before - torch.cuda.mem_get_info()[0]
+    assert held[None] - held["0"] <= 48 * T * (N // MIN + 2) + (8 << 20), held
+
+
 def test_forest_in_several_batches(gpu, orc, rng, monkeypatch):
     """Trees are built a batch at a time (all at once when memory allows); two per batch must give the same graph,
     for the K-NN graph (buckets of both kinds, so both streams of the bucket step are in use) and the query search."""
