@@ -689,6 +689,14 @@ __global__ __launch_bounds__(kBlock) void k_side(const float* __restrict__ point
 // Either way lane l then decides point l of the 64.  A level of 1M x 100, 50 trees: 1.49 -> 0.99 ms, of 10M x 32, 10 trees: 2.53 -> 2.15, of 1M x 256, 20 trees:
 // 1.52 -> 1.31 (a few per cent of it by the tighter bound of bf16.hpp), against eight (or two) lanes per point that multiply byte by byte, two vector instructions
 // each, and ask for a point's place, its row and its header in turn.  Headers by loads of their own: 1.11, 2.38; rows on multiples of 128 bytes: 1.35 for 256 dimensions.
+struct SideLds {                                            // besides the record of the hyperplane
+    float4 head[kBlock / 64][64];
+    int ids[kWideChunk];                                    // members of the chunk, bit 31 as it will be stored
+    uint16_t undecided[kWideChunk];
+    int left, n_undecided;
+};
+constexpr size_t kSideRecordMost = (size_t)160 * 1024 - sizeof(SideLds);      // bytes of the record (D up to 38,384)
+
 template <bool LINE>
 __global__ __launch_bounds__(kBlock) void k_side_q8(const float* __restrict__ points, const uint8_t* __restrict__ q8, TreeParams P,
                                                     int* __restrict__ perm0, int* __restrict__ perm1,
@@ -700,10 +708,9 @@ __global__ __launch_bounds__(kBlock) void k_side_q8(const float* __restrict__ po
     extern __shared__ __align__(16) float side_lds[];      // record of the node's hyperplane (k_level_planes)
     constexpr int kRounds = kWideChunk / kBlock;
     constexpr int kTiles = LINE ? 8 : 4, kRows = 64 / kTiles;       // of the 64 points of a wavefront; lanes of a row
-    __shared__ float4 head_s[kBlock / 64][64];
-    __shared__ int ids[kWideChunk];                         // members of the chunk, bit 31 as it will be stored
-    __shared__ uint16_t undecided[kWideChunk];
-    __shared__ int left_s, n_und_s;
+    __shared__ SideLds own;
+    int* ids = own.ids;
+    uint16_t* undecided = own.undecided;
     const int c = blockIdx.x;
     if (c >= ctr->queue[slot].chunks) return;
     if (c == 0 && threadIdx.x == 0) phase_tick(ctr, 0);
@@ -719,7 +726,7 @@ __global__ __launch_bounds__(kBlock) void k_side_q8(const float* __restrict__ po
     const float* rec = planes + (size_t)ni * (size_t)(4 + nvec_len(P.D));
     for (int i = tid; i < (4 + nvec_len(P.D)) >> 2; i += kBlock)
         reinterpret_cast<float4*>(side_lds)[i] = reinterpret_cast<const float4*>(rec)[i];
-    if (tid == 0) { left_s = 0; n_und_s = 0; }
+    if (tid == 0) { own.left = 0; own.n_undecided = 0; }
     const float b = rec[0], length = rec[1], sum = rec[2];
     const size_t pitch = (size_t)q8_pitch(P.D);
     const uint8_t* op = ops + (size_t)ni * side_op_bytes(P.D);
@@ -727,7 +734,7 @@ __global__ __launch_bounds__(kBlock) void k_side_q8(const float* __restrict__ po
     const int below_at = 16 * (LINE ? 2 * (lane >> 4) + ((lane >> 1) & 1) : lane >> 4);
     const uint8_t* part = op + 16 + (lane & 1) * pitch + below_at;
     const int steps = LINE ? (int)((pitch + 127) >> 7) : 1;
-    float4* heads = head_s[tid >> 6];
+    float4* heads = own.head[tid >> 6];
     pm::v4i normal = *reinterpret_cast<const pm::v4i*>(part);       // of the first step, which is the only one of most rows
     __syncthreads();
     int lefts = 0;
@@ -782,25 +789,25 @@ __global__ __launch_bounds__(kBlock) void k_side_q8(const float* __restrict__ po
         const bool right = certain && approx < b;
         ids[r * kBlock + tid] = right ? id[r] | (int)0x80000000 : id[r];
         lefts += valid && certain && !right ? 1 : 0;
-        if (valid && !certain) undecided[atomicAdd(&n_und_s, 1)] = (uint16_t)(r * kBlock + tid);
+        if (valid && !certain) undecided[atomicAdd(&own.n_undecided, 1)] = (uint16_t)(r * kBlock + tid);
         wave_lds_sync();
     }
     __syncthreads();
-    resolve_exact(kBlock >> 5, tid >> 5, undecided, n_und_s, side_lds + 4, 0, side_lds, points, P.D,
+    resolve_exact(kBlock >> 5, tid >> 5, undecided, own.n_undecided, side_lds + 4, 0, side_lds, points, P.D,
                   [&](int local) { return ids[local] & kIdMask; },
                   [&](int local, bool right) {
                       if (right) ids[local] |= (int)0x80000000;            // build_tree_check_points_side.cu:149
                       lefts += right ? 0 : 1;
                   });
     lefts = wave_sum_i(lefts);
-    if (lane == 0 && lefts) atomicAdd(&left_s, lefts);
+    if (lane == 0 && lefts) atomicAdd(&own.left, lefts);
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < kRounds; ++r)
         if (r * kBlock + tid < n) perm[pos0 + r * kBlock + tid] = ids[r * kBlock + tid];
     if (tid == 0) {
-        chunk_left[c] = left_s;
-        stat_add(stat, c, 1, n_und_s);
+        chunk_left[c] = own.left;
+        stat_add(stat, c, 1, own.n_undecided);
     }
 }
 
@@ -2630,7 +2637,7 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
 
     int cur = 0;
     const size_t side_lds = (size_t)(4 + nvec_len(D)) * sizeof(float);
-    RSFK_CHECK(side_lds <= 150 * 1024, "tree batch: D too large for the LDS of the side test");
+    RSFK_CHECK(side_lds <= kSideRecordMost, "tree batch: D too large for the LDS of the side test");
     // k_level_planes: four nodes per workgroup while their records fit in 48 KB, else one
     const int plane_waves = 4 * side_lds <= 48 * 1024 ? 4 : 1;
     if (side_lds > 48 * 1024) {

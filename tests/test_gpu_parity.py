@@ -188,14 +188,14 @@ def test_screen_is_chosen_by_the_largest_error(gpu, orc, rng, top, row_bytes):
 
 
 # Side tests of the wide levels by the 8-bit copy: rows of 64 bytes and of one line to several, whole or ending in half a line; chunks of any size; rows of NaN,
-# equal rows, and a common offset that leaves every point to the exact test.
-@pytest.mark.parametrize("D", [1, 47, 48, 49, 111, 112, 113, 176, 240, 241, 305, 1100])
+# equal rows, and a common offset that leaves every point to the exact test; rows whose hyperplane takes more than 48 KB of LDS.
+@pytest.mark.parametrize("D", [1, 47, 48, 49, 111, 112, 113, 176, 240, 241, 305, 1100, 13001])
 @pytest.mark.parametrize("kind", ["n", "nan", "dup", "offset"])
 def test_tree_wide_levels_by_the_8_bit_copy(gpu, orc, rng, monkeypatch, D, kind):
     for name, v in (("SCREEN", "q8"), ("MID", "0"), ("SMALL", "64")):
         monkeypatch.setenv("RSFK_TREE_" + name, v)
     monkeypatch.setenv("RSFK_PM_LEVELS", "0")
-    N, MIN, MAX = 5000 if D < 300 else 2500, 17, 34
+    N, MIN, MAX = 5000 if D < 300 else 2500 if D < 2000 else 300, 17, 34
     X = rng.standard_normal((N, D)).astype(np.float32)
     if kind == "nan":
         X[rng.random(N) < 0.02, D // 2] = np.nan
