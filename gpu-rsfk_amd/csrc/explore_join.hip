@@ -997,8 +997,8 @@ struct JoinSelf {
 // One wavefront per q.  Per-wavefront LDS (ints): cq[KP] | pid[32] | reach[32] | pn[32] | perr[32] | pper[32] | pe[32] | self[64] | LINES: rows[2][32] of 128 bytes, KP = K rounded up to 32.
 // Workgroups (x, y): every gridDim.y-th tile of R(q), the y-th first.
 // LINES: rows through LDS.  A lane that loads its 16 bytes of a row by itself asks for a line eight times, and the address units were busy 79 % of the
-// time; lines loaded whole cost a wavefront per SIMD and its LDS.  1M x 256 7.0 -> 6.57 ms, 300,000 x 200 1.64 -> 1.60, 100,000 x 784 1.97 -> 1.70, 60,000 x 200 with
-// K = 130 5.3 -> 4.6, 20,000 x 300 with K = 250 7.4 -> 5.3; 200,000 x 130 0.88 -> 0.95: from 161 dimensions on.
+// time; lines loaded whole cost a wavefront per SIMD and its LDS.  1M x 256 7.0 -> 6.57 ms, 100,000 x 784 1.97 -> 1.70, 60,000 x 200 with K = 130 5.3 -> 4.6, 20,000 x 300
+// with K = 250 7.4 -> 5.3 (the rule and both its sides are at the launch).
 template <int WAVES, bool BOUNDS, bool LINES>
 __global__ __launch_bounds__(64 * WAVES, LINES ? 4 : 5) void k_explore_join(JoinCopy jc, int N, int K, const int* __restrict__ old_idx,
                                                               const float* __restrict__ bars,
@@ -1655,7 +1655,13 @@ int launch_explore_join(ExploreWorkspace* w, const JoinCopy& jc, int N, int D, i
     // 64 clusters 21,000 38 35 36 36, 26,000 45 42 42 44, 32,000 51 50 51 54, 45,000 67 68 73 76, 60,000 88 92 98 102; uniform x 100 21,000 70 71
     // 75 77, 32,000 96 103 110 114, 60,000 164 184 200 213.
     const unsigned parts = (unsigned)std::max(1, std::min(16, 65536 / N));
-    const bool lines = D > 160;
+    // (k_explore_join) Whole lines through LDS or each lane its own 16 bytes: rows are fetched 64 dimensions at a time, so a last step of up to 32 costs what
+    // a full one does, and with up to 32 neighbours, where rows are read once, that decides up to 288 dimensions.  Own -> lines, us: K = 32, 20,000 x 161 92 -> 97,
+    // 192 96 -> 97, 208 94 -> 108, 240 113 -> 109, 272 114 -> 121, 289 137 -> 122, 600 228 -> 200; 300,000 x 160 1322 -> 1345, 176 1388 -> 1352, 208 1637 -> 1646, 256
+    // 1809 -> 1688, 320 2235 -> 2011; K = 24, 1M x 176 3919 -> 4048, 224 4760 -> 4762, 256 4900 -> 4715; K = 12, 60,000 x 208 120 -> 139, 240 141 -> 139, 257 138 -> 154, 320 173 ->
+    // 156.  More neighbours: K = 50, 100,000 x 144 1148 -> 1151, 161 1217 -> 1169, 200 1459 -> 1461, 20,000 x 161 221 -> 223, 192 232 -> 221, 200 239 -> 248, 288 310 -> 291;
+    // K = 140, 8,000 x 130 499 -> 539, 161 601 -> 551, 224 683 -> 621.
+    const bool lines = KP > 32 ? D > 160 : D > 288 || (D > 224 && D <= 256);
     const int wave_ints = KP + 256 + (lines ? 2 * 32 * 32 : 0);
     const size_t lds = (size_t)kWaves * (size_t)wave_ints * sizeof(int);
     const int ksteps = (D + 15) / 16;

@@ -942,7 +942,7 @@ def test_explore_with_a_workgroup_per_point(gpu, orc, rng, monkeypatch, N, D, K,
 
 
 @pytest.mark.parametrize("codes", [True, False])
-@pytest.mark.parametrize("D", [129, 191, 192, 193, 288, 292])
+@pytest.mark.parametrize("D", [129, 161, 191, 192, 193, 225, 257, 288, 292])
 @pytest.mark.parametrize("K", [31, 32, 33, 45, 63])
 def test_explore_of_long_vectors(gpu, orc, rng, monkeypatch, D, K, codes):
     """More than 128 dimensions: with the join's codes up to 288 of them (192 where D is not a multiple of 4) are read without the tile,
