@@ -375,6 +375,22 @@ bool merge_direct(int D, int dpad, bool coded)
     return dpad <= ((D & 3) == 0 ? kDirectCoded : kDirectCodedOdd);
 }
 
+// Rows of the candidates by four lanes in turn (exact_direct) or by a lane each?  The former saves requests, and takes instructions for lanes that have no
+// candidate too: it needs long rows and many candidates, and where codes leave a point few of them, points beyond the last cache (256 MB) as well.  Merge,
+// own -> quads: without codes, 100,000 points, K = 10 x 128 177 -> 219 us, K = 12 x 100 167 -> 209, K = 16 x 40 137 -> 156, x 96 210 -> 203 (1M 1.97 -> 2.06 ms), x 128
+// 293 -> 241, K = 18 x 64 188 -> 178, K = 20 x 40 180 -> 181, x 48 198 -> 184 (1M 1.83 -> 1.78), x 64 239 -> 194, K = 24 x 28 207 -> 192, x 48 290 -> 233, K = 32 x 20 282 -> 296,
+// x 24 305 -> 295 (1M 2.46 -> 2.24), x 36 441 -> 364, K = 45 x 12 507 -> 539, x 24 611 -> 600, x 40 939 -> 766; 1M x 100, K = 32 6.41 -> 4.52 ms.  With codes, K = 8, 300,000 x 256
+// 0.82 -> 1.11 ms, K = 16, 20,000 x 208 78 -> 95 us, K = 24, 1M x 208 4.83 -> 5.26, K = 28, 1M x 256 5.86 -> 5.90, K = 32, 300,000 x 132 1.38 -> 1.52, x 256 1.93 -> 1.98, 450,000 x 288
+// 3.15 -> 3.03, 1M x 132 4.35 -> 4.67, x 160 4.56 -> 4.76, x 208 5.72 -> 5.62, x 256 5.92 -> 5.61, x 288 7.18 -> 6.74.
+// (RSFK_MERGE_QUADS=0|1: never, always)
+bool merge_quads(int N, int D, int K, bool coded)
+{
+    const char* e = std::getenv("RSFK_MERGE_QUADS");
+    if (e && *e) return e[0] == '1';
+    if (coded) return K >= 32 && D > 200 && (size_t)N * (size_t)D >= (size_t)1 << 27;
+    return (K >= 24 && D >= 24) || (K >= 18 && D >= 48);
+}
+
 // Exploration of the points whose candidates the join has marked (explore_join.hip): entry (p, k) of
 // the graph has the mask of neighbour slots at pass[p K + k] (entries without a valid neighbour have none).  One wavefront per point: gather
 // the marked ids, drop repeats and ids the row holds (hash set), exact distances, merge.  Points with
@@ -382,12 +398,13 @@ bool merge_direct(int D, int dpad, bool coded)
 // per wavefront, or for the general kernel; share > 0: to the point's share of it, explore_ws_share_lists).  todo_in: the points to work on,
 // or null for all.  Per-wavefront LDS (ints): with the tile tile[64*20] | xrow[dpad] | table[table_size] | srow[K] | marked[3/4 table_size]
 // | with codes: tbound[table_size] | without the tile: the ranks (merge_rank_at).
-// kFormTile: the candidates' rows go through the transposing tile (not merge_direct).  The forms are kernels of their own, so that none carries
-// the registers of another: without the tile 75 without codes, held to the 72 of seven wavefronts per SIMD, 85 with codes, held to the 80 of six
-// (10M x 32 17.33 ms, 17.98 with six wavefronts, 24.2 with the 99 registers of code of its own choice; 1M x 256 5.65, 6.33 with seven).
-enum { kFormTile, kFormDirect, kFormDirectCoded };
+// kFormTile: the candidates' rows go through the transposing tile (not merge_direct); kFormOwn: a lane reads its candidate's row; kFormDirect, kFormDirectCoded: four
+// lanes read rows in turn (exact_direct, merge_quads), without and with codes.  The forms are kernels of their own, so that none carries
+// the registers of another: by quads and without codes 75, held to the 72 of seven wavefronts per SIMD (two are spilled, 12 bytes of scratch a lane), with codes
+// 85, held to the 80 of six (10M x 32 17.33 ms, 17.98 with six wavefronts, 24.2 with the 99 registers of code of its own choice; 1M x 256 5.65, 6.33 with seven).
+enum { kFormTile, kFormOwn, kFormDirect, kFormDirectCoded };
 template <int SL, int WAVES, int FORM>
-__global__ __launch_bounds__(64 * WAVES, FORM == kFormTile || SL > 1 ? 1 : FORM == kFormDirect ? 7 : 6) void k_explore_merge(const float* __restrict__ points, int N, int D, int K,
+__global__ __launch_bounds__(64 * WAVES, FORM == kFormTile || FORM == kFormOwn || SL > 1 ? 1 : FORM == kFormDirect ? 7 : 6) void k_explore_merge(const float* __restrict__ points, int N, int D, int K,
                                                                const int* __restrict__ old_idx, int* __restrict__ knn_idx,
                                                                float* __restrict__ knn_dist, int table_size,
                                                                int wave_lds_ints, int dpad,
@@ -551,7 +568,7 @@ __global__ __launch_bounds__(64 * WAVES, FORM == kFormTile || SL > 1 ? 1 : FORM 
     float reach = INFINITY;                               // what the row's last slot will be at most
     auto batch = [&](const int* list, int n) {
         n_exact += n;
-        if (!TILE) exact_direct<SL, true, true>(L, list, n, points, D, vec_ok, row, reach);
+        if (!TILE) exact_direct<SL, FORM != kFormOwn, true>(L, list, n, points, D, vec_ok, row, reach);
         else exact_batch<SL, kMergeChunk, true, kChainGroup, true>(L, list, n, points, D, vec_ok, row, reach);    // two steps of gathers in flight
     };
     if (tbound == nullptr || U <= kFewCandidates) {
@@ -1077,8 +1094,10 @@ int launch_merge(const float* points, int N, int D, int K, const int* old_idx, i
     const size_t lds = (size_t)WAVES * (size_t)wave_ints * sizeof(int);
     const int n_work = todo_in ? n_in : N;
     dim3 grid(grid_for_dies(((size_t)n_work + WAVES - 1) / WAVES)), block(64 * WAVES);
-    auto* kernel = !direct ? k_explore_merge<SL, WAVES, kFormTile> : bounds.codes ? k_explore_merge<SL, WAVES, kFormDirectCoded>
-                                                                                 : k_explore_merge<SL, WAVES, kFormDirect>;
+    auto* kernel = !direct                                         ? k_explore_merge<SL, WAVES, kFormTile>
+                   : !merge_quads(N, D, K, bounds.codes != nullptr) ? k_explore_merge<SL, WAVES, kFormOwn>
+                   : bounds.codes                                  ? k_explore_merge<SL, WAVES, kFormDirectCoded>
+                                                                   : k_explore_merge<SL, WAVES, kFormDirect>;
     RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     hipLaunchKernelGGL(kernel, grid, block, lds, stream, points, N, D, K, old_idx, knn_idx, knn_dist, table, wave_ints, dpad, pass,
                        bounds, todo_in, n_in, todo_out, share, n_out, stat, order);

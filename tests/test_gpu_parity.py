@@ -786,6 +786,26 @@ def test_explore_join_of_rows_of_many_neighbours(gpu, orc, rng, monkeypatch, N, 
         assert_knn_equal(gi, gd, oi, od)
 
 
+# rows shorter than what four lanes load, of whole pieces and not, of several steps; without codes and (more than 128 dimensions) with them; one and two
+# slots per lane, few candidates per point
+@pytest.mark.parametrize("quads", ["0", "1"])
+@pytest.mark.parametrize("N,D,K", [(1500, 5, 9), (1500, 23, 24), (1300, 48, 18), (1200, 47, 33), (1200, 130, 31), (900, 208, 32), (800, 288, 45), (900, 70, 80), (700, 189, 12)])
+def test_explore_reads_rows_by_one_lane_or_four(gpu, orc, rng, monkeypatch, N, D, K, quads):
+    monkeypatch.setenv("RSFK_MERGE_QUADS", quads)
+    if K > 64:
+        monkeypatch.setenv("RSFK_OPTIONAL_MB", "0")
+    X = rng.standard_normal((N, D)).astype(np.float32)
+    perm, ls, lz, _ = orc.build_tree(X, K + 1, 2 * K + 2, 5000, 0)
+    oi, od = orc.init_lists(N, K, self_in=True)
+    orc.bucket_knn(X, K, perm, lz, oi, od, starts=ls)
+    gi, gd = oi.copy(), od.copy()
+    for _ in range(2):
+        _say("explore rows", N, D, K, quads)
+        orc.explore(X, K, oi, od)
+        gpu.explore(X, K, gi, gd, 1)
+        assert_knn_equal(gi, gd, oi, od)
+
+
 # a wavefront for every 32 neighbours of a point, a workgroup for every point
 @pytest.mark.parametrize("N,D,K", [(13430000, 2, 129), (16800000, 201, 64)])
 def test_explore_of_more_points_than_a_launch_has_threads_for(gpu, N, D, K):
