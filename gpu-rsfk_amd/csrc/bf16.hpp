@@ -55,7 +55,7 @@ struct Q8Copy {
 // then has a side of its own) they must not decide, and what underflow does has to be in the band.
 // 8-bit copy: not used at all when a finite row has a coordinate beyond q8_most(D) (mean_rho is infinite then).  Up to there
 // |n.x| <= 2 D q8_most^2 = 1e38, and neither evaluation nor the offset can overflow; a row or a normal that is not finite has a
-// band that is NaN or infinite.  e1 has kQ8Least in it and the bound of the 1-norm kNormalLeast, whose product is above the
+// band that is NaN or infinite.  e1 has kQ8Least in it and L(n) kNormalLeast, whose product is above the
 // 2e-45 D that underflow amounts to.
 // bfloat16 copy: sum |n_d||x_d|, which is part of the band, is compared with 1e38 at every point.  (The same for the 8-bit copy, or
 // limits per row and per hyperplane: tail kernel and chains of 20,000 x 64, 50 trees 1.02 -> 1.06 and 1.04 ms.)

@@ -99,9 +99,10 @@ typedef __attribute__((ext_vector_type(16))) float f32x16;
 
 constexpr int kMaxBins = 6144;
 constexpr int kMaxShift = 13;
-// entry numbers are ints, and the passes over the graph look 768 entries ahead of the one they test
-constexpr size_t kDirectMost = (size_t)1 << 18;
+// entry numbers are ints, and the passes over the graph look up to 4,095 entries beyond the one they test (the staged scatters and rows; k_bin_count 3,072)
 constexpr size_t kMaxEntries = ((size_t)1 << 31) - 4096;
+// entries of the largest graph that k_rev_direct takes
+constexpr size_t kDirectMost = (size_t)1 << 18;
 constexpr int kRowsBlock = 512;             // threads of k_bin_rows
 
 // RSFK_JOIN_WG=0: the wavefront-per-q join also where the workgroup-per-q one applies.
@@ -288,9 +289,10 @@ __global__ __launch_bounds__(kRowsBlock) void k_bin_rows(const int2* __restrict_
 // The same reversed graph for small inputs, in one launch.  What bounds the five above there is their launches.  A workgroup has `per` points and goes
 // through the whole graph (from the L2): it counts the entries of the points before its own, which is where its rows begin, and lists the numbers of its
 // own in LDS, which are then counted, scanned and placed; if they are more than fit, it goes through the graph twice more.
-// 3,000 x 30 13.4 us against 22 in five launches, the call (two passes) 748 -> 705; 10,000 x 32 17.2 against 25, 592 -> 579; 20,000 x 32 54 against 24, the call 1.72
-// ms with the five and 1.76 with the one: up to 2^18 entries.  (Bound by its instructions, six per entry in every workgroup: a branch and an addition per
-// entry 15.1, 20.6, 60 us; the next entries on their way, or workgroups that begin in different places, the same.)
+// Points x neighbours, us in one launch and the kernels of the five: 3,000 x 30 13 and 29, 10,000 x 16 17 and 25, 8,000 x 25 21 and 28, 16,000 x 16 (256,000 entries) 24.9 and
+// 25.4, 2,600 x 100 25 and 51, 8,200 x 32 25 and 31, 20,000 x 16 (320,000) 30 and 26, 10,000 x 32 29 and 31, 40,000 x 10 36 and 26, 14,000 x 32 39 and 29, 20,000 x 32 (640,000) 53 and
+// 33: up to 2^18 entries.  (Bound by its instructions, six per entry in every workgroup: a branch and an addition per entry instead 15, 21 and 60 us for 3,000 x 30,
+// 10,000 x 16 and 20,000 x 32; the next entries on their way, or workgroups that begin in different places, the same.)
 constexpr int kDirectThreads = 1024, kDirectCap = 8192, kDirectMostPer = 4096;
 typedef int i32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 
@@ -1425,12 +1427,6 @@ bool explore_join_enabled(int N, int K)
     if (K > kMaxKJoin) return false;          // (rows of more than 256 neighbours: the general kernel only)
     int shift, n_bins;
     return (size_t)N * (size_t)K < kMaxEntries && rev_bins(N, &shift, &n_bins);
-}
-
-size_t explore_ws_bytes(int N, int K)
-{
-    const size_t mw = (size_t)((K + 31) / 32);
-    return (size_t)N * ((size_t)K * (12 + 4 * mw) + 32) + ((size_t)20 << 20);
 }
 
 int explore_ws_alloc(ExploreWorkspace** out, int N, int K, bool with_bounds, bool graph_only)

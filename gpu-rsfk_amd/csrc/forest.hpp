@@ -196,7 +196,6 @@ void release_copy_buffers();
 struct ExploreWorkspace;
 bool explore_join_enabled(int N, int K);
 bool explore_merge_fits(int D, int K);
-size_t explore_ws_bytes(int N, int K);
 // graph_only: room for the reversed graph alone (launch_reversed_graph), as blocks the caller can do without (ws_try_alloc)
 int explore_ws_alloc(ExploreWorkspace** out, int N, int K, bool with_bounds = false, bool graph_only = false);
 bool explore_ws_takes(int N, int K);
