@@ -807,9 +807,10 @@ int launch_ann_forest(const float* points, const float* queries, int N, int NQ, 
     const size_t lds = ann_forest_lds(D, K);
     // Rows of a few lines in an L2 are read sooner by a lane each: four lanes that exchange what they load take more instructions, and save
     // requests that only count where there are many, from farther away.  A call, own rows -> quads, K = 16, 50 trees, 10,000 queries: 5,000 x 24 +7 %, x 48 -1,
-    // x 60 -7, x 96 -14; 40,000 x 24 +2, x 48 -9, x 96 -16; 1,000 x 64 0; K = 10, 12 trees, 10,000 queries: 5,000 x 24 +4, x 72 +3, 3,000 x 150 -6; K = 16, 20
+    // x 60 -7, x 96 -14; 20,000 x 40 -2; 40,000 x 24 +2, x 32 -4, x 48 -9, x 96 -16; 300,000 x 24 -1, x 32 -2; K = 32, 20 trees, 23,234 queries: 367,009 x 29 (clusters) -17; 1,000 x 64 0; K = 10, 12 trees, 10,000 queries: 5,000 x 24 +4, x 72 +3, 3,000 x 150 -6; K = 16, 20
     // trees, 8,000 queries: 3,000 x 56 +4, 20,000 x 56 -4, 20,000 x 112 -14; K = 10, 20 trees: 2,000 x 100 +3 to +5; K = 107, 50 trees, 62,271 queries: 1,909 x 3 +29.
-    const bool quads = D > 128 || (D > 48 && T * K >= 250 && (size_t)N * (size_t)D >= (size_t)1 << 18);
+    const size_t words = (size_t)N * (size_t)D;
+    const bool quads = D > 128 || (D > 48 && T * K >= 250 && words >= (size_t)1 << 18) || (D >= 28 && T * K >= 500 && words >= (size_t)1 << 20);
 #define RSFK_ANN_CASE(SLV)                                                                                                    \
     do {                                                                                                                     \
         auto* kernel = quads ? k_ann_forest<SLV, true> : k_ann_forest<SLV, false>;                                            \

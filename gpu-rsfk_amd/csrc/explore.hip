@@ -378,7 +378,7 @@ bool merge_direct(int D, int dpad, bool coded)
 // Rows of the candidates by four lanes in turn (exact_direct) or by a lane each?  The former saves requests, and takes instructions for lanes that have no
 // candidate too: it needs long rows and many candidates, and where codes leave a point few of them, points beyond the last cache (256 MB) as well.  Merge,
 // own -> quads: without codes, 100,000 points, K = 10 x 128 177 -> 219 us, K = 12 x 100 167 -> 209, K = 16 x 40 137 -> 156, x 96 210 -> 203 (1M 1.97 -> 2.06 ms), x 128
-// 293 -> 241, K = 18 x 64 188 -> 178, K = 20 x 40 180 -> 181, x 48 198 -> 184 (1M 1.83 -> 1.78), x 64 239 -> 194, K = 24 x 28 207 -> 192, x 48 290 -> 233, K = 32 x 20 282 -> 296,
+// 293 -> 241, 755,473 x 115 (sparse) 2.97 -> 1.95 ms, 1M x 112, 10 trees 1.86 -> 2.18, K = 18 x 64 188 -> 178, K = 20 x 40 180 -> 181, x 48 198 -> 184 (1M 1.83 -> 1.78), x 64 239 -> 194, K = 24 x 28 207 -> 192, x 48 290 -> 233, K = 32 x 20 282 -> 296,
 // x 24 305 -> 295 (1M 2.46 -> 2.24), x 36 441 -> 364, K = 45 x 12 507 -> 539, x 24 611 -> 600, x 40 939 -> 766; 1M x 100, K = 32 6.41 -> 4.52 ms.  With codes, K = 8, 300,000 x 256
 // 0.82 -> 1.11 ms, K = 16, 20,000 x 208 78 -> 95 us, K = 24, 1M x 208 4.83 -> 5.26, K = 28, 1M x 256 5.86 -> 5.90, K = 32, 300,000 x 132 1.38 -> 1.52, x 256 1.93 -> 1.98, 450,000 x 288
 // 3.15 -> 3.03, 1M x 132 4.35 -> 4.67, x 160 4.56 -> 4.76, x 208 5.72 -> 5.62, x 256 5.92 -> 5.61, x 288 7.18 -> 6.74.
@@ -388,7 +388,7 @@ bool merge_quads(int N, int D, int K, bool coded)
     const char* e = std::getenv("RSFK_MERGE_QUADS");
     if (e && *e) return e[0] == '1';
     if (coded) return K >= 32 && D > 200 && (size_t)N * (size_t)D >= (size_t)1 << 27;
-    return (K >= 24 && D >= 24) || (K >= 18 && D >= 48);
+    return (K >= 24 && D >= 24) || (K >= 18 && D >= 48) || (K >= 16 && D >= 96);
 }
 
 // Exploration of the points whose candidates the join has marked (explore_join.hip): entry (p, k) of
