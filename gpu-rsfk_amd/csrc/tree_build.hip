@@ -184,8 +184,9 @@ __device__ __forceinline__ void make_hyperplane_wave(const float* __restrict__ x
 // (KU: pieces of a row a lane has in flight, 8-bit copy)
 // INSIDE: the header comes with the row, as its first piece, above nothing of the normal (header_inside says where; 16 floats that can be read have to be before
 // nvec0): the row then comes in loads of whole lines, each once, where a load of its own asks for the first line again while it is on its way.  Middle phase
-// of 123,457 x 37, 12 trees 0.202 -> 0.182 ms, of 3,000 x 200, 10 trees 0.046 -> 0.043.  Not in the tail kernel, which is bound by its instructions: 5,000 x 24, 50
-// trees 135 -> 138 us, 8,000 x 32, 8 trees 114 -> 117, 5,000 x 52, 50 trees 156 -> 160, 200,000 x 32, 12 trees 363 -> 367.
+// of 123,457 x 37, 12 trees 0.202 -> 0.182 ms, of 3,000 x 200, 10 trees 0.046 -> 0.043.  In the tail kernel, which is bound by its instructions, only where the row is
+// then a single step of its lanes (up to 16 dimensions: 458,955 x 15, 27 trees 1.77 -> 1.65 ms, 1M x 2, 10 trees 1.48 -> 1.43); with longer rows it is the same, and to decide it at each row
+// costs 1 to 3 % (5,000 x 24, 50 trees 135 -> 138 us, 8,000 x 32, 8 trees 114 -> 117, 5,000 x 52, 50 trees 156 -> 160, 200,000 x 32, 12 trees 363 -> 367).
 template <int LPP>
 bool header_inside(int D) { return (q8_padded(D) >> 4) % LPP != 0; }      // (the last step has a lane to spare)
 
@@ -1017,7 +1018,7 @@ constexpr int kMaxGroup = 16;        // nodes of one level of a subtree worked o
 // it has to stay within 80 registers (81 and five wavefronts: 1M x 100, 50 trees 10.8 -> 12.3 ms).
 // LPP: lanes per point in the screen (side_screen8), eight with the bfloat16 copy; KU: 16-byte pieces of a point's row each of them has in
 // flight.
-template <bool Q8, int TB, bool CHAIN, int LPP, int KU>
+template <bool Q8, int TB, bool CHAIN, int LPP, int KU, bool INSIDE>
 __global__ __launch_bounds__(TB, CHAIN ? 4 : 6) void k_tail(const float* __restrict__ points,
                                                  const uint16_t* __restrict__ pb16, const uint8_t* __restrict__ q8, TreeParams P,
                                                  const int* __restrict__ perm0, const int* __restrict__ perm1,
@@ -1162,7 +1163,7 @@ __global__ __launch_bounds__(TB, CHAIN ? 4 : 6) void k_tail(const float* __restr
                     h1[u] = hp_s[jj[u]][1];
                     h2[u] = hp_s[jj[u]][2];
                 }
-                side_screen8<kTailBatch, Q8, LPP, KU>(nvec, Dv, jj, bb, h1, h2, pb16, q8, id, P.D, P.band, valid, right, redo);
+                side_screen8<kTailBatch, Q8, LPP, KU, INSIDE>(nvec, Dv, jj, bb, h1, h2, pb16, q8, id, P.D, P.band, valid, right, redo);
 #pragma unroll
                 for (int u = 0; u < kTailBatch; ++u) {
                     if (valid[u] && sub == 0) {
@@ -2790,11 +2791,12 @@ int build_tree_batch(TreeBatchWorkspace* w, const float* points, const uint16_t*
         const size_t lds = besides + (size_t)G * plane;
 #define RSFK_TAIL_LAUNCH(Q, T, C, L, U)                                                                                       \
         do {                                                                                                               \
-            RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_tail<Q, T, C, L, U>),                                \
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));                          \
-            hipLaunchKernelGGL((k_tail<Q, T, C, L, U>), dim3(n_tail), dim3(T), lds, stream, points, pb16, q8, P, w->perm[0],   \
-                               w->perm[1], w->perm[0], w->tail, n_tail, leaf_most, node_most, G, w->leaf_cap, w->leaf_start,            \
-                               w->leaf_size, w->stats, w->ctr, w->recs, w->rec_cap, w->stat, w->chain, w->tail_cap);         \
+            constexpr bool two = (L) == 2;                                                                                   \
+            auto* kernel = two && header_inside<L>(D) ? k_tail<Q, T, C, L, U, two> : k_tail<Q, T, C, L, U, false>;              \
+            RSFK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)); \
+            hipLaunchKernelGGL(kernel, dim3(n_tail), dim3(T), lds, stream, points, pb16, q8, P, w->perm[0], w->perm[1], w->perm[0],  \
+                               w->tail, n_tail, leaf_most, node_most, G, w->leaf_cap, w->leaf_start, w->leaf_size, w->stats, w->ctr, \
+                               w->recs, w->rec_cap, w->stat, w->chain, w->tail_cap);                                          \
         } while (0)
         // Lanes per point: as many as there are pieces of 16 coordinates, up to four; few subtrees wait for the loads of a point, and
         // four lanes with four pieces in flight each take longer rows (eight beyond 256 dimensions).  With many subtrees eight lanes keep the
