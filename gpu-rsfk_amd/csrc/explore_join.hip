@@ -965,7 +965,8 @@ __device__ __forceinline__ float join_floor(float n_c, float kappa) { return 0.5
 // ballot over the wavefront holds the 32-bit masks of two points, low half for m = 8 (i / 4) + i % 4, high half for m + 4.  Lane m < 32 is left with
 // the mask of point m.  reach: join_reach of the tile's points (LDS).  No branch and no wait for LDS between the sixteen, and a mask goes to its lane in
 // one instruction: 10M x 32 23.06 -> 21.96 ms, 1M x 100 3.23 -> 2.86, 123,457 x 37 with K = 45 0.443 -> 0.367, 70,000 x 784 with K = 90 5.36 -> 5.05, 1M x 256
-// (whose codes are stored pair by pair) 7.0 either way.
+// (whose codes are stored pair by pair) 7.0 either way.  (write_lane_u32 is declared by the name of the compiler's intrinsic: with a compiler that names it otherwise
+// the library does not link, for want of that symbol.)
 __device__ __forceinline__ uint32_t join_masks(const f32x16& g, const float* reach, int mbase, float floor_c)
 {
     uint32_t mine = 0;
@@ -999,7 +1000,7 @@ struct JoinSelf {
 // One wavefront per q.  Per-wavefront LDS (ints): cq[KP] | pid[32] | reach[32] | pn[32] | perr[32] | pper[32] | pe[32] | self[64] | LINES: rows[2][32] of 128 bytes, KP = K rounded up to 32.
 // Workgroups (x, y): every gridDim.y-th tile of R(q), the y-th first.
 // LINES: rows through LDS.  A lane that loads its 16 bytes of a row by itself asks for a line eight times, and the address units were busy 79 % of the
-// time; lines loaded whole cost a wavefront per SIMD and its LDS.  1M x 256 7.0 -> 6.57 ms, 100,000 x 784 1.97 -> 1.70, 60,000 x 200 with K = 130 5.3 -> 4.6, 20,000 x 300
+// time (1M x 256; 52 % by lines); lines loaded whole cost a wavefront per SIMD and its LDS.  1M x 256 7.0 -> 6.57 ms, 100,000 x 784 1.97 -> 1.70, 60,000 x 200 with K = 130 5.3 -> 4.6, 20,000 x 300
 // with K = 250 7.4 -> 5.3 (the rule and both its sides are at the launch).
 template <int WAVES, bool BOUNDS, bool LINES>
 __global__ __launch_bounds__(64 * WAVES, LINES ? 4 : 5) void k_explore_join(JoinCopy jc, int N, int K, const int* __restrict__ old_idx,

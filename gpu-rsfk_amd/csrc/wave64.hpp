@@ -33,8 +33,7 @@ __device__ __forceinline__ float read_lane_f(float v, int lane)
 }
 __device__ __forceinline__ int read_lane_i(int v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
 
-// v with lane `lane` (a constant) replaced by the wave-uniform x: v_writelane, for which the compiler has an intrinsic and no builtin.  The declaration takes the
-// intrinsic's name; with a compiler that names it otherwise the library does not link (undefined symbol of this name).
+// v with lane `lane` (a constant) replaced by the wave-uniform x: v_writelane, for which the compiler has an intrinsic and no builtin
 __device__ uint32_t write_lane_u32(uint32_t x, uint32_t lane, uint32_t v) __asm("llvm.amdgcn.writelane.i32");
 
 // DPP controls
